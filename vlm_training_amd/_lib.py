@@ -1,4 +1,5 @@
-"""ctypes binding of libdsa_attn.so (the C ABI declared in include/dsa_attn.h).
+"""Bindings of the two in-tree libraries: libdsa_attn.so by ctypes (the C ABI declared in include/dsa_attn.h), and
+_dsa_host.so, the extension module with the operators' host side (csrc/dsa_host.cpp).
 
 There is no CPU or eager fallback: if the library is missing, every operator raises.
 """
@@ -10,6 +11,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdsa_attn.so")
+HOST_PATH = os.path.join(_HERE, "_dsa_host.so")
 
 DSA_DTYPE_BF16 = 0
 DSA_DTYPE_FP32 = 1
@@ -94,6 +96,7 @@ _SIGNATURES = {
 
 EXPORTS = tuple(_SIGNATURES)
 _lib = None
+_host = None
 
 
 class DsaLibraryError(RuntimeError):
@@ -116,6 +119,20 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def host():
+    """The extension module with the operators' host side; raise loudly when it has not been built."""
+    global _host
+    load()
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise DsaLibraryError(f"{HOST_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}` "
+                                  "(or __graft_entry__.build()); there is no fallback path")
+        import torch  # noqa: F401  (the module links against its libraries)
+        from . import _dsa_host
+        _host = _dsa_host
+    return _host
 
 
 def check(rc: int, what: str):

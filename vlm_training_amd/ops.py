@@ -1,6 +1,7 @@
 """Host side of the DSA packed-attention operator: torch tensors in, HIP kernels through the C ABI.
 
-``dsa_varlen_attn`` is the operator (a ``torch.autograd.Function`` underneath).  With no indexer
+``dsa_varlen_attn`` is the operator; its checks, allocations, launches and autograd node are C++ (csrc/dsa_host.cpp).  The
+stage wrappers below drive single stages through the C ABI.  With no indexer
 inputs it is dense causal varlen attention, i.e. what the reference gets from
 ``varlen_attn(q, k, v, cu_seq_q=cu, cu_seq_k=cu, max_q=m, max_k=m, window_size=(-1, 0))``
 (train/model_attention.py:123-132, models/qwen3_vl/model.py:41-46, models/qwen3_5/model.py:93-98).
@@ -56,6 +57,13 @@ def _as_bf16_x3(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor):
     return ys[0], ys[1], ys[2]
 
 
+def _check_finite(*tensors):
+    # the device ranks NaN above +inf without a word; under DSA_DEBUG_NAN (one device-to-host copy) it is an error, as it
+    # is in the CPU restatement of the selection
+    if not all(torch.isfinite(_as_bf16(t).float()).all() for t in tensors):
+        raise ValueError("non-finite indexer inputs: their scores have no defined rank")
+
+
 def _check_cu(cu_seqlens: torch.Tensor, T: int, max_seqlen: Optional[int] = None):
     if cu_seqlens.dim() != 1 or cu_seqlens.numel() < 2:
         raise ValueError("cu_seqlens must be 1-D with at least two entries")
@@ -74,10 +82,6 @@ def _check_cu(cu_seqlens: torch.Tensor, T: int, max_seqlen: Optional[int] = None
         if max_seqlen is not None and longest > max_seqlen:
             raise ValueError(f"max_seqlen={max_seqlen} is below the longest segment ({longest})")
     return cu_seqlens.contiguous()
-
-
-_KERNEL_HEAD_DIMS = (64, 128, 256)                   # head_dim instantiations of the tile and gather kernels
-_KERNEL_HEAD_DIMS_DENSE = (64, 96, 128, 256)         # without a key selection the tile kernels also come at head_dim 96
 
 
 def _check_qkv(q, k, v):
@@ -154,10 +158,7 @@ def index_topk(q_idx, k_idx, w_idx, cu_seqlens, max_seqlen: int, top_k: int,
     ws = torch.empty((max(ws_bytes, 4),), dtype=torch.uint8, device=q_idx.device)
     qi, ki, wi = _as_bf16_x3(q_idx, k_idx, w_idx)                      # keep the casts alive over the launch
     if os.environ.get("DSA_DEBUG_NAN"):
-        # the device ranks NaN above +inf without a word; with this switch (one device-to-host copy) it is an error,
-        # as it is in the CPU restatement of the selection
-        if not (torch.isfinite(qi.float()).all() and torch.isfinite(ki.float()).all() and torch.isfinite(wi.float()).all()):
-            raise ValueError("non-finite indexer inputs: their scores have no defined rank")
+        _check_finite(qi, ki, wi)
     if bitmap is not None:
         sel = torch.empty((T, top_k), dtype=torch.float32, device=q_idx.device) if return_scores else None
         rc = lib.dsa_index_topk_bitmap(_ptr(qi), _ptr(ki), _ptr(wi), _ptr(cu), T, cu.numel() - 1, Hi, Di, top_k, scale,
@@ -226,26 +227,6 @@ def indexer_bwd(q_idx, k_idx, w_idx, idx, n, dscore, cu_seqlens, max_seqlen: int
     return dq, dk, dw
 
 
-class _IndexerKL(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q_idx, k_idx, w_idx, mass, cu_seqlens, max_seqlen, top_k, index_scale, idx=None, n=None, sel=None):
-        T = q_idx.shape[0]
-        if sel is None:
-            idx, n, sel = index_topk(q_idx, k_idx, w_idx, cu_seqlens, max_seqlen, top_k, index_scale, return_scores=True)
-        loss_rows, dscore = indexer_kl(sel, mass, n, grad_scale=1.0 / max(T, 1))
-        ctx.save_for_backward(q_idx, k_idx, w_idx, idx, n, dscore, cu_seqlens)
-        ctx.max_seqlen, ctx.index_scale = max_seqlen, index_scale
-        return loss_rows.mean()
-
-    @staticmethod
-    def backward(ctx, g):
-        q_idx, k_idx, w_idx, idx, n, dscore, cu = ctx.saved_tensors
-        # the gradients are linear in dscore: scale the (T,K) table by the incoming gradient, not the three results
-        dq, dk, dw = indexer_bwd(q_idx, k_idx, w_idx, idx, n, dscore * g.to(torch.float32), cu, ctx.max_seqlen,
-                                 ctx.index_scale)
-        return (dq.to(q_idx.dtype), dk.to(k_idx.dtype), dw.to(w_idx.dtype), None, None, None, None, None, None, None, None)
-
-
 @torch.compiler.disable
 def indexer_kl_loss(indexer_q, indexer_k, indexer_w, mass, cu_seqlens, max_seqlen: Optional[int], top_k: int,
                     index_scale: Optional[float] = None, selection=None):
@@ -256,11 +237,14 @@ def indexer_kl_loss(indexer_q, indexer_k, indexer_w, mass, cu_seqlens, max_seqle
     inputs and top_k.  ``selection=(idx, n, scores)`` as returned by ``dsa_varlen_attn(..., return_indices=True,
     return_scores=True)`` saves a second run of the indexer; without it the selection is recomputed here (it is
     deterministic, hence the same)."""
-    T = indexer_q.shape[0]
-    max_seqlen = T if max_seqlen is None else int(max_seqlen)
+    max_seqlen = indexer_q.shape[0] if max_seqlen is None else int(max_seqlen)
     idx, n, sel = selection if selection is not None else (None, None, None)
-    return _IndexerKL.apply(indexer_q, indexer_k, indexer_w, mass, cu_seqlens, max_seqlen, int(top_k), index_scale, idx, n,
-                            sel)
+    if os.environ.get("DSA_DEBUG_META"):
+        _check_cu(cu_seqlens, indexer_q.shape[0], max_seqlen)
+    if sel is None and os.environ.get("DSA_DEBUG_NAN"):
+        _check_finite(indexer_q, indexer_k, indexer_w)
+    return _lib.host().indexer_kl_loss(indexer_q, indexer_k, indexer_w, mass, cu_seqlens, max_seqlen, int(top_k), index_scale, idx, n,
+                                       sel)
 
 
 def set_tile_crossover(crossover: int) -> int:
@@ -435,76 +419,14 @@ def _split_combine_qkv(dq, dk, dv):
     return oq, okv[0], okv[1]
 
 
-class _DsaVarlenAttn(torch.autograd.Function):
-    """bf16 inputs go to the kernels as they are.  fp32 inputs with 4*D <= 256 are carried as split-bf16
-    operands (x = hi + lo) stacked along head_dim, which keeps near-fp32 logits on the bf16 MFMA path:
-        Q' = [q_hi, q_lo, q_hi, 0]   K' = [k_hi, k_hi, k_lo, 0]   ->  Q'.K' = q.k - q_lo.k_lo
-        V' = [v_hi, v_lo, v_hi, 0]   ->  out = out'[0:D] + out'[D:2D]
-        dO' = [g_hi, g_hi, g_lo, 0]  ->  dO'.V' = g.v - g_lo.v_lo ;  dq = dq'[0:D] + dq'[2D:3D],
-                                         dk = dk'[0:D] + dk'[D:2D], dv = dv'[0:D] + dv'[2D:3D]
-    Other dtypes / larger head_dim are rounded to bf16 once."""
+class _DsaVarlenAttn:
+    """The attention node on a selection the caller holds (``AttnNode`` in csrc/dsa_host.cpp)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, cu_seqlens, max_seqlen, idx, n, softmax_scale, causal=True, want_mass=False, bitmap=None):
-        in_dtype = q.dtype
-        D = q.shape[-1]
-        split = in_dtype == torch.float32 and 4 * D <= 256
-        if split:
-            qb, kb, vb = _split_stack_qkv(q, k, v)
-        else:
-            qb, kb, vb = _as_bf16(q), _as_bf16(k), _as_bf16(v)
-        fwd_ws = None
-        lib = _lib.load()
-        if idx is not None and lib.dsa_get_tile_crossover() > 0:     # (crossover 0: no kernel reads a bitmap)
-            # the selection bitmap - left by the top-k kernel (`bitmap`), else built by the forward - is kept for the
-            # backward; nothing else is held in between (delta, the key-tile order and the partial sums of cut walks
-            # are allocated when the backward runs)
-            fwd_ws = bitmap if bitmap is not None else torch.empty(
-                (max(lib.dsa_attn_fwd_workspace_bytes(qb.shape[0], int(max_seqlen), 1), 4),), dtype=torch.uint8, device=qb.device)
-        out, lse = attn_fwd(qb, kb, vb, idx, n, cu_seqlens, int(max_seqlen), softmax_scale, causal, ws=fwd_ws,
-                            bitmap_ready=fwd_ws is not None and bitmap is not None)
-        ctx.fwd_ws = fwd_ws
-        ctx.causal = bool(causal)
-        ctx.save_for_backward(qb, kb, vb, out, lse, cu_seqlens, *(() if idx is None else (idx, n)))
-        ctx.has_idx = idx is not None
-        ctx.max_seqlen = int(max_seqlen)
-        ctx.softmax_scale = softmax_scale
-        ctx.in_dtype = in_dtype
-        ctx.split = split
-        ctx.D = D
-        if split:
-            res = _split_combine(out, 1)
-        else:
-            res = out if in_dtype == torch.bfloat16 else out.to(in_dtype)
-        if not want_mass:
-            return res
-        # from the very operands and log-sum-exp of the forward, so that every row sums to one
-        mass = attn_mass(qb, kb, lse, idx, n, cu_seqlens, int(max_seqlen), softmax_scale, bitmap=fwd_ws)
-        ctx.mark_non_differentiable(mass)
-        return res, mass
-
-    @staticmethod
-    def backward(ctx, dout, *_):
-        saved = ctx.saved_tensors
-        qb, kb, vb, out, lse, cu = saved[:6]
-        idx, n = (saved[6], saved[7]) if ctx.has_idx else (None, None)
-        D = ctx.D
-        if ctx.split:
-            db = _split_stack(dout.float(), 1)
-        else:
-            db = _as_bf16(dout)
-        if ctx.fwd_ws is not None or idx is None:        # the forward's bitmap is read where it lies
-            dq, dk, dv = attn_bwd_saved_bitmap(db, qb, kb, vb, out, lse, idx, n, cu, ctx.max_seqlen, ctx.softmax_scale,
-                                               ctx.fwd_ws, causal=ctx.causal)
-            ctx.fwd_ws = None
-        else:
-            dq, dk, dv = attn_bwd(db, qb, kb, vb, out, lse, idx, n, cu, ctx.max_seqlen, ctx.softmax_scale,
-                                  causal=ctx.causal)
-        if ctx.split:
-            dq, dk, dv = _split_combine_qkv(dq, dk, dv)
-        elif ctx.in_dtype != torch.bfloat16:
-            dq, dk, dv = dq.to(ctx.in_dtype), dk.to(ctx.in_dtype), dv.to(ctx.in_dtype)
-        return dq, dk, dv, None, None, None, None, None, None, None, None
+    def apply(q, k, v, cu_seqlens, max_seqlen, idx, n, softmax_scale, causal=True, want_mass=False, bitmap=None):
+        res = _lib.host().attn_node(q, k, v, _check_cu(cu_seqlens, q.shape[0]), int(max_seqlen), idx, n, float(softmax_scale), bool(causal),
+                                    bool(want_mass), bitmap)
+        return tuple(res) if want_mass else res[0]
 
 
 @torch.compiler.disable                                  # a compiled caller (the reference compiles per block) breaks the graph here
@@ -530,49 +452,13 @@ def dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen: Optional[int] = None, *, in
     next one and the output cut back (the scale stays that of the true head_dim).  ``causal=False`` (dense only) attends every key of the own segment, the
     vision towers' form of the call (models/qwen3_vl/model.py:423-428).
     """
-    _require_cuda(q, k, v, cu_seqlens)
-    T, Hq, Hkv, D = _check_qkv(q, k, v)
-    max_seqlen = T if max_seqlen is None else int(max_seqlen)
-    cu = _check_cu(cu_seqlens, T, max_seqlen)
-    scale = float(softmax_scale) if softmax_scale is not None else D ** -0.5
-    sparse = indexer_q is not None or indexer_k is not None or indexer_w is not None
-    idx = n = bitmap = None
-    if sparse and not causal:
-        raise ValueError("DSA key selection is defined for causal attention only")
-    if sparse:
-        if indexer_q is None or indexer_k is None or indexer_w is None or top_k is None:
-            raise ValueError("DSA needs indexer_q, indexer_k, indexer_w and top_k together")
-        if indexer_q.shape[0] != T:
-            raise ValueError("indexer tensors must cover the same T packed tokens as q")
-        lib = _lib.load()
-        if lib.dsa_get_tile_crossover() > 0:
-            # the top-k kernel leaves the inverted selection here: forward and backward read it, nothing builds it again
-            bitmap = torch.empty((max(lib.dsa_attn_fwd_workspace_bytes(T, int(max_seqlen), 1), 4),), dtype=torch.uint8,
-                                 device=q.device)
-        with torch.no_grad():
-            if return_scores:
-                idx, n, sel_scores = index_topk(indexer_q, indexer_k, indexer_w, cu, int(max_seqlen), int(top_k), index_scale,
-                                                return_scores=True, bitmap=bitmap)
-            else:
-                idx, n = index_topk(indexer_q, indexer_k, indexer_w, cu, int(max_seqlen), int(top_k), index_scale, bitmap=bitmap)
-    elif return_indices or return_scores:
-        raise ValueError("return_indices / return_scores need the indexer inputs")
-    dims = _KERNEL_HEAD_DIMS if sparse else _KERNEL_HEAD_DIMS_DENSE
-    d_kernel = next((d for d in dims if d >= D), None)
-    if d_kernel is None:
-        raise ValueError(f"head_dim {D} is beyond the kernels' largest ({_KERNEL_HEAD_DIMS[-1]})")
-    if d_kernel != D:
-        # e.g. the 72-wide heads of the 1152/16 vision towers: zero columns change neither q.k nor the used part of p.v
-        q, k, v = (torch.nn.functional.pad(x, (0, d_kernel - D)) for x in (q, k, v))
-    if return_mass and not sparse:
-        raise ValueError("return_mass needs the indexer inputs")
-    out = _DsaVarlenAttn.apply(q.contiguous(), k.contiguous(), v.contiguous(), cu, int(max_seqlen), idx, n, scale,
-                               bool(causal), bool(return_mass), bitmap)
-    mass = None
-    if return_mass:
-        out, mass = out
-    if d_kernel != D:
-        out = out[..., :D]
-    res = (out,) + ((idx, n) if return_indices else ()) + ((mass,) if return_mass else ()) + (
-        (sel_scores,) if return_scores else ())
-    return res if len(res) > 1 else out
+    if os.environ.get("DSA_DEBUG_META"):
+        _require_cuda(q, k, v, cu_seqlens)
+        T = _check_qkv(q, k, v)[0]
+        _check_cu(cu_seqlens, T, T if max_seqlen is None else int(max_seqlen))
+    if indexer_q is not None and os.environ.get("DSA_DEBUG_NAN"):
+        _check_finite(indexer_q, indexer_k, indexer_w)
+    res = _lib.host().varlen_attn(q, k, v, cu_seqlens, None if max_seqlen is None else int(max_seqlen), indexer_q, indexer_k, indexer_w,
+                                  None if top_k is None else int(top_k), index_scale, None if softmax_scale is None else float(softmax_scale),
+                                  bool(return_indices), bool(causal), bool(return_mass), bool(return_scores))
+    return tuple(res) if len(res) > 1 else res[0]
