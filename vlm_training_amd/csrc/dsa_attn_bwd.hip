@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64) void dsa_bwd_dq_kernel(
     const int lane = threadIdx.x, g = lane >> 4, m = lane & 15;
     const int kvh = blockIdx.x % Hkv, t = blockIdx.x / Hkv;
     const int G = Hq / Hkv;
-    const int s0 = cu[find_segment(cu, N, t)];
+    const int s0 = cu[find_segment_wave(cu, N, t)];
     if (t - s0 < pos_min) return;                     // rows before the split belong to the tile kernel
     // the count is held to [0, K] and every row id to the batch: a bad list cannot reach outside the tensors
     const int nt = HAS_IDX ? min(nsel[t], K) : (t - s0 + 1);
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void dsa_bitmap_kernel(const int32_t *__restri
                                                              uint32_t *__restrict__ bitmap) {
     extern __shared__ uint32_t words[];
     const int t = blockIdx.x, tid = threadIdx.x;
-    const int s0 = cu[find_segment(cu, N, t)];
+    const int s0 = cu[find_segment_wave(cu, N, t)];
     for (int i = tid; i < ldw; i += 256) words[i] = 0u;
     __syncthreads();
     // entries outside the row's ldw words (a list that names keys of another segment, or a max_seqlen below the

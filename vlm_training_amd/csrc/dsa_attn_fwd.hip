@@ -32,7 +32,7 @@ __global__ __launch_bounds__(64) void dsa_attn_fwd_kernel(
     const int lane = threadIdx.x, g = lane >> 4, m = lane & 15;
     const int kvh = blockIdx.x % Hkv, t = blockIdx.x / Hkv;
     const int G = Hq / Hkv;
-    const int s0 = cu[find_segment(cu, N, t)];
+    const int s0 = cu[find_segment_wave(cu, N, t)];
     if (t - s0 < pos_min) return;                             // rows before the split belong to the tile kernel
     // a caller's own list is trusted for its order only: the count is held to [0, K] and every row id to the batch, so
     // that a bad list gives a wrong result, never an access outside the tensors

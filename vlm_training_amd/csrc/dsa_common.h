@@ -65,6 +65,20 @@ __device__ __forceinline__ int find_segment(const int32_t *__restrict__ cu, int 
     return lo;
 }
 
+// the same by a whole wave (t wave-uniform, every lane active): the offsets are fetched 64 at a time, one per lane, in one
+// memory round trip each instead of one round trip per step of a binary search
+__device__ __forceinline__ int find_segment_wave(const int32_t *__restrict__ cu, int N, int t) {
+    const int lane = threadIdx.x & 63;
+    int below = 0;                 // offsets cu[0 .. N-1] that are <= t; the segment is the last of them
+    for (int base = 0; base < N; base += 64) {
+        const int c = cu[min(base + lane, N - 1)];
+        const int hits = (int)__popcll(__builtin_amdgcn_ballot_w64(base + lane < N && c <= t));
+        below += hits;
+        if (hits < 64) break;
+    }
+    return max(below - 1, 0);
+}
+
 __device__ __forceinline__ float wave_xor_f(float v, int m) { return __shfl_xor(v, m, 64); }
 // maximum / sum over the two lanes 32 apart, on every lane: v_permlane32_swap exchanges the wave's halves in
 // the vector ALU (no LDS round trip, so LDS reads in flight are not waited for)
@@ -76,3 +90,29 @@ __device__ __forceinline__ float half_sum_f(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+
+// ---- memory straight into LDS (buffer_load ... lds) ------------------------------------------------------------------
+// A wave's load puts 64 x 16 bytes at consecutive LDS addresses, lane by lane, without passing through registers.  It is
+// inline assembly because the compiler's own intrinsic makes every later LDS read wait for every such load; here the
+// kernel waits itself (wait_vmcnt, then a barrier) before anything reads the bytes.  A compiler-made vmcnt wait only ever
+// waits longer for the loads it does not know of.
+typedef uint32_t buffer_rsrc __attribute__((ext_vector_type(4)));
+// a buffer of `bytes` bytes (held to 32 bits) starting at p (wave-uniform): reads past its end give zero
+__device__ __forceinline__ buffer_rsrc make_buffer_rsrc(const void *p, int64_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint32_t n = bytes < 0 ? 0u : bytes > 0xffffffffll ? 0xffffffffu : (uint32_t)bytes;
+    return buffer_rsrc{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
+}
+// 16 bytes per lane from byte voff + soff of the buffer to LDS byte `lds` (wave-uniform) + 16 * lane.  (The wait states
+// cover a scalar operand that a vector instruction wrote just before, and M0.)
+__device__ __forceinline__ void buffer_load_lds16(buffer_rsrc rsrc, int voff, int soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
+}
+template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+// the barrier alone: LDS operations of this wave may still be in flight
+__device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" : : : "memory"); }

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(TOPK_THREADS) void dsa_topk_rows_kernel(
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int t = row_begin + blockIdx.x;
-    const int seg = find_segment(cu, N, t);
+    const int seg = find_segment_wave(cu, N, t);
     const int s0 = cu[seg];
     // a row never reaches past its ld columns: with a max_seqlen below the longest segment (a caller's mistake) the
     // selection of the long rows is wrong, but nothing outside the score rows is read
