@@ -35,7 +35,7 @@ size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw);
 hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, const uint32_t *bitmap, int ldw,
                                 const int32_t *n, const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K,
                                 float scale, float *partial, float *mass, hipStream_t stream);
-hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const uint32_t *bitmap, int ldw,
+hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split,
                                int causal, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
@@ -301,7 +301,8 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, const int32
                 if (e != hipSuccess) return hip_fail(e, "bitmap launch");
             }
         }
-        e = dsa_launch_tile_fwd(q, k, v, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, split, causal, out, lse, st);
+        const int64_t strides[6] = {(int64_t)Hq * D, D, (int64_t)Hkv * D, D, (int64_t)Hkv * D, D};
+        e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, split, causal, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "tile forward launch");
     }
     if (max_seqlen > split) {

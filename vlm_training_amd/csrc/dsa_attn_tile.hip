@@ -1,5 +1,5 @@
-// Tile kernels: attention forward / dQ / dK,dV over 32x32 MFMA tiles with the selection applied as a
-// bitmap mask.  They do the same arithmetic as the gather kernels but visit every (query block, key
+// Tile kernels: dQ / dK,dV, attention mass and indexer backward over 32x32 MFMA tiles with the selection applied
+// as a bitmap mask (the forward: dsa_tile_fwd.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
 // 4*G*D flop on the matrix cores - on MI355X the tile walk is cheaper down to a few percent density.
@@ -12,204 +12,10 @@
 //   over D) or transposed with ds_read_b64_tr_b16 (contraction over rows/keys) - both conflict-free.
 //   The second GEMM of each chain takes its B operand straight from the C layout of the first
 //   (the contraction order over the 32 keys/rows of a tile is permuted identically on both operands).
-#include "dsa_common.h"
-#include <type_traits>
+#include "dsa_tile.h"
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }   // v_exp_f32; exp2(-inf) = 0
-
-// ---- LDS tile: 32 rows of D bf16 with a pitch of D*2 + 64 bytes (+ 128 at head_dim 96); chunk = 16 bytes ----
-// The LDS of gfx950 has 64 four-byte banks (256 B per clock).  A 16-byte read is served 16 lanes at a
-// time and a transposed 8-byte read 32 lanes at a time, so a row-wise operand read (16 consecutive rows,
-// same chunk) and a transposed read (4 consecutive rows x 64 B) must each cover all banks once.  The
-// 64-byte skew per row separates 4 consecutive rows, the XOR of the chunk's two low bits with row bits
-// 2-3 separates rows 4 apart: both read patterns and the row-wise staging writes are conflict-free.
-// (The skew needs a pitch of 64 modulo 256 bytes: head_dim 96 pads its rows to the pitch of head_dim 128.)
-template <int D> constexpr int tile_pitch() { return D == 96 ? 320 : D * 2 + 64; }
-template <int D> constexpr int tile_bytes() { return 32 * tile_pitch<D>(); }
-__device__ __forceinline__ int tile_sw(int row) { return (row >> 2) & 3; }
-template <int D>
-__device__ __forceinline__ int tile_off(int row, int chunk) { return row * tile_pitch<D>() + ((chunk ^ tile_sw(row)) << 4); }
-
-// accumulate in place (kept as a function so that the accumulation sites read alike)
-__device__ __forceinline__ void mfma32_acc(f32x16 &c, bf16x8 a, bf16x8 b) { c = mfma32(a, b, c); }
-// all-ones if bit `b` of `word` is set, else 0 (v_bfe_i32 when b is a compile-time constant)
-__device__ __forceinline__ uint32_t bit_mask(uint32_t word, int b) {
-    return (uint32_t)(((int32_t)(word << (31 - b))) >> 31);
-}
-// x where keep is all-ones, -inf where it is 0 (one v_bfi_b32 / v_bitop3_b32)
-__device__ __forceinline__ float keep_or_neginf(float x, uint32_t keep) {
-    return __uint_as_float((keep & __float_as_uint(x)) | (~keep & 0xff800000u));
-}
-// bits j <= d of a 32-key tile (keys at or before the diagonal when d = query column - tile start)
-__device__ __forceinline__ uint32_t causal_bits(int d) { return d >= 31 ? 0xffffffffu : (d < 0 ? 0u : ((2u << d) - 1u)); }
-// Issue order for a chain of NM MFMAs that each consume RPM LDS reads: keep AHEAD MFMAs' worth of reads
-// in flight (the machine scheduler otherwise sinks every read next to its use and the chain runs at
-// LDS latency).  Applies to the instructions of the enclosing basic block, in program order.
-template <int NM, int AHEAD, int RPM, int FIRST = 0>
-__device__ __forceinline__ void sched_reads_ahead() {
-    __builtin_amdgcn_sched_group_barrier(0x100, FIRST + AHEAD * RPM, 0);   // FIRST: other reads issued up front
-#pragma unroll
-    for (int i = 0; i < NM - AHEAD; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
-}
-// Per-lane LDS byte offsets of the two read patterns, computed once per kernel so that every operand
-// read in the loops is "tile base + lane offset + immediate" (the swizzle only XORs chunk bits 0-1, so
-// k-step / d-tile indices move the address by a lane constant plus a compile-time multiple of 64 B).
-//   row-wise A operand of mfma32: lane (i = row j, h) takes elements [16*ks + 8h, +8) of row j
-//   transposed A operand: lane l takes column c = 32*dt + (l & 31)... of the 8 rows {R..R+3, R+8..R+11}.
-//   ds_read_b64_tr_b16: within 16 lanes, lane s supplies the address of 4 consecutive elements of row
-//   R + s/4 at column m0 + 4*(s%4); lane s receives rows R..R+3 of column m0 + s.
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
-template <int D>
-struct LaneOffsets {
-    int row[2];      // row-wise operand of row j: k-steps ks with ks % 2 == c
-    int tr[4];       // transposed operand: rows 4h + s/4 + {0, 8, 16, 24}
-    __device__ __forceinline__ void init(int lane) {
-        const int h = lane >> 5, j = lane & 31, s = lane & 15;
-        const int swj = tile_sw(j);
-#pragma unroll
-        for (int c = 0; c < 2; ++c) row[c] = j * tile_pitch<D>() + ((((c ^ (swj >> 1)) << 1) | (h ^ (swj & 1))) << 4);
-        const int low = ((lane >> 4) & 1) * 2 + ((s & 3) >> 1), sub = (s & 1) << 3;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = 4 * h + (s >> 2) + 8 * v;
-            tr[v] = r * tile_pitch<D>() + ((low ^ tile_sw(r)) << 4) + sub;
-        }
-    }
-    // row-wise A operand of k-step ks (elements [16ks + 8h, +8) of row j)
-    __device__ __forceinline__ bf16x8 rowop(const unsigned char *tile, int ks) const {
-        return *reinterpret_cast<const bf16x8 *>(tile + row[ks & 1] + (ks >> 1) * 64);
-    }
-    __device__ __forceinline__ static bf16x8 tr_pair(lds_u8 *p0, lds_u8 *p1) {
-        const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p0);
-        const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p1);
-        typedef short s16x8 __attribute__((ext_vector_type(8)));
-        const s16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-        return __builtin_bit_cast(bf16x8, r);
-    }
-    // transposed A operand of d-tile dt over rows {R..R+3, R+8..R+11}, R = 4h (pair 0) or 16 + 4h (pair 1)
-    __device__ __forceinline__ bf16x8 trop(const unsigned char *tile, int pair, int dt) const {
-        return tr_pair((lds_u8 *)tile + tr[2 * pair] + dt * 64, (lds_u8 *)tile + tr[2 * pair + 1] + dt * 64);
-    }
-    // same with the lane addresses already formed (p[v] = tile + tr[v]): one immediate per read
-    __device__ __forceinline__ static bf16x8 trop_at(lds_u8 *const *p, int pair, int dt, int imm) {
-        return tr_pair(p[2 * pair] + dt * 64 + imm, p[2 * pair + 1] + dt * 64 + imm);
-    }
-};
-__device__ __forceinline__ bf16x8 pack8(const float *x) {
-    const u32x4 w = {pack2bf(x[0], x[1]), pack2bf(x[2], x[3]), pack2bf(x[4], x[5]), pack2bf(x[6], x[7])};
-    return __builtin_bit_cast(bf16x8, w);
-}
-__device__ __forceinline__ f32x16 zero16() {
-    f32x16 z;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) z[v] = 0.f;
-    return z;
-}
-
-// Write one 32-column d-tile of a C-layout accumulator as bf16 (lane = row j; a lane holds the four
-// columns 8*g4 + 4*h + {0..3} of every group g4, so a 16-byte chunk of the row is split over the two
-// lanes 32 apart).  The halves of the wave exchange 8-byte pieces - lane (j,0) takes chunk 2m whole,
-// lane (j,1) chunk 2m+1 - and every lane stores 16 bytes.  Both lanes of a row must be active.
-__device__ __forceinline__ void store_c_tile(bf16_t *row_dt, const f32x16 &acc, float mul, int h) {
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const uint32_t a0 = pack2bf(acc[8 * m] * mul, acc[8 * m + 1] * mul), a1 = pack2bf(acc[8 * m + 2] * mul, acc[8 * m + 3] * mul);
-        const uint32_t b0 = pack2bf(acc[8 * m + 4] * mul, acc[8 * m + 5] * mul), b1 = pack2bf(acc[8 * m + 6] * mul, acc[8 * m + 7] * mul);
-        const auto r0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);   // upper lanes of a <-> lower lanes of b
-        const auto r1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-        const u32x4 w = {r0[0], r1[0], r0[1], r1[1]};
-        *reinterpret_cast<u32x4 *>(row_dt + 8 * (2 * m + h)) = w;
-    }
-}
-
-// slot -> (segment, block) for blocks of `blk` columns handed out segment by segment; within a segment
-// the blocks are numbered from the end when `reverse` (heaviest causal blocks first).  Returns false
-// for spare slots.  The segment bounds are fetched 64 segments at a time, one per lane (one memory
-// round trip instead of one per segment), and walked with lane reads.
-__device__ __forceinline__ bool locate_block(const int32_t *cu, int N, int slot, int blk, bool reverse, int &s0, int &L,
-                                             int &b) {
-    const int lane = threadIdx.x & 63;
-    for (int base = 0; base < N; base += 64) {
-        const int seg = min(base + lane, N - 1);
-        const int lo = cu[seg], len = cu[seg + 1] - lo;
-        const int cnt = min(64, N - base);
-        for (int w = 0; w < cnt; ++w) {
-            L = __builtin_amdgcn_readlane(len, w);
-            const int nb = (L + blk - 1) / blk;
-            if (slot < nb) {
-                s0 = __builtin_amdgcn_readlane(lo, w);
-                b = reverse ? nb - 1 - slot : slot;
-                return true;
-            }
-            slot -= nb;
-        }
-    }
-    return false;
-}
-
-// The same hand-out, heaviest block first over the whole batch: slot 0 takes the last block of the longest segment,
-// then every block with the next lower index in segment order, and so on - a block's walk grows with its index, so
-// long walks start first wherever their segment lies in the batch (with the segment-by-segment order the long
-// walks of a late segment start late and the launch ends on them).  For up to 64 segments (their lengths live in
-// one wave's lanes); larger batches fall back to the segment-by-segment order.
-__device__ __forceinline__ int wave_sum_i(int x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-    return x;
-}
-__device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, int N, int slot, int blk, int &s0, int &L,
-                                                            int &b) {
-    if (N > 64) return locate_block(cu, N, slot, blk, true, s0, L, b);
-    const int lane = threadIdx.x & 63;
-    const int seg = min(lane, N - 1);
-    const int lo = cu[seg], len = cu[seg + 1] - lo;
-    const int nb = lane < N ? (len + blk - 1) / blk : 0;
-    int most = nb;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
-    // blocks with index >= x over all segments
-    auto count_ge = [&](int x) { return wave_sum_i(max(nb - x, 0)); };
-    if (slot >= count_ge(0)) return false;
-    int lo_b = 0, hi_b = most;                           // count_ge(lo_b) > slot >= count_ge(hi_b)
-    while (hi_b - lo_b > 1) {
-        const int mid = (lo_b + hi_b) >> 1;
-        if (count_ge(mid) > slot) lo_b = mid; else hi_b = mid;
-    }
-    b = lo_b;
-    const int rank = slot - count_ge(b + 1);             // among the segments that have a block b, in segment order
-    const uint64_t has = __builtin_amdgcn_ballot_w64(nb > b);
-    // the rank-th set bit of `has`
-    const int below = (int)__popcll(has & ((1ull << lane) - 1ull));
-    const uint64_t me = __builtin_amdgcn_ballot_w64(nb > b && below == rank);
-    const int w = (int)__builtin_ctzll(me);
-    s0 = __builtin_amdgcn_readlane(lo, w);
-    L = __builtin_amdgcn_readlane(len, w);
-    return true;
-}
-
-// Query blocks are handed out heaviest first: over the whole batch for launches of a few rounds of workgroups (they
-// would otherwise end on the long walks of a late segment: forward -11 %, dQ -15 % on 8192 tokens in seven
-// segments), segment by segment for larger ones, where the blocks of a segment that run side by side share their
-// K / V tiles in L2 (the batch-wide order is 2-3 % slower there).
-#define DSA_BATCH_ORDER_MAX_BLOCKS (6 * 256)
-#define LOCATE_QUERY_BLOCK(cu, N, slot, blk, s0, L, b)                                                           \
-    (gridDim.x <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
-                                             : locate_block(cu, N, slot, blk, true, s0, L, b))
-
-// ==================================================================================================
-// forward: query-stationary.  Workgroup = 4 waves x 32 rows = 128 rows = 128/Gp queries of one
-// segment and one kv head; loops over 32-key tiles of the causal range.
-//   S^T[key,row] = K[key,:].Q[row,:]   (A = K tile row-wise from LDS, B = Q^T in registers)
-//   online softmax on the C layout (lane = row; one cross-lane step per statistic)
-//   O^T[d,row]  += V^T[d,key] P^T[key,row]   (A = V tile transposed from LDS, B = P^T from the C layout)
-// K/V tiles are fetched two tiles ahead into registers and one tile ahead into LDS (double buffer),
-// so a global load has two tile-times to land; one barrier per tile.
-// ==================================================================================================
+// K/V tiles of the query-stationary kernels are fetched two tiles ahead into registers and one tile ahead into LDS (double
+// buffer), so a global load has two tile-times to land; one barrier per tile.
 // Every global load of the pipeline is issued unconditionally (indices past the end are clamped to
 // the last tile) and nothing is computed from a loaded value before the matching STORE, so the
 // compiler can wait with exact vmcnt counts and a load has two tile-times to land.  The kernel issues
@@ -237,139 +43,6 @@ __device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, i
         }                                                                                          \
         if (it < (NT)) COMPUTE(it, 0);                                                             \
     }
-
-template <int D, bool HAS_IDX, int GSHIFT, int NW>
-__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
-    const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v,
-    const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale_log2, int pos_split, int causal, bf16_t *__restrict__ out, float *__restrict__ lse) {
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NBUF = (D > 128) ? 1 : 2;           // double buffering where 64 KiB of static LDS allow it
-    constexpr int NT = NW * 64, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT;
-    constexpr int CH = 32 * CPR, LOADS = (CH + NT - 1) / NT;   // 16-byte chunks per matrix; per thread (head_dim 96: not all threads)
-    static_assert(CH % 64 == 0, "whole waves stage or do not");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][2][TILE_B];   // [buffer][K|V]
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    const int G = Hq / Hkv;
-    const int kvh = blockIdx.x % Hkv;
-    int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
-    if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
-    const int qc0 = blk * QBW;
-    if (qc0 >= pos_split || qc0 >= L) return;                       // rows past the split belong to the gather kernel
-
-    const int r = wv * 32 + j;
-    const int qcol = qc0 + (r >> GSHIFT), head = r & (Gp - 1);
-    const bool row_ok = qcol < L && head < G;
-    const int t = s0 + min(qcol, L - 1), hq = kvh * G + min(head, G - 1);
-    u32x4 kst[2][LOADS], vst[2][LOADS];
-#define FWD_LOAD(SET, TILE)                                                                         \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) if (CH % NT == 0 || i * NT + tid < CH) {     \
-        const int c = i * NT + tid;                                                               \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        const int64_t off = ((int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * Hkv + kvh) * D + ch * 8; \
-        kst[SET][i] = *reinterpret_cast<const u32x4 *>(k + off);                                   \
-        vst[SET][i] = *reinterpret_cast<const u32x4 *>(v + off);                                   \
-    }
-    FWD_LOAD(0, 0)                                      // ahead of the q rows: staging waits for this tile only
-    bf16x8 qB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-        qB[ks] = row_ok ? load_bf16x8(q + ((int64_t)t * Hq + hq) * D + 16 * ks + 8 * h) : zero_bf16x8();
-    const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
-    const int klim = causal ? qcol : L - 1;             // last key column this row may attend (dense mode)
-    const uint32_t *wrow = bitmap + (int64_t)t * ldw;
-
-    f32x16 oacc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) oacc[dt] = zero16();
-    float mrun = -INFINITY, lsum = 0.f;
-    uint32_t word_next = HAS_IDX ? wrow[0] : 0u;        // unconditional loads; rows that are not live are masked at use
-
-#define FWD_STORE(SET, BUF, TILE)                                                                        \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) if (CH % NT == 0 || i * NT + tid < CH) {     \
-        const int c = i * NT + tid;                                                               \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        *reinterpret_cast<u32x4 *>(&lds[BUF][0][tile_off<D>(row, ch)]) = kst[SET][i];              \
-        *reinterpret_cast<u32x4 *>(&lds[BUF][1][tile_off<D>(row, ch)]) = vst[SET][i];              \
-    }
-// Online softmax of one tile.  The row maximum is not searched in every tile: P is formed against the running
-// reference first, and only when a lane's sum says that some probability may have passed 2^8 - or a live row has not met
-// a selected key yet - does the wave look for the tile's maximum, move the reference, rescale the sums and form P
-// again: the first tile of a block, then rarely.  In between P stays below 2^8, exact in fp32 and safe in bf16, and
-// never underflows as a whole, because the reference is a maximum the row has really met.  (Searching the maximum in
-// every tile, 16 more vector instructions per tile, was 4-5 % slower at 32 768 tokens.)
-#define FWD_SOFTMAX                                                                                \
-        float s2[16], pr[16];                                                                      \
-        _Pragma("unroll") for (int vi = 0; vi < 16; ++vi)                                          \
-            s2[vi] = keep_or_neginf(sacc[vi], bit_mask(word, 8 * (vi >> 2) + (vi & 3)));           \
-        float psum = 0.f;                                                                          \
-        {                                                                                          \
-            const float mneg = (mrun == -INFINITY) ? 0.f : -mrun;                                  \
-            _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) {                                    \
-                pr[vi] = fast_exp2(fmaf(s2[vi], scale_log2, mneg));                                \
-                psum += pr[vi];                                                                    \
-            }                                                                                      \
-        }                                                                                          \
-        if (__builtin_amdgcn_ballot_w64(row_ok && (mrun == -INFINITY || !(psum <= 256.f)))) {      \
-            float mloc = -INFINITY;                                                                \
-            _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) mloc = fmaxf(mloc, s2[vi]);          \
-            mloc = half_max_f(mloc) * scale_log2;                                                  \
-            if (mloc > mrun) {                                                                     \
-                const float alpha = fast_exp2(mrun - mloc);   /* mrun = -inf: 0, and the sums are 0 */ \
-                lsum *= alpha;                                                                     \
-                _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;               \
-                mrun = mloc;                                                                       \
-            }                                                                                      \
-            const float mneg = (mrun == -INFINITY) ? 0.f : -mrun;                                  \
-            psum = 0.f;                                                                            \
-            _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) {                                    \
-                pr[vi] = fast_exp2(fmaf(s2[vi], scale_log2, mneg));                                \
-                psum += pr[vi];                                                                    \
-            }                                                                                      \
-        }                                                                                          \
-        lsum += psum;                                                                              \
-        const bf16x8 pB0 = pack8(pr), pB1 = pack8(pr + 8);
-#define FWD_COMPUTE(TILE, BUF)                                                                      \
-    {                                                                                              \
-        const int kc0 = (TILE) * 32;                                                               \
-        const unsigned char *kt = lds[BUF][0], *vt = lds[BUF][1];                                  \
-        uint32_t word = row_ok ? word_next : 0u;                                                   \
-        if (HAS_IDX) word_next = wrow[min((TILE) + 1, ntiles - 1)];                                \
-        if (!HAS_IDX) word = row_ok ? causal_bits(klim - kc0) : 0u;                                \
-        word >>= 4 * h;                                  /* element vi then sits at bit 8*(vi/4) + vi%4 */ \
-        f32x16 sacc = zero16();                                                                    \
-        {                                                /* all K operands in flight before the first MFMA */ \
-            bf16x8 ka[KS];                                                                         \
-            _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) ka[ks] = lo.rowop(kt, ks); \
-            _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) sacc = mfma32(ka[ks], qB[ks], sacc); \
-            sched_reads_ahead<KS, 4, 1>();                                                         \
-        }                                                                                          \
-        FWD_SOFTMAX                                                                                \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) {                                        \
-            mfma32_acc(oacc[dt], lo.trop(vt, 0, dt), pB0);                          \
-            mfma32_acc(oacc[dt], lo.trop(vt, 1, dt), pB1);                     \
-        }                                                                                          \
-        sched_reads_ahead<2 * DT, 3, 2>();                                                         \
-    }
-    TILE_PIPELINE(ntiles, FWD_LOAD, FWD_STORE, FWD_COMPUTE)
-#undef FWD_LOAD
-#undef FWD_STORE
-#undef FWD_COMPUTE
-#undef FWD_SOFTMAX
-
-    float l = half_sum_f(lsum);
-    if (row_ok) {
-        const float inv = 1.f / l;
-        bf16_t *op = out + ((int64_t)t * Hq + hq) * D;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, oacc[dt], inv, h);
-        if (h == 0) lse[(int64_t)hq * T + t] = (mrun + log2f(l)) * LN2_F;
-    }
-}
 
 // ==================================================================================================
 // attention mass: the indexer's training target.  Same walk and S^T = K Q^T as the forward, with the
@@ -2139,28 +1812,6 @@ static inline int group_shift(int Hq, int Hkv) {
 template <int D> constexpr int tile_waves() { return (D == 128 || D == 96) ? DSA_TILE_WAVES_128 : 4; }
 static inline int tile_waves_of(int D) { return (D == 128 || D == 96) ? DSA_TILE_WAVES_128 : 4; }
 template <int D, bool HAS_IDX, int GS>
-static hipError_t launch_fwd_i(dim3 grid, hipStream_t stream, const void *q, const void *k, const void *v,
-                         const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float sl2,
-                         int pos_split, int causal, void *out, float *lse) {
-    constexpr int NW = tile_waves<D>();
-    if constexpr (NW == 8) {
-        // A launch of a few rounds of workgroups is bound by what a workgroup pays before its first tile and after
-        // its last (memory round trips, row stores), and with eight waves only one workgroup fits a CU.  Such
-        // launches run the four-wave form, two workgroups per CU, whose fixed parts overlap (forward -9 % on 8192
-        // tokens in seven segments; the dQ kernel measured 19 % slower that way and keeps eight waves).
-        if (grid.x <= DSA_BATCH_ORDER_MAX_BLOCKS) {
-            const int Gp = 1 << GS;
-            const dim3 grid4((unsigned)(((int64_t)T / ((32 * 4) / Gp) + N + 1) * Hkv));
-            hipLaunchKernelGGL((dsa_tile_fwd_kernel<D, HAS_IDX, GS, 4>), grid4, dim3(256), 0, stream, (const bf16_t *)q,
-                               (const bf16_t *)k, (const bf16_t *)v, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, pos_split, causal, (bf16_t *)out, lse);
-            return hipSuccess;
-        }
-    }
-    hipLaunchKernelGGL((dsa_tile_fwd_kernel<D, HAS_IDX, GS, NW>), grid, dim3(64 * NW), 0, stream, (const bf16_t *)q,
-                       (const bf16_t *)k, (const bf16_t *)v, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, pos_split, causal, (bf16_t *)out, lse);
-    return hipSuccess;
-}
-template <int D, bool HAS_IDX, int GS>
 static hipError_t launch_dq_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                         const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
                         int T, int Hq, int Hkv, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
@@ -2227,14 +1878,6 @@ static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, 
     }                                                                                     \
     if (launch_status != hipSuccess) return launch_status;
 
-extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const uint32_t *bitmap, int ldw,
-                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale,
-                                          int pos_split, int causal, void *out, float *lse, hipStream_t stream) {
-    const int gs = group_shift(Hq, Hkv);
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * tile_waves_of(D)) >> gs) + N + 1) * Hkv));
-    TILE_SWITCH_96(launch_fwd_i, grid, stream, q, k, v, bitmap, ldw, cu, N, T, Hq, Hkv, scale * LOG2E_F, pos_split, causal, out, lse)
-    return hipGetLastError();
-}
 // kv heads a workgroup of the attention-mass kernel takes (a power of two, at most what its registers hold; with
 // one query head per kv head a lane also holds all sixteen sums of a tile to itself, which costs the top size)
 template <int D>

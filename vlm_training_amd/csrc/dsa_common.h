@@ -113,6 +113,11 @@ __device__ __forceinline__ void buffer_load_lds16(buffer_rsrc rsrc, int voff, in
     asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
 }
+// the same with 4 bytes per lane, to LDS byte `lds` + 4 * lane
+__device__ __forceinline__ void buffer_load_lds4(buffer_rsrc rsrc, int voff, int soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dword %0, %1, %2 offen lds"
+                 : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
+}
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 // the barrier alone: LDS operations of this wave may still be in flight
 __device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" : : : "memory"); }

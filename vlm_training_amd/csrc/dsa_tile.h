@@ -1,0 +1,243 @@
+// Helpers shared by the tile kernels (32x32 MFMA tiles over packed segments): LDS tiles, masks, the hand-out of blocks.
+#pragma once
+#include "dsa_common.h"
+#include <type_traits>
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }   // v_exp_f32; exp2(-inf) = 0
+
+// ---- LDS tile: 32 rows of D bf16 with a pitch of D*2 + 64 bytes (+ 128 at head_dim 96); chunk = 16 bytes ----
+// The LDS of gfx950 has 64 four-byte banks (256 B per clock).  A 16-byte read is served 16 lanes at a
+// time and a transposed 8-byte read 32 lanes at a time, so a row-wise operand read (16 consecutive rows,
+// same chunk) and a transposed read (4 consecutive rows x 64 B) must each cover all banks once.  The
+// 64-byte skew per row separates 4 consecutive rows, the XOR of the chunk's two low bits with row bits
+// 2-3 separates rows 4 apart: both read patterns and the row-wise staging writes are conflict-free.
+// (The skew needs a pitch of 64 modulo 256 bytes: head_dim 96 pads its rows to the pitch of head_dim 128.)
+template <int D> constexpr int tile_pitch() { return D == 96 ? 320 : D * 2 + 64; }
+template <int D> constexpr int tile_bytes() { return 32 * tile_pitch<D>(); }
+__device__ __forceinline__ int tile_sw(int row) { return (row >> 2) & 3; }
+template <int D>
+__device__ __forceinline__ int tile_off(int row, int chunk) { return row * tile_pitch<D>() + ((chunk ^ tile_sw(row)) << 4); }
+
+// accumulate in place (kept as a function so that the accumulation sites read alike)
+__device__ __forceinline__ void mfma32_acc(f32x16 &c, bf16x8 a, bf16x8 b) { c = mfma32(a, b, c); }
+// all-ones if bit `b` of `word` is set, else 0 (v_bfe_i32 when b is a compile-time constant)
+__device__ __forceinline__ uint32_t bit_mask(uint32_t word, int b) {
+    return (uint32_t)(((int32_t)(word << (31 - b))) >> 31);
+}
+// x where keep is all-ones, -inf where it is 0 (one v_bfi_b32 / v_bitop3_b32)
+__device__ __forceinline__ float keep_or_neginf(float x, uint32_t keep) {
+    return __uint_as_float((keep & __float_as_uint(x)) | (~keep & 0xff800000u));
+}
+// bits j <= d of a 32-key tile (keys at or before the diagonal when d = query column - tile start)
+__device__ __forceinline__ uint32_t causal_bits(int d) { return d >= 31 ? 0xffffffffu : (d < 0 ? 0u : ((2u << d) - 1u)); }
+// Issue order for a chain of NM MFMAs that each consume RPM LDS reads: keep AHEAD MFMAs' worth of reads
+// in flight (the machine scheduler otherwise sinks every read next to its use and the chain runs at
+// LDS latency).  Applies to the instructions of the enclosing basic block, in program order.
+template <int NM, int AHEAD, int RPM, int FIRST = 0>
+__device__ __forceinline__ void sched_reads_ahead() {
+    __builtin_amdgcn_sched_group_barrier(0x100, FIRST + AHEAD * RPM, 0);   // FIRST: other reads issued up front
+#pragma unroll
+    for (int i = 0; i < NM - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+}
+// Per-lane LDS byte offsets of the two read patterns, computed once per kernel so that every operand
+// read in the loops is "tile base + lane offset + immediate" (the swizzle only XORs chunk bits 0-1, so
+// k-step / d-tile indices move the address by a lane constant plus a compile-time multiple of 64 B).
+//   row-wise A operand of mfma32: lane (i = row j, h) takes elements [16*ks + 8h, +8) of row j
+//   transposed A operand: lane l takes column c = 32*dt + (l & 31)... of the 8 rows {R..R+3, R+8..R+11}.
+//   ds_read_b64_tr_b16: within 16 lanes, lane s supplies the address of 4 consecutive elements of row
+//   R + s/4 at column m0 + 4*(s%4); lane s receives rows R..R+3 of column m0 + s.
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+template <int D>
+struct LaneOffsets {
+    int row[2];      // row-wise operand of row j: k-steps ks with ks % 2 == c
+    int tr[4];       // transposed operand: rows 4h + s/4 + {0, 8, 16, 24}
+    __device__ __forceinline__ void init(int lane) {
+        const int h = lane >> 5, j = lane & 31, s = lane & 15;
+        const int swj = tile_sw(j);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) row[c] = j * tile_pitch<D>() + ((((c ^ (swj >> 1)) << 1) | (h ^ (swj & 1))) << 4);
+        const int low = ((lane >> 4) & 1) * 2 + ((s & 3) >> 1), sub = (s & 1) << 3;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 4 * h + (s >> 2) + 8 * v;
+            tr[v] = r * tile_pitch<D>() + ((low ^ tile_sw(r)) << 4) + sub;
+        }
+    }
+    // row-wise A operand of k-step ks (elements [16ks + 8h, +8) of row j)
+    __device__ __forceinline__ bf16x8 rowop(const unsigned char *tile, int ks) const {
+        return *reinterpret_cast<const bf16x8 *>(tile + row[ks & 1] + (ks >> 1) * 64);
+    }
+    __device__ __forceinline__ static bf16x8 tr_pair(lds_u8 *p0, lds_u8 *p1) {
+        const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p0);
+        const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p1);
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        const s16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        return __builtin_bit_cast(bf16x8, r);
+    }
+    // transposed A operand of d-tile dt over rows {R..R+3, R+8..R+11}, R = 4h (pair 0) or 16 + 4h (pair 1)
+    __device__ __forceinline__ bf16x8 trop(const unsigned char *tile, int pair, int dt) const {
+        return tr_pair((lds_u8 *)tile + tr[2 * pair] + dt * 64, (lds_u8 *)tile + tr[2 * pair + 1] + dt * 64);
+    }
+    // same with the lane addresses already formed (p[v] = tile + tr[v]): one immediate per read
+    __device__ __forceinline__ static bf16x8 trop_at(lds_u8 *const *p, int pair, int dt, int imm) {
+        return tr_pair(p[2 * pair] + dt * 64 + imm, p[2 * pair + 1] + dt * 64 + imm);
+    }
+};
+__device__ __forceinline__ bf16x8 pack8(const float *x) {
+    const u32x4 w = {pack2bf(x[0], x[1]), pack2bf(x[2], x[3]), pack2bf(x[4], x[5]), pack2bf(x[6], x[7])};
+    return __builtin_bit_cast(bf16x8, w);
+}
+__device__ __forceinline__ f32x16 zero16() {
+    f32x16 z;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) z[v] = 0.f;
+    return z;
+}
+
+// Write one 32-column d-tile of a C-layout accumulator as bf16 (lane = row j; a lane holds the four
+// columns 8*g4 + 4*h + {0..3} of every group g4, so a 16-byte chunk of the row is split over the two
+// lanes 32 apart).  The halves of the wave exchange 8-byte pieces - lane (j,0) takes chunk 2m whole,
+// lane (j,1) chunk 2m+1 - and every lane stores 16 bytes.  Both lanes of a row must be active.
+// `chunks`: 16-byte chunks of the row that exist from this d-tile on (4 and more: all of it).
+__device__ __forceinline__ void store_c_tile(bf16_t *row_dt, const f32x16 &acc, float mul, int h, int chunks = 4) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const uint32_t a0 = pack2bf(acc[8 * m] * mul, acc[8 * m + 1] * mul), a1 = pack2bf(acc[8 * m + 2] * mul, acc[8 * m + 3] * mul);
+        const uint32_t b0 = pack2bf(acc[8 * m + 4] * mul, acc[8 * m + 5] * mul), b1 = pack2bf(acc[8 * m + 6] * mul, acc[8 * m + 7] * mul);
+        const auto r0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);   // upper lanes of a <-> lower lanes of b
+        const auto r1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+        const u32x4 w = {r0[0], r1[0], r0[1], r1[1]};
+        if (2 * m + h < chunks) *reinterpret_cast<u32x4 *>(row_dt + 8 * (2 * m + h)) = w;
+    }
+}
+
+// slot -> (segment, block) for blocks of `blk` columns handed out segment by segment; within a segment
+// the blocks are numbered from the end when `reverse` (heaviest causal blocks first).  Returns false
+// for spare slots.  The segment bounds are fetched 64 segments at a time, one per lane (one memory
+// round trip instead of one per segment), and walked with lane reads.
+__device__ __forceinline__ bool locate_block(const int32_t *cu, int N, int slot, int blk, bool reverse, int &s0, int &L,
+                                             int &b) {
+    const int lane = threadIdx.x & 63;
+    for (int base = 0; base < N; base += 64) {
+        const int seg = min(base + lane, N - 1);
+        const int lo = cu[seg], len = cu[seg + 1] - lo;
+        const int cnt = min(64, N - base);
+        for (int w = 0; w < cnt; ++w) {
+            L = __builtin_amdgcn_readlane(len, w);
+            const int nb = (L + blk - 1) / blk;
+            if (slot < nb) {
+                s0 = __builtin_amdgcn_readlane(lo, w);
+                b = reverse ? nb - 1 - slot : slot;
+                return true;
+            }
+            slot -= nb;
+        }
+    }
+    return false;
+}
+
+// The same hand-out, heaviest block first over the whole batch: slot 0 takes the last block of the longest segment,
+// then every block with the next lower index in segment order, and so on - a block's walk grows with its index, so
+// long walks start first wherever their segment lies in the batch (with the segment-by-segment order the long
+// walks of a late segment start late and the launch ends on them).  For up to 64 segments (their lengths live in
+// one wave's lanes); larger batches fall back to the segment-by-segment order.
+// Sum / maximum (of values >= 0) over the wave, wave-uniform: DPP steps inside the rows of sixteen lanes, then across them -
+// no LDS round trips (the search below takes about ten of these sums in front of a workgroup's first load; by lane
+// shuffles they cost it 2 us).
+template <class F>
+__device__ __forceinline__ int wave_fold_i(int x, F f) {
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));      // row_shr:1
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));      // row_shr:2
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));      // row_shr:4
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));      // row_shr:8: lane 15 of a row has the row
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));      // row_bcast:15 into rows 1 and 3
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));      // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(x, 63);
+}
+__device__ __forceinline__ int wave_sum_i(int x) { return wave_fold_i(x, [](int a, int b) { return a + b; }); }
+__device__ __forceinline__ int wave_max_i(int x) { return wave_fold_i(x, [](int a, int b) { return max(a, b); }); }
+__device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, int N, int slot, int blk, int &s0, int &L,
+                                                            int &b) {
+    if (N > 64) return locate_block(cu, N, slot, blk, true, s0, L, b);
+    const int lane = threadIdx.x & 63;
+    const int seg = min(lane, N - 1);
+    const int lo = cu[seg], len = cu[seg + 1] - lo;
+    const int nb = lane < N ? (len + blk - 1) / blk : 0;
+    const int most = wave_max_i(nb);
+    // blocks with index >= x over all segments
+    auto count_ge = [&](int x) { return wave_sum_i(max(nb - x, 0)); };
+    if (slot >= count_ge(0)) return false;
+    int lo_b = 0, hi_b = most;                           // count_ge(lo_b) > slot >= count_ge(hi_b)
+    while (hi_b - lo_b > 1) {
+        const int mid = (lo_b + hi_b) >> 1;
+        if (count_ge(mid) > slot) lo_b = mid; else hi_b = mid;
+    }
+    b = lo_b;
+    const int rank = slot - count_ge(b + 1);             // among the segments that have a block b, in segment order
+    const uint64_t has = __builtin_amdgcn_ballot_w64(nb > b);
+    // the rank-th set bit of `has`
+    const int below = (int)__popcll(has & ((1ull << lane) - 1ull));
+    const uint64_t me = __builtin_amdgcn_ballot_w64(nb > b && below == rank);
+    const int w = (int)__builtin_ctzll(me);
+    s0 = __builtin_amdgcn_readlane(lo, w);
+    L = __builtin_amdgcn_readlane(len, w);
+    return true;
+}
+
+// Query blocks are handed out heaviest first: over the whole batch for launches of a few rounds of workgroups (they
+// would otherwise end on the long walks of a late segment: forward -11 %, dQ -15 % on 8192 tokens in seven
+// segments), segment by segment for larger ones, where the blocks of a segment that run side by side share their
+// K / V tiles in L2 (the batch-wide order is 2-3 % slower there).
+#define DSA_BATCH_ORDER_MAX_BLOCKS (6 * 256)
+#define LOCATE_QUERY_BLOCK(cu, N, slot, blk, s0, L, b)                                                           \
+    (gridDim.x <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
+                                             : locate_block(cu, N, slot, blk, true, s0, L, b))
+
+// ---- LDS tiles filled straight from memory ------------------------------------------------------------------------------
+// 32 rows of D bf16 (head_dim 96: of 128, the last quarter zero).  A load puts 1 KiB of one wave at consecutive addresses, so
+// rows cannot be padded one by one; instead groups of rows (1 KiB at head_dim 64, four rows else) are 16 bytes apart, and the
+// 16-byte chunk c of row r sits at position c ^ x(r), x = 4 (r & 3) (head_dim 64: 4 (bit 1 of r) + 2 (bit 2)): sixteen
+// consecutive rows at one chunk (row-wise operand) and four consecutive rows at four neighbouring chunks (transposed operand,
+// 32 lanes) each cover the 64 banks once.  The XOR is applied to the source address of a load.
+template <int D>
+struct DirectTile {
+    static constexpr int ROW_B = D == 96 ? 256 : 2 * D;                  // bytes per row
+    static constexpr int CPR = ROW_B / 16;                               // chunks per row
+    static constexpr int GROUP = D == 64 ? 8 : 4;                        // rows between two gaps
+    static constexpr int GROUP_B = GROUP * ROW_B + 16;
+    static constexpr int BYTES = 32 / GROUP * GROUP_B;
+    static constexpr int LOADS = 32 * ROW_B / 1024;                      // wave loads of a tile
+    static constexpr int LOAD_ROWS = 1024 / ROW_B;                       // rows of one of them (1 at most for head_dim 512)
+    static constexpr int SOURCES = D == 256 ? 2 : 1;                     // pieces after which x repeats (from an even piece on)
+    __device__ __forceinline__ static int load_lds(int p) {              // LDS offset of wave load p
+        return p * LOAD_ROWS / GROUP * GROUP_B + p * LOAD_ROWS % GROUP * ROW_B;
+    }
+    __device__ __forceinline__ static int xor_of(int row) { return D == 64 ? ((row >> 1) & 1) * 4 + ((row >> 2) & 1) * 2 : (row & 3) << 2; }
+    // byte offset, from the first row of the tile, that `lane` reads in wave load p; chunks at and past `chunks` read as zero
+    __device__ __forceinline__ static int source(int p, int lane, int row_stride_b, int chunks) {
+        const int row = p * LOAD_ROWS + lane / CPR, c = (lane % CPR) ^ xor_of(row);
+        return c < chunks ? row * row_stride_b + c * 16 : (int)0x80000000;
+    }
+    int rowq[4], trq[4];
+    __device__ __forceinline__ void init(int lane) {
+        const int h = lane >> 5, j = lane & 31, s = lane & 15, i = s >> 2;
+        const int low = ((lane >> 4) & 1) * 2 + ((s & 3) >> 1), sub = (s & 1) << 3;
+        const int rb = j / GROUP * GROUP_B + j % GROUP * ROW_B;
+        const int tr_row = 4 * h + i, tb = tr_row / GROUP * GROUP_B + tr_row % GROUP * ROW_B;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            rowq[q] = D == 64 ? rb + (((2 * q + h) ^ xor_of(j)) << 4) : rb + ((q ^ (j & 3)) << 6) + h * 16;
+            trq[q] = D == 64 ? tb + (((4 * (q & 1) + low) ^ xor_of(tr_row)) << 4) + sub : tb + ((q ^ i) << 6) + low * 16 + sub;
+        }
+    }
+    // k-step ks of a row-wise operand: which of rowq, and what to add
+    static constexpr int row_q(int ks) { return D == 64 ? ks : (ks >> 1) & 3; }
+    static constexpr int row_imm(int ks) { return D == 64 ? 0 : (ks >> 3) * 256 + (ks & 1) * 32; }
+    static constexpr int tr_q(int dt) { return dt & 3; }
+    static constexpr int tr_imm(int dt, int v) { return (D == 64 ? 0 : (dt >> 2) * 256) + v * (8 / GROUP) * GROUP_B; }
+};

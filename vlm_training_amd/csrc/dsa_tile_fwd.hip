@@ -1,0 +1,398 @@
+// Attention forward over 32x32 MFMA tiles, query-stationary, selection (or the causal limit) as a bit mask.
+//
+// A workgroup holds 32*NW rows - a row is one (query, head of the kv group) - of one segment and kv head and walks the keys in
+// tiles of 32:
+//   S^T[key,row] = K[key,:].Q[row,:]            (A = K tile row-wise from LDS, B = Q^T in registers)
+//   online softmax on the C layout (lane = row; one cross-lane step per statistic)
+//   O^T[d,row]  += V^T[d,key] P^T[key,row]      (A = V tile transposed from LDS, B = P^T from the C layout)
+//
+// Each wave runs three tiles at once: step t issues the MFMAs of O += P(t) V(t) and of S(t+2) in pairs, and the softmax of
+// tile t+1 stands between the pairs, a fixed number of elements behind each (every pair ends in an empty asm statement its
+// results pass through, which fixes that order).  So the vector work of a tile - as long as its matrix work - runs in the
+// MFMAs' shadow of the same wave, and the LDS operands are read four MFMA pairs ahead, across the tile's end.
+//
+// K and V tiles go from memory straight into LDS (buffer_load ... lds), rings of four: step t requests K(t+5) and V(t+3), at
+// its end waits for what step t-1 requested and meets the barrier; rows past the segment and columns past the true head_dim
+// read as zero.  The selection words take the same way, each wave its own rows' into its own slots.
+//
+// What bounds it: with a selection the vector instructions (about 94 and 16 exponentials beside 16 MFMAs at head_dim 128, 32
+// of them the mask) and the power of the chip (1.75-1.9 GHz under this load); without one the softmax of tiles every row
+// attends whole drops the mask.  Same box, us, against the previous kernel (register staging, phases one after the other):
+// 32 768 tokens dense 1423 -> 1296, with a selection 1402 -> 1418; 8192 tokens with a selection 65 -> 62; head_dim 256, 16 384
+// tokens 219 -> 211; vision towers at head_dim 96 458 -> 367, at 64 342 -> 276.
+#include "dsa_tile.h"
+
+template <int D, int NW>
+constexpr size_t fwd_lds_bytes(bool has_idx) { return 8 * (size_t)DirectTile<D>::BYTES + (has_idx ? NW * 4 * 256 : 0); }
+
+template <int D, bool HAS_IDX, int NW>
+__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
+    const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
+    int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
+    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int causal,
+    bf16_t *__restrict__ out, float *__restrict__ lse) {
+    typedef DirectTile<D> TL;
+    constexpr int KS = D / 16, DT = D / 32;
+    constexpr int LPW = (TL::LOADS + NW - 1) / NW;          // wave loads per wave, step and operand
+    constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);        // everything a wave requests in a step
+    static_assert(TL::LOADS % NW == 0, "every wave loads the same number of pieces");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];    // 4 K slots | 4 V slots | selection words
+
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = Hq / Hkv, kvh = blockIdx.x % Hkv, QBW = (NW * 32) >> gshift;
+    int s0, L, blk;
+    if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    L = __builtin_amdgcn_readfirstlane(L);
+    if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
+    const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
+    if (qc0 >= pos_split || qc0 >= L) return;           // rows past the split belong to the gather kernel
+    const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
+
+    const int r = wv * 32 + j;
+    const int qcol = qc0 + (r >> gshift), head = r & ((1 << gshift) - 1);
+    const bool row_ok = qcol < L && head < G;
+    const int t = s0 + min(qcol, L - 1), hq = kvh * G + min(head, G - 1);
+    const int klim = causal ? qcol : L - 1;             // last key column this row may attend (dense mode)
+
+    // ---- requests ----
+    const int chunks = d_real / 8;
+    const int64_t k_step = 32 * k_tok * 2, v_step = 32 * v_tok * 2;      // bytes per tile
+    const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k + (int64_t)s0 * k_tok + (int64_t)kvh * k_head);
+    const unsigned char *vptr = reinterpret_cast<const unsigned char *>(v + (int64_t)s0 * v_tok + (int64_t)kvh * v_head);
+    constexpr int NV = LPW < TL::SOURCES ? LPW : TL::SOURCES;   // the lane's source offsets repeat after that many pieces
+    int kvoff[NV], vvoff[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        kvoff[i] = TL::source(wv * LPW + i, lane, (int)k_tok * 2, chunks);
+        vvoff[i] = TL::source(wv * LPW + i, lane, (int)v_tok * 2, chunks);
+    }
+    const uint32_t lds0 = lds_address(dyn_lds);
+    // Addresses of the next tile to request, in scalar registers (the asm statements keep them there); what is left of the
+    // block's keys from its first row on, in bytes, bounds the buffer
+    const int Lend = min(L, ntiles * 32);
+    auto next = [](const unsigned char *&p, int64_t step) __attribute__((always_inline)) {
+        p += step;
+        asm volatile("" : "+s"(p));
+    };
+    auto left = [&](int tile, int tok_b) __attribute__((always_inline)) { return max(min(Lend - tile * 32, 32), 0) * tok_b; };
+    auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
+        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV], i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
+                          lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
+        if (i == LPW - 1) next(kptr, k_step);
+    };
+    auto load_v_piece = [&](int tile, int i) __attribute__((always_inline)) {
+        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV], i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
+                          lds0 + (4 + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
+        if (i == LPW - 1) next(vptr, v_step);
+    };
+    auto load_k = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) load_k_piece(tile, i);
+    };
+    auto load_v = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) load_v_piece(tile, i);
+    };
+    unsigned char *const words = dyn_lds + 8 * TL::BYTES + wv * 1024;     // [tile % 4][lane]
+    const int wq0 = __builtin_amdgcn_readfirstlane(min(qc0 + ((wv * 32) >> gshift), L - 1));   // the wave's first query
+    const unsigned char *wptr = reinterpret_cast<const unsigned char *>(bitmap + (int64_t)(s0 + wq0) * ldw);
+    const int wvoff = (t - s0 - wq0) * ldw * 4;         // (at most 31 rows of bitmap)
+    auto load_w = [&](int tile) __attribute__((always_inline)) {
+        if (HAS_IDX) {
+            buffer_load_lds4(make_buffer_rsrc(wptr, 32 * ldw * 4), wvoff, 0, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
+            if (tile + 1 < ntiles) next(wptr, 4);        // (past the block's tiles: the last word again, never used)
+        }
+    };
+    bf16x8 qB[KS];
+    const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
+    load_k(0); load_w(0); load_k(1); load_w(1); load_v(0); load_k(2); load_w(2); load_v(1); load_k(3); load_w(3); load_v(2);
+
+    TL tl;
+    tl.init(lane);
+    f32x16 oacc[DT], sE, sO;                            // S of even and of odd tiles
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = zero16();
+    uint32_t pE[8], pO[8];                              // P of even and of odd tiles, packed (keys 0-15 | 16-31)
+    float mrun = -INFINITY, lsum = 0.f;
+    wait_vmcnt<0>();
+    barrier_only();
+
+    int ka_[4], va_[4];                                 // operand addresses in the K tile of S(t+2) and in V(t)
+    auto k_addr = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ka_[i] = tl.rowq[i] + (tile & 3) * TL::BYTES;
+    };
+    auto v_addr = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) va_[i] = tl.trq[i] + (4 + (tile & 3)) * TL::BYTES;
+    };
+    auto read_k = [&](int ks) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8 *>(dyn_lds + ka_[TL::row_q(ks)] + TL::row_imm(ks));
+    };
+    auto read_v = [&](int i) __attribute__((always_inline)) {             // MFMA i of P V: keys of half i / DT, d-tile i % DT
+        const int pair = i / DT, dt = i % DT;
+        lds_u8 *p = (lds_u8 *)dyn_lds + va_[TL::tr_q(dt)];
+        return LaneOffsets<D>::tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
+    };
+    // The keys of a tile this lane keeps, as they lie in memory; live(word): element vi then sits at bit 8*(vi/4) + vi%4
+    const uint32_t row_mask = row_ok ? 0xffffffffu : 0u;
+    auto live = [&](uint32_t w) __attribute__((always_inline)) { return (w >> (4 * h)) & row_mask; };
+    auto word_of = [&](int tile) __attribute__((always_inline)) {
+        return HAS_IDX ? *reinterpret_cast<const uint32_t *>(words + (tile & 3) * 256 + lane * 4) : causal_bits(klim - tile * 32);
+    };
+    // The row maximum is not searched in every tile: P is formed against the running reference first, and only when a
+    // lane's sum says that some probability may have passed 2^8 - or a live row has not met a selected key yet - does the wave
+    // look for the tile's maximum, move the reference, rescale the sums and form P again: the first tile of a block, then
+    // rarely.  In between P stays below 2^8, exact in fp32 and safe in bf16, and never underflows as a whole, because the
+    // reference is a maximum the row has really met.
+    auto masked = [&](float s, uint32_t word, int vi) __attribute__((always_inline)) {
+        return keep_or_neginf(s, bit_mask(word, 8 * (vi >> 2) + (vi & 3)));
+    };
+    auto settle = [&](const f32x16 &s, uint32_t word, uint32_t (&p)[8], float &psum) __attribute__((always_inline)) {
+        if (__builtin_amdgcn_ballot_w64(row_ok && (mrun == -INFINITY || !(psum <= 256.f)))) {
+            asm volatile("" : "+v"(word));              // (nothing of the fast path is kept alive for this one)
+            float mloc = -INFINITY;
+#pragma unroll
+            for (int vi = 0; vi < 16; ++vi) mloc = fmaxf(mloc, masked(s[vi], word, vi));
+            mloc = half_max_f(mloc) * scale_log2;
+            if (mloc > mrun) {
+                const float alpha = fast_exp2(mrun - mloc);   // mrun = -inf: 0, and the sums are 0
+                lsum *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+                mrun = mloc;
+            }
+            const float mneg = (mrun == -INFINITY) ? 0.f : -mrun;
+            psum = 0.f;
+#pragma unroll
+            for (int vi = 0; vi < 16; vi += 2) {
+                const float a = fast_exp2(fmaf(masked(s[vi], word, vi), scale_log2, mneg));
+                psum += a;
+                const float b = fast_exp2(fmaf(masked(s[vi + 1], word, vi + 1), scale_log2, mneg));
+                psum += b;
+                p[vi >> 1] = pack2bf(a, b);
+            }
+        }
+        lsum += psum;
+    };
+    // S of tiles 0 and 1, P of tile 0
+    auto gemm_s = [&](f32x16 &s) __attribute__((always_inline)) {
+        s = zero16();
+        bf16x8 ka[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) ka[ks] = read_k(ks);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) s = mfma32(ka[ks], qB[ks], s);
+    };
+    k_addr(0);
+    gemm_s(sE);
+    if (ntiles > 1) {
+        k_addr(1);
+        gemm_s(sO);
+    }
+    {
+        float psum = INFINITY;                          // (no reference yet: the maximum is searched for)
+        if (!row_ok) psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pE[i] = 0u;
+        settle(sE, live(word_of(0)), pE, psum);
+    }
+    __syncthreads();                                    // every wave is done with K(0) and K(1): their slots may be filled again
+    load_k(4);
+    constexpr int AHEAD = KS % 4 ? 3 : 4;               // (divides KS: an operand keeps its register from step to step)
+    static_assert(KS % AHEAD == 0);
+    bf16x8 kr[AHEAD], vr[AHEAD];                        // operands of the next MFMA pairs
+    k_addr(2);
+    v_addr(0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) { kr[i] = read_k(i); vr[i] = read_v(i); }
+    uint32_t word_next = word_of(1);                    // (one-tile blocks never use it)
+
+    // piece r of what step t requests: K(t+5), V(t+3) and the selection words of tile t+4
+    auto request = [&](int t_, int r_) __attribute__((always_inline)) {
+        if (r_ < LPW) load_k_piece(t_ + 5, r_);
+        else if (r_ < 2 * LPW) load_v_piece(t_ + 3, r_ - LPW);
+        else load_w(t_ + 4);
+    };
+    // Step t: O += P(t) V(t) with `p`; softmax of tile t+1 from `s` into `pn` (SM); S(t+2) into `sn` (NEXT).
+    auto step = [&](auto masked_, auto sm_, auto next_, auto req_, int t_, const uint32_t (&p)[8], const f32x16 &s, uint32_t (&pn)[8],
+                    f32x16 &sn) __attribute__((always_inline)) {
+        constexpr bool MASKED = decltype(masked_)::value, SM = decltype(sm_)::value, NEXT = decltype(next_)::value, REQ = decltype(req_)::value;
+        const u32x4 w0 = {p[0], p[1], p[2], p[3]}, w1 = {p[4], p[5], p[6], p[7]};
+        const bf16x8 pB0 = __builtin_bit_cast(bf16x8, w0), pB1 = __builtin_bit_cast(bf16x8, w1);
+        const uint32_t word = MASKED ? live(word_next) : 0xffffffffu;
+        float psum = 0.f;
+        const float mneg = (mrun == -INFINITY) ? 0.f : -mrun;
+        f32x16 snew;
+        // The softmax of an element is a chain of dependent instructions (mask, scale, exponential, sum, pack) and a wave
+        // issues in order: behind each MFMA stand the first part of one element's chain, the exponential of the element before
+        // and the sum of the one before that, so that no instruction waits for the one in front of it.
+        constexpr int H = 2 * KS - 2;                   // half-steps an element can start in
+        float y[16], e[16];
+        auto behind = [&](int hs) __attribute__((always_inline)) {
+#pragma unroll
+            for (int vi = 16 * (hs - 2) / H; vi < 16 * (hs - 1) / H; ++vi)
+                if (hs >= 2) {
+                    psum += e[vi];
+                    if (vi & 1) {
+                        pn[vi >> 1] = pack2bf(e[vi - 1], e[vi]);
+                        asm volatile("" : "+v"(pn[vi >> 1]));
+                    }
+                }
+#pragma unroll
+            for (int vi = 16 * (hs - 1) / H; vi < 16 * hs / H; ++vi)
+                if (hs >= 1 && hs <= H) {
+                    e[vi] = fast_exp2(y[vi]);
+                    asm volatile("" : "+v"(e[vi]));
+                }
+#pragma unroll
+            for (int vi = 16 * hs / H; vi < 16 * (hs + 1) / H; ++vi)
+                if (hs < H) {
+                    y[vi] = fmaf(MASKED ? masked(s[vi], word, vi) : s[vi], scale_log2, mneg);
+                    asm volatile("" : "+v"(y[vi]));
+                }
+            asm volatile("" : "+v"(psum) : : "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            oacc[i % DT] = mfma32(vr[i % AHEAD], i < DT ? pB0 : pB1, oacc[i % DT]);
+            // this step's requests, spread over its first half: one after the other they would queue for the way into LDS
+#pragma unroll
+            for (int r_ = 0; r_ < LPS; ++r_)
+                if (REQ && r_ * (KS / 2) / LPS == i) request(t_, r_);
+            // refill: the operand AHEAD pairs on, of this step's tiles or, past their end, of the next step's
+            if (i == KS - AHEAD && SM) v_addr(t_ + 1);
+            if (i + AHEAD < KS || SM) vr[i % AHEAD] = read_v((i + AHEAD) % KS);
+            if (SM) behind(2 * i);
+            else __builtin_amdgcn_sched_barrier(0);
+            if (NEXT) {
+                snew = mfma32(kr[i % AHEAD], qB[i], i == 0 ? zero16() : snew);
+                if (i == KS - AHEAD) k_addr(t_ + 3);
+                kr[i % AHEAD] = read_k((i + AHEAD) % KS);
+                if (i == 0 && MASKED) word_next = word_of(t_ + 2);
+            }
+            if (SM) behind(2 * i + 1);
+        }
+        if (SM) settle(s, word, pn, psum);
+        if (NEXT) sn = snew;
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    auto meet = [&]() __attribute__((always_inline)) {
+        wait_vmcnt<LPS>();                              // all but what this step requested
+        barrier_only();
+    };
+    auto full_step = [&](auto masked_, int t_, const uint32_t (&p)[8], const f32x16 &s, uint32_t (&pn)[8], f32x16 &sn) __attribute__((always_inline)) {
+        step(masked_, yes, yes, yes, t_, p, s, pn, sn);
+        meet();
+    };
+    int tt = 0;
+    if (!HAS_IDX) {
+        // tiles every row of the block attends whole: the softmax without mask arithmetic (a loop of its own, not a branch
+        // in the loop: two bodies that meet again would keep two sets of accumulators)
+        const int whole = (causal ? qc0 : L) / 32;
+        for (; tt + 3 < ntiles && tt + 2 < whole; tt += 2) {
+            full_step(no, tt, pE, sO, pO, sE);
+            full_step(no, tt + 1, pO, sE, pE, sO);
+        }
+        word_next = word_of(tt + 1);
+    }
+    if constexpr (D > 128) {
+        // (S of up to two tiles past the end is formed for nothing: the exact tail below costs registers this head_dim lacks)
+        for (; tt + 2 < ntiles; tt += 2) {
+            full_step(yes, tt, pE, sO, pO, sE);
+            full_step(yes, tt + 1, pO, sE, pE, sO);
+        }
+        if (tt + 1 < ntiles) {
+            full_step(yes, tt, pE, sO, pO, sE);
+            step(yes, no, no, no, tt + 1, pO, sE, pE, sO);
+        } else {
+            step(yes, no, no, no, tt, pE, sO, pO, sE);
+        }
+    } else {
+        for (; tt + 3 < ntiles; tt += 2) {
+            full_step(yes, tt, pE, sO, pO, sE);
+            full_step(yes, tt + 1, pO, sE, pE, sO);
+        }
+        // at most three tiles are left
+        if (tt + 2 < ntiles) {
+            full_step(yes, tt, pE, sO, pO, sE);
+            step(yes, yes, no, yes, tt + 1, pO, sE, pE, sO);
+            meet();
+            step(yes, no, no, no, tt + 2, pE, sO, pO, sE);
+        } else if (tt + 1 < ntiles) {
+            step(yes, yes, no, yes, tt, pE, sO, pO, sE);
+            meet();
+            step(yes, no, no, no, tt + 1, pO, sE, pE, sO);
+        } else {
+            step(yes, no, no, no, tt, pE, sO, pO, sE);
+        }
+    }
+    wait_vmcnt<0>();                                    // no load is left on its way into LDS when the workgroup ends
+
+    float l = half_sum_f(lsum);
+    if (row_ok) {
+        const float inv = 1.f / l;
+        bf16_t *op = out + ((int64_t)t * Hq + hq) * d_real;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, oacc[dt], inv, h, chunks - 4 * dt);
+        if (h == 0) lse[(int64_t)hq * T + t] = (mrun + log2f(l)) * LN2_F;
+    }
+}
+
+template <int D, bool HAS_IDX, int NW>
+static hipError_t launch_fwd_n(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
+                               void *out, float *lse) {
+    const auto kernel = &dsa_tile_fwd_kernel<D, HAS_IDX, NW>;
+    constexpr size_t lds = fwd_lds_bytes<D, NW>(HAS_IDX);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
+                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, (bf16_t *)out, lse);
+    return hipSuccess;
+}
+template <int D, bool HAS_IDX>
+static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
+                               void *out, float *lse) {
+    // At head_dim 96 and 128 eight waves share each staged tile - except in launches of a few rounds of workgroups, which
+    // are bound by what a workgroup pays before its first tile and after its last: there two four-wave workgroups per CU
+    // overlap those parts.
+    if constexpr (D == 128 || D == 96) {
+        const int64_t blocks = ((int64_t)T / ((32 * 8) >> gshift) + N + 1) * Hkv;
+        if (blocks > DSA_BATCH_ORDER_MAX_BLOCKS)
+            return launch_fwd_n<D, HAS_IDX, 8>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
+    }
+    return launch_fwd_n<D, HAS_IDX, 4>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
+}
+
+// d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 96, 128, 256 runs it; 96 without a
+// bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
+extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
+                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
+                                          int pos_split, int causal, void *out, float *lse, hipStream_t stream) {
+    int gs = 0;
+    while ((1 << gs) < Hq / Hkv) ++gs;
+    const float sl2 = scale * LOG2E_F;
+    hipError_t e = hipErrorInvalidValue;
+#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, sl2, pos_split, causal, out, lse)
+    if (bitmap) {
+        if (d_real <= 64) FWD_CASE(64, true);
+        else if (d_real <= 128) FWD_CASE(128, true);
+        else if (d_real <= 256) FWD_CASE(256, true);
+    } else {
+        if (d_real <= 64) FWD_CASE(64, false);
+        else if (d_real <= 96) FWD_CASE(96, false);
+        else if (d_real <= 128) FWD_CASE(128, false);
+        else if (d_real <= 256) FWD_CASE(256, false);
+    }
+#undef FWD_CASE
+    return e != hipSuccess ? e : hipGetLastError();
+}
