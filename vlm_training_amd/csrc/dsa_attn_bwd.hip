@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64) void dsa_bwd_dq_kernel(
     __shared__ __attribute__((aligned(16))) unsigned char klds[32 * ROW_B];
 
     const int lane = threadIdx.x, g = lane >> 4, m = lane & 15;
-    const int kvh = blockIdx.x % Hkv, t = blockIdx.x / Hkv;
+    const int kvh = blockIdx.x / T, t = blockIdx.x % T;
     const int G = Hq / Hkv;
     const int s0 = cu[find_segment_wave(cu, N, t)];
     if (t - s0 < pos_min) return;                     // rows before the split belong to the tile kernel
