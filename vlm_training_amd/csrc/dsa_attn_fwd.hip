@@ -13,10 +13,9 @@
 //                                       padded rows, transposed 2-byte reads), B = P^T taken directly
 //                                       from the C layout of S^T (no cross-lane movement)
 // Loads of tile i+1 are issued before the softmax/PV work of tile i.  The grid goes through the queries of
-// one kv head, then of the next: the rows that run at any time then gather from one head's K and V, which the
-// 256 MB Infinity Cache holds up to half a million keys (all eight heads of 131 072 tokens are 537 MB, and with
-// a kv head per XCD this kernel and the dQ gather drew every row past L2 from HBM at 6.5 TB/s: 89 -> 76 ms
-// and 94 -> 78 ms for the 81 920 rows beyond position 49 152).
+// one kv head, then of the next: the rows that run at any time then gather from one head's K and V (67 MB at
+// 131 072 tokens, against 537 MB for eight heads, which no cache holds).  With a kv head per XCD instead, the
+// 81 920 rows beyond position 49 152 took 89.1 ms here, now 76.9, and 94.2 ms in the dQ gather, now 79.9.
 #include "dsa_common.h"
 
 template <int D, bool HAS_IDX>
