@@ -268,6 +268,16 @@ int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const void *k, co
  */
 int dsa_dense_fwd(const void *q, const void *k, const void *v, const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv,
                   int D, float softmax_scale, int dtype, int max_seqlen, int causal, void *out, float *lse, void *stream);
+/*
+ * dsa_dense_fwd on tensors as the caller has them: element (t, h, d) of q lies at q + t*q_tok_stride + h*q_head_stride + d
+ * (strides in elements, likewise k and v), so a (1, H, T, D) tensor of an HF module is read without a transposing copy, and
+ * D is the true head_dim: any multiple of 8 up to 256.  Base pointers on 16-byte boundaries, strides multiples of 8, token
+ * strides below 2^24.  out (T,Hq,D) and lse (Hq,T) are contiguous.
+ */
+int dsa_dense_fwd_strided(const void *q, int64_t q_tok_stride, int64_t q_head_stride, const void *k, int64_t k_tok_stride,
+                          int64_t k_head_stride, const void *v, int64_t v_tok_stride, int64_t v_head_stride,
+                          const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
+                          int max_seqlen, int causal, void *out, float *lse, void *stream);
 int dsa_dense_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
                   const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
                   int max_seqlen, int causal, void *dq, void *dk, void *dv, void *ws, size_t ws_bytes, void *stream);

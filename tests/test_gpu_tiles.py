@@ -1,0 +1,40 @@
+"""The tile kernels where they can go wrong: tensors read in place, head_dims between the kernels' own, tile edges."""
+import pytest
+import torch
+
+from oracle import dsa_ref as R
+from tests.util import assert_close_bf16
+import vlm_training_amd as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _cu(lens):
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    return torch.tensor(cu, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,lens,causal", [
+    (8, 2, 1, (1,), True), (64, 8, 2, (31, 33, 1), True), (72, 4, 4, (64, 97), False), (80, 3, 1, (65, 2), True),
+    (128, 4, 1, (129, 160, 32), True), (200, 4, 2, (96, 5), False), (256, 8, 1, (70, 33), True)])
+def test_dense_forward_reads_hf_tensors_in_place(D, Hq, Hkv, lens, causal):
+    print("strided dense forward", D, Hq, Hkv, lens, causal, flush=True)
+    g = torch.Generator().manual_seed(D)
+    cu, T = _cu(lens), sum(lens)
+    q, k, v = (torch.randn(1, h, T, D, generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
+    packed = [x[0].transpose(0, 1) for x in (q, k, v)]
+    ref = R.dense_varlen_causal(*packed, cu, causal=causal)
+    with torch.no_grad():
+        views = [x.to(DEV)[0].transpose(0, 1) for x in (q, k, v)]
+        got = M.dispatch_varlen_attention(*views, cu.to(DEV), max(lens), causal=causal)
+        same = M.dispatch_varlen_attention(*(x.contiguous() for x in views), cu.to(DEV), max(lens), causal=causal)
+    assert got.shape == (T, Hq, D) and got.is_contiguous()
+    assert_close_bf16(got, ref, "strided forward")
+    assert torch.equal(got, same)
+    if causal:
+        with torch.no_grad():
+            hf = M.varlen_attention_forward(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV))[0]
+        assert torch.equal(hf[0], got)

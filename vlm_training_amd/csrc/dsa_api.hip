@@ -666,6 +666,24 @@ extern "C" int dsa_dense_fwd(const void *q, const void *k, const void *v, const 
                         nullptr, 0, stream);
 }
 
+extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_head, const void *k, int64_t k_tok, int64_t k_head, const void *v,
+                                     int64_t v_tok, int64_t v_head, const int32_t *cu, int T, int N, int Hq, int Hkv, int D,
+                                     float softmax_scale, int dtype, int max_seqlen, int causal, void *out, float *lse, void *stream) {
+    if (D < 8 || D > 256 || D % 8) return fail(DSA_ERR_UNSUPPORTED, "head_dim=%d: need a multiple of 8 up to 256", D);
+    if (int rc = check_attn(T, N, cu, Hq, Hkv, 64, 0, dtype, nullptr, nullptr)) return rc;     // (head_dim checked above)
+    if (!q || !k || !v || !out || !lse) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
+    const int64_t strides[6] = {q_tok, q_head, k_tok, k_head, v_tok, v_head};
+    for (int i = 0; i < 6; ++i)
+        if (strides[i] < 0 || strides[i] % 8 || (i % 2 == 0 && strides[i] >= (1 << 24)))
+            return fail(DSA_ERR_ARG, "strides must be multiples of 8, token strides below 2^24");
+    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) return fail(DSA_ERR_ARG, "tensors must lie on 16-byte boundaries");
+    if (T == 0) return DSA_OK;
+    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, causal, out, lse,
+                                             (hipStream_t)stream);
+    return e == hipSuccess ? DSA_OK : hip_fail(e, "tile forward launch");
+}
+
 extern "C" int dsa_dense_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
                              const int32_t *cu, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
                              int max_seqlen, int causal, void *dq, void *dk, void *dv, void *ws, size_t ws_bytes,

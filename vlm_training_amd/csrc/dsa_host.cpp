@@ -253,9 +253,13 @@ public:
     }
 };
 
+bool needs_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
+    return at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+}
+
 variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, const OptTensor &idx, const OptTensor &n,
                         double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
-    if (!(at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))) {
+    if (!needs_grad(q, k, v)) {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::OptionalDeviceGuard guard(q.device());
         const AttnArgs a{max_seqlen, scale, causal, want_mass, q.scalar_type() == at::kFloat && 4 * q.size(2) <= 256, q.scalar_type()};
@@ -273,6 +277,21 @@ Qkv checked_qkv(const Tensor &q, const Tensor &k, const Tensor &v) {
     TORCH_CHECK_VALUE(s.Hkv > 0 && s.Hq % s.Hkv == 0, "Hq=", s.Hq, " must be a multiple of Hkv=", s.Hkv);
     TORCH_CHECK_VALUE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "q, k, v must share a dtype");
     return s;
+}
+
+// q, k and v can go to the dense forward as they lie in memory: no transposing copy, no padding of the head_dim
+bool readable_in_place(const Tensor &t) {
+    return t.scalar_type() == at::kBFloat16 && t.stride(2) == 1 && t.size(2) % 8 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
+           t.stride(0) < (1 << 24) && ((uintptr_t)t.data_ptr() & 15) == 0;
+}
+// the dense forward without a graph
+Tensor dense_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, double scale, bool causal) {
+    const Qkv s{q.size(0), q.size(1), k.size(1), q.size(2)};
+    const Tensor out = empty({s.T, s.Hq, s.D}, at::kBFloat16, q), lse = empty({s.Hq, s.T}, at::kFloat, q);
+    check(dsa_dense_fwd_strided(ptr(q), q.stride(0), q.stride(1), ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1), iptr(cu), (int)s.T,
+                                (int)cu.numel() - 1, (int)s.Hq, (int)s.Hkv, (int)s.D, (float)scale, DSA_DTYPE_BF16, (int)max_seqlen, causal, ptr(out),
+                                fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
+    return out;
 }
 
 // the operator: out [, idx, n] [, mass] [, scores]
@@ -307,6 +326,8 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
     TORCH_CHECK_VALUE(d_kernel, "head_dim ", sh.D, " is beyond the kernels' largest (256)");
     TORCH_CHECK_VALUE(sparse || !return_mass, "return_mass needs the indexer inputs");
     Tensor q = q_, k = k_, v = v_;
+    if (!sparse && !needs_grad(q, k, v) && readable_in_place(q) && readable_in_place(k) && readable_in_place(v))
+        return {dense_forward(q, k, v, cu, max_seqlen, scale, causal)};
     if (d_kernel != sh.D) {
         // zero columns change neither q.k nor the used part of p.v
         const int64_t pad = d_kernel - sh.D;
