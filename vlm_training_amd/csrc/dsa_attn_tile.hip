@@ -73,6 +73,9 @@ __device__ __forceinline__ float group_sum(float x) {
 // second set hands its sums to the first through LDS once per tile.  A slot of the result is therefore written
 // once, by one lane, with the finished sum: no table per kv head, nothing read back.  Only a batch with more kv
 // heads than a workgroup holds is cut into groups with one table each.
+// A slot depends on its own tile alone, so a walk can be cut anywhere: launches that leave the chip idle (one workgroup
+// per CU: 64 queries of a 2B stack's 8192 tokens are 128 workgroups for 256 CUs) run pieces of `chunk` tiles as workgroups
+// of their own, each counting the selected keys in front of its piece first (there 189 -> 89 us).
 template <int D> constexpr int mass_heads_max() { return 1024 / D; }      // 16 / 8 / 4 kv heads at head_dim 64 / 128 / 256
 template <int HPG> constexpr int mass_sets() { return HPG >= 2 ? 2 : 1; }
 template <int D, int HPG> constexpr size_t mass_lds_bytes() {
@@ -82,7 +85,7 @@ template <int D, int GSHIFT, int HPG>
 __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const float *__restrict__ lse,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale_log2, int K, int ngroups, float final_mul, float *__restrict__ table) {
+    float scale_log2, int K, int ngroups, int chunk, float final_mul, float *__restrict__ table) {
     constexpr int NS = mass_sets<HPG>(), HPW = HPG / NS;       // wave sets; kv heads per wave
     constexpr int KS = D / 16, CPR = D / 8, TILE_B = tile_bytes<D>(), NT = 256 * NS;
     constexpr int Gp = 1 << GSHIFT, QBW = (4 * 32) >> GSHIFT;
@@ -109,10 +112,12 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
     const int qcol = qc0 + (r >> GSHIFT), head = r & (Gp - 1);
     const bool row_ok = qcol < L && head < G;
     const int t = s0 + min(qcol, L - 1);
-    const int ntiles = min(qc0 + QBW - 1, L - 1) / 32 + 1;
+    // this workgroup's piece of the walk: tiles [it0, ntiles)
+    const int it0 = (int)blockIdx.y * chunk, ntiles = min((min(qc0 + QBW - 1, L - 1) / 32 + 1), it0 + chunk);
+    if (it0 >= ntiles) return;
     const uint32_t *wrow = bitmap + (int64_t)t * ldw;
     float *prow = table + ((int64_t)grp * T + t) * K;
-    if (ngroups == 1) {
+    if (ngroups == 1 && it0 == 0) {
         // the table is the result itself: slots past a row's selection (rows shorter than K keys) are zero
         for (int qq = 0; qq < QBW && qc0 + qq < L; ++qq) {
             float *zr = table + (int64_t)(s0 + qc0 + qq) * K;
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
         const int row = c / (HPG * CPR), hh = (c / CPR) % HPG, ch = c % CPR;                       \
         *reinterpret_cast<u32x4 *>(&dyn_lds[hh * TILE_B + tile_off<D>(row, ch)]) = kst[i];         \
     }
-    MASS_LOAD(0)
+    MASS_LOAD(it0)
     bf16x8 qB[HPW][KS];
     float lse2[HPW];
 #pragma unroll
@@ -151,11 +156,14 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
         const float lse_row = lse[(int64_t)hq * T + t];
         lse2[hh] = (row_ok && kvh0 + kv_rel < Hkv) ? lse_row * LOG2E_F : INFINITY;
     }
-    uint32_t word_next = qcol < L ? wrow[0] : 0u;
-    int seen = 0;                                        // selected keys of this row in the tiles already walked
+    uint32_t word_next = qcol < L ? wrow[it0] : 0u;
+    int seen = 0;                                        // selected keys of this row in the tiles before this one
+    for (int w = 0; w < it0; w += 8)                     // (it0 is a multiple of 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) seen += __popc(wrow[w + u]);
     MASS_STORE()
     __syncthreads();
-    for (int it = 0; it < ntiles; ++it) {
+    for (int it = it0; it < ntiles; ++it) {
         MASS_LOAD(min(it + 1, ntiles - 1))               // lands during this tile's matrix work
         const uint32_t word_full = word_next;
         { const uint32_t wl = wrow[min(it + 1, ntiles - 1)]; word_next = qcol < L ? wl : 0u; }
@@ -1894,7 +1902,7 @@ extern "C" int dsa_mass_groups(int Hq, int Hkv, int D) {
 template <int D, int GS, int HPG>
 static hipError_t launch_mass_h(dim3 grid, hipStream_t stream, const void *q, const void *k, const float *lse,
                                 const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float sl2,
-                                int K, int ngroups, float final_mul, float *table) {
+                                int K, int ngroups, int chunk, float final_mul, float *table) {
     if constexpr (HPG > mass_heads_max<D>()) {
         return hipErrorInvalidValue;
     } else {
@@ -1902,21 +1910,21 @@ static hipError_t launch_mass_h(dim3 grid, hipStream_t stream, const void *q, co
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)mass_lds_bytes<D, HPG>());
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL((dsa_tile_mass_kernel<D, GS, HPG>), grid, dim3(256 * mass_sets<HPG>()), (mass_lds_bytes<D, HPG>()), stream,
-                           (const bf16_t *)q, (const bf16_t *)k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul,
-                           table);
+                           (const bf16_t *)q, (const bf16_t *)k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk,
+                           final_mul, table);
         return hipSuccess;
     }
 }
 template <int D, bool HAS_IDX, int GS>
 static hipError_t launch_mass_i(dim3 grid, hipStream_t stream, const void *q, const void *k, const float *lse,
                           const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float sl2,
-                          int K, int ngroups, float final_mul, float *table) {
+                          int K, int ngroups, int chunk, float final_mul, float *table) {
     switch (mass_hpg<D>(Hq, Hkv)) {
-        case 1: return launch_mass_h<D, GS, 1>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul, table);
-        case 2: return launch_mass_h<D, GS, 2>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul, table);
-        case 4: return launch_mass_h<D, GS, 4>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul, table);
-        case 8: return launch_mass_h<D, GS, 8>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul, table);
-        default: return launch_mass_h<D, GS, 16>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, final_mul, table);
+        case 1: return launch_mass_h<D, GS, 1>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk, final_mul, table);
+        case 2: return launch_mass_h<D, GS, 2>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk, final_mul, table);
+        case 4: return launch_mass_h<D, GS, 4>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk, final_mul, table);
+        case 8: return launch_mass_h<D, GS, 8>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk, final_mul, table);
+        default: return launch_mass_h<D, GS, 16>(grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk, final_mul, table);
     }
 }
 // attention mass of the selected keys: the heads of a query summed in registers, scaled by 1/Hq and written into
@@ -1927,11 +1935,16 @@ extern "C" hipError_t dsa_launch_tile_mass(const void *q, const void *k, const f
                                            int D, int K, float scale, float *partial, float *mass, hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
     const int ngroups = dsa_mass_groups(Hq, Hkv, D);
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * 4) >> gs) + N + 1) * ngroups));
+    const int64_t blocks = ((int64_t)T / ((32 * 4) >> gs) + N + 1) * ngroups;
+    // walks (ldw tiles at most) stay whole from four workgroups per CU on; below, pieces of at least 8 tiles (a tile takes
+    // about 3 us, the q rows of a piece as long as one or two tiles), as many as give the chip about four rounds
+    const int64_t chunk_fit = blocks * ldw / (2 * 4 * 256) / 8 * 8;
+    const int chunk = blocks >= 4 * 256 ? ldw : (int)std::max<int64_t>(chunk_fit, 8);
+    const dim3 grid((unsigned)blocks, (unsigned)((ldw + chunk - 1) / chunk));
     const float inv_hq = 1.f / (float)Hq;
     float *table = ngroups == 1 ? mass : partial;
     const float final_mul = ngroups == 1 ? inv_hq : 1.f;
-    TILE_SWITCH(launch_mass_i, grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, scale * LOG2E_F, K, ngroups, final_mul, table)
+    TILE_SWITCH(launch_mass_i, grid, stream, q, k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, scale * LOG2E_F, K, ngroups, chunk, final_mul, table)
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ngroups == 1) return e;
     const unsigned parts = (unsigned)((K / 4 + 255) / 256 > 0 ? (K / 4 + 255) / 256 : 1);

@@ -203,6 +203,7 @@ public:
         ctx->saved_data["p"] = a.split;
         if (!want_mass) return {f.res};
         ctx->mark_non_differentiable({f.mass});
+        ctx->set_materialize_grads(false);               // (no (T,K) table of zeros as the mass's gradient)
         return {f.res, f.mass};
     }
 
