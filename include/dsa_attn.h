@@ -278,6 +278,11 @@ int dsa_dense_fwd_strided(const void *q, int64_t q_tok_stride, int64_t q_head_st
                           int64_t k_head_stride, const void *v, int64_t v_tok_stride, int64_t v_head_stride,
                           const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
                           int max_seqlen, int causal, void *out, float *lse, void *stream);
+/* The backward for contiguous rows of any head_dim that is a multiple of 8 up to 128, read and written where they lie (no
+ * zero-padding to a kernel's head_dim).  scratch: dsa_attn_bwd_scratch_bytes. */
+int dsa_dense_bwd_rows(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
+                       const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
+                       int max_seqlen, int causal, void *dq, void *dk, void *dv, void *scratch, size_t scratch_bytes, void *stream);
 int dsa_dense_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
                   const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
                   int max_seqlen, int causal, void *dq, void *dk, void *dv, void *ws, size_t ws_bytes, void *stream);

@@ -38,3 +38,24 @@ def test_dense_forward_reads_hf_tensors_in_place(D, Hq, Hkv, lens, causal):
         with torch.no_grad():
             hf = M.varlen_attention_forward(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV))[0]
         assert torch.equal(hf[0], got)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,lens,causal", [
+    (8, 2, 1, (1, 34), True), (40, 4, 2, (129, 63), False), (72, 2, 2, (64, 97, 130), False), (72, 1, 1, (1500,), True),
+    (80, 6, 2, (161, 31), True), (88, 2, 1, (70,), False), (112, 3, 3, (33, 128, 257), True), (120, 2, 1, (900, 5), True)])
+def test_dense_gradients_between_the_kernels_head_dims(D, Hq, Hkv, lens, causal):
+    print("dense gradients", D, Hq, Hkv, lens, causal, flush=True)
+    g = torch.Generator().manual_seed(D)
+    cu, T = _cu(lens), sum(lens)
+    q, k, v, dout = (torch.randn(T, h, D, generator=g).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    ref = [x.float().requires_grad_(True) for x in (q, k, v)]
+    want = R.dense_varlen_causal(*ref, cu, causal=causal)
+    want.backward(dout.float())
+    got = [x.to(DEV).requires_grad_(True) for x in (q, k, v)]
+    out = M.dispatch_varlen_attention(*got, cu.to(DEV), max(lens), causal=causal)
+    out.backward(dout.to(DEV))
+    assert out.shape == (T, Hq, D)
+    assert_close_bf16(out, want, "out")
+    for name, a, b in zip("qkv", got, ref):
+        assert a.grad.shape == b.grad.shape
+        assert_close_bf16(a.grad, b.grad, "d" + name)

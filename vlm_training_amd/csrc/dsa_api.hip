@@ -651,6 +651,22 @@ extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const 
                         delta, bitmap, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream);
 }
 
+extern "C" int dsa_dense_bwd_rows(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
+                                  const int32_t *cu, int T, int N, int Hq, int Hkv, int D, float softmax_scale, int dtype,
+                                  int max_seqlen, int causal, void *dq, void *dk, void *dv, void *scratch, size_t scratch_bytes,
+                                  void *stream) {
+    if (D < 8 || D > 128 || D % 8) return fail(DSA_ERR_UNSUPPORTED, "head_dim=%d: need a multiple of 8 up to 128", D);
+    if (int rc = check_bwd(dout, q, k, v, out, lse, nullptr, nullptr, cu, T, N, Hq, Hkv, 64, 0, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
+    if (T == 0) return DSA_OK;
+    const size_t need = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
+    if (!scratch || scratch_bytes < need) return fail(DSA_ERR_WORKSPACE, "backward scratch: have %zu bytes, need %zu", scratch_bytes, need);
+    const size_t partial_bytes = bwd_partial_bytes_for(T, N, Hkv, D);
+    float *partial = partial_bytes ? (float *)((char *)scratch + align_up((size_t)T * Hq * 4, 256)) : nullptr;
+    int32_t *order = (int32_t *)((char *)scratch + need - align_up(dsa_tile_order_bytes(T), 256));
+    return attn_bwd_run(dout, q, k, v, out, lse, nullptr, nullptr, cu, T, N, Hq, Hkv, D, 0, softmax_scale, max_seqlen, causal, dq, dk, dv,
+                        (float *)scratch, nullptr, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream);
+}
+
 extern "C" int dsa_attn_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out,
                             const float *lse, const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N,
                             int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, int causal,

@@ -564,9 +564,9 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, int pos_split, int causal, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
+    float scale, int pos_split, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
+    constexpr int KS = D / 16, DT = (D + 31) / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
     constexpr int NBUF = (D > 128) ? 1 : 2;
     constexpr int NT = NW * 64, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT;
     constexpr int CH = 32 * CPR, LOADS = (CH + NT - 1) / NT;   // 16-byte chunks per matrix; per thread (head_dim 96: not all threads)
@@ -577,6 +577,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     LaneOffsets<D> lo;
     lo.init(lane);
     const int G = Hq / Hkv;
+    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
     const int kvh = blockIdx.x % Hkv;
     int s0, L, blk;
     if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
@@ -593,8 +594,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 #define DQ_LOAD(SET, TILE)                                                                          \
     _Pragma("unroll") for (int i = 0; i < LOADS; ++i) if (CH % NT == 0 || i * NT + tid < CH) {     \
         const int c = i * NT + tid;                                                               \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        const int64_t off = ((int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * Hkv + kvh) * D + ch * 8; \
+        const int row = c / CPR, ch = HAS_IDX ? c % CPR : min(c % CPR, chunks - 1);   /* (spare columns: any finite values) */ \
+        const int64_t off = ((int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * Hkv + kvh) * dr + ch * 8; \
         kst[SET][i] = *reinterpret_cast<const u32x4 *>(k + off);                                   \
         vst[SET][i] = *reinterpret_cast<const u32x4 *>(v + off);                                   \
     }
@@ -602,9 +603,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     bf16x8 qB[KS], doB[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-        const int64_t off = ((int64_t)t * Hq + hq) * D + 16 * ks + 8 * h;
-        qB[ks] = row_ok ? load_bf16x8(q + off) : zero_bf16x8();
-        doB[ks] = row_ok ? load_bf16x8(dout + off) : zero_bf16x8();
+        const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
+        const bool there = row_ok && (HAS_IDX || 2 * ks + h < chunks);
+        qB[ks] = there ? load_bf16x8(q + off) : zero_bf16x8();
+        doB[ks] = there ? load_bf16x8(dout + off) : zero_bf16x8();
     }
     // the two accumulators of a tile start from -lse/scale and -delta of the lane's row, so that S - lse/scale and
     // dP - delta come out of the MFMAs (one multiply per element instead of a multiply-add and a subtraction)
@@ -623,8 +625,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             p[j] = 0.f;
 #pragma unroll
             for (int ks = j; ks < KS; ks += 8) {
-                const int64_t off = ((int64_t)t * Hq + hq) * D + 16 * ks + 8 * h;
-                const bf16x8 o8 = row_ok ? load_bf16x8(out_for_delta + off) : zero_bf16x8();
+                const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
+                const bf16x8 o8 = row_ok && (HAS_IDX || 2 * ks + h < chunks) ? load_bf16x8(out_for_delta + off) : zero_bf16x8();
                 p[j] = dot8_chain(doB[ks], o8, p[j]);
             }
         }
@@ -690,9 +692,9 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 #undef DQ_COMPUTE
 
     if (row_ok) {
-        bf16_t *op = dq + ((int64_t)t * Hq + hq) * D;
+        bf16_t *op = dq + ((int64_t)t * Hq + hq) * dr;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, acc[dt], scale, h);
+        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, acc[dt], scale, h, chunks - 4 * dt);
     }
 }
 
@@ -953,16 +955,16 @@ __device__ __forceinline__ void store_c_tile_f32(float *row_dt, const f32x16 &ac
         *reinterpret_cast<f32x4 *>(row_dt + 8 * g4 + 4 * h) = w;
     }
 }
-// fp32 partial dK / dV of piece `piece` of a tile in pieces: [slot][kv head][dK | dV][128 keys][D]
+// fp32 partial dK / dV of piece `piece` of a tile in pieces: [slot][kv head][dK | dV][128 keys][D to the next 32]
 __device__ __forceinline__ float *piece_partial(float *partial, int mslot, int piece, int Hkv, int kvh, int D) {
     return partial + ((int64_t)(mslot + piece) * Hkv + kvh) * (2 * 128 * (int64_t)D);
 }
 // Adds the pieces of every tile that was cut, in piece order, and writes its dK (times the softmax scale) and dV
-// rows.  Grid: (cut tiles at most, kv heads, DSA_PIECES_Z slices of a tile's rows).
+// rows of D elements (`pitch` in the partial sums).  Grid: (cut tiles at most, kv heads, DSA_PIECES_Z slices of a tile's rows).
 #define DSA_PIECES_Z 4
 __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_t *__restrict__ order, int cap,
                                                                     const float *__restrict__ partial, const int32_t *__restrict__ cu,
-                                                                    int N, int Hkv, int D, int qb, int seq_clamp, float scale,
+                                                                    int N, int Hkv, int D, int pitch, int qb, int seq_clamp, float scale,
                                                                     bf16_t *__restrict__ dk, bf16_t *__restrict__ dv) {
     if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(order[2])) return;
     const int entry = __builtin_amdgcn_readfirstlane(order[4 + 4 * cap + blockIdx.x]);
@@ -976,7 +978,7 @@ __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_
     if (nblocks <= pb) return;                           // (its walk fits one piece after all: piece 0 wrote the rows itself)
     const int np = (nblocks + pb - 1) / pb, kvh = blockIdx.y;
     const int keys = min(128, L - c0), cpr = D / 4;      // 16-byte chunks per row
-    const int64_t slot_f = 2 * 128 * (int64_t)D;         // floats per (slot, kv head)
+    const int64_t slot_f = 2 * 128 * (int64_t)pitch;         // floats per (slot, kv head)
     const float *base = partial + ((int64_t)mslot * Hkv + kvh) * slot_f;
     constexpr int U = 4;                                 // independent chunks per thread and pass
     const int chunks = 2 * keys * cpr;                   // dK rows, then dV rows
@@ -987,7 +989,7 @@ __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_
         for (int u = 0; u < U; ++u) {
             const int c = min(c0_ + u, chunks - 1);
             const int m = c / (keys * cpr), rest = c % (keys * cpr);
-            off[u] = ((int64_t)m * 128 + rest / cpr) * D + (rest % cpr) * 4;
+            off[u] = ((int64_t)m * 128 + rest / cpr) * pitch + (rest % cpr) * 4;
             acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         for (int pc = 0; pc < np; pc += 2) {             // piece order: the sum does not depend on the schedule
@@ -1366,10 +1368,10 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, int causal, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
+    float scale, int causal, int d_real, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
     bf16_t *__restrict__ dv) {
     static_assert(D <= 128, "head_dim 256 runs dsa_tile_dkvpc_kernel");
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
+    constexpr int KS = D / 16, DT = (D + 31) / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
     constexpr int NCHUNK = 32 * CPR, STG = 256, CPT = (NCHUNK + STG - 1) / STG;
     constexpr bool ALL_STAGE = NCHUNK % STG == 0;        // (head_dim 96: the last chunk of half of the staging threads is spare)
     constexpr int Gp = 1 << GSHIFT, QB = 32 >> GSHIFT;
@@ -1388,6 +1390,7 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wv & 3;
     const int G = Hq / Hkv;
+    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
     const int kvh = blockIdx.x % Hkv;
     int s0, L, blk, piece, mslot, pb;
     if (!locate_key_tile(order, cu, N, blockIdx.x / Hkv, s0, L, blk, piece, mslot, pb)) return;
@@ -1421,7 +1424,7 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     // segment end, so only block 0 (rows past the end) and the steps past the last block need their rows zeroed.
     const int ctid = tid & 255;                          // used by the dS chain's waves
     const int last = nblocks - 1;
-    const int64_t blk_bytes = (int64_t)QB * Hq * D * 2;
+    const int64_t blk_bytes = (int64_t)QB * Hq * dr * 2;
     const unsigned char *qp[CPT], *dp[CPT];
     int64_t dlast[CPT];
     int lds_off[CPT];
@@ -1430,13 +1433,14 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     for (int i = 0; i < CPT; ++i) {
         staged[i] = ALL_STAGE || i * STG + ctid < NCHUNK; // a spare chunk loads the tile's last chunk again and stores nothing
         const int c = min(i * STG + ctid, NCHUNK - 1), srow = c / CPR, sch = c % CPR;
+        const int src_ch = HAS_IDX ? sch : min(sch, chunks - 1);     // (spare columns: any finite values; k and v are zero there)
         const int hd = min(srow & (Gp - 1), G - 1);
         const int qr = srow >> GSHIFT;
         const int over = max(q0 + last * QB + qr - (Lq - 1), 0);     // rows past the end in the last block
-        const int64_t off = ((int64_t)(s0 + q0 + last * QB + qr - over) * Hq + kvh * G + hd) * D + sch * 8;
+        const int64_t off = ((int64_t)(s0 + q0 + last * QB + qr - over) * Hq + kvh * G + hd) * dr + src_ch * 8;
         qp[i] = reinterpret_cast<const unsigned char *>(q + off);
         dp[i] = reinterpret_cast<const unsigned char *>(dout + off);
-        dlast[i] = -(int64_t)over * Hq * D * 2;
+        dlast[i] = -(int64_t)over * Hq * dr * 2;
         row_dead_last[i] = over > 0;
         head_ok[i] = (srow & (Gp - 1)) < G;
         lds_off[i] = tile_off<D>(srow, sch);
@@ -1546,7 +1550,7 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
         gload(1, qst1, dost1, aux_st1);
         bf16x8 vB[KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) vB[ks] = load_bf16x8(v + krow * D + 16 * ks + 8 * h);
+        for (int ks = 0; ks < KS; ++ks) vB[ks] = HAS_IDX || 2 * ks + h < chunks ? load_bf16x8(v + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
         lstore(0, qst0, dost0, aux_st0);
         lstore(1, qst1, dost1, aux_st1);
         gload(2, qst0, dost0, aux_st0);
@@ -1641,13 +1645,13 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
 #undef DKV2_DS_STEP
 #undef DKV2_DS_STEADY
         if (npieces > 1) {                               // a piece of the walk: fp32 partial sums, added by the reduction
-            float *pk = piece_partial(partial, mslot, piece, Hkv, kvh, D) + (kg * 32 + j) * D;
+            float *pk = piece_partial(partial, mslot, piece, Hkv, kvh, 32 * DT) + (kg * 32 + j) * 32 * DT;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) store_c_tile_f32(pk + dt * 32, dkacc[dt], h);
         } else if (key_ok) {
-            bf16_t *pk = dk + krow * D;
+            bf16_t *pk = dk + krow * dr;
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) store_c_tile(pk + dt * 32, dkacc[dt], scale, h);
+            for (int dt = 0; dt < DT; ++dt) store_c_tile(pk + dt * 32, dkacc[dt], scale, h, chunks - 4 * dt);
         }
         return;
     }
@@ -1655,7 +1659,7 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     // ================= P chain: S and softmax of block s, dV of block s-1 =================
     bf16x8 kB[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kB[ks] = load_bf16x8(k + krow * D + 16 * ks + 8 * h);
+    for (int ks = 0; ks < KS; ++ks) kB[ks] = HAS_IDX || 2 * ks + h < chunks ? load_bf16x8(k + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
     uint32_t mw[16];
     auto read_aux = [&](int b) __attribute__((always_inline)) {                         // selection words of step b
         const uint32_t *mask_s = reinterpret_cast<const uint32_t *>(aux_ring + (b & 3) * AUX_SLOT) + 64 + kg * 32;
@@ -1789,13 +1793,13 @@ __global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
     step(yes, no, yes, nblocks);
     __syncthreads();
     if (npieces > 1) {
-        float *pv_ = piece_partial(partial, mslot, piece, Hkv, kvh, D) + (128 + kg * 32 + j) * D;
+        float *pv_ = piece_partial(partial, mslot, piece, Hkv, kvh, 32 * DT) + (128 + kg * 32 + j) * 32 * DT;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) store_c_tile_f32(pv_ + dt * 32, dvacc[dt], h);
     } else if (key_ok) {
-        bf16_t *pv_ = dv + krow * D;
+        bf16_t *pv_ = dv + krow * dr;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(pv_ + dt * 32, dvacc[dt], 1.f, h);
+        for (int dt = 0; dt < DT; ++dt) store_c_tile(pv_ + dt * 32, dvacc[dt], 1.f, h, chunks - 4 * dt);
     }
 }
 template <int D>
@@ -1817,22 +1821,22 @@ static inline int group_shift(int Hq, int Hkv) {
 #ifndef DSA_TILE_WAVES_128
 #define DSA_TILE_WAVES_128 8
 #endif
-template <int D> constexpr int tile_waves() { return (D == 128 || D == 96) ? DSA_TILE_WAVES_128 : 4; }
-static inline int tile_waves_of(int D) { return (D == 128 || D == 96) ? DSA_TILE_WAVES_128 : 4; }
+template <int D> constexpr int tile_waves() { return (D <= 128 && D > 64) ? DSA_TILE_WAVES_128 : 4; }
+static inline int tile_waves_of(int D) { return (D <= 128 && D > 64) ? DSA_TILE_WAVES_128 : 4; }
 template <int D, bool HAS_IDX, int GS>
 static hipError_t launch_dq_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                         const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                        int T, int Hq, int Hkv, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
+                        int T, int Hq, int Hkv, int d_real, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
                         float *delta_out) {
     hipLaunchKernelGGL((dsa_tile_dq_kernel<D, HAS_IDX, GS, tile_waves<D>()>), grid, dim3(64 * tile_waves<D>()), 0, stream, (const bf16_t *)dout,
                        (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv,
-                       scale, pos_split, causal, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
+                       scale, pos_split, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
     return hipSuccess;
 }
 template <int D, bool HAS_IDX, int GS>
 static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                         int T, int Hq, int Hkv, float scale, int causal, const int32_t *order, float *partial, void *dk,
+                         int T, int Hq, int Hkv, int d_real, float scale, int causal, const int32_t *order, float *partial, void *dk,
                          void *dv) {
     // LDS above 64 KiB has to be requested per kernel and device; asked for on every launch (a host-side table
     // lookup), so that neither a second device nor a second thread can meet a kernel that was never configured
@@ -1842,7 +1846,7 @@ static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, 
         if (e2 != hipSuccess) return e2;
         hipLaunchKernelGGL((dsa_tile_dkv2_kernel<D, HAS_IDX, GS>), grid, dim3(512), dkv2_lds_bytes<D>(), stream,
                            (const bf16_t *)dout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap,
-                           ldw, cu, N, T, Hq, Hkv, scale, causal, order, partial, (bf16_t *)dk, (bf16_t *)dv);
+                           ldw, cu, N, T, Hq, Hkv, scale, causal, d_real, order, partial, (bf16_t *)dk, (bf16_t *)dv);
         return hipSuccess;
     } else {
     const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_tile_dkvpc_kernel<D, HAS_IDX, GS>),
@@ -1874,15 +1878,22 @@ static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, 
     }                                                                                     \
     if (launch_status != hipSuccess) return launch_status;
 
-// the same with head_dim 96 (dense only: no selection bitmap), for the three attention kernels
-#define TILE_SWITCH_96(FN, ...)                                                           \
-    hipError_t launch_status = hipSuccess;                                                \
-    switch (D) {                                                                          \
-        case 64: if (bitmap) { GS_SWITCH(FN, 64, true, __VA_ARGS__) } else { GS_SWITCH(FN, 64, false, __VA_ARGS__) } break;    \
-        case 96: if (bitmap) return hipErrorInvalidValue; GS_SWITCH(FN, 96, false, __VA_ARGS__) break;                         \
-        case 128: if (bitmap) { GS_SWITCH(FN, 128, true, __VA_ARGS__) } else { GS_SWITCH(FN, 128, false, __VA_ARGS__) } break; \
-        case 256: if (bitmap) { GS_SWITCH(FN, 256, true, __VA_ARGS__) } else { GS_SWITCH(FN, 256, false, __VA_ARGS__) } break; \
-        default: return hipErrorInvalidValue;                                             \
+// The same for the kernels that take rows of d_real elements, a multiple of 8: without a selection the kernel of the next
+// head_dim of 64, 80, 96, 128 reads and writes such rows where they lie (80: five k-steps instead of six for the S and dP of
+// 72- and 80-wide vision heads)
+static inline int dense_kernel_dim(int d_real) { return d_real <= 64 ? 64 : d_real <= 80 ? 80 : d_real <= 96 ? 96 : d_real <= 128 ? 128 : d_real; }
+#define TILE_SWITCH_DENSE(FN, ...)                                                        \
+    hipError_t launch_status = hipErrorInvalidValue;                                      \
+    if (bitmap) switch (d_real) {                                                         \
+        case 64: GS_SWITCH(FN, 64, true, __VA_ARGS__) break;                              \
+        case 128: GS_SWITCH(FN, 128, true, __VA_ARGS__) break;                            \
+        case 256: GS_SWITCH(FN, 256, true, __VA_ARGS__) break;                            \
+    } else switch (dense_kernel_dim(d_real)) {                                            \
+        case 64: GS_SWITCH(FN, 64, false, __VA_ARGS__) break;                             \
+        case 80: GS_SWITCH(FN, 80, false, __VA_ARGS__) break;                             \
+        case 96: GS_SWITCH(FN, 96, false, __VA_ARGS__) break;                             \
+        case 128: GS_SWITCH(FN, 128, false, __VA_ARGS__) break;                           \
+        case 256: GS_SWITCH(FN, 256, false, __VA_ARGS__) break;                           \
     }                                                                                     \
     if (launch_status != hipSuccess) return launch_status;
 
@@ -2002,13 +2013,13 @@ extern "C" hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_id
 }
 extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,
                                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
-                                         const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale,
+                                         const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
                                          int pos_split, int causal, void *dq, const void *out_for_delta, float *delta_out,
                                          hipStream_t stream) {
     // out_for_delta != null: the kernel forms delta = rowsum(dO * O) of its rows itself and writes it to delta_out
     const int gs = group_shift(Hq, Hkv);
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * tile_waves_of(D)) >> gs) + N + 1) * Hkv));
-    TILE_SWITCH_96(launch_dq_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, pos_split, causal, dq, out_for_delta, delta_out)
+    const dim3 grid((unsigned)(((int64_t)T / ((32 * tile_waves_of(d_real)) >> gs) + N + 1) * Hkv));
+    TILE_SWITCH_DENSE(launch_dq_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out)
     return hipGetLastError();
 }
 // bytes of fp32 partial sums a launch of T tokens may use for key-tile walks in pieces (0: launches of this size are
@@ -2020,17 +2031,18 @@ extern "C" size_t dsa_tile_dkv_partial_bytes(int T) {
 }
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
-                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int causal,
+                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal,
                                           int32_t *order, float *partial, size_t partial_bytes, void *dk, void *dv,
                                           hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
+    const int pitch = bitmap ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;      // row of a partial sum
     const int tiles_ub = T / 128 + N;                    // 128-key tiles of all segments, at most
     dim3 grid((unsigned)((tiles_ub + 1) * Hkv));
     // `order` (dsa_tile_order_bytes(T) bytes, or null): the tiles are listed longest walk first before the launch.
     // A launch of at most four workgroups per CU may also cut long walks into pieces (`partial`: fp32 partial sums), so
     // that it does not end on a few long walks with most of the chip idle.
-    const int wg_per_tile = Hkv * (D > 128 ? 2 : 1);
-    const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * D * sizeof(float))) : 0;
+    const int wg_per_tile = Hkv * (d_real > 128 ? 2 : 1);
+    const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * pitch * sizeof(float))) : 0;
     const bool pieces = order && causal && slot_pairs >= Hkv && (int64_t)tiles_ub * wg_per_tile <= 4 * 256;
     int item_cap = 0;
     if (order && (N > 1 || pieces)) {
@@ -2044,10 +2056,10 @@ extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const
         order = nullptr;                                 // one segment: its tiles are in order already
     }
     if (!pieces) partial = nullptr;
-    TILE_SWITCH_96(launch_dkv_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, causal, order, partial, dk, dv)
+    TILE_SWITCH_DENSE(launch_dkv_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv)
     if (pieces)
         hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(tiles_ub, Hkv, DSA_PIECES_Z), dim3(256), 0, stream, order,
-                           order_entries_cap(T), partial, cu, N, Hkv, D, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
+                           order_entries_cap(T), partial, cu, N, Hkv, d_real, pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
                            (bf16_t *)dk, (bf16_t *)dv);
     return hipGetLastError();
 }

@@ -122,7 +122,10 @@ void attn_forward_kernels(const Tensor &q, const Tensor &k, const Tensor &v, con
     const int T = (int)q.size(0), Hq = (int)q.size(1), D = (int)q.size(2), Hkv = (int)k.size(1), N = (int)cu.numel() - 1;
     const int K = idx.defined() ? (int)idx.size(1) : 0;
     const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-    if (bitmap_ready)
+    if (!idx.defined() && D % 64)                        // rows between the kernels' head_dims, read where they lie
+        check(dsa_dense_fwd_strided(ptr(q), q.stride(0), D, ptr(k), k.stride(0), D, ptr(v), v.stride(0), D, iptr(cu), T, N, Hq, Hkv, D, (float)a.scale,
+                                    DSA_DTYPE_BF16, (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
+    else if (bitmap_ready)
         check(dsa_attn_fwd_saved_bitmap(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, DSA_DTYPE_BF16,
                                         (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd_saved_bitmap");
     else
@@ -229,7 +232,12 @@ public:
             db = as_bf16(g);
         }
         Tensor dq = empty({T, Hq, D}, at::kBFloat16, q), dk = empty({T, Hkv, D}, at::kBFloat16, q), dv = empty({T, Hkv, D}, at::kBFloat16, q);
-        if (ws.defined() || !idx.defined()) {                               // the forward's bitmap is read where it lies
+        if (!idx.defined() && D % 64) {
+            const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
+            const Tensor scratch = empty_bytes(sc_bytes, q);
+            check(dsa_dense_bwd_rows(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(cu), T, N, Hq, Hkv, D, (float)scale, DSA_DTYPE_BF16,
+                                     max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(scratch), sc_bytes, stream_of(q)), "dsa_dense_bwd_rows");
+        } else if (ws.defined() || !idx.defined()) {                               // the forward's bitmap is read where it lies
             const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
             const Tensor scratch = empty_bytes(sc_bytes, q);
             check(dsa_attn_bwd_saved_bitmap(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K,
@@ -280,6 +288,7 @@ Qkv checked_qkv(const Tensor &q, const Tensor &k, const Tensor &v) {
     return s;
 }
 
+bool aligned16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
 // q, k and v can go to the dense forward as they lie in memory: no transposing copy, no padding of the head_dim
 bool readable_in_place(const Tensor &t) {
     return t.scalar_type() == at::kBFloat16 && t.stride(2) == 1 && t.size(2) % 8 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
@@ -329,6 +338,8 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
     Tensor q = q_, k = k_, v = v_;
     if (!sparse && !needs_grad(q, k, v) && readable_in_place(q) && readable_in_place(k) && readable_in_place(v))
         return {dense_forward(q, k, v, cu, max_seqlen, scale, causal)};
+    // the tile kernels take rows of any multiple of 8 up to 128 where they lie (a selection's kernels do not)
+    if (!sparse && q.scalar_type() == at::kBFloat16 && sh.D <= 128 && sh.D % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(v)) d_kernel = sh.D;
     if (d_kernel != sh.D) {
         // zero columns change neither q.k nor the used part of p.v
         const int64_t pad = d_kernel - sh.D;

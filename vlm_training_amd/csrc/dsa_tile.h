@@ -12,8 +12,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // same chunk) and a transposed read (4 consecutive rows x 64 B) must each cover all banks once.  The
 // 64-byte skew per row separates 4 consecutive rows, the XOR of the chunk's two low bits with row bits
 // 2-3 separates rows 4 apart: both read patterns and the row-wise staging writes are conflict-free.
-// (The skew needs a pitch of 64 modulo 256 bytes: head_dim 96 pads its rows to the pitch of head_dim 128.)
-template <int D> constexpr int tile_pitch() { return D == 96 ? 320 : D * 2 + 64; }
+// (The skew needs a pitch of 64 modulo 256 bytes: head_dim 80 and 96 pad their rows to the pitch of head_dim 128.)
+template <int D> constexpr int tile_pitch() { return D == 96 || D == 80 ? 320 : D * 2 + 64; }
 template <int D> constexpr int tile_bytes() { return 32 * tile_pitch<D>(); }
 __device__ __forceinline__ int tile_sw(int row) { return (row >> 2) & 3; }
 template <int D>
@@ -199,14 +199,14 @@ __device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, i
                                              : locate_block(cu, N, slot, blk, true, s0, L, b))
 
 // ---- LDS tiles filled straight from memory ------------------------------------------------------------------------------
-// 32 rows of D bf16 (head_dim 96: of 128, the last quarter zero).  A load puts 1 KiB of one wave at consecutive addresses, so
+// 32 rows of D bf16 (head_dim 80 and 96: of 128, columns past the true head_dim zero).  A load puts 1 KiB of one wave at consecutive addresses, so
 // rows cannot be padded one by one; instead groups of rows (1 KiB at head_dim 64, four rows else) are 16 bytes apart, and the
 // 16-byte chunk c of row r sits at position c ^ x(r), x = 4 (r & 3) (head_dim 64: 4 (bit 1 of r) + 2 (bit 2)): sixteen
 // consecutive rows at one chunk (row-wise operand) and four consecutive rows at four neighbouring chunks (transposed operand,
 // 32 lanes) each cover the 64 banks once.  The XOR is applied to the source address of a load.
 template <int D>
 struct DirectTile {
-    static constexpr int ROW_B = D == 96 ? 256 : 2 * D;                  // bytes per row
+    static constexpr int ROW_B = D == 96 || D == 80 ? 256 : 2 * D;                  // bytes per row
     static constexpr int CPR = ROW_B / 16;                               // chunks per row
     static constexpr int GROUP = D == 64 ? 8 : 4;                        // rows between two gaps
     static constexpr int GROUP_B = GROUP * ROW_B + 16;

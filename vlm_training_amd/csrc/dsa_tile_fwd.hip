@@ -32,7 +32,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int causal,
     bf16_t *__restrict__ out, float *__restrict__ lse) {
     typedef DirectTile<D> TL;
-    constexpr int KS = D / 16, DT = D / 32;
+    constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;   // MFMAs of S, of P V (head_dim 80: five and six)
+    static_assert(KS <= NP);
     constexpr int LPW = (TL::LOADS + NW - 1) / NW;          // wave loads per wave, step and operand
     constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);        // everything a wave requests in a step
     static_assert(TL::LOADS % NW == 0, "every wave loads the same number of pieces");
@@ -203,13 +204,15 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     }
     __syncthreads();                                    // every wave is done with K(0) and K(1): their slots may be filled again
     load_k(4);
-    constexpr int AHEAD = KS % 4 ? 3 : 4;               // (divides KS: an operand keeps its register from step to step)
-    static_assert(KS % AHEAD == 0);
-    bf16x8 kr[AHEAD], vr[AHEAD];                        // operands of the next MFMA pairs
+    constexpr int KA = KS % 5 == 0 ? 5 : KS % 4 ? 3 : 4, VA = NP % 4 ? 3 : 4;   // (divide KS and NP: an operand keeps its register from step to step)
+    static_assert(KS % KA == 0 && NP % VA == 0);
+    bf16x8 kr[KA], vr[VA];                              // operands of the next MFMA pairs
     k_addr(2);
     v_addr(0);
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i) { kr[i] = read_k(i); vr[i] = read_v(i); }
+    for (int i = 0; i < KA; ++i) kr[i] = read_k(i);
+#pragma unroll
+    for (int i = 0; i < VA; ++i) vr[i] = read_v(i);
     uint32_t word_next = word_of(1);                    // (one-tile blocks never use it)
 
     // piece r of what step t requests: K(t+5), V(t+3) and the selection words of tile t+4
@@ -231,7 +234,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         // The softmax of an element is a chain of dependent instructions (mask, scale, exponential, sum, pack) and a wave
         // issues in order: behind each MFMA stand the first part of one element's chain, the exponential of the element before
         // and the sum of the one before that, so that no instruction waits for the one in front of it.
-        constexpr int H = 2 * KS - 2;                   // half-steps an element can start in
+        constexpr int H = 2 * NP - 2;                   // half-steps an element can start in
         float y[16], e[16];
         auto behind = [&](int hs) __attribute__((always_inline)) {
 #pragma unroll
@@ -259,21 +262,21 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            oacc[i % DT] = mfma32(vr[i % AHEAD], i < DT ? pB0 : pB1, oacc[i % DT]);
+        for (int i = 0; i < NP; ++i) {
+            oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
             // this step's requests, spread over its first half: one after the other they would queue for the way into LDS
 #pragma unroll
             for (int r_ = 0; r_ < LPS; ++r_)
-                if (REQ && r_ * (KS / 2) / LPS == i) request(t_, r_);
-            // refill: the operand AHEAD pairs on, of this step's tiles or, past their end, of the next step's
-            if (i == KS - AHEAD && SM) v_addr(t_ + 1);
-            if (i + AHEAD < KS || SM) vr[i % AHEAD] = read_v((i + AHEAD) % KS);
+                if (REQ && r_ * (NP / 2) / LPS == i) request(t_, r_);
+            // refill: the operand a few pairs on, of this step's tiles or, past their end, of the next step's
+            if (i == NP - VA && SM) v_addr(t_ + 1);
+            if (i + VA < NP || SM) vr[i % VA] = read_v((i + VA) % NP);
             if (SM) behind(2 * i);
             else __builtin_amdgcn_sched_barrier(0);
-            if (NEXT) {
-                snew = mfma32(kr[i % AHEAD], qB[i], i == 0 ? zero16() : snew);
-                if (i == KS - AHEAD) k_addr(t_ + 3);
-                kr[i % AHEAD] = read_k((i + AHEAD) % KS);
+            if (NEXT && i < KS) {
+                snew = mfma32(kr[i % KA], qB[i], i == 0 ? zero16() : snew);
+                if (i == KS - KA) k_addr(t_ + 3);
+                kr[i % KA] = read_k((i + KA) % KS);
                 if (i == 0 && MASKED) word_next = word_of(t_ + 2);
             }
             if (SM) behind(2 * i + 1);
@@ -362,10 +365,10 @@ template <int D, bool HAS_IDX>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
                                void *out, float *lse) {
-    // At head_dim 96 and 128 eight waves share each staged tile - except in launches of a few rounds of workgroups, which
+    // At head_dim 80 to 128 eight waves share each staged tile - except in launches of a few rounds of workgroups, which
     // are bound by what a workgroup pays before its first tile and after its last: there two four-wave workgroups per CU
     // overlap those parts.
-    if constexpr (D == 128 || D == 96) {
+    if constexpr (D > 64 && D <= 128) {
         const int64_t blocks = ((int64_t)T / ((32 * 8) >> gshift) + N + 1) * Hkv;
         if (blocks > DSA_BATCH_ORDER_MAX_BLOCKS)
             return launch_fwd_n<D, HAS_IDX, 8>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
@@ -373,8 +376,8 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     return launch_fwd_n<D, HAS_IDX, 4>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
 }
 
-// d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 96, 128, 256 runs it; 96 without a
-// bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
+// d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
+// without a bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
 extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
                                           int pos_split, int causal, void *out, float *lse, hipStream_t stream) {
@@ -389,6 +392,7 @@ extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const vo
         else if (d_real <= 256) FWD_CASE(256, true);
     } else {
         if (d_real <= 64) FWD_CASE(64, false);
+        else if (d_real <= 80) FWD_CASE(80, false);
         else if (d_real <= 96) FWD_CASE(96, false);
         else if (d_real <= 128) FWD_CASE(128, false);
         else if (d_real <= 256) FWD_CASE(256, false);
