@@ -123,6 +123,11 @@ int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, con
                     const float *dscore, const int32_t *cu_seqlens, int T, int N, int Hi, int Di, int K, float scale,
                     int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
                     void *stream);
+/* The same with every gradient multiplied by *grad (one fp32 on the device: the gradient of the loss; null: 1). */
+int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
+                           const float *dscore, const float *grad, const int32_t *cu_seqlens, int T, int N, int Hi, int Di, int K,
+                           float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
+                           void *stream);
 size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen);
 
 /*

@@ -27,8 +27,8 @@ hipError_t dsa_launch_gather_dq(const void *dout, const void *q, const void *k, 
                                 const float *delta, const int32_t *idx, const int32_t *n, const int32_t *cu, int N,
                                 int T, int Hq, int Hkv, int D, int K, float scale, int pos_min, void *dq,
                                 hipStream_t stream);
-hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore,
-                                  const uint32_t *bitmap, int32_t *prefix, int ldw, const int32_t *cu, int N, int T, int Hi,
+hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore, const float *grad,
+                                  const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N, int T, int Hi,
                                   int Di, int K, float cscale, void *dq_idx, void *dk_idx, float *dw, float *partial,
                                   hipStream_t stream, hipStream_t stream_q);
 size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw);
@@ -443,14 +443,14 @@ static OverlapCtx *overlap_ctx(hipStream_t main_stream) {
 // ---- indexer backward: gradients of the selected scores w.r.t. the indexer's inputs --------------------
 extern "C" size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen) {
     if (T <= 0) return 0;
-    const int ldw = bitmap_ldw(max_seqlen);                    // selection bitmap + slot prefix table + partial dk sums
-    return 2 * align_up((size_t)T * ldw * 4, 256) + align_up(dsa_indexer_bwd_partial_bytes(T, Di, ldw), 256);
+    const int ldw = bitmap_ldw(max_seqlen);                    // selection bitmap + slot prefix table + partial dk sums + fp32 head weights
+    return 2 * align_up((size_t)T * ldw * 4, 256) + align_up(dsa_indexer_bwd_partial_bytes(T, Di, ldw), 256) + (size_t)T * 64 * 4;
 }
 
-extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
-                               const float *dscore, const int32_t *cu, int T, int N, int Hi, int Di, int K, float scale,
-                               int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
-                               void *stream) {
+extern "C" int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
+                                      const float *dscore, const float *grad, const int32_t *cu, int T, int N, int Hi, int Di, int K,
+                                      float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws,
+                                      size_t ws_bytes, void *stream) {
     if (int rc = check_packed(T, N, cu)) return rc;
     if (dtype != DSA_DTYPE_BF16) return fail(DSA_ERR_UNSUPPORTED, "indexer tensors must be bf16 (dtype code %d)", dtype);
     if (Hi < 1 || Hi > 64) return fail(DSA_ERR_UNSUPPORTED, "Hi=%d: 1..64 indexer heads", Hi);
@@ -468,6 +468,7 @@ extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void 
     uint32_t *bitmap = (uint32_t *)ws;
     int32_t *prefix = (int32_t *)((char *)ws + bm);
     float *partial = (float *)((char *)ws + 2 * bm);
+    float *w_f32 = (float *)((char *)ws + need - (size_t)T * 64 * 4);
     hipError_t e = dsa_launch_bitmap(idx, n, cu, N, T, K, ldw, bitmap, st);
     if (e != hipSuccess) return hip_fail(e, "bitmap launch");
     // the query side (dq_idx, dw) and the key side (dk_idx) read the same inputs and write different outputs: side by
@@ -490,7 +491,7 @@ extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void 
         sq = ov->aux;
     }
     int rc = DSA_OK;
-    e = dsa_launch_indexer_bwd(q_idx, k_idx, w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, Di, K, scale, dq_idx, dk_idx, dw,
+    e = dsa_launch_indexer_bwd(q_idx, k_idx, w_idx, dscore, grad, bitmap, prefix, w_f32, ldw, cu, N, T, Hi, Di, K, scale, dq_idx, dk_idx, dw,
                                partial, st, sq);
     if (e != hipSuccess) rc = hip_fail(e, "indexer backward launch");
     if (ov) {
@@ -499,6 +500,14 @@ extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void 
         if (e != hipSuccess && rc == DSA_OK) rc = hip_fail(e, "join of the second stream");
     }
     return rc;
+}
+
+extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
+                               const float *dscore, const int32_t *cu, int T, int N, int Hi, int Di, int K, float scale,
+                               int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
+                               void *stream) {
+    return dsa_indexer_bwd_scaled(q_idx, k_idx, w_idx, idx, n, dscore, nullptr, cu, T, N, Hi, Di, K, scale, dtype, max_seqlen, dq_idx,
+                                  dk_idx, dw, ws, ws_bytes, stream);
 }
 
 extern "C" size_t dsa_attn_bwd_workspace_bytes(int T, int Hq, int max_seqlen, int has_idx) {

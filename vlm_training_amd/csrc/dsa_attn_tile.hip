@@ -1,5 +1,5 @@
-// Tile kernels: dQ / dK,dV, attention mass and indexer backward over 32x32 MFMA tiles with the selection applied
-// as a bitmap mask (the forward: dsa_tile_fwd.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
+// Tile kernels: dQ / dK,dV and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask (the forward:
+// dsa_tile_fwd.hip, the indexer backward: dsa_tile_idx.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
 // 4*G*D flop on the matrix cores - on MI355X the tile walk is cheaper down to a few percent density.
@@ -254,302 +254,6 @@ __global__ __launch_bounds__(256) void dsa_mass_reduce_kernel(const float *__res
                 for (int kvh = 0; kvh < Hkv; ++kvh) acc += partial[kvh * plane + row + jj];
             mass[row + jj] = acc * inv_hq;
         }
-    }
-}
-
-// ==================================================================================================
-// Indexer backward.  The indexer score of a selected pair is  I[t,s] = c * sum_h w[t,h] relu(r[t,h,s]),
-// r = q_idx[t,h,:] . k_idx[s,:]  (multi-query attention with ReLU in place of the softmax: Hi heads, one key
-// head).  Given dscore[t,j] = dLoss/dI at the selected keys (slot j of key s = its rank in the ascending
-// selection list = selected keys of earlier tiles + those below it in the tile's word):
-//     G[t,h,s]   = dscore[t,s] * w[t,h] * (r > 0)
-//     dq_idx[t,h,:] = c * sum_s G[t,h,s] k_idx[s,:]      dw[t,h] = c * sum_s dscore[t,s] relu(r[t,h,s])
-//     dk_idx[s,:]   = c * sum_t sum_h G[t,h,s] q_idx[t,h,:]
-// Query side = the dQ walk (rows = (query, indexer head), padded to 32 or 64 rows per query so that the 32
-// rows of a wave belong to one query): S^T = K Q^T, G^T on the C layout, dQ^T += K^T G^T.  Key side = the
-// key-stationary walk: a wave owns 32 keys (rows in registers) and walks the later queries in blocks of
-// 32 heads of one query: S = Q K^T, G on the C layout, dK^T += Q^T G.  Every output row is reduced by one
-// wave in a fixed order: deterministic, no atomics.
-// ==================================================================================================
-template <int D, int GSHIFT, int NW>
-__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_idxq_kernel(
-    const bf16_t *__restrict__ q_idx, const bf16_t *__restrict__ k_idx, const bf16_t *__restrict__ w_idx,
-    const float *__restrict__ dscore, const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N,
-    int T, int Hi, int K, float cscale, bf16_t *__restrict__ dq_idx, float *__restrict__ dw) {
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>(), LOADS = 32 * CPR / (NW * 64);
-    constexpr int NBUF = 2, NT = NW * 64, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT;
-    static_assert(LOADS >= 1 && GSHIFT >= 5, "a wave's 32 rows are heads of one query");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][TILE_B];
-    __shared__ __attribute__((aligned(16))) float dl_s[NW][32];      // per wave: the gradients of the current tile's 32 keys
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x, QBW, s0, L, blk)) return;
-    L = min(L, ldw * 32);
-    const int qc0 = blk * QBW;
-    if (qc0 >= L) return;
-    const int r = wv * 32 + j;
-    const int qcol = qc0 + (r >> GSHIFT), head = r & (Gp - 1);
-    const bool row_ok = qcol < L && head < Hi;
-    const int t = s0 + min(qcol, L - 1), hrow = min(head, Hi - 1);
-    u32x4 kst[2][LOADS];
-#define IDXQ_LOAD(SET, TILE)                                                                        \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                            \
-        const int c = i * NT + tid;                                                                \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        kst[SET][i] = *reinterpret_cast<const u32x4 *>(k_idx + (int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * D + ch * 8); \
-    }
-    IDXQ_LOAD(0, 0)
-    bf16x8 qB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-        qB[ks] = row_ok ? load_bf16x8(q_idx + ((int64_t)t * Hi + hrow) * D + 16 * ks + 8 * h) : zero_bf16x8();
-    const float wrow_v = row_ok ? (float)w_idx[(int64_t)t * Hi + hrow] : 0.f;
-    const int ntiles = min(qc0 + QBW - 1, L - 1) / 32 + 1;
-    const uint32_t *wrow = bitmap + (int64_t)t * ldw;
-    const float *drow = dscore + (int64_t)t * K;
-    // selection words run two tiles ahead of the compute and the gradients of a tile's keys one tile ahead: lane j
-    // fetches the gradient of key column j of the next tile (both halves of the wave the same)
-    uint32_t word_cur = qcol < L ? wrow[0] : 0u, word_nx = qcol < L ? wrow[min(1, ntiles - 1)] : 0u;
-    int seen = 0;
-    auto fetch_dl = [&](uint32_t word, int before) {
-        return drow[min(before + (int)__popc(word & ((1u << j) - 1u)), K - 1)];
-    };
-    float dl_nx = fetch_dl(word_cur, 0);
-    f32x16 acc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = zero16();
-    float dwacc = 0.f;
-
-#define IDXQ_STORE(SET, BUF, TILE)                                                                  \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                            \
-        const int c = i * NT + tid;                                                                \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        *reinterpret_cast<u32x4 *>(&lds[BUF][tile_off<D>(row, ch)]) = kst[SET][i];                 \
-    }
-#define IDXQ_COMPUTE(TILE, BUF)                                                                     \
-    {                                                                                              \
-        const unsigned char *kt = lds[BUF];                                                        \
-        const uint32_t word_full = word_cur;                                                       \
-        const float dl = ((word_full >> j) & 1u) ? dl_nx : 0.f;                                    \
-        seen += __popc(word_full);                                                                 \
-        word_cur = word_nx;                                                                        \
-        dl_nx = fetch_dl(word_cur, seen);                /* for the next tile */                   \
-        { const uint32_t wl = wrow[min((TILE) + 2, ntiles - 1)]; word_nx = qcol < L ? wl : 0u; }   \
-        f32x16 sacc = zero16();                                                                    \
-        {                                                                                          \
-            bf16x8 ka[KS];                                                                         \
-            _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) ka[ks] = lo.rowop(kt, ks);           \
-            _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) sacc = mfma32(ka[ks], qB[ks], sacc); \
-            sched_reads_ahead<KS, 4, 1>();                                                         \
-        }                                                                                          \
-        /* the wave's 32 gradients go through its own 128 bytes of LDS: one write and four 16-byte reads per lane     \
-           (element vi is key column 8*(vi/4) + 4h + vi%4) instead of sixteen lane permutes */      \
-        if (h == 0) dl_s[wv][j] = dl;                                                              \
-        float ds[16];                                                                              \
-        _Pragma("unroll") for (int g4 = 0; g4 < 4; ++g4) {                                         \
-            const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&dl_s[wv][8 * g4 + 4 * h]);          \
-            _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                        \
-                const float sv = sacc[4 * g4 + e];       /* the row's weight multiplies the finished sum instead */ \
-                ds[4 * g4 + e] = sv > 0.f ? d4[e] : 0.f;                                           \
-                dwacc = fmaf(ds[4 * g4 + e], sv, dwacc); /* dscore * relu(s) */                     \
-            }                                                                                      \
-        }                                                                                          \
-        const bf16x8 dB0 = pack8(ds), dB1 = pack8(ds + 8);                                         \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) {                                        \
-            mfma32_acc(acc[dt], lo.trop(kt, 0, dt), dB0);                                          \
-            mfma32_acc(acc[dt], lo.trop(kt, 1, dt), dB1);                                          \
-        }                                                                                          \
-        sched_reads_ahead<2 * DT, 3, 2>();                                                         \
-    }
-    TILE_PIPELINE(ntiles, IDXQ_LOAD, IDXQ_STORE, IDXQ_COMPUTE)
-#undef IDXQ_LOAD
-#undef IDXQ_STORE
-#undef IDXQ_COMPUTE
-
-    const float dwt = half_sum_f(dwacc);
-    if (row_ok) {
-        bf16_t *op = dq_idx + ((int64_t)t * Hi + hrow) * D;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, acc[dt], cscale * wrow_v, h);
-        if (h == 0) dw[(int64_t)t * Hi + hrow] = dwt * cscale;
-    }
-}
-
-// key side.  Workgroup = 4 waves x 32 keys = one 128-key tile of a segment; step b of its walk = all heads
-// (HB blocks of 32) of query L-1-b: from the end of the segment down to the tile, so that the workgroups of a
-// segment that run side by side read the same index-query rows at about the same time and share them in L2.
-template <int D, int GSHIFT>
-__global__ __launch_bounds__(256) void dsa_tile_idxk_kernel(
-    const bf16_t *__restrict__ q_idx, const bf16_t *__restrict__ k_idx, const bf16_t *__restrict__ w_idx,
-    const float *__restrict__ dscore, const uint32_t *__restrict__ bitmap, const int32_t *__restrict__ prefix, int ldw,
-    const int32_t *__restrict__ cu, int N, int T, int Hi, int K, float cscale, int chunk_steps,
-    float *__restrict__ partial) {
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NBUF = 2, HB = (1 << GSHIFT) / 32, LOADS = HB * 32 * CPR / 256;
-    static_assert(GSHIFT >= 5 && LOADS >= 1, "steps of 32*HB heads of one query");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][HB][TILE_B];
-    __shared__ __attribute__((aligned(16))) float w_s[NBUF][HB * 32];
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    int s0, L, blk;
-    if (!locate_block(cu, N, blockIdx.x, 128, false, s0, L, blk)) return;
-    L = min(L, ldw * 32);
-    if (blk * 128 >= L) return;
-    const int c0 = blk * 128, kc = c0 + wv * 32;
-    const int mykey = kc + j;
-    const bool key_ok = mykey < L;
-    const int64_t krow = (int64_t)s0 + min(mykey, L - 1);
-    const bool kw_ok = kc < L;                           // the word column of this wave's keys exists
-    const int kw = kw_ok ? kc >> 5 : 0;
-    bf16x8 kB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kB[ks] = load_bf16x8(k_idx + krow * D + 16 * ks + 8 * h);
-    f32x16 dkacc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) dkacc[dt] = zero16();
-    // queries L-1 down to c0 can have selected keys of this tile; the walk is cut into pieces of chunk_steps queries
-    // (blockIdx.y), each piece leaving a partial sum: a tile at the start of a long segment would otherwise be one
-    // long serial walk
-    const int st0 = blockIdx.y * chunk_steps, nsteps = min(L - c0 - st0, chunk_steps);
-    if (nsteps <= 0) return;
-
-    // selection word and slot base of (query of a step, this wave's key column): fetched two LOAD calls before the
-    // LOAD that forms the gradient's address from them (register set s serves the odd steps, set 1 the even ones)
-    const int last_step = nsteps - 1;
-    auto word_of = [&](int step, uint32_t &wq, int32_t &bq) {
-        const int64_t o = (int64_t)(s0 + L - 1 - st0 - min(step, last_step)) * ldw + kw;
-        wq = kw_ok ? bitmap[o] : 0u;
-        bq = prefix[o];
-    };
-    uint32_t wordp[2], word0;
-    int32_t basep[2], base0;
-    word_of(0, word0, base0);
-    word_of(1, wordp[0], basep[0]);
-    word_of(2, wordp[1], basep[1]);
-
-    u32x4 qst[2][LOADS];
-    float dl_st[2] = {0.f, 0.f}, dl_buf[NBUF] = {0.f, 0.f};
-    bool sel_st[2] = {false, false};
-    uint32_t w_st[2] = {0u, 0u};
-#define IDXK_LOAD(SET, STEP)                                                                        \
-    {                                                                                              \
-        const int rel = (STEP), qc = L - 1 - st0 - rel;                                            \
-        _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                        \
-            const int c = i * 256 + tid;                                                           \
-            const int row = c / CPR, ch = c % CPR;       /* row = head, padded to 32*HB */          \
-            qst[SET][i] = *reinterpret_cast<const u32x4 *>(q_idx + ((int64_t)(s0 + qc) * Hi + min(row, Hi - 1)) * D + ch * 8); \
-        }                                                                                          \
-        w_st[SET] = reinterpret_cast<const unsigned short *>(w_idx)[(int64_t)(s0 + qc) * Hi + min(tid & (32 * HB - 1), Hi - 1)]; \
-        const uint32_t word = wordp[SET];                                                          \
-        const int base = basep[SET];                                                               \
-        word_of(rel + 2, wordp[SET], basep[SET]);        /* for this register set's next step */    \
-        sel_st[SET] = (word >> j) & 1u;                                                            \
-        dl_st[SET] = dscore[(int64_t)(s0 + qc) * K + min(base + (int)__popc(word & ((1u << j) - 1u)), K - 1)]; \
-    }
-#define IDXK_STORE(SET, BUF, STEP)                                                                  \
-    {                                                                                              \
-        const u32x4 z4 = {0u, 0u, 0u, 0u};                                                         \
-        _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                        \
-            const int c = i * 256 + tid;                                                           \
-            const int row = c / CPR, ch = c % CPR;                                                 \
-            /* padded heads are zeroed: they add nothing to dK */                                   \
-            *reinterpret_cast<u32x4 *>(&lds[BUF][row >> 5][tile_off<D>(row & 31, ch)]) = row < Hi ? qst[SET][i] : z4; \
-        }                                                                                          \
-        if (tid < 32 * HB) w_s[BUF][tid] = tid < Hi ? __uint_as_float(w_st[SET] << 16) : 0.f;       \
-        dl_buf[BUF] = sel_st[SET] ? dl_st[SET] : 0.f;                                              \
-    }
-#define IDXK_COMPUTE(STEP, BUF)                                                                     \
-    {                                                                                              \
-        const float dl = dl_buf[BUF];                    /* gradient of (query of the step, this lane's key) */ \
-        _Pragma("unroll") for (int hb = 0; hb < HB; ++hb) {                                        \
-            const unsigned char *qt = lds[BUF][hb];                                                \
-            f32x16 sacc = zero16();                                                                \
-            {                                                                                      \
-                bf16x8 qa[KS];                                                                     \
-                _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) qa[ks] = lo.rowop(qt, ks);       \
-                _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) sacc = mfma32(qa[ks], kB[ks], sacc); \
-            }                                                                                      \
-            float gs[16];                                                                          \
-            _Pragma("unroll") for (int g4 = 0; g4 < 4; ++g4) {                                     \
-                const f32x4 w4 = *reinterpret_cast<const f32x4 *>(&w_s[BUF][hb * 32 + 8 * g4 + 4 * h]); \
-                _Pragma("unroll") for (int e = 0; e < 4; ++e) gs[4 * g4 + e] = sacc[4 * g4 + e] > 0.f ? dl * w4[e] : 0.f; \
-            }                                                                                      \
-            const bf16x8 gB0 = pack8(gs), gB1 = pack8(gs + 8);                                     \
-            _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) {                                    \
-                mfma32_acc(dkacc[dt], lo.trop(qt, 0, dt), gB0);                                    \
-                mfma32_acc(dkacc[dt], lo.trop(qt, 1, dt), gB1);                                    \
-            }                                                                                      \
-        }                                                                                          \
-    }
-    {                                                    // step 0 into register set 0, with the words fetched above
-        const uint32_t w1 = wordp[0];
-        const int32_t b1 = basep[0];
-        wordp[0] = word0;
-        basep[0] = base0;
-        IDXK_LOAD(0, -2 + 2)                             /* consumes (word0, base0); its own prefetch is overwritten below */
-        wordp[0] = w1;
-        basep[0] = b1;
-    }
-    TILE_PIPELINE(nsteps, IDXK_LOAD, IDXK_STORE, IDXK_COMPUTE)
-#undef IDXK_LOAD
-#undef IDXK_STORE
-#undef IDXK_COMPUTE
-
-    if (key_ok) {
-        float *pk = partial + ((int64_t)blockIdx.y * T + krow) * D + 4 * h;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const f32x4 o4 = {dkacc[dt][4 * g4] * cscale, dkacc[dt][4 * g4 + 1] * cscale, dkacc[dt][4 * g4 + 2] * cscale,
-                                  dkacc[dt][4 * g4 + 3] * cscale};
-                *reinterpret_cast<f32x4 *>(pk + dt * 32 + 8 * g4) = o4;
-            }
-    }
-}
-
-// dk_idx[s,:] = sum of the partial sums of the pieces of its tile's walk, in piece order
-__global__ __launch_bounds__(256) void dsa_idxk_reduce_kernel(const float *__restrict__ partial,
-                                                               const int32_t *__restrict__ cu, int N, int T, int D,
-                                                               int chunk_steps, int max_cols, bf16_t *__restrict__ dk_idx) {
-    const int s = blockIdx.x * (256 / 32) + (threadIdx.x >> 5), c4 = (threadIdx.x & 31) * 4;   // 32 threads x 4 columns per pass
-    if (s >= T) return;
-    const int seg = find_segment(cu, N, s);
-    const int s0 = cu[seg], L = min(cu[seg + 1] - s0, max_cols);     // as the walk: no column past the bitmap row
-    const int c0 = ((s - s0) >> 7) << 7;
-    if (c0 >= L) return;
-    const int pieces = (L - c0 + chunk_steps - 1) / chunk_steps;
-    for (int c = c4; c < D; c += 128) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int pc = 0; pc < pieces; ++pc) acc += *reinterpret_cast<const f32x4 *>(partial + ((int64_t)pc * T + s) * D + c);
-        const u32x2 o = {pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3])};
-        *reinterpret_cast<u32x2 *>(dk_idx + (int64_t)s * D + c) = o;
-    }
-}
-
-// prefix[t][w] = selected keys of query t in the words before w (the slot of the first selected key of word w)
-__global__ __launch_bounds__(64) void dsa_bitmap_prefix_kernel(const uint32_t *__restrict__ bitmap, int ldw,
-                                                                int32_t *__restrict__ prefix) {
-    const int lane = threadIdx.x;
-    const uint32_t *row = bitmap + (int64_t)blockIdx.x * ldw;
-    int32_t *orow = prefix + (int64_t)blockIdx.x * ldw;
-    int carry = 0;
-    for (int w0 = 0; w0 < ldw; w0 += 64) {
-        const int w = w0 + lane;
-        const int c = w < ldw ? (int)__popc(row[w]) : 0;
-        int incl = c;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int u = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += u;
-        }
-        if (w < ldw) orow[w] = carry + incl - c;
-        carry += __shfl(incl, 63, 64);
     }
 }
 
@@ -1961,54 +1665,6 @@ extern "C" hipError_t dsa_launch_tile_mass(const void *q, const void *k, const f
     const unsigned parts = (unsigned)((K / 4 + 255) / 256 > 0 ? (K / 4 + 255) / 256 : 1);
     hipLaunchKernelGGL(dsa_mass_reduce_kernel, dim3(T, parts < 8 ? parts : 8), dim3(256), 0, stream, partial, n, T, K, ngroups,
                        inv_hq, mass);
-    return hipGetLastError();
-}
-// indexer backward: prefix table, query side (dq_idx, dw), key side (dk_idx).  D = indexer head_dim (64 or 128),
-// at most 64 indexer heads.
-// Queries per piece of a key tile's walk in the indexer backward.  A piece is one workgroup and about 1.3 us per query:
-// the finer the pieces, the better a launch of few thousand of them balances over 512 workgroup slots (32 768 tokens:
-// 6.26 -> 5.95 ms with 256 instead of 512, 6.31 with 128; 8192 tokens: 0.44 -> 0.31 -> 0.25 ms), the more fp32 partial
-// sums (one (T, Di) plane per piece index).  Depends on T, and on the bound of the longest segment only where the
-// planes would pass 1.25 GiB.
-static int idxk_chunk(int T, int Di, int ldw) {
-    int c = T <= 16384 ? 128 : 256;
-    while ((size_t)((ldw * 32 + c - 1) / c) * T * Di * 4 > ((size_t)5 << 28) && c < (1 << 20)) c *= 2;
-    return c;
-}
-template <int D, int GS>
-static void launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore,
-                             const uint32_t *bitmap, const int32_t *prefix, int ldw, const int32_t *cu, int N, int T, int Hi,
-                             int K, float cscale, void *dq_idx, void *dk_idx, float *dw, float *partial, hipStream_t stream_q) {
-    constexpr int NW = tile_waves<D>();
-    // (the key side, the longer pass, is issued first: with two streams it gets the GPU first)
-    const int chunk = idxk_chunk(T, D, ldw);
-    const dim3 gk((unsigned)((int64_t)T / 128 + N + 1), (unsigned)((ldw * 32 + chunk - 1) / chunk));
-    hipLaunchKernelGGL((dsa_tile_idxk_kernel<D, GS>), gk, dim3(256), 0, stream, (const bf16_t *)q_idx, (const bf16_t *)k_idx,
-                       (const bf16_t *)w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, chunk, partial);
-    hipLaunchKernelGGL(dsa_idxk_reduce_kernel, dim3((unsigned)((T + 7) / 8)), dim3(256), 0, stream, partial, cu, N, T, D,
-                       chunk, ldw * 32, (bf16_t *)dk_idx);
-    const dim3 gq((unsigned)((int64_t)T / ((32 * NW) >> GS) + N + 1));
-    hipLaunchKernelGGL((dsa_tile_idxq_kernel<D, GS, NW>), gq, dim3(64 * NW), 0, stream_q, (const bf16_t *)q_idx,
-                       (const bf16_t *)k_idx, (const bf16_t *)w_idx, dscore, bitmap, ldw, cu, N, T, Hi, K, cscale,
-                       (bf16_t *)dq_idx, dw);
-}
-extern "C" size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw) {
-    const int chunk = idxk_chunk(T, Di, ldw);
-    return (size_t)((ldw * 32 + chunk - 1) / chunk) * T * Di * 4;
-}
-extern "C" hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore,
-                                             const uint32_t *bitmap, int32_t *prefix, int ldw, const int32_t *cu, int N,
-                                             int T, int Hi, int Di, int K, float cscale, void *dq_idx, void *dk_idx,
-                                             float *dw, float *partial, hipStream_t stream, hipStream_t stream_q) {
-    if (Hi < 1 || Hi > 64 || !(Di == 64 || Di == 128)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(dsa_bitmap_prefix_kernel, dim3(T), dim3(64), 0, stream, bitmap, ldw, prefix);
-    if (Di == 128) {
-        if (Hi > 32) launch_idx_bwd_i<128, 6>(stream, q_idx, k_idx, w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, dq_idx, dk_idx, dw, partial, stream_q);
-        else launch_idx_bwd_i<128, 5>(stream, q_idx, k_idx, w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, dq_idx, dk_idx, dw, partial, stream_q);
-    } else {
-        if (Hi > 32) launch_idx_bwd_i<64, 6>(stream, q_idx, k_idx, w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, dq_idx, dk_idx, dw, partial, stream_q);
-        else launch_idx_bwd_i<64, 5>(stream, q_idx, k_idx, w_idx, dscore, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, dq_idx, dk_idx, dw, partial, stream_q);
-    }
     return hipGetLastError();
 }
 extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,

@@ -358,7 +358,7 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
 // ---- the indexer's training loss ---------------------------------------------------------------------------------
 struct IndexerGrads { Tensor dq, dk, dw; };
 IndexerGrads indexer_bwd(const Tensor &q_idx, const Tensor &k_idx, const Tensor &w_idx, const Tensor &idx, const Tensor &n, const Tensor &dscore_,
-                         const Tensor &cu, int64_t max_seqlen, std::optional<double> index_scale) {
+                         const Tensor &grad, const Tensor &cu, int64_t max_seqlen, std::optional<double> index_scale) {
     const int64_t T = q_idx.size(0), Hi = q_idx.size(1), Di = q_idx.size(2), K = idx.size(1);
     const double scale = index_scale_of(index_scale, Hi, Di);
     IndexInputs in = index_inputs(q_idx, k_idx, w_idx);
@@ -371,9 +371,9 @@ IndexerGrads indexer_bwd(const Tensor &q_idx, const Tensor &k_idx, const Tensor 
     IndexerGrads g{empty({T, Hi, d_kernel}, at::kBFloat16, in.q), empty({T, d_kernel}, at::kBFloat16, in.q), empty({T, Hi}, at::kFloat, in.q)};
     const size_t ws_bytes = dsa_indexer_bwd_workspace_bytes((int)T, (int)d_kernel, (int)max_seqlen);
     const Tensor ws = empty_bytes(ws_bytes, in.q);
-    check(dsa_indexer_bwd(ptr(in.q), ptr(in.k), ptr(in.w), iptr(idx), iptr(n), fptr(dscore), iptr(cu), (int)T, (int)cu.numel() - 1, (int)Hi,
+    check(dsa_indexer_bwd_scaled(ptr(in.q), ptr(in.k), ptr(in.w), iptr(idx), iptr(n), fptr(dscore), fptr(grad), iptr(cu), (int)T, (int)cu.numel() - 1, (int)Hi,
                           (int)d_kernel, (int)K, (float)scale, DSA_DTYPE_BF16, (int)max_seqlen, ptr(g.dq), ptr(g.dk), fptr(g.dw), ptr(ws), ws_bytes,
-                          stream_of(in.q)), "dsa_indexer_bwd");
+                          stream_of(in.q)), "dsa_indexer_bwd_scaled");
     if (d_kernel != Di) {
         g.dq = g.dq.narrow(-1, 0, Di).contiguous();
         g.dk = g.dk.narrow(-1, 0, Di).contiguous();
@@ -411,8 +411,8 @@ public:
         std::optional<double> scale;
         const auto it = ctx->saved_data.find("s");
         if (it != ctx->saved_data.end()) scale = it->second.toDouble();
-        // the gradients are linear in dscore: scale the (T,K) table by the incoming gradient, not the three results
-        const IndexerGrads g = indexer_bwd(s[0], s[1], s[2], s[3], s[4], s[5] * grads[0].to(at::kFloat), s[6], ctx->saved_data["m"].toInt(), scale);
+        // the gradients are linear in dscore: the kernels multiply their sums by the incoming gradient
+        const IndexerGrads g = indexer_bwd(s[0], s[1], s[2], s[3], s[4], s[5], grads[0].to(at::kFloat).contiguous(), s[6], ctx->saved_data["m"].toInt(), scale);
         return {g.dq.to(s[0].scalar_type()), g.dk.to(s[1].scalar_type()), g.dw.to(s[2].scalar_type()), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(),
                 Tensor(), Tensor(), Tensor()};
     }

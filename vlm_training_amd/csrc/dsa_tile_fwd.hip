@@ -79,12 +79,12 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     };
     auto left = [&](int tile, int tok_b) __attribute__((always_inline)) { return max(min(Lend - tile * 32, 32), 0) * tok_b; };
     auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV], i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
+        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2, 0,
                           lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) next(kptr, k_step);
     };
     auto load_v_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV], i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
+        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2, 0,
                           lds0 + (4 + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) next(vptr, v_step);
     };
