@@ -307,11 +307,12 @@ int dsa_dense_bwd(const void *dout, const void *q, const void *k, const void *v,
  *   q_out (T,Hq,D), k_out (T,Hkv,D) bf16 contiguous;  q_rstd (T,Hq), k_rstd (T,Hkv) fp32: 1/rms of
  *   every row, kept for the backward pass.  D in {64, 128, 256}.
  * dsa_qk_norm_rope_bwd: gq, gk = gradients of q_out, k_out (same layout) -> dq_in, dk_in (strided like
- * the inputs, bf16) and dqw, dkw (D) fp32.  `ws` holds dsa_qk_norm_rope_bwd_workspace_bytes(T, D) bytes
+ * the inputs, bf16) and dqw, dkw (D) fp32 (bf16 with `norm_flags & DSA_NORM_GRAD_BF16`).  `ws` holds dsa_qk_norm_rope_bwd_workspace_bytes(T, D) bytes
  * of per-workgroup partial sums that are added up in a fixed order (no atomics, deterministic).
  */
 #define DSA_NORM_OFFSET 1      /* scale by 1 + w */
 #define DSA_NORM_WEIGHT_BF16 2 /* qw, kw point at bf16 */
+#define DSA_NORM_GRAD_BF16 4   /* backward: dqw, dkw point at bf16 */
 size_t dsa_qk_norm_rope_bwd_workspace_bytes(int T, int D);
 int dsa_qk_norm_rope_fwd(const void *q_in, int64_t q_tok_stride, int64_t q_head_stride, const void *k_in,
                          int64_t k_tok_stride, int64_t k_head_stride, const void *qw, const void *kw, float eps,

@@ -62,7 +62,7 @@ hipError_t dsa_launch_qk_norm_rope_bwd(const void *gq, const void *gk, const voi
                                        int w_bf16, float w_offset, const void *cosp, const void *sinp, int cs_f32, int R,
                                        const float *q_rstd, const float *k_rstd, int T, int Hq, int Hkv, int D, void *dq_in,
                                        int64_t dq_tok, int64_t dq_head, void *dk_in, int64_t dk_tok, int64_t dk_head,
-                                       float *dqw, float *dkw, float *part, hipStream_t stream);
+                                       void *dqw, void *dkw, int grad_bf16, float *part, hipStream_t stream);
 hipError_t dsa_launch_sigmoid_gate_fwd(const void *x, const void *gate, int64_t gate_tok, int64_t gate_head, int D, int H,
                                        int64_t rows, void *y, hipStream_t stream);
 hipError_t dsa_launch_split_stack(const float *x, int64_t rows, int D, int order, void *y, hipStream_t stream);
@@ -766,7 +766,7 @@ extern "C" int dsa_qk_norm_rope_bwd(const void *gq, const void *gk, const void *
     hipError_t e = dsa_launch_qk_norm_rope_bwd(gq, gk, q_in, q_tok, q_head, k_in, k_tok, k_head, qw, kw, (norm_flags & DSA_NORM_WEIGHT_BF16) != 0,
                                                (norm_flags & DSA_NORM_OFFSET) ? 1.f : 0.f,
                                                cosp, sinp, cs_dtype == DSA_DTYPE_FP32, R, q_rstd, k_rstd, T, Hq, Hkv, D, dq_in,
-                                               dq_tok, dq_head, dk_in, dk_tok, dk_head, dqw, dkw, (float *)ws,
+                                               dq_tok, dq_head, dk_in, dk_tok, dk_head, dqw, dkw, (norm_flags & DSA_NORM_GRAD_BF16) != 0, (float *)ws,
                                                (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "qk_norm_rope backward launch");
 }

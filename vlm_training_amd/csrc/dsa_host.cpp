@@ -481,15 +481,17 @@ public:
         auto grad_of = [&](const Tensor &g, int64_t H) { return g.defined() ? as_bf16(g) : at::zeros({T, H, D}, q.options()); };
         const Tensor gq = grad_of(grads[0], Hq), gk = grad_of(grads[1], Hkv);
         const Tensor dq = empty({T, Hq, D}, at::kBFloat16, q), dk = empty({T, Hkv, D}, at::kBFloat16, q);
-        const Tensor dqw = empty({D}, at::kFloat, q), dkw = empty({D}, at::kFloat, q);
+        const auto qt = (at::ScalarType)ctx->saved_data["q"].toInt(), kt = (at::ScalarType)ctx->saved_data["k"].toInt();
+        const bool wide = qt != at::kBFloat16 || kt != at::kBFloat16;          // two bf16 gradients come from the kernel as they are
+        const Tensor dqw = empty({D}, wide ? at::kFloat : at::kBFloat16, q), dkw = empty({D}, wide ? at::kFloat : at::kBFloat16, q);
         const size_t ws_bytes = dsa_qk_norm_rope_bwd_workspace_bytes((int)T, (int)D);
         const Tensor ws = empty_bytes(ws_bytes, q);
         const int cs_code = cs.scalar_type() == at::kBFloat16 ? DSA_DTYPE_BF16 : DSA_DTYPE_FP32;
         check(dsa_qk_norm_rope_bwd(ptr(gq), ptr(gk), ptr(q), q.stride(0), q.stride(1), ptr(k), k.stride(0), k.stride(1), ptr(qw), ptr(kw),
-                                   (int)ctx->saved_data["f"].toInt(), ptr(cs), ptr(sn), cs_code, (int)cs.size(1), fptr(qr), fptr(kr), (int)T, (int)Hq,
-                                   (int)Hkv, (int)D, ptr(dq), Hq * D, D, ptr(dk), Hkv * D, D, fptr(dqw), fptr(dkw), ptr(ws), ws_bytes, stream_of(q)),
+                                   (int)ctx->saved_data["f"].toInt() | (wide ? 0 : DSA_NORM_GRAD_BF16), ptr(cs), ptr(sn), cs_code, (int)cs.size(1), fptr(qr), fptr(kr), (int)T, (int)Hq,
+                                   (int)Hkv, (int)D, ptr(dq), Hq * D, D, ptr(dk), Hkv * D, D, (float *)ptr(dqw), (float *)ptr(dkw), ptr(ws), ws_bytes, stream_of(q)),
               "dsa_qk_norm_rope_bwd");
-        return {dq, dk, dqw.to((at::ScalarType)ctx->saved_data["q"].toInt()), dkw.to((at::ScalarType)ctx->saved_data["k"].toInt()), Tensor(), Tensor(),
+        return {dq, dk, dqw.to(qt), dkw.to(kt), Tensor(), Tensor(),
                 Tensor(), Tensor()};
     }
 };

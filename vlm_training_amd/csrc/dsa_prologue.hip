@@ -6,7 +6,11 @@
 // HBM-bound element-wise work with one reduction per (token, head) row: a row of D bf16 is spread over
 // D/8 lanes (16 bytes per lane), so a wave handles 512/D rows per step; the row reduction and the
 // rotate_half partner (R/16 lanes away) are cross-lane moves inside those D/8 lanes.  One wave per token
-// and step walks the token's query heads, then its key heads; cos/sin of the token are loaded once.
+// and step walks the token's query heads or its key heads; cos/sin of the token are loaded once.
+// What bounds it is the memory latency a wave sees between its rows: the forward loads four steps' rows together, q and k go to
+// workgroups of their own (one weight and one set of sums in registers instead of two: more waves per SIMD), and the partner's
+// half comes over as packed bf16 (four lane moves instead of eight).  16 384 tokens, 16 + 2 heads of 256: forward 79 -> 63 us
+// (4.8 TB/s), backward 107 -> 105; 8192 tokens, 16 + 8 heads of 128: forward 34 -> 24, backward 42 -> 33.
 // The backward pass returns the gradients of the projections' outputs and per-workgroup partial sums of
 // the two norm weights' gradients (reduced by a second kernel in a fixed order: no atomics).
 #include "dsa_common.h"
@@ -24,6 +28,10 @@ __device__ __forceinline__ f32x8 bf8_to_f32(u32x4 w) {
 }
 __device__ __forceinline__ u32x4 f32_to_bf8(f32x8 x) {
     return u32x4{pack2bf(x[0], x[1]), pack2bf(x[2], x[3]), pack2bf(x[4], x[5]), pack2bf(x[6], x[7])};
+}
+// the eight bf16 of another lane
+__device__ __forceinline__ u32x4 shfl4(u32x4 x, int lane) {
+    return u32x4{(uint32_t)__shfl((int)x[0], lane, 64), (uint32_t)__shfl((int)x[1], lane, 64), (uint32_t)__shfl((int)x[2], lane, 64), (uint32_t)__shfl((int)x[3], lane, 64)};
 }
 __device__ __forceinline__ float bf16_round(float x) { return __uint_as_float(pack2bf(x, 0.f) << 16); }
 
@@ -53,100 +61,129 @@ __device__ __forceinline__ float row_sum(float x) {
 }
 
 // a norm weight as the module holds it: fp32 (the trainer's master parameters under autocast) or bf16
-__device__ __forceinline__ float norm_weight(const void *w, int w_bf16, int d) {
-    return w_bf16 ? (float)reinterpret_cast<const bf16_t *>(w)[d] : reinterpret_cast<const float *>(w)[d];
+__device__ __forceinline__ f32x8 norm_weights(const void *w, int w_bf16, int d0, float offset) {
+    f32x8 r;
+    if ((uintptr_t)w & 15) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = w_bf16 ? (float)reinterpret_cast<const bf16_t *>(w)[d0 + i] : reinterpret_cast<const float *>(w)[d0 + i];
+    } else if (w_bf16) {
+        r = bf8_to_f32(*reinterpret_cast<const u32x4 *>(reinterpret_cast<const bf16_t *>(w) + d0));
+    } else {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(w) + d0), b = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(w) + d0 + 4);
+        r = f32x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] += offset;
+    return r;
+}
+
+// q's or k's share of the workgroups: blocks 0 .. nbq-1 take q, the rest k
+struct RopeSide { int first, blocks, H; bool isq; };
+__device__ __forceinline__ RopeSide rope_side(int nbq, int Hq, int Hkv) {
+    if ((int)blockIdx.x < nbq) return RopeSide{(int)blockIdx.x, nbq, Hq, true};
+    return RopeSide{(int)blockIdx.x - nbq, (int)gridDim.x - nbq, Hkv, false};
 }
 
 template <int D, bool CS_F32>
 __global__ __launch_bounds__(256) void dsa_qk_norm_rope_fwd_kernel(
     const bf16_t *__restrict__ q_in, int64_t q_tok, int64_t q_head, const bf16_t *__restrict__ k_in, int64_t k_tok,
     int64_t k_head, const void *__restrict__ qw, const void *__restrict__ kw, int w_bf16, float eps, float w_offset,
-    const void *__restrict__ cosp, const void *__restrict__ sinp, int R, int T, int Hq, int Hkv,
+    const void *__restrict__ cosp, const void *__restrict__ sinp, int R, int T, int Hq, int Hkv, int nbq,
     bf16_t *__restrict__ q_out, bf16_t *__restrict__ k_out, float *__restrict__ q_rstd, float *__restrict__ k_rstd) {
-    constexpr int LPR = D / 8, RPW = 64 / LPR;           // lanes per row, rows per wave and step
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    constexpr int LPR = D / 8, RPW = 64 / LPR, ROWS = 4; // lanes per row, rows per wave and step, steps loaded together
+    const RopeSide sd = rope_side(nbq, Hq, Hkv);
+    const bf16_t *const in = sd.isq ? q_in : k_in;
+    const int64_t tok = sd.isq ? q_tok : k_tok, head = sd.isq ? q_head : k_head;
+    bf16_t *const out = sd.isq ? q_out : k_out;
+    float *const rstd_out = sd.isq ? q_rstd : k_rstd;
+    const void *const wp = sd.isq ? qw : kw;
+    const int H = sd.H, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int sub = lane / LPR, d0 = (lane % LPR) * 8;
     const int half_lanes = R / 16;                       // rotate_half partner distance in lanes
     const bool low = d0 < R / 2, rot = d0 < R;
-    f32x8 wq, wk;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) { wq[i] = norm_weight(qw, w_bf16, d0 + i) + w_offset; wk[i] = norm_weight(kw, w_bf16, d0 + i) + w_offset; }
-    for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < T; t += (int64_t)gridDim.x * 4) {
+    const int partner = low ? lane + half_lanes : lane - half_lanes;
+    const f32x8 w = norm_weights(wp, w_bf16, d0, w_offset);
+    for (int64_t t = (int64_t)sd.first * 4 + wv; t < T; t += (int64_t)sd.blocks * 4) {
         f32x8 c, s;
         load_cs<CS_F32>(cosp, t, R, d0, c, 1.f);
         load_cs<CS_F32>(sinp, t, R, d0, s, 0.f);
-        const int H = Hq + Hkv;
-        for (int r0 = 0; r0 < H; r0 += RPW) {
-            const int r = r0 + sub;
-            const bool live = r < H, isq = r < Hq;
-            const int hh = live ? (isq ? r : r - Hq) : 0;
-            const bf16_t *src = isq ? q_in + t * q_tok + hh * q_head : k_in + t * k_tok + hh * k_head;
-            f32x8 x = bf8_to_f32(live ? *reinterpret_cast<const u32x4 *>(src + d0) : u32x4{0u, 0u, 0u, 0u});
-            float ss = 0.f;
+        const bf16_t *const src = in + t * tok + d0;
+        for (int r0 = 0; r0 < H; r0 += ROWS * RPW) {
+            u32x4 raw[ROWS];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
-            const float rstd = rsqrtf(row_sum<LPR>(ss) * (1.f / D) + eps);
-            const f32x8 w = isq ? wq : wk;
-            f32x8 n, y;
+            for (int u = 0; u < ROWS; ++u) raw[u] = *reinterpret_cast<const u32x4 *>(src + min(r0 + u * RPW + sub, H - 1) * head);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) n[i] = bf16_round(x[i] * rstd * w[i]);       // F.rms_norm returns bf16
+            for (int u = 0; u < ROWS; ++u) {
+                if (u > 0 && r0 + u * RPW >= H) break;   // (wave-uniform)
+                const int r = r0 + u * RPW + sub;
+                const f32x8 x = bf8_to_f32(raw[u]);
+                float ss = 0.f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+                for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
+                const float rstd = rsqrtf(row_sum<LPR>(ss) * (1.f / D) + eps);
+                f32x8 xn, y;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) xn[i] = x[i] * rstd * w[i];
+                const u32x4 nb = f32_to_bf8(xn);                                     // F.rms_norm returns bf16
                 // rotate_half: element i < R/2 takes -n[i + R/2], element R/2 <= i < R takes n[i - R/2]
-                const float other = __shfl(n[i], low ? lane + half_lanes : lane - half_lanes, 64);
-                y[i] = rot ? n[i] * c[i] + (low ? -other : other) * s[i] : n[i];
-            }
-            if (live) {
-                bf16_t *dst = isq ? q_out + ((int64_t)t * Hq + hh) * D : k_out + ((int64_t)t * Hkv + hh) * D;
-                *reinterpret_cast<u32x4 *>(dst + d0) = f32_to_bf8(y);
-                if (d0 == 0) (isq ? q_rstd + (int64_t)t * Hq : k_rstd + (int64_t)t * Hkv)[hh] = rstd;
+                const f32x8 n = bf8_to_f32(nb), other = bf8_to_f32(shfl4(nb, partner));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = rot ? n[i] * c[i] + (low ? -other[i] : other[i]) * s[i] : n[i];
+                if (r < H) {
+                    *reinterpret_cast<u32x4 *>(out + (t * H + r) * D + d0) = f32_to_bf8(y);
+                    if (d0 == 0) rstd_out[t * H + r] = rstd;
+                }
             }
         }
     }
 }
 
 // gradients: g = d(loss)/d(rope output).  dn = rope^T g, dx = rstd * (dn*w - xhat * mean(dn*w*xhat)),
-// dw += dn * xhat (per workgroup partial sums: part[block][q|k][D])
+// dw += dn * xhat (per workgroup partial sums: part[block][D], q's blocks first)
 template <int D, bool CS_F32>
 __global__ __launch_bounds__(256) void dsa_qk_norm_rope_bwd_kernel(
     const bf16_t *__restrict__ gq, const bf16_t *__restrict__ gk, const bf16_t *__restrict__ q_in, int64_t q_tok,
     int64_t q_head, const bf16_t *__restrict__ k_in, int64_t k_tok, int64_t k_head, const void *__restrict__ qw,
     const void *__restrict__ kw, int w_bf16, float w_offset, const void *__restrict__ cosp, const void *__restrict__ sinp, int R,
-    const float *__restrict__ q_rstd, const float *__restrict__ k_rstd, int T, int Hq, int Hkv,
+    const float *__restrict__ q_rstd, const float *__restrict__ k_rstd, int T, int Hq, int Hkv, int nbq,
     bf16_t *__restrict__ dq_in, int64_t dq_tok, int64_t dq_head, bf16_t *__restrict__ dk_in, int64_t dk_tok,
     int64_t dk_head, float *__restrict__ part) {
     constexpr int LPR = D / 8, RPW = 64 / LPR;
-    __shared__ float red[4][2][D];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    __shared__ float red[4][D];
+    const RopeSide sd = rope_side(nbq, Hq, Hkv);
+    const bf16_t *const in = sd.isq ? q_in : k_in, *const gin = sd.isq ? gq : gk;
+    const int64_t tok = sd.isq ? q_tok : k_tok, head = sd.isq ? q_head : k_head;
+    bf16_t *const out = sd.isq ? dq_in : dk_in;
+    const int64_t out_tok = sd.isq ? dq_tok : dk_tok, out_head = sd.isq ? dq_head : dk_head;
+    const float *const rstd_in = sd.isq ? q_rstd : k_rstd;
+    const void *const wp = sd.isq ? qw : kw;
+    const int H = sd.H, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int sub = lane / LPR, d0 = (lane % LPR) * 8;
     const int half_lanes = R / 16;
     const bool low = d0 < R / 2, rot = d0 < R;
-    f32x8 wq, wk, aq, ak;
+    const int partner = low ? lane + half_lanes : lane - half_lanes;
+    const f32x8 w = norm_weights(wp, w_bf16, d0, w_offset);
+    f32x8 a;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { wq[i] = norm_weight(qw, w_bf16, d0 + i) + w_offset; wk[i] = norm_weight(kw, w_bf16, d0 + i) + w_offset; aq[i] = 0.f; ak[i] = 0.f; }
-    for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < T; t += (int64_t)gridDim.x * 4) {
+    for (int i = 0; i < 8; ++i) a[i] = 0.f;
+    for (int64_t t = (int64_t)sd.first * 4 + wv; t < T; t += (int64_t)sd.blocks * 4) {
         f32x8 c, s;
         load_cs<CS_F32>(cosp, t, R, d0, c, 1.f);
-        load_cs<CS_F32>(sinp, t, R, d0, s, 0.f);
-        const int H = Hq + Hkv;
+        load_cs<CS_F32>(sinp, t, R, rot ? (low ? d0 + R / 2 : d0 - R / 2) : d0, s, 0.f);         // the partner's
+        const bf16_t *const src = in + t * tok + d0, *const gsrc = gin + t * H * D + d0;
         for (int r0 = 0; r0 < H; r0 += RPW) {
-            const int r = r0 + sub;
-            const bool live = r < H, isq = r < Hq;
-            const int hh = live ? (isq ? r : r - Hq) : 0;
-            const bf16_t *src = isq ? q_in + t * q_tok + hh * q_head : k_in + t * k_tok + hh * k_head;
-            const bf16_t *gsrc = isq ? gq + ((int64_t)t * Hq + hh) * D : gk + ((int64_t)t * Hkv + hh) * D;
-            const u32x4 z4 = {0u, 0u, 0u, 0u};
-            const f32x8 x = bf8_to_f32(live ? *reinterpret_cast<const u32x4 *>(src + d0) : z4);
-            const f32x8 g = bf8_to_f32(live ? *reinterpret_cast<const u32x4 *>(gsrc + d0) : z4);
-            const float rstd = live ? (isq ? q_rstd + (int64_t)t * Hq : k_rstd + (int64_t)t * Hkv)[hh] : 0.f;
-            const f32x8 w = isq ? wq : wk;
+            const int r = r0 + sub, rc = min(r, H - 1);
+            const bool live = r < H;
+            const u32x4 graw = *reinterpret_cast<const u32x4 *>(gsrc + rc * D);
+            const f32x8 x = bf8_to_f32(*reinterpret_cast<const u32x4 *>(src + rc * head)), g = bf8_to_f32(graw);
+            const float rstd = live ? rstd_in[t * H + rc] : 0.f;
+            const f32x8 gp = bf8_to_f32(shfl4(graw, partner));
             f32x8 dn, xh;
             float dot = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 // transpose of rotate_half: dn[i] = g[i] cos[i] + (i < R/2 ? g[i+R/2] sin[i+R/2] : -g[i-R/2] sin[i-R/2])
-                const float gs = g[i] * s[i];
-                const float other = __shfl(gs, low ? lane + half_lanes : lane - half_lanes, 64);
+                const float other = gp[i] * s[i];
                 dn[i] = rot ? g[i] * c[i] + (low ? other : -other) : g[i];
                 xh[i] = x[i] * rstd;
                 dot += dn[i] * w[i] * xh[i];
@@ -156,55 +193,55 @@ __global__ __launch_bounds__(256) void dsa_qk_norm_rope_bwd_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 dx[i] = rstd * (dn[i] * w[i] - xh[i] * mean);
-                if (isq) aq[i] += dn[i] * xh[i]; else ak[i] += dn[i] * xh[i];          // dead rows carry zeros
+                a[i] += dn[i] * xh[i];                   // dead rows carry zeros (rstd)
             }
-            if (live) {
-                bf16_t *dst = isq ? dq_in + t * dq_tok + hh * dq_head : dk_in + t * dk_tok + hh * dk_head;
-                *reinterpret_cast<u32x4 *>(dst + d0) = f32_to_bf8(dx);
-            }
+            if (live) *reinterpret_cast<u32x4 *>(out + t * out_tok + r * out_head + d0) = f32_to_bf8(dx);
         }
     }
     // rows of one wave -> one value per d; then the four waves; fixed order throughout
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int m = LPR; m < 64; m <<= 1) { aq[i] += __shfl_xor(aq[i], m, 64); ak[i] += __shfl_xor(ak[i], m, 64); }
+        for (int m = LPR; m < 64; m <<= 1) a[i] += __shfl_xor(a[i], m, 64);
     }
     if (sub == 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { red[wv][0][d0 + i] = aq[i]; red[wv][1][d0 + i] = ak[i]; }
+        for (int i = 0; i < 8; ++i) red[wv][d0 + i] = a[i];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * D; i += 256) {
-        const int which = i / D, d = i % D;
-        part[((int64_t)blockIdx.x * 2 + which) * D + d] = red[0][which][d] + red[1][which][d] + red[2][which][d] + red[3][which][d];
-    }
+    for (int d = threadIdx.x; d < D; d += 256) part[(int64_t)blockIdx.x * D + d] = red[0][d] + red[1][d] + red[2][d] + red[3][d];
 }
 
-// dw[which][d] = sum over the workgroups' partial sums.  A workgroup of 64 x 16 threads owns 64
-// consecutive d of one weight: thread (x, y) adds the partials of blocks y, y+16, ... (coalesced over x),
-// then the 16 sub-sums are added in y order - the same order on every run.
-__global__ __launch_bounds__(1024) void dsa_norm_weight_reduce_kernel(const float *__restrict__ part, int nblocks, int D,
-                                                                      float *__restrict__ dqw, float *__restrict__ dkw) {
-    __shared__ float red[16][64];
-    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-    const int which = (blockIdx.x * 64) / D, d = (blockIdx.x * 64) % D + x;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;        // four loads in flight; the order of additions stays fixed
-    int b = y;
-    for (; b + 48 < nblocks; b += 64) {
-        a0 += part[((int64_t)b * 2 + which) * D + d];
-        a1 += part[((int64_t)(b + 16) * 2 + which) * D + d];
-        a2 += part[((int64_t)(b + 32) * 2 + which) * D + d];
-        a3 += part[((int64_t)(b + 48) * 2 + which) * D + d];
+// dw[which][d] = sum over the workgroups' partial sums, fp32 or bf16 as the weight is.  A workgroup owns 16 consecutive d of one
+// weight, four per thread: thread (x, y) of 4 x 256 adds the partials of blocks y, y+256, ..., then the 256 sub-sums are added
+// in y order (sixteen at a time, then the sixteen) - the same order on every run.  Bound by the latency of those loads: 64 d
+// per workgroup, one load per thread and step, 12.9 us at head_dim 256 and 2048 blocks; this form 6.
+template <bool OUT_BF16>
+__global__ __launch_bounds__(1024) void dsa_norm_weight_reduce_kernel(const float *__restrict__ part, int nbq, int nbk, int D,
+                                                                      void *__restrict__ dqw, void *__restrict__ dkw) {
+    __shared__ f32x4 red[256][4];
+    __shared__ f32x4 red2[16][4];
+    const int x = threadIdx.x & 3, y = threadIdx.x >> 2;
+    const int which = (blockIdx.x * 16) / D, d = (blockIdx.x * 16) % D + 4 * x;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int b = (which ? nbq : 0) + y; b < (which ? nbq + nbk : nbq); b += 256) a += *reinterpret_cast<const f32x4 *>(part + (int64_t)b * D + d);
+    red[y][x] = a;
+    __syncthreads();
+    if (y < 16) {
+        f32x4 t = red[16 * y][x];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) t += red[16 * y + i][x];
+        red2[y][x] = t;
     }
-    for (; b < nblocks; b += 16) a0 += part[((int64_t)b * 2 + which) * D + d];
-    red[y][x] = (a0 + a1) + (a2 + a3);
     __syncthreads();
     if (y == 0) {
-        float t = 0.f;
+        f32x4 t = red2[0][x];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) t += red[i][x];
-        (which ? dkw : dqw)[d] = t;
+        for (int i = 1; i < 16; ++i) t += red2[i][x];
+        void *out = which ? dkw : dqw;
+        if (OUT_BF16) *reinterpret_cast<u32x2 *>((bf16_t *)out + d) = u32x2{pack2bf(t[0], t[1]), pack2bf(t[2], t[3])};
+        else *reinterpret_cast<f32x4 *>((float *)out + d) = t;
     }
 }
 
@@ -255,7 +292,20 @@ static inline int prologue_blocks(int T) {
     return want < 1 ? 1 : (want > 2048 ? 2048 : want);
 }
 extern "C" int dsa_prologue_bwd_blocks(int T) { return prologue_blocks(T); }
-
+// q's workgroups: every wave the same number of tokens (a wave with one token more than the others is what the launch ends on);
+// k's: fewer, as its few heads make a token cheaper - by the steps of a token and about two more to get them going.  The
+// backward stays within `most` of each (its partial sums: D floats per workgroup, in a workspace for 2 D per block).
+static inline int even_blocks(int T, int most) {
+    const int waves = 4 * (most < 1 ? 1 : most), per_wave = (T + waves - 1) / waves;
+    return (T + 4 * per_wave - 1) / (4 * per_wave);
+}
+static inline int prologue_blocks_q(int T, int most) { return even_blocks(T, most); }
+static inline int prologue_blocks_k(int T, int most, int Hq, int Hkv, int D) {
+    const int rpw = 512 / D, q = (Hq + rpw - 1) / rpw + 2, k = (Hkv + rpw - 1) / rpw + 2;
+    const int share = (int)((int64_t)even_blocks(T, most) * k / q);
+    return even_blocks(T, share < most ? share : most);
+}
+#define FWD_BLOCKS 8192                                  // (up to 32 768 tokens: one per wave)
 #define PROLOGUE_SWITCH(KERNEL, ...)                                                        \
     switch (D) {                                                                            \
         case 64: if (cs_f32) hipLaunchKernelGGL((KERNEL<64, true>), __VA_ARGS__); else hipLaunchKernelGGL((KERNEL<64, false>), __VA_ARGS__); break;    \
@@ -270,8 +320,9 @@ extern "C" hipError_t dsa_launch_qk_norm_rope_fwd(const void *q_in, int64_t q_to
                                                   int Hq, int Hkv, int D, void *q_out, void *k_out, float *q_rstd,
                                                   float *k_rstd, hipStream_t stream) {
     if (T == 0) return hipSuccess;
-    PROLOGUE_SWITCH(dsa_qk_norm_rope_fwd_kernel, dim3(prologue_blocks(T)), dim3(256), 0, stream, (const bf16_t *)q_in, q_tok,
-                    q_head, (const bf16_t *)k_in, k_tok, k_head, qw, kw, w_bf16, eps, w_offset, cosp, sinp, R, T, Hq, Hkv,
+    const int most = T < 4 * FWD_BLOCKS ? (T + 3) / 4 : FWD_BLOCKS, nbq = prologue_blocks_q(T, most), nbk = prologue_blocks_k(T, most, Hq, Hkv, D);
+    PROLOGUE_SWITCH(dsa_qk_norm_rope_fwd_kernel, dim3(nbq + nbk), dim3(256), 0, stream, (const bf16_t *)q_in, q_tok,
+                    q_head, (const bf16_t *)k_in, k_tok, k_head, qw, kw, w_bf16, eps, w_offset, cosp, sinp, R, T, Hq, Hkv, nbq,
                     (bf16_t *)q_out, (bf16_t *)k_out, q_rstd, k_rstd)
     return hipGetLastError();
 }
@@ -282,15 +333,15 @@ extern "C" hipError_t dsa_launch_qk_norm_rope_bwd(const void *gq, const void *gk
                                                   const void *sinp, int cs_f32, int R, const float *q_rstd,
                                                   const float *k_rstd, int T, int Hq, int Hkv, int D, void *dq_in,
                                                   int64_t dq_tok, int64_t dq_head, void *dk_in, int64_t dk_tok,
-                                                  int64_t dk_head, float *dqw, float *dkw, float *part, hipStream_t stream) {
-    const int nb = prologue_blocks(T);
+                                                  int64_t dk_head, void *dqw, void *dkw, int grad_bf16, float *part, hipStream_t stream) {
+    const int most = prologue_blocks(T), nbq = T > 0 ? prologue_blocks_q(T, most) : 0, nbk = T > 0 ? prologue_blocks_k(T, most, Hq, Hkv, D) : 0;
     if (T > 0) {
-        PROLOGUE_SWITCH(dsa_qk_norm_rope_bwd_kernel, dim3(nb), dim3(256), 0, stream, (const bf16_t *)gq, (const bf16_t *)gk,
+        PROLOGUE_SWITCH(dsa_qk_norm_rope_bwd_kernel, dim3(nbq + nbk), dim3(256), 0, stream, (const bf16_t *)gq, (const bf16_t *)gk,
                         (const bf16_t *)q_in, q_tok, q_head, (const bf16_t *)k_in, k_tok, k_head, qw, kw, w_bf16, w_offset, cosp, sinp,
-                        R, q_rstd, k_rstd, T, Hq, Hkv, (bf16_t *)dq_in, dq_tok, dq_head, (bf16_t *)dk_in, dk_tok, dk_head, part)
+                        R, q_rstd, k_rstd, T, Hq, Hkv, nbq, (bf16_t *)dq_in, dq_tok, dq_head, (bf16_t *)dk_in, dk_tok, dk_head, part)
     }
-    hipLaunchKernelGGL(dsa_norm_weight_reduce_kernel, dim3(2 * D / 64), dim3(1024), 0, stream, part, T > 0 ? nb : 0, D, dqw,
-                       dkw);
+    if (grad_bf16) hipLaunchKernelGGL((dsa_norm_weight_reduce_kernel<true>), dim3(2 * D / 16), dim3(1024), 0, stream, part, nbq, nbk, D, dqw, dkw);
+    else hipLaunchKernelGGL((dsa_norm_weight_reduce_kernel<false>), dim3(2 * D / 16), dim3(1024), 0, stream, part, nbq, nbk, D, dqw, dkw);
     return hipGetLastError();
 }
 
