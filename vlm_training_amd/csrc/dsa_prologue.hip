@@ -11,6 +11,9 @@
 // workgroups of their own (one weight and one set of sums in registers instead of two: more waves per SIMD), and the partner's
 // half comes over as packed bf16 (four lane moves instead of eight).  16 384 tokens, 16 + 2 heads of 256: forward 79 -> 63 us
 // (4.8 TB/s), backward 107 -> 105; 8192 tokens, 16 + 8 heads of 128: forward 34 -> 24, backward 42 -> 33.
+// Everything here is read once and written once, so it goes past the caches (non-temporal loads and stores): written lines left
+// in the Infinity Cache had to be pushed out by the next kernel's reads - 16 384 tokens, 16 heads of 256, norm, rotation and gate
+// with backward 372 -> 332 us (5.5 TB/s over all); a layer whose next kernel reads the result (8192 tokens) is not slower for it.
 // The backward pass returns the gradients of the projections' outputs and per-workgroup partial sums of
 // the two norm weights' gradients (reduced by a second kernel in a fixed order: no atomics).
 #include "dsa_common.h"
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(256) void dsa_qk_norm_rope_fwd_kernel(
         for (int r0 = 0; r0 < H; r0 += ROWS * RPW) {
             u32x4 raw[ROWS];
 #pragma unroll
-            for (int u = 0; u < ROWS; ++u) raw[u] = *reinterpret_cast<const u32x4 *>(src + min(r0 + u * RPW + sub, H - 1) * head);
+            for (int u = 0; u < ROWS; ++u) raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + min(r0 + u * RPW + sub, H - 1) * head));
 #pragma unroll
             for (int u = 0; u < ROWS; ++u) {
                 if (u > 0 && r0 + u * RPW >= H) break;   // (wave-uniform)
@@ -130,7 +133,7 @@ __global__ __launch_bounds__(256) void dsa_qk_norm_rope_fwd_kernel(
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = rot ? n[i] * c[i] + (low ? -other[i] : other[i]) * s[i] : n[i];
                 if (r < H) {
-                    *reinterpret_cast<u32x4 *>(out + (t * H + r) * D + d0) = f32_to_bf8(y);
+                    __builtin_nontemporal_store(f32_to_bf8(y), reinterpret_cast<u32x4 *>(out + (t * H + r) * D + d0));
                     if (d0 == 0) rstd_out[t * H + r] = rstd;
                 }
             }
@@ -174,8 +177,8 @@ __global__ __launch_bounds__(256) void dsa_qk_norm_rope_bwd_kernel(
         for (int r0 = 0; r0 < H; r0 += RPW) {
             const int r = r0 + sub, rc = min(r, H - 1);
             const bool live = r < H;
-            const u32x4 graw = *reinterpret_cast<const u32x4 *>(gsrc + rc * D);
-            const f32x8 x = bf8_to_f32(*reinterpret_cast<const u32x4 *>(src + rc * head)), g = bf8_to_f32(graw);
+            const u32x4 graw = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gsrc + rc * D));
+            const f32x8 x = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + rc * head))), g = bf8_to_f32(graw);
             const float rstd = live ? rstd_in[t * H + rc] : 0.f;
             const f32x8 gp = bf8_to_f32(shfl4(graw, partner));
             f32x8 dn, xh;
@@ -195,7 +198,7 @@ __global__ __launch_bounds__(256) void dsa_qk_norm_rope_bwd_kernel(
                 dx[i] = rstd * (dn[i] * w[i] - xh[i] * mean);
                 a[i] += dn[i] * xh[i];                   // dead rows carry zeros (rstd)
             }
-            if (live) *reinterpret_cast<u32x4 *>(out + t * out_tok + r * out_head + d0) = f32_to_bf8(dx);
+            if (live) __builtin_nontemporal_store(f32_to_bf8(dx), reinterpret_cast<u32x4 *>(out + t * out_tok + r * out_head + d0));
         }
     }
     // rows of one wave -> one value per d; then the four waves; fixed order throughout
@@ -254,12 +257,12 @@ __global__ __launch_bounds__(256) void dsa_sigmoid_gate_fwd_kernel(const bf16_t 
     for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < chunks; c += (int64_t)gridDim.x * 256) {
         const int64_t e = c * 8, t = e / ((int64_t)H * D);
         const int rem = (int)(e - t * H * D), hh = rem / D, d = rem % D;
-        const f32x8 a = bf8_to_f32(*reinterpret_cast<const u32x4 *>(x + e));
-        const f32x8 g = bf8_to_f32(*reinterpret_cast<const u32x4 *>(gate + t * gate_tok + hh * gate_head + d));
+        const f32x8 a = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + e)));
+        const f32x8 g = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + t * gate_tok + hh * gate_head + d)));
         f32x8 r;
 #pragma unroll
         for (int i = 0; i < 8; ++i) r[i] = a[i] * bf16_round(1.f / (1.f + __expf(-g[i])));   // torch.sigmoid returns bf16
-        *reinterpret_cast<u32x4 *>(y + e) = f32_to_bf8(r);
+        __builtin_nontemporal_store(f32_to_bf8(r), reinterpret_cast<u32x4 *>(y + e));
     }
 }
 __global__ __launch_bounds__(256) void dsa_sigmoid_gate_bwd_kernel(const bf16_t *__restrict__ gy, const bf16_t *__restrict__ x,
@@ -271,9 +274,9 @@ __global__ __launch_bounds__(256) void dsa_sigmoid_gate_bwd_kernel(const bf16_t 
     for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < chunks; c += (int64_t)gridDim.x * 256) {
         const int64_t e = c * 8, t = e / ((int64_t)H * D);
         const int rem = (int)(e - t * H * D), hh = rem / D, d = rem % D;
-        const f32x8 gyv = bf8_to_f32(*reinterpret_cast<const u32x4 *>(gy + e));
-        const f32x8 a = bf8_to_f32(*reinterpret_cast<const u32x4 *>(x + e));
-        const f32x8 g = bf8_to_f32(*reinterpret_cast<const u32x4 *>(gate + t * gate_tok + hh * gate_head + d));
+        const f32x8 gyv = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gy + e)));
+        const f32x8 a = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + e)));
+        const f32x8 g = bf8_to_f32(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + t * gate_tok + hh * gate_head + d)));
         f32x8 r1, r2;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -281,8 +284,8 @@ __global__ __launch_bounds__(256) void dsa_sigmoid_gate_bwd_kernel(const bf16_t 
             r1[i] = gyv[i] * sg;
             r2[i] = gyv[i] * a[i] * sg * (1.f - sg);
         }
-        *reinterpret_cast<u32x4 *>(dx + e) = f32_to_bf8(r1);
-        *reinterpret_cast<u32x4 *>(dgate + t * dgate_tok + hh * dgate_head + d) = f32_to_bf8(r2);
+        __builtin_nontemporal_store(f32_to_bf8(r1), reinterpret_cast<u32x4 *>(dx + e));
+        __builtin_nontemporal_store(f32_to_bf8(r2), reinterpret_cast<u32x4 *>(dgate + t * dgate_tok + hh * dgate_head + d));
     }
 }
 
