@@ -44,8 +44,11 @@ hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, co
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                               int Hq, int Hkv, int D, float scale, int causal, int32_t *order, float *partial,
+                               int Hq, int Hkv, int D, float scale, int causal, int32_t *order, int listed, float *partial,
                                size_t partial_bytes, void *dk, void *dv, hipStream_t stream);
+hipError_t dsa_launch_tile_order_delta(const void *dout, const void *out, const int32_t *cu, int N, int T, int Hq, int Hkv, int D,
+                                       int has_idx, int causal, int32_t *order, const float *partial, size_t partial_bytes,
+                                       float *delta, hipStream_t stream);
 size_t dsa_tile_order_bytes(int T);
 size_t dsa_tile_dkv_partial_bytes(int T);
 int dsa_mass_groups(int Hq, int Hkv, int D);
@@ -399,10 +402,14 @@ extern "C" int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const fl
 // made on first use outside any capture) between a fork and a join event, so that to the caller everything still
 // happens on the stream it passed.  A stream under capture takes the second one into the capture through the events.
 // mode 1 runs the passes side by side for key-side launches of at most this many workgroups (larger ones fill the GPU
-// alone) whose work bound T * max_seqlen * Hq * D reaches the second figure (about 0.4 ms of backward: below it the
-// fork, the join and the delta pass that the query side otherwise absorbs cost what the overlap gains)
+// alone) whose work bound T * max_seqlen * Hq * D reaches the second figure: below it the host issues a step more slowly than
+// the GPU runs it, and the fork, the join and the pass over dO and O (with the key side's list in the same launch) cost more
+// than the overlap gains.  Step times, one after the other -> side by side: fp32 2048 tokens 217 -> 170 us; head_dim 128 packed
+// rows of 4096-8192 tokens, 5-19 % less; 10 000-16 384 tokens, 0-3 % less; 1000 tokens at 2e9, 130 -> 105; 700 tokens at 7e8,
+// level.  Without a causal mask the walks of a segment are all equally long, and small launches win nothing.
 #define DSA_BWD_OVERLAP_MAX_WG (6 * 256)
-#define DSA_BWD_OVERLAP_MIN_WORK 6.0e10
+#define DSA_BWD_OVERLAP_MIN_WORK 2.0e9
+#define DSA_BWD_OVERLAP_MIN_WORK_FULL 6.0e10
 struct OverlapCtx {
     hipStream_t aux = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
@@ -539,7 +546,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0) {
         const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);
         const double work = (double)T * max_seqlen * Hq * D;
-        if (ov_mode == 2 || (dkv_wg <= DSA_BWD_OVERLAP_MAX_WG && work >= DSA_BWD_OVERLAP_MIN_WORK)) {
+        if (ov_mode == 2 || (dkv_wg <= DSA_BWD_OVERLAP_MAX_WG && work >= (causal ? DSA_BWD_OVERLAP_MIN_WORK : DSA_BWD_OVERLAP_MIN_WORK_FULL))) {
             ov_lock = std::unique_lock<std::mutex>(g_overlap_mu);
             ov = overlap_ctx(st);
             if (!ov) ov_lock.unlock();
@@ -549,7 +556,13 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     // (no row beyond the tile/gather split) - then that kernel forms it from the dO rows it loads anyway - and the
     // key side, which reads every delta, runs after it
     const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && split > 0 && max_seqlen <= split && !ov;
-    if ((parts & DSA_BWD_DELTA) && !fuse_delta) {
+    int listed = 0;                                      // the launch order of the key tiles is there
+    if ((parts & DSA_BWD_DELTA) && ov) {
+        e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, idx != nullptr, causal, order, partial, partial_bytes, delta, st);
+        if (e == hipSuccess) listed = 1;
+        else if (e != hipErrorNotReady) return hip_fail(e, "order and delta launch");   // (not ready: this launch needs no list)
+    }
+    if ((parts & DSA_BWD_DELTA) && !fuse_delta && !listed) {
         e = dsa_launch_delta(dout, out, T, Hq, D, delta, st);
         if (e != hipSuccess) return hip_fail(e, "delta launch");
     }
@@ -567,7 +580,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     int rc = DSA_OK;
     // (side by side, the key side is issued first: it is the longer pass and starts with its longest walks)
     if (ov) {
-        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, partial,
+        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, listed, partial,
                                 partial_bytes, dk, dv, st);
         if (e != hipSuccess) rc = hip_fail(e, "tile dkv launch");
     }
@@ -583,7 +596,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
         }
     }
     if (rc == DSA_OK && !ov && (parts & DSA_BWD_DKV)) {
-        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, partial,
+        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, listed, partial,
                                 partial_bytes, dk, dv, st);
         if (e != hipSuccess) rc = hip_fail(e, "tile dkv launch");
     }

@@ -11,27 +11,10 @@
 //                                                         every key row from it without atomics.
 #include "dsa_common.h"
 
-// ------------------------------------------------------------------------------------------------
-// delta: 16 lanes per (t,h) row; lane i sums the 8-element chunks i, i+16, ... in one chain, then a butterfly over the 16
-// lanes (dsa_tile_dq_kernel reproduces this order when it forms delta itself)
-// ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void dsa_bwd_delta_kernel(const bf16_t *__restrict__ dout,
                                                             const bf16_t *__restrict__ out, int T, int Hq, int D,
                                                             float *__restrict__ delta) {
-    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    const int sub = threadIdx.x & 15;
-    float acc = 0.f;
-    if (row < (int64_t)T * Hq) {
-        for (int c = sub * 8; c < D; c += 128) {
-            acc = dot8_chain(load_bf16x8(dout + row * D + c), load_bf16x8(out + row * D + c), acc);
-        }
-    }
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if (sub == 0 && row < (int64_t)T * Hq) {
-        const int t = (int)(row / Hq), h = (int)(row % Hq);
-        delta[(int64_t)h * T + t] = acc;
-    }
+    delta_row(dout, out, T, Hq, D, (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4), threadIdx.x & 15, delta);
 }
 
 // ------------------------------------------------------------------------------------------------

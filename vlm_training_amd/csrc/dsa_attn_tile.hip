@@ -437,9 +437,9 @@ static_assert(DSA_ORDER_MAX_TILES + 1 >= 2 * DSA_ORDER_MAX_SEGS, "the rank table
 __device__ __forceinline__ void order_entry(int32_t *order, int slot, int seg, int tile, int piece, int mslot) {
     *reinterpret_cast<int4 *>(order + 4 + 4 * slot) = make_int4(seg, tile, piece, mslot);
 }
-__global__ __launch_bounds__(1024) void dsa_tile_order_kernel(const int32_t *__restrict__ cu, int N, int cap, int mode, int qb,
-                                                              int wg_per_tile, int item_cap, int slot_cap,
-                                                              int32_t *__restrict__ order) {
+struct TileOrder { int cap, mode, qb, wg_per_tile, item_cap, slot_cap; };
+__device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N, const TileOrder &o_, int32_t *__restrict__ order) {
+    const int cap = o_.cap, mode = o_.mode, qb = o_.qb, wg_per_tile = o_.wg_per_tile, item_cap = o_.item_cap, slot_cap = o_.slot_cap;
     __shared__ int nt[DSA_ORDER_MAX_SEGS];               // tiles per segment
     __shared__ int cnt[DSA_ORDER_MAX_TILES + 1];         // cnt[r]: segments with at least r tiles; then: slots before rank r
     __shared__ int part[1024];
@@ -609,6 +609,17 @@ __global__ __launch_bounds__(1024) void dsa_tile_order_kernel(const int32_t *__r
         for (int i = 0; i < N; ++i)
             if (nt[i] >= r) order_entry(order, slot++, i, nt[i] - r, 0, -1);
     }
+}
+__global__ __launch_bounds__(1024) void dsa_tile_order_kernel(const int32_t *__restrict__ cu, int N, TileOrder o, int32_t *__restrict__ order) {
+    tile_order(cu, N, o, order);
+}
+// the list by the first workgroup and delta, 64 rows each, by the others: the two things the passes of a backward on two streams
+// wait for, in one launch (the list alone takes 8 to 14 us, most of it latency)
+__global__ __launch_bounds__(1024) void dsa_tile_order_delta_kernel(const int32_t *__restrict__ cu, int N, TileOrder o, int32_t *__restrict__ order,
+                                                                    const bf16_t *__restrict__ dout, const bf16_t *__restrict__ out, int T,
+                                                                    int Hq, int D, float *__restrict__ delta) {
+    if (blockIdx.x == 0) tile_order(cu, N, o, order);
+    else delta_row(dout, out, T, Hq, D, (int64_t)(blockIdx.x - 1) * 64 + (threadIdx.x >> 4), threadIdx.x & 15, delta);
 }
 static inline int order_entries_cap(int T) { return T / 128 + DSA_ORDER_MAX_SEGS + 1 + DSA_ORDER_EXTRA; }
 extern "C" size_t dsa_tile_order_bytes(int T) { return ((size_t)order_entries_cap(T) * 5 + 4) * sizeof(int32_t); }
@@ -1685,37 +1696,49 @@ extern "C" size_t dsa_tile_dkv_partial_bytes(int T) {
     const size_t b = (size_t)T * 16384;
     return b < ((size_t)128 << 20) ? b : ((size_t)128 << 20);
 }
+// How the key-side launch of these sizes hands out its tiles.  `order` (dsa_tile_order_bytes(T) bytes, or null): the tiles are
+// listed longest walk first before the launch.  A launch of at most four workgroups per CU may also cut long walks into pieces
+// (`partial`: fp32 partial sums), so that it does not end on a few long walks with most of the chip idle.
+struct DkvPlan { int tiles_ub, pitch; bool listed, pieces; TileOrder o; };
+static DkvPlan dkv_plan(int T, int N, int Hq, int Hkv, int d_real, bool has_idx, int causal, const void *order, const void *partial, size_t partial_bytes) {
+    DkvPlan p;
+    p.tiles_ub = T / 128 + N;                            // 128-key tiles of all segments, at most
+    p.pitch = has_idx ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;             // row of a partial sum
+    const int wg_per_tile = Hkv * (d_real > 128 ? 2 : 1);
+    const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * p.pitch * sizeof(float))) : 0;
+    p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= 4 * 256;
+    p.listed = order && (N > 1 || p.pieces);             // (one segment: its tiles are in order already)
+    const int cap = order_entries_cap(T), item_cap = p.pieces ? std::min(cap, p.tiles_ub + (1024 + wg_per_tile - 1) / wg_per_tile) : cap;
+    p.o = TileOrder{cap, p.pieces ? 2 : ((p.tiles_ub + 1) * Hkv > 4 * 256 ? 1 : 0), 32 >> group_shift(Hq, Hkv), wg_per_tile, item_cap,
+                    (int)(slot_pairs / Hkv < (1 << 20) ? slot_pairs / Hkv : (1 << 20))};       // (sums stay below 2^21)
+    return p;
+}
+// delta and, where the key-side launch of the same sizes will want it, its list
+extern "C" hipError_t dsa_launch_tile_order_delta(const void *dout, const void *out, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real,
+                                                  int has_idx, int causal, int32_t *order, const float *partial, size_t partial_bytes,
+                                                  float *delta, hipStream_t stream) {
+    const DkvPlan p = dkv_plan(T, N, Hq, Hkv, d_real, has_idx != 0, causal, order, partial, partial_bytes);
+    if (!p.listed) return hipErrorNotReady;
+    hipLaunchKernelGGL(dsa_tile_order_delta_kernel, dim3((unsigned)(1 + ((int64_t)T * Hq + 63) / 64)), dim3(1024), 0, stream, cu, N, p.o, order,
+                       (const bf16_t *)dout, (const bf16_t *)out, T, Hq, d_real, delta);
+    return hipGetLastError();
+}
+// listed: dsa_launch_tile_order_delta has left the list in `order`
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal,
-                                          int32_t *order, float *partial, size_t partial_bytes, void *dk, void *dv,
+                                          int32_t *order, int listed, float *partial, size_t partial_bytes, void *dk, void *dv,
                                           hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
-    const int pitch = bitmap ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;      // row of a partial sum
-    const int tiles_ub = T / 128 + N;                    // 128-key tiles of all segments, at most
-    dim3 grid((unsigned)((tiles_ub + 1) * Hkv));
-    // `order` (dsa_tile_order_bytes(T) bytes, or null): the tiles are listed longest walk first before the launch.
-    // A launch of at most four workgroups per CU may also cut long walks into pieces (`partial`: fp32 partial sums), so
-    // that it does not end on a few long walks with most of the chip idle.
-    const int wg_per_tile = Hkv * (d_real > 128 ? 2 : 1);
-    const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * pitch * sizeof(float))) : 0;
-    const bool pieces = order && causal && slot_pairs >= Hkv && (int64_t)tiles_ub * wg_per_tile <= 4 * 256;
-    int item_cap = 0;
-    if (order && (N > 1 || pieces)) {
-        const int cap = order_entries_cap(T);
-        item_cap = pieces ? std::min(cap, tiles_ub + (1024 + wg_per_tile - 1) / wg_per_tile) : cap;
-        hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, cap,
-                           pieces ? 2 : (grid.x > 4 * 256 ? 1 : 0), 32 >> gs, wg_per_tile, item_cap, (int)(slot_pairs / Hkv < (1 << 20) ? slot_pairs / Hkv : (1 << 20)),   /* (sums stay below 2^21) */
-                           order);
-        if (pieces) grid.x = (unsigned)(item_cap * Hkv);
-    } else {
-        order = nullptr;                                 // one segment: its tiles are in order already
-    }
-    if (!pieces) partial = nullptr;
+    const DkvPlan p = dkv_plan(T, N, Hq, Hkv, d_real, bitmap != nullptr, causal, order, partial, partial_bytes);
+    dim3 grid((unsigned)((p.pieces ? p.o.item_cap : p.tiles_ub + 1) * Hkv));
+    if (!p.listed) order = nullptr;
+    else if (!listed) hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, p.o, order);
+    if (!p.pieces) partial = nullptr;
     TILE_SWITCH_DENSE(launch_dkv_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv)
-    if (pieces)
-        hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(tiles_ub, Hkv, DSA_PIECES_Z), dim3(256), 0, stream, order,
-                           order_entries_cap(T), partial, cu, N, Hkv, d_real, pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
+    if (p.pieces)
+        hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(p.tiles_ub, Hkv, DSA_PIECES_Z), dim3(256), 0, stream, order,
+                           p.o.cap, partial, cu, N, Hkv, d_real, p.pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
                            (bf16_t *)dk, (bf16_t *)dv);
     return hipGetLastError();
 }

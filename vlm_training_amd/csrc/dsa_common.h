@@ -48,6 +48,23 @@ __device__ __forceinline__ float dot8_chain(bf16x8 a, bf16x8 b, float acc) {
     return acc;
 }
 
+// delta[h,t] = sum_d dO[t,h,d] * O[t,h,d] of row (t, h) by 16 lanes (`sub` of them): lane i sums the 8-element chunks i, i+16, ...
+// in one chain, then a butterfly over the 16 lanes (dsa_tile_dq_kernel reproduces this order when it forms delta itself)
+__device__ __forceinline__ void delta_row(const bf16_t *__restrict__ dout, const bf16_t *__restrict__ out, int T, int Hq, int D, int64_t row, int sub,
+                                          float *__restrict__ delta) {
+    float acc = 0.f;
+    if (row < (int64_t)T * Hq) {
+        for (int c = sub * 8; c < D; c += 128)
+            acc = dot8_chain(load_bf16x8(dout + row * D + c), load_bf16x8(out + row * D + c), acc);
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (sub == 0 && row < (int64_t)T * Hq) {
+        const int t = (int)(row / Hq), h = (int)(row % Hq);
+        delta[(int64_t)h * T + t] = acc;
+    }
+}
+
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
