@@ -123,11 +123,11 @@ int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, con
                     const float *dscore, const int32_t *cu_seqlens, int T, int N, int Hi, int Di, int K, float scale,
                     int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
                     void *stream);
-/* The same with every gradient multiplied by *grad (one fp32 on the device: the gradient of the loss; null: 1). */
+/* The same with every gradient multiplied by *grad (one fp32 on the device: the gradient of the loss; null: 1); dw in dw_dtype. */
 int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
                            const float *dscore, const float *grad, const int32_t *cu_seqlens, int T, int N, int Hi, int Di, int K,
-                           float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
-                           void *stream);
+                           float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, void *dw, int dw_dtype, void *ws,
+                           size_t ws_bytes, void *stream);
 size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen);
 
 /*
@@ -333,6 +333,15 @@ int dsa_sigmoid_gate_fwd(const void *x, const void *gate, int64_t gate_tok_strid
 int dsa_sigmoid_gate_bwd(const void *gy, const void *x, const void *gate, int64_t gate_tok_stride,
                          int64_t gate_head_stride, int T, int H, int D, void *dx, void *dgate, int64_t dgate_tok_stride,
                          int64_t dgate_head_stride, void *stream);
+
+/*
+ * n (at most DSA_PACK_MAX) contiguous (T, width[i]) bf16 tensors side by side in the rows of dst (dst_row elements apart): row t
+ * of source i goes to column dst_col[i] in groups of group[i] elements, dst_group[i] apart.  All multiples of 8, pointers on
+ * 16-byte boundaries.  (The gradients of a layer's projections, for one weight-gradient GEMM.)
+ */
+#define DSA_PACK_MAX 8
+int dsa_pack_columns(int n, const void *const *src, const int32_t *width, const int32_t *group, const int32_t *dst_col,
+                     const int32_t *dst_group, int T, void *dst, int64_t dst_row, void *stream);
 
 /*
  * fp32 operands on the bf16 kernels (no reference counterpart: the reference runs the operator in bf16 under autocast;

@@ -59,3 +59,37 @@ def test_dense_gradients_between_the_kernels_head_dims(D, Hq, Hkv, lens, causal)
     for name, a, b in zip("qkv", got, ref):
         assert a.grad.shape == b.grad.shape
         assert_close_bf16(a.grad, b.grad, "d" + name)
+
+
+@pytest.mark.parametrize("gated,T,wanted", [(False, 2048, "both"), (True, 2051, "both"), (True, 2065, "out"), (False, 2065, "loss")])
+def test_projections_in_one_node_equal_the_modules_one_by_one(gated, T, wanted):
+    """Module by module (a forward hook rules the shared node out) against the shared node: outputs bit for bit, gradients to the
+    rounding of a GEMM's split."""
+    print("shared projections", gated, T, wanted, flush=True)
+    from types import SimpleNamespace
+    torch.manual_seed(T)
+    cfg = SimpleNamespace(hidden_size=256, num_attention_heads=4, num_key_value_heads=2, head_dim=64, rms_norm_eps=1e-6)
+    m = (M.SelfAttention if gated else M.Qwen3VLTextAttention)(cfg, dsa=M.DsaConfig(index_heads=8, index_dim=64, top_k=16)).to(DEV, torch.bfloat16)
+    x = torch.randn(1, T, 256, device=DEV).bfloat16()
+    gy = torch.randn(1, T, 256, device=DEV).bfloat16()
+    ang = torch.outer(torch.arange(T, device=DEV).float(), 0.1 ** torch.arange(16, device=DEV).float())
+    cos, sin = torch.cat((ang, ang), -1).cos().bfloat16(), torch.cat((ang, ang), -1).sin().bfloat16()
+    cu = torch.tensor([0, T - T // 3, T], dtype=torch.int32, device=DEV)
+    res = []
+    for hook in (False, True):
+        handle = m.k_proj.register_forward_hook(lambda *a: None) if hook else None
+        xi = x.clone().requires_grad_(True)
+        m.zero_grad(set_to_none=True)
+        y = m(xi, cos, sin, cu, T)
+        loss = M.indexer_losses(m)
+        outs, gs = {"both": ((y, loss), (gy, None)), "out": ((y,), (gy,)), "loss": ((loss,), (None,))}[wanted]
+        torch.autograd.backward(outs, gs)
+        res.append([y.detach(), loss.detach(), xi.grad] + [p.grad for p in m.parameters()])
+        if handle:
+            handle.remove()
+    for a, b in zip(*res):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.shape == b.shape and a.dtype == b.dtype
+            assert (a.float() - b.float()).norm() <= 1e-2 * b.float().norm() + 1e-9
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])

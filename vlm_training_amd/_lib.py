@@ -39,7 +39,7 @@ _SIGNATURES = {
                                 c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t,
                                 c_void_p]),
     "dsa_indexer_bwd_scaled": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
-                                       c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                                       c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                        c_size_t, c_void_p]),
     "dsa_indexer_bwd_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "dsa_attn_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
@@ -91,6 +91,7 @@ _SIGNATURES = {
                                      c_int, c_int, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
                                      c_void_p, c_void_p, c_size_t, c_void_p]),
     "dsa_sigmoid_gate_fwd": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_int, c_int, c_void_p, c_void_p]),
+    "dsa_pack_columns": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p]),
     "dsa_split_bf16_stack": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p]),
     "dsa_split_bf16_combine": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p]),
     "dsa_round_bf16_x3": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -29,7 +29,7 @@ hipError_t dsa_launch_gather_dq(const void *dout, const void *q, const void *k, 
                                 hipStream_t stream);
 hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore, const float *grad,
                                   const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N, int T, int Hi,
-                                  int Di, int K, float cscale, void *dq_idx, void *dk_idx, float *dw, float *partial,
+                                  int Di, int K, float cscale, void *dq_idx, void *dk_idx, void *dw, int dw_bf16, float *partial,
                                   hipStream_t stream, hipStream_t stream_q);
 size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw);
 hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, const uint32_t *bitmap, int ldw,
@@ -68,6 +68,8 @@ hipError_t dsa_launch_qk_norm_rope_bwd(const void *gq, const void *gk, const voi
                                        void *dqw, void *dkw, int grad_bf16, float *part, hipStream_t stream);
 hipError_t dsa_launch_sigmoid_gate_fwd(const void *x, const void *gate, int64_t gate_tok, int64_t gate_head, int D, int H,
                                        int64_t rows, void *y, hipStream_t stream);
+hipError_t dsa_launch_pack_columns(int n, const void *const *src, const int32_t *width, const int32_t *group, const int32_t *dst_col,
+                                   const int32_t *dst_group, int T, void *dst, int64_t dst_row, hipStream_t stream);
 hipError_t dsa_launch_split_stack(const float *x, int64_t rows, int D, int order, void *y, hipStream_t stream);
 hipError_t dsa_launch_split_combine(const void *y, int64_t rows, int D, int part, float *out, hipStream_t stream);
 hipError_t dsa_launch_round_bf16_x3(const float *a, const float *b, const float *c, int64_t na, int64_t nb, int64_t nc, void *ya,
@@ -456,12 +458,13 @@ extern "C" size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen)
 
 extern "C" int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
                                       const float *dscore, const float *grad, const int32_t *cu, int T, int N, int Hi, int Di, int K,
-                                      float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws,
+                                      float scale, int dtype, int max_seqlen, void *dq_idx, void *dk_idx, void *dw, int dw_dtype, void *ws,
                                       size_t ws_bytes, void *stream) {
     if (int rc = check_packed(T, N, cu)) return rc;
     if (dtype != DSA_DTYPE_BF16) return fail(DSA_ERR_UNSUPPORTED, "indexer tensors must be bf16 (dtype code %d)", dtype);
     if (Hi < 1 || Hi > 64) return fail(DSA_ERR_UNSUPPORTED, "Hi=%d: 1..64 indexer heads", Hi);
     if (!(Di == 64 || Di == 128)) return fail(DSA_ERR_UNSUPPORTED, "Di=%d: the indexer backward covers 64 and 128", Di);
+    if (dw_dtype != DSA_DTYPE_BF16 && dw_dtype != DSA_DTYPE_FP32) return fail(DSA_ERR_ARG, "dw dtype code %d", dw_dtype);
     if (K < 1) return fail(DSA_ERR_ARG, "top_k=%d must be >= 1", K);
     if (!q_idx || !k_idx || !w_idx || !idx || !n || !dscore || !dq_idx || !dk_idx || !dw) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
@@ -499,7 +502,7 @@ extern "C" int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, cons
     }
     int rc = DSA_OK;
     e = dsa_launch_indexer_bwd(q_idx, k_idx, w_idx, dscore, grad, bitmap, prefix, w_f32, ldw, cu, N, T, Hi, Di, K, scale, dq_idx, dk_idx, dw,
-                               partial, st, sq);
+                               dw_dtype == DSA_DTYPE_BF16, partial, st, sq);
     if (e != hipSuccess) rc = hip_fail(e, "indexer backward launch");
     if (ov) {
         e = hipEventRecord(ov->join, ov->aux);
@@ -514,7 +517,7 @@ extern "C" int dsa_indexer_bwd(const void *q_idx, const void *k_idx, const void 
                                int dtype, int max_seqlen, void *dq_idx, void *dk_idx, float *dw, void *ws, size_t ws_bytes,
                                void *stream) {
     return dsa_indexer_bwd_scaled(q_idx, k_idx, w_idx, idx, n, dscore, nullptr, cu, T, N, Hi, Di, K, scale, dtype, max_seqlen, dq_idx,
-                                  dk_idx, dw, ws, ws_bytes, stream);
+                                  dk_idx, dw, DSA_DTYPE_FP32, ws, ws_bytes, stream);
 }
 
 extern "C" size_t dsa_attn_bwd_workspace_bytes(int T, int Hq, int max_seqlen, int has_idx) {
@@ -801,6 +804,23 @@ extern "C" int dsa_sigmoid_gate_bwd(const void *gy, const void *x, const void *g
     hipError_t e = dsa_launch_sigmoid_gate_bwd(gy, x, gate, gate_tok, gate_head, D, H, T, dx, dgate, dgate_tok, dgate_head,
                                                (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "sigmoid gate backward launch");
+}
+
+// ---- several (T, width) bf16 tensors side by side in one row-major buffer ----
+extern "C" int dsa_pack_columns(int n, const void *const *src, const int32_t *width, const int32_t *group, const int32_t *dst_col,
+                                const int32_t *dst_group, int T, void *dst, int64_t dst_row, void *stream) {
+    if (n < 1 || n > DSA_PACK_MAX || T < 0 || !src || !width || !group || !dst_col || !dst_group || dst_row < 8 || dst_row % 8)
+        return fail(DSA_ERR_ARG, "n=%d T=%d row=%lld", n, T, (long long)dst_row);
+    for (int i = 0; i < n; ++i) {
+        if (width[i] < 8 || width[i] % 8 || group[i] < 8 || group[i] % 8 || width[i] % group[i] || dst_col[i] < 0 || dst_col[i] % 8 ||
+            dst_group[i] < group[i] || dst_group[i] % 8 || dst_col[i] + (int64_t)(width[i] / group[i] - 1) * dst_group[i] + group[i] > dst_row)
+            return fail(DSA_ERR_ARG, "source %d: width %d in groups of %d at column %d, %d apart", i, width[i], group[i], dst_col[i], dst_group[i]);
+        if (T > 0 && (!src[i] || ((uintptr_t)src[i] & 15))) return fail(DSA_ERR_ARG, "source %d: null or not on a 16-byte boundary", i);
+    }
+    if (T == 0) return DSA_OK;
+    if (!dst || ((uintptr_t)dst & 15)) return fail(DSA_ERR_ARG, "destination null or not on a 16-byte boundary");
+    hipError_t e = dsa_launch_pack_columns(n, src, width, group, dst_col, dst_group, T, dst, dst_row, (hipStream_t)stream);
+    return e == hipSuccess ? DSA_OK : hip_fail(e, "pack columns launch");
 }
 
 // ---- fp32 operands carried as stacked split-bf16 rows (the host operator's fp32 path for head_dim <= 64) ----

@@ -369,6 +369,47 @@ extern "C" hipError_t dsa_launch_sigmoid_gate_bwd(const void *gy, const void *x,
     return hipGetLastError();
 }
 
+// ---- several (T, width) bf16 tensors side by side in one row-major buffer: the gradients of a layer's projections, so that one
+// GEMM gives all their weight gradients.  A source row of `width` elements goes to column dst_col in groups of `group` elements
+// dst_group apart (the two halves of an interleaved projection).  A thread keeps its 16-byte column over the rows: the search for
+// its source is done once, and four rows are in flight.  Bound by memory: 102 MB of gradients (8192 tokens, six projections), 38 us = 5.4 TB/s.
+struct PackArgs { const bf16_t *src[8]; int width[8], group[8], dst_col[8], dst_group[8], n; };
+__global__ __launch_bounds__(256) void dsa_pack_columns_kernel(PackArgs a, int T, bf16_t *__restrict__ dst, int64_t dst_row) {
+    int c = (blockIdx.x * 256 + threadIdx.x) * 8, i = 0;
+    while (i < a.n && c >= a.width[i]) c -= a.width[i++];
+    if (i == a.n) return;
+    const bf16_t *const src = a.src[i] + c;
+    const int64_t w = a.width[i];
+    bf16_t *const d = dst + a.dst_col[i] + c / a.group[i] * a.dst_group[i] + c % a.group[i];
+    constexpr int U = 4;
+    for (int t0 = blockIdx.y * U; t0 < T; t0 += gridDim.y * U) {
+        u32x4 x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + min(t0 + u, T - 1) * w));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (t0 + u < T) *reinterpret_cast<u32x4 *>(d + (t0 + u) * dst_row) = x[u];
+    }
+}
+extern "C" hipError_t dsa_launch_pack_columns(int n, const void *const *src, const int32_t *width, const int32_t *group, const int32_t *dst_col,
+                                              const int32_t *dst_group, int T, void *dst, int64_t dst_row, hipStream_t stream) {
+    PackArgs a;
+    int64_t chunks = 0;
+    a.n = n;
+    for (int i = 0; i < n; ++i) {
+        a.src[i] = (const bf16_t *)src[i];
+        a.width[i] = width[i];
+        a.group[i] = group[i];
+        a.dst_col[i] = dst_col[i];
+        a.dst_group[i] = dst_group[i];
+        chunks += width[i] / 8;
+    }
+    const int rows = (T + 3) / 4;
+    hipLaunchKernelGGL(dsa_pack_columns_kernel, dim3((unsigned)((chunks + 255) / 256), (unsigned)(rows < 2048 ? rows : 2048)), dim3(256), 0, stream, a, T,
+                       (bf16_t *)dst, dst_row);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------------------------------
 // fp32 operands on the bf16 kernels: x = hi + lo with hi = bf16(x), lo = bf16(x - hi), the parts stacked along
 // head_dim into rows of 4*D bf16 so that the products of the stacked operands give back near-fp32 logits:

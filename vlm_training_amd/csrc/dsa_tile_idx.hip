@@ -158,7 +158,7 @@ template <int D, int GSHIFT, int NW>
 __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel(
     const bf16_t *__restrict__ q_idx, const bf16_t *__restrict__ k_idx, const bf16_t *__restrict__ w_idx,
     const float *__restrict__ dscore, const float *__restrict__ grad, const uint32_t *__restrict__ bitmap, int ldw,
-    const int32_t *__restrict__ cu, int N, int T, int Hi, int K, float cscale, bf16_t *__restrict__ dq_idx, float *__restrict__ dw) {
+    const int32_t *__restrict__ cu, int N, int T, int Hi, int K, float cscale, bf16_t *__restrict__ dq_idx, void *__restrict__ dw, int dw_bf16) {
     typedef DirectTile<D> TL;
     constexpr int KS = D / 16, DT = D / 32, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT, LPW = TL::LOADS / NW;
     static_assert(TL::LOADS % NW == 0 && GSHIFT >= 5, "a wave's 32 rows are heads of one query");
@@ -247,7 +247,10 @@ __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel
         bf16_t *op = dq_idx + ((int64_t)t * Hi + hrow) * D;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, acc[dt], cscale * wrow_v, h);
-        if (h == 0) dw[(int64_t)t * Hi + hrow] = dwt * cscale;
+        if (h == 0) {
+            if (dw_bf16) reinterpret_cast<bf16_t *>(dw)[(int64_t)t * Hi + hrow] = (bf16_t)(dwt * cscale);
+            else reinterpret_cast<float *>(dw)[(int64_t)t * Hi + hrow] = dwt * cscale;
+        }
     }
 }
 
@@ -433,7 +436,7 @@ static int idxk_chunk(int T, int Di, int ldw) {
 template <int D, int GS>
 static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const void *k_idx, const void *w_idx, const float *w_f32, const float *dscore,
                              const float *grad, const uint32_t *bitmap, const int32_t *prefix, int ldw, const int32_t *cu, int N, int T, int Hi,
-                             int K, float cscale, void *dq_idx, void *dk_idx, float *dw, float *partial, hipStream_t stream_q) {
+                             int K, float cscale, void *dq_idx, void *dk_idx, void *dw, int dw_bf16, float *partial, hipStream_t stream_q) {
     constexpr int NW = D == 128 ? 8 : 4;                 // (waves that share the staged key tiles)
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_tile_idxk_kernel<D, GS>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)idxk_lds_bytes<D>());
@@ -451,7 +454,7 @@ static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const 
     const dim3 gq((unsigned)((int64_t)T / ((32 * NW) >> GS) + N + 1));
     hipLaunchKernelGGL((dsa_tile_idxq_kernel<D, GS, NW>), gq, dim3(64 * NW), (idxq_lds_bytes<D, NW>()), stream_q, (const bf16_t *)q_idx,
                        (const bf16_t *)k_idx, (const bf16_t *)w_idx, dscore, grad, bitmap, ldw, cu, N, T, Hi, K, cscale,
-                       (bf16_t *)dq_idx, dw);
+                       (bf16_t *)dq_idx, dw, dw_bf16);
     return hipGetLastError();
 }
 extern "C" size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw) {
@@ -462,11 +465,11 @@ extern "C" size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw) {
 extern "C" hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore, const float *grad,
                                              const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N,
                                              int T, int Hi, int Di, int K, float cscale, void *dq_idx, void *dk_idx,
-                                             float *dw, float *partial, hipStream_t stream, hipStream_t stream_q) {
+                                             void *dw, int dw_bf16, float *partial, hipStream_t stream, hipStream_t stream_q) {
     if (Hi < 1 || Hi > 64 || !(Di == 64 || Di == 128)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(dsa_bitmap_prefix_kernel, dim3(T), dim3(64), 0, stream, bitmap, ldw, prefix, (const bf16_t *)w_idx, Hi, w_f32);
 #define IDX_BWD(D_, GS_) launch_idx_bwd_i<D_, GS_>(stream, q_idx, k_idx, w_idx, w_f32, dscore, grad, bitmap, prefix, ldw, cu, N, T, Hi, K, \
-                                                   cscale, dq_idx, dk_idx, dw, partial, stream_q)
+                                                   cscale, dq_idx, dk_idx, dw, dw_bf16, partial, stream_q)
     if (Di == 128) return Hi > 32 ? IDX_BWD(128, 6) : IDX_BWD(128, 5);
     return Hi > 32 ? IDX_BWD(64, 6) : IDX_BWD(64, 5);
 #undef IDX_BWD

@@ -8,7 +8,7 @@
 * ``DsaIndexer``            - the lightning indexer's projections as module parameters (the reference holds no
   indexer): hidden -> Hi*Di index queries, hidden -> Di index key (one per token), hidden -> Hi head weights.
 
-The projections stay torch GEMMs.  Norm + RoPE + layout is one kernel (``qk_norm_rope``), the attention is
+The projections stay torch GEMMs (plain ones share one autograd node: ``_projections``).  Norm + RoPE + layout is one kernel (``qk_norm_rope``), the attention is
 ``dsa_varlen_attn`` (dense causal without an indexer: the reference's behaviour), the gate is one kernel.
 With an indexer the layer keeps the top-k keys per query and leaves the indexer's KL loss in ``self.indexer_loss``
 (the selection passes no gradient; the loss is what trains the indexer); ``indexer_losses(model)`` adds them up
@@ -22,6 +22,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
+from . import _lib
 from .dtensor_utils import _dtensor_rewrap, _dtensor_unwrap, _local
 from .model_attention import run_varlen_attn
 from .ops import dsa_varlen_attn, indexer_kl_loss
@@ -58,14 +59,42 @@ class DsaIndexer(nn.Module):
         return iq, self.k_proj(h), self.w_proj(h)
 
 
+def _fusible(lin, x) -> bool:
+    w = getattr(lin, "weight", None)
+    return (type(lin) is nn.Linear and lin.bias is None and type(w) is nn.Parameter and w.dtype == torch.bfloat16 and w.device == x.device
+            and w.shape[0] % 8 == 0 and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks))
+
+
+@torch.compiler.disable
+def _projections(x, linears, indexer, gate_dim: int = 0):
+    """Outputs of ``linears`` (and of the indexer's projections, which read ``x`` detached) as one autograd node whose backward
+    runs one weight-gradient GEMM for all of them (``ProjectionNode`` in csrc/dsa_host.cpp).  ``gate_dim``: the first output
+    comes as its two interleaved halves.  None where the modules have to be called one by one: other module types, biases,
+    hooks, sharded or non-bf16 weights, autocast, no gradient wanted."""
+    mods = list(linears) + ([indexer.q_proj, indexer.k_proj, indexer.w_proj] if indexer is not None else [])
+    if not (type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled()
+            and x.numel() >= 1 << 19          # (256 tokens of 2048; below, a step is bound by the host and the GEMMs are all short)
+            and not torch.is_autocast_enabled("cuda") and all(_fusible(m, x) for m in mods)):
+        return None
+    if indexer is not None and (type(indexer) is not DsaIndexer or indexer._forward_hooks or indexer._forward_pre_hooks
+                                or indexer._backward_hooks or indexer._backward_pre_hooks):
+        return None
+    h = x.reshape(-1, x.shape[-1])
+    return _lib.host().project(h, [m.weight for m in mods], len(linears), gate_dim)
+
+
 def _bf16(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)
 
 
-def attention_core(module, q_lin, k_lin, v_lin, cos, sin, cu_seqlens, max_seqlen, x=None, gate=None, offset=False):
+def _index_of(indexer, outs):
+    return (outs[0].view(outs[0].shape[0], indexer.cfg.index_heads, indexer.cfg.index_dim), outs[1], outs[2]) if outs else None
+
+
+def attention_core(module, q_lin, k_lin, v_lin, cos, sin, cu_seqlens, max_seqlen, x=None, gate=None, offset=False, index=None):
     """(T,Hq,D), (T,Hkv,D), (T,Hkv,D) projection outputs (views with any token / head stride) -> (T,Hq,D).
 
-    ``module`` supplies ``q_norm`` / ``k_norm`` (weight, eps) and optionally ``indexer``; the indexer's loss is left
+    ``index``: the indexer's three projections of ``x`` if the caller has them already.  ``module`` supplies ``q_norm`` / ``k_norm`` (weight, eps) and optionally ``indexer``; the indexer's loss is left
     in ``module.indexer_loss``."""
     eps = getattr(module.q_norm, "eps", None)
     if eps is None:
@@ -79,14 +108,14 @@ def attention_core(module, q_lin, k_lin, v_lin, cos, sin, cu_seqlens, max_seqlen
         out = dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen)
     else:
         cfg = indexer.cfg
-        iq, ik, iw = indexer(x)
+        iq, ik, iw = indexer(x) if index is None else index
         want_loss = torch.is_grad_enabled() and any(p.requires_grad for p in indexer.parameters())
         if want_loss:
             out, idx, n, mass, sel = dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen, indexer_q=iq, indexer_k=ik, indexer_w=iw,
                                                      top_k=cfg.top_k, index_scale=cfg.index_scale, return_indices=True,
                                                      return_mass=True, return_scores=True)
-            module.indexer_loss = cfg.loss_weight * indexer_kl_loss(iq, ik, iw, mass, cu_seqlens, max_seqlen, cfg.top_k,
-                                                                     cfg.index_scale, selection=(idx, n, sel))
+            loss = indexer_kl_loss(iq, ik, iw, mass, cu_seqlens, max_seqlen, cfg.top_k, cfg.index_scale, selection=(idx, n, sel))
+            module.indexer_loss = loss if cfg.loss_weight == 1.0 else cfg.loss_weight * loss
         else:
             out = dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen, indexer_q=iq, indexer_k=ik, indexer_w=iw,
                                   top_k=cfg.top_k, index_scale=cfg.index_scale)
@@ -153,6 +182,11 @@ class Qwen3VLTextAttention(nn.Module):
     def forward(self, x, cos, sin, cu_seqlens, max_seqlen):
         total = x.shape[1]
         # head counts come from the projections' outputs, so a head-sharded (tensor-parallel) layer sees its own
+        lin = _projections(x, (self.q_proj, self.k_proj, self.v_proj), self.indexer)
+        if lin is not None:
+            q, k, v = (y.view(total, -1, self.head_dim) for y in lin[:3])
+            out = attention_core(self, q, k, v, cos, sin, cu_seqlens, max_seqlen, x=x, index=_index_of(self.indexer, lin[3:]))
+            return self.o_proj(out.reshape(1, total, -1).to(x.dtype))
         q = self.q_proj(x).view(total, -1, self.head_dim)
         k = self.k_proj(x).view(total, -1, self.head_dim)
         v = self.v_proj(x).view(total, -1, self.head_dim)
@@ -189,6 +223,12 @@ class SelfAttention(nn.Module):
     def forward(self, x, cos, sin, cu_seqlens, max_seqlen):
         total = x.shape[1]
         D = self.head_dim
+        lin = _projections(x, (self.q_proj, self.k_proj, self.v_proj), self.indexer, gate_dim=D)
+        if lin is not None:
+            q, gate, k, v = (y.view(total, -1, D) for y in lin[:4])
+            out = attention_core(self, q, k, v, cos, sin, cu_seqlens, max_seqlen, x=x, gate=gate, offset=True,
+                                 index=_index_of(self.indexer, lin[4:]))
+            return self.o_proj(out.reshape(1, total, -1).to(x.dtype))
         qg = self.q_proj(x).view(total, -1, 2 * D)              # per head [q | gate]: both halves are read in place
         k = self.k_proj(x).view(total, -1, D)
         v = self.v_proj(x).view(total, -1, D)
