@@ -76,36 +76,44 @@ __device__ __forceinline__ float group_sum(float x) {
 // A slot depends on its own tile alone, so a walk can be cut anywhere: launches that leave the chip idle (one workgroup
 // per CU: 64 queries of a 2B stack's 8192 tokens are 128 workgroups for 256 CUs) run pieces of `chunk` tiles as workgroups
 // of their own, each counting the selected keys in front of its piece first (there 189 -> 89 us).
+// Each wave runs two heads at once: the MFMAs of S for the next (tile, head) with the exponentials of this one behind them.  Key
+// tiles of all the heads go from memory straight into LDS, two slots: at the last head of tile t - every wave has read tile t by
+// then - the wave waits for tile t+1, meets the one barrier per tile and requests tile t+2.  The second set leaves its sums, added
+// up over the heads of a query first, in LDS in front of that barrier and the first set finishes tile t behind the next one.
+// What bounds it: the vector pipe, 16 exponentials of 16 clocks and 32 other instructions per head, tile and wave (384 clocks
+// against 256 of MFMA).  32 768 tokens, 32 heads of 128: 1110 -> 875 us (operands staged through registers, S and exponentials
+// one after the other, two barriers per tile before).
 template <int D> constexpr int mass_heads_max() { return 1024 / D; }      // 16 / 8 / 4 kv heads at head_dim 64 / 128 / 256
 template <int HPG> constexpr int mass_sets() { return HPG >= 2 ? 2 : 1; }
-template <int D, int HPG> constexpr size_t mass_lds_bytes() {
-    return (size_t)HPG * tile_bytes<D>() + (mass_sets<HPG>() == 2 ? 4 * 64 * 16 * sizeof(float) : 0);
+template <int D, int GSHIFT, int HPG> constexpr size_t mass_lds_bytes() {
+    return 2 * (size_t)HPG * DirectTile<D>::BYTES + 4 * 4 * 256 + (mass_sets<HPG>() == 2 ? 2 * 4 * 64 * (16 >> GSHIFT) * sizeof(float) : 0);
 }
 template <int D, int GSHIFT, int HPG>
 __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const float *__restrict__ lse,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
     float scale_log2, int K, int ngroups, int chunk, float final_mul, float *__restrict__ table) {
+    typedef DirectTile<D> TL;
     constexpr int NS = mass_sets<HPG>(), HPW = HPG / NS;       // wave sets; kv heads per wave
-    constexpr int KS = D / 16, CPR = D / 8, TILE_B = tile_bytes<D>(), NT = 256 * NS;
-    constexpr int Gp = 1 << GSHIFT, QBW = (4 * 32) >> GSHIFT;
-    constexpr int CH = 32 * HPG * CPR, LOADS = CH / NT;  // 16-byte chunks of one key tile of all HPG heads; per thread
-    static_assert(CH % NT == 0 && LOADS >= 1, "every thread stages the same number of chunks");
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_lds[];   // [HPG][TILE_B] | sums of the second set
-    float *const xbuf = reinterpret_cast<float *>(dyn_lds + HPG * TILE_B);
+    constexpr int KS = D / 16, NT = 256 * NS, Gp = 1 << GSHIFT, QBW = (4 * 32) >> GSHIFT, U = 16 / Gp;
+    constexpr int LPW = HPG * TL::LOADS / (4 * NS);            // wave loads per wave and tile
+    static_assert(HPG * TL::LOADS % (4 * NS) == 0 && LPW >= 1 && (LPW % 2 == 0 || TL::SOURCES == 1), "every wave loads the same number of pieces");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];   // [2][HPG] K tiles | words [quarter][tile % 4] | sums of the second set
+    constexpr int SLOT = HPG * TL::BYTES;
+    unsigned char *const words = dyn_lds + 2 * SLOT;
+    float *const xbuf = reinterpret_cast<float *>(words + 4 * 4 * 256);
 
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wq = wv & 3, set = wv >> 2;                // query quarter of the block; wave set
-    LaneOffsets<D> lo;
-    lo.init(lane);
     const int G = Hq / Hkv;
     const int grp = blockIdx.x % ngroups, kvh0 = grp * HPG;
     int s0, L, blk;
     // (heaviest block first over the whole batch: 1.21 against 1.37 ms for the segment-by-segment order at 32 768 tokens)
     if (!locate_block_heaviest_first(cu, N, blockIdx.x / ngroups, QBW, s0, L, blk)) return;
-    L = min(L, ldw * 32);                               // a bitmap row has ldw words whatever the caller's max_seqlen
-    const int qc0 = blk * QBW;
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    L = min(__builtin_amdgcn_readfirstlane(L), ldw * 32);      // a bitmap row has ldw words whatever the caller's max_seqlen
+    const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
     if (qc0 >= L) return;
 
     const int r = wq * 32 + j;
@@ -115,6 +123,35 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
     // this workgroup's piece of the walk: tiles [it0, ntiles)
     const int it0 = (int)blockIdx.y * chunk, ntiles = min((min(qc0 + QBW - 1, L - 1) / 32 + 1), it0 + chunk);
     if (it0 >= ntiles) return;
+
+    // ---- requests ----
+    const uint32_t lds0 = lds_address(dyn_lds);
+    const int tok_b = Hkv * D * 2;                       // bytes from one key row to the next
+    const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k + (int64_t)(s0 + it0 * 32) * Hkv * D);
+    int koff[TL::SOURCES];
+#pragma unroll
+    for (int i = 0; i < TL::SOURCES; ++i) koff[i] = TL::source(i, lane, tok_b, D / 8);
+    const int wq0 = min(qc0 + ((wq * 32) >> GSHIFT), L - 1);   // the wave's first query
+    const unsigned char *wptr = reinterpret_cast<const unsigned char *>(bitmap + (int64_t)(s0 + wq0) * ldw + it0);
+    const int wvoff = (t - s0 - wq0) * ldw * 4;
+    // the tiles of all heads (kv heads past the last one, in a short last group, repeat it and count for nothing: lse = +inf
+    // below; rows past the segment read as zero) and the selection words; called for tile it0, it0+1, ... in turn
+    auto request = [&](int tile) __attribute__((always_inline)) {
+        const buffer_rsrc keys = make_buffer_rsrc(kptr, (int64_t)max(min(L - tile * 32, 32), 0) * tok_b);
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) {
+            const int g = wv * LPW + i, hh = g / TL::LOADS, p = g % TL::LOADS;
+            buffer_load_lds16(keys, koff[i % TL::SOURCES] + (p / TL::SOURCES * TL::SOURCES) * TL::LOAD_ROWS * tok_b + min(kvh0 + hh, Hkv - 1) * D * 2, 0,
+                              lds0 + (tile & 1) * SLOT + hh * TL::BYTES + TL::load_lds(p));
+        }
+        kptr += (int64_t)32 * tok_b;
+        if (set == 0) {
+            buffer_load_lds4(make_buffer_rsrc(wptr, tile < ntiles ? 32 * (int64_t)ldw * 4 : 0), wvoff, 0, lds0 + 2 * SLOT + wq * 1024 + (tile & 3) * 256);
+            wptr += 4;
+        }
+    };
+    request(it0);
+    request(it0 + 1);
     const uint32_t *wrow = bitmap + (int64_t)t * ldw;
     float *prow = table + ((int64_t)grp * T + t) * K;
     if (ngroups == 1 && it0 == 0) {
@@ -124,23 +161,6 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
             for (int jj = qc0 + qq + 1 + tid; jj < K; jj += NT) zr[jj] = 0.f;
         }
     }
-    u32x4 kst[LOADS];
-    // one key row of the group's kv heads is contiguous in memory (HPG * D elements); kv heads past the last one
-    // (a short last group) read the last head again and count for nothing (lse = +inf below)
-#define MASS_LOAD(TILE)                                                                             \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                            \
-        const int c = i * NT + tid;                                                                \
-        const int row = c / (HPG * CPR), hh = (c / CPR) % HPG, ch = c % CPR;                       \
-        kst[i] = *reinterpret_cast<const u32x4 *>(                                                 \
-            k + ((int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * Hkv + min(kvh0 + hh, Hkv - 1)) * D + ch * 8); \
-    }
-#define MASS_STORE()                                                                                \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                            \
-        const int c = i * NT + tid;                                                                \
-        const int row = c / (HPG * CPR), hh = (c / CPR) % HPG, ch = c % CPR;                       \
-        *reinterpret_cast<u32x4 *>(&dyn_lds[hh * TILE_B + tile_off<D>(row, ch)]) = kst[i];         \
-    }
-    MASS_LOAD(it0)
     bf16x8 qB[HPW][KS];
     float lse2[HPW];
 #pragma unroll
@@ -156,73 +176,117 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
         const float lse_row = lse[(int64_t)hq * T + t];
         lse2[hh] = (row_ok && kvh0 + kv_rel < Hkv) ? lse_row * LOG2E_F : INFINITY;
     }
-    uint32_t word_next = qcol < L ? wrow[it0] : 0u;
     int seen = 0;                                        // selected keys of this row in the tiles before this one
     for (int w = 0; w < it0; w += 8)                     // (it0 is a multiple of 8)
 #pragma unroll
         for (int u = 0; u < 8; ++u) seen += __popc(wrow[w + u]);
-    MASS_STORE()
-    __syncthreads();
-    for (int it = it0; it < ntiles; ++it) {
-        MASS_LOAD(min(it + 1, ntiles - 1))               // lands during this tile's matrix work
-        const uint32_t word_full = word_next;
-        { const uint32_t wl = wrow[min(it + 1, ntiles - 1)]; word_next = qcol < L ? wl : 0u; }
-        float p[16];
+    TL tl;
+    tl.init(lane);
+    wait_vmcnt<0>();
+    barrier_only();
+
+    int ka[4];                                           // operand addresses in the tile of the next S
+    bf16x8 kr[4];
+    auto read_k = [&](int ks) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8 *>(dyn_lds + ka[TL::row_q(ks)] + TL::row_imm(ks));
+    };
+    auto first_reads = [&](int tile, int hh) __attribute__((always_inline)) {
 #pragma unroll
-        for (int vi = 0; vi < 16; ++vi) p[vi] = 0.f;
+        for (int i = 0; i < 4; ++i) ka[i] = tl.rowq[i] + (tile & 1) * SLOT + (set * HPW + hh) * TL::BYTES;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kr[i] = read_k(i);
+    };
+    float val[U];                                        // the elements u * Gp + head of the last tile's sums
+    // tile's sums finished and stored: the lanes of a query share the stores, lane `head` has the elements vi = u*Gp + head
+    auto finish = [&](int tile) __attribute__((always_inline)) {
+        if (set != 0) return;
+        const uint32_t wl = *reinterpret_cast<const uint32_t *>(words + wq * 1024 + (tile & 3) * 256 + lane * 4);
+        const uint32_t word = qcol < L ? wl : 0u;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float x = val[u];
+            if (NS == 2) x += xbuf[(((tile & 1) * 4 + wq) * U + u) * 64 + lane];
+            const int vi = u * Gp + head;
+            const int bit = 8 * (vi >> 2) + (vi & 3) + 4 * h;    // the key's column in the tile
+            if ((word >> bit) & 1u) prow[seen + __popc(word & ((1u << bit) - 1u))] = x * final_mul;
+        }
+        seen += __popc(word);
+    };
+    float p[16];
+    // exponentials of (this tile, head hh) from `s` behind the MFMAs of the next S into `sn` (NEXT: with `qn`)
+    auto stage = [&](auto next_, int hh, const f32x16 &s, const bf16x8 (&qn)[KS], f32x16 &sn) __attribute__((always_inline)) {
+        constexpr bool NEXT = decltype(next_)::value;
+        const float neg = -lse2[hh];
+        f32x16 snew;
+        auto behind = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int vi = 16 * i / KS; vi < 16 * (i + 1) / KS; ++vi) {
+                const float e = fast_exp2(fmaf(s[vi], scale_log2, neg));
+                p[vi] = hh == 0 ? e : p[vi] + e;
+                asm volatile("" : "+v"(p[vi]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            if (NEXT) {
+                snew = mfma32(kr[i & 3], qn[i], i == 0 ? zero16() : snew);
+                if (i + 4 < KS) kr[i & 3] = read_k(i + 4);
+            }
+            behind(i);
+        }
+        if (NEXT) sn = snew;
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    f32x16 sA, sB;
+    // one tile: S of its first head in sA; leaves S of the next tile's first head there (LAST: there is none)
+    auto tile_step = [&](auto last_, int it) __attribute__((always_inline)) {
+        constexpr bool LAST = decltype(last_)::value;
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
-            // (issuing the matrix work of head hh+1 between the exponentials of head hh in a hand-fixed order
-            // measured no faster than what the scheduler makes of this loop)
-            const unsigned char *kt = dyn_lds + (set * HPW + hh) * TILE_B;
-            f32x16 sacc = zero16();
-            constexpr int KH = KS >= 8 ? KS / 2 : KS;    // K operands in flight: half a tile row (registers are short here)
-#pragma unroll
-            for (int k0 = 0; k0 < KS; k0 += KH) {
-                bf16x8 ka[KH];
-#pragma unroll
-                for (int ks = 0; ks < KH; ++ks) ka[ks] = lo.rowop(kt, k0 + ks);
-#pragma unroll
-                for (int ks = 0; ks < KH; ++ks) sacc = mfma32(ka[ks], qB[hh][k0 + ks], sacc);
-            }
-#pragma unroll
-            for (int vi = 0; vi < 16; ++vi) p[vi] += fast_exp2(fmaf(sacc[vi], scale_log2, -lse2[hh]));
-        }
-        if (NS == 2 && set == 1) {                       // the second set's sums: [quarter][element / 4][lane] x 16 bytes
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const f32x4 v4 = {p[4 * c], p[4 * c + 1], p[4 * c + 2], p[4 * c + 3]};
-                *reinterpret_cast<f32x4 *>(xbuf + ((wq * 4 + c) * 64 + lane) * 4) = v4;
-            }
-        }
-        __syncthreads();                                 // every wave is done with this tile's K; the sums are in place
-        MASS_STORE()
-        if (set == 0) {
-            if (NS == 2) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const f32x4 v4 = *reinterpret_cast<const f32x4 *>(xbuf + ((wq * 4 + c) * 64 + lane) * 4);
-                    p[4 * c] += v4[0]; p[4 * c + 1] += v4[1]; p[4 * c + 2] += v4[2]; p[4 * c + 3] += v4[3];
+            f32x16 &s = hh & 1 ? sB : sA, &sn = hh & 1 ? sA : sB;
+            if (hh + 1 < HPW) {
+                first_reads(it, hh + 1);
+                stage(yes, hh, s, qB[hh + 1 < HPW ? hh + 1 : 0], sn);
+            } else {
+                // every wave has read this tile; the sums of the one before are in place
+                wait_vmcnt<0>();
+                asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+                barrier_only();
+                if (it > it0) finish(it - 1);
+                if (!LAST) {
+                    request(it + 2);
+                    first_reads(it + 1, 0);
+                    stage(yes, hh, s, qB[0], sn);
+                    if (hh % 2 == 0) sA = sB;            // (an odd number of heads)
+                } else {
+                    stage(no, hh, s, qB[0], sn);
                 }
             }
-#pragma unroll
-            for (int vi = 0; vi < 16; ++vi) p[vi] = group_sum<GSHIFT>(p[vi]);
-            // the lanes of a query share the stores: lane `head` writes the elements vi = u*Gp + head
-#pragma unroll
-            for (int u = 0; u < 16 / Gp; ++u) {
-                float val = p[u * Gp];
-#pragma unroll
-                for (int g = 1; g < Gp; ++g) val = head == g ? p[u * Gp + g] : val;
-                const int vi = u * Gp + head;
-                const int bit = 8 * (vi >> 2) + (vi & 3) + 4 * h;    // the key's column in the tile
-                if ((word_full >> bit) & 1u) prow[seen + __popc(word_full & ((1u << bit) - 1u))] = val * final_mul;
-            }
         }
-        seen += __popc(word_full);
-        __syncthreads();                                 // the next tile's K is staged; the sums have been read
+#pragma unroll
+        for (int vi = 0; vi < 16; ++vi) p[vi] = group_sum<GSHIFT>(p[vi]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            val[u] = p[u * Gp];
+#pragma unroll
+            for (int g = 1; g < Gp; ++g) val[u] = head == g ? p[u * Gp + g] : val[u];
+            if (NS == 2 && set == 1) xbuf[(((it & 1) * 4 + wq) * U + u) * 64 + lane] = val[u];
+        }
+    };
+    first_reads(it0, 0);
+    sA = zero16();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        sA = mfma32(kr[ks & 3], qB[0][ks], sA);
+        if (ks + 4 < KS) kr[ks & 3] = read_k(ks + 4);
     }
-#undef MASS_LOAD
-#undef MASS_STORE
+    for (int it = it0; it + 1 < ntiles; ++it) tile_step(no, it);
+    tile_step(yes, ntiles - 1);
+    wait_vmcnt<0>();                                    // no load is left on its way into LDS when the workgroup ends
+    __syncthreads();
+    finish(ntiles - 1);
 }
 
 // mass[t,j] = inv_hq * sum over the tables of partial[g][t][j] for j < n[t], else 0.  One workgroup per query row
@@ -1629,13 +1693,13 @@ template <int D, int GS, int HPG>
 static hipError_t launch_mass_h(dim3 grid, hipStream_t stream, const void *q, const void *k, const float *lse,
                                 const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float sl2,
                                 int K, int ngroups, int chunk, float final_mul, float *table) {
-    if constexpr (HPG > mass_heads_max<D>()) {
+    if constexpr (HPG > (GS == 0 ? mass_heads_max<D>() / 2 : mass_heads_max<D>())) {     // (mass_hpg asks for no more)
         return hipErrorInvalidValue;
     } else {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_tile_mass_kernel<D, GS, HPG>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)mass_lds_bytes<D, HPG>());
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)mass_lds_bytes<D, GS, HPG>());
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((dsa_tile_mass_kernel<D, GS, HPG>), grid, dim3(256 * mass_sets<HPG>()), (mass_lds_bytes<D, HPG>()), stream,
+        hipLaunchKernelGGL((dsa_tile_mass_kernel<D, GS, HPG>), grid, dim3(256 * mass_sets<HPG>()), (mass_lds_bytes<D, GS, HPG>()), stream,
                            (const bf16_t *)q, (const bf16_t *)k, lse, bitmap, ldw, cu, N, T, Hq, Hkv, sl2, K, ngroups, chunk,
                            final_mul, table);
         return hipSuccess;
