@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <optional>
 #include <vector>
 
@@ -301,6 +302,26 @@ Tensor dense_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Te
     check(dsa_dense_fwd_strided(ptr(q), q.stride(0), q.stride(1), ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1), iptr(cu), (int)s.T,
                                 (int)cu.numel() - 1, (int)s.Hq, (int)s.Hkv, (int)s.D, (float)scale, DSA_DTYPE_BF16, (int)max_seqlen, causal, ptr(out),
                                 fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
+    return out;
+}
+
+// The same for an HF module's (1, H, T, D) tensors, (1, T, Hq, D) out: every view and check of that call in one place (a short
+// generation-time batch spends 8 us on the GPU, and the views, wrappers and checks in Python took the host 15).  Nothing where
+// the general path has to be taken.
+std::optional<Tensor> hf_dense_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &mask, std::optional<int64_t> max_seqlen) {
+    auto fits = [](const Tensor &t) {
+        return t.dim() == 4 && t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.size(0) == 1 && t.stride(3) == 1 && t.size(3) % 8 == 0 &&
+               t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && t.stride(2) < (1 << 24) && aligned16(t);
+    };
+    if (!fits(q) || !fits(k) || !fits(v) || !mask.is_cuda() || needs_grad(q, k, v) || std::getenv("DSA_DEBUG_META")) return std::nullopt;
+    const int64_t Hq = q.size(1), Hkv = k.size(1), T = q.size(2), D = q.size(3);
+    if (k.sizes() != v.sizes() || k.size(2) != T || k.size(3) != D || D > 256 || !Hkv || Hq % Hkv) return std::nullopt;
+    const c10::OptionalDeviceGuard guard(q.device());
+    const Tensor cu = checked_cu(mask.dim() == 1 ? mask : mask.squeeze());
+    const Tensor out = empty({1, T, Hq, D}, at::kBFloat16, q), lse = empty({Hq, T}, at::kFloat, q);
+    check(dsa_dense_fwd_strided(ptr(q), q.stride(2), q.stride(1), ptr(k), k.stride(2), k.stride(1), ptr(v), v.stride(2), v.stride(1), iptr(cu), (int)T,
+                                (int)cu.numel() - 1, (int)Hq, (int)Hkv, (int)D, (float)std::pow((double)D, -0.5), DSA_DTYPE_BF16,
+                                (int)max_seqlen.value_or(T), 1, ptr(out), fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
     return out;
 }
 
@@ -636,6 +657,7 @@ Tensor sigmoid_gate(const Tensor &x, const Tensor &gate) { return SigmoidGateNod
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const auto nogil = py::call_guard<py::gil_scoped_release>();
     m.def("varlen_attn", &varlen_attn, nogil);
+    m.def("hf_dense_forward", &hf_dense_forward, nogil);
     m.def("attn_node", &attn_node, nogil);
     m.def("indexer_kl_loss", &indexer_kl_loss, nogil);
     m.def("qk_norm_rope", &qk_norm_rope, nogil);

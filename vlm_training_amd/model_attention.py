@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
 from .ops import dsa_varlen_attn
 
 _DSA_KEYS = ("indexer_q", "indexer_k", "indexer_w", "top_k", "index_scale", "return_indices", "return_mass", "return_scores")
@@ -74,8 +75,7 @@ def _hf_indexer_to_packed(x):
 _BOUND_ATTR = "_dsa_longest_segment"      # (version, storage offset, numel, bound), kept on the tensor that owns the memory
 
 
-@torch.compiler.disable                 # reads a value back from the device and writes an attribute: never part of a traced graph
-def longest_segment(cu_seqlens) -> int:
+def _longest_segment(cu_seqlens):
     """Longest segment of a packed row, read back from the device once per ``cu_seqlens`` tensor: every layer of a
     step hands over the same tensor (or a view of it), so the copy (and its stall) is paid once per batch instead of
     once per layer as in the reference (train/model_attention.py:120-121).
@@ -101,12 +101,21 @@ def longest_segment(cu_seqlens) -> int:
     return bound
 
 
+# reads a value back from the device and writes an attribute: never part of a traced graph
+longest_segment = torch.compiler.disable(_longest_segment)
+
+
 def varlen_attention_forward(query, key, value, attention_mask, max_seqlen=None, **dsa):
     """(1,Hq,T,D),(1,Hkv,T,D),(1,Hkv,T,D), cu_seqlens -> ((1,T,Hq,D), None).
 
     ``max_seqlen`` (keyword, not in the reference's signature): the longest segment if the caller holds it; otherwise
     it is read from ``cu_seqlens`` once per tensor (``longest_segment``).  The selection bitmap and the score rows of
     the DSA path are sized by it, so a tight bound matters there."""
+    if not dsa and type(query) is type(key) is type(value) is torch.Tensor and not torch.compiler.is_compiling():
+        out = _lib.host().hf_dense_forward(query, key, value, attention_mask,
+                                           int(max_seqlen) if max_seqlen is not None else _longest_segment(attention_mask.squeeze()))
+        if out is not None:
+            return out, None
     # tensor-parallel runs hand over DTensors sharded by head: the kernels see the local shard
     # (train/model_attention.py:104-106)
     query, key, value = (x.to_local() if hasattr(x, "to_local") else x for x in (query, key, value))
