@@ -1,5 +1,5 @@
-// Tile kernels: dQ / dK,dV and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask (the forward:
-// dsa_tile_fwd.hip, the indexer backward: dsa_tile_idx.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
+// Tile kernels: dK / dV, dQ at head_dim 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask (the forward:
+// dsa_tile_fwd.hip, dQ but for head_dim 128: dsa_tile_dq.hip, the indexer backward: dsa_tile_idx.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
 // 4*G*D flop on the matrix cores - on MI355X the tile walk is cheaper down to a few percent density.
@@ -13,36 +13,6 @@
 //   The second GEMM of each chain takes its B operand straight from the C layout of the first
 //   (the contraction order over the 32 keys/rows of a tile is permuted identically on both operands).
 #include "dsa_tile.h"
-
-// K/V tiles of the query-stationary kernels are fetched two tiles ahead into registers and one tile ahead into LDS (double
-// buffer), so a global load has two tile-times to land; one barrier per tile.
-// Every global load of the pipeline is issued unconditionally (indices past the end are clamped to
-// the last tile) and nothing is computed from a loaded value before the matching STORE, so the
-// compiler can wait with exact vmcnt counts and a load has two tile-times to land.  The kernel issues
-// LOAD(0, 0) itself, before the loads of its stationary rows.
-#define TILE_PIPELINE(NT, LOAD, STORE, COMPUTE)                                                     \
-    {                                                                                              \
-        const int nt_last = (NT) - 1;                                                              \
-        STORE(0, 0, 0);                                                                            \
-        LOAD(0, min(1, nt_last));                                                                  \
-        LOAD(1, min(2, nt_last));                                                                  \
-        __syncthreads();                                                                           \
-        int it = 0;                                                                                \
-        for (; it + 1 < (NT); it += 2) {                                                           \
-            /* LDS buffer 0 holds tile it, register set 0 tile it+1, register set 1 tile it+2 */     \
-            COMPUTE(it, 0);                                                                        \
-            if (NBUF == 1) __syncthreads();                                                        \
-            STORE(0, NBUF - 1, it + 1);                                                            \
-            LOAD(0, min(it + 3, nt_last));                                                         \
-            __syncthreads();                                                                       \
-            COMPUTE(it + 1, NBUF - 1);                                                             \
-            if (NBUF == 1) __syncthreads();                                                        \
-            STORE(1, 0, min(it + 2, nt_last));                                                     \
-            LOAD(1, min(it + 4, nt_last));                                                         \
-            __syncthreads();                                                                       \
-        }                                                                                          \
-        if (it < (NT)) COMPUTE(it, 0);                                                             \
-    }
 
 // ==================================================================================================
 // attention mass: the indexer's training target.  Same walk and S^T = K Q^T as the forward, with the
@@ -321,6 +291,34 @@ __global__ __launch_bounds__(256) void dsa_mass_reduce_kernel(const float *__res
     }
 }
 
+// K/V tiles of the query-stationary kernels are fetched two tiles ahead into registers and one tile ahead into LDS (double
+// buffer), so a global load has two tile-times to land; one barrier per tile.
+// Every global load of the pipeline is issued unconditionally (indices past the end are clamped to
+// the last tile) and nothing is computed from a loaded value before the matching STORE, so the
+// compiler can wait with exact vmcnt counts and a load has two tile-times to land.  The kernel issues
+// LOAD(0, 0) itself, before the loads of its stationary rows.
+#define TILE_PIPELINE(NT, LOAD, STORE, COMPUTE)                                                     \
+    {                                                                                              \
+        const int nt_last = (NT) - 1;                                                              \
+        STORE(0, 0, 0);                                                                            \
+        LOAD(0, min(1, nt_last));                                                                  \
+        LOAD(1, min(2, nt_last));                                                                  \
+        __syncthreads();                                                                           \
+        int it = 0;                                                                                \
+        for (; it + 1 < (NT); it += 2) {                                                           \
+            /* LDS buffer 0 holds tile it, register set 0 tile it+1, register set 1 tile it+2 */     \
+            COMPUTE(it, 0);                                                                        \
+            STORE(0, 1, it + 1);                                                            \
+            LOAD(0, min(it + 3, nt_last));                                                         \
+            __syncthreads();                                                                       \
+            COMPUTE(it + 1, 1);                                                             \
+            STORE(1, 0, min(it + 2, nt_last));                                                     \
+            LOAD(1, min(it + 4, nt_last));                                                         \
+            __syncthreads();                                                                       \
+        }                                                                                          \
+        if (it < (NT)) COMPUTE(it, 0);                                                             \
+    }
+
 // ==================================================================================================
 // dQ: query-stationary, same walk as the forward.
 //   S^T = K Q^T, dP^T = V dO^T  (A = K / V tiles row-wise, B = Q^T / dO^T in registers)
@@ -328,14 +326,14 @@ __global__ __launch_bounds__(256) void dsa_mass_reduce_kernel(const float *__res
 //   dQ^T[d,row] += K^T[d,key] dS^T[key,row]   (A = K tile transposed, B = dS^T from the C layout)
 // ==================================================================================================
 template <int D, bool HAS_IDX, int GSHIFT, int NW>
-__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_dq_kernel(
+__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_dq128_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
     float scale, int pos_split, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
     constexpr int KS = D / 16, DT = (D + 31) / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NBUF = (D > 128) ? 1 : 2;
+    constexpr int NBUF = 2;
     constexpr int NT = NW * 64, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT;
     constexpr int CH = 32 * CPR, LOADS = (CH + NT - 1) / NT;   // 16-byte chunks per matrix; per thread (head_dim 96: not all threads)
     static_assert(CH % 64 == 0, "whole waves stage or do not");
@@ -348,7 +346,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
     const int kvh = blockIdx.x % Hkv;
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(causal, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
     const int qc0 = blk * QBW;
     if (qc0 >= pos_split || qc0 >= L) return;
@@ -475,7 +473,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 //           of workgroups),
 //   mode 1: the segments by length, each one's tiles together (workgroups that run side by side then walk the
 //           same q / dO rows and share them in L2, which is worth more than the balance once a launch runs
-//           for many rounds),
+//           for many rounds - or without a causal mask, whose walks are equally long within a segment: 4000 patches,
+//           forward and backward, 170 -> 154 us),
 //   mode 2: as mode 0, and long walks cut into pieces of `pb` steps (a step = `qb` queries), for launches with
 //           fewer workgroups than a few rounds of the chip: a launch then ends with its longest walk, however
 //           few the workgroups.  A tile in pieces leaves one fp32 partial dK / dV per piece, added in piece
@@ -1589,29 +1588,7 @@ constexpr size_t dkv2_lds_bytes() {   // q/dO ring, P ring, row-data ring and on
 // ==================================================================================================
 // launchers: instantiate per head_dim, mask kind and (power-of-two padded) group size
 // ==================================================================================================
-static inline int group_shift(int Hq, int Hkv) {
-    const int G = Hq / Hkv;
-    int gshift = 0;
-    while ((1 << gshift) < G) ++gshift;
-    return gshift;
-}
 
-// waves per workgroup of the query-stationary kernels: all of them share the staged K / V tiles
-#ifndef DSA_TILE_WAVES_128
-#define DSA_TILE_WAVES_128 8
-#endif
-template <int D> constexpr int tile_waves() { return (D <= 128 && D > 64) ? DSA_TILE_WAVES_128 : 4; }
-static inline int tile_waves_of(int D) { return (D <= 128 && D > 64) ? DSA_TILE_WAVES_128 : 4; }
-template <int D, bool HAS_IDX, int GS>
-static hipError_t launch_dq_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
-                        const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                        int T, int Hq, int Hkv, int d_real, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
-                        float *delta_out) {
-    hipLaunchKernelGGL((dsa_tile_dq_kernel<D, HAS_IDX, GS, tile_waves<D>()>), grid, dim3(64 * tile_waves<D>()), 0, stream, (const bf16_t *)dout,
-                       (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv,
-                       scale, pos_split, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
-    return hipSuccess;
-}
 template <int D, bool HAS_IDX, int GS>
 static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
@@ -1657,10 +1634,7 @@ static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, 
     }                                                                                     \
     if (launch_status != hipSuccess) return launch_status;
 
-// The same for the kernels that take rows of d_real elements, a multiple of 8: without a selection the kernel of the next
-// head_dim of 64, 80, 96, 128 reads and writes such rows where they lie (80: five k-steps instead of six for the S and dP of
-// 72- and 80-wide vision heads)
-static inline int dense_kernel_dim(int d_real) { return d_real <= 64 ? 64 : d_real <= 80 ? 80 : d_real <= 96 ? 96 : d_real <= 128 ? 128 : d_real; }
+// the same for the kernel that takes rows of d_real elements
 #define TILE_SWITCH_DENSE(FN, ...)                                                        \
     hipError_t launch_status = hipErrorInvalidValue;                                      \
     if (bitmap) switch (d_real) {                                                         \
@@ -1742,16 +1716,27 @@ extern "C" hipError_t dsa_launch_tile_mass(const void *q, const void *k, const f
                        inv_hq, mass);
     return hipGetLastError();
 }
-extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,
-                                         const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
-                                         const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                         int pos_split, int causal, void *dq, const void *out_for_delta, float *delta_out,
-                                         hipStream_t stream) {
-    // out_for_delta != null: the kernel forms delta = rowsum(dO * O) of its rows itself and writes it to delta_out
+template <int D, bool HAS_IDX, int GS>
+static hipError_t launch_dq_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
+                        const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
+                        int T, int Hq, int Hkv, int d_real, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
+                        float *delta_out) {
+    hipLaunchKernelGGL((dsa_tile_dq128_kernel<D, HAS_IDX, GS, 8>), grid, dim3(512), 0, stream, (const bf16_t *)dout,
+                       (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv,
+                       scale, pos_split, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
+    return hipSuccess;
+}
+// dQ at head_dim 97 to 128 (dsa_tile_dq.hip runs the others and says why)
+extern "C" hipError_t dsa_launch_tile_dq_128(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
+                                             const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real,
+                                             float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
+                                             float *delta_out, hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * tile_waves_of(d_real)) >> gs) + N + 1) * Hkv));
-    TILE_SWITCH_DENSE(launch_dq_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out)
-    return hipGetLastError();
+    const dim3 grid((unsigned)(((int64_t)T / ((32 * 8) >> gs) + N + 1) * Hkv));
+    hipError_t launch_status = hipErrorInvalidValue;
+    if (bitmap) { GS_SWITCH(launch_dq_i, 128, true, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out) }
+    else { GS_SWITCH(launch_dq_i, 128, false, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out) }
+    return launch_status != hipSuccess ? launch_status : hipGetLastError();
 }
 // bytes of fp32 partial sums a launch of T tokens may use for key-tile walks in pieces (0: launches of this size are
 // never cut); a slot = the dK and dV of one 128-key tile and kv head
@@ -1773,7 +1758,7 @@ static DkvPlan dkv_plan(int T, int N, int Hq, int Hkv, int d_real, bool has_idx,
     p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= 4 * 256;
     p.listed = order && (N > 1 || p.pieces);             // (one segment: its tiles are in order already)
     const int cap = order_entries_cap(T), item_cap = p.pieces ? std::min(cap, p.tiles_ub + (1024 + wg_per_tile - 1) / wg_per_tile) : cap;
-    p.o = TileOrder{cap, p.pieces ? 2 : ((p.tiles_ub + 1) * Hkv > 4 * 256 ? 1 : 0), 32 >> group_shift(Hq, Hkv), wg_per_tile, item_cap,
+    p.o = TileOrder{cap, p.pieces ? 2 : (!causal || (p.tiles_ub + 1) * Hkv > 4 * 256 ? 1 : 0), 32 >> group_shift(Hq, Hkv), wg_per_tile, item_cap,
                     (int)(slot_pairs / Hkv < (1 << 20) ? slot_pairs / Hkv : (1 << 20))};       // (sums stay below 2^21)
     return p;
 }

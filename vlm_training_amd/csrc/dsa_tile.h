@@ -193,9 +193,11 @@ __device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, i
 // would otherwise end on the long walks of a late segment: forward -11 %, dQ -15 % on 8192 tokens in seven
 // segments), segment by segment for larger ones, where the blocks of a segment that run side by side share their
 // K / V tiles in L2 (the batch-wide order is 2-3 % slower there).
+// Without a causal mask the walks of a segment are equally long and there is nothing to balance inside it: segment by segment
+// (12 288 patches of 13 images, forward and backward: 485 us, in the batch-wide order 549).
 #define DSA_BATCH_ORDER_MAX_BLOCKS (6 * 256)
-#define LOCATE_QUERY_BLOCK(cu, N, slot, blk, s0, L, b)                                                           \
-    (gridDim.x <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
+#define LOCATE_QUERY_BLOCK(causal, cu, N, slot, blk, s0, L, b)                                                   \
+    ((causal) && gridDim.x <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
                                              : locate_block(cu, N, slot, blk, true, s0, L, b))
 
 // ---- LDS tiles filled straight from memory ------------------------------------------------------------------------------
@@ -241,3 +243,15 @@ struct DirectTile {
     static constexpr int tr_q(int dt) { return dt & 3; }
     static constexpr int tr_imm(int dt, int v) { return (D == 64 ? 0 : (dt >> 2) * 256) + v * (8 / GROUP) * GROUP_B; }
 };
+
+// ---- launches ----
+// log2 of the rows a query takes: its group's heads, padded to a power of two
+static inline int group_shift(int Hq, int Hkv) {
+    const int G = Hq / Hkv;
+    int gshift = 0;
+    while ((1 << gshift) < G) ++gshift;
+    return gshift;
+}
+// Rows of d_real elements, a multiple of 8: without a selection the kernel of the next head_dim of 64, 80, 96, 128 reads and writes
+// such rows where they lie (80: five k-steps instead of six for the S and dP of 72- and 80-wide vision heads)
+static inline int dense_kernel_dim(int d_real) { return d_real <= 64 ? 64 : d_real <= 80 ? 80 : d_real <= 96 ? 96 : d_real <= 128 ? 128 : d_real; }

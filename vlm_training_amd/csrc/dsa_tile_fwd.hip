@@ -43,7 +43,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = Hq / Hkv, kvh = blockIdx.x % Hkv, QBW = (NW * 32) >> gshift;
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(causal, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
