@@ -40,6 +40,34 @@ def test_dense_forward_reads_hf_tensors_in_place(D, Hq, Hkv, lens, causal):
         assert torch.equal(hf[0], got)
 
 
+def _alike(T, H, D, how, g):
+    """(T, H, D) bf16 whose token stride is ``how``: 0 (every token the same row), or less than a row (rows overlap)."""
+    if how == 0:
+        return torch.randn(1, H, D, generator=g).bfloat16().to(DEV).expand(T, H, D)
+    flat = torch.randn((T - 1) * how + H * D, generator=g).bfloat16().to(DEV)
+    return flat.as_strided((T, H, D), (how, D, 1))
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "qkv"])
+@pytest.mark.parametrize("D,Hq,Hkv,how,lens,causal", [
+    (64, 4, 2, 0, (33, 1, 64), True), (128, 4, 1, 0, (70, 129), True), (72, 2, 2, 0, (97, 31), False), (256, 4, 2, 0, (40,), True),
+    (64, 4, 2, 8, (33, 65), True), (128, 2, 1, 64, (1, 70), True), (80, 2, 2, 136, (97,), False), (200, 2, 1, 8, (34, 3), True)])
+def test_dense_forward_of_expanded_and_overlapping_rows(D, Hq, Hkv, how, lens, causal, which):
+    """Token strides shorter than a row give what their contiguous copies give."""
+    print("short token strides", D, Hq, Hkv, how, lens, causal, which, flush=True)
+    g = torch.Generator().manual_seed(D + how)
+    cu, T = _cu(lens).to(DEV), sum(lens)
+    x = {n: _alike(T, h, D, how, g) if n in which else torch.randn(T, h, D, generator=g).bfloat16().to(DEV)
+         for n, h in (("q", Hq), ("k", Hkv), ("v", Hkv))}
+    with torch.no_grad():
+        got = M.dispatch_varlen_attention(x["q"], x["k"], x["v"], cu, max(lens), causal=causal)
+        want = M.dispatch_varlen_attention(*(x[n].contiguous() for n in "qkv"), cu, max(lens), causal=causal)
+        assert torch.equal(got, want)
+        if causal:
+            hf = M.varlen_attention_forward(*(x[n].transpose(0, 1).unsqueeze(0) for n in "qkv"), cu)[0]
+            assert torch.equal(hf[0], want)
+
+
 @pytest.mark.parametrize("D,Hq,Hkv,lens,causal", [
     (8, 2, 1, (1, 34), True), (40, 4, 2, (129, 63), False), (72, 2, 2, (64, 97, 130), False), (72, 1, 1, (1500,), True),
     (80, 6, 2, (161, 31), True), (88, 2, 1, (70,), False), (112, 3, 3, (33, 128, 257), True), (120, 2, 1, (900, 5), True)])

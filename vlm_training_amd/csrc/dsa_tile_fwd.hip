@@ -71,13 +71,17 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     }
     const uint32_t lds0 = lds_address(dyn_lds);
     // Addresses of the next tile to request, in scalar registers (the asm statements keep them there); what is left of the
-    // block's keys from its first row on, in bytes, bounds the buffer
+    // block's keys from its first row on, in bytes, bounds the buffer (the last row ends with its own elements: a token
+    // stride may be shorter than a row, or zero, in an expanded tensor)
     const int Lend = min(L, ntiles * 32);
     auto next = [](const unsigned char *&p, int64_t step) __attribute__((always_inline)) {
         p += step;
         asm volatile("" : "+s"(p));
     };
-    auto left = [&](int tile, int tok_b) __attribute__((always_inline)) { return max(min(Lend - tile * 32, 32), 0) * tok_b; };
+    auto left = [&](int tile, int tok_b) __attribute__((always_inline)) {
+        const int rows = max(min(Lend - tile * 32, 32), 0);
+        return rows ? (rows - 1) * tok_b + d_real * 2 : 0;
+    };
     auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
         buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2, 0,
                           lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
