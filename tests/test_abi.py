@@ -168,3 +168,17 @@ def test_integration_notes_name_every_exported_symbol():
     unknown = [name for name in named if name.startswith("dsa_") and name not in _lib.EXPORTS
                and not name.startswith(("dsa_attn.h", "dsa_varlen_attn", "dsa_ref"))]
     assert not unknown, unknown
+
+
+def test_loads_into_lds_carry_their_whole_offset_in_the_bounded_address():
+    """A buffer's bounds check covers the lane's offset; the scalar offset of the instruction is outside it, so a request past a
+    tensor's end would not be held back if a tile's or a piece's offset went there."""
+    csrc = os.path.join(ROOT, "vlm_training_amd", "csrc")
+    loads = []
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".h", ".hip")):
+            loads += re.findall(r'buffer_load_dword\w* ([^\\"]*)', open(os.path.join(csrc, name)).read())
+    loads = [x for x in loads if " lds" in x]
+    assert loads
+    for operands in loads:
+        assert operands.split(",")[2].split()[0] == "0", operands

@@ -40,6 +40,27 @@ def test_dense_forward_reads_hf_tensors_in_place(D, Hq, Hkv, lens, causal):
         assert torch.equal(hf[0], got)
 
 
+@pytest.mark.parametrize("Hi,Di,lens", [
+    (1, 32, (1,)), (64, 128, (63, 1)), (8, 64, (64,)), (33, 128, (65, 3)), (64, 64, (126, 2)), (5, 32, (193,)), (64, 128, (30, 34, 257))])
+def test_indexer_scores_where_the_keys_end(Hi, Di, lens):
+    """The last tile's rows and the tiles requested past it: whatever lies behind the keys, the scores are those of the keys."""
+    print("keys end", Hi, Di, lens, flush=True)
+    g = torch.Generator().manual_seed(Di + Hi)
+    cu, T = _cu(lens), sum(lens)
+    q, k, w = (torch.randn(*s, generator=g).bfloat16() for s in ((T, Hi, Di), (T, Di), (T, Hi)))
+    behind = torch.full((T + 256, Di), float("nan")).bfloat16()
+    behind[:T] = k
+    got = M.ops.indexer_scores(q.to(DEV), behind.to(DEV)[:T], w.to(DEV), cu.to(DEV), max(lens)).cpu()
+    # fp32 sums of Di exact products, then of Hi terms, in any order and by adders that may cut: 2^-23 of the sum of magnitudes each
+    prod = torch.einsum("thd,sd->ths", q.double(), k.double())
+    want = (w.double()[:, :, None] * prod.relu()).sum(1) * (Di * Hi) ** -0.5
+    size = (w.double().abs()[:, :, None] * torch.einsum("thd,sd->ths", q.double().abs(), k.double().abs())).sum(1) * (Di * Hi) ** -0.5
+    for a, b in zip(cu[:-1].tolist(), cu[1:].tolist()):
+        for t in range(a, b):
+            d = (got[t, :t - a + 1].double() - want[t, a:t + 1]).abs()
+            assert (d <= (Di + Hi + 2) * 2.0 ** -23 * size[t, a:t + 1]).all()
+
+
 def _alike(T, H, D, how, g):
     """(T, H, D) bf16 whose token stride is ``how``: 0 (every token the same row), or less than a row (rows overlap)."""
     if how == 0:

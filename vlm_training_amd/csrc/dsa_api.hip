@@ -15,7 +15,7 @@ hipError_t dsa_launch_topk(const float *scores, int64_t ld, int row_begin, int r
 hipError_t dsa_launch_indexer_kl(const float *sel, const float *mass, const int32_t *n, int T, int K, float grad_scale,
                                  float *loss, float *dscore, hipStream_t stream);
 hipError_t dsa_launch_indexer(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu, int N,
-                              int T, int Hi, int Di, float scale, int row_begin, int row_end, int skip_dense_k,
+                              int Hi, int Di, float scale, int row_begin, int row_end, int skip_dense_k,
                               float *scores, int64_t ld, hipStream_t stream);
 hipError_t dsa_launch_attn_fwd(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K, float scale, int pos_min,
@@ -118,7 +118,7 @@ extern "C" int dsa_indexer_scores(const void *q_idx, const void *k_idx, const vo
     if (row_begin < 0 || row_end > T || row_begin > row_end) return fail(DSA_ERR_ARG, "bad row range [%d,%d)", row_begin, row_end);
     if (Hi < 1 || Hi > 64 || !(Di == 32 || Di == 64 || Di == 128))
         return fail(DSA_ERR_UNSUPPORTED, "indexer geometry Hi=%d Di=%d: need Hi<=64 and Di in {32,64,128}", Hi, Di);
-    hipError_t e = dsa_launch_indexer(q_idx, k_idx, w_idx, cu, N, T, Hi, Di, scale, row_begin, row_end, skip_dense_k,
+    hipError_t e = dsa_launch_indexer(q_idx, k_idx, w_idx, cu, N, Hi, Di, scale, row_begin, row_end, skip_dense_k,
                                       scores, ld, (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "indexer launch");
 }

@@ -111,12 +111,12 @@ __global__ __launch_bounds__(256 * mass_sets<HPG>(), 1) void dsa_tile_mass_kerne
 #pragma unroll
         for (int i = 0; i < LPW; ++i) {
             const int g = wv * LPW + i, hh = g / TL::LOADS, p = g % TL::LOADS;
-            buffer_load_lds16(keys, koff[i % TL::SOURCES] + (p / TL::SOURCES * TL::SOURCES) * TL::LOAD_ROWS * tok_b + min(kvh0 + hh, Hkv - 1) * D * 2, 0,
+            buffer_load_lds16(keys, koff[i % TL::SOURCES] + (p / TL::SOURCES * TL::SOURCES) * TL::LOAD_ROWS * tok_b + min(kvh0 + hh, Hkv - 1) * D * 2,
                               lds0 + (tile & 1) * SLOT + hh * TL::BYTES + TL::load_lds(p));
         }
         kptr += (int64_t)32 * tok_b;
         if (set == 0) {
-            buffer_load_lds4(make_buffer_rsrc(wptr, tile < ntiles ? 32 * (int64_t)ldw * 4 : 0), wvoff, 0, lds0 + 2 * SLOT + wq * 1024 + (tile & 3) * 256);
+            buffer_load_lds4(make_buffer_rsrc(wptr, tile < ntiles ? 32 * (int64_t)ldw * 4 : 0), wvoff, lds0 + 2 * SLOT + wq * 1024 + (tile & 3) * 256);
             wptr += 4;
         }
     };

@@ -124,16 +124,17 @@ __device__ __forceinline__ buffer_rsrc make_buffer_rsrc(const void *p, int64_t b
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
 }
-// 16 bytes per lane from byte voff + soff of the buffer to LDS byte `lds` (wave-uniform) + 16 * lane.  (The wait states
-// cover a scalar operand that a vector instruction wrote just before, and M0.)
-__device__ __forceinline__ void buffer_load_lds16(buffer_rsrc rsrc, int voff, int soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
+// 16 bytes per lane from byte voff of the buffer to LDS byte `lds` (wave-uniform) + 16 * lane.  The scalar offset of the
+// instruction stays 0: the bounds check need not include it, so a piece's or a tile's offset goes into voff or into the
+// buffer's start.  (The wait states cover a scalar operand that a vector instruction wrote just before, and M0.)
+__device__ __forceinline__ void buffer_load_lds16(buffer_rsrc rsrc, int voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 : : "v"(voff), "s"(rsrc), "s"(lds) : "memory", "m0");
 }
 // the same with 4 bytes per lane, to LDS byte `lds` + 4 * lane
-__device__ __forceinline__ void buffer_load_lds4(buffer_rsrc rsrc, int voff, int soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dword %0, %1, %2 offen lds"
-                 : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
+__device__ __forceinline__ void buffer_load_lds4(buffer_rsrc rsrc, int voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds"
+                 : : "v"(voff), "s"(rsrc), "s"(lds) : "memory", "m0");
 }
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 // the barrier alone: LDS operations of this wave may still be in flight

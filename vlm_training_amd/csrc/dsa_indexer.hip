@@ -40,7 +40,7 @@ __device__ __forceinline__ f32x16 zero_acc() {
 template <int HT, int DI>
 __global__ __launch_bounds__(IDX_WAVES * 64, 2) void dsa_indexer_scores_kernel(
     const bf16_t *__restrict__ q_idx, const bf16_t *__restrict__ k_idx, const bf16_t *__restrict__ w_idx,
-    const int32_t *__restrict__ cu, int N, int T, int Hi, float scale, int row_begin, int row_end, int skip_dense_k,
+    const int32_t *__restrict__ cu, int N, int Hi, float scale, int row_begin, int row_end, int skip_dense_k,
     float *__restrict__ scores, int64_t ld) {
     constexpr int KS = DI / 16;                 // MFMA k-steps
     constexpr int ROW_B = DI * 2, CPR = DI / 8; // bytes and 16-byte chunks per key row
@@ -74,19 +74,25 @@ __global__ __launch_bounds__(IDX_WAVES * 64, 2) void dsa_indexer_scores_kernel(
     const int ntiles = (hi - kt0) / IDX_BK + 1;
     // Keys in LDS: unpadded rows (a load writes 1 KiB of consecutive LDS per wave), chunk c of row r at position
     // c ^ swizzle(r), so that the sixteen rows of an operand read fall on sixteen different 16-byte columns of the banks;
-    // the swizzle is applied to the source address.  Rows past the batch read as zero (bounds of the buffer resource).
+    // the swizzle is applied to the source address.  A tile's buffer starts at its first key and ends behind the last key any of
+    // the workgroup's queries sees: rows past that, and tiles past the last one, read as zero without touching memory.
     auto swizzle = [](int row) { return DI == 128 ? (row & 15) : DI == 64 ? ((row >> 1) & 7) : ((row >> 2) & 3); };
-    const buffer_rsrc keys = make_buffer_rsrc(k_idx + (int64_t)kt0 * DI, (int64_t)(T - kt0) * ROW_B);
     const int src_row = tid / CPR;               // (every later load of a tile starts a multiple of 16 rows further)
     const int voff = src_row * ROW_B + (((tid % CPR) ^ swizzle(src_row)) << 4);
     const uint32_t lds0 = lds_address(&lds[0][0]) + wv * 1024;
-    auto load_tile = [&](int it, int buf) __attribute__((always_inline)) {   // buf: byte offset of the buffer
+    const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k_idx + (int64_t)kt0 * DI);
+    int rows_left = hi + 1 - kt0;
+    auto load_tile = [&](int buf) __attribute__((always_inline)) {   // the next tile, into the buffer at byte offset buf
+        const buffer_rsrc keys = make_buffer_rsrc(kptr, max(min(rows_left, IDX_BK), 0) * ROW_B);
 #pragma unroll
-        for (int r = 0; r < LOADS; ++r) buffer_load_lds16(keys, voff, it * TILE_B + r * (IDX_WAVES * 1024), lds0 + buf + r * (IDX_WAVES * 1024));
+        for (int r = 0; r < LOADS; ++r) buffer_load_lds16(keys, voff + r * (IDX_WAVES * 1024), lds0 + buf + r * (IDX_WAVES * 1024));
+        kptr += TILE_B;
+        rows_left -= IDX_BK;
+        asm volatile("" : "+s"(kptr), "+s"(rows_left));
     };
-    load_tile(0, 0);
-    load_tile(1, TILE_B);
-    load_tile(2, 2 * TILE_B);
+    load_tile(0);
+    load_tile(TILE_B);
+    load_tile(2 * TILE_B);
     // A operand: this wave's query, heads 32*ht + lane%32, k = 16*ks + 8*(lane/32) + e
     bf16x8 a[HT][KS];
     float wreg[HT][16];
@@ -149,7 +155,7 @@ __global__ __launch_bounds__(IDX_WAVES * 64, 2) void dsa_indexer_scores_kernel(
     // variable of its own)
     int cb = 0, nb = TILE_B, n2 = 2 * TILE_B, sb = 3 * TILE_B;
     for (int it = 0; it < ntiles; ++it) {
-        load_tile(it + 3, sb);                   // its buffer was last read before the previous barrier
+        load_tile(sb);                           // tile it+3; its buffer was last read before the previous barrier
         const bool mine = it >= it_lo && it <= it_hi;    // wave-uniform
         const int kt = kt0 + it * IDX_BK;
         if (mine) {
@@ -183,25 +189,25 @@ __global__ __launch_bounds__(IDX_WAVES * 64, 2) void dsa_indexer_scores_kernel(
 
 template <int HT, int DI>
 static hipError_t launch_indexer(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu, int N,
-                                 int T, int Hi, float scale, int row_begin, int row_end, int skip_dense_k,
+                                 int Hi, float scale, int row_begin, int row_end, int skip_dense_k,
                                  float *scores, int64_t ld, hipStream_t stream) {
     const int rows = row_end - row_begin;
     const int grid = (rows + IDX_WAVES - 1) / IDX_WAVES;
     hipLaunchKernelGGL((dsa_indexer_scores_kernel<HT, DI>), dim3(grid), dim3(IDX_WAVES * 64), 0, stream,
-                       (const bf16_t *)q_idx, (const bf16_t *)k_idx, (const bf16_t *)w_idx, cu, N, T, Hi, scale,
+                       (const bf16_t *)q_idx, (const bf16_t *)k_idx, (const bf16_t *)w_idx, cu, N, Hi, scale,
                        row_begin, row_end, skip_dense_k, scores, ld);
     return hipGetLastError();
 }
 
 // returns hipErrorInvalidValue for geometries the kernel does not cover
 extern "C" hipError_t dsa_launch_indexer(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu,
-                                         int N, int T, int Hi, int Di, float scale, int row_begin, int row_end,
+                                         int N, int Hi, int Di, float scale, int row_begin, int row_end,
                                          int skip_dense_k, float *scores, int64_t ld, hipStream_t stream) {
     if (row_end <= row_begin) return hipSuccess;
     const int HT = (Hi + 31) / 32;
 #define IDX_CASE(ht, di) \
     if (HT == ht && Di == di) \
-        return launch_indexer<ht, di>(q_idx, k_idx, w_idx, cu, N, T, Hi, scale, row_begin, row_end, skip_dense_k, scores, ld, stream);
+        return launch_indexer<ht, di>(q_idx, k_idx, w_idx, cu, N, Hi, scale, row_begin, row_end, skip_dense_k, scores, ld, stream);
     IDX_CASE(1, 32) IDX_CASE(1, 64) IDX_CASE(1, 128)
     IDX_CASE(2, 32) IDX_CASE(2, 64) IDX_CASE(2, 128)
 #undef IDX_CASE

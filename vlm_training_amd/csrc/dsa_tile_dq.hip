@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     // piece i of K (or V) tile `tile`; called in tile order.  Rows past the segment and columns past the true head_dim read as zero.
     auto load_piece = [&](const unsigned char *&p, int base, int tile, int i) __attribute__((always_inline)) {
         buffer_load_lds16(make_buffer_rsrc(p, left(tile)),
-                          voff[i % NV] + i / NV * NV * TL::LOAD_ROWS * tok_b, 0, lds0 + (base + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
+                          voff[i % NV] + i / NV * NV * TL::LOAD_ROWS * tok_b, lds0 + (base + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) {
             p += (int64_t)32 * tok_b;
             asm volatile("" : "+s"(p));
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int wvoff = (t - s0 - wq0) * ldw * 4;          // (at most 31 rows of bitmap)
     auto load_w = [&](int tile) __attribute__((always_inline)) {
         if (HAS_IDX) {
-            buffer_load_lds4(make_buffer_rsrc(wptr, 32 * (int64_t)ldw * 4), wvoff, 0, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
+            buffer_load_lds4(make_buffer_rsrc(wptr, 32 * (int64_t)ldw * 4), wvoff, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
             if (tile + 1 < ntiles) {                      // (past the block's tiles: the last word again, never used)
                 wptr += 4;
                 asm volatile("" : "+s"(wptr));

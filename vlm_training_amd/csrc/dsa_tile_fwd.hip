@@ -83,12 +83,12 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         return rows ? (rows - 1) * tok_b + d_real * 2 : 0;
     };
     auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2, 0,
+        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
                           lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) next(kptr, k_step);
     };
     auto load_v_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2, 0,
+        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
                           lds0 + (4 + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) next(vptr, v_step);
     };
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int wvoff = (t - s0 - wq0) * ldw * 4;         // (at most 31 rows of bitmap)
     auto load_w = [&](int tile) __attribute__((always_inline)) {
         if (HAS_IDX) {
-            buffer_load_lds4(make_buffer_rsrc(wptr, 32 * ldw * 4), wvoff, 0, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
+            buffer_load_lds4(make_buffer_rsrc(wptr, 32 * ldw * 4), wvoff, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
             if (tile + 1 < ntiles) next(wptr, 4);        // (past the block's tiles: the last word again, never used)
         }
     };

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel
     const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k_idx + (int64_t)s0 * D);
     const int Lend = min(L, ntiles * 32), koff = TL::source(wv * LPW, lane, 2 * D, D / 8);
     auto load_k = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(kptr, max(min(Lend - tile * 32, 32), 0) * 2 * D), koff + i * TL::LOAD_ROWS * 2 * D, 0,
+        buffer_load_lds16(make_buffer_rsrc(kptr, max(min(Lend - tile * 32, 32), 0) * 2 * D), koff + i * TL::LOAD_ROWS * 2 * D,
                           lds0 + (tile & 7) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) {
             kptr += 32 * 2 * D;
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel
         const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)words, tile & 63) & (tile < ntiles ? 0xffffffffu : 0u);
         const int slot = seen + (int)__builtin_amdgcn_mbcnt_lo(word, 0u);
         const bool sel = lane < 32 && ((word >> j) & 1u);
-        buffer_load_lds4(grads, sel ? slot * 4 : IDX_NOT_THERE, 0, grad_lds + (tile & 3) * 256);
+        buffer_load_lds4(grads, sel ? slot * 4 : IDX_NOT_THERE, grad_lds + (tile & 3) * 256);
         seen += __popc(word);
     };
 #pragma unroll
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void dsa_tile_idxk_kernel(
     auto load_q = [&](auto odd_, int u, int i) __attribute__((always_inline)) {
         constexpr int hb = HB == 2 && decltype(odd_)::value ? 1 : 0;
         const int heads = u < ntiles ? (HB == 2 && hb == 0 ? 32 : Hi - 32 * hb) : 0;
-        buffer_load_lds16(make_buffer_rsrc(qptr, heads * 2 * D), qoff + i * TL::LOAD_ROWS * 2 * D, 0,
+        buffer_load_lds16(make_buffer_rsrc(qptr, heads * 2 * D), qoff + i * TL::LOAD_ROWS * 2 * D,
                           lds0 + (u & 7) * TL::BYTES + TL::load_lds(wv * LPW + i));
         if (i == LPW - 1) {
             qptr += HB == 2 && hb == 0 ? 32 * 2 * D : -(int64_t)(Hi + 32 * hb) * 2 * D;
@@ -321,10 +321,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void dsa_tile_idxk_kernel(
         const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)words, step & 63) & (live && kc < L ? 0xffffffffu : 0u);
         const int slot = __builtin_amdgcn_readlane(bases, step & 63) + (int)__builtin_amdgcn_mbcnt_lo(word, 0u);
         const bool sel = lane < 32 && ((word >> j) & 1u);
-        buffer_load_lds4(make_buffer_rsrc(dptr, live ? (int64_t)K * 4 : 0), sel ? slot * 4 : IDX_NOT_THERE, 0, aux_lds + (step & 3) * 256);
+        buffer_load_lds4(make_buffer_rsrc(dptr, live ? (int64_t)K * 4 : 0), sel ? slot * 4 : IDX_NOT_THERE, aux_lds + (step & 3) * 256);
     };
     auto load_weights = [&](int step) __attribute__((always_inline)) {
-        buffer_load_lds4(make_buffer_rsrc(wptr, step < nsteps ? 256 : 0), lane * 4, 0, aux_lds + 1024 + (step & 3) * 256);
+        buffer_load_lds4(make_buffer_rsrc(wptr, step < nsteps ? 256 : 0), lane * 4, aux_lds + 1024 + (step & 3) * 256);
         dptr -= (int64_t)K * 4;
         wptr -= 256;
         asm volatile("" : "+s"(dptr), "+s"(wptr));
