@@ -80,17 +80,26 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     };
     auto left = [&](int tile, int tok_b) __attribute__((always_inline)) {
         const int rows = max(min(Lend - tile * 32, 32), 0);
-        return rows ? (rows - 1) * tok_b + d_real * 2 : 0;
+        return (uint32_t)(rows ? (rows - 1) * tok_b + d_real * 2 : 0);
     };
+    uint32_t kleft = left(0, (int)k_tok * 2), vleft = left(0, (int)v_tok * 2);
     auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(kptr, left(tile, (int)k_tok * 2)), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
+        buffer_load_lds16(make_buffer_rsrc(kptr, kleft), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
                           lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
-        if (i == LPW - 1) next(kptr, k_step);
+        if (i == LPW - 1) {
+            next(kptr, k_step);
+            kleft = left(tile + 1, (int)k_tok * 2);
+            asm volatile("" : "+s"(kleft));
+        }
     };
     auto load_v_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(vptr, left(tile, (int)v_tok * 2)), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
+        buffer_load_lds16(make_buffer_rsrc(vptr, vleft), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
                           lds0 + (4 + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
-        if (i == LPW - 1) next(vptr, v_step);
+        if (i == LPW - 1) {
+            next(vptr, v_step);
+            vleft = left(tile + 1, (int)v_tok * 2);
+            asm volatile("" : "+s"(vleft));
+        }
     };
     auto load_k = [&](int tile) __attribute__((always_inline)) {
 #pragma unroll
