@@ -182,3 +182,35 @@ def test_loads_into_lds_carry_their_whole_offset_in_the_bounded_address():
     assert loads
     for operands in loads:
         assert operands.split(",")[2].split()[0] == "0", operands
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_forward_mode_differentiation_is_refused(grad):
+    """The operators have no jvp: a dual input raises, whether or not a graph is built (checked before the device)."""
+    import torch.autograd.forward_ad as fwAD
+    import vlm_training_amd as M
+    host = _lib.host()
+    g = torch.Generator().manual_seed(0)
+    x = lambda *s: torch.randn(*s, generator=g).bfloat16().requires_grad_(grad)  # noqa: E731
+    cu = torch.tensor([0, 4], dtype=torch.int32)
+    T, H, D = 4, 1, 64
+    thd = (T, H, D)
+    calls = {
+        "dense": (lambda q, k, v: M.dsa_varlen_attn(q, k, v, cu, T), (thd, thd, thd)),
+        "dispatch": (lambda q, k, v: M.dispatch_varlen_attention(q, k, v, cu, T, causal=False), (thd, thd, thd)),
+        "hf": (lambda q, k, v: M.varlen_attention_forward(q, k, v, cu, max_seqlen=T), ((1, H, T, D),) * 3),
+        "node": (lambda q, k, v: host.attn_node(q, k, v, cu, T, None, None, 1.0, True, False, None), (thd, thd, thd)),
+        "norm": (lambda q, k, a, b: M.qk_norm_rope(q, k, a, b, torch.ones(T, 16), torch.ones(T, 16)), (thd, thd, (D,), (D,))),
+        "gate": (lambda a, b: M.sigmoid_gate(a, b), (thd, thd)),
+        "loss": (lambda q, k, w: M.indexer_kl_loss(q, k, w, torch.ones(T, 2), cu, T, 2), ((T, 2, 64), (T, 64), (T, 2))),
+        "project": (lambda a, w: host.project(a, [w], 1, 0), ((T, 8), (8, 8))),
+    }
+    for name, (call, shapes) in calls.items():
+        for dual in range(len(shapes)):
+            for no_grad in (False, True):
+                with fwAD.dual_level(), torch.set_grad_enabled(not no_grad):
+                    args = [x(*s) for s in shapes]
+                    args[dual] = fwAD.make_dual(args[dual], torch.ones_like(args[dual]))
+                    with pytest.raises(NotImplementedError):
+                        call(*args)
+                        print(name, dual, no_grad)

@@ -42,6 +42,14 @@ void need_gpu(const Tensor &t) {
         TORCH_CHECK(false, "dsa attention runs on the GPU only (tensor on ", t.device().str(), "); there is no CPU path");
 }
 
+// The operators have no forward-mode derivative.  Asked of every differentiable input before anything else: a dual tensor need not
+// require a gradient, so a call that builds no graph would drop its tangent without a word.
+bool has_tangent(const Tensor &t) { return t.defined() && t._fw_grad(0).defined(); }
+void no_forward_mode(std::initializer_list<const Tensor *> inputs, const char *what) {
+    for (const Tensor *t : inputs)
+        TORCH_CHECK_NOT_IMPLEMENTED(!has_tangent(*t), what, ": forward-mode differentiation is not implemented");
+}
+
 Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const Tensor &like) {
     return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
 }
@@ -269,6 +277,7 @@ bool needs_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
 
 variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, const OptTensor &idx, const OptTensor &n,
                         double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
+    no_forward_mode({&q, &k, &v}, "attention");
     if (!needs_grad(q, k, v)) {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::OptionalDeviceGuard guard(q.device());
@@ -313,7 +322,9 @@ std::optional<Tensor> hf_dense_forward(const Tensor &q, const Tensor &k, const T
         return t.dim() == 4 && t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.size(0) == 1 && t.stride(3) == 1 && t.size(3) % 8 == 0 &&
                t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && t.stride(2) < (1 << 24) && aligned16(t);
     };
-    if (!fits(q) || !fits(k) || !fits(v) || !mask.is_cuda() || needs_grad(q, k, v) || std::getenv("DSA_DEBUG_META")) return std::nullopt;
+    if (!fits(q) || !fits(k) || !fits(v) || !mask.is_cuda() || needs_grad(q, k, v) || has_tangent(q) || has_tangent(k) || has_tangent(v) ||
+        std::getenv("DSA_DEBUG_META"))
+        return std::nullopt;
     const int64_t Hq = q.size(1), Hkv = k.size(1), T = q.size(2), D = q.size(3);
     if (k.sizes() != v.sizes() || k.size(2) != T || k.size(3) != D || D > 256 || !Hkv || Hq % Hkv) return std::nullopt;
     const c10::OptionalDeviceGuard guard(q.device());
@@ -329,6 +340,7 @@ std::optional<Tensor> hf_dense_forward(const Tensor &q, const Tensor &k, const T
 variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &cu_, std::optional<int64_t> max_seqlen_,
                           const OptTensor &iq, const OptTensor &ik, const OptTensor &iw, std::optional<int64_t> top_k, std::optional<double> index_scale,
                           std::optional<double> softmax_scale, bool return_indices, bool causal, bool return_mass, bool return_scores) {
+    no_forward_mode({&q_, &k_, &v_}, "dsa_varlen_attn");
     need_gpu(q_); need_gpu(k_); need_gpu(v_); need_gpu(cu_);
     const Qkv sh = checked_qkv(q_, k_, v_);
     const c10::OptionalDeviceGuard guard(q_.device());
@@ -442,6 +454,7 @@ public:
 
 Tensor indexer_kl_loss(const Tensor &q_idx, const Tensor &k_idx, const Tensor &w_idx, const Tensor &mass, const Tensor &cu_, int64_t max_seqlen,
                        int64_t top_k, std::optional<double> index_scale, const OptTensor &idx, const OptTensor &n, const OptTensor &sel) {
+    no_forward_mode({&q_idx, &k_idx, &w_idx, &mass}, "indexer_kl_loss");
     need_gpu(q_idx); need_gpu(k_idx); need_gpu(w_idx); need_gpu(mass); need_gpu(cu_);
     TORCH_CHECK_VALUE(q_idx.dim() == 3 && k_idx.dim() == 2 && w_idx.dim() == 2, "indexer tensors must be q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi)");
     const c10::OptionalDeviceGuard guard(q_idx.device());
@@ -520,6 +533,7 @@ public:
 
 variable_list qk_norm_rope(const Tensor &q, const Tensor &k, const Tensor &qw, const Tensor &kw, const Tensor &cos, const Tensor &sin, double eps,
                            bool offset) {
+    no_forward_mode({&q, &k, &qw, &kw, &cos, &sin}, "qk_norm_rope");
     return QkNormRopeNode::apply(q, k, qw, kw, cos, sin, eps, offset);
 }
 
@@ -640,6 +654,8 @@ public:
 };
 
 variable_list project(const Tensor &x, const std::vector<Tensor> &weights, int64_t n_input, int64_t gate_dim) {
+    no_forward_mode({&x}, "project");
+    for (const Tensor &w : weights) no_forward_mode({&w}, "project");
     need_gpu(x);
     TORCH_CHECK_VALUE(x.dim() == 2 && x.scalar_type() == at::kBFloat16 && !weights.empty() && n_input >= 0 && n_input <= (int64_t)weights.size() &&
                       weights.size() + (gate_dim ? 1 : 0) <= DSA_PACK_MAX, "project: a (T, width) bf16 input and up to 8 outputs");
@@ -650,7 +666,10 @@ variable_list project(const Tensor &x, const std::vector<Tensor> &weights, int64
     return ProjectionNode::apply(x, at::TensorList(weights), n_input, gate_dim);
 }
 
-Tensor sigmoid_gate(const Tensor &x, const Tensor &gate) { return SigmoidGateNode::apply(x, gate); }
+Tensor sigmoid_gate(const Tensor &x, const Tensor &gate) {
+    no_forward_mode({&x, &gate}, "sigmoid_gate");
+    return SigmoidGateNode::apply(x, gate);
+}
 
 }  // namespace
 
