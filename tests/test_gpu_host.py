@@ -38,3 +38,65 @@ def test_no_tangent_is_dropped(sparse):
         torch.func.vmap(lambda q: M.dsa_varlen_attn(q, *qkv[1:], cu, T, **more))(torch.stack([qkv[0], qkv[0]]))
     with pytest.raises(RuntimeError):
         torch.func.grad(lambda q: M.dsa_varlen_attn(q, *qkv[1:], cu, T, **more).sum())(qkv[0])
+
+
+def _layer(gated, T, frozen):
+    from types import SimpleNamespace
+    torch.manual_seed(T)
+    cfg = SimpleNamespace(hidden_size=256, num_attention_heads=4, num_key_value_heads=2, head_dim=64, rms_norm_eps=1e-6)
+    m = (M.SelfAttention if gated else M.Qwen3VLTextAttention)(cfg, dsa=M.DsaConfig(index_heads=8, index_dim=64, top_k=16)).to(DEV, torch.bfloat16)
+    for name, p in m.named_parameters():
+        p.requires_grad_(not frozen(name))
+    ang = torch.outer(torch.arange(T, device=DEV).float(), 0.1 ** torch.arange(16, device=DEV).float())
+    emb = torch.cat((ang, ang), -1)
+    return m, (emb.cos().bfloat16(), emb.sin().bfloat16(), torch.tensor([0, T - T // 3, T], dtype=torch.int32, device=DEV), T)
+
+
+def _nodes(t):
+    seen, todo = set(), [t.grad_fn]
+    while todo:
+        n = todo.pop()
+        if n is not None and n not in seen:
+            seen.add(n)
+            todo += [e for e, _ in n.next_functions]
+    return [n.name() for n in seen]
+
+
+@pytest.mark.parametrize("gated", [False, True])
+def test_frozen_projections_stay_out_of_the_graph(gated):
+    print("frozen", gated, flush=True)
+    T = 2048                                              # large enough for the shared node
+    x = _randn(1, T, 256)
+    # the indexer trained beside a frozen backbone: the layer's output has no graph, the loss reaches the indexer alone
+    m, rest = _layer(gated, T, lambda n: not n.startswith("indexer."))
+    y = m(x, *rest)
+    assert not y.requires_grad and M.indexer_losses(m).requires_grad
+    M.indexer_losses(m).backward()
+    assert all((p.grad is not None) == n.startswith("indexer.") for n, p in m.named_parameters())
+    # everything frozen, the input trained: no projection forms a weight gradient
+    m, rest = _layer(gated, T, lambda n: True)
+    xi = x.clone().requires_grad_(True)
+    y = m(xi, *rest)
+    assert not any("ProjectionNode" in n for n in _nodes(y))
+    y.backward(torch.ones_like(y))
+    assert xi.grad is not None and all(p.grad is None for p in m.parameters())
+    # everything trained: the shared node is there
+    m, rest = _layer(gated, T, lambda n: False)
+    assert any("ProjectionNode" in n for n in _nodes(m(x, *rest)))
+
+
+def test_shared_projections_form_the_gradients_that_are_taken():
+    from torch.profiler import ProfilerActivity, profile
+    from vlm_training_amd import _lib
+    T, W = 64, 32
+    x, ws = _randn(T, W, grad=True), [_randn(n, W, seed=n, grad=True) for n in (8, 16, 24)]
+    gs = [_randn(T, w.shape[0], seed=7) for w in ws]
+    want = torch.autograd.grad([x @ w.t() for w in ws], [x] + ws, gs)
+    for take in ([0], [1], [3], [0, 2], [1, 3], [0, 1, 2, 3]):
+        ys = _lib.host().project(x, ws, 3, 0)
+        with profile(activities=[ProfilerActivity.CPU]) as prof:
+            got = torch.autograd.grad(ys, [([x] + ws)[i] for i in take], gs)
+        gemms = sum(e.count for e in prof.key_averages() if e.key == "aten::mm")
+        assert gemms == (0 in take) + any(i > 0 for i in take), (take, gemms)
+        for i, a in zip(take, got):
+            assert a.shape == want[i].shape and (a.float() - want[i].float()).norm() <= 1e-2 * want[i].float().norm(), (take, i)

@@ -646,9 +646,17 @@ public:
         }
         if (ctx->needs_input_grad(0) && input_cols)
             res[0] = at::mm(g.narrow(1, 0, input_cols), input_weights.size() == 1 ? input_weights[0] : at::cat(input_weights));
-        const Tensor dw = at::mm(g.t(), x);
+        // the columns of the weights whose gradient somebody takes (all of them but for torch.autograd.grad)
+        int64_t first = -1, last = -1;
         for (int64_t i = 0; i < n_w; ++i)
-            if (at_row[i] >= 0) res[1 + i] = dw.narrow(0, at_row[i], s[1 + i].size(0));
+            if (at_row[i] >= 0 && ctx->needs_input_grad(1 + i)) {
+                if (first < 0) first = at_row[i];
+                last = at_row[i] + s[1 + i].size(0);
+            }
+        if (first < 0) return res;
+        const Tensor dw = at::mm(g.narrow(1, first, last - first).t(), x);
+        for (int64_t i = 0; i < n_w; ++i)
+            if (at_row[i] >= 0 && ctx->needs_input_grad(1 + i)) res[1 + i] = dw.narrow(0, at_row[i] - first, s[1 + i].size(0));
         return res;
     }
 };

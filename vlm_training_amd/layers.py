@@ -62,7 +62,7 @@ class DsaIndexer(nn.Module):
 def _fusible(lin, x) -> bool:
     w = getattr(lin, "weight", None)
     return (type(lin) is nn.Linear and lin.bias is None and type(w) is nn.Parameter and w.dtype == torch.bfloat16 and w.device == x.device
-            and w.shape[0] % 8 == 0 and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks))
+            and w.requires_grad and w.shape[0] % 8 == 0 and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks))
 
 
 @torch.compiler.disable
@@ -70,7 +70,9 @@ def _projections(x, linears, indexer, gate_dim: int = 0):
     """Outputs of ``linears`` (and of the indexer's projections, which read ``x`` detached) as one autograd node whose backward
     runs one weight-gradient GEMM for all of them (``ProjectionNode`` in csrc/dsa_host.cpp).  ``gate_dim``: the first output
     comes as its two interleaved halves.  None where the modules have to be called one by one: other module types, biases,
-    hooks, sharded or non-bf16 weights, autocast, no gradient wanted."""
+    hooks, sharded or non-bf16 weights, autocast, no gradient wanted - and frozen weights: outputs of one node all require a
+    gradient as soon as one of its inputs does, so a frozen q, k or v beside a trained indexer would put the whole attention
+    into the graph."""
     mods = list(linears) + ([indexer.q_proj, indexer.k_proj, indexer.w_proj] if indexer is not None else [])
     if not (type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled()
             and x.numel() >= 1 << 19          # (256 tokens of 2048; below, a step is bound by the host and the GEMMs are all short)
