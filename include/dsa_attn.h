@@ -10,6 +10,8 @@
  * Conventions
  *   - every pointer is a DEVICE pointer unless it says "host"; tensors are row-major contiguous;
  *   - q (T,Hq,D), k/v (T,Hkv,D), q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi): bf16 (dtype code below);
+ *   - k, v, k_idx and (for the indexer's gradients) q_idx lie on 16-byte boundaries: they are loaded into LDS 16 bytes per
+ *     lane (DSA_ERR_ARG otherwise; the host operators copy a view that starts elsewhere);
  *   - cu_seqlens (N+1) int32, cu[0]=0, cu[N]=T, non-decreasing (zero-length segments allowed, the pad
  *     tail is one more segment: data/energon_dataloader.py:431-464, models/qwen3_vl/model.py:757-765);
  *   - idx (T,K) int32: global packed row ids of the selected keys, ascending, padded with -1;

@@ -214,3 +214,24 @@ def test_forward_mode_differentiation_is_refused(grad):
                     with pytest.raises(NotImplementedError):
                         call(*args)
                         print(name, dual, no_grad)
+
+
+def test_operands_loaded_into_lds_have_to_lie_on_16_byte_boundaries():
+    """Refused before any launch, so this runs without a GPU; the pointers are never followed."""
+    lib = _lib.load()
+    a, odd = 1 << 20, (1 << 20) + 2
+    T, N, Hq, Hkv, D, K = 64, 1, 4, 2, 64, 8
+
+    def fwd(k, v):
+        return lib.dsa_attn_fwd(a, k, v, None, None, a, T, N, Hq, Hkv, D, 0, 1.0, 0, T, 1, a, a, None, 0, None)
+
+    def bwd(k, v):
+        return lib.dsa_attn_bwd(a, a, k, v, a, a, None, None, a, T, N, Hq, Hkv, D, 0, 1.0, 0, T, 1, a, a, a, a, 1 << 40, None)
+
+    calls = [lambda: fwd(odd, a), lambda: fwd(a, odd), lambda: bwd(odd, a), lambda: bwd(a, odd),
+             lambda: lib.dsa_attn_mass(a, odd, a, a, a, a, T, N, Hq, Hkv, D, K, 1.0, 0, T, a, a, 1 << 40, None),
+             lambda: lib.dsa_indexer_scores(a, odd, a, a, T, N, 4, 64, 1.0, 0, 0, T, 0, a, T, None),
+             lambda: lib.dsa_indexer_bwd(odd, a, a, a, a, a, a, T, N, 4, 64, K, 1.0, 0, T, a, a, a, a, 1 << 40, None),
+             lambda: lib.dsa_indexer_bwd(a, odd, a, a, a, a, a, T, N, 4, 64, K, 1.0, 0, T, a, a, a, a, 1 << 40, None)]
+    for i, call in enumerate(calls):
+        assert call() == -1 and b"16-byte" in lib.dsa_last_error(), i

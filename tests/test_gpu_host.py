@@ -100,3 +100,52 @@ def test_shared_projections_form_the_gradients_that_are_taken():
         assert gemms == (0 in take) + any(i > 0 for i in take), (take, gemms)
         for i, a in zip(take, got):
             assert a.shape == want[i].shape and (a.float() - want[i].float()).norm() <= 1e-2 * want[i].float().norm(), (take, i)
+
+
+def _shifted(t):
+    """The same values, contiguous, one element behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:].copy_(t.reshape(-1))
+    return buf[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("D,dtype,sparse,gather", [
+    (64, "bf16", True, False), (128, "bf16", True, False), (256, "bf16", True, False), (72, "bf16", False, False), (128, "bf16", False, 0),
+    (256, "bf16", False, False), (64, "fp32", True, False), (128, "bf16", True, True)])
+def test_views_that_start_anywhere(D, dtype, sparse, gather):
+    """Contiguous views on no 16-byte boundary give the bits of aligned tensors: forward, gradients, mass, indexer's loss.
+    ``gather``: with the gather kernels alone."""
+    print("views", D, dtype, sparse, gather, flush=True)
+    lens = (70, 33, 129)
+    T, Hq, Hkv, Hi, Di, K = sum(lens), 4, 2, 8, 64, 16
+    cu = torch.tensor([0, 70, 103, 232], dtype=torch.int32, device=DEV)
+    dt = torch.float32 if dtype == "fp32" else torch.bfloat16
+    shapes = dict(q=(T, Hq, D), k=(T, Hkv, D), v=(T, Hkv, D), dout=(T, Hq, D), iq=(T, Hi, Di), ik=(T, Di), iw=(T, Hi))
+    base = {n: _randn(*s, seed=i).to(dt) for i, (n, s) in enumerate(shapes.items())}
+    old = M.ops.set_tile_crossover(0) if gather else None
+    try:
+        res = []
+        for place in (lambda t: t.clone(), _shifted):
+            x = {n: place(t) for n, t in base.items()}
+            assert all((t.data_ptr() & 15 == 0) == (place is not _shifted) for t in x.values())
+            leaves = [x[n].requires_grad_(True) for n in ("q", "k", "v") + (("iq", "ik", "iw") if sparse else ())]
+            if sparse:
+                out, idx, n, mass, sel = M.dsa_varlen_attn(*leaves[:3], cu, max(lens), indexer_q=x["iq"], indexer_k=x["ik"], indexer_w=x["iw"],
+                                                           top_k=K, return_indices=True, return_mass=True, return_scores=True)
+                loss = M.indexer_kl_loss(*leaves[3:], mass, cu, max(lens), K, selection=(idx, n, sel))
+                torch.autograd.backward((out, loss), (x["dout"], None))
+                with torch.no_grad():
+                    plain = M.dsa_varlen_attn(*(t.detach() for t in leaves[:3]), cu, max(lens), indexer_q=x["iq"], indexer_k=x["ik"],
+                                              indexer_w=x["iw"], top_k=K)
+                res.append([out, idx, n, mass, sel, loss, plain] + [t.grad for t in leaves])
+            else:
+                out = M.dispatch_varlen_attention(*leaves, cu, max(lens), causal=False)
+                out.backward(x["dout"])
+                with torch.no_grad():
+                    plain = M.dispatch_varlen_attention(*(t.detach() for t in leaves), cu, max(lens))
+                res.append([out, plain] + [t.grad for t in leaves])
+    finally:
+        if gather:
+            M.ops.set_tile_crossover(old)
+    for a, b in zip(*res):
+        assert torch.equal(a, b)

@@ -109,12 +109,19 @@ static int check_packed(int T, int N, const int32_t *cu) {
     return DSA_OK;
 }
 
+// operands the kernels load straight into LDS, 16 bytes per lane
+static int check_aligned(const void *a, const void *b, const char *what) {
+    if (((uintptr_t)a | (uintptr_t)b) & 15) return fail(DSA_ERR_ARG, "%s must lie on 16-byte boundaries", what);
+    return DSA_OK;
+}
+
 extern "C" int dsa_indexer_scores(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu, int T,
                                   int N, int Hi, int Di, float scale, int dtype, int row_begin, int row_end,
                                   int skip_dense_k, float *scores, int64_t ld, void *stream) {
     if (int rc = check_packed(T, N, cu)) return rc;
     if (dtype != DSA_DTYPE_BF16) return fail(DSA_ERR_UNSUPPORTED, "indexer inputs must be bf16 (dtype code %d)", dtype);
     if (!q_idx || !k_idx || !w_idx || !scores) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (int rc = check_aligned(k_idx, k_idx, "k_idx")) return rc;
     if (row_begin < 0 || row_end > T || row_begin > row_end) return fail(DSA_ERR_ARG, "bad row range [%d,%d)", row_begin, row_end);
     if (Hi < 1 || Hi > 64 || !(Di == 32 || Di == 64 || Di == 128))
         return fail(DSA_ERR_UNSUPPORTED, "indexer geometry Hi=%d Di=%d: need Hi<=64 and Di in {32,64,128}", Hi, Di);
@@ -288,6 +295,7 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, const int32
     if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
     if (!causal && idx) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
     if (!q || !k || !v || !out || !lse) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
     const int split = pos_split_for(idx, K);
@@ -361,6 +369,7 @@ static int attn_mass_run(const void *q, const void *k, const float *lse, const i
                          const void *saved_bitmap, size_t saved_bytes, void *ws, size_t ws_bytes, void *stream) {
     if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
     if (!q || !k || !lse || !idx || !n || !mass) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (int rc = check_aligned(k, k, "k")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
     const int ldw = bitmap_ldw(max_seqlen);
@@ -467,6 +476,7 @@ extern "C" int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, cons
     if (dw_dtype != DSA_DTYPE_BF16 && dw_dtype != DSA_DTYPE_FP32) return fail(DSA_ERR_ARG, "dw dtype code %d", dw_dtype);
     if (K < 1) return fail(DSA_ERR_ARG, "top_k=%d must be >= 1", K);
     if (!q_idx || !k_idx || !w_idx || !idx || !n || !dscore || !dq_idx || !dk_idx || !dw) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (int rc = check_aligned(q_idx, k_idx, "q_idx and k_idx")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
     const size_t need = dsa_indexer_bwd_workspace_bytes(T, Di, max_seqlen);
@@ -617,6 +627,7 @@ static int check_bwd(const void *dout, const void *q, const void *k, const void 
     if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
     if (!causal && idx) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
     if (!dout || !q || !k || !v || !out || !lse || !dq || !dk || !dv) return fail(DSA_ERR_ARG, "null tensor pointer");
+    if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     return DSA_OK;
 }

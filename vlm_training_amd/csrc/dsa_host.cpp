@@ -55,7 +55,12 @@ Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const Tensor &like) {
 }
 Tensor empty_bytes(size_t bytes, const Tensor &like) { return empty({(int64_t)std::max<size_t>(bytes, 4)}, at::kByte, like); }
 
-Tensor as_bf16(const Tensor &t) { return (t.scalar_type() == at::kBFloat16 ? t : t.to(at::kBFloat16)).contiguous(); }
+bool aligned16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
+// contiguous bf16 on a 16-byte boundary: keys, values and index queries go into LDS 16 bytes at a time (a view can start anywhere)
+Tensor as_bf16(const Tensor &t) {
+    const Tensor c = (t.scalar_type() == at::kBFloat16 ? t : t.to(at::kBFloat16)).contiguous();
+    return aligned16(c) ? c : c.clone();
+}
 
 Tensor checked_cu(const Tensor &cu) {
     TORCH_CHECK_VALUE(cu.dim() == 1 && cu.numel() >= 2, "cu_seqlens must be 1-D with at least two entries");
@@ -298,11 +303,10 @@ Qkv checked_qkv(const Tensor &q, const Tensor &k, const Tensor &v) {
     return s;
 }
 
-bool aligned16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
 // q, k and v can go to the dense forward as they lie in memory: no transposing copy, no padding of the head_dim
 bool readable_in_place(const Tensor &t) {
     return t.scalar_type() == at::kBFloat16 && t.stride(2) == 1 && t.size(2) % 8 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
-           t.stride(0) < (1 << 24) && ((uintptr_t)t.data_ptr() & 15) == 0;
+           t.stride(0) < (1 << 24) && aligned16(t);
 }
 // the dense forward without a graph
 Tensor dense_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, double scale, bool causal) {
@@ -372,7 +376,7 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
     if (!sparse && !needs_grad(q, k, v) && readable_in_place(q) && readable_in_place(k) && readable_in_place(v))
         return {dense_forward(q, k, v, cu, max_seqlen, scale, causal)};
     // the tile kernels take rows of any multiple of 8 up to 128 where they lie (a selection's kernels do not)
-    if (!sparse && q.scalar_type() == at::kBFloat16 && sh.D <= 128 && sh.D % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(v)) d_kernel = sh.D;
+    if (!sparse && q.scalar_type() == at::kBFloat16 && sh.D <= 128 && sh.D % 8 == 0) d_kernel = sh.D;
     if (d_kernel != sh.D) {
         // zero columns change neither q.k nor the used part of p.v
         const int64_t pad = d_kernel - sh.D;
@@ -620,8 +624,7 @@ public:
                 const int64_t w = s[1 + i].size(0);
                 for (int p = 0; p < halves; ++p)
                     if (grads[o + p].defined()) {
-                        Tensor g = as_bf16(grads[o + p]);
-                        if (!aligned16(g)) g = g.clone();
+                        const Tensor g = as_bf16(grads[o + p]);
                         keep.push_back(g);
                         src.push_back(ptr(g));
                         width.push_back((int32_t)(w / halves));

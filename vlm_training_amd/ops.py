@@ -34,7 +34,12 @@ def _require_cuda(*tensors):
 
 def _as_bf16(t: torch.Tensor) -> torch.Tensor:
     # fp32/fp16 inputs are rounded to bf16 once; the kernels compute in bf16 MFMA with fp32 accumulation
-    return (t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)).contiguous()
+    return _on_16_bytes((t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)).contiguous())
+
+
+def _on_16_bytes(t: torch.Tensor) -> torch.Tensor:
+    # keys, values and index queries go into LDS 16 bytes at a time; a view can start anywhere
+    return t.clone() if t.data_ptr() & 15 else t
 
 
 def _as_bf16_x3(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor):
@@ -272,6 +277,7 @@ def attn_fwd(q, k, v, idx, n, cu_seqlens, max_seqlen: int, softmax_scale: float,
     keeps it for the backward, so that the selection bitmap is built once.  ``bitmap_ready``: ``ws`` already holds the
     bitmap of this selection (``index_topk(..., bitmap=ws)``) and is only read."""
     T, Hq, Hkv, D = _check_qkv(q, k, v)
+    k, v = _on_16_bytes(k), _on_16_bytes(v)
     cu = _check_cu(cu_seqlens, T)
     out = torch.empty((T, Hq, D), dtype=torch.bfloat16, device=q.device)
     lse = torch.empty((Hq, T), dtype=torch.float32, device=q.device)
@@ -335,6 +341,7 @@ def attn_bwd(dout, q, k, v, out, lse, idx, n, cu_seqlens, max_seqlen: int, softm
     """Stage D4.  ``parts``/``buffers`` exist for per-kernel timing: ``buffers=(dq, dk, dv, ws)`` reuses
     the outputs and workspace of an earlier full call."""
     T, Hq, Hkv, D = _check_qkv(q, k, v)
+    k, v = _on_16_bytes(k), _on_16_bytes(v)
     cu = _check_cu(cu_seqlens, T)
     K = idx.shape[1] if idx is not None else 0
     lib = _lib.load()
@@ -357,6 +364,7 @@ def attn_bwd_saved_bitmap(dout, q, k, v, out, lse, idx, n, cu_seqlens, max_seqle
     """Stage D4 reading the selection bitmap out of the forward's workspace ``fwd_ws`` (None for dense attention); the
     scratch it allocates lives for the call only."""
     T, Hq, Hkv, D = _check_qkv(q, k, v)
+    k, v = _on_16_bytes(k), _on_16_bytes(v)
     cu = _check_cu(cu_seqlens, T)
     K = idx.shape[1] if idx is not None else 0
     lib = _lib.load()
