@@ -149,3 +149,44 @@ def test_views_that_start_anywhere(D, dtype, sparse, gather):
             M.ops.set_tile_crossover(old)
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+def test_a_selection_the_caller_holds_is_checked():
+    """Shapes, types and places that do not fit are refused before any launch; strided ones are copied."""
+    from vlm_training_amd import _lib
+    host = _lib.host()
+    T, Hq, Hkv, D, Hi, Di, K = 40, 4, 2, 64, 8, 64, 16
+    cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    q, k, v = _randn(T, Hq, D), _randn(T, Hkv, D, seed=1), _randn(T, Hkv, D, seed=2)
+    iq, ik, iw = _randn(T, Hi, Di, grad=True), _randn(T, Di, grad=True), _randn(T, Hi, grad=True)
+    out, idx, n, mass, sel = M.dsa_varlen_attn(q, k, v, cu, T, indexer_q=iq, indexer_k=ik, indexer_w=iw, top_k=K, return_indices=True,
+                                               return_mass=True, return_scores=True)
+
+    def node(idx=idx, n=n, q=q, k=k, v=v, cu=cu, mass=False, bitmap=None):
+        return host.attn_node(q, k, v, cu, T, idx, n, D ** -0.5, True, mass, bitmap)
+
+    def loss(idx=idx, n=n, sel=sel, mass=mass, ik=ik, iw=iw):
+        return M.indexer_kl_loss(iq, ik, iw, mass, cu, T, K, selection=(idx, n, sel))
+
+    wide_idx, wide_n = torch.zeros(T, 2 * K, dtype=torch.int32, device=DEV), torch.zeros(T, 2, dtype=torch.int32, device=DEV)
+    wide_idx[:, :K], wide_n[:, 1] = idx, n
+    assert torch.equal(node()[0], out) and torch.equal(node(wide_idx[:, :K], wide_n[:, 1])[0], out)
+    want, got = loss(), loss(wide_idx[:, :K], wide_n[:, 1])
+    assert torch.equal(want, got)
+    for a, b in zip(torch.autograd.grad(want, [iq, ik, iw]), torch.autograd.grad(got, [iq, ik, iw])):
+        assert torch.equal(a, b)
+    for bad in (dict(idx=idx[:-1]), dict(idx=idx[:, 0]), dict(idx=idx.long()), dict(n=n[:-1]), dict(n=n.long()), dict(n=n[:, None]),
+                dict(idx=idx.cpu()), dict(n=n.cpu())):
+        for call in (node, loss):
+            with pytest.raises(ValueError):
+                call(**bad)
+    for bad in (dict(k=k[:-1]), dict(v=v[:, :1]), dict(q=q[..., :32]), dict(idx=None), dict(n=None), dict(idx=None, n=None, mass=True),
+                dict(cu=cu[:1]), dict(q=q[:, :3]), dict(q=q.float()), dict(bitmap=torch.zeros(8, dtype=torch.int32, device=DEV))):
+        with pytest.raises(ValueError):
+            node(**bad)
+    with pytest.raises(RuntimeError):
+        node(k=k.cpu())
+    for bad in (dict(sel=sel[:, :K - 1].contiguous(), mass=mass[:, :K - 1].contiguous()), dict(mass=mass[:-1]), dict(ik=ik[:-1]), dict(iw=iw[:, :4]),
+                dict(ik=ik[:, :32]), dict(idx=None), dict(mass=mass.bfloat16()), dict(sel=sel.cpu())):
+        with pytest.raises(ValueError):
+            loss(**bad)

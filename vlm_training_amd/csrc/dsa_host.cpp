@@ -280,19 +280,6 @@ bool needs_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
     return at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
 }
 
-variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, const OptTensor &idx, const OptTensor &n,
-                        double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
-    no_forward_mode({&q, &k, &v}, "attention");
-    if (!needs_grad(q, k, v)) {
-        at::AutoDispatchBelowADInplaceOrView below;
-        const c10::OptionalDeviceGuard guard(q.device());
-        const AttnArgs a{max_seqlen, scale, causal, want_mass, q.scalar_type() == at::kFloat && 4 * q.size(2) <= 256, q.scalar_type()};
-        AttnForward f = attn_forward(q, k, v, cu, idx.value_or(Tensor()), n.value_or(Tensor()), bitmap.value_or(Tensor()), a);
-        return want_mass ? variable_list{f.res, f.mass} : variable_list{f.res};
-    }
-    return AttnNode::apply(q, k, v, cu, idx, n, bitmap, max_seqlen, scale, causal, want_mass);
-}
-
 struct Qkv { int64_t T, Hq, Hkv, D; };
 Qkv checked_qkv(const Tensor &q, const Tensor &k, const Tensor &v) {
     TORCH_CHECK_VALUE(q.dim() == 3 && k.dim() == 3 && v.dim() == 3, "q, k, v must be (T, H, D)");
@@ -301,6 +288,40 @@ Qkv checked_qkv(const Tensor &q, const Tensor &k, const Tensor &v) {
     TORCH_CHECK_VALUE(s.Hkv > 0 && s.Hq % s.Hkv == 0, "Hq=", s.Hq, " must be a multiple of Hkv=", s.Hkv);
     TORCH_CHECK_VALUE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "q, k, v must share a dtype");
     return s;
+}
+
+// a selection the caller holds: a (T, K) table of keys and (T) counts, int32, contiguous, beside the tensors it indexes
+struct Picked { Tensor idx, n; };
+Picked checked_selection(const OptTensor &idx, const OptTensor &n, int64_t T, const Tensor &beside) {
+    TORCH_CHECK_VALUE(idx.has_value() == n.has_value(), "idx and n belong together");
+    if (!idx) return {};
+    TORCH_CHECK_VALUE(idx->dim() == 2 && idx->size(0) == T && idx->size(1) >= 1 && n->dim() == 1 && n->size(0) == T && idx->scalar_type() == at::kInt &&
+                      n->scalar_type() == at::kInt, "a selection is idx (T,K) int32 and n (T,) int32 for T=", T, ", got ", idx->sizes(), " ",
+                      idx->scalar_type(), " and ", n->sizes(), " ", n->scalar_type());
+    TORCH_CHECK_VALUE(idx->device() == beside.device() && n->device() == beside.device(), "idx and n must lie on ", beside.device());
+    return {idx->contiguous(), n->contiguous()};
+}
+
+variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu_, int64_t max_seqlen, const OptTensor &idx_,
+                        const OptTensor &n_, double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
+    no_forward_mode({&q, &k, &v}, "attention");
+    need_gpu(q); need_gpu(k); need_gpu(v); need_gpu(cu_);
+    const Qkv sh = checked_qkv(q, k, v);
+    TORCH_CHECK_VALUE(k.device() == q.device() && v.device() == q.device(), "q, k, v must lie on one device");
+    const c10::OptionalDeviceGuard guard(q.device());
+    const Tensor cu = checked_cu(cu_);
+    const Picked sel = checked_selection(idx_, n_, sh.T, q);
+    const OptTensor idx = sel.idx.defined() ? OptTensor(sel.idx) : std::nullopt, n = sel.n.defined() ? OptTensor(sel.n) : std::nullopt;
+    TORCH_CHECK_VALUE(idx || (!want_mass && !bitmap), "the attention mass and the bitmap belong to a selection");
+    TORCH_CHECK_VALUE(!bitmap || (bitmap->scalar_type() == at::kByte && bitmap->is_contiguous() && bitmap->device() == q.device()),
+                      "the bitmap must be contiguous bytes on ", q.device());
+    if (!needs_grad(q, k, v)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const AttnArgs a{max_seqlen, scale, causal, want_mass, q.scalar_type() == at::kFloat && 4 * q.size(2) <= 256, q.scalar_type()};
+        AttnForward f = attn_forward(q, k, v, cu, idx.value_or(Tensor()), n.value_or(Tensor()), bitmap.value_or(Tensor()), a);
+        return want_mass ? variable_list{f.res, f.mass} : variable_list{f.res};
+    }
+    return AttnNode::apply(q, k, v, cu, idx, n, bitmap, max_seqlen, scale, causal, want_mass);
 }
 
 // q, k and v can go to the dense forward as they lie in memory: no transposing copy, no padding of the head_dim
@@ -427,12 +448,19 @@ public:
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::OptionalDeviceGuard guard(q_idx.device());
         const int64_t T = q_idx.size(0);
+        TORCH_CHECK_VALUE(k_idx.size(0) == T && k_idx.size(1) == q_idx.size(2) && w_idx.size(0) == T && w_idx.size(1) == q_idx.size(1),
+                          "indexer tensor shapes disagree: ", q_idx.sizes(), " ", k_idx.sizes(), " ", w_idx.sizes());
         Selection s;
-        if (sel_) s = {*idx_, *n_, *sel_};
-        else s = select_keys(q_idx, k_idx, w_idx, cu, (int)max_seqlen, top_k, index_scale_of(index_scale, q_idx.size(1), q_idx.size(2)), true, Tensor());
+        if (sel_) {
+            TORCH_CHECK_VALUE(idx_ && n_, "a selection is (idx, n, scores)");
+            const Picked p = checked_selection(idx_, n_, T, q_idx);
+            TORCH_CHECK_VALUE(p.idx.sizes() == sel_->sizes(), "idx must have the shape of the scores: ", p.idx.sizes(), " ", sel_->sizes());
+            s = {p.idx, p.n, *sel_};
+        } else s = select_keys(q_idx, k_idx, w_idx, cu, (int)max_seqlen, top_k, index_scale_of(index_scale, q_idx.size(1), q_idx.size(2)), true, Tensor());
         const int64_t K = s.scores.size(1);
-        TORCH_CHECK_VALUE(s.scores.size(0) == T && mass_.sizes() == s.scores.sizes() && s.n.dim() == 1 && s.n.size(0) == T &&
-                          s.scores.scalar_type() == at::kFloat && mass_.scalar_type() == at::kFloat, "sel_scores and mass must be (T,K) fp32, n (T,) int32");
+        TORCH_CHECK_VALUE(mass_.sizes() == s.scores.sizes() && s.scores.scalar_type() == at::kFloat && mass_.scalar_type() == at::kFloat,
+                          "sel_scores and mass must be (T,K) fp32");
+        TORCH_CHECK_VALUE(s.scores.device() == q_idx.device() && mass_.device() == q_idx.device(), "sel_scores and mass must lie on ", q_idx.device());
         const Tensor sc = s.scores.contiguous(), mass = mass_.contiguous();
         const Tensor loss = empty({T}, at::kFloat, q_idx), dscore = empty({T, K}, at::kFloat, q_idx);
         check(dsa_indexer_kl(fptr(sc), fptr(mass), iptr(s.n), (int)T, (int)K, 1.f / (float)std::max<int64_t>(T, 1), fptr(loss), fptr(dscore),
