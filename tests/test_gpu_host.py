@@ -190,3 +190,12 @@ def test_a_selection_the_caller_holds_is_checked():
                 dict(ik=ik[:, :32]), dict(idx=None), dict(mass=mass.bfloat16()), dict(sel=sel.cpu())):
         with pytest.raises(ValueError):
             loss(**bad)
+
+
+def test_gradients_of_shared_projections_own_their_memory():
+    m, rest = _layer(True, 2048, lambda n: False)
+    y = m(_randn(1, 2048, 256), *rest)
+    torch.autograd.backward((y, M.indexer_losses(m)), (torch.ones_like(y), None))
+    stores = [p.grad.untyped_storage() for p in m.parameters()]
+    assert len({s.data_ptr() for s in stores}) == len(stores)
+    assert all(s.nbytes() == p.numel() * p.element_size() for s, p in zip(stores, m.parameters()))

@@ -604,7 +604,9 @@ public:
 // runs ONE weight-gradient GEMM - the separate ones have 32 to 2048 output rows over a long contraction and leave most of the chip
 // idle - and one input-gradient GEMM over the first `n_input` outputs (the others read the input detached), which also takes
 // the place of the sums of their input gradients.  8192 tokens, 2048 wide, six projections: nine GEMMs and two sums 574 us ->
-// two GEMMs and the copies 447 us.
+// two GEMMs and the copies 467 us (20 of them so that every weight's gradient owns its memory).  For as long as it runs the
+// backward holds, beyond what separate linears would, the packed gradients (T x columns), the input's weights laid end to end and
+// the weight gradients a second time: 102 + 17 + 26 MB there.
 class ProjectionNode : public torch::autograd::Function<ProjectionNode> {
 public:
     static variable_list forward(AutogradContext *ctx, const Tensor &x, at::TensorList weights, int64_t n_input, int64_t gate_dim) {
@@ -686,8 +688,16 @@ public:
             }
         if (first < 0) return res;
         const Tensor dw = at::mm(g.narrow(1, first, last - first).t(), x);
+        // Every weight gets a gradient of its own: autograd keeps what it is handed as .grad, and parts of one buffer would be
+        // freed, saved and resized together.
+        variable_list parts, own;
         for (int64_t i = 0; i < n_w; ++i)
-            if (at_row[i] >= 0 && ctx->needs_input_grad(1 + i)) res[1 + i] = dw.narrow(0, at_row[i] - first, s[1 + i].size(0));
+            if (at_row[i] >= 0 && ctx->needs_input_grad(1 + i)) {
+                parts.push_back(dw.narrow(0, at_row[i] - first, s[1 + i].size(0)));
+                res[1 + i] = parts.back().numel() == dw.numel() ? dw : empty(parts.back().sizes(), at::kBFloat16, x);
+                own.push_back(res[1 + i]);
+            }
+        if (parts.size() > 1) at::_foreach_copy_(own, parts);
         return res;
     }
 };
