@@ -199,3 +199,76 @@ def test_gradients_of_shared_projections_own_their_memory():
     stores = [p.grad.untyped_storage() for p in m.parameters()]
     assert len({s.data_ptr() for s in stores}) == len(stores)
     assert all(s.nbytes() == p.numel() * p.element_size() for s, p in zip(stores, m.parameters()))
+
+
+def _count_calls(counts, how, m):
+    """Put something in front of the layer's projections that counts their calls; returns what takes it away again."""
+    from torch.nn.modules import module as nnm
+    lins = (m.q_proj, m.indexer.k_proj)
+
+    def hook(mod, *args):
+        if mod in lins:
+            counts.append(mod)
+    if how in ("register_module_forward_hook", "register_module_forward_pre_hook", "register_module_full_backward_hook",
+               "register_module_full_backward_pre_hook"):
+        handles = [getattr(nnm, how)(hook)]
+    elif how == "forward":
+        class Handle:
+            def __init__(self, lin):
+                self.lin, plain = lin, lin.forward
+                lin.forward = lambda x: (counts.append(lin), plain(x))[1]
+
+            def remove(self):
+                del self.lin.forward
+        handles = [Handle(lin) for lin in lins]
+    elif how == "indexer":
+        plain = m.indexer.forward
+        m.indexer.forward = lambda x: (counts.append(x), counts.append(x), plain(x))[2]
+
+        class Handle:
+            def remove(self):
+                del m.indexer.forward
+        handles = [Handle()]
+    elif how in ("class", "foreign"):
+        class Other(torch.nn.Module):                     # an indexer that is none of this package's
+            def __init__(self, inner):
+                super().__init__()
+                self.inner, self.cfg = inner, inner.cfg
+
+            def forward(self, x):
+                counts.extend((x, x))
+                return self.inner(x)
+
+        class Handle:
+            def __init__(self):
+                self.indexer, self.plain = m.indexer, torch.nn.Linear.forward
+                if how == "foreign":
+                    m.indexer = Other(m.indexer)
+                else:
+                    torch.nn.Linear.forward = lambda lin, x: (hook(lin), self.plain(lin, x))[1]
+
+            def remove(self):
+                m.indexer, torch.nn.Linear.forward = self.indexer, self.plain
+        handles = [Handle()]
+    else:
+        handles = [getattr(lin, how)(hook) for lin in lins]
+    return handles
+
+
+@pytest.mark.parametrize("how", ["register_module_forward_hook", "register_module_forward_pre_hook", "register_module_full_backward_hook",
+                                 "register_module_full_backward_pre_hook", "forward", "indexer", "class", "foreign", "register_forward_hook",
+                                 "register_forward_pre_hook", "register_full_backward_hook", "register_full_backward_pre_hook"])
+def test_what_stands_around_the_projections_is_run(how):
+    print("around the projections", how, flush=True)
+    m, rest = _layer(False, 2048, lambda n: False)
+    counts = []
+    handles = _count_calls(counts, how, m)
+    try:
+        y = m(_randn(1, 2048, 256, grad=True), *rest)
+        torch.autograd.backward((y, M.indexer_losses(m)), (torch.ones_like(y), None))
+    finally:
+        for h in handles:
+            h.remove()
+    assert len(counts) == 2
+    counts.clear()
+    assert any("ProjectionNode" in n for n in _nodes(m(_randn(1, 2048, 256), *rest))) and not counts

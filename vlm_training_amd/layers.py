@@ -59,10 +59,21 @@ class DsaIndexer(nn.Module):
         return iq, self.k_proj(h), self.w_proj(h)
 
 
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+_GLOBAL_HOOKS = tuple(getattr(nn.modules.module, "_global" + h) for h in _HOOKS)     # (dicts, filled in place)
+_FORWARD = {cls: (cls.forward, cls.__call__) for cls in (nn.Linear, DsaIndexer)}
+
+
+def _plain(mod, cls) -> bool:
+    """Calling ``mod`` runs the forward of ``cls`` and nothing else: no subclass, no hooks, no forward put on instance or class."""
+    return (type(mod) is cls and "forward" not in vars(mod) and (cls.forward, cls.__call__) == _FORWARD[cls]
+            and not any(getattr(mod, h) for h in _HOOKS))
+
+
 def _fusible(lin, x) -> bool:
     w = getattr(lin, "weight", None)
-    return (type(lin) is nn.Linear and lin.bias is None and type(w) is nn.Parameter and w.dtype == torch.bfloat16 and w.device == x.device
-            and w.requires_grad and w.shape[0] % 8 == 0 and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks))
+    return (_plain(lin, nn.Linear) and lin.bias is None and type(w) is nn.Parameter and w.dtype == torch.bfloat16 and w.device == x.device
+            and w.requires_grad and w.shape[0] % 8 == 0)
 
 
 @torch.compiler.disable
@@ -70,16 +81,15 @@ def _projections(x, linears, indexer, gate_dim: int = 0):
     """Outputs of ``linears`` (and of the indexer's projections, which read ``x`` detached) as one autograd node whose backward
     runs one weight-gradient GEMM for all of them (``ProjectionNode`` in csrc/dsa_host.cpp).  ``gate_dim``: the first output
     comes as its two interleaved halves.  None where the modules have to be called one by one: other module types, biases,
-    hooks, sharded or non-bf16 weights, autocast, no gradient wanted - and frozen weights: outputs of one node all require a
-    gradient as soon as one of its inputs does, so a frozen q, k or v beside a trained indexer would put the whole attention
-    into the graph."""
+    hooks (their own or on all modules), a replaced forward, sharded or non-bf16 weights, autocast, no gradient wanted - and
+    frozen weights: outputs of one node all require a gradient as soon as one of its inputs does, so a frozen q, k or v beside
+    a trained indexer would put the whole attention into the graph."""
+    if indexer is not None and not _plain(indexer, DsaIndexer):
+        return None
     mods = list(linears) + ([indexer.q_proj, indexer.k_proj, indexer.w_proj] if indexer is not None else [])
     if not (type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled()
             and x.numel() >= 1 << 19          # (256 tokens of 2048; below, a step is bound by the host and the GEMMs are all short)
-            and not torch.is_autocast_enabled("cuda") and all(_fusible(m, x) for m in mods)):
-        return None
-    if indexer is not None and (type(indexer) is not DsaIndexer or indexer._forward_hooks or indexer._forward_pre_hooks
-                                or indexer._backward_hooks or indexer._backward_pre_hooks):
+            and not torch.is_autocast_enabled("cuda") and not any(_GLOBAL_HOOKS) and all(_fusible(m, x) for m in mods)):
         return None
     h = x.reshape(-1, x.shape[-1])
     return _lib.host().project(h, [m.weight for m in mods], len(linears), gate_dim)
