@@ -104,7 +104,8 @@ def _check_qkv(q, k, v):
 
 
 # ------------------------------------------------------------------------------------------------
-# stage wrappers (also used by the tests to look at each stage on its own)
+# stage wrappers: each stage on its own, for the bench, the traceable operator and the tests (the operator below drives the
+# same entry points from C++)
 # ------------------------------------------------------------------------------------------------
 def indexer_scores(q_idx, k_idx, w_idx, cu_seqlens, max_seqlen: int, index_scale: Optional[float] = None,
                    skip_dense_k: int = 0) -> torch.Tensor:
@@ -380,9 +381,6 @@ def attn_bwd_saved_bitmap(dout, q, k, v, out, lse, idx, n, cu_seqlens, max_seqle
     return dq, dk, dv
 
 
-# ------------------------------------------------------------------------------------------------
-# the operator
-# ------------------------------------------------------------------------------------------------
 def _split_stack(x: torch.Tensor, order: int) -> torch.Tensor:
     """fp32 (T,H,D) -> bf16 (T,H,4D): hi = bf16(x), lo = bf16(x - hi) stacked along head_dim, order 0 = [hi, lo, hi, 0],
     order 1 = [hi, hi, lo, 0] (one kernel)."""
@@ -427,6 +425,9 @@ def _split_combine_qkv(dq, dk, dv):
     return oq, okv[0], okv[1]
 
 
+# ------------------------------------------------------------------------------------------------
+# the operator
+# ------------------------------------------------------------------------------------------------
 class _DsaVarlenAttn:
     """The attention node on a selection the caller holds (``AttnNode`` in csrc/dsa_host.cpp)."""
 
@@ -444,7 +445,7 @@ def dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen: Optional[int] = None, *, in
                     return_mass: bool = False, return_scores: bool = False):
     """Packed causal attention over ``cu_seqlens`` segments, optionally sparsified by the DSA indexer.
 
-    q (T,Hq,D), k/v (T,Hkv,D) contiguous, cu_seqlens (N+1,) int32 on the device, max_seqlen host int
+    q (T,Hq,D), k/v (T,Hkv,D), cu_seqlens (N+1,) int32 on the device, max_seqlen host int
     (the reference's callers already hold it: models/qwen3_vl/model.py:765) - any upper bound of the
     longest segment gives the same result, and ``None`` stands for the bound T, which needs no
     device-to-host copy of the segment lengths (train/model_attention.py:120-121 syncs for it).  Without indexer inputs
@@ -456,9 +457,17 @@ def dsa_varlen_attn(q, k, v, cu_seqlens, max_seqlen: Optional[int] = None, *, in
     KL loss that trains the indexer.  ``return_scores=True`` appends the (T, top_k) fp32 indexer scores of the selected
     keys (every row is then scored, also those whose whole window is selected), which ``indexer_kl_loss`` takes as
     ``selection=(idx, n, scores)`` instead of running the indexer again.
-    Gradients flow to q, k, v only.  A head_dim between the kernels' 64 / 128 / 256 is zero-padded to the
-    next one and the output cut back (the scale stays that of the true head_dim).  ``causal=False`` (dense only) attends every key of the own segment, the
-    vision towers' form of the call (models/qwen3_vl/model.py:423-428).
+    Gradients flow to q, k, v only; a tangent on one of them (forward-mode differentiation) raises NotImplementedError.
+    ``causal=False`` (dense only) attends every key of the own segment, the vision towers' form of the call
+    (models/qwen3_vl/model.py:423-428).
+
+    Strides and starting addresses are the caller's.  A dense call that builds no graph reads bf16 views with a contiguous
+    last dimension where they lie (a (1, H, T, D) tensor's transposed view, an expanded one), if head_dim and strides are
+    multiples of 8 elements and the first element lies on a 16-byte boundary; every other call makes contiguous copies of what is not
+    contiguous on a 16-byte boundary.  Head_dims between the kernels' own: without indexer inputs any multiple of 8 up to 128
+    (up to 256 when no graph is built) is read and written in rows of its own width; the others, and every such head_dim with
+    indexer inputs, are zero-padded to the next of 64 / 96 (dense only) / 128 / 256 and the output cut back (the scale stays
+    that of the true head_dim).
     """
     if os.environ.get("DSA_DEBUG_META"):
         _require_cuda(q, k, v, cu_seqlens)
