@@ -139,8 +139,8 @@ size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen);
  * q head h reads kv head h / (Hq/Hkv) (models/qwen3/model.py:125-129).  softmax in fp32.
  * causal == 0 (only with idx == NULL) attends every key of the own segment: the vision towers' call,
  * varlen_attn(..., window_size=(-1,-1)) (models/qwen3_vl/model.py:423-428, models/qwen3_5/model.py:388-393).
- * head_dim D: 64, 128 or 256; with idx == NULL also 96 (forward and backward), which the 72-wide heads of the
- * 1152 / 16 vision towers are padded to.
+ * head_dim D: 64, 128 or 256; with idx == NULL also 96 (dsa_dense_fwd_strided and dsa_dense_bwd_rows take rows of any
+ * multiple of 8 without padding: the 72-wide heads of the 1152 / 16 vision towers).
  */
 int dsa_attn_fwd(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n,
                  const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale,
@@ -193,8 +193,8 @@ int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const float *lse, c
 /*
  * Tuning knob (process-wide, no reference counterpart): query rows whose position in their segment is
  * below top_k * crossover run on the dense MFMA tile kernels with the selection as a bitmap mask, the
- * rest on the gather kernels.  Default 24 (one 131 072-token sequence with top-k 2048: forward 115 -> 110 ms and
- * dQ 123 -> 120 ms against 16; 32 is level with it); 0 = gather only; INT_MAX/top_k or more = tiles only.
+ * rest on the gather kernels.  Default 24 (one 131 072-token sequence with top-k 2048: forward 101 -> 96 ms and
+ * dQ 107 -> 104 ms against 16; 32 is level with it); 0 = gather only; INT_MAX/top_k or more = tiles only.
  * idx == NULL (dense causal attention) always uses the tile kernels.
  */
 int dsa_set_tile_crossover(int crossover);
@@ -204,8 +204,8 @@ int dsa_get_tile_crossover(void);
  * Tuning knob (process-wide, no reference counterpart): the backward's query-side pass (dQ) and key-side pass (dK/dV)
  * read the same inputs and write different outputs.  1 (default): when the key-side launch has at most 1536
  * workgroups - a short batch, or one GPU's share of head-sharded attention, which ends on its longest walks with most
- * CUs idle - and T * max_seqlen * Hq * D is at least 6e10 (below that the fork and join cost what the overlap gains)
- * the query side runs on a second stream of the library's own (default priority, one per device, created
+ * CUs idle - and T * max_seqlen * Hq * D is at least 2e9 (6e10 without a causal mask; below that the fork and join cost
+ * what the overlap gains) the query side runs on a second stream of the library's own (default priority, one per device, created
  * on the first such call outside a capture) between a fork and a join event on the caller's stream, so that to the
  * caller the whole call is still ordered on the stream it passed; under stream capture the second stream joins the
  * capture through those events.  0: never (one stream).  2: for every launch size.  Results are the same bits in all

@@ -4,7 +4,7 @@
 //   p = exp(q.k*scale - lse),  dP = dO.v,  dS = p * (dP - delta)
 //   dQ[t]  = scale * sum_{s in sel(t)} dS[t,s] k[s]      query side by gather, one wave per (t, kv head),
 //                                                         for the rows where the selection is sparse
-//                                                         (dsa_bwd_dq_kernel; dense rows: dsa_tile_dq_kernel)
+//                                                         (dsa_bwd_dq_kernel; dense rows: the tile dQ kernels)
 //   inverted selection: bitmap[t][w] bit b <=> query t selected key column 32w+b of its segment
 //                                                         (dsa_bitmap_kernel); the key-side passes
 //                                                         dsa_tile_dkv2_kernel / dsa_tile_dkvpc_kernel reduce

@@ -1,5 +1,6 @@
-// Tile kernels: dK / dV, dQ at head_dim 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask (the forward:
-// dsa_tile_fwd.hip, dQ but for head_dim 128: dsa_tile_dq.hip, the indexer backward: dsa_tile_idx.hip).  They do the same arithmetic as the gather kernels but visit every (query block, key
+// Tile kernels: dK / dV, dQ at head_dim 97 to 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap
+// mask (the forward: dsa_tile_fwd.hip, dQ elsewhere: dsa_tile_dq.hip, the indexer backward: dsa_tile_idx.hip).  They do the same
+// arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
 // 4*G*D flop on the matrix cores - on MI355X the tile walk is cheaper down to a few percent density.
@@ -19,8 +20,7 @@
 // saved log-sum-exp instead of the online softmax and no V: P = exp(S*scale - lse) on the selected
 // keys, summed over the heads of a query that share the kv head (lanes of one query are adjacent:
 // DPP adds), and written to the slot the key has in the query's ascending selection list
-// (slot = selected keys of earlier tiles + selected keys below it in the tile's word).  One partial
-// (T,K) table per kv head; dsa_mass_reduce_kernel adds them in a fixed order.
+// (slot = selected keys of earlier tiles + selected keys below it in the tile's word).
 // ==================================================================================================
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float x) {

@@ -49,7 +49,7 @@ __device__ __forceinline__ float dot8_chain(bf16x8 a, bf16x8 b, float acc) {
 }
 
 // delta[h,t] = sum_d dO[t,h,d] * O[t,h,d] of row (t, h) by 16 lanes (`sub` of them): lane i sums the 8-element chunks i, i+16, ...
-// in one chain, then a butterfly over the 16 lanes (dsa_tile_dq_kernel reproduces this order when it forms delta itself)
+// in one chain, then a butterfly over the 16 lanes (the tile dQ kernels reproduce this order when they form delta themselves)
 __device__ __forceinline__ void delta_row(const bf16_t *__restrict__ dout, const bf16_t *__restrict__ out, int T, int Hq, int D, int64_t row, int sub,
                                           float *__restrict__ delta) {
     float acc = 0.f;

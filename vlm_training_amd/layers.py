@@ -8,7 +8,8 @@
 * ``DsaIndexer``            - the lightning indexer's projections as module parameters (the reference holds no
   indexer): hidden -> Hi*Di index queries, hidden -> Di index key (one per token), hidden -> Hi head weights.
 
-The projections stay torch GEMMs (plain ones share one autograd node: ``_projections``).  Norm + RoPE + layout is one kernel (``qk_norm_rope``), the attention is
+The projections stay torch GEMMs (plain ones share one autograd node: ``_projections``).  Norm + RoPE + layout is one
+kernel (``qk_norm_rope``), the attention is
 ``dsa_varlen_attn`` (dense causal without an indexer: the reference's behaviour), the gate is one kernel.
 With an indexer the layer keeps the top-k keys per query and leaves the indexer's KL loss in ``self.indexer_loss``
 (the selection passes no gradient; the loss is what trains the indexer); ``indexer_losses(model)`` adds them up
