@@ -272,3 +272,13 @@ def test_what_stands_around_the_projections_is_run(how):
     assert len(counts) == 2
     counts.clear()
     assert any("ProjectionNode" in n for n in _nodes(m(_randn(1, 2048, 256), *rest))) and not counts
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gradients_of_the_operator_own_their_memory(dtype):
+    T, Hq, Hkv, D = 40, 4, 2, 64
+    q, k, v = (_randn(T, h, D, seed=i).to(dtype).requires_grad_(True) for i, h in enumerate((Hq, Hkv, Hkv)))
+    M.dsa_varlen_attn(q, k, v, torch.tensor([0, T], dtype=torch.int32, device=DEV), T).sum().backward()
+    stores = [t.grad.untyped_storage() for t in (q, k, v)]
+    assert len({s.data_ptr() for s in stores}) == 3
+    assert all(s.nbytes() == t.numel() * t.element_size() for s, t in zip(stores, (q, k, v)))

@@ -264,8 +264,7 @@ public:
                                DSA_DTYPE_BF16, max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(w), ws_bytes, stream_of(q)), "dsa_attn_bwd");
         }
         if (split) {
-            const Tensor oq = empty({T, Hq, D / 4}, at::kFloat, q), okv = empty({2, T, Hkv, D / 4}, at::kFloat, q);
-            const Tensor ok = okv.select(0, 0), ov = okv.select(0, 1);
+            const Tensor oq = empty({T, Hq, D / 4}, at::kFloat, q), ok = empty({T, Hkv, D / 4}, at::kFloat, q), ov = empty({T, Hkv, D / 4}, at::kFloat, q);
             check(dsa_split_bf16_combine_qkv(ptr(dq), ptr(dk), ptr(dv), (int64_t)T * Hq, (int64_t)T * Hkv, D / 4, fptr(oq), fptr(ok), fptr(ov), stream_of(q)),
                   "dsa_split_bf16_combine_qkv");
             dq = oq; dk = ok; dv = ov;

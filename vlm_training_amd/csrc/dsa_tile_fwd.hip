@@ -72,7 +72,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const uint32_t lds0 = lds_address(dyn_lds);
     // Addresses of the next tile to request, in scalar registers (the asm statements keep them there); what is left of the
     // block's keys from its first row on, in bytes, bounds the buffer (the last row ends with its own elements: a token
-    // stride may be shorter than a row, or zero, in an expanded tensor)
+    // stride may be shorter than a row, or zero, in an expanded tensor; rows past the segment are then bytes of live rows,
+    // and masked as ever)
     const int Lend = min(L, ntiles * 32);
     auto next = [](const unsigned char *&p, int64_t step) __attribute__((always_inline)) {
         p += step;
