@@ -282,3 +282,29 @@ def test_gradients_of_the_operator_own_their_memory(dtype):
     stores = [t.grad.untyped_storage() for t in (q, k, v)]
     assert len({s.data_ptr() for s in stores}) == 3
     assert all(s.nbytes() == t.numel() * t.element_size() for s, t in zip(stores, (q, k, v)))
+
+
+@pytest.mark.parametrize("gate", [0, 8])
+def test_shared_projections_can_be_differentiated_twice(gate):
+    """create_graph gives what the separate linears give, first and second gradients."""
+    from vlm_training_amd import _lib
+    T, W = 48, 32
+    x, ws = _randn(T, W, grad=True), [_randn(n, W, seed=n, grad=True) for n in (32, 16, 24)]
+
+    def separate(x, ws):
+        ys = [h @ w.t() for h, w in zip((x, x, x.detach()), ws)]
+        halves = ys[0].view(T, -1, 2 * gate).split(gate, 2) if gate else ys[:1]
+        return [*halves, *ys[1:]]
+
+    res = []
+    for call in (lambda: separate(x, ws), lambda: _lib.host().project(x, ws, 2, gate)):
+        for skip in (0, 1):                               # (1: without the first output or its first half)
+            some = call()[skip:]
+            first = torch.autograd.grad([y.float().square().sum() for y in some], [x] + ws, create_graph=True, allow_unused=True)
+            second = torch.autograd.grad([g.float().square().sum() for g in first if g is not None], [x] + ws, allow_unused=True)
+            res.append([*first, *second])
+    for a, b in zip(res[0] + res[1], res[2] + res[3]):
+        assert (a is None) == (b is None)
+        if a is not None:
+            # bf16 sums in another order: two roundings per product and sum, through two gradients
+            assert a.shape == b.shape and (a.float() - b.float()).norm() <= 2e-2 * a.float().norm()

@@ -629,11 +629,37 @@ public:
         ctx->set_materialize_grads(false);
         return outs;
     }
+    // create_graph: the separate linears' gradients in operations that autograd follows
+    static variable_list differentiable_backward(AutogradContext *ctx, const variable_list &s, const variable_list &grads, int64_t n_input, int64_t D) {
+        const int64_t n_w = (int64_t)s.size() - 1, T = s[0].size(0);
+        variable_list res(n_w + 3);
+        for (int64_t i = 0, o = 0; i < n_w; ++i) {
+            Tensor g = grads[o];
+            if (D && i == 0) {
+                Tensor b = grads[o + 1];
+                if (g.defined() || b.defined()) {
+                    if (!g.defined()) g = at::zeros_like(b);
+                    if (!b.defined()) b = at::zeros_like(g);
+                    g = at::cat({g, b}, 2).reshape({T, -1});
+                }
+                ++o;
+            }
+            ++o;
+            if (!g.defined()) continue;
+            if (ctx->needs_input_grad(1 + i)) res[1 + i] = at::mm(g.t(), i < n_input ? s[0] : s[0].detach());
+            if (i < n_input && ctx->needs_input_grad(0)) {
+                const Tensor dx = at::mm(g, s[1 + i]);
+                res[0] = res[0].defined() ? res[0] + dx : dx;
+            }
+        }
+        return res;
+    }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
-        at::AutoDispatchBelowADInplaceOrView below;
         const variable_list s = ctx->get_saved_variables();
         const Tensor &x = s[0];
         const c10::OptionalDeviceGuard guard(x.device());
+        if (at::GradMode::is_enabled()) return differentiable_backward(ctx, s, grads, ctx->saved_data["n"].toInt(), ctx->saved_data["g"].toInt());
+        at::AutoDispatchBelowADInplaceOrView below;
         const int64_t n_w = (int64_t)s.size() - 1, n_input = ctx->saved_data["n"].toInt(), D = ctx->saved_data["g"].toInt(), T = x.size(0);
         variable_list res(n_w + 3);
         std::vector<Tensor> keep;
