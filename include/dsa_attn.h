@@ -256,7 +256,7 @@ int dsa_attn_bwd_parts(const void *dout, const void *q, const void *k, const voi
  * tensors between forward and backward the same way, torch/nn/attention/varlen.py:206-214).  `fwd_ws` is the
  * workspace a dsa_attn_fwd call with the same idx, n, cu_seqlens and max_seqlen filled (the inverted selection
  * bitmap; ignored when idx == NULL); it is only read.  `scratch` holds dsa_attn_bwd_scratch_bytes() bytes that
- * nothing outlives: delta, the launch order of the key tiles and - only for launches of at most 1024 key-tile
+ * nothing outlives: delta, the launch order of the key tiles and - only for launches of at most 1536 key-tile
  * workgroups, which may be cut into pieces - fp32 partial sums (at most 128 MiB).  So between forward and backward
  * a layer holds the bitmap alone.  Refused (DSA_ERR_ARG) while the tile crossover is 0: that forward builds no bitmap.
  */

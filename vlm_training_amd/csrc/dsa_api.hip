@@ -7,6 +7,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "dsa_common.h"
 #include "../../include/dsa_attn.h"
 
 extern "C" {
@@ -651,10 +652,9 @@ extern "C" int dsa_attn_bwd_parts(const void *dout, const void *q, const void *k
 }
 
 // Scratch of the backward that nothing outlives: delta, the launch order of the key tiles and - only for launches small
-// enough to be cut into pieces (at most 1024 workgroups before the cut) - the fp32 partial sums of those pieces.
+// enough to be cut into pieces (dkv_pieces_max_wg workgroups before the cut) - the fp32 partial sums of those pieces.
 static size_t bwd_partial_bytes_for(int T, int N, int Hkv, int D) {
-    const int64_t wg_per_tile = (int64_t)Hkv * (D > 128 ? 2 : 1);
-    if (((int64_t)T / 128 + N) * wg_per_tile > 4 * 256) return 0;
+    if (((int64_t)T / 128 + N) * Hkv > dkv_pieces_max_wg(D)) return 0;
     return dsa_tile_dkv_partial_bytes(T);
 }
 extern "C" size_t dsa_attn_bwd_scratch_bytes(int T, int N, int Hq, int Hkv, int D) {

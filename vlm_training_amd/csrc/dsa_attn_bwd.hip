@@ -7,7 +7,7 @@
 //                                                         (dsa_bwd_dq_kernel; dense rows: the tile dQ kernels)
 //   inverted selection: bitmap[t][w] bit b <=> query t selected key column 32w+b of its segment
 //                                                         (dsa_bitmap_kernel); the key-side passes
-//                                                         dsa_tile_dkv2_kernel / dsa_tile_dkvpc_kernel reduce
+//                                                         (dsa_tile_dkv.hip) reduce
 //                                                         every key row from it without atomics.
 #include "dsa_common.h"
 

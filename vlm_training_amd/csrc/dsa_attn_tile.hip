@@ -1,5 +1,6 @@
-// Tile kernels: dK / dV, dQ at head_dim 97 to 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap
-// mask (the forward: dsa_tile_fwd.hip, dQ elsewhere: dsa_tile_dq.hip, the indexer backward: dsa_tile_idx.hip).  They do the same
+// Tile kernels: dQ at head_dim 97 to 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask, and the
+// launch of dK / dV (the forward: dsa_tile_fwd.hip, dQ elsewhere: dsa_tile_dq.hip, dK / dV: dsa_tile_dkv.hip, the indexer backward:
+// dsa_tile_idx.hip).  They do the same
 // arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
@@ -469,45 +470,42 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 // behind it, and the hardware starts workgroups in grid order: handed out segment by segment, the long
 // walks of a late long segment start late and the launch ends on them.  This kernel (one workgroup) lists
 // the 128-key tiles of all segments longest walk first -
-//   mode 0: by the number of tiles behind them, across segments (best balance; for launches of a few rounds
-//           of workgroups),
-//   mode 1: the segments by length, each one's tiles together (workgroups that run side by side then walk the
-//           same q / dO rows and share them in L2, which is worth more than the balance once a launch runs
-//           for many rounds - or without a causal mask, whose walks are equally long within a segment: 4000 patches,
+//   mode 0: by the number of tiles behind them, across segments (32 768 tokens in eight segments, segment by segment in order
+//           of length: 2380 instead of 2297 us - CUs busy 0.83 instead of 0.91 of the launch; octave by octave of the walk's
+//           length, segments together within one: level),
+//   mode 1: the segments by length, each one's tiles together, without a causal mask: walks are equally long within a
+//           segment, and workgroups that run side by side walk the same q / dO rows and share them in L2 (4000 patches,
 //           forward and backward, 170 -> 154 us),
-//   mode 2: as mode 0, and long walks cut into pieces of `pb` steps (a step = `qb` queries), for launches with
-//           fewer workgroups than a few rounds of the chip: a launch then ends with its longest walk, however
-//           few the workgroups.  A tile in pieces leaves one fp32 partial dK / dV per piece, added in piece
-//           order by dsa_dkv_pieces_reduce_kernel.  Walks are cut only if the longest is more than twice the
-//           steps a CU gets in a balanced launch (all walks x `wg_per_tile` workgroups / 256); pb = the largest
-//           power of two up to half of that (at least 32), doubled until at most `item_cap` entries and
-//           `slot_cap` partial slots are needed; it depends on cu_seqlens and these parameters only.
+//   mode 2: long walks cut into equal pieces of at most `pb` steps (a step = `qb` queries), listed by length, for launches of up
+//           to three rounds of workgroups: a launch then ends with its longest walk, however few the workgroups.  A tile in
+//           pieces leaves one fp32 partial dK / dV per piece, added in piece order by dsa_dkv_pieces_reduce_kernel.  pb (see
+//           below) depends on cu_seqlens and the parameters of the launch only.
 // Table:
 //   order[0] = number of entries (or -1: too many segments or tiles for the table, use the plain order),
-//   order[1] = pb (0: no walk is cut), order[2] = number of tiles that are cut,
-//   order[4 + 4 s .. 7 + 4 s] = segment, tile, piece, first partial slot of the tile (-1: not cut) of entry s,
+//   order[1] = queries of a piece, pb steps of qb (0: no walk is cut), order[2] = number of tiles that are cut,
+//   order[4 + 4 s .. 7 + 4 s] = first row and length of the segment, tile | piece << 13, first partial slot of the tile (-1: not
+//   cut) of entry s,
 //   behind the `cap` entries: the entry of the first piece of every cut tile.
 // The pieces of a tile are counted from the walk's length bound 128 r / qb of its rank r (tiles behind it,
 // itself included); a tile whose own walk is shorter leaves its last pieces empty (the kernels and the
 // reduction count the pieces from the walk itself).
 // The order changes the schedule only; every tile is still reduced in a fixed order.
 // ==================================================================================================
-#define DSA_ORDER_MAX_SEGS 4096
 #define DSA_ORDER_MAX_TILES 8192                         // tiles of the longest segment
 #define DSA_ORDER_EXTRA 4096                             // entries beyond one per tile (pieces)
 #define DSA_ORDER_SPLIT_MAX_TILES 1024                   // mode 2: one thread per rank
 static_assert(DSA_ORDER_MAX_TILES + 1 >= 2 * DSA_ORDER_MAX_SEGS, "the rank tables of the by-segment order share cnt[]");
-__device__ __forceinline__ void order_entry(int32_t *order, int slot, int seg, int tile, int piece, int mslot) {
-    *reinterpret_cast<int4 *>(order + 4 + 4 * slot) = make_int4(seg, tile, piece, mslot);
+__device__ __forceinline__ void order_entry(int32_t *order, const int32_t *cu, int slot, int seg, int tile, int piece, int mslot) {
+    const int s0 = cu[seg];
+    *reinterpret_cast<int4 *>(order + 4 + 4 * slot) = make_int4(s0, cu[seg + 1] - s0, tile | piece << 13, mslot);
 }
-struct TileOrder { int cap, mode, qb, wg_per_tile, item_cap, slot_cap; };
+struct TileOrder { int cap, mode, qb, wg_per_tile, item_cap, slot_cap, slots, share8, extra; };
 __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N, const TileOrder &o_, int32_t *__restrict__ order) {
     const int cap = o_.cap, mode = o_.mode, qb = o_.qb, wg_per_tile = o_.wg_per_tile, item_cap = o_.item_cap, slot_cap = o_.slot_cap;
     __shared__ int nt[DSA_ORDER_MAX_SEGS];               // tiles per segment
     __shared__ int cnt[DSA_ORDER_MAX_TILES + 1];         // cnt[r]: segments with at least r tiles; then: slots before rank r
     __shared__ int part[1024];
-    __shared__ unsigned long long part64[16];
-    __shared__ int maxnt_s, sum_a, sum_b;
+    __shared__ int maxnt_s, sum_a;
     const int tid = threadIdx.x;
     if (N > DSA_ORDER_MAX_SEGS) {
         if (tid == 0) { order[0] = -1; order[1] = 0; order[2] = 0; }
@@ -554,7 +552,7 @@ __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N
         if (tid == 0) order[0] = total;
         for (int rk = 0; rk < N; ++rk) {
             const int seg = seg_of[rk], f = first[rk];
-            for (int j = tid; j < nt[seg]; j += 1024) order_entry(order, f + j, seg, j, 0, -1);
+            for (int j = tid; j < nt[seg]; j += 1024) order_entry(order, cu, f + j, seg, j, 0, -1);
         }
         return;
     }
@@ -565,70 +563,67 @@ __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N
     }
     __syncthreads();
     if (mode == 2 && maxnt <= DSA_ORDER_SPLIT_MAX_TILES) {
-        // thread tid owns rank r = maxnt - tid; pieces of a tile of rank r: ceil((128 r / qb) / pb)
-        const int r = maxnt - tid;
-        const int c = r >= 1 ? cnt[r] : 0, steps = r >= 1 ? r * (128 / qb) : 0;
-        // steps of all walks against the longest one: with `ideal` steps per CU in a balanced launch, walks are cut
-        // only if the longest is more than twice that (below, the pieces' own cost - a pipeline fill each, fp32 partial
-        // sums written and read back - outweighs the balance), into pieces of about half of it
+        // A tile of rank r is cut into ceil((128 r / qb) / pb) pieces of equal length.  pb = `share8` eighths of the steps
+        // that a balanced launch gives each of its `slots` concurrent workgroups, and `extra` (a piece costs as much as 7 to 9 steps
+        // besides its own, and its partial sums), or the first of the larger candidates (a quarter of an octave apart) whose entries and
+        // partial sums fit; a wave counts two candidates.
         if (tid == 0) sum_a = 0;
         __syncthreads();
-        if (c) atomicAdd(&sum_a, c * steps);
-        __syncthreads();
-        const int longest = maxnt * (128 / qb);
-        const int ideal = (int)(((int64_t)sum_a * wg_per_tile + 255) / 256);
-        __syncthreads();
-        int pb = 32;
-        while (2 * pb <= ideal / 2) pb <<= 1;            // the largest power of two up to ideal / 2, at least 32
-        if (longest <= 2 * ideal) pb = 1 << 30;
-        for (;; pb <<= 1) {
-            const int np = (steps + pb - 1) / pb;
-            if (tid == 0) { sum_a = 0; sum_b = 0; }
-            __syncthreads();
-            if (c) {
-                atomicAdd(&sum_a, c * np);
-                if (np > 1) atomicAdd(&sum_b, c * np);
-            }
-            __syncthreads();
-            const bool fits = sum_a <= item_cap && sum_a <= cap && sum_b <= slot_cap;
-            const bool whole = pb >= longest;                     // no walk is cut any more
-            __syncthreads();
-            if (fits || whole) break;
+        const int spt = 128 / qb, longest = maxnt * spt;          // steps of a rank
+        {
+            int mine = 0;
+            for (int r = 1 + tid; r <= maxnt; r += 1024) mine += cnt[r] * r * spt;
+            if (mine) atomicAdd(&sum_a, mine);
         }
-        const int np = (steps + pb - 1) / pb, items = c * np, mults = np > 1 ? c * np : 0;
-        // entries, partial slots and cut tiles of the larger ranks: one scan over the triple (21 bits each of a 64-bit
-        // word: the caps keep every sum below 2^21)
-        const unsigned long long mine = (unsigned long long)items | ((unsigned long long)mults << 21) | ((unsigned long long)(np > 1 ? c : 0) << 42);
-        unsigned long long incl = mine;                  // inclusive scan: inside the wave by lane shifts, then over the 16 waves
+        __syncthreads();
+        const int64_t ideal = ((int64_t)sum_a * wg_per_tile + o_.slots - 1) / o_.slots;
+        const int pb0 = max((int)min(ideal * o_.share8 / 8 + o_.extra, (int64_t)longest), max(8, 32 / qb));
+        auto candidate = [&](int k) { return (pb0 * (4 + (k & 3)) << (k >> 2)) / 4; };
         const int ln = tid & 63, wvi = tid >> 6;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned int lo32 = __shfl_up((unsigned int)incl, d, 64), hi32 = __shfl_up((unsigned int)(incl >> 32), d, 64);
-            if (ln >= d) incl += (unsigned long long)lo32 | ((unsigned long long)hi32 << 32);
+        for (int k = wvi; k < 32; k += 16) {
+            const int pbk = candidate(k);
+            int ni = 0, nm = 0;
+            for (int r = 1 + ln; r <= maxnt; r += 64) {
+                const int np = (r * spt + pbk - 1) / pbk;
+                ni += cnt[r] * np;
+                if (np > 1) nm += cnt[r] * np;
+            }
+            ni = wave_sum_i(ni);
+            nm = wave_sum_i(nm);
+            if (ln == 0) part[k] = ni <= item_cap && ni <= cap && nm <= slot_cap;
         }
-        if (ln == 63) part64[wvi] = incl;
         __syncthreads();
-        unsigned long long wave_before = 0ull, all = 0ull;
-        for (int w2 = 0; w2 < 16; ++w2) {
-            const unsigned long long t2 = part64[w2];
-            if (w2 < wvi) wave_before += t2;
-            all += t2;
+        int pb = 1 << 30;
+        for (int k = 31; k >= 0; --k)
+            if (part[k]) pb = candidate(k);
+        __syncthreads();
+        // thread tid owns rank r = tid + 1.  Entries are listed by length (then by rank, then by segment): its entries, partial slots
+        // and cut tiles start behind those of the ranks in front of it.
+        const int r = 1 + tid, c = r <= maxnt ? cnt[r] : 0, steps = r * spt, np = (steps + pb - 1) / pb;
+        if (r <= maxnt) part[tid] = ((steps + np - 1) / np << 13) | np;         // at most 2^16 steps, 2^13 pieces
+        __syncthreads();
+        int slot = 0, ms = 0, mt = 0, total = 0, cuts = 0;
+        const int me = r <= maxnt ? part[tid] : 0;
+        for (int o = maxnt; o >= 1; --o) {
+            const int it = part[o - 1], no = it & 8191, co = cnt[o];
+            total += co * no;
+            if (no > 1) cuts += co;
+            if ((it >> 13) > (me >> 13) || ((it >> 13) == (me >> 13) && o > r)) {
+                slot += co * no;
+                if (no > 1) { ms += co * no; mt += co; }
+            }
         }
-        const unsigned long long excl = wave_before + incl - mine;
-        const int before[3] = {(int)(excl & 0x1fffffull), (int)((excl >> 21) & 0x1fffffull), (int)(excl >> 42)};
-        const int total = (int)(all & 0x1fffffull);
         if (total > cap || total > item_cap) {           // (only when even whole walks do not fit)
             if (tid == 0) order[0] = -1;
             return;
         }
-        if (tid == 0) { order[0] = total; order[1] = pb >= longest ? 0 : pb; order[2] = (int)(all >> 42); }
+        if (tid == 0) { order[0] = total; order[1] = pb >= longest ? 0 : pb * qb; order[2] = cuts; }
         if (c) {
-            int slot = before[0], ms = before[1], mt = before[2];
             int32_t *cut = order + 4 + 4 * cap;          // entries of the first pieces of the cut tiles, for the reduction
             for (int i = 0; i < N; ++i)
                 if (nt[i] >= r) {
                     if (np > 1) cut[mt++] = slot;
-                    for (int pc = 0; pc < np; ++pc) order_entry(order, slot++, i, nt[i] - r, pc, np > 1 ? ms : -1);
+                    for (int pc = 0; pc < np; ++pc) order_entry(order, cu, slot++, i, nt[i] - r, pc, np > 1 ? ms : -1);
                     if (np > 1) ms += np;
                 }
         }
@@ -670,7 +665,7 @@ __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N
     for (int r = 1 + tid; r <= maxnt; r += 1024) {
         int slot = cnt[r];
         for (int i = 0; i < N; ++i)
-            if (nt[i] >= r) order_entry(order, slot++, i, nt[i] - r, 0, -1);
+            if (nt[i] >= r) order_entry(order, cu, slot++, i, nt[i] - r, 0, -1);
     }
 }
 __global__ __launch_bounds__(1024) void dsa_tile_order_kernel(const int32_t *__restrict__ cu, int N, TileOrder o, int32_t *__restrict__ order) {
@@ -686,60 +681,8 @@ __global__ __launch_bounds__(1024) void dsa_tile_order_delta_kernel(const int32_
 }
 static inline int order_entries_cap(int T) { return T / 128 + DSA_ORDER_MAX_SEGS + 1 + DSA_ORDER_EXTRA; }
 extern "C" size_t dsa_tile_order_bytes(int T) { return ((size_t)order_entries_cap(T) * 5 + 4) * sizeof(int32_t); }
-// the tile (and the piece of its walk) of workgroup slot `slot`: from the order table when there is one, else
-// segment by segment
-__device__ __forceinline__ bool locate_key_tile(const int32_t *order, const int32_t *cu, int N, int slot, int &s0, int &L, int &blk,
-                                                int &piece, int &mslot, int &pb) {
-    piece = 0;
-    mslot = -1;
-    pb = 0;
-    if (order) {
-        const int total = __builtin_amdgcn_readfirstlane(order[0]);
-        if (total >= 0) {
-            if (slot >= total) return false;
-            // (every lane reads the same words; the lane reads tell the compiler that the results are wave-uniform)
-            const int4 e = *reinterpret_cast<const int4 *>(order + 4 + 4 * slot);
-            const int seg = min(max(__builtin_amdgcn_readfirstlane(e.x), 0), N - 1);
-            blk = __builtin_amdgcn_readfirstlane(e.y);
-            piece = max(__builtin_amdgcn_readfirstlane(e.z), 0);
-            mslot = __builtin_amdgcn_readfirstlane(e.w);
-            pb = max(__builtin_amdgcn_readfirstlane(order[1]), 0);
-            s0 = __builtin_amdgcn_readfirstlane(cu[seg]);
-            L = __builtin_amdgcn_readfirstlane(cu[seg + 1]) - s0;
-            return blk >= 0;
-        }
-    }
-    return locate_block(cu, N, slot, 128, false, s0, L, blk);
-}
-// A walk of `nblocks` steps (block nblocks-1-b at step b, `QB` queries each, the queries q0 .. Lq-1) cut into pieces
-// of `pb` steps: narrows q0, Lq and nblocks to piece `piece` and returns the number of pieces (1: the whole walk,
-// 0: this piece is empty).  Block boundaries stay where they are, so a piece's blocks are the walk's own.
-__device__ __forceinline__ int walk_piece(int pb, int piece, int QB, int &q0, int &Lq, int &nblocks) {
-    if (pb <= 0 || nblocks <= pb) return piece == 0 ? 1 : 0;
-    const int np = (nblocks + pb - 1) / pb;
-    if (piece >= np) return 0;
-    const int b_lo = piece * pb, b_hi = min(b_lo + pb, nblocks);
-    if (b_lo > 0) Lq = q0 + (nblocks - b_lo) * QB;
-    q0 += (nblocks - b_hi) * QB;
-    nblocks = b_hi - b_lo;
-    return np;
-}
-// one 32-column d-tile of a C-layout accumulator as fp32 (lane = row j; a lane holds the four columns
-// 8*g4 + 4*h + {0..3} of every group g4)
-__device__ __forceinline__ void store_c_tile_f32(float *row_dt, const f32x16 &acc, int h) {
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-        const f32x4 w = {acc[4 * g4], acc[4 * g4 + 1], acc[4 * g4 + 2], acc[4 * g4 + 3]};
-        *reinterpret_cast<f32x4 *>(row_dt + 8 * g4 + 4 * h) = w;
-    }
-}
-// fp32 partial dK / dV of piece `piece` of a tile in pieces: [slot][kv head][dK | dV][128 keys][D to the next 32]
-__device__ __forceinline__ float *piece_partial(float *partial, int mslot, int piece, int Hkv, int kvh, int D) {
-    return partial + ((int64_t)(mslot + piece) * Hkv + kvh) * (2 * 128 * (int64_t)D);
-}
 // Adds the pieces of every tile that was cut, in piece order, and writes its dK (times the softmax scale) and dV
-// rows of D elements (`pitch` in the partial sums).  Grid: (cut tiles at most, kv heads, DSA_PIECES_Z slices of a tile's rows).
-#define DSA_PIECES_Z 4
+// rows of D elements (`pitch` in the partial sums).  Grid: (cut tiles at most, kv heads, pitch / 8 slices of 256 units).
 __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_t *__restrict__ order, int cap,
                                                                     const float *__restrict__ partial, const int32_t *__restrict__ cu,
                                                                     int N, int Hkv, int D, int pitch, int qb, int seq_clamp, float scale,
@@ -752,869 +695,38 @@ __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_
     L = min(L, seq_clamp);
     const int c0 = blk * 128;
     if (c0 >= L) return;
+    pb /= qb;
     const int nblocks = (L - c0 + qb - 1) / qb;          // (pieces only exist for causal launches: the walk starts at the tile)
     if (nblocks <= pb) return;                           // (its walk fits one piece after all: piece 0 wrote the rows itself)
     const int np = (nblocks + pb - 1) / pb, kvh = blockIdx.y;
-    const int keys = min(128, L - c0), cpr = D / 4;      // 16-byte chunks per row
+    // a thread's unit: eight columns of a row, in the two halves of a wave's store
+    const int DT = pitch / 32, unit = blockIdx.z * 256 + threadIdx.x, j = unit & 31, part = unit >> 5;     // part: [dK | dV][key group][d-tile][8 columns]
+    const int m = part / (16 * DT), grp = part / (4 * DT) % 4, col = part % (4 * DT) * 8, key = grp * 32 + j;
+    if (m > 1 || key >= min(128, L - c0) || col >= D) return;
     const int64_t slot_f = 2 * 128 * (int64_t)pitch;         // floats per (slot, kv head)
-    const float *base = partial + ((int64_t)mslot * Hkv + kvh) * slot_f;
-    constexpr int U = 4;                                 // independent chunks per thread and pass
-    const int chunks = 2 * keys * cpr;                   // dK rows, then dV rows
-    for (int c0_ = (blockIdx.z * 256 + threadIdx.x) * U; c0_ < chunks; c0_ += DSA_PIECES_Z * 256 * U) {
-        f32x4 acc[U];
-        int64_t off[U];
+    const float *src = partial + ((int64_t)mslot * Hkv + kvh) * slot_f + part * 256 + j * 4;
+    f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+    constexpr int U = 4;                                 // pieces whose loads are in flight together
+    for (int pc = 0; pc < np; pc += U) {                 // piece order: the sum does not depend on the schedule
+        f32x4 x0[U], x1[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int c = min(c0_ + u, chunks - 1);
-            const int m = c / (keys * cpr), rest = c % (keys * cpr);
-            off[u] = ((int64_t)m * 128 + rest / cpr) * pitch + (rest % cpr) * 4;
-            acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        for (int pc = 0; pc < np; pc += 2) {             // piece order: the sum does not depend on the schedule
-            const bool two = pc + 1 < np;
-            const float *src0 = base + (int64_t)pc * Hkv * slot_f, *src1 = base + (int64_t)(two ? pc + 1 : pc) * Hkv * slot_f;
-            f32x4 x0[U], x1[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                x0[u] = *reinterpret_cast<const f32x4 *>(src0 + off[u]);
-                x1[u] = *reinterpret_cast<const f32x4 *>(src1 + off[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                acc[u] += x0[u];
-                if (two) acc[u] += x1[u];
-            }
+            const float *p = src + (int64_t)min(pc + u, np - 1) * Hkv * slot_f;
+            x0[u] = *reinterpret_cast<const f32x4 *>(p);
+            x1[u] = *reinterpret_cast<const f32x4 *>(p + 128);
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int c = c0_ + u;
-            if (c < chunks) {
-                const int m = c / (keys * cpr), rest = c % (keys * cpr);
-                const float mul = m ? 1.f : scale;
-                bf16_t *outp = m ? dv : dk;
-                uint32_t *dst = reinterpret_cast<uint32_t *>(outp + ((int64_t)(s0 + c0 + rest / cpr) * Hkv + kvh) * D + (rest % cpr) * 4);
-                dst[0] = pack2bf(acc[u][0] * mul, acc[u][1] * mul);
-                dst[1] = pack2bf(acc[u][2] * mul, acc[u][3] * mul);
-            }
-        }
+        for (int u = 0; u < U; ++u)
+            if (pc + u < np) { a0 += x0[u]; a1 += x1[u]; }
     }
-}
-
-// ==================================================================================================
-// dK, dV for head_dim 256, producer/consumer form, key-stationary ("scatter by key": every key row is
-// reduced by one wave, in a fixed query order - or, when the launch cuts the walk into pieces, by one wave per
-// piece and a sum over the pieces in piece order - so the result needs no atomics and is bit-reproducible).
-// A workgroup owns a 128-key tile (4 groups of 32 keys) of one segment and kv head and
-// walks the later queries in blocks of 32 (query, head) rows, from the end of the segment down to the key
-// tile: workgroups that run side by side then read the same q / dO rows at about the same time and share
-// them in L2.
-//   waves 0-3 (producers, one per key group): S = Q K^T and dP = dO V^T against the group's K / V rows
-//     held in registers (128 of them), then P and dS = P * (dP - delta) in bf16, written to LDS in MFMA B
-//     layout.
-//   waves 4-7 (consumers, one per key group): dV^T += dO^T P and dK^T += Q^T dS for block b-1,
-//     A operands read transposed from the staged q / dO block, B operands read back from LDS.  They
-//     also do all the staging (global -> registers -> LDS one block ahead).
-// A consumer's accumulators for all of head_dim would fill 256 registers, so a workgroup covers one half
-// of head_dim (`dhalf`, the low bit of its index: the consumers accumulate and write that half, the producers
-// repeat S and dP: 48 instead of 32 MFMAs per 32x32 block pair and half).
-// LDS (dynamic, ~158 KiB): q/dO blocks in a ring of three, P/dS (and, for blocks of large probabilities,
-// the bf16 rounding remainder of P) in a ring of two, row statistics and selection words in a ring of
-// three.  One barrier per block.  (head_dim <= 128 runs dsa_tile_dkv2_kernel below.)
-// ==================================================================================================
-template <int D, bool HAS_IDX, int GSHIFT>
-__global__ __launch_bounds__(512, 1) void dsa_tile_dkvpc_kernel(
-    const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
-    const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
-    const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, int causal, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
-    bf16_t *__restrict__ dv) {
-    static_assert(D == 256, "head_dim <= 128 runs dsa_tile_dkv2_kernel");
-    constexpr int KS = D / 16, DT = D / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NQD = 3, LEAD = 1;                     // q/dO ring slots; blocks staged ahead of the producers
-    constexpr int DTC = DT / 2;                          // d-tiles of one half of head_dim
-    // the two halves of head_dim are neighbours in the grid, so that the longest walks of both start in the first round
-    const int dhalf = blockIdx.x & 1, bx = blockIdx.x >> 1;
-    const int dt0 = dhalf * DTC;
-    constexpr int NCHUNK = 32 * CPR;                     // 16-byte chunks per staged operand
-    constexpr int CPT = NCHUNK / 256;                    // chunks per consumer thread and operand
-    constexpr int Gp = 1 << GSHIFT, QB = 32 >> GSHIFT;
-    constexpr int QD_SLOT = 2 * TILE_B;                  // q block | dO block
-    // 4 key groups x {P (rows 0-15 | 16-31), dS (same), rounding remainder of P (same)} x 64 lanes x 16 B
-    constexpr int PD_GROUP = 6 * 1024, PD_SLOT = 4 * PD_GROUP;
-    constexpr int AUX_SLOT = (32 + 32 + 4 * 32) * 4;     // lse | delta | selection words [key group][query]
-    static_assert(CPT >= 1 && NCHUNK % 256 == 0, "every consumer thread stages whole chunks");
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_lds[];
-    unsigned char *const qd_ring = dyn_lds;                          // NQD slots
-    unsigned char *const pd_ring = dyn_lds + NQD * QD_SLOT;          // 2 slots
-    unsigned char *const aux_ring = pd_ring + 2 * PD_SLOT;           // NQD slots
-    uint32_t *const split_flag = reinterpret_cast<uint32_t *>(aux_ring + NQD * AUX_SLOT);   // [P/dS slot][key group]
-    auto qslot = [](int b) { return b % 3; };
-
-    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);         // wave-uniform for the compiler too
-    const int kg = wv & 3;
-    const bool consumer = wv >= 4;
-    const int G = Hq / Hkv;
-    const int kvh = bx % Hkv;
-    int s0, L, blk, piece, mslot, pb;
-    if (!locate_key_tile(order, cu, N, bx / Hkv, s0, L, blk, piece, mslot, pb)) return;
-    if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
-    if (blk * 128 >= L) return;                         // (whole workgroup, before its first barrier)
-    const int c0 = blk * 128, kc = c0 + kg * 32;
-    const int mykey = kc + j;
-    const bool key_ok = mykey < L;
-    const int64_t krow = (int64_t)(s0 + min(mykey, L - 1)) * Hkv + kvh;
-    const float scale_log2 = scale * LOG2E_F;
-    // the walk: queries q0 .. Lq-1 in nblocks steps - all queries that can see this key tile, or one piece of them
-    int q0_ = causal ? c0 : 0, Lq_ = L, nblocks_ = (L - q0_ + QB - 1) / QB;
-    const int npieces = walk_piece((causal && partial && mslot >= 0) ? pb : 0, piece, QB, q0_, Lq_, nblocks_);
-    if (npieces == 0) return;
-    const int q0 = q0_, Lq = Lq_, nblocks = nblocks_;
-
-    if (consumer) {
-        // ================= consumers: stage block b+2, then dV^T, dK^T of block b-1 =================
-        const int ctid = tid - 256;
-        const uint32_t *aux_base;
-        int aux_q = 0, aux_stride = 1;
-        bool aux_mask_ok = false;
-        if (ctid < 64) {                                 // 0..31: lse of row ctid, 32..63: delta of row ctid-32
-            const int row = ctid & 31;
-            const int hd = min(row & (Gp - 1), G - 1);
-            aux_q = row >> GSHIFT;
-            aux_base = reinterpret_cast<const uint32_t *>((ctid < 32 ? lse : delta) + (int64_t)(kvh * G + hd) * T + s0);
-        } else if (HAS_IDX && ctid < 64 + 4 * QB) {      // selection word of (key group w, query qi)
-            const int w = (ctid - 64) / QB;
-            aux_q = (ctid - 64) % QB;
-            aux_stride = ldw;
-            aux_mask_ok = (c0 >> 5) + w < ldw;
-            aux_base = bitmap + (int64_t)s0 * ldw + (aux_mask_ok ? (c0 >> 5) + w : 0);
-        } else {
-            aux_base = reinterpret_cast<const uint32_t *>(lse);
-        }
-        // Per-thread element offsets of block 0 and what the last block adds to them (its rows past the
-        // segment end re-read row L-1); in between a block moves every address by the same stride, so
-        // the loop does no index arithmetic per row.
-        const int last = nblocks - 1;
-        const int64_t blk_bytes = (int64_t)QB * Hq * D * 2;
-        const unsigned char *qp[CPT], *dp[CPT];          // this thread's chunks of the block loaded last
-        int64_t dlast[CPT];
-        int lds_off[CPT];
-        bool row_dead_last[CPT], head_ok[CPT];
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int c = i * 256 + ctid, srow = c / CPR, sch = c % CPR;
-            const int hd = min(srow & (Gp - 1), G - 1);
-            const int qr = srow >> GSHIFT;
-            const int over = max(q0 + last * QB + qr - (Lq - 1), 0);     // rows past the end in the last block
-            const int64_t off = ((int64_t)(s0 + q0 + last * QB + qr - over) * Hq + kvh * G + hd) * D + sch * 8;
-            qp[i] = reinterpret_cast<const unsigned char *>(q + off);
-            dp[i] = reinterpret_cast<const unsigned char *>(dout + off);
-            dlast[i] = -(int64_t)over * Hq * D * 2;
-            row_dead_last[i] = over > 0;
-            head_ok[i] = (srow & (Gp - 1)) < G;
-            lds_off[i] = tile_off<D>(srow, sch);
-        }
-        const int64_t aux_blk_bytes = (int64_t)aux_stride * QB * 4;
-        const int aux_over = max(q0 + last * QB + aux_q - (Lq - 1), 0);
-        const int64_t aux_dlast = -(int64_t)aux_stride * aux_over * 4;
-        const unsigned char *ap =
-            reinterpret_cast<const unsigned char *>(aux_base + (int64_t)aux_stride * (q0 + last * QB + aux_q - aux_over));
-        // one register set (four chunks per operand and thread): a global load has one block-time to land
-        u32x4 qst0[CPT], dost0[CPT];
-        uint32_t aux_st0;
-        // loads the block of step b (block last - b), called with b = 0, 1, 2, ... in turn; past step
-        // `last` it reads block 0 again
-        auto gload = [&](int b, u32x4 (&qst)[CPT], u32x4 (&dost)[CPT], uint32_t &aux_st) {
-            if (b >= 1 && b <= last) {
-#pragma unroll
-                for (int i = 0; i < CPT; ++i) { qp[i] -= blk_bytes; dp[i] -= blk_bytes; }
-                ap -= aux_blk_bytes;
-                if (b == 1) {                            // leaving the last block: undo its row clamp
-#pragma unroll
-                    for (int i = 0; i < CPT; ++i) { qp[i] -= dlast[i]; dp[i] -= dlast[i]; }
-                    ap -= aux_dlast;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) {
-                qst[i] = *reinterpret_cast<const u32x4 *>(qp[i]);
-                dost[i] = *reinterpret_cast<const u32x4 *>(dp[i]);
-            }
-            aux_st = *reinterpret_cast<const uint32_t *>(ap);
-        };
-        auto lstore = [&](int b, const u32x4 (&qst)[CPT], const u32x4 (&dost)[CPT], uint32_t aux_st) {   // step b -> ring slot b % 3
-            unsigned char *slot = qd_ring + qslot(b) * QD_SLOT;
-            float *lse_s = reinterpret_cast<float *>(aux_ring + qslot(b) * AUX_SLOT);
-            float *dlt_s = lse_s + 32;
-            uint32_t *mask_s = reinterpret_cast<uint32_t *>(dlt_s + 32);
-            // rows past the segment (last block only) and padded heads are zeroed: they add nothing to dK, dV
-            const bool tail = b == 0 || b > last;
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) {
-                u32x4 qv = qst[i], dv4 = dost[i];
-                if (tail || G != Gp) {
-                    const bool live = head_ok[i] && !(b > last || (b == 0 && row_dead_last[i]));
-                    const u32x4 z4 = {0u, 0u, 0u, 0u};
-                    qv = live ? qv : z4;
-                    dv4 = live ? dv4 : z4;
-                }
-                *reinterpret_cast<u32x4 *>(slot + lds_off[i]) = qv;
-                *reinterpret_cast<u32x4 *>(slot + TILE_B + lds_off[i]) = dv4;
-            }
-            // a row that is not live (past the segment, past the walk, a padded head) has q = dO = 0 but would read a
-            // live row's lse: with lse far below zero its P = exp(0 - lse) overflows and 0 * inf reaches dK and dV.  It gets
-            // an lse that makes P vanish instead.
-            const bool row_dead = b > last || (b == 0 && aux_over > 0) || ((ctid & 31) & (Gp - 1)) >= G;
-            if (ctid < 32) lse_s[ctid] = row_dead ? 1e30f : __uint_as_float(aux_st) * LOG2E_F;
-            else if (ctid < 64) dlt_s[ctid - 32] = row_dead ? 0.f : __uint_as_float(aux_st);
-            else if (HAS_IDX && ctid < 64 + 4 * QB)
-                mask_s[((ctid - 64) / QB) * 32 + (ctid - 64) % QB] =
-                    (aux_mask_ok && !(b > last || (b == 0 && aux_over > 0))) ? aux_st : 0u;
-        };
-        gload(0, qst0, dost0, aux_st0);
-        lstore(0, qst0, dost0, aux_st0);
-        gload(1, qst0, dost0, aux_st0);
-        __syncthreads();                                 // the first step staged
-
-        f32x16 dkacc[DTC], dvacc[DTC];
-#pragma unroll
-        for (int dt = 0; dt < DTC; ++dt) { dkacc[dt] = zero16(); dvacc[dt] = zero16(); }
-        auto consume = [&](int b) {
-            const unsigned char *qt = qd_ring + qslot(b) * QD_SLOT + dt0 * 64;
-            lds_u8 *pt[4];                  // lane addresses in the q block; the dO block sits TILE_B behind
-#pragma unroll
-            for (int vv = 0; vv < 4; ++vv) {
-                pt[vv] = (lds_u8 *)qt + lo.tr[vv];
-                asm volatile("" : "+v"(pt[vv]));         // keep "address + immediate" reads: no re-association
-            }
-            const unsigned char *pd = pd_ring + (b & 1) * PD_SLOT + kg * PD_GROUP + lane * 16;
-            const bf16x8 pB0 = *reinterpret_cast<const bf16x8 *>(pd), pB1 = *reinterpret_cast<const bf16x8 *>(pd + 1024);
-            const bf16x8 dB0 = *reinterpret_cast<const bf16x8 *>(pd + 2048), dB1 = *reinterpret_cast<const bf16x8 *>(pd + 3072);
-#pragma unroll
-            for (int dt = 0; dt < DTC; ++dt) {
-                dvacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 0, dt, TILE_B), pB0, dvacc[dt]);
-                dkacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 0, dt, 0), dB0, dkacc[dt]);
-                dvacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 1, dt, TILE_B), pB1, dvacc[dt]);
-                dkacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 1, dt, 0), dB1, dkacc[dt]);
-            }
-            sched_reads_ahead<4 * DTC, 3, 2, 4>();
-            // blocks that hold a large probability also carry what bf16 rounded off P (see store_pd): dV += dO^T P_lo
-            if (__builtin_amdgcn_readfirstlane(split_flag[(b & 1) * 4 + kg])) {
-                const bf16x8 pL0 = *reinterpret_cast<const bf16x8 *>(pd + 4096), pL1 = *reinterpret_cast<const bf16x8 *>(pd + 5120);
-#pragma unroll
-                for (int dt = 0; dt < DTC; ++dt) {
-                    dvacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 0, dt, TILE_B), pL0, dvacc[dt]);
-                    dvacc[dt] = mfma32(LaneOffsets<D>::trop_at(pt, 1, dt, TILE_B), pL1, dvacc[dt]);
-                }
-            }
-        };
-        // one consumer step: stage step b+1 from the register set, refill the set with step b+2, then the MFMAs of step b-1
-        for (int b = 0; b <= nblocks; ++b) {
-            lstore(b + LEAD, qst0, dost0, aux_st0);      // its slot was last read (as step b+1-3) before the previous barrier
-            gload(b + LEAD + 1, qst0, dost0, aux_st0);
-            if (b >= 1) consume(b - 1);
-            __syncthreads();
-        }
-        if (npieces > 1) {                               // a piece of the walk: fp32 partial sums, added by the reduction
-            float *pk = piece_partial(partial, mslot, piece, Hkv, kvh, D) + (kg * 32 + j) * D + dt0 * 32, *pv_ = pk + 128 * D;
-#pragma unroll
-            for (int dt = 0; dt < DTC; ++dt) {
-                store_c_tile_f32(pk + dt * 32, dkacc[dt], h);
-                store_c_tile_f32(pv_ + dt * 32, dvacc[dt], h);
-            }
-        } else if (key_ok) {
-            bf16_t *pk = dk + krow * D + dt0 * 32, *pv_ = dv + krow * D + dt0 * 32;
-#pragma unroll
-            for (int dt = 0; dt < DTC; ++dt) {
-                store_c_tile(pk + dt * 32, dkacc[dt], scale, h);
-                store_c_tile(pv_ + dt * 32, dvacc[dt], 1.f, h);
-            }
-        }
-        return;
-    }
-
-    // ================= producers: S and dP of a block, then its softmax =================
-    bf16x8 kB[KS], vB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        kB[ks] = load_bf16x8(k + krow * D + 16 * ks + 8 * h);
-        vB[ks] = load_bf16x8(v + krow * D + 16 * ks + 8 * h);
-    }
-    // P and dS go to the consumers in bf16.  dV[s] = sum over (query, head) of P dO piles the rounding of P (2^-9
-    // relative) onto one key row; where probabilities are large (few keys per query: short rows, small top-k) and many
-    // rows meet in one key, that noise reaches several 1e-2.  A block whose largest P is at least DKV_SPLIT_MIN
-    // therefore also carries P - bf16(P), and the consumers add dO^T times it; blocks of small probabilities (the bulk of
-    // any long row) skip both the arithmetic and the extra MFMAs.
-    constexpr float DKV_SPLIT_MIN = 0.015625f;
-    auto store_pd = [&](int b, const float *pv, const float *dsv) {  // -> ring slot b % 2, MFMA B layout
-        unsigned char *pd = pd_ring + (b & 1) * PD_SLOT + kg * PD_GROUP + lane * 16;
-        const bf16x8 p0 = pack8(pv), p1 = pack8(pv + 8);
-        *reinterpret_cast<bf16x8 *>(pd) = p0;
-        *reinterpret_cast<bf16x8 *>(pd + 1024) = p1;
-        *reinterpret_cast<bf16x8 *>(pd + 2048) = pack8(dsv);
-        *reinterpret_cast<bf16x8 *>(pd + 3072) = pack8(dsv + 8);
-        float pm = pv[0];
-#pragma unroll
-        for (int vi = 1; vi < 16; ++vi) pm = fmaxf(pm, pv[vi]);
-        const bool big = __builtin_amdgcn_ballot_w64(pm >= DKV_SPLIT_MIN) != 0ull;   // wave-uniform
-        if (big) {
-            const u32x4 w0 = __builtin_bit_cast(u32x4, p0), w1 = __builtin_bit_cast(u32x4, p1);
-            float lo[16];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                lo[2 * e] = pv[2 * e] - __uint_as_float(w0[e] << 16);
-                lo[2 * e + 1] = pv[2 * e + 1] - __uint_as_float(w0[e] & 0xffff0000u);
-                lo[8 + 2 * e] = pv[8 + 2 * e] - __uint_as_float(w1[e] << 16);
-                lo[9 + 2 * e] = pv[9 + 2 * e] - __uint_as_float(w1[e] & 0xffff0000u);
-            }
-            *reinterpret_cast<bf16x8 *>(pd + 4096) = pack8(lo);
-            *reinterpret_cast<bf16x8 *>(pd + 5120) = pack8(lo + 8);
-        }
-        if (lane == 0) split_flag[(b & 1) * 4 + kg] = big ? 1u : 0u;
-    };
-    __syncthreads();                                     // the first step staged
-    // GEMMs, then softmax, block by block; the row statistics are taken from LDS group by group (the K and V rows
-    // leave no registers to hold them across the GEMMs)
-    for (int b = 0; b <= nblocks; ++b) {
-        if (b < nblocks) {
-            const unsigned char *qt = qd_ring + qslot(b) * QD_SLOT, *dot = qt + TILE_B;
-            f32x16 sacc = zero16(), pacc = zero16();
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                sacc = mfma32(lo.rowop(qt, ks), kB[ks], sacc);
-                pacc = mfma32(lo.rowop(dot, ks), vB[ks], pacc);
-            }
-            sched_reads_ahead<2 * KS, 4, 1>();
-            const float *lse_s = reinterpret_cast<const float *>(aux_ring + qslot(b) * AUX_SLOT);
-            const float *dlt_s = lse_s + 32;
-            const uint32_t *mask_s = reinterpret_cast<const uint32_t *>(dlt_s + 32) + kg * 32;
-            const int qcb = q0 + (nblocks - 1 - b) * QB;
-            const bool diag = causal && qcb < kc + 32;
-            float pv[16], dsv[16];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const f32x4 l4g = *reinterpret_cast<const f32x4 *>(&lse_s[8 * g4 + 4 * h]);
-                const f32x4 d4g = *reinterpret_cast<const f32x4 *>(&dlt_s[8 * g4 + 4 * h]);
-                uint32_t keep = 0u;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int vi = 4 * g4 + e, row = 8 * g4 + 4 * h + e;
-                    if (e == 0 || GSHIFT < 2) {          // rows of one query share the mask bit
-                        const int qi = row >> GSHIFT;
-                        uint32_t w = HAS_IDX ? mask_s[qi] : 0xffffffffu;
-                        if (diag) w &= causal_bits(qcb + qi - kc);
-                        keep = bit_mask(w, j);
-                    }
-                    const float p = fast_exp2(keep_or_neginf(fmaf(sacc[vi], scale_log2, -l4g[e]), keep));
-                    pv[vi] = p;
-                    dsv[vi] = p * (pacc[vi] - d4g[e]);
-                }
-            }
-            store_pd(b, pv, dsv);
-        }
-        __syncthreads();
-    }
-}
-template <int D>
-constexpr size_t dkvpc_lds_bytes() {   // three q/dO and row-data slots, two P/dS slots, the split flags
-    return 3 * ((size_t)2 * tile_bytes<D>() + (32 + 32 + 4 * 32) * 4) + 2 * (4 * 6 * 1024) + 2 * 4 * 4;
-}
-
-// ==================================================================================================
-// dK, dV for head_dim <= 128, "two chains" form.  The same key-stationary walk as dsa_tile_dkvpc_kernel
-// (a workgroup owns a 128-key tile of one segment and kv head and walks the later queries from the
-// segment end down, 32 (query, head) rows per step); the eight waves are split by GEMM chain, so that
-// neither P nor dS has to be handed over in full and every wave runs 16 MFMAs per step:
-//   waves 0-3 (P chain, one per 32-key group): S = Q K^T against the group's K rows in registers,
-//     started from -lse/scale so that P = exp2(S * scale*log2e) needs no subtraction, the selection bit
-//     applied before the exponential; dV^T += dO^T P with P going from the C layout of the first GEMM
-//     straight into the B operand of the second.  P also goes to LDS in bf16 for the other chain.
-//     Step s: S of block s, then the MFMAs of dV for block s-1 with the softmax of block s behind them.
-//   waves 4-7 (dS chain): dP = dO V^T against the group's V rows, started from -delta; dS = P (dP - delta)
-//     with the bf16 P read back from LDS; dK^T += Q^T dS, dS staying in registers.  Step s: block s-1.
-//     These waves also stage the q / dO blocks and the row data (two steps ahead in LDS, two more in
-//     registers).
-// One barrier per step; block s sits in ring slot s % 4 from step s-2 (staged) to step s+1 (last read),
-// P of block s in slot s % 2 of its ring from step s to step s+1.
-// Measured on this kernel's instruction mix (no memory traffic): one wave of each chain on a SIMD needs
-// about 1270 clocks per step against 1090 for the 32 MFMAs alone; the kernel runs at about 2000.
-// ==================================================================================================
-template <int D, bool HAS_IDX, int GSHIFT>
-__global__ __launch_bounds__(512, 1) void dsa_tile_dkv2_kernel(
-    const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
-    const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
-    const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, int causal, int d_real, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
-    bf16_t *__restrict__ dv) {
-    static_assert(D <= 128, "head_dim 256 runs dsa_tile_dkvpc_kernel");
-    constexpr int KS = D / 16, DT = (D + 31) / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NCHUNK = 32 * CPR, STG = 256, CPT = (NCHUNK + STG - 1) / STG;
-    constexpr bool ALL_STAGE = NCHUNK % STG == 0;        // (head_dim 96: the last chunk of half of the staging threads is spare)
-    constexpr int Gp = 1 << GSHIFT, QB = 32 >> GSHIFT;
-    constexpr int QD_SLOT = 2 * TILE_B;                  // q block | dO block
-    constexpr int P_GROUP = 2 * 1024, P_SLOT = 4 * P_GROUP;   // per key group: P rows 0-15 | 16-31, 64 lanes x 16 B each
-    constexpr int AUX_SLOT = (32 + 32 + 4 * 32) * 4;     // lse | delta | selection words [key group][query]
-    static_assert(CPT >= 1 && NCHUNK % 64 == 0, "whole waves stage a chunk or do not");
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_lds[];
-    unsigned char *const qd_ring = dyn_lds;                          // 4 slots
-    unsigned char *const p_ring = dyn_lds + 4 * QD_SLOT;             // 2 slots
-    unsigned char *const aux_ring = p_ring + 2 * P_SLOT;             // 4 slots
-
-    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kg = wv & 3;
-    const int G = Hq / Hkv;
-    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
-    const int kvh = blockIdx.x % Hkv;
-    int s0, L, blk, piece, mslot, pb;
-    if (!locate_key_tile(order, cu, N, blockIdx.x / Hkv, s0, L, blk, piece, mslot, pb)) return;
-    if (HAS_IDX) L = min(L, ldw * 32);
-    if (blk * 128 >= L) return;                         // (whole workgroup, before its first barrier)
-    const int c0 = blk * 128, kc = c0 + kg * 32;
-    const int mykey = kc + j;
-    const bool key_ok = mykey < L;
-    const int64_t krow = (int64_t)(s0 + min(mykey, L - 1)) * Hkv + kvh;
-    const float scale_log2 = scale * LOG2E_F, inv_scale = 1.f / scale;
-    // the walk: queries q0 .. Lq-1 in nblocks steps (step s handles block nblocks-1-s) - all queries that can see
-    // this key tile, or one piece of them
-    int q0_ = causal ? c0 : 0, Lq_ = L, nblocks_ = (L - q0_ + QB - 1) / QB;
-    const int npieces = walk_piece((causal && partial && mslot >= 0) ? pb : 0, piece, QB, q0_, Lq_, nblocks_);
-    if (npieces == 0) return;
-    const int q0 = q0_, Lq = Lq_, nblocks = nblocks_;
-
-    // an accumulator in C layout that starts from a per-row value (lane (key, h) holds rows 8 g4 + 4 h + e)
-    auto rows_init = [&](const float *rowv) __attribute__((always_inline)) {
-        f32x16 c;
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-            const f32x4 r = *reinterpret_cast<const f32x4 *>(&rowv[8 * g4 + 4 * h]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) c[4 * g4 + e] = r[e];
-        }
-        return c;
-    };
-    // Staging: 16-byte chunks of the q and dO blocks, CPT of each per thread, and one word of row data per thread of
-    // the first 64 + 4 QB (lse, delta, selection words).  Step b reads block nblocks-1-b; the walk starts at the
-    // segment end, so only block 0 (rows past the end) and the steps past the last block need their rows zeroed.
-    const int ctid = tid & 255;                          // used by the dS chain's waves
-    const int last = nblocks - 1;
-    const int64_t blk_bytes = (int64_t)QB * Hq * dr * 2;
-    const unsigned char *qp[CPT], *dp[CPT];
-    int64_t dlast[CPT];
-    int lds_off[CPT];
-    bool row_dead_last[CPT], head_ok[CPT], staged[CPT];
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-        staged[i] = ALL_STAGE || i * STG + ctid < NCHUNK; // a spare chunk loads the tile's last chunk again and stores nothing
-        const int c = min(i * STG + ctid, NCHUNK - 1), srow = c / CPR, sch = c % CPR;
-        const int src_ch = HAS_IDX ? sch : min(sch, chunks - 1);     // (spare columns: any finite values; k and v are zero there)
-        const int hd = min(srow & (Gp - 1), G - 1);
-        const int qr = srow >> GSHIFT;
-        const int over = max(q0 + last * QB + qr - (Lq - 1), 0);     // rows past the end in the last block
-        const int64_t off = ((int64_t)(s0 + q0 + last * QB + qr - over) * Hq + kvh * G + hd) * dr + src_ch * 8;
-        qp[i] = reinterpret_cast<const unsigned char *>(q + off);
-        dp[i] = reinterpret_cast<const unsigned char *>(dout + off);
-        dlast[i] = -(int64_t)over * Hq * dr * 2;
-        row_dead_last[i] = over > 0;
-        head_ok[i] = (srow & (Gp - 1)) < G;
-        lds_off[i] = tile_off<D>(srow, sch);
-    }
-    // row data: every thread loads one word and stores one word, threads without a share into a spare LDS word.
-    // lse and delta go in as -lse/scale and -delta (the chains start their accumulators from them), selection words
-    // as they are (zero for key groups past the bitmap row)
-    const uint32_t *aux_base = reinterpret_cast<const uint32_t *>(lse);
-    int aux_q = 0, aux_stride = 0, aux_lds = 4 * AUX_SLOT;          // spare word behind the four slots
-    float aux_mul = 0.f;
-    uint32_t aux_and = 0u;
-    bool aux_is_word = false, aux_pad = false;
-    uint32_t aux_dead_value = 0u;                    // what a row that is not live stores: word 0, delta 0, -lse/scale -1e30
-    if (ctid < 64) {                                 // 0..31: lse of row ctid, 32..63: delta of row ctid-32
-        const int row = ctid & 31;
-        const int hd = min(row & (Gp - 1), G - 1);
-        aux_pad = (row & (Gp - 1)) >= G;
-        aux_dead_value = ctid < 32 ? __float_as_uint(-1e30f) : 0u;
-        aux_q = row >> GSHIFT;
-        aux_stride = 1;
-        aux_base = reinterpret_cast<const uint32_t *>((ctid < 32 ? lse : delta) + (int64_t)(kvh * G + hd) * T + s0);
-        aux_mul = ctid < 32 ? -inv_scale : -1.f;
-        aux_lds = ctid * 4;
-    } else if (HAS_IDX && ctid < 64 + 4 * QB) {      // selection word of (key group w, query qi)
-        const int w = (ctid - 64) / QB;
-        aux_q = (ctid - 64) % QB;
-        aux_stride = ldw;
-        const bool ok = (c0 >> 5) + w < ldw;
-        aux_base = bitmap + (int64_t)s0 * ldw + (ok ? (c0 >> 5) + w : 0);
-        aux_and = ok ? 0xffffffffu : 0u;
-        aux_is_word = true;
-        aux_lds = (64 + w * 32 + aux_q) * 4;
-    }
-    const int64_t aux_blk_bytes = (int64_t)aux_stride * QB * 4;
-    const int aux_over = max(q0 + last * QB + aux_q - (Lq - 1), 0);
-    const int64_t aux_dlast = -(int64_t)aux_stride * aux_over * 4;
-    const unsigned char *ap =
-        reinterpret_cast<const unsigned char *>(aux_base + (int64_t)aux_stride * (q0 + last * QB + aux_q - aux_over));
-    u32x4 qst0[CPT], dost0[CPT], qst1[CPT], dost1[CPT];     // two register sets: a load has two steps to land
-    uint32_t aux_st0, aux_st1;
-    auto aux_value = [&](uint32_t x) __attribute__((always_inline)) {
-        return aux_is_word ? (x & aux_and) : __float_as_uint(__uint_as_float(x) * aux_mul);
-    };
-    // general forms (first and last steps): gload is called with b = 0, 1, 2, ... in turn; past step `last` it reads
-    // the first block again and lstore zeroes what it stores
-    auto gload = [&](int b, u32x4 (&qst)[CPT], u32x4 (&dost)[CPT], uint32_t &aux_st) __attribute__((always_inline)) {
-        if (b >= 1 && b <= last) {
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) { qp[i] -= blk_bytes; dp[i] -= blk_bytes; }
-            ap -= aux_blk_bytes;
-            if (b == 1) {                            // leaving the last block: undo its row clamp
-#pragma unroll
-                for (int i = 0; i < CPT; ++i) { qp[i] -= dlast[i]; dp[i] -= dlast[i]; }
-                ap -= aux_dlast;
-            }
-        }
-        aux_st = *reinterpret_cast<const uint32_t *>(ap);   // first: its consumer then never waits for younger loads
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            qst[i] = *reinterpret_cast<const u32x4 *>(qp[i]);
-            dost[i] = *reinterpret_cast<const u32x4 *>(dp[i]);
-        }
-    };
-    auto lstore = [&](int b, const u32x4 (&qst)[CPT], const u32x4 (&dost)[CPT], uint32_t aux_st) __attribute__((always_inline)) {
-        unsigned char *slot = qd_ring + (b & 3) * QD_SLOT;
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const bool live = head_ok[i] && !(b > last || (b == 0 && row_dead_last[i]));
-            const u32x4 z4 = {0u, 0u, 0u, 0u};
-            if (ALL_STAGE || staged[i]) {
-                *reinterpret_cast<u32x4 *>(slot + lds_off[i]) = live ? qst[i] : z4;
-                *reinterpret_cast<u32x4 *>(slot + TILE_B + lds_off[i]) = live ? dost[i] : z4;
-            }
-        }
-        // a row that is not live (past the segment, past the walk, a padded head) has q = dO = 0 but would read a live
-        // row's lse: with lse far below zero its P = exp(0 - lse) overflows and 0 * inf reaches dK and dV.  Its selection
-        // word is cleared, and its S starts so low that P vanishes also where no selection masks it.
-        const bool dead = b > last || (b == 0 && aux_over > 0) || aux_pad;
-        *reinterpret_cast<uint32_t *>(aux_ring + (aux_lds < 4 * AUX_SLOT ? (b & 3) * AUX_SLOT : 0) + aux_lds) =
-            dead ? aux_dead_value : aux_value(aux_st);
-    };
-    // steady forms (blocks 2 .. last of a group whose heads fill the padded group): no branch, no select
-    auto gload_steady = [&](u32x4 (&qst)[CPT], u32x4 (&dost)[CPT], uint32_t &aux_st) __attribute__((always_inline)) {
-        ap -= aux_blk_bytes;
-        aux_st = *reinterpret_cast<const uint32_t *>(ap);
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            qp[i] -= blk_bytes;
-            dp[i] -= blk_bytes;
-            qst[i] = *reinterpret_cast<const u32x4 *>(qp[i]);
-            dost[i] = *reinterpret_cast<const u32x4 *>(dp[i]);
-        }
-    };
-    auto lstore_steady = [&](int b, const u32x4 (&qst)[CPT], const u32x4 (&dost)[CPT], uint32_t aux_st) __attribute__((always_inline)) {
-        unsigned char *slot = qd_ring + (b & 3) * QD_SLOT;
-#pragma unroll
-        for (int i = 0; i < CPT; ++i)
-            if (ALL_STAGE || staged[i]) {
-                *reinterpret_cast<u32x4 *>(slot + lds_off[i]) = qst[i];
-                *reinterpret_cast<u32x4 *>(slot + TILE_B + lds_off[i]) = dost[i];
-            }
-        *reinterpret_cast<uint32_t *>(aux_ring + (aux_lds < 4 * AUX_SLOT ? (b & 3) * AUX_SLOT : 0) + aux_lds) = aux_value(aux_st);
-    };
-    if (wv >= 4) {
-        // ================= dS chain: staging, then dP, dS, dK of the block the P chain finished a step earlier =================
-        gload(0, qst0, dost0, aux_st0);
-        gload(1, qst1, dost1, aux_st1);
-        bf16x8 vB[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) vB[ks] = HAS_IDX || 2 * ks + h < chunks ? load_bf16x8(v + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
-        lstore(0, qst0, dost0, aux_st0);
-        lstore(1, qst1, dost1, aux_st1);
-        gload(2, qst0, dost0, aux_st0);
-        gload(3, qst1, dost1, aux_st1);
-        __syncthreads();                                 // steps 0 and 1 staged
-
-        f32x16 dkacc[DT];
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) dkacc[dt] = zero16();
-        // dS of elements 8 half .. 8 half + 7 (C layout) as an MFMA B operand: the other chain's bf16 P times this
-        // chain's dP - delta
-        auto ds_half = [&](const u32x4 &w, const f32x16 &pacc, int half) __attribute__((always_inline)) {
-            float ds[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                ds[2 * e] = __uint_as_float(w[e] << 16) * pacc[8 * half + 2 * e];
-                ds[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u) * pacc[8 * half + 2 * e + 1];
-            }
-            return pack8(ds);
-        };
-        // block b: dP = dO V^T starting from -delta, dS, dK^T += Q^T dS.  Operand reads run three to four MFMAs ahead
-        // (every MFMA step ends in an empty asm statement that the next operand passes through, which fixes the
-        // order); the second half of dS is formed behind the first MFMAs of dK.
-        auto block = [&](int b) __attribute__((always_inline)) {
-            const unsigned char *qt = qd_ring + (b & 3) * QD_SLOT, *dot = qt + TILE_B;
-            const unsigned char *pd = p_ring + (b & 1) * P_SLOT + kg * P_GROUP + lane * 16;
-            f32x16 pacc = rows_init(reinterpret_cast<const float *>(aux_ring + (b & 3) * AUX_SLOT) + 32);
-            bf16x8 a[4], t[4];
-#pragma unroll
-            for (int i = 0; i < 4 && i < KS; ++i) a[i] = lo.rowop(dot, i);
-            const u32x4 w0 = *reinterpret_cast<const u32x4 *>(pd), w1 = *reinterpret_cast<const u32x4 *>(pd + 1024);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                pacc = mfma32(a[ks & 3], vB[ks], pacc);
-                if (ks + 4 < KS) a[ks & 3] = lo.rowop(dot, ks + 4);
-                if (ks + 3 >= KS) t[ks + 3 - KS] = lo.trop(qt, (ks + 3 - KS) / DT, (ks + 3 - KS) % DT);
-                if (ks + 1 < KS) asm volatile("" : "+v"(a[(ks + 1) & 3]) : : "memory");
-                else asm volatile("" : "+v"(t[0]) : : "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            const bf16x8 dB0 = ds_half(w0, pacc, 0);
-            uint32_t dw[4];
-#pragma unroll
-            for (int m = 0; m < 2 * DT; ++m) {
-                if (m < DT) dkacc[m] = mfma32(t[m & 3], dB0, dkacc[m]);
-                else {
-                    const u32x4 d1 = {dw[0], dw[1], dw[2], dw[3]};
-                    dkacc[m - DT] = mfma32(t[m & 3], __builtin_bit_cast(bf16x8, d1), dkacc[m - DT]);
-                }
-                if (m + 3 < 2 * DT) t[(m + 3) & 3] = lo.trop(qt, (m + 3) / DT, (m + 3) % DT);
-                if (m < DT) {                            // the four pairs of the second half of dS, spread behind these MFMAs
-#pragma unroll
-                    for (int e = 4 * m / DT; e < 4 * (m + 1) / DT; ++e) {
-                        dw[e] = pack2bf(__uint_as_float(w1[e] << 16) * pacc[8 + 2 * e], __uint_as_float(w1[e] & 0xffff0000u) * pacc[9 + 2 * e]);
-                        asm volatile("" : "+v"(dw[e]));
-                    }
-                }
-                if (m + 1 < 2 * DT) asm volatile("" : "+v"(t[(m + 1) & 3]) : : "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-#define DKV2_DS_STEP(S, QS, DS_, AS)                                                                \
-    {                                                                                              \
-        lstore((S) + 2, QS, DS_, AS); /* its slot was last read (as step S-2) before the previous barrier */ \
-        gload((S) + 4, QS, DS_, AS);                                                               \
-        if ((S) >= 1) block((S) - 1);                                                              \
-        __syncthreads();                                                                             \
-    }
-#define DKV2_DS_STEADY(S, QS, DS_, AS)                                                              \
-    {                                                                                              \
-        lstore_steady((S) + 2, QS, DS_, AS);                                                       \
-        gload_steady(QS, DS_, AS);                                                                 \
-        block((S) - 1);                                                                            \
-        __syncthreads();                                                                             \
-    }
-        DKV2_DS_STEP(0, qst0, dost0, aux_st0)
-        int s = 1;
-        if (s <= nblocks) {
-            DKV2_DS_STEP(1, qst1, dost1, aux_st1)
-            s = 2;
-        }
-        if (G == Gp)                                     // steps whose staged block is 2 .. last and whose loaded block is 2 .. last
-            for (; s + 5 <= last; s += 2) {
-                DKV2_DS_STEADY(s, qst0, dost0, aux_st0)
-                DKV2_DS_STEADY(s + 1, qst1, dost1, aux_st1)
-            }
-        for (; s + 1 <= nblocks; s += 2) {
-            DKV2_DS_STEP(s, qst0, dost0, aux_st0)
-            DKV2_DS_STEP(s + 1, qst1, dost1, aux_st1)
-        }
-        if (s <= nblocks) DKV2_DS_STEP(s, qst0, dost0, aux_st0)
-#undef DKV2_DS_STEP
-#undef DKV2_DS_STEADY
-        if (npieces > 1) {                               // a piece of the walk: fp32 partial sums, added by the reduction
-            float *pk = piece_partial(partial, mslot, piece, Hkv, kvh, 32 * DT) + (kg * 32 + j) * 32 * DT;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) store_c_tile_f32(pk + dt * 32, dkacc[dt], h);
-        } else if (key_ok) {
-            bf16_t *pk = dk + krow * dr;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) store_c_tile(pk + dt * 32, dkacc[dt], scale, h, chunks - 4 * dt);
-        }
-        return;
-    }
-
-    // ================= P chain: S and softmax of block s, dV of block s-1 =================
-    bf16x8 kB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kB[ks] = HAS_IDX || 2 * ks + h < chunks ? load_bf16x8(k + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
-    uint32_t mw[16];
-    auto read_aux = [&](int b) __attribute__((always_inline)) {                         // selection words of step b
-        const uint32_t *mask_s = reinterpret_cast<const uint32_t *>(aux_ring + (b & 3) * AUX_SLOT) + 64 + kg * 32;
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (HAS_IDX && (e == 0 || GSHIFT < 2)) mw[4 * g4 + e] = mask_s[(8 * g4 + 4 * h + e) >> GSHIFT];
-    };
-    f32x16 dvacc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) dvacc[dt] = zero16();
-    // P of element vi (C layout) of step b from its S accumulator (which started from -lse/scale); pm collects the
-    // block's largest P
-    auto element = [&](auto may_diag, int b, int vi, const f32x16 &sacc, float sl2, uint32_t &keep, float &pm) __attribute__((always_inline)) {
-        const int g4 = vi >> 2, e = vi & 3, row = 8 * g4 + 4 * h + e;
-        if (e == 0 || GSHIFT < 2) {                      // rows of one query share the mask bit
-            const int qcb = q0 + (nblocks - 1 - b) * QB, qi = row >> GSHIFT;
-            uint32_t w = HAS_IDX ? mw[vi] : 0xffffffffu;
-            if (decltype(may_diag)::value && causal && qcb < kc + 32) w &= causal_bits(qcb + qi - kc);
-            keep = bit_mask(w, j);
-        }
-        const float p = fast_exp2(keep_or_neginf(sacc[vi] * sl2, keep));
-        pm = fmaxf(pm, p);
-        return p;
-    };
-    auto store_p = [&](int b, int half, bf16x8 p) __attribute__((always_inline)) {
-        *reinterpret_cast<bf16x8 *>(p_ring + (b & 1) * P_SLOT + kg * P_GROUP + half * 1024 + lane * 16) = p;
-    };
-    // P goes on in bf16.  dV[s] = sum over (query, head) of P dO piles the rounding of P (2^-9 relative) onto one key
-    // row; where probabilities are large (few keys per query) and many rows meet in one key, that noise reaches
-    // several 1e-2.  A block whose largest P is at least DKV_SPLIT_MIN therefore also adds dO^T (P - bf16(P)).
-    constexpr float DKV_SPLIT_MIN = 0.015625f;
-    auto remainder = [&](auto may_diag, int b, const f32x16 &sc, float pm, bf16x8 p0, bf16x8 p1) __attribute__((always_inline)) {
-        if (__builtin_amdgcn_ballot_w64(pm >= DKV_SPLIT_MIN) != 0ull) {   // wave-uniform, rare: P is formed again
-            const u32x4 w0 = __builtin_bit_cast(u32x4, p0), w1 = __builtin_bit_cast(u32x4, p1);
-            float pv[16], lo_[16], pm2 = 0.f;
-            uint32_t keep = 0u;
-#pragma unroll
-            for (int vi = 0; vi < 16; ++vi) pv[vi] = element(may_diag, b, vi, sc, scale_log2, keep, pm2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                lo_[2 * e] = pv[2 * e] - __uint_as_float(w0[e] << 16);
-                lo_[2 * e + 1] = pv[2 * e + 1] - __uint_as_float(w0[e] & 0xffff0000u);
-                lo_[8 + 2 * e] = pv[8 + 2 * e] - __uint_as_float(w1[e] << 16);
-                lo_[9 + 2 * e] = pv[9 + 2 * e] - __uint_as_float(w1[e] & 0xffff0000u);
-            }
-            const unsigned char *dot = qd_ring + (b & 3) * QD_SLOT + TILE_B;
-            const bf16x8 l0 = pack8(lo_), l1 = pack8(lo_ + 8);
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                dvacc[dt] = mfma32(lo.trop(dot, 0, dt), l0, dvacc[dt]);
-                dvacc[dt] = mfma32(lo.trop(dot, 1, dt), l1, dvacc[dt]);
-            }
-        }
-    };
-    // Step s: S of block s (KS MFMAs), then the 2 DT MFMAs of dV^T += dO^T P of block s-1 with the softmax of
-    // 16 / (2 DT) elements of block s behind each of them (operand reads three MFMAs ahead; every MFMA step ends in
-    // empty asm statements that its results and the next MFMA's operand pass through, which fixes the order).
-    bf16x8 pq0 = zero_bf16x8(), pq1 = zero_bf16x8();     // P of the block before, as B operands (rows 0-15 | 16-31)
-    auto step = [&](auto may_diag, auto has_cur, auto has_prev, int s) __attribute__((always_inline)) {
-        constexpr bool CUR = decltype(has_cur)::value, PREV = decltype(has_prev)::value;
-        constexpr int NM = 2 * DT;                       // elements 16 m / NM .. 16 (m + 1) / NM behind MFMA m
-        const unsigned char *qt = qd_ring + (s & 3) * QD_SLOT, *dprev = qd_ring + ((s - 1) & 3) * QD_SLOT + TILE_B;
-        f32x16 sacc;
-        if (CUR) {
-            sacc = rows_init(reinterpret_cast<const float *>(aux_ring + (s & 3) * AUX_SLOT));
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) sacc = mfma32(lo.rowop(qt, ks), kB[ks], sacc);
-            sched_reads_ahead<KS, (KS >= 4 ? 4 : KS), 1, 4>();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        float pv[2], pm = 0.f, sl2 = scale_log2;
-        uint32_t keep = 0u, pw[8];
-        bf16x8 t[4];
-        if (PREV) {
-#pragma unroll
-            for (int i = 0; i < 3 && i < NM; ++i) t[i] = lo.trop(dprev, i / DT, i % DT);
-        }
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            if (PREV) {
-                dvacc[m % DT] = mfma32(t[m & 3], m < DT ? pq0 : pq1, dvacc[m % DT]);
-                if (m + 3 < NM) t[(m + 3) & 3] = lo.trop(dprev, (m + 3) / DT, (m + 3) % DT);
-            }
-            if (CUR) {
-#pragma unroll
-                for (int vi = 16 * m / NM; vi < 16 * (m + 1) / NM; ++vi) {   // P is packed pair by pair as it is formed
-                    pv[vi & 1] = element(may_diag, s, vi, sacc, sl2, keep, pm);
-                    if (vi & 1) {
-                        pw[vi >> 1] = pack2bf(pv[0], pv[1]);
-                        asm volatile("" : "+v"(pw[vi >> 1]));
-                    } else {
-                        asm volatile("" : "+v"(pv[0]));
-                    }
-                }
-            }
-            if (PREV && m + 1 < NM) asm volatile("" : "+v"(sl2), "+v"(pm), "+v"(t[(m + 1) & 3]) : : "memory");
-            else asm volatile("" : "+v"(sl2), "+v"(pm) : : "memory");
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (CUR) {
-            const u32x4 w0 = {pw[0], pw[1], pw[2], pw[3]}, w1 = {pw[4], pw[5], pw[6], pw[7]};
-            pq0 = __builtin_bit_cast(bf16x8, w0);
-            pq1 = __builtin_bit_cast(bf16x8, w1);
-            store_p(s, 0, pq0);
-            store_p(s, 1, pq1);
-            remainder(may_diag, s, sacc, pm, pq0, pq1);
-            if (s + 1 < nblocks) read_aux(s + 1);
-        }
-    };
-    const std::true_type yes;
-    const std::false_type no;
-    __syncthreads();                                     // steps 0 and 1 staged
-    read_aux(0);
-    // The blocks that can touch the causal diagonal come last; the steady loop before them has no mask
-    // arithmetic besides the selection bits.
-    const int nb_diag = causal ? max(kc + 32 - q0 + QB - 1, 0) / QB : 0;   // (none for a piece that starts past the diagonal)
-    const int steady = max(nblocks - nb_diag, 1);        // steps [1, steady) see blocks fully past the diagonal
-    step(yes, yes, no, 0);
-    __syncthreads();
-    int s = 1;
-    for (; s < steady; ++s) {
-        step(no, yes, yes, s);
-        __syncthreads();
-    }
-    for (; s < nblocks; ++s) {
-        step(yes, yes, yes, s);
-        __syncthreads();
-    }
-    step(yes, no, yes, nblocks);
-    __syncthreads();
-    if (npieces > 1) {
-        float *pv_ = piece_partial(partial, mslot, piece, Hkv, kvh, 32 * DT) + (128 + kg * 32 + j) * 32 * DT;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile_f32(pv_ + dt * 32, dvacc[dt], h);
-    } else if (key_ok) {
-        bf16_t *pv_ = dv + krow * dr;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(pv_ + dt * 32, dvacc[dt], 1.f, h, chunks - 4 * dt);
-    }
-}
-template <int D>
-constexpr size_t dkv2_lds_bytes() {   // q/dO ring, P ring, row-data ring and one spare word
-    return 4 * ((size_t)2 * tile_bytes<D>() + (32 + 32 + 4 * 32) * 4) + 2 * (4 * 2 * 1024) + 16;
+    const float mul = m ? 1.f : scale;
+    const u32x4 w = {pack2bf(a0[0] * mul, a0[1] * mul), pack2bf(a0[2] * mul, a0[3] * mul), pack2bf(a1[0] * mul, a1[1] * mul), pack2bf(a1[2] * mul, a1[3] * mul)};
+    *reinterpret_cast<u32x4 *>((m ? dv : dk) + ((int64_t)(s0 + c0 + key) * Hkv + kvh) * D + col) = w;
 }
 
 // ==================================================================================================
 // launchers: instantiate per head_dim, mask kind and (power-of-two padded) group size
 // ==================================================================================================
-
-template <int D, bool HAS_IDX, int GS>
-static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
-                         const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                         int T, int Hq, int Hkv, int d_real, float scale, int causal, const int32_t *order, float *partial, void *dk,
-                         void *dv) {
-    // LDS above 64 KiB has to be requested per kernel and device; asked for on every launch (a host-side table
-    // lookup), so that neither a second device nor a second thread can meet a kernel that was never configured
-    if constexpr (D <= 128) {
-        const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_tile_dkv2_kernel<D, HAS_IDX, GS>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkv2_lds_bytes<D>());
-        if (e2 != hipSuccess) return e2;
-        hipLaunchKernelGGL((dsa_tile_dkv2_kernel<D, HAS_IDX, GS>), grid, dim3(512), dkv2_lds_bytes<D>(), stream,
-                           (const bf16_t *)dout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap,
-                           ldw, cu, N, T, Hq, Hkv, scale, causal, d_real, order, partial, (bf16_t *)dk, (bf16_t *)dv);
-        return hipSuccess;
-    } else {
-    const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_tile_dkvpc_kernel<D, HAS_IDX, GS>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)dkvpc_lds_bytes<D>());
-    if (ea != hipSuccess) return ea;
-    // two workgroups per key tile and kv head, one per half of head_dim (a consumer wave holds 128 accumulator registers)
-    hipLaunchKernelGGL((dsa_tile_dkvpc_kernel<D, HAS_IDX, GS>), dim3(grid.x * 2), dim3(512), dkvpc_lds_bytes<D>(), stream,
-                       (const bf16_t *)dout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap,
-                       ldw, cu, N, T, Hq, Hkv, scale, causal, order, partial, (bf16_t *)dk, (bf16_t *)dv);
-    return hipSuccess;
-    }
-}
 
 #define GS_SWITCH(FN, DD, HI, ...)                                    \
     switch (gs) {                                                     \
@@ -1631,22 +743,6 @@ static hipError_t launch_dkv_i(dim3 grid, hipStream_t stream, const void *dout, 
         case 128: if (bitmap) { GS_SWITCH(FN, 128, true, __VA_ARGS__) } else { GS_SWITCH(FN, 128, false, __VA_ARGS__) } break; \
         case 256: if (bitmap) { GS_SWITCH(FN, 256, true, __VA_ARGS__) } else { GS_SWITCH(FN, 256, false, __VA_ARGS__) } break; \
         default: return hipErrorInvalidValue;                                             \
-    }                                                                                     \
-    if (launch_status != hipSuccess) return launch_status;
-
-// the same for the kernel that takes rows of d_real elements
-#define TILE_SWITCH_DENSE(FN, ...)                                                        \
-    hipError_t launch_status = hipErrorInvalidValue;                                      \
-    if (bitmap) switch (d_real) {                                                         \
-        case 64: GS_SWITCH(FN, 64, true, __VA_ARGS__) break;                              \
-        case 128: GS_SWITCH(FN, 128, true, __VA_ARGS__) break;                            \
-        case 256: GS_SWITCH(FN, 256, true, __VA_ARGS__) break;                            \
-    } else switch (dense_kernel_dim(d_real)) {                                            \
-        case 64: GS_SWITCH(FN, 64, false, __VA_ARGS__) break;                             \
-        case 80: GS_SWITCH(FN, 80, false, __VA_ARGS__) break;                             \
-        case 96: GS_SWITCH(FN, 96, false, __VA_ARGS__) break;                             \
-        case 128: GS_SWITCH(FN, 128, false, __VA_ARGS__) break;                           \
-        case 256: GS_SWITCH(FN, 256, false, __VA_ARGS__) break;                           \
     }                                                                                     \
     if (launch_status != hipSuccess) return launch_status;
 
@@ -1753,13 +849,14 @@ static DkvPlan dkv_plan(int T, int N, int Hq, int Hkv, int d_real, bool has_idx,
     DkvPlan p;
     p.tiles_ub = T / 128 + N;                            // 128-key tiles of all segments, at most
     p.pitch = has_idx ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;             // row of a partial sum
-    const int wg_per_tile = Hkv * (d_real > 128 ? 2 : 1);
+    const int wg_per_tile = Hkv, kg = dkv_key_groups(d_real, T, N, Hkv);
     const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * p.pitch * sizeof(float))) : 0;
-    p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= 4 * 256;
+    p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= dkv_pieces_max_wg(d_real);
     p.listed = order && (N > 1 || p.pieces);             // (one segment: its tiles are in order already)
     const int cap = order_entries_cap(T), item_cap = p.pieces ? std::min(cap, p.tiles_ub + (1024 + wg_per_tile - 1) / wg_per_tile) : cap;
-    p.o = TileOrder{cap, p.pieces ? 2 : (!causal || (p.tiles_ub + 1) * Hkv > 4 * 256 ? 1 : 0), 32 >> group_shift(Hq, Hkv), wg_per_tile, item_cap,
-                    (int)(slot_pairs / Hkv < (1 << 20) ? slot_pairs / Hkv : (1 << 20))};       // (sums stay below 2^21)
+    p.o = TileOrder{cap, p.pieces ? 2 : (causal ? 0 : 1), 32 >> group_shift(Hq, Hkv), wg_per_tile, item_cap,
+                    (int)(slot_pairs / Hkv < (1 << 20) ? slot_pairs / Hkv : (1 << 20)),       // (sums stay below 2^21)
+                    dkv_slots(kg), kg == 1 ? 8 : 6, kg == 1 ? 16 : 32};          // see tile_order
     return p;
 }
 // delta and, where the key-side launch of the same sizes will want it, its list
@@ -1772,6 +869,10 @@ extern "C" hipError_t dsa_launch_tile_order_delta(const void *dout, const void *
                        (const bf16_t *)dout, (const bf16_t *)out, T, Hq, d_real, delta);
     return hipGetLastError();
 }
+extern "C" hipError_t dsa_launch_dkv_tiles(unsigned grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
+                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
+                                           int T, int Hq, int Hkv, int d_real, float scale, int causal, const int32_t *order, float *partial,
+                                           void *dk, void *dv);
 // listed: dsa_launch_tile_order_delta has left the list in `order`
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
@@ -1784,9 +885,10 @@ extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const
     if (!p.listed) order = nullptr;
     else if (!listed) hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, p.o, order);
     if (!p.pieces) partial = nullptr;
-    TILE_SWITCH_DENSE(launch_dkv_i, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv)
+    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv);
+    if (e != hipSuccess) return e;
     if (p.pieces)
-        hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(p.tiles_ub, Hkv, DSA_PIECES_Z), dim3(256), 0, stream, order,
+        hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(p.tiles_ub, Hkv, p.pitch / 8), dim3(256), 0, stream, order,
                            p.o.cap, partial, cu, N, Hkv, d_real, p.pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
                            (bf16_t *)dk, (bf16_t *)dv);
     return hipGetLastError();

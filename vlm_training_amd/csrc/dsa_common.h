@@ -12,6 +12,17 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define DSA_WAVE 64
+// Groups of 32 keys that a wave of the key-side kernel takes: two up to head_dim 128 (each operand read feeds two MFMAs, two workgroups
+// per CU), except at head_dim 97 to 128 in launches of at most DKV_FEW_WG workgroups, which leave CUs idle: there a workgroup's own
+// pace counts, and four waves of one group each walk twice as fast.
+#define DKV_FEW_WG 192
+static inline int dkv_key_groups(int D, int T, int N, int Hkv) {
+    return D > 128 || (D > 96 && ((int64_t)T / 128 + N) * Hkv <= DKV_FEW_WG) ? 1 : 2;
+}
+// key-side workgroups that run at a time, and the launches whose walks may be cut into pieces: up to three rounds of them (a longer
+// launch of whole walks, longest first, ends level)
+static inline int dkv_slots(int key_groups) { return 256 * key_groups; }
+static inline int64_t dkv_pieces_max_wg(int D) { return D > 128 ? 3 * 256 : 3 * 512; }
 #define LOG2E_F 1.4426950408889634f
 #define LN2_F 0.6931471805599453f
 
@@ -135,6 +146,10 @@ __device__ __forceinline__ void buffer_load_lds16(buffer_rsrc rsrc, int voff, ui
 __device__ __forceinline__ void buffer_load_lds4(buffer_rsrc rsrc, int voff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds"
                  : : "v"(voff), "s"(rsrc), "s"(lds) : "memory", "m0");
+}
+// the same from each lane's own address
+__device__ __forceinline__ void global_load_lds4(const void *p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dword %0, off" : : "v"(p), "s"(lds) : "memory", "m0");
 }
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 // the barrier alone: LDS operations of this wave may still be in flight

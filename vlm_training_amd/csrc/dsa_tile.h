@@ -216,7 +216,7 @@ struct DirectTile {
     static constexpr int LOADS = 32 * ROW_B / 1024;                      // wave loads of a tile
     static constexpr int LOAD_ROWS = 1024 / ROW_B;                       // rows of one of them (1 at most for head_dim 512)
     static constexpr int SOURCES = D == 256 ? 2 : 1;                     // pieces after which x repeats (from an even piece on)
-    __device__ __forceinline__ static int load_lds(int p) {              // LDS offset of wave load p
+    __device__ __forceinline__ static constexpr int load_lds(int p) {              // LDS offset of wave load p
         return p * LOAD_ROWS / GROUP * GROUP_B + p * LOAD_ROWS % GROUP * ROW_B;
     }
     __device__ __forceinline__ static int xor_of(int row) { return D == 64 ? ((row >> 1) & 1) * 4 + ((row >> 2) & 1) * 2 : (row & 3) << 2; }
@@ -243,6 +243,60 @@ struct DirectTile {
     static constexpr int tr_q(int dt) { return dt & 3; }
     static constexpr int tr_imm(int dt, int v) { return (D == 64 ? 0 : (dt >> 2) * 256) + v * (8 / GROUP) * GROUP_B; }
 };
+
+// ---- walks of key tiles (dK, dV) ----
+#define DSA_ORDER_MAX_SEGS 4096
+// the tile (and the piece of its walk) of workgroup slot `slot`: from the order table when there is one, else
+// segment by segment
+__device__ __forceinline__ bool locate_key_tile(const int32_t *order, const int32_t *cu, int N, int slot, int &s0, int &L, int &blk,
+                                                int &piece, int &mslot, int &pb) {
+    piece = 0;
+    mslot = -1;
+    pb = 0;
+    if (order && N <= DSA_ORDER_MAX_SEGS) {
+        // (every lane reads the same words; the lane reads tell the compiler that the results are wave-uniform.  The table has room
+        // for every slot of a launch of that many segments: header and entry come in one round trip.)
+        const int4 hd = *reinterpret_cast<const int4 *>(order), e = *reinterpret_cast<const int4 *>(order + 4 + 4 * slot);
+        const int total = __builtin_amdgcn_readfirstlane(hd.x);
+        if (total >= 0) {
+            if (slot >= total) return false;
+            const int tp = __builtin_amdgcn_readfirstlane(e.z);
+            s0 = __builtin_amdgcn_readfirstlane(e.x);
+            L = __builtin_amdgcn_readfirstlane(e.y);
+            blk = tp & 8191;
+            piece = tp >> 13;
+            mslot = __builtin_amdgcn_readfirstlane(e.w);
+            pb = max(__builtin_amdgcn_readfirstlane(hd.y), 0);
+            return true;
+        }
+    }
+    return locate_block(cu, N, slot, 128, false, s0, L, blk);
+}
+// A walk of `nblocks` steps (block nblocks-1-b at step b, `QB` queries each, the queries q0 .. Lq-1) cut into equal pieces of
+// at most `pb` steps: narrows q0, Lq and nblocks to piece `piece` and returns the number of pieces (1: the whole walk,
+// 0: this piece is empty).  Block boundaries stay where they are, so a piece's blocks are the walk's own.
+__device__ __forceinline__ int walk_piece(int pb, int piece, int QB, int &q0, int &Lq, int &nblocks) {
+    if (pb <= 0 || nblocks <= pb) return piece == 0 ? 1 : 0;
+    const int np = (nblocks + pb - 1) / pb, len = (nblocks + np - 1) / np;
+    if (piece >= np) return 0;
+    const int b_lo = min(piece * len, nblocks), b_hi = min(b_lo + len, nblocks);
+    if (b_lo > 0) Lq = q0 + (nblocks - b_lo) * QB;
+    q0 += (nblocks - b_hi) * QB;
+    nblocks = b_hi - b_lo;
+    return np;
+}
+// fp32 partial dK / dV of piece `piece` of a tile in pieces: [slot][kv head][dK | dV][key group][d-tile][8 columns][lane][4], as
+// the accumulators lie in a wave, so that its stores are whole
+__device__ __forceinline__ float *piece_partial(float *partial, int mslot, int piece, int Hkv, int kvh, int DT) {
+    return partial + ((int64_t)(mslot + piece) * Hkv + kvh) * (2 * 128 * 32 * (int64_t)DT);
+}
+__device__ __forceinline__ void store_c_tile_f32(float *p, const f32x16 &acc, int lane) {
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+        const f32x4 w = {acc[4 * g4], acc[4 * g4 + 1], acc[4 * g4 + 2], acc[4 * g4 + 3]};
+        *reinterpret_cast<f32x4 *>(p + g4 * 256 + lane * 4) = w;
+    }
+}
 
 // ---- launches ----
 // log2 of the rows a query takes: its group's heads, padded to a power of two
