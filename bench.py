@@ -323,7 +323,7 @@ def main():
     unit = w.Hq * w.D * S                 # one flop-unit: a multiply-add pass over every selected (query, key, head, d)
     kern = {   # algorithmic flop per launch of the three attention kernels (selected pairs only)
         "attn_fwd": ("dsa_tile_fwd_kernel", 4 * unit),          # QK^T + PV
-        "bwd_dq": ("dsa_tile_dq128_kernel" if 96 < w.D <= 128 else "dsa_tile_dq_kernel", 6 * unit),   # QK^T + dO V^T + dS K
+        "bwd_dq": ("dsa_tile_dq_kernel", 6 * unit),   # QK^T + dO V^T + dS K
         # QK^T + dO V^T + P^T dO + dS^T Q (head_dim 256: the producer/consumer form, each half of head_dim forms S and dP)
         "bwd_dkv": ("dsa_tile_dkv_kernel", 8 * unit),
     }

@@ -1,5 +1,5 @@
-"""The key-side kernel (dK, dV): tile edges, pieces, operands on odd addresses; and, in the compiled code, the wait states that its
-inline MFMAs need."""
+"""The backward tile kernels (dQ; dK, dV): tile edges, pieces, operands on odd addresses; and, in the compiled code, the wait states that
+their inline instructions need."""
 import os
 import re
 import shutil
@@ -17,7 +17,7 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 
 
 def _registers(token):
-    m = re.match(r"([va])(?:\[(\d+):(\d+)\]|(\d+))$", token)
+    m = re.match(r"([vas])(?:\[(\d+):(\d+)\]|(\d+))$", token)
     if not m:
         return []
     lo, hi = (m.group(2), m.group(3)) if m.group(2) else (m.group(4), m.group(4))
@@ -27,7 +27,7 @@ def _registers(token):
 def _hazards(listing):
     """(MFMAs on accumulation registers, findings).  In program order: an operand of such an MFMA that a vector instruction wrote
     needs two wait states between them, a vector instruction or store that reads its result eleven (eight passes; an instruction
-    counts as one wait state, s_nop n as n + 1)."""
+    counts as one wait state, s_nop n as n + 1).  A buffer load needs five behind a vector instruction that wrote its scalar operand."""
     count, found, clock, formed, written = 0, [], 0, {}, {}
     for line in listing.splitlines():
         text = line.split("//")[0].strip()
@@ -51,9 +51,15 @@ def _hazards(listing):
             for r in (r for a in args for r in _registers(a)):
                 if r[0] == "a" and clock - formed.get(r, -99) < 12:
                     found.append(text)
-            for a in args[:2 if op.startswith("v_permlane32_swap") else 1]:
+            for a in args[:2 if op.startswith(("v_permlane32_swap", "v_add_co", "v_div_scale")) else 1]:
                 for r in _registers(a):
                     written[r] = clock
+        elif op.startswith("s_"):
+            for r in _registers(args[0]):
+                written.pop(r, None)
+        elif op.startswith("buffer_load"):
+            if any(r[0] == "s" and clock - written.get(r, -99) < 6 for a in args for r in _registers(a.split(" ")[0])):
+                found.append(text)
         elif "store" in op or op.startswith("ds_write"):
             if any(r[0] == "a" and clock - formed.get(r, -99) < 12 for a in args for r in _registers(a.split(" ")[0])):
                 found.append(text)
@@ -66,20 +72,24 @@ def test_wait_states_checker_sees_planted_hazards():
     assert _hazards("v_mov_b32_e32 v3, 0\n s_nop 0\n" + mfma)[1] and not _hazards("v_mov_b32_e32 v3, 0\n s_nop 1\n" + mfma)[1]
     assert _hazards(mfma + "\n s_nop 9\n v_accvgpr_read_b32 v1, a15")[1] and not _hazards(mfma + "\n s_nop 11\n v_accvgpr_read_b32 v1, a15")[1]
     assert _hazards(mfma + "\n scratch_store_dwordx4 off, a[0:3], off")[1]
+    first, load = "v_readfirstlane_b32 s5, v1\n s_nop ", "\n buffer_load_dwordx4 v2, s[4:7], 0 offen lds"
+    assert _hazards(first + "3" + load)[1] and not _hazards(first + "4" + load)[1]
 
 
 def test_inline_mfmas_keep_their_wait_states(tmp_path):
-    """The compiler does not see the MFMAs that the key-side kernel issues on accumulation registers, so it holds none of their
-    hazards back: the built library is searched for them."""
+    """The compiler does not see the MFMAs that these kernels issue on accumulation registers, nor their loads into LDS, so it holds none
+    of their hazards back: the built library is searched for them."""
     lib = shutil.copy(_lib.LIB_PATH, tmp_path)
     subprocess.run([OBJDUMP, "--offloading", lib], cwd=tmp_path, check=True, capture_output=True)
-    count, found = 0, []
+    count, kernels, found = 0, set(), []
     for name in sorted(os.listdir(tmp_path)):
         path = tmp_path / name
-        if name.endswith("gfx950") and b"dsa_tile_dkv_kernel" in path.read_bytes():
+        held = {k for k in (b"dsa_tile_dkv_kernel", b"dsa_tile_dq_kernel") if name.endswith("gfx950") and k in path.read_bytes()}
+        if held:
+            kernels |= held
             c, f = _hazards(subprocess.run([OBJDUMP, "-d", str(path)], check=True, capture_output=True, text=True).stdout)
             count, found = count + c, found + f
-    assert count > 1000 and not found, (count, found[:5])
+    assert len(kernels) == 2 and count > 1000 and not found, (kernels, count, found[:5])
 
 
 def _case(D, Hq, Hkv, lens, seed):
@@ -96,7 +106,10 @@ def _case(D, Hq, Hkv, lens, seed):
 @pytest.mark.parametrize("D,Hq,Hkv,lens", [
     (64, 2, 2, (1, 31, 32, 33, 127, 128, 129, 257)), (64, 6, 2, (65, 2, 160, 97)), (72, 4, 4, (63, 64, 65, 190)), (96, 4, 2, (96, 33, 129)),
     (128, 3, 1, (1, 31, 33, 129, 160)), (128, 8, 8, (32, 127, 64)), (128, 16, 1, (65, 130, 5)), (128, 4, 2, (640, 3)), (256, 4, 4, (33, 128, 65)),
-    (256, 16, 2, (129, 31, 64)), (256, 32, 2, (70, 300)), (256, 2, 1, (700,))])
+    (256, 16, 2, (129, 31, 64)), (256, 32, 2, (70, 300)), (256, 2, 1, (700,)),
+    # enough workgroups for 64 rows or keys per wave, without and with pieces
+    (64, 12, 12, (1, 31, 32, 33, 127, 128, 129, 257, 63) * 6), (72, 12, 12, (63, 64, 65, 190, 255, 256) * 7), (96, 16, 8, (96, 33, 129, 2) * 16),
+    (128, 12, 4, (1, 31, 33, 129, 160) * 32), (128, 16, 16, (32, 127, 64, 193) * 12), (128, 32, 32, (700, 300, 33)), (64, 32, 32, (900, 129, 33))])
 def test_key_and_query_gradients_at_the_edges_of_tiles(D, Hq, Hkv, lens, causal):
     print("key side", D, Hq, Hkv, lens, causal, flush=True)
     q, k, v, do, cu = _case(D, Hq, Hkv, lens, D + Hq)

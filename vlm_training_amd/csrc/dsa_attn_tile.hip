@@ -1,6 +1,5 @@
-// Tile kernels: dQ at head_dim 97 to 128 and attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask, and the
-// launch of dK / dV (the forward: dsa_tile_fwd.hip, dQ elsewhere: dsa_tile_dq.hip, dK / dV: dsa_tile_dkv.hip, the indexer backward:
-// dsa_tile_idx.hip).  They do the same
+// Attention mass over 32x32 MFMA tiles with the selection applied as a bitmap mask, and the launch of dK / dV (the forward:
+// dsa_tile_fwd.hip, dQ: dsa_tile_dq.hip, dK / dV: dsa_tile_dkv.hip, the indexer backward: dsa_tile_idx.hip).  They do the same
 // arithmetic as the gather kernels but visit every (query block, key
 // tile) pair of the causal triangle, so they win wherever the selection is dense: one selected pair
 // costs the gather kernels 2*D*e bytes of L2 traffic per kv head, a causal pair costs these kernels
@@ -289,179 +288,6 @@ __global__ __launch_bounds__(256) void dsa_mass_reduce_kernel(const float *__res
                 for (int kvh = 0; kvh < Hkv; ++kvh) acc += partial[kvh * plane + row + jj];
             mass[row + jj] = acc * inv_hq;
         }
-    }
-}
-
-// K/V tiles of the query-stationary kernels are fetched two tiles ahead into registers and one tile ahead into LDS (double
-// buffer), so a global load has two tile-times to land; one barrier per tile.
-// Every global load of the pipeline is issued unconditionally (indices past the end are clamped to
-// the last tile) and nothing is computed from a loaded value before the matching STORE, so the
-// compiler can wait with exact vmcnt counts and a load has two tile-times to land.  The kernel issues
-// LOAD(0, 0) itself, before the loads of its stationary rows.
-#define TILE_PIPELINE(NT, LOAD, STORE, COMPUTE)                                                     \
-    {                                                                                              \
-        const int nt_last = (NT) - 1;                                                              \
-        STORE(0, 0, 0);                                                                            \
-        LOAD(0, min(1, nt_last));                                                                  \
-        LOAD(1, min(2, nt_last));                                                                  \
-        __syncthreads();                                                                           \
-        int it = 0;                                                                                \
-        for (; it + 1 < (NT); it += 2) {                                                           \
-            /* LDS buffer 0 holds tile it, register set 0 tile it+1, register set 1 tile it+2 */     \
-            COMPUTE(it, 0);                                                                        \
-            STORE(0, 1, it + 1);                                                            \
-            LOAD(0, min(it + 3, nt_last));                                                         \
-            __syncthreads();                                                                       \
-            COMPUTE(it + 1, 1);                                                             \
-            STORE(1, 0, min(it + 2, nt_last));                                                     \
-            LOAD(1, min(it + 4, nt_last));                                                         \
-            __syncthreads();                                                                       \
-        }                                                                                          \
-        if (it < (NT)) COMPUTE(it, 0);                                                             \
-    }
-
-// ==================================================================================================
-// dQ: query-stationary, same walk as the forward.
-//   S^T = K Q^T, dP^T = V dO^T  (A = K / V tiles row-wise, B = Q^T / dO^T in registers)
-//   dS^T = P^T * (dP^T - delta)  on the C layout
-//   dQ^T[d,row] += K^T[d,key] dS^T[key,row]   (A = K tile transposed, B = dS^T from the C layout)
-// ==================================================================================================
-template <int D, bool HAS_IDX, int GSHIFT, int NW>
-__global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_dq128_kernel(
-    const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
-    const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
-    const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, int pos_split, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
-    float *delta_out) {
-    constexpr int KS = D / 16, DT = (D + 31) / 32, CPR = D / 8, TILE_B = tile_bytes<D>();
-    constexpr int NBUF = 2;
-    constexpr int NT = NW * 64, Gp = 1 << GSHIFT, QBW = (NW * 32) >> GSHIFT;
-    constexpr int CH = 32 * CPR, LOADS = (CH + NT - 1) / NT;   // 16-byte chunks per matrix; per thread (head_dim 96: not all threads)
-    static_assert(CH % 64 == 0, "whole waves stage or do not");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NBUF][2][TILE_B];
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = lane >> 5, j = lane & 31;
-    LaneOffsets<D> lo;
-    lo.init(lane);
-    const int G = Hq / Hkv;
-    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
-    const int kvh = blockIdx.x % Hkv;
-    int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(causal, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
-    if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
-    const int qc0 = blk * QBW;
-    if (qc0 >= pos_split || qc0 >= L) return;
-
-    const int r = wv * 32 + j;
-    const int qcol = qc0 + (r >> GSHIFT), head = r & (Gp - 1);
-    const bool row_ok = qcol < L && head < G;
-    const int t = s0 + min(qcol, L - 1), hq = kvh * G + min(head, G - 1);
-    const float scale_log2 = scale * LOG2E_F;
-    u32x4 kst[2][LOADS], vst[2][LOADS];
-#define DQ_LOAD(SET, TILE)                                                                          \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) if (CH % NT == 0 || i * NT + tid < CH) {     \
-        const int c = i * NT + tid;                                                               \
-        const int row = c / CPR, ch = HAS_IDX ? c % CPR : min(c % CPR, chunks - 1);   /* (spare columns: any finite values) */ \
-        const int64_t off = ((int64_t)(s0 + min((TILE) * 32 + row, L - 1)) * Hkv + kvh) * dr + ch * 8; \
-        kst[SET][i] = *reinterpret_cast<const u32x4 *>(k + off);                                   \
-        vst[SET][i] = *reinterpret_cast<const u32x4 *>(v + off);                                   \
-    }
-    DQ_LOAD(0, 0)                                       // ahead of the q / dO rows: staging waits for this tile only
-    bf16x8 qB[KS], doB[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
-        const bool there = row_ok && (HAS_IDX || 2 * ks + h < chunks);
-        qB[ks] = there ? load_bf16x8(q + off) : zero_bf16x8();
-        doB[ks] = there ? load_bf16x8(dout + off) : zero_bf16x8();
-    }
-    // the two accumulators of a tile start from -lse/scale and -delta of the lane's row, so that S - lse/scale and
-    // dP - delta come out of the MFMAs (one multiply per element instead of a multiply-add and a subtraction)
-    const float neg_lse = -lse[(int64_t)hq * T + t] / scale;
-    // delta = rowsum(dO * O) of the lane's row: read, or - when every query row of the launch belongs to this kernel -
-    // formed here from the dO row the lane already holds and written out for the key-side pass (one launch and one
-    // pass over dO and O less)
-    float dlt;
-    if (out_for_delta) {                                 // (kernel argument: the same for every wave)
-        // the order of dsa_bwd_delta_kernel, so that both give the same bits: chain j of this lane covers the 8-element
-        // chunks 2*ks+h with ks = j, j+8, ... (that kernel's lane 2*j+h), then its butterfly over 16 lanes - the three
-        // steps between lanes of one parity here, the last one across the lane pair
-        float p[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            p[j] = 0.f;
-#pragma unroll
-            for (int ks = j; ks < KS; ks += 8) {
-                const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
-                const bf16x8 o8 = row_ok && (HAS_IDX || 2 * ks + h < chunks) ? load_bf16x8(out_for_delta + off) : zero_bf16x8();
-                p[j] = dot8_chain(doB[ks], o8, p[j]);
-            }
-        }
-        const float part = ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
-        dlt = half_sum_f(part);
-        if (row_ok && h == 0) delta_out[(int64_t)hq * T + t] = dlt;
-    } else {
-        dlt = delta[(int64_t)hq * T + t];
-    }
-    const float neg_dlt = -dlt;
-    const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
-    const int klim = causal ? qcol : L - 1;             // last key column this row may attend (dense mode)
-    const uint32_t *wrow = bitmap + (int64_t)t * ldw;
-
-    f32x16 acc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = zero16();
-    uint32_t word_next = HAS_IDX ? wrow[0] : 0u;        // unconditional loads; rows that are not live are masked at use
-
-#define DQ_STORE(SET, BUF, TILE)                                                                         \
-    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) if (CH % NT == 0 || i * NT + tid < CH) {     \
-        const int c = i * NT + tid;                                                               \
-        const int row = c / CPR, ch = c % CPR;                                                     \
-        *reinterpret_cast<u32x4 *>(&lds[BUF][0][tile_off<D>(row, ch)]) = kst[SET][i];              \
-        *reinterpret_cast<u32x4 *>(&lds[BUF][1][tile_off<D>(row, ch)]) = vst[SET][i];              \
-    }
-#define DQ_COMPUTE(TILE, BUF)                                                                       \
-    {                                                                                              \
-        const int kc0 = (TILE) * 32;                                                               \
-        const unsigned char *kt = lds[BUF][0], *vt = lds[BUF][1];                                  \
-        uint32_t word = row_ok ? word_next : 0u;                                                   \
-        if (HAS_IDX) word_next = wrow[min((TILE) + 1, ntiles - 1)];                                \
-        if (!HAS_IDX) word = row_ok ? causal_bits(klim - kc0) : 0u;                                \
-        word >>= 4 * h;                                                                            \
-        f32x16 sacc, pacc;                                                                         \
-        _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) { sacc[vi] = neg_lse; pacc[vi] = neg_dlt; } \
-        _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) {                                        \
-            sacc = mfma32(lo.rowop(kt, ks), qB[ks], sacc);                              \
-            pacc = mfma32(lo.rowop(vt, ks), doB[ks], pacc);                             \
-        }                                                                                          \
-        sched_reads_ahead<2 * KS, 4, 1>();                                                         \
-        float ds[16];                                                                              \
-        /* tiles in which every live row keeps all 32 keys skip the mask arithmetic */             \
-        if (__builtin_amdgcn_ballot_w64(row_ok && (word & 0x0f0f0f0fu) != 0x0f0f0f0fu) == 0ull) {     \
-            _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) ds[vi] = fast_exp2(sacc[vi] * scale_log2) * pacc[vi]; \
-        } else {                                                                                   \
-            _Pragma("unroll") for (int vi = 0; vi < 16; ++vi) {                                    \
-                const float x = keep_or_neginf(sacc[vi] * scale_log2,                              \
-                                               bit_mask(word, 8 * (vi >> 2) + (vi & 3)));          \
-                ds[vi] = fast_exp2(x) * pacc[vi];                                                  \
-            }                                                                                      \
-        }                                                                                          \
-        const bf16x8 dB0 = pack8(ds), dB1 = pack8(ds + 8);                                         \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) {                                        \
-            mfma32_acc(acc[dt], lo.trop(kt, 0, dt), dB0);                           \
-            mfma32_acc(acc[dt], lo.trop(kt, 1, dt), dB1);                      \
-        }                                                                                          \
-        sched_reads_ahead<2 * DT, 3, 2>();                                                         \
-    }
-    TILE_PIPELINE(ntiles, DQ_LOAD, DQ_STORE, DQ_COMPUTE)
-#undef DQ_LOAD
-#undef DQ_STORE
-#undef DQ_COMPUTE
-
-    if (row_ok) {
-        bf16_t *op = dq + ((int64_t)t * Hq + hq) * dr;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, acc[dt], scale, h, chunks - 4 * dt);
     }
 }
 
@@ -812,28 +638,6 @@ extern "C" hipError_t dsa_launch_tile_mass(const void *q, const void *k, const f
                        inv_hq, mass);
     return hipGetLastError();
 }
-template <int D, bool HAS_IDX, int GS>
-static hipError_t launch_dq_i(dim3 grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
-                        const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                        int T, int Hq, int Hkv, int d_real, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
-                        float *delta_out) {
-    hipLaunchKernelGGL((dsa_tile_dq128_kernel<D, HAS_IDX, GS, 8>), grid, dim3(512), 0, stream, (const bf16_t *)dout,
-                       (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv,
-                       scale, pos_split, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
-    return hipSuccess;
-}
-// dQ at head_dim 97 to 128 (dsa_tile_dq.hip runs the others and says why)
-extern "C" hipError_t dsa_launch_tile_dq_128(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
-                                             const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real,
-                                             float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
-                                             float *delta_out, hipStream_t stream) {
-    const int gs = group_shift(Hq, Hkv);
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * 8) >> gs) + N + 1) * Hkv));
-    hipError_t launch_status = hipErrorInvalidValue;
-    if (bitmap) { GS_SWITCH(launch_dq_i, 128, true, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out) }
-    else { GS_SWITCH(launch_dq_i, 128, false, grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out) }
-    return launch_status != hipSuccess ? launch_status : hipGetLastError();
-}
 // bytes of fp32 partial sums a launch of T tokens may use for key-tile walks in pieces (0: launches of this size are
 // never cut); a slot = the dK and dV of one 128-key tile and kv head
 extern "C" size_t dsa_tile_dkv_partial_bytes(int T) {
@@ -849,7 +653,7 @@ static DkvPlan dkv_plan(int T, int N, int Hq, int Hkv, int d_real, bool has_idx,
     DkvPlan p;
     p.tiles_ub = T / 128 + N;                            // 128-key tiles of all segments, at most
     p.pitch = has_idx ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;             // row of a partial sum
-    const int wg_per_tile = Hkv, kg = dkv_key_groups(d_real, T, N, Hkv);
+    const int wg_per_tile = Hkv, kg = dkv_key_groups(d_real, T, N, Hkv, causal);
     const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * p.pitch * sizeof(float))) : 0;
     p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= dkv_pieces_max_wg(d_real);
     p.listed = order && (N > 1 || p.pieces);             // (one segment: its tiles are in order already)

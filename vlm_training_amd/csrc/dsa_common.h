@@ -13,11 +13,12 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define DSA_WAVE 64
 // Groups of 32 keys that a wave of the key-side kernel takes: two up to head_dim 128 (each operand read feeds two MFMAs, two workgroups
-// per CU), except at head_dim 97 to 128 in launches of at most DKV_FEW_WG workgroups, which leave CUs idle: there a workgroup's own
-// pace counts, and four waves of one group each walk twice as fast.
-#define DKV_FEW_WG 192
-static inline int dkv_key_groups(int D, int T, int N, int Hkv) {
-    return D > 128 || (D > 96 && ((int64_t)T / 128 + N) * Hkv <= DKV_FEW_WG) ? 1 : 2;
+// per CU), except in launches of few workgroups, which leave CUs idle: there a workgroup's own pace counts, and four waves of one group
+// each walk twice as fast.  The line in workgroups, both sides measured around it (two groups against one, us): without a mask 256,
+// 98 / 84 and 272, 67 / 57, but 384, 171 / 200; causal in one segment 192, 230 / 199 and 224, 242 / 318, in three 240, 123 / 117 (a long
+// walk is cut into pieces, which then needs free slots) and 340, 216 / 260.
+static inline int dkv_key_groups(int D, int T, int N, int Hkv, int causal) {
+    return D > 128 || ((int64_t)T / 128 + N) * Hkv <= (causal ? 160 + 32 * (N < 3 ? N : 3) : 288) ? 1 : 2;
 }
 // key-side workgroups that run at a time, and the launches whose walks may be cut into pieces: up to three rounds of them (a longer
 // launch of whole walks, longest first, ends level)
@@ -131,6 +132,11 @@ __device__ __forceinline__ buffer_rsrc make_buffer_rsrc(const void *p, int64_t b
     const uint32_t n = bytes < 0 ? 0u : bytes > 0xffffffffll ? 0xffffffffu : (uint32_t)bytes;
     return buffer_rsrc{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
                        (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+// the same from scalars (a pointer and a size that scalar instructions formed)
+__device__ __forceinline__ buffer_rsrc scalar_buffer_rsrc(const void *p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return buffer_rsrc{(uint32_t)a, (uint32_t)(a >> 32), bytes, 0x00020000u};
 }
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;

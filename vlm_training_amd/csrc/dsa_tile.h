@@ -6,21 +6,6 @@
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }   // v_exp_f32; exp2(-inf) = 0
 
-// ---- LDS tile: 32 rows of D bf16 with a pitch of D*2 + 64 bytes (+ 128 at head_dim 96); chunk = 16 bytes ----
-// The LDS of gfx950 has 64 four-byte banks (256 B per clock).  A 16-byte read is served 16 lanes at a
-// time and a transposed 8-byte read 32 lanes at a time, so a row-wise operand read (16 consecutive rows,
-// same chunk) and a transposed read (4 consecutive rows x 64 B) must each cover all banks once.  The
-// 64-byte skew per row separates 4 consecutive rows, the XOR of the chunk's two low bits with row bits
-// 2-3 separates rows 4 apart: both read patterns and the row-wise staging writes are conflict-free.
-// (The skew needs a pitch of 64 modulo 256 bytes: head_dim 80 and 96 pad their rows to the pitch of head_dim 128.)
-template <int D> constexpr int tile_pitch() { return D == 96 || D == 80 ? 320 : D * 2 + 64; }
-template <int D> constexpr int tile_bytes() { return 32 * tile_pitch<D>(); }
-__device__ __forceinline__ int tile_sw(int row) { return (row >> 2) & 3; }
-template <int D>
-__device__ __forceinline__ int tile_off(int row, int chunk) { return row * tile_pitch<D>() + ((chunk ^ tile_sw(row)) << 4); }
-
-// accumulate in place (kept as a function so that the accumulation sites read alike)
-__device__ __forceinline__ void mfma32_acc(f32x16 &c, bf16x8 a, bf16x8 b) { c = mfma32(a, b, c); }
 // all-ones if bit `b` of `word` is set, else 0 (v_bfe_i32 when b is a compile-time constant)
 __device__ __forceinline__ uint32_t bit_mask(uint32_t word, int b) {
     return (uint32_t)(((int32_t)(word << (31 - b))) >> 31);
@@ -31,63 +16,16 @@ __device__ __forceinline__ float keep_or_neginf(float x, uint32_t keep) {
 }
 // bits j <= d of a 32-key tile (keys at or before the diagonal when d = query column - tile start)
 __device__ __forceinline__ uint32_t causal_bits(int d) { return d >= 31 ? 0xffffffffu : (d < 0 ? 0u : ((2u << d) - 1u)); }
-// Issue order for a chain of NM MFMAs that each consume RPM LDS reads: keep AHEAD MFMAs' worth of reads
-// in flight (the machine scheduler otherwise sinks every read next to its use and the chain runs at
-// LDS latency).  Applies to the instructions of the enclosing basic block, in program order.
-template <int NM, int AHEAD, int RPM, int FIRST = 0>
-__device__ __forceinline__ void sched_reads_ahead() {
-    __builtin_amdgcn_sched_group_barrier(0x100, FIRST + AHEAD * RPM, 0);   // FIRST: other reads issued up front
-#pragma unroll
-    for (int i = 0; i < NM - AHEAD; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
-}
-// Per-lane LDS byte offsets of the two read patterns, computed once per kernel so that every operand
-// read in the loops is "tile base + lane offset + immediate" (the swizzle only XORs chunk bits 0-1, so
-// k-step / d-tile indices move the address by a lane constant plus a compile-time multiple of 64 B).
-//   row-wise A operand of mfma32: lane (i = row j, h) takes elements [16*ks + 8h, +8) of row j
-//   transposed A operand: lane l takes column c = 32*dt + (l & 31)... of the 8 rows {R..R+3, R+8..R+11}.
-//   ds_read_b64_tr_b16: within 16 lanes, lane s supplies the address of 4 consecutive elements of row
-//   R + s/4 at column m0 + 4*(s%4); lane s receives rows R..R+3 of column m0 + s.
+// A transposed operand of mfma32: ds_read_b64_tr_b16 - within 16 lanes, lane s supplies the address of 4 consecutive elements of row
+// R + s/4 at column m0 + 4*(s%4) and receives rows R..R+3 of column m0 + s - twice
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
-template <int D>
-struct LaneOffsets {
-    int row[2];      // row-wise operand of row j: k-steps ks with ks % 2 == c
-    int tr[4];       // transposed operand: rows 4h + s/4 + {0, 8, 16, 24}
-    __device__ __forceinline__ void init(int lane) {
-        const int h = lane >> 5, j = lane & 31, s = lane & 15;
-        const int swj = tile_sw(j);
-#pragma unroll
-        for (int c = 0; c < 2; ++c) row[c] = j * tile_pitch<D>() + ((((c ^ (swj >> 1)) << 1) | (h ^ (swj & 1))) << 4);
-        const int low = ((lane >> 4) & 1) * 2 + ((s & 3) >> 1), sub = (s & 1) << 3;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = 4 * h + (s >> 2) + 8 * v;
-            tr[v] = r * tile_pitch<D>() + ((low ^ tile_sw(r)) << 4) + sub;
-        }
-    }
-    // row-wise A operand of k-step ks (elements [16ks + 8h, +8) of row j)
-    __device__ __forceinline__ bf16x8 rowop(const unsigned char *tile, int ks) const {
-        return *reinterpret_cast<const bf16x8 *>(tile + row[ks & 1] + (ks >> 1) * 64);
-    }
-    __device__ __forceinline__ static bf16x8 tr_pair(lds_u8 *p0, lds_u8 *p1) {
-        const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p0);
-        const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p1);
-        typedef short s16x8 __attribute__((ext_vector_type(8)));
-        const s16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-        return __builtin_bit_cast(bf16x8, r);
-    }
-    // transposed A operand of d-tile dt over rows {R..R+3, R+8..R+11}, R = 4h (pair 0) or 16 + 4h (pair 1)
-    __device__ __forceinline__ bf16x8 trop(const unsigned char *tile, int pair, int dt) const {
-        return tr_pair((lds_u8 *)tile + tr[2 * pair] + dt * 64, (lds_u8 *)tile + tr[2 * pair + 1] + dt * 64);
-    }
-    // same with the lane addresses already formed (p[v] = tile + tr[v]): one immediate per read
-    __device__ __forceinline__ static bf16x8 trop_at(lds_u8 *const *p, int pair, int dt, int imm) {
-        return tr_pair(p[2 * pair] + dt * 64 + imm, p[2 * pair + 1] + dt * 64 + imm);
-    }
-};
+__device__ __forceinline__ bf16x8 tr_pair(lds_u8 *p0, lds_u8 *p1) {
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p0);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)p1);
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return __builtin_bit_cast(bf16x8, r);
+}
 __device__ __forceinline__ bf16x8 pack8(const float *x) {
     const u32x4 w = {pack2bf(x[0], x[1]), pack2bf(x[2], x[3]), pack2bf(x[4], x[5]), pack2bf(x[6], x[7])};
     return __builtin_bit_cast(bf16x8, w);
@@ -242,6 +180,42 @@ struct DirectTile {
     static constexpr int row_imm(int ks) { return D == 64 ? 0 : (ks >> 3) * 256 + (ks & 1) * 32; }
     static constexpr int tr_q(int dt) { return dt & 3; }
     static constexpr int tr_imm(int dt, int v) { return (D == 64 ? 0 : (dt >> 2) * 256) + v * (8 / GROUP) * GROUP_B; }
+};
+
+// ---- one wave per SIMD: sums in accumulation registers, phases of mixed operands ----
+// c += a b with c in accumulation registers, named here: left to itself the compiler keeps 128 to 256 registers of sums where the
+// vector instructions need them, and spills.  It does not see an MFMA in this statement, so its hazards are held by hand: an operand
+// that a vector instruction wrote needs two wait states (operands come from LDS or are formed many MFMAs ahead), a result that one
+// reads eleven; the last MFMA on a tuple in front of a join or of the stores (`last`) waits itself.  tests/test_key_side.py looks for both in the compiled kernels (a copy of a tuple
+// that the compiler placed a wait state too close was enough to spoil dK).
+__device__ __forceinline__ void mfma32_agpr(f32x16 &c, bf16x8 a, bf16x8 b, bool last) {
+    if (last) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+a"(c) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    __builtin_amdgcn_sched_barrier(0);                   // (nor does it see where the vector instructions behind it belong)
+}
+// the tuple's value lies in accumulation registers here; in front of its uses: the tuples leave them one by one
+__device__ __forceinline__ void settle(f32x16 &c) { asm volatile("" : "+a"(c)); }
+// a wave's N pieces of a tile, one behind the other; N0, N1, N2 = LDS bytes from one to the next (see buffer_load_lds16)
+template <int N, int N0, int N1, int N2>
+__device__ __forceinline__ void buffer_load_lds16_n(buffer_rsrc rsrc, const int (&voff)[N], uint32_t lds) {
+    static_assert(N == 1 || N == 2 || N == 4, "");
+    if constexpr (N == 1)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff[0]), "s"(rsrc), "s"(lds) : "memory", "m0");
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds\n\ts_add_u32 m0, m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(lds), "n"(N0) : "memory", "m0", "scc");
+    if constexpr (N == 4)
+        asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\ts_add_u32 m0, m0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds"
+                     "\n\ts_add_u32 m0, m0, %7\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\ts_add_u32 m0, m0, %8\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds"
+                     : : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds), "n"(N0), "n"(N1), "n"(N2) : "memory", "m0", "scc");
+}
+// Order of a phase's NR row-wise and NT transposed operands: `PRE` transposed ones, then both kinds evenly mixed.
+template <int NR, int NT, int PRE>
+struct PhaseOrder {
+    static constexpr int M = NR + NT;
+    static constexpr int rows_before(int m) { return m <= PRE || M == PRE ? 0 : (m - PRE) * NR / (M - PRE); }
+    static constexpr bool is_row(int m) { return rows_before(m + 1) > rows_before(m); }
+    static constexpr int index(int m) { return is_row(m) ? rows_before(m) : m - rows_before(m); }
 };
 
 // ---- walks of key tiles (dK, dV) ----

@@ -7,8 +7,8 @@
 //                                    -lse/scale and -delta, so that P = exp2(S * scale*log2e) and dS = P dP need no subtraction)
 //   dV^T += dO^T P, dK^T += Q^T dS  (A = the blocks transposed, B = P / dS from the C layout)
 // One wave per SIMD, each with all four chains of its keys and 512 registers: 64 keys up to head_dim 128 (two waves a workgroup, two
-// workgroups a CU), 32 keys at head_dim 256 and in launches of few workgroups at 128 (four waves, one workgroup: dkv_key_groups).  The sums of dK and dV fill up to 256 accumulation
-// registers, K and V rows 128 of the others.  An operand read from LDS feeds the MFMAs of both key groups, P and dS never leave
+// workgroups a CU), 32 keys at head_dim 256 and in launches of few workgroups (four waves, one workgroup: dkv_key_groups).  The sums of
+// dK and dV fill up to 256 accumulation registers, K and V rows 128 of the others.  An operand read from LDS feeds the MFMAs of both key groups, P and dS never leave
 // the wave, nothing is formed twice.  Step s runs dV(s) mixed with S(s+1), the products of dS(s) behind them, then dK(s) mixed with
 // dP(s+1), P(s+1) behind them in three stages (logit, exponential, packing) that do not wait for each other.  q and dO blocks, row
 // data and selection words go from memory straight into LDS, two to three steps ahead, one barrier per step.
@@ -32,40 +32,6 @@ template <int D, int KG> constexpr int dkv_aux_bytes() { return dkv_ring<D, KG>(
 template <int D, int KG> constexpr size_t dkv_lds_bytes() {
     return dkv_ring<D, KG>() * 2 * (size_t)DirectTile<D>::BYTES + 4 / KG * (size_t)dkv_aux_bytes<D, KG>();
 }
-// c += a b with c in accumulation registers, named here: left to itself the compiler keeps 128 to 256 registers of sums where the
-// vector instructions need them, and spills.  It does not see an MFMA in this statement, so its hazards are held by hand: an operand
-// that a vector instruction wrote needs two wait states (operands come from LDS or are formed many MFMAs ahead), a result that one
-// reads eleven; the last MFMA on a tuple in front of a join or of the stores (`last`) waits itself.  tests/test_key_side.py looks for both in the compiled kernels (a copy of a tuple
-// that the compiler placed a wait state too close was enough to spoil dK).
-__device__ __forceinline__ void mfma32_agpr(f32x16 &c, bf16x8 a, bf16x8 b, bool last) {
-    if (last) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+a"(c) : "v"(a), "v"(b));
-    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-    __builtin_amdgcn_sched_barrier(0);                   // (nor does it see where the vector instructions behind it belong)
-}
-// the tuple's value lies in accumulation registers here; in front of its uses: the tuples leave them one by one
-__device__ __forceinline__ void settle(f32x16 &c) { asm volatile("" : "+a"(c)); }
-// a wave's N pieces of a tile, one behind the other; N0, N1, N2 = LDS bytes from one to the next (see buffer_load_lds16)
-template <int N, int N0, int N1, int N2>
-__device__ __forceinline__ void buffer_load_lds16_n(buffer_rsrc rsrc, const int (&voff)[N], uint32_t lds) {
-    static_assert(N == 1 || N == 2 || N == 4, "");
-    if constexpr (N == 1)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff[0]), "s"(rsrc), "s"(lds) : "memory", "m0");
-    if constexpr (N == 2)
-        asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds\n\ts_add_u32 m0, m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(lds), "n"(N0) : "memory", "m0", "scc");
-    if constexpr (N == 4)
-        asm volatile("s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\ts_add_u32 m0, m0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds"
-                     "\n\ts_add_u32 m0, m0, %7\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\ts_add_u32 m0, m0, %8\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds"
-                     : : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds), "n"(N0), "n"(N1), "n"(N2) : "memory", "m0", "scc");
-}
-// Order of a phase's NR row-wise and NT transposed operands: `PRE` transposed ones, then both kinds evenly mixed.
-template <int NR, int NT, int PRE>
-struct PhaseOrder {
-    static constexpr int M = NR + NT;
-    static constexpr int rows_before(int m) { return m <= PRE || M == PRE ? 0 : (m - PRE) * NR / (M - PRE); }
-    static constexpr bool is_row(int m) { return rows_before(m + 1) > rows_before(m); }
-    static constexpr int index(int m) { return is_row(m) ? rows_before(m) : m - rows_before(m); }
-};
 template <int D, int KG, bool HAS_IDX, int GSHIFT, bool UNALIGNED>
 __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
@@ -83,7 +49,8 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     // loop has no registers left for them, the lane's source offsets and the last K operand of each key group
     constexpr int AUX = dkv_aux_bytes<D, KG>();
     constexpr bool TIGHT = D == 128 && KG == 2;
-    constexpr int AHEAD = KG == 2 ? 2 : 4;               // operands read ahead: four MFMAs
+    constexpr int AHEAD = TIGHT ? 2 : 4;                 // operands read ahead: four MFMAs or more
+    constexpr bool PAIRS = KG == 2 && !TIGHT;            // operands waited for and refilled in pairs
     constexpr bool KEEP_P = D <= (KG == 1 ? 128 : 80);                    // P stays in fp32 until dS is formed (else its bf16 form is unpacked)
     static_assert(TL::LOADS % NW == 0 && (RING & (RING - 1)) == 0 && AHEAD <= NP, "");
     extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];
@@ -127,11 +94,11 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     const int64_t blk_b = (int64_t)QB * tok_b;
     auto block_bytes = [&](int b) __attribute__((always_inline)) { return b > last ? 0 : b == 0 ? first_b : full_b; };
     // the wave's pieces of q (or dO) of block b; called in turn.  Rows past the walk and columns past the true head_dim read as zero.
-    auto load_tile = [&](const int (&voff)[LPW], const unsigned char *&p, int b, int tile) __attribute__((always_inline)) {
-        const int bytes = UNALIGNED ? 0 : block_bytes(b);
+    auto load_tile = [&](const int (&voff)[LPW], const unsigned char *&p, int b, int tile, uint32_t bytes) __attribute__((always_inline)) {
+        if (UNALIGNED) bytes = 0u;
         constexpr int P1 = LPW > 1 ? 1 : 0, P2 = LPW > 2 ? 2 : P1, P3 = LPW > 2 ? 3 : P2;
         buffer_load_lds16_n<LPW, TL::load_lds(P1), TL::load_lds(P2) - TL::load_lds(P1), TL::load_lds(P3) - TL::load_lds(P2)>(
-            make_buffer_rsrc(p, bytes), voff, lds0 + (b & (RING - 1)) * SLOT + tile * TL::BYTES + TL::load_lds(wv * LPW));
+            scalar_buffer_rsrc(p, bytes), voff, lds0 + (b & (RING - 1)) * SLOT + tile * TL::BYTES + TL::load_lds(wv * LPW));
         p -= blk_b;
         asm volatile("" : "+s"(p));
     };
@@ -181,8 +148,8 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     }
 #pragma unroll
     for (int b = 0; b < RING - 2; ++b) {
-        load_tile(voff, qptr, b, 0);
-        load_tile(voff, dptr, b, 1);
+        load_tile(voff, qptr, b, 0, block_bytes(b));
+        load_tile(voff, dptr, b, 1, block_bytes(b));
         load_rows(b + 1);
         load_words(b + 1);
     }
@@ -262,7 +229,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     };
     auto tr_op = [&](int i, int off) __attribute__((always_inline)) {
         const int pair = i / DT, dt = i % DT;
-        return LaneOffsets<D>::tr_pair(aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair) + off, aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair + 1) + off);
+        return tr_pair(aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair) + off, aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair + 1) + off);
     };
     const int jb = 31 - j, key_bias = (causal ? 0 : 0x40000000) - kc - 31;      // key_bias + jb = bias - the lane's first key
     // Step s: phase X = dV(s) and S(s+1), behind them dS(s); phase Y = dK(s) and dP(s+1), behind them P(s+1).
@@ -290,6 +257,17 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
 #pragma unroll
             for (int m = 0; m < AHEAD; ++m) op[m] = fetch(m);
         }
+        // Operands in pairs where registers allow: one wait in front of two of them, both refilled behind the second (a wait takes an
+        // issue slot)
+        auto pair = [&](int m) __attribute__((always_inline)) {
+            if (PAIRS && m % 2 == 0) asm volatile("" : "+v"(op[m % AHEAD]), "+v"(op[(m + 1) % AHEAD]));
+        };
+        auto refill = [&](int m) __attribute__((always_inline)) {
+            if (PAIRS && m % 2 == 0) return;
+#pragma unroll
+            for (int x = PAIRS ? m - 1 : m; x <= m; ++x)
+                if (x + AHEAD < M || NEXT) op[x % AHEAD] = fetch(x + AHEAD);
+        };
         f32x16 snew[KG], pnew[KG];
         int vo[LPW];
         if (NEXT) {
@@ -311,6 +289,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
         constexpr int E = 16 * KG, SX = SL - 2;          // dS: product behind MFMA 1 + u, packed behind the next
 #pragma unroll
         for (int m = 0; m < NX; ++m) {
+            pair(m);
 #pragma unroll
             for (int g = 0; g < KG; ++g) {
                 const int i = PO::index(m), n = m * KG + g, u = n - 1;
@@ -320,10 +299,10 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
                     const u32x4 w = {pw[g][4 * (i / DT)], pw[g][4 * (i / DT) + 1], pw[g][4 * (i / DT) + 2], pw[g][4 * (i / DT) + 3]};
                     mfma32_agpr(dvacc[g][i % DT], op[m % AHEAD], __builtin_bit_cast(bf16x8, w), !NEXT);
                 }
-                if (g == KG - 1 && (m + AHEAD < M || NEXT)) op[m % AHEAD] = fetch(m + AHEAD);
+                if (g == KG - 1) refill(m);
                 if (NEXT) {
-                    if (n == 1) load_tile(vo, qptr, s + RING - 1, 0);
-                    if (n == SL / 4) load_tile(vo, dptr, s + RING - 1, 1);
+                    if (n == 1) load_tile(vo, qptr, s + RING - 1, 0, s + RING - 1 <= last ? full_b : 0);
+                    if (n == SL / 4) load_tile(vo, dptr, s + RING - 1, 1, s + RING - 1 <= last ? full_b : 0);
                     if (n == SL / 2) load_rows(s + RING);
                     if (n == 3 * SL / 4) load_words(s + RING);
                 }
@@ -379,6 +358,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
         constexpr int SY = SL - 3;                       // logits behind MFMA 1 + u, P behind the next, packed behind the one after
 #pragma unroll
         for (int m = 0; m < NX; ++m) {
+            pair(NX + m);
 #pragma unroll
             for (int g = 0; g < KG; ++g) {
                 const int i = PO::index(m), n = m * KG + g, u = n - 1, mm = NX + m;
@@ -388,7 +368,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
                     const u32x4 w = {dw[g][4 * (i / DT)], dw[g][4 * (i / DT) + 1], dw[g][4 * (i / DT) + 2], dw[g][4 * (i / DT) + 3]};
                     mfma32_agpr(dkacc[g][i % DT], op[mm % AHEAD], __builtin_bit_cast(bf16x8, w), !NEXT || (UNALIGNED && i >= DT));
                 }
-                if (g == KG - 1 && (mm + AHEAD < M || NEXT)) op[mm % AHEAD] = fetch(mm + AHEAD);
+                if (g == KG - 1) refill(mm);
                 if (NEXT && u >= 0) {
 #pragma unroll
                     for (int e = E * u / SY; e < E * (u + 1) / SY; ++e) {
@@ -561,12 +541,12 @@ static hipError_t launch_dkv_gs(unsigned grid, hipStream_t stream, const DkvArgs
         default: return launch_dkv<D, KG, HAS_IDX, 4>(grid, stream, a);
     }
 }
-template <bool HAS_IDX>
-static hipError_t launch_dkv_128(unsigned grid, hipStream_t stream, const DkvArgs &a) {
+template <int D, bool HAS_IDX>
+static hipError_t launch_dkv_kg(unsigned grid, hipStream_t stream, const DkvArgs &a) {
 #if !DKV_UNALIGNED
-    if (dkv_key_groups(a.d_real, a.T, a.N, a.Hkv) == 1) return launch_dkv_gs<128, 1, HAS_IDX>(grid, stream, a);
+    if (dkv_key_groups(a.d_real, a.T, a.N, a.Hkv, a.causal) == 1) return launch_dkv_gs<D, 1, HAS_IDX>(grid, stream, a);
 #endif
-    return launch_dkv_gs<128, 2, HAS_IDX>(grid, stream, a);
+    return launch_dkv_gs<D, 2, HAS_IDX>(grid, stream, a);
 }
 // grid: workgroups (one per key tile or piece, and kv head).  The file is compiled twice, the second time (DKV_UNALIGNED) for q or dO on no
 // 16-byte boundary; k and v lie on one (the entry points see to it).
@@ -583,14 +563,14 @@ extern "C" hipError_t dsa_launch_dkv_tiles(DKV_LAUNCH_ARGS) {
 #endif
     const DkvArgs a{dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv};
     if (bitmap) switch (d_real) {
-        case 64: return launch_dkv_gs<64, 2, true>(grid, stream, a);
-        case 128: return launch_dkv_128<true>(grid, stream, a);
+        case 64: return launch_dkv_kg<64, true>(grid, stream, a);
+        case 128: return launch_dkv_kg<128, true>(grid, stream, a);
         case 256: return launch_dkv_gs<256, 1, true>(grid, stream, a);
     } else switch (dense_kernel_dim(d_real)) {
-        case 64: return launch_dkv_gs<64, 2, false>(grid, stream, a);
-        case 80: return launch_dkv_gs<80, 2, false>(grid, stream, a);
-        case 96: return launch_dkv_gs<96, 2, false>(grid, stream, a);
-        case 128: return launch_dkv_128<false>(grid, stream, a);
+        case 64: return launch_dkv_kg<64, false>(grid, stream, a);
+        case 80: return launch_dkv_kg<80, false>(grid, stream, a);
+        case 96: return launch_dkv_kg<96, false>(grid, stream, a);
+        case 128: return launch_dkv_kg<128, false>(grid, stream, a);
         case 256: return launch_dkv_gs<256, 1, false>(grid, stream, a);
     }
     return hipErrorInvalidValue;

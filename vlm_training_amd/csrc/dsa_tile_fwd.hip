@@ -151,7 +151,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     auto read_v = [&](int i) __attribute__((always_inline)) {             // MFMA i of P V: keys of half i / DT, d-tile i % DT
         const int pair = i / DT, dt = i % DT;
         lds_u8 *p = (lds_u8 *)dyn_lds + va_[TL::tr_q(dt)];
-        return LaneOffsets<D>::tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
+        return tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
     };
     // The keys of a tile this lane keeps, as they lie in memory; live(word): element vi then sits at bit 8*(vi/4) + vi%4
     const uint32_t row_mask = row_ok ? 0xffffffffu : 0u;

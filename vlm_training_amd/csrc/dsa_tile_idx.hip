@@ -54,7 +54,7 @@ __device__ __forceinline__ void gated_walk(unsigned char *ring, int lane, int nt
     auto read_tr = [&](int i) __attribute__((always_inline)) {           // MFMA i of the second product: rows of half i / DT, d-tile i % DT
         const int pair = i / DT, dt = i % DT;
         lds_u8 *p = (lds_u8 *)ring + ta[TL::tr_q(dt)];
-        return LaneOffsets<D>::tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
+        return tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
     };
     auto gemm_s = [&](f32x16 &s) __attribute__((always_inline)) {
         s = zero16();
