@@ -15,11 +15,15 @@
 // its end waits for what step t-1 requested and meets the barrier; rows past the segment and columns past the true head_dim
 // read as zero.  The selection words take the same way, each wave its own rows' into its own slots.
 //
-// What bounds it: with a selection the vector instructions (about 94 and 16 exponentials beside 16 MFMAs at head_dim 128, 32
-// of them the mask) and the power of the chip (1.75-1.9 GHz under this load); without one the softmax of tiles every row
-// attends whole drops the mask.  Same box, us, against the previous kernel (register staging, phases one after the other):
-// 32 768 tokens dense 1423 -> 1296, with a selection 1402 -> 1418; 8192 tokens with a selection 65 -> 62; head_dim 256, 16 384
-// tokens 219 -> 211; vision towers at head_dim 96 458 -> 367, at 64 342 -> 276.
+// What bounds it: the power of the chip (MFMA busy 0.61 of a CU's time without a selection, at 1.79 GHz) and, with a selection, the
+// vector instructions (about 92 and 16 exponentials beside 16 MFMAs at head_dim 128, 32 of them the mask); without one the softmax of
+// tiles every row attends whole drops the mask.  Both make every instruction beside the MFMAs count: a tile's buffer size comes from two
+// constants, its pieces follow one another under one buffer, operand addresses move on in place.  Same box, us, against a size formed per
+// piece, addresses formed per tile and eight waves per workgroup in large launches: 32 768 tokens dense 1289 -> 1229, with a selection
+// 1408 -> 1371; 8192 tokens with a selection 62.5 -> 59; 512 tokens 15.9 -> 15.1; head_dim 256, 16 384 tokens 210 -> 195; vision towers at
+// head_dim 72 354 -> 335, at 64 282 -> 269.  Four waves per workgroup, two workgroups per CU: eight waves that share each staged tile took
+// 1255 dense.  64 rows per wave, one wave per SIMD: level at 32 768 tokens (MFMA busy 0.52 at 1.95 GHz), slower in short launches.
+// At head_dim 256 the loop must not read spilled registers: such a read waits for every tile on its way into LDS (+ 20 %).
 #include "dsa_tile.h"
 
 template <int D, int NW>
@@ -70,46 +74,27 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         vvoff[i] = TL::source(wv * LPW + i, lane, (int)v_tok * 2, chunks);
     }
     const uint32_t lds0 = lds_address(dyn_lds);
-    // Addresses of the next tile to request, in scalar registers (the asm statements keep them there); what is left of the
-    // block's keys from its first row on, in bytes, bounds the buffer (the last row ends with its own elements: a token
-    // stride may be shorter than a row, or zero, in an expanded tensor; rows past the segment are then bytes of live rows,
-    // and masked as ever)
-    const int Lend = min(L, ntiles * 32);
+    // Addresses of the next tile to request, in scalar registers (the asm statements keep them there); the bytes of its rows that exist
+    // bound the buffer (the last row ends with its own elements: a token stride may be shorter than a row, or zero, in an expanded
+    // tensor; rows past the segment are then bytes of live rows, and masked as ever)
     auto next = [](const unsigned char *&p, int64_t step) __attribute__((always_inline)) {
         p += step;
         asm volatile("" : "+s"(p));
     };
-    auto left = [&](int tile, int tok_b) __attribute__((always_inline)) {
-        const int rows = max(min(Lend - tile * 32, 32), 0);
-        return (uint32_t)(rows ? (rows - 1) * tok_b + d_real * 2 : 0);
-    };
-    uint32_t kleft = left(0, (int)k_tok * 2), vleft = left(0, (int)v_tok * 2);
-    auto load_k_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(kptr, kleft), kvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)k_tok * 2,
-                          lds0 + (tile & 3) * TL::BYTES + TL::load_lds(wv * LPW + i));
-        if (i == LPW - 1) {
-            next(kptr, k_step);
-            kleft = left(tile + 1, (int)k_tok * 2);
-            asm volatile("" : "+s"(kleft));
-        }
-    };
-    auto load_v_piece = [&](int tile, int i) __attribute__((always_inline)) {
-        buffer_load_lds16(make_buffer_rsrc(vptr, vleft), vvoff[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)v_tok * 2,
-                          lds0 + (4 + (tile & 3)) * TL::BYTES + TL::load_lds(wv * LPW + i));
-        if (i == LPW - 1) {
-            next(vptr, v_step);
-            vleft = left(tile + 1, (int)v_tok * 2);
-            asm volatile("" : "+s"(vleft));
-        }
-    };
-    auto load_k = [&](int tile) __attribute__((always_inline)) {
+    const int gone = max(ntiles * 32 - L, 0);           // rows of the last tile that do not exist
+    const uint32_t k_full = 31 * (int)k_tok * 2 + d_real * 2, v_full = 31 * (int)v_tok * 2 + d_real * 2;
+    const uint32_t k_last = k_full - gone * (int)k_tok * 2, v_last = v_full - gone * (int)v_tok * 2;
+    auto load_tile = [&](const unsigned char *&p, const int (&first)[NV], int tile, int slot, uint32_t full, uint32_t last, int64_t tile_b) __attribute__((always_inline)) {
+        int voff[LPW];
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) load_k_piece(tile, i);
+        for (int i = 0; i < LPW; ++i) voff[i] = first[i % NV] + i / NV * NV * TL::LOAD_ROWS * (int)(tile_b / 32);
+        constexpr int P1 = LPW > 1 ? 1 : 0, P2 = LPW > 2 ? 2 : P1, P3 = LPW > 2 ? 3 : P2;
+        buffer_load_lds16_n<LPW, TL::load_lds(P1), TL::load_lds(P2) - TL::load_lds(P1), TL::load_lds(P3) - TL::load_lds(P2)>(
+            scalar_buffer_rsrc(p, tile < ntiles - 1 ? full : tile == ntiles - 1 ? last : 0u), voff, lds0 + slot * TL::BYTES + TL::load_lds(wv * LPW));
+        next(p, tile_b);
     };
-    auto load_v = [&](int tile) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < LPW; ++i) load_v_piece(tile, i);
-    };
+    auto load_k = [&](int tile) __attribute__((always_inline)) { load_tile(kptr, kvoff, tile, tile & 3, k_full, k_last, k_step); };
+    auto load_v = [&](int tile) __attribute__((always_inline)) { load_tile(vptr, vvoff, tile, 4 + (tile & 3), v_full, v_last, v_step); };
     unsigned char *const words = dyn_lds + 8 * TL::BYTES + wv * 1024;     // [tile % 4][lane]
     const int wq0 = __builtin_amdgcn_readfirstlane(min(qc0 + ((wv * 32) >> gshift), L - 1));   // the wave's first query
     const unsigned char *wptr = reinterpret_cast<const unsigned char *>(bitmap + (int64_t)(s0 + wq0) * ldw);
@@ -117,7 +102,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     auto load_w = [&](int tile) __attribute__((always_inline)) {
         if (HAS_IDX) {
             buffer_load_lds4(make_buffer_rsrc(wptr, 32 * ldw * 4), wvoff, lds0 + 8 * TL::BYTES + wv * 1024 + (tile & 3) * 256);
-            if (tile + 1 < ntiles) next(wptr, 4);        // (past the block's tiles: the last word again, never used)
+            next(wptr, tile + 1 < ntiles ? 4 : 0);       // (past the block's tiles: the last word again, never used)
         }
     };
     bf16x8 qB[KS];
@@ -136,22 +121,26 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     wait_vmcnt<0>();
     barrier_only();
 
-    int ka_[4], va_[4];                                 // operand addresses in the K tile of S(t+2) and in V(t)
-    auto k_addr = [&](int tile) __attribute__((always_inline)) {
+    lds_u8 *ka_[4], *va_[4];                            // operand addresses: of the K tile of S(t+2) and of V(t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ka_[i] = tl.rowq[i] + (tile & 3) * TL::BYTES;
-    };
-    auto v_addr = [&](int tile) __attribute__((always_inline)) {
+    for (int i = 0; i < 4; ++i) {
+        ka_[i] = (lds_u8 *)dyn_lds + tl.rowq[i];
+        va_[i] = (lds_u8 *)dyn_lds + tl.trq[i] + 4 * TL::BYTES;
+    }
+    auto advance = [&](lds_u8 *(&a)[4], int tile) __attribute__((always_inline)) {         // from tile - 1 to tile
+        const int by = tile & 3 ? TL::BYTES : -3 * TL::BYTES;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) va_[i] = tl.trq[i] + (4 + (tile & 3)) * TL::BYTES;
+        for (int i = 0; i < 4; ++i) {
+            a[i] += by;
+            asm volatile("" : "+v"(a[i]));
+        }
     };
     auto read_k = [&](int ks) __attribute__((always_inline)) {
-        return *reinterpret_cast<const bf16x8 *>(dyn_lds + ka_[TL::row_q(ks)] + TL::row_imm(ks));
+        return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(ka_[TL::row_q(ks)] + TL::row_imm(ks));
     };
     auto read_v = [&](int i) __attribute__((always_inline)) {             // MFMA i of P V: keys of half i / DT, d-tile i % DT
         const int pair = i / DT, dt = i % DT;
-        lds_u8 *p = (lds_u8 *)dyn_lds + va_[TL::tr_q(dt)];
-        return tr_pair(p + TL::tr_imm(dt, 2 * pair), p + TL::tr_imm(dt, 2 * pair + 1));
+        return tr_pair(va_[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair), va_[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair + 1));
     };
     // The keys of a tile this lane keeps, as they lie in memory; live(word): element vi then sits at bit 8*(vi/4) + vi%4
     const uint32_t row_mask = row_ok ? 0xffffffffu : 0u;
@@ -203,12 +192,9 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) s = mfma32(ka[ks], qB[ks], s);
     };
-    k_addr(0);
     gemm_s(sE);
-    if (ntiles > 1) {
-        k_addr(1);
-        gemm_s(sO);
-    }
+    advance(ka_, 1);
+    if (ntiles > 1) gemm_s(sO);
     {
         float psum = INFINITY;                          // (no reference yet: the maximum is searched for)
         if (!row_ok) psum = 0.f;
@@ -221,18 +207,17 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     constexpr int KA = KS % 5 == 0 ? 5 : KS % 4 ? 3 : 4, VA = NP % 4 ? 3 : 4;   // (divide KS and NP: an operand keeps its register from step to step)
     static_assert(KS % KA == 0 && NP % VA == 0);
     bf16x8 kr[KA], vr[VA];                              // operands of the next MFMA pairs
-    k_addr(2);
-    v_addr(0);
+    advance(ka_, 2);
 #pragma unroll
     for (int i = 0; i < KA; ++i) kr[i] = read_k(i);
 #pragma unroll
     for (int i = 0; i < VA; ++i) vr[i] = read_v(i);
     uint32_t word_next = word_of(1);                    // (one-tile blocks never use it)
 
-    // piece r of what step t requests: K(t+5), V(t+3) and the selection words of tile t+4
+    // what step t requests: K(t+5), V(t+3), the selection words of tile t+4
     auto request = [&](int t_, int r_) __attribute__((always_inline)) {
-        if (r_ < LPW) load_k_piece(t_ + 5, r_);
-        else if (r_ < 2 * LPW) load_v_piece(t_ + 3, r_ - LPW);
+        if (r_ == 0) load_k(t_ + 5);
+        else if (r_ == 1) load_v(t_ + 3);
         else load_w(t_ + 4);
     };
     // Step t: O += P(t) V(t) with `p`; softmax of tile t+1 from `s` into `pn` (SM); S(t+2) into `sn` (NEXT).
@@ -280,16 +265,16 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
             // this step's requests, spread over its first half: one after the other they would queue for the way into LDS
 #pragma unroll
-            for (int r_ = 0; r_ < LPS; ++r_)
-                if (REQ && r_ * (NP / 2) / LPS == i) request(t_, r_);
+            for (int r_ = 0; r_ < (HAS_IDX ? 3 : 2); ++r_)
+                if (REQ && r_ * (NP / 2) / 3 == i) request(t_, r_);
             // refill: the operand a few pairs on, of this step's tiles or, past their end, of the next step's
-            if (i == NP - VA && SM) v_addr(t_ + 1);
+            if (i == NP - VA && SM) advance(va_, t_ + 1);
             if (i + VA < NP || SM) vr[i % VA] = read_v((i + VA) % NP);
             if (SM) behind(2 * i);
             else __builtin_amdgcn_sched_barrier(0);
             if (NEXT && i < KS) {
                 snew = mfma32(kr[i % KA], qB[i], i == 0 ? zero16() : snew);
-                if (i == KS - KA) k_addr(t_ + 3);
+                if (i == KS - KA) advance(ka_, t_ + 3);
                 kr[i % KA] = read_k((i + KA) % KS);
                 if (i == 0 && MASKED) word_next = word_of(t_ + 2);
             }
@@ -362,10 +347,11 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     }
 }
 
-template <int D, bool HAS_IDX, int NW>
-static hipError_t launch_fwd_n(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
+template <int D, bool HAS_IDX>
+static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
                                void *out, float *lse) {
+    constexpr int NW = 4;
     const auto kernel = &dsa_tile_fwd_kernel<D, HAS_IDX, NW>;
     constexpr size_t lds = fwd_lds_bytes<D, NW>(HAS_IDX);
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -375,21 +361,6 @@ static hipError_t launch_fwd_n(hipStream_t stream, const void *q, const void *k,
                        st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, (bf16_t *)out, lse);
     return hipSuccess;
 }
-template <int D, bool HAS_IDX>
-static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
-                               void *out, float *lse) {
-    // At head_dim 80 to 128 eight waves share each staged tile - except in launches of a few rounds of workgroups, which
-    // are bound by what a workgroup pays before its first tile and after its last: there two four-wave workgroups per CU
-    // overlap those parts.
-    if constexpr (D > 64 && D <= 128) {
-        const int64_t blocks = ((int64_t)T / ((32 * 8) >> gshift) + N + 1) * Hkv;
-        if (blocks > DSA_BATCH_ORDER_MAX_BLOCKS)
-            return launch_fwd_n<D, HAS_IDX, 8>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
-    }
-    return launch_fwd_n<D, HAS_IDX, 4>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, out, lse);
-}
-
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
 // without a bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
 extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
