@@ -28,7 +28,7 @@ hipError_t dsa_launch_gather_dq(const void *dout, const void *q, const void *k, 
                                 const float *delta, const int32_t *idx, const int32_t *n, const int32_t *cu, int N,
                                 int T, int Hq, int Hkv, int D, int K, float scale, int pos_min, void *dq,
                                 hipStream_t stream);
-hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore, const float *grad,
+hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n, const float *dscore, const float *grad,
                                   const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N, int T, int Hi,
                                   int Di, int K, float cscale, void *dq_idx, void *dk_idx, void *dw, int dw_bf16, float *partial,
                                   hipStream_t stream, hipStream_t stream_q);
@@ -512,7 +512,7 @@ extern "C" int dsa_indexer_bwd_scaled(const void *q_idx, const void *k_idx, cons
         sq = ov->aux;
     }
     int rc = DSA_OK;
-    e = dsa_launch_indexer_bwd(q_idx, k_idx, w_idx, dscore, grad, bitmap, prefix, w_f32, ldw, cu, N, T, Hi, Di, K, scale, dq_idx, dk_idx, dw,
+    e = dsa_launch_indexer_bwd(q_idx, k_idx, w_idx, idx, n, dscore, grad, bitmap, prefix, w_f32, ldw, cu, N, T, Hi, Di, K, scale, dq_idx, dk_idx, dw,
                                dw_dtype == DSA_DTYPE_BF16, partial, st, sq);
     if (e != hipSuccess) rc = hip_fail(e, "indexer backward launch");
     if (ov) {

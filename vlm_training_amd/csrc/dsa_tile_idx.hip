@@ -5,6 +5,7 @@
 //     G[t,h,s]   = dscore[t,s] * w[t,h] * (r > 0)
 //     dq_idx[t,h,:] = c * sum_s G[t,h,s] k_idx[s,:]      dw[t,h] = c * sum_s dscore[t,s] relu(r[t,h,s])
 //     dk_idx[s,:]   = c * sum_t sum_h G[t,h,s] q_idx[t,h,:]
+// (the query side of a selection that is short against the segments: dsa_tile_idxg.hip)
 // Query side: rows = (query, indexer head), padded to 32 or 64 rows per query so that the 32 rows of a wave belong to one query;
 // the wave walks the key tiles: S^T = K Q^T, G^T on the C layout, dQ^T += K^T G^T.  Key side: a wave owns 32 keys (rows in
 // registers) and walks the later queries in tiles of 32 heads of one query: S = Q K^T, G on the C layout, dK^T += Q^T G.  Every
@@ -435,8 +436,17 @@ static int idxk_chunk(int T, int Di, int ldw) {
     while ((size_t)((ldw * 32 + c - 1) / c) * T * Di * 4 > ((size_t)5 << 28) && c < (1 << 20)) c *= 2;
     return c;
 }
+extern "C" hipError_t dsa_launch_indexer_bwd_gather(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
+                                                    const float *dscore, const float *grad, int ldw, const int32_t *cu, int N, int T, int Hi, int Di, int K,
+                                                    float cscale, void *dq_idx, void *dw, int dw_bf16, hipStream_t stream);   // dsa_tile_idxg.hip
+// The query side over the selected keys alone (dsa_tile_idxg.hip) instead of over every causal tile: where the longest segment is this
+// much longer than the selection.  Whole backward, us, tiles against gather, 64 heads of 128: selection of 2048 keys in segments of 2048
+// 609 / 646, 3072: 1246 / 1200, 4096: 2146 / 1951, 5120: 2351 / 2016; 16 384 tokens in one 7441 / 4805; 512 keys in segments of 1536
+// 518 / 426; 256 keys in segments of 300 197 / 250.  32 heads (a tile is half the matrix work for the same keys) of 64: 1024 keys in
+// segments of 2048 193 / 196, 3072: 393 / 353, 4096: 646 / 529; of 700 to 1800: 146 / 163; of 128, in 2048: 331 / 362.
+static bool idx_bwd_gathers(int Hi, int K, int longest) { return 2 * (int64_t)longest >= (Hi > 32 ? 3 : 6) * (int64_t)K; }
 template <int D, int GS>
-static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const void *k_idx, const void *w_idx, const float *w_f32, const float *dscore,
+static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n, const float *w_f32, const float *dscore,
                              const float *grad, const uint32_t *bitmap, const int32_t *prefix, int ldw, const int32_t *cu, int N, int T, int Hi,
                              int K, float cscale, void *dq_idx, void *dk_idx, void *dw, int dw_bf16, float *partial, hipStream_t stream_q) {
     // (waves that share the staged key tiles: two workgroups of four on a CU do not meet at each other's barriers, so the gating of
@@ -455,6 +465,8 @@ static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const 
                        (const bf16_t *)k_idx, w_f32, dscore, grad, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, chunk, partial);
     hipLaunchKernelGGL(dsa_idxk_reduce_kernel, dim3((unsigned)((T + 7) / 8)), dim3(256), 0, stream, partial, cu, N, T, D,
                        chunk, ldw * 32, (bf16_t *)dk_idx);
+    if (idx_bwd_gathers(Hi, K, ldw * 32))
+        return dsa_launch_indexer_bwd_gather(q_idx, k_idx, w_idx, idx, n, dscore, grad, ldw, cu, N, T, Hi, D, K, cscale, dq_idx, dw, dw_bf16, stream_q);
     const dim3 gq((unsigned)((int64_t)T / ((32 * NW) >> GS) + N + 1));
     hipLaunchKernelGGL((dsa_tile_idxq_kernel<D, GS, NW>), gq, dim3(64 * NW), (idxq_lds_bytes<D, NW>()), stream_q, (const bf16_t *)q_idx,
                        (const bf16_t *)k_idx, (const bf16_t *)w_idx, dscore, grad, bitmap, ldw, cu, N, T, Hi, K, cscale,
@@ -466,13 +478,13 @@ extern "C" size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw) {
     return (size_t)((ldw * 32 + chunk - 1) / chunk) * T * Di * 4;
 }
 // w_f32: T * 64 floats of scratch; grad: one fp32 factor of every gradient on the device, or null
-extern "C" hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const float *dscore, const float *grad,
-                                             const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N,
+extern "C" hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
+                                             const float *dscore, const float *grad, const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N,
                                              int T, int Hi, int Di, int K, float cscale, void *dq_idx, void *dk_idx,
                                              void *dw, int dw_bf16, float *partial, hipStream_t stream, hipStream_t stream_q) {
     if (Hi < 1 || Hi > 64 || !(Di == 64 || Di == 128)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(dsa_bitmap_prefix_kernel, dim3(T), dim3(64), 0, stream, bitmap, ldw, prefix, (const bf16_t *)w_idx, Hi, w_f32);
-#define IDX_BWD(D_, GS_) launch_idx_bwd_i<D_, GS_>(stream, q_idx, k_idx, w_idx, w_f32, dscore, grad, bitmap, prefix, ldw, cu, N, T, Hi, K, \
+#define IDX_BWD(D_, GS_) launch_idx_bwd_i<D_, GS_>(stream, q_idx, k_idx, w_idx, idx, n, w_f32, dscore, grad, bitmap, prefix, ldw, cu, N, T, Hi, K, \
                                                    cscale, dq_idx, dk_idx, dw, dw_bf16, partial, stream_q)
     if (Di == 128) return Hi > 32 ? IDX_BWD(128, 6) : IDX_BWD(128, 5);
     return Hi > 32 ? IDX_BWD(64, 6) : IDX_BWD(64, 5);
