@@ -558,7 +558,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     OverlapCtx *ov = nullptr;
     const int ov_mode = g_bwd_overlap.load(std::memory_order_relaxed);
     if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0) {
-        const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);
+        const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);     // (head_dim 256: one workgroup per CU, half as many fill it)
         const double work = (double)T * max_seqlen * Hq * D;
         if (ov_mode == 2 || (dkv_wg <= DSA_BWD_OVERLAP_MAX_WG && work >= (causal ? DSA_BWD_OVERLAP_MIN_WORK : DSA_BWD_OVERLAP_MIN_WORK_FULL))) {
             ov_lock = std::unique_lock<std::mutex>(g_overlap_mu);
