@@ -36,7 +36,8 @@ __global__ __launch_bounds__(64, 1) void dsa_tile_idxg_kernel(
     const uint32_t lds0 = lds_address(dyn_lds);
     const buffer_rsrc keys = make_buffer_rsrc(k_idx + (int64_t)s0 * D, (int64_t)L * 2 * D);
     const buffer_rsrc ids = make_buffer_rsrc(idx + (int64_t)t * K, (int64_t)n * 4), grads = make_buffer_rsrc(dscore + (int64_t)t * K, (int64_t)n * 4);
-    const int row = lane / TL::CPR, key0 = ((lane % TL::CPR) ^ TL::xor_of(row)) * 16 - s0 * 2 * D;    // (indices outside the segment leave the buffer)
+    const int row = lane / TL::CPR;
+    const uint32_t key0 = ((lane % TL::CPR) ^ TL::xor_of(row)) * 16 - (uint32_t)s0 * (2 * D);    // (indices outside the segment leave the buffer)
     auto load_ids = [&](int tile) __attribute__((always_inline)) { buffer_load_lds4(ids, tile * 128 + lane * 4, lds0 + IDS + (tile & 7) * 256); };
     auto load_grads = [&](int tile) __attribute__((always_inline)) { buffer_load_lds4(grads, tile * 128 + lane * 4, lds0 + GRADS + (tile & 3) * 256); };
     int voff[LOADS];                                     // the lane's 16 bytes of each piece of the tile requested next
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(64, 1) void dsa_tile_idxg_kernel(
     };
     auto find_keys = [&](int tile, int p) __attribute__((always_inline)) {
         asm volatile("" : "+v"(id[p]));                  // (read in any case: no branch)
-        voff[p] = tile * 32 + p * TL::LOAD_ROWS + row < n ? id[p] * (2 * D) + key0 : (int)0x80000000;        // (past the list: zeros)
+        voff[p] = tile * 32 + p * TL::LOAD_ROWS + row < n ? (int)((uint32_t)id[p] * (2 * D) + key0) : (int)0x80000000;        // (past the list: zeros)
     };
     auto load_keys = [&](int tile) __attribute__((always_inline)) {
         constexpr int P1 = TL::load_lds(1), P2 = TL::load_lds(2) - P1, P3 = TL::load_lds(3) - TL::load_lds(2);
