@@ -391,8 +391,11 @@ __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N
     if (mode == 2 && maxnt <= DSA_ORDER_SPLIT_MAX_TILES) {
         // A tile of rank r is cut into ceil((128 r / qb) / pb) pieces of equal length.  pb = `share8` eighths of the steps
         // that a balanced launch gives each of its `slots` concurrent workgroups, and `extra` (a piece costs as much as 7 to 9 steps
-        // besides its own, and its partial sums), or the first of the larger candidates (a quarter of an octave apart) whose entries and
-        // partial sums fit; a wave counts two candidates.
+        // besides its own, and its partial sums), or the first of the larger candidates (an eighth of an octave apart) whose entries and
+        // partial sums fit.  Launches of one workgroup per CU start from a quarter of `extra`, up to the usual pb only with candidates
+        // whose pieces all run at once.  Key side with the list and the sum over pieces, us, against the usual pb alone and candidates a
+        // quarter of an octave apart: 2048 tokens in four segments at head_dim 256 70 -> 57, 16 384 in 33 330 -> 310, 4000 in three 114 ->
+        // 98; one segment of 4000: level; two workgroups per CU (8192 tokens in seven segments at 128): 131 -> 143, so not there.
         if (tid == 0) sum_a = 0;
         __syncthreads();
         const int spt = 128 / qb, longest = maxnt * spt;          // steps of a rank
@@ -403,25 +406,32 @@ __device__ __forceinline__ void tile_order(const int32_t *__restrict__ cu, int N
         }
         __syncthreads();
         const int64_t ideal = ((int64_t)sum_a * wg_per_tile + o_.slots - 1) / o_.slots;
-        const int pb0 = max((int)min(ideal * o_.share8 / 8 + o_.extra, (int64_t)longest), max(8, 32 / qb));
-        auto candidate = [&](int k) { return (pb0 * (4 + (k & 3)) << (k >> 2)) / 4; };
-        const int ln = tid & 63, wvi = tid >> 6;
-        for (int k = wvi; k < 32; k += 16) {
-            const int pbk = candidate(k);
+        const int64_t even = ideal * o_.share8 / 8 + o_.extra;
+        const int pb0 = max((int)min(ideal * o_.share8 / 8 + (o_.slots > 256 ? o_.extra : o_.extra / 4), (int64_t)longest), max(8, 32 / qb));
+        auto candidate = [&](int k) { return (pb0 * (8 + (k & 7)) << (k >> 3)) / 8; };
+        {
+            const int k = tid >> 4, pbk = candidate(k);              // 16 threads a candidate
+            const float inv = 1.f / (float)pbk;
             int ni = 0, nm = 0;
-            for (int r = 1 + ln; r <= maxnt; r += 64) {
-                const int np = (r * spt + pbk - 1) / pbk;
+            for (int r = 1 + (tid & 15); r <= maxnt; r += 16) {
+                const int up = r * spt + pbk - 1;                    // (below 2^24: a float holds it)
+                int np = (int)((float)up * inv);
+                np += (np + 1) * pbk <= up;
+                np -= np * pbk > up;
                 ni += cnt[r] * np;
                 if (np > 1) nm += cnt[r] * np;
             }
-            ni = wave_sum_i(ni);
-            nm = wave_sum_i(nm);
-            if (ln == 0) part[k] = ni <= item_cap && ni <= cap && nm <= slot_cap;
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) {
+                ni += __shfl_xor(ni, off, 64);
+                nm += __shfl_xor(nm, off, 64);
+            }
+            if ((tid & 15) == 0)
+                part[k] = ni <= item_cap && ni <= cap && nm <= slot_cap && (pbk >= min(even, (int64_t)longest) || (int64_t)ni * wg_per_tile <= o_.slots);
         }
         __syncthreads();
-        int pb = 1 << 30;
-        for (int k = 31; k >= 0; --k)
-            if (part[k]) pb = candidate(k);
+        const uint64_t fits = __ballot(part[tid & 63] != 0);
+        const int pb = fits ? candidate(__ffsll((unsigned long long)fits) - 1) : 1 << 30;
         __syncthreads();
         // thread tid owns rank r = tid + 1.  Entries are listed by length (then by rank, then by segment): its entries, partial slots
         // and cut tiles start behind those of the ranks in front of it.
