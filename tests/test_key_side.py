@@ -147,3 +147,29 @@ def test_operands_on_odd_addresses_give_the_gradients(D, Hq, Hkv, lens, K):
         # the rounding remainder of P decided per 32 keys)
         for name, a, b in zip(("dk", "dv"), got[1:], want[1:]):
             assert_close_bf16(a, b, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,nseg", [(64, 1), (64, 40), (96, 1), (128, 1), (256, 1), (256, 40)])
+def test_score_gradients_of_the_key_side_come_from_unrounded_probabilities(D, nseg, dtype):
+    """Every probability is 1/96 (keys orthogonal to the queries), which bf16 rounds up by 2e-3; delta is 0 and the terms dS = P dP of a
+    key all have its sign, so a rounded P would be a bias of 2e-3 in every element of dK.  What remains is rounding: of dS (2^-8 at most,
+    96 independent terms per key) and of dK itself (2^-8 at most, once for the two keys of a pair): an element is off by 2^-7 at most, the
+    mean over the 48 pairs of eight kv heads has a standard deviation of 2^-8 / sqrt(3 * 384) = 1.2e-4, and 8e-4 is more than six of them.
+    One segment and forty: 32 and, up to head_dim 128, 64 keys per wave."""
+    print("unrounded P", D, nseg, dtype, flush=True)
+    g = torch.Generator().manual_seed(D + nseg)
+    L, H = 96, 8
+    T = L * nseg
+    q, k, v, do = (torch.zeros(T, H, D) for _ in range(4))
+    q[..., 0] = 1.0
+    v[::2, :, 1] = (1 + torch.rand(T // 2, H, generator=g)).bfloat16().float()
+    v[1::2, :, 1] = -v[::2, :, 1]
+    do[..., 1] = (1 + torch.rand(T, H, generator=g)).bfloat16().float()
+    got = [x.to(dtype).to(DEV).requires_grad_(True) for x in (q, k, v)]
+    cu = torch.arange(0, T + 1, L, dtype=torch.int32, device=DEV)
+    ops.dsa_varlen_attn(*got, cu, L, softmax_scale=1.0, causal=False).backward(do.to(dtype).to(DEV))
+    want = v[..., 1].double() * do[..., 1].double().view(nseg, L, H).sum(1).repeat_interleave(L, 0) / L
+    ratio = got[1].grad[..., 0].double().cpu() / want - 1
+    assert ratio.abs().max() <= 2.0 ** -7 and abs(ratio.mean().item()) <= 8e-4, (ratio.abs().max(), ratio.mean())

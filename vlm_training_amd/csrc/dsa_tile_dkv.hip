@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     constexpr bool TIGHT = D == 128 && KG == 2;
     constexpr int AHEAD = TIGHT ? 2 : 4;                 // operands read ahead: four MFMAs or more
     constexpr bool PAIRS = KG == 2 && !TIGHT;            // operands waited for and refilled in pairs
-    constexpr bool KEEP_P = D <= (KG == 1 ? 128 : 80);                    // P stays in fp32 until dS is formed (else its bf16 form is unpacked)
+    constexpr bool KEEP_P = KG == 1 || D <= 80;          // P stays in fp32 until dS is formed (else its bf16 form is unpacked)
     static_assert(TL::LOADS % NW == 0 && (RING & (RING - 1)) == 0 && AHEAD <= NP, "");
     extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];
 
