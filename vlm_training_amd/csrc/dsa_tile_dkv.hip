@@ -10,11 +10,12 @@
 // workgroups a CU), 32 keys at head_dim 256 and in launches of few workgroups (four waves, one workgroup: dkv_key_groups).  The sums of
 // dK and dV fill up to 256 accumulation registers, K and V rows 128 of the others.  An operand read from LDS feeds the MFMAs of both key groups, P and dS never leave
 // the wave, nothing is formed twice.  Step s runs dV(s) mixed with S(s+1), the products of dS(s) behind them, then dK(s) mixed with
-// dP(s+1), P(s+1) behind them in three stages (logit, exponential, packing) that do not wait for each other.  q and dO blocks, row
+// dP(s+1), P(s+1) behind them in three stages (logit, exponential, packing) that do not wait for each other.  P stays in fp32 until dS is
+// formed (from its bf16 form dK is 3.0e-3 off 64 bits instead of 2.5e-3, and unpacking that is another 32 instructions).  q and dO blocks, row
 // data and selection words go from memory straight into LDS, two to three steps ahead, one barrier per step.
 //
-// What bounds it: the issue of one instruction stream per SIMD - at head_dim 128 64 MFMAs (2048 clocks) beside about 230 vector
-// instructions (245 with a selection), 60 LDS reads and as many scalar ones take 3000 - and the chip's power (MFMA busy 0.69 of a CU's
+// What bounds it: the issue of one instruction stream per SIMD - at head_dim 128 64 MFMAs (2048 clocks) beside about 160 vector
+// instructions (210 with a selection), 60 LDS reads and as many scalar ones take 3000 - and the chip's power (MFMA busy 0.69 of a CU's
 // time, 1.85 GHz under this load).  Same box, us, against the kernels before (eight waves; at head_dim 128 one wave per chain, P handed
 // over in LDS; at 256 each half of head_dim formed S and dP; q and dO through registers): 32 768 tokens dense 2630 -> 2200, with a
 // selection 2680 -> 2285; head_dim 256, 16 384 tokens in short segments 548 -> 327; towers at head_dim 64 / 72, whole backward
@@ -28,7 +29,7 @@
 
 // KG: groups of 32 keys per wave
 template <int D, int KG> constexpr int dkv_ring() { return D == 128 && KG == 1 ? 8 : 4; }                // q/dO blocks in LDS
-template <int D, int KG> constexpr int dkv_aux_bytes() { return dkv_ring<D, KG>() * 512 + 512 + (D == 128 && KG == 2 ? 3072 : 0); }
+template <int D, int KG> constexpr int dkv_aux_bytes() { return dkv_ring<D, KG>() * 512 + 512 + (D == 128 && KG == 2 ? 5120 : 0); }
 template <int D, int KG> constexpr size_t dkv_lds_bytes() {
     return dkv_ring<D, KG>() * 2 * (size_t)DirectTile<D>::BYTES + 4 / KG * (size_t)dkv_aux_bytes<D, KG>();
 }
@@ -46,12 +47,11 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     constexpr int RPW = Gp < 4 ? Gp : 4;                 // neighbouring rows of a lane that are one query's
     constexpr int SLOT = 2 * TL::BYTES;                  // q block | dO block
     // LDS of a wave: RING x (lse, delta | selection words), 2 x row data as the chains start from it, and at head_dim 128, where the
-    // loop has no registers left for them, the lane's source offsets and the last K operand of each key group
+    // loop has no registers left for them, the lane's source offsets and the last K and V operand of each key group
     constexpr int AUX = dkv_aux_bytes<D, KG>();
     constexpr bool TIGHT = D == 128 && KG == 2;
     constexpr int AHEAD = TIGHT ? 2 : 4;                 // operands read ahead: four MFMAs or more
     constexpr bool PAIRS = KG == 2 && !TIGHT;            // operands waited for and refilled in pairs
-    constexpr bool KEEP_P = KG == 1 || D <= 80;          // P stays in fp32 until dS is formed (else its bf16 form is unpacked)
     static_assert(TL::LOADS % NW == 0 && (RING & (RING - 1)) == 0 && AHEAD <= NP, "");
     extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];
 
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
         load_rows(b + 1);
         load_words(b + 1);
     }
-    unsigned char *const klast = aux + RING * 512 + 1536 + lane * 16;
+    unsigned char *const klast = aux + RING * 512 + 1536 + lane * 16, *const vlast = klast + 2048;
     bf16x8 kB[KG][KS], vB[KG][KS];
 #pragma unroll
     for (int g = 0; g < KG; ++g) {
@@ -164,7 +164,10 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
             kB[g][ks] = there ? load_bf16x8(k + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
             vB[g][ks] = there ? load_bf16x8(v + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
         }
-        if (TIGHT) *reinterpret_cast<bf16x8 *>(klast + g * 1024) = kB[g][KS - 1];
+        if (TIGHT) {
+            *reinterpret_cast<bf16x8 *>(klast + g * 1024) = kB[g][KS - 1];
+            *reinterpret_cast<bf16x8 *>(vlast + g * 1024) = vB[g][KS - 1];
+        }
     }
     f32x16 dkacc[KG][DT], dvacc[KG][DT];
 #pragma unroll
@@ -208,7 +211,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     constexpr float DKV_SPLIT_MIN = 0.015625f;
     f32x16 pacc[KG];                                     // dP of the block ahead
     uint32_t pw[KG][8];                                  // its P in bf16
-    float pf[KG][KEEP_P ? 16 : 1];
+    float pf[KG][16];                                    // and in fp32, for dS
     bf16x8 op[AHEAD];
     lds_u8 *aR[4], *aT[4];                               // operand addresses: row-wise of block s+1, transposed of block s
     {
@@ -283,7 +286,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
             for (int g = 0; g < KG; ++g) snew[g] = rows_init(s + 1, 0);
         }
         // ---- X ----
-        bf16x8 kl[KG];
+        bf16x8 kl[KG], vl[KG];
         uint32_t dw[KG][8];
         float dsv[2 * KG * 16];
         constexpr int E = 16 * KG, SX = SL - 2;          // dS: product behind MFMA 1 + u, packed behind the next
@@ -312,9 +315,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
                     for (int e = E * u / SX; e < E * (u + 1) / SX; ++e) {
                         if (e >= E) continue;
                         const int ge = e / 16, vi = e % 16;
-                        const uint32_t w = pw[ge][vi >> 1];
-                        const float p = KEEP_P ? pf[ge][KEEP_P ? vi : 0] : __uint_as_float(vi & 1 ? w & 0xffff0000u : w << 16);
-                        dsv[e] = p * pacc[ge][vi];
+                        dsv[e] = pf[ge][vi] * pacc[ge][vi];
                         asm volatile("" : "+v"(dsv[e]));
                     }
 #pragma unroll
@@ -363,12 +364,13 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
             for (int g = 0; g < KG; ++g) {
                 const int i = PO::index(m), n = m * KG + g, u = n - 1, mm = NX + m;
                 if (PO::is_row(m)) {
-                    pnew[g] = mfma32(op[mm % AHEAD], vB[g][i], pnew[g]);
+                    pnew[g] = mfma32(op[mm % AHEAD], TIGHT && i == KS - 1 ? vl[g] : vB[g][i], pnew[g]);
                 } else {
                     const u32x4 w = {dw[g][4 * (i / DT)], dw[g][4 * (i / DT) + 1], dw[g][4 * (i / DT) + 2], dw[g][4 * (i / DT) + 3]};
                     mfma32_agpr(dkacc[g][i % DT], op[mm % AHEAD], __builtin_bit_cast(bf16x8, w), !NEXT || (UNALIGNED && i >= DT));
                 }
                 if (g == KG - 1) refill(mm);
+                if (TIGHT && m == NX - 3) vl[g] = *reinterpret_cast<const bf16x8 *>(vlast + g * 1024);
                 if (NEXT && u >= 0) {
 #pragma unroll
                     for (int e = E * u / SY; e < E * (u + 1) / SY; ++e) {
@@ -396,22 +398,18 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
             }
         }
         if (NEXT) {
-            if (KEEP_P) {
 #pragma unroll
-                for (int e = 0; e < E; ++e) pf[e / 16][KEEP_P ? e % 16 : 0] = y[e];
-            }
+            for (int e = 0; e < E; ++e) pf[e / 16][e % 16] = y[e];
             // dV also takes what bf16 rounds off the larger probabilities: few keys per query and many rows in one key pile that
-            // rounding up.  Wave-uniform and rare: P is formed again.
+            // rounding up.  Wave-uniform and rare.
             if (__builtin_amdgcn_ballot_w64(pm >= DKV_SPLIT_MIN) != 0ull) {
 #pragma unroll
                 for (int g = 0; g < KG; ++g) {
                     float lo[16];
-                    if (!KEEP_P) asm volatile("" : "+v"(snew[g]));     // (left to itself the compiler keeps the first P in registers)
 #pragma unroll
                     for (int vi = 0; vi < 16; ++vi) {
                         const uint32_t w = pn[g][vi >> 1];
-                        if (!KEEP_P && HAS_IDX && vi % 4 == 0) words(16 * g + vi);
-                        lo[vi] = (KEEP_P ? y[16 * g + vi] : fast_exp2(logit(16 * g + vi))) - __uint_as_float(vi & 1 ? w & 0xffff0000u : w << 16);
+                        lo[vi] = y[16 * g + vi] - __uint_as_float(vi & 1 ? w & 0xffff0000u : w << 16);
                     }
                     bf16x8 l0 = pack8(lo), l1 = pack8(lo + 8);
                     asm volatile("s_nop 1" : "+v"(l0), "+v"(l1));
