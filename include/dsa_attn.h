@@ -141,6 +141,7 @@ size_t dsa_indexer_bwd_workspace_bytes(int T, int Di, int max_seqlen);
  * varlen_attn(..., window_size=(-1,-1)) (models/qwen3_vl/model.py:423-428, models/qwen3_5/model.py:388-393).
  * head_dim D: 64, 128 or 256; with idx == NULL also 96 (dsa_dense_fwd_strided and dsa_dense_bwd_rows take rows of any
  * multiple of 8 without padding: the 72-wide heads of the 1152 / 16 vision towers).
+ * softmax_scale: any finite value, here and in every call below.
  */
 int dsa_attn_fwd(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n,
                  const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale,

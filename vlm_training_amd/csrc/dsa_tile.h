@@ -280,6 +280,9 @@ static inline int group_shift(int Hq, int Hkv) {
     while ((1 << gshift) < G) ++gshift;
     return gshift;
 }
+// The factor of the logits for a softmax scale: kernels that divide by it, or mask in front of it, cannot take one at or next to zero.  At
+// 2^-80 instead a logit below 2^40 is below 2^-40, which the exponential takes for zero as well; gradients take the scale itself.
+static inline float logit_scale(float scale) { return scale > -0x1p-80f && scale < 0x1p-80f ? 0x1p-80f : scale; }
 // Rows of d_real elements, a multiple of 8: without a selection the kernel of the next head_dim of 64, 80, 96, 128 reads and writes
 // such rows where they lie (80: five k-steps instead of six for the S and dP of 72- and 80-wide vision heads)
 static inline int dense_kernel_dim(int d_real) { return d_real <= 64 ? 64 : d_real <= 80 ? 80 : d_real <= 96 ? 96 : d_real <= 128 ? 128 : d_real; }

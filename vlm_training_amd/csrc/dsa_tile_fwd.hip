@@ -29,7 +29,10 @@
 template <int D, int NW>
 constexpr size_t fwd_lds_bytes(bool has_idx) { return 8 * (size_t)DirectTile<D>::BYTES + (has_idx ? NW * 4 * 256 : 0); }
 
-template <int D, bool HAS_IDX, int NW>
+// NEG: the softmax scale is negative.  A masked key's logit is -inf in front of the scale, and the largest one is searched for there, so
+// the kernel's scale is positive and the sign goes into q (an instance of its own: at head_dim 256 as little as a test of the sign in front
+// of the loop made it spill).
+template <int D, bool HAS_IDX, int NW, bool NEG>
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
@@ -108,7 +111,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     bf16x8 qB[KS];
     const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
+    for (int ks = 0; ks < KS; ++ks) {
+        qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
+        if (NEG) qB[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, qB[ks]) ^ 0x80008000u);
+    }
     load_k(0); load_w(0); load_k(1); load_w(1); load_v(0); load_k(2); load_w(2); load_v(1); load_k(3); load_w(3); load_v(2);
 
     TL tl;
@@ -349,16 +355,16 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 
 template <int D, bool HAS_IDX>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float sl2, int pos_split, int causal,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
-    const auto kernel = &dsa_tile_fwd_kernel<D, HAS_IDX, NW>;
+    const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false>;
     constexpr size_t lds = fwd_lds_bytes<D, NW>(HAS_IDX);
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
-                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, sl2, pos_split, causal, (bf16_t *)out, lse);
+                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, causal, (bf16_t *)out, lse);
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
@@ -368,9 +374,9 @@ extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const vo
                                           int pos_split, int causal, void *out, float *lse, hipStream_t stream) {
     int gs = 0;
     while ((1 << gs) < Hq / Hkv) ++gs;
-    const float sl2 = scale * LOG2E_F;
+    scale = logit_scale(scale);
     hipError_t e = hipErrorInvalidValue;
-#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, sl2, pos_split, causal, out, lse)
+#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, causal, out, lse)
     if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
         else if (d_real <= 128) FWD_CASE(128, true);
