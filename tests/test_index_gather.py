@@ -43,3 +43,30 @@ def test_query_side_over_the_selected_keys(Hi, Di, lens, K):
     # sums of n products in fp32: n 2^-24 of their absolute sum, an element of S that rounds across zero adds less than 2^-20 of its terms
     bound = (K + 64) * 2.0 ** -24 * scale * dscore.abs().max() * (q.double().norm(dim=2) * k.double().norm(dim=1).max()) * max(K, 1) ** 0.5
     assert ((dw.double().cpu() - want_w).abs() <= bound + 1e-6).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hi,Di,K", [(64, 128, 64), (40, 64, 64), (32, 128, 32), (9, 64, 32)])
+def test_a_segment_takes_its_kernel_whatever_it_is_packed_with(Hi, Di, K):
+    """Selected keys alone or every tile is decided by a segment's own length (96 here): its gradients are the same to the bit in any batch
+    and under any bound of the longest segment."""
+    print("index gather, packed", Hi, Di, K, flush=True)
+    g = torch.Generator().manual_seed(Hi + Di)
+    lens = (90, 300, 95, 96, 1, 97, 33)
+    T, cu = sum(lens), [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    q, k, w = (torch.randn(*s, generator=g).mul_(0.5).bfloat16().to(DEV) for s in ((T, Hi, Di), (T, Di), (T, Hi)))
+    dscore = torch.randn(T, K, generator=g).to(DEV)
+
+    def grads(a, b, offsets, bound):
+        offs = torch.tensor(offsets, dtype=torch.int32, device=DEV)
+        idx, n = ops.index_topk(q[a:b], k[a:b], w[a:b], offs, bound, K)
+        dq, _, dw = ops.indexer_bwd(q[a:b], k[a:b], w[a:b], idx, n, dscore[a:b], offs, bound)
+        return dq, dw
+
+    packed, loose = grads(0, T, cu, max(lens)), grads(0, T, cu, T)
+    for a, b in zip(cu, cu[1:]):
+        alone = grads(a, b, [0, b - a], b - a)
+        for x, y, z in zip(alone, packed, loose):
+            assert torch.equal(x, y[a:b]) and torch.equal(x, z[a:b]), (a, b)

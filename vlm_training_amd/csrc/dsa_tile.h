@@ -272,6 +272,17 @@ __device__ __forceinline__ void store_c_tile_f32(float *p, const f32x16 &acc, in
     }
 }
 
+// ---- indexer backward ----
+// The query side over the selected keys alone (dsa_tile_idxg.hip) instead of over every causal tile (dsa_tile_idx.hip): a segment this much
+// longer than the selection.  Whole backward, us, tiles against gather, 64 heads of 128: selection of 2048 keys in segments of 2048
+// 609 / 646, 3072: 1246 / 1200, 4096: 2146 / 1951, 5120: 2351 / 2016; 16 384 tokens in one 7441 / 4805; 512 keys in segments of 1536
+// 518 / 426; 256 keys in segments of 300 197 / 250.  32 heads (a tile is half the matrix work for the same keys) of 64: 1024 keys in
+// segments of 2048 193 / 196, 3072: 393 / 353, 4096: 646 / 529; of 700 to 1800: 146 / 163; of 128, in 2048: 331 / 362.
+// Each segment by its own length: a launch whose bound of the longest one reaches the line runs both kernels, and the workgroups of the
+// other's segments leave at once.  Against one kernel by that bound: segments of 680 to 1799, 512 keys 157 -> 150 (64 heads: 371 -> 381); one
+// of 4096 beside 24 of 256 523 -> 490; four of 2048, 512 keys, under a bound of 8192 680 -> 570; 32 768 tokens level.
+__host__ __device__ inline bool idx_segment_gathers(int Hi, int K, int L) { return 2 * (int64_t)L >= (Hi > 32 ? 3 : 6) * (int64_t)K; }
+
 // ---- launches ----
 // log2 of the rows a query takes: its group's heads, padded to a power of two
 static inline int group_shift(int Hq, int Hkv) {

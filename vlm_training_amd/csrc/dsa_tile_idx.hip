@@ -174,7 +174,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = min(__builtin_amdgcn_readfirstlane(L), ldw * 32);
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
-    if (qc0 >= L) return;
+    if (qc0 >= L || idx_segment_gathers(Hi, K, L)) return;
     const int ntiles = min(qc0 + QBW - 1, L - 1) / 32 + 1;
     const int qw = qc0 + ((wv * 32) >> GSHIFT), t = s0 + min(qw, L - 1);         // the wave's query
     const int head = ((wv * 32) & (Gp - 1)) + j;
@@ -439,12 +439,6 @@ static int idxk_chunk(int T, int Di, int ldw) {
 extern "C" hipError_t dsa_launch_indexer_bwd_gather(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n,
                                                     const float *dscore, const float *grad, int ldw, const int32_t *cu, int N, int T, int Hi, int Di, int K,
                                                     float cscale, void *dq_idx, void *dw, int dw_bf16, hipStream_t stream);   // dsa_tile_idxg.hip
-// The query side over the selected keys alone (dsa_tile_idxg.hip) instead of over every causal tile: where the longest segment is this
-// much longer than the selection.  Whole backward, us, tiles against gather, 64 heads of 128: selection of 2048 keys in segments of 2048
-// 609 / 646, 3072: 1246 / 1200, 4096: 2146 / 1951, 5120: 2351 / 2016; 16 384 tokens in one 7441 / 4805; 512 keys in segments of 1536
-// 518 / 426; 256 keys in segments of 300 197 / 250.  32 heads (a tile is half the matrix work for the same keys) of 64: 1024 keys in
-// segments of 2048 193 / 196, 3072: 393 / 353, 4096: 646 / 529; of 700 to 1800: 146 / 163; of 128, in 2048: 331 / 362.
-static bool idx_bwd_gathers(int Hi, int K, int longest) { return 2 * (int64_t)longest >= (Hi > 32 ? 3 : 6) * (int64_t)K; }
 template <int D, int GS>
 static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n, const float *w_f32, const float *dscore,
                              const float *grad, const uint32_t *bitmap, const int32_t *prefix, int ldw, const int32_t *cu, int N, int T, int Hi,
@@ -465,8 +459,11 @@ static hipError_t launch_idx_bwd_i(hipStream_t stream, const void *q_idx, const 
                        (const bf16_t *)k_idx, w_f32, dscore, grad, bitmap, prefix, ldw, cu, N, T, Hi, K, cscale, chunk, partial);
     hipLaunchKernelGGL(dsa_idxk_reduce_kernel, dim3((unsigned)((T + 7) / 8)), dim3(256), 0, stream, partial, cu, N, T, D,
                        chunk, ldw * 32, (bf16_t *)dk_idx);
-    if (idx_bwd_gathers(Hi, K, ldw * 32))
-        return dsa_launch_indexer_bwd_gather(q_idx, k_idx, w_idx, idx, n, dscore, grad, ldw, cu, N, T, Hi, D, K, cscale, dq_idx, dw, dw_bf16, stream_q);
+    // segment by segment: the bound of the longest one only says which of the two kernels can have any
+    if (idx_segment_gathers(Hi, K, ldw * 32)) {
+        e = dsa_launch_indexer_bwd_gather(q_idx, k_idx, w_idx, idx, n, dscore, grad, ldw, cu, N, T, Hi, D, K, cscale, dq_idx, dw, dw_bf16, stream_q);
+        if (e != hipSuccess) return e;
+    }
     const dim3 gq((unsigned)((int64_t)T / ((32 * NW) >> GS) + N + 1));
     hipLaunchKernelGGL((dsa_tile_idxq_kernel<D, GS, NW>), gq, dim3(64 * NW), (idxq_lds_bytes<D, NW>()), stream_q, (const bf16_t *)q_idx,
                        (const bf16_t *)k_idx, (const bf16_t *)w_idx, dscore, grad, bitmap, ldw, cu, N, T, Hi, K, cscale,

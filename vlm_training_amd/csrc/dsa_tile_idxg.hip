@@ -29,7 +29,7 @@ __global__ __launch_bounds__(64, 1) void dsa_tile_idxg_kernel(
     const int seg = find_segment_wave(cu, N, t);
     const int s0 = __builtin_amdgcn_readfirstlane(cu[seg]);
     const int L = min(__builtin_amdgcn_readfirstlane(cu[seg + 1]) - s0, ldw * 32);    // (no key past the longest segment the caller names)
-    if (t - s0 >= L) return;
+    if (t - s0 >= L || !idx_segment_gathers(Hi, K, L)) return;
     const int n = __builtin_amdgcn_readfirstlane(max(min(nsel[t], K), 0)), ntiles = max((n + 31) / 32, 1);
 
     // ---- requests ----
