@@ -25,7 +25,7 @@
 #define TOPK_BINS 2048                                  // 11-bit digits (the last pass uses 1024 of them)
 #define TOPK_CAND 256                                   // see topk_tau
 #define TOPK_LIST 6144                                  // most scores of a long row that are held
-#define TOPK_LONG_MAX 131072                            // longest row swept once (a bit per column in LDS), and most keys selected of it
+#define TOPK_LONG_MAX 131072                            // longest row swept once (a bit per column in LDS, whatever the launch's bound), and most keys selected of it
 #define TOPK_LONG_K 4096
 
 // the score a key stands for (-0.0 comes back as +0.0: score_key folds the two)
@@ -362,17 +362,20 @@ __device__ __forceinline__ bool topk_tau(TopkLong &m, float (&x)[R], Any any, In
 __device__ __noinline__ void topk_radix_memory(TopkShared &sh, const TopkRow &r) {
     topk_radix(sh, r, false, [&](int i) -> uint32_t { return score_key(r.row[i]); });
 }
-// Rows of min_row scores and more, one sweep over memory: the scores from a threshold on that a sample of 4096 puts at about 1.75 K of them
+// words of a row's bit per column, as many for every thread
+__host__ __device__ inline int topk_long_words(int columns) { return (columns + 32 * TOPK_THREADS - 1) / (32 * TOPK_THREADS) * TOPK_THREADS; }
+// Rows of min_row to TOPK_LONG_MAX scores, one sweep over memory: the scores from a threshold on that a sample of 4096 puts at about 1.75 K of them
 // go into a list in LDS, as many as `cap` (another sweep, the threshold moved, when fewer than K or more than cap passed); tau and
 // need_eq come from the list, the selected columns are marked in a bit each and the bits compacted.  What does not fit - scores that are
 // not finite, two moved thresholds that did not help, hundreds of scores equal to tau - takes the radix select.
 //
 // What bounds it: memory, and a fixed 20 us a row around the sweep (the sample's scattered reads, two selections of seven barriers), three
 // workgroups a CU.  Same box, us, against five sweeps of the radix select, rows at the end of one segment: 2048 rows of 20 480 columns
-// 140 -> 94, 32 768: 225 -> 110, 65 536: 506 -> 203, 131 072: 1020 -> 338; all 16 384 rows of one segment 438 -> 407, all 12 288: level.
+// 140 -> 94, 32 768: 225 -> 110, 65 536: 506 -> 203, 131 072: 1020 -> 322, and under a bound of 131 104
+// 20 480: 141 -> 120, 65 536: 514 -> 204; all 16 384 rows of one segment 438 -> 407, all 12 288: level.
 // Held in registers and selected this way, rows of up to 8192 scores took 309 us where the radix select over LDS takes 261 (32 768 tokens).
 __global__ __launch_bounds__(TOPK_THREADS, 3) void dsa_topk_long_kernel(
-    const float *__restrict__ scores, int64_t ld, int row_begin, const int32_t *__restrict__ cu, int N, int K, int min_row, int cap, int nwords,
+    const float *__restrict__ scores, int64_t ld, int row_begin, const int32_t *__restrict__ cu, int N, int K, int min_row, int cap,
     int32_t *__restrict__ idx_out, int32_t *__restrict__ n_out, uint32_t *__restrict__ bitmap, int ldw, float *__restrict__ sel_out) {
     extern __shared__ __attribute__((aligned(16))) unsigned char long_lds[];     // TopkLong | cap scores | their columns | a bit per column
     TopkLong &m = *reinterpret_cast<TopkLong *>(long_lds);
@@ -381,8 +384,8 @@ __global__ __launch_bounds__(TOPK_THREADS, 3) void dsa_topk_long_kernel(
     uint32_t *const words = reinterpret_cast<uint32_t *>(list_i + cap);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     TopkRow r;
-    if (!topk_row(scores, ld, row_begin, cu, N, K, min_row, 0x7fffffff, idx_out, n_out, bitmap, ldw, sel_out, r)) return;
-    const int nvalid = r.nvalid;
+    if (!topk_row(scores, ld, row_begin, cu, N, K, min_row, TOPK_LONG_MAX, idx_out, n_out, bitmap, ldw, sel_out, r)) return;
+    const int nvalid = r.nvalid, nwords = topk_long_words(nvalid);
 
     // a sample: 256 runs of 16 columns over the row
     constexpr int SR = 16;
@@ -532,18 +535,20 @@ extern "C" hipError_t dsa_launch_topk(const float *scores, int64_t ld, int row_b
     hipLaunchKernelGGL(dsa_topk_rows_kernel<true>, dim3(rows), dim3(TOPK_THREADS), (size_t)held * 4, stream, scores, ld, row_begin, cu, N, K, 0, held,
                        idx, n, bitmap, ldw, sel);
     if (longest <= held) return hipGetLastError();
-    if (longest <= TOPK_LONG_MAX && K <= TOPK_LONG_K && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(scores) & 15) == 0) {
+    int next = held + 1;                                 // rows of at least that many columns are left
+    if (K <= TOPK_LONG_K && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(scores) & 15) == 0) {
         const int cap = (std::min(std::max(2 * K + 512, 4096), TOPK_LIST) + TOPK_THREADS - 1) / TOPK_THREADS * TOPK_THREADS;
-        const int nwords = (int)((longest + 32 * TOPK_THREADS - 1) / (32 * TOPK_THREADS)) * TOPK_THREADS;
-        const size_t lds = sizeof(TopkLong) + (size_t)cap * 8 + (size_t)nwords * 4;
+        const int most = (int)std::min<int64_t>(longest, TOPK_LONG_MAX);
+        const size_t lds = sizeof(TopkLong) + (size_t)cap * 8 + (size_t)topk_long_words(most) * 4;
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dsa_topk_long_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(dsa_topk_long_kernel, dim3(rows), dim3(TOPK_THREADS), lds, stream, scores, ld, row_begin, cu, N, K, held + 1, cap, nwords, idx, n,
+        hipLaunchKernelGGL(dsa_topk_long_kernel, dim3(rows), dim3(TOPK_THREADS), lds, stream, scores, ld, row_begin, cu, N, K, next, cap, idx, n,
                            bitmap, ldw, sel);
-    } else {
-        hipLaunchKernelGGL(dsa_topk_rows_kernel<false>, dim3(rows), dim3(TOPK_THREADS), 0, stream, scores, ld, row_begin, cu, N, K, held + 1, all, idx, n,
-                           bitmap, ldw, sel);
+        if (longest == most) return hipGetLastError();
+        next = TOPK_LONG_MAX + 1;
     }
+    hipLaunchKernelGGL(dsa_topk_rows_kernel<false>, dim3(rows), dim3(TOPK_THREADS), 0, stream, scores, ld, row_begin, cu, N, K, next, all, idx, n,
+                       bitmap, ldw, sel);
     return hipGetLastError();
 }
 
