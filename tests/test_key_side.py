@@ -109,7 +109,10 @@ def _case(D, Hq, Hkv, lens, seed):
     (256, 16, 2, (129, 31, 64)), (256, 32, 2, (70, 300)), (256, 2, 1, (700,)),
     # enough workgroups for 64 rows or keys per wave, without and with pieces
     (64, 12, 12, (1, 31, 32, 33, 127, 128, 129, 257, 63) * 6), (72, 12, 12, (63, 64, 65, 190, 255, 256) * 7), (96, 16, 8, (96, 33, 129, 2) * 16),
-    (128, 12, 4, (1, 31, 33, 129, 160) * 32), (128, 16, 16, (32, 127, 64, 193) * 12), (128, 32, 32, (700, 300, 33)), (64, 32, 32, (900, 129, 33))])
+    (128, 12, 4, (1, 31, 33, 129, 160) * 32), (128, 16, 16, (32, 127, 64, 193) * 12), (128, 32, 32, (700, 300, 33)), (64, 32, 32, (900, 129, 33)),
+    # 64 rows and keys per wave with a causal mask too: many workgroups, or (the last two: keys, in pieces) much work
+    (64, 24, 24, (1, 31, 32, 33, 127, 128, 129, 257, 63) * 6), (72, 24, 24, (63, 64, 65, 190, 255, 256) * 7), (96, 48, 24, (96, 33, 129, 2) * 16),
+    (128, 48, 24, (1, 31, 33, 129, 160) * 10), (64, 128, 16, (1500, 700, 300, 33)), (128, 64, 8, (2200, 700, 129, 33))])
 def test_key_and_query_gradients_at_the_edges_of_tiles(D, Hq, Hkv, lens, causal):
     print("key side", D, Hq, Hkv, lens, causal, flush=True)
     q, k, v, do, cu = _case(D, Hq, Hkv, lens, D + Hq)
@@ -150,13 +153,13 @@ def test_operands_on_odd_addresses_give_the_gradients(D, Hq, Hkv, lens, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("D,nseg", [(64, 1), (64, 40), (80, 40), (96, 1), (96, 40), (128, 1), (128, 40), (256, 1), (256, 40)])
+@pytest.mark.parametrize("D,nseg", [(64, 1), (64, 48), (80, 48), (96, 1), (96, 48), (128, 1), (128, 48), (256, 1), (256, 48)])
 def test_score_gradients_of_the_key_side_come_from_unrounded_probabilities(D, nseg, dtype):
     """Every probability is 1/96 (keys orthogonal to the queries), which bf16 rounds up by 2e-3; delta is 0 and the terms dS = P dP of a
     key all have its sign, so a rounded P would be a bias of 2e-3 in every element of dK.  What remains is rounding: of dS (2^-8 at most,
     96 independent terms per key) and of dK itself (2^-8 at most, once for the two keys of a pair): an element is off by 2^-7 at most, the
     mean over the 48 pairs of eight kv heads has a standard deviation of 2^-8 / sqrt(3 * 384) = 1.2e-4, and 8e-4 is more than six of them.
-    One segment and forty: 32 and, up to head_dim 128, 64 keys per wave."""
+    One segment and forty-eight: 32 and, up to head_dim 128, 64 keys per wave."""
     print("unrounded P", D, nseg, dtype, flush=True)
     g = torch.Generator().manual_seed(D + nseg)
     L, H = 96, 8

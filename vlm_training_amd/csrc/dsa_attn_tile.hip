@@ -663,7 +663,7 @@ static DkvPlan dkv_plan(int T, int N, int Hq, int Hkv, int d_real, bool has_idx,
     DkvPlan p;
     p.tiles_ub = T / 128 + N;                            // 128-key tiles of all segments, at most
     p.pitch = has_idx ? d_real : (dense_kernel_dim(d_real) + 31) / 32 * 32;             // row of a partial sum
-    const int wg_per_tile = Hkv, kg = dkv_key_groups(d_real, T, N, Hkv, causal);
+    const int wg_per_tile = Hkv, kg = dkv_key_groups(d_real, T, N, Hq, Hkv, causal);
     const int64_t slot_pairs = partial ? (int64_t)(partial_bytes / ((size_t)2 * 128 * p.pitch * sizeof(float))) : 0;
     p.pieces = order && causal && slot_pairs >= Hkv && (int64_t)p.tiles_ub * wg_per_tile <= dkv_pieces_max_wg(d_real);
     p.listed = order && (N > 1 || p.pieces);             // (one segment: its tiles are in order already)

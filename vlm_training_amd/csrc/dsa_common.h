@@ -12,18 +12,28 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define DSA_WAVE 64
-// Groups of 32 keys that a wave of the key-side kernel takes: two up to head_dim 128 (each operand read feeds two MFMAs, two workgroups
-// per CU), except in launches of few workgroups, which leave CUs idle: there a workgroup's own pace counts, and four waves of one group
-// each walk twice as fast.  The line in workgroups, both sides measured around it (two groups against one, us): without a mask 256,
-// 98 / 84 and 272, 67 / 57, but 384, 171 / 200; causal in one segment 192, 230 / 199 and 224, 242 / 318, in three 240, 123 / 117 (a long
-// walk is cut into pieces, which then needs free slots) and 340, 216 / 260.
-static inline int dkv_key_groups(int D, int T, int N, int Hkv, int causal) {
-    return D > 128 || ((int64_t)T / 128 + N) * Hkv <= (causal ? 160 + 32 * (N < 3 ? N : 3) : 288) ? 1 : 2;
-}
 // key-side workgroups that run at a time, and the launches whose walks may be cut into pieces: up to three rounds of them (a longer
 // launch of whole walks, longest first, ends level)
 static inline int dkv_slots(int key_groups) { return 256 * key_groups; }
 static inline int64_t dkv_pieces_max_wg(int D) { return D > 128 ? 3 * 256 : 3 * 512; }
+// Groups of 32 keys that a wave of the key-side kernel takes: two up to head_dim 128 (each operand read feeds two MFMAs, two workgroups
+// per CU), or one, four waves to a workgroup: its walk is twice as fast, and a CU holds one of them.
+// With a causal mask walks are cut into pieces or finish in turn, and what counts is the launch's work, workgroups times the mean length of
+// a segment in steps (32 rows: 32, 16, .. queries): little of it ends with the pace of single walks, much with the CU's; below
+// 96 workgroups single walks count at any length.  Two groups against one, us, head_dim 128: 4 heads per kv head, one segment of 1408 tokens, 96 workgroups (17 000) 89 / 67, of 2432 and 160 (49 000) 135 /
+// 143; 2 heads per kv head, 8064 and 128 (64 000) 153 / 190, eight of 1152 and 320 (23 000) 87 / 78, three of 2944 and 288 (53 000) 131 /
+// 142.  Over 1050 launches (head_dim 64 to 128, 1 to 8 heads, equal and log-normal segments, with a selection and without) the choice is
+// on average 1.3 % slower than the better one; lines on the workgroups alone were 4.2 to 5.
+// Without a mask the tiles of a segment walk equally long: one group as long as all of them have a CU to themselves, T / 128 for each kv head
+// (one segment, 252: 607 / 457, 268: 627 / 854).
+static inline int dkv_key_groups(int D, int T, int N, int Hq, int Hkv, int causal) {
+    if (D > 128) return 1;
+    if (!causal) return (int64_t)(T / 128) * Hkv <= 256 ? 1 : 2;
+    int rows = 1;                                        // of a query: its group's heads, padded to a power of two
+    while (rows * Hkv < Hq) rows *= 2;
+    const int64_t wg = ((int64_t)T / 128 + N) * Hkv;
+    return wg < 96 || (wg <= dkv_pieces_max_wg(D) && wg * T / N * rows <= 40000 * 32) ? 1 : 2;
+}
 #define LOG2E_F 1.4426950408889634f
 #define LN2_F 0.6931471805599453f
 

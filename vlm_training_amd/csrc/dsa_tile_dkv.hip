@@ -7,7 +7,7 @@
 //                                    -lse/scale and -delta, so that P = exp2(S * scale*log2e) and dS = P dP need no subtraction)
 //   dV^T += dO^T P, dK^T += Q^T dS  (A = the blocks transposed, B = P / dS from the C layout)
 // One wave per SIMD, each with all four chains of its keys and 512 registers: 64 keys up to head_dim 128 (two waves a workgroup, two
-// workgroups a CU), 32 keys at head_dim 256 and in launches of few workgroups (four waves, one workgroup: dkv_key_groups).  The sums of
+// workgroups a CU), 32 keys at head_dim 256 and in launches of little work (four waves, one workgroup: dkv_key_groups).  The sums of
 // dK and dV fill up to 256 accumulation registers, K and V rows 128 of the others.  An operand read from LDS feeds the MFMAs of both key groups, P and dS never leave
 // the wave, nothing is formed twice.  Step s runs dV(s) mixed with S(s+1), the products of dS(s) behind them, then dK(s) mixed with
 // dP(s+1), P(s+1) behind them in three stages (logit, exponential, packing) that do not wait for each other.  P stays in fp32 until dS is
@@ -542,7 +542,7 @@ static hipError_t launch_dkv_gs(unsigned grid, hipStream_t stream, const DkvArgs
 template <int D, bool HAS_IDX>
 static hipError_t launch_dkv_kg(unsigned grid, hipStream_t stream, const DkvArgs &a) {
 #if !DKV_UNALIGNED
-    if (dkv_key_groups(a.d_real, a.T, a.N, a.Hkv, a.causal) == 1) return launch_dkv_gs<D, 1, HAS_IDX>(grid, stream, a);
+    if (dkv_key_groups(a.d_real, a.T, a.N, a.Hq, a.Hkv, a.causal) == 1) return launch_dkv_gs<D, 1, HAS_IDX>(grid, stream, a);
 #endif
     return launch_dkv_gs<D, 2, HAS_IDX>(grid, stream, a);
 }

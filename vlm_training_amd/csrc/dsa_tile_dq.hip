@@ -4,7 +4,7 @@
 //   dQ^T[d,row] += K^T[d,key] dS^T[key,row]   (A = K tile transposed, B = dS^T from the C layout)
 //
 // One wave per SIMD with 512 registers and 64 rows (RG = 2 groups of 32), so that each operand read from LDS feeds two MFMAs; 32 rows at
-// head_dim 256, where a row alone fills the registers, and in launches of few workgroups (dq_one_row_group).  Step t runs dQ(t) mixed
+// head_dim 256, where a row alone fills the registers, and in launches of little work (dq_one_row_group).  Step t runs dQ(t) mixed
 // with dP(t+1), the logits and exponentials P(t+1) behind them, then S(t+2), the products and packing of dS(t+1) behind it; operand reads
 // run four ahead through all of it, in pairs where two groups share them.  K and V tiles go from memory straight into LDS, rings of five
 // and three: step t requests K(t+4), V(t+3) and the selection words of tile t+3, at its end waits for what step t-1 requested and meets
@@ -379,12 +379,21 @@ static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *
                        bitmap, ldw, cu, N, T, Hq, Hkv, gs, scale, pos_split, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
     return hipGetLastError();
 }
-// 32 rows per wave instead of 64 for launches of few workgroups (wg: of 256 rows): each walk is then twice as fast and two workgroups share
-// a CU; with more of them the halved operand reads win.  Head_dim 128, us, 64 rows against 32: causal, one segment, 256 workgroups 74 /
-// 61, 375: 115 / 110, 437: 139 / 149; three segments 375: 60 / 51, 562: 106 / 100, 750: 165 / 164; without a mask 125: 116 / 100, 188: 140 /
-// 146 and 101 / 95, 250: 265 / 272.
-static bool dq_one_row_group(int causal, int64_t wg, int N) {
-    return wg <= (causal ? 320 + 64 * (N < 5 ? N : 5) : 160);
+// 32 rows per wave instead of 64: each walk is then twice as fast, two workgroups share a CU, and blocks are half as long, which wastes fewer
+// rows at the ends of segments; the operand reads they share are worth 5 to 10 %.  wg: workgroups of 256 rows, at most.
+// With a causal mask (blocks go heaviest first) the finer blocks win while the launch's work, workgroups times the mean length of a segment,
+// is small (measured up to 1280 of them).  64 rows against 32, us, head_dim 128: one segment 3968 tokens 256 workgroups 124 / 102, 6016 and 384 211 / 194, 8064 and 512
+// 323 / 344; eight segments of 1920 and 512 90 / 90, of 2432 and 640 147 / 132; 35 of mean 330 and 496 38 % more.
+// Without a mask every block of a segment walks equally long, so that what counts is the number of rounds: of 256 workgroups, or of 256
+// half as long.  Four segments, head_dim 128: 128 workgroups 36 / 24, 224 65 / 66, 288 155 / 123, 384 205 / 178, 512 306 / 313, 640 525 / 489;
+// short segments take 32 rows (of 320 to 512: 5 to 12 % less, log-normal ones more).
+// Over 880 causal launches, with a selection and without, and 490 without a mask (head_dim 64 to 128) the choice is on average 0.3 and 0.5 %
+// slower than the better one; lines on the workgroups alone were 1.3 to 4 and 7.
+static bool dq_one_row_group(int causal, int T, int N, int Hkv, int gs) {
+    const int64_t rows = (int64_t)T << gs, wg = (rows / 256 + N) * Hkv;
+    if (causal) return wg <= 416 || (wg <= 1280 && wg * T / N <= 2000000);
+    if (wg > 1024) return false;
+    return T / N < 1500 || (rows / 128 * Hkv + 255) / 256 < 2 * (((2 * (rows / 256) + N) * Hkv + 511) / 512);
 }
 // d_real: elements of a row, without a selection any multiple of 8 (dense_kernel_dim).  out_for_delta != null: the kernel forms
 // delta = rowsum(dO * O) of its rows itself and writes it to delta_out
@@ -394,7 +403,7 @@ extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const 
                                          int pos_split, int causal, void *dq, const void *out_for_delta, float *delta_out,
                                          hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
-    const bool one_group = dq_one_row_group(causal, (((int64_t)T << gs) / 256 + N) * Hkv, N);
+    const bool one_group = dq_one_row_group(causal, T, N, Hkv, gs);
 #define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, causal, dq, out_for_delta, delta_out
 #define DQ_CASE(D_, HI) return one_group ? launch_dq_i<D_, HI, 1>(DQ_ARGS) : launch_dq_i<D_, HI, 2>(DQ_ARGS)
     if (bitmap) switch (d_real) {
