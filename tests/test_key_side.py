@@ -24,33 +24,40 @@ def _registers(token):
     return [(m.group(1), r) for r in range(int(lo), int(hi) + 1)]
 
 
-def _hazards(listing):
-    """(MFMAs on accumulation registers, findings).  In program order: an operand of such an MFMA that a vector instruction wrote
-    needs two wait states between them, a vector instruction or store that reads its result eleven (eight passes; an instruction
-    counts as one wait state, s_nop n as n + 1).  A buffer load needs five behind a vector instruction that wrote its scalar operand."""
-    count, found, clock, formed, written = 0, [], 0, {}, {}
+def _instructions(listing):
+    """Functions of a listing: lists of (address, mnemonic, operands, text).  Where no address is printed, one instruction is four bytes."""
+    functions, address = [[]], 0
     for line in listing.splitlines():
-        text = line.split("//")[0].strip()
+        text, _, note = line.partition("//")
+        text = text.strip()
         if not text or text.endswith(":"):
-            formed, written = ({}, {}) if text.endswith(">:") and "kernel" in text else (formed, written)
+            if text.endswith(">:"):
+                functions.append([])
             continue
         op, _, rest = text.partition(" ")
-        args = [a.strip() for a in rest.split(",")]
+        m = re.match(r"\s*([0-9A-Fa-f]+):", note)
+        address = int(m.group(1), 16) if m else address + 4
+        functions[-1].append((address, op, [a.strip() for a in rest.split(",")], text))
+    return functions
+
+
+def _scan(block, written, formed, found):
+    """One basic block, entered with the wait states since registers were written by a vector instruction or formed by an MFMA on
+    accumulation registers; returns them at its end."""
+    clock, written, formed = 0, {r: -n for r, n in written.items()}, {r: -n for r, n in formed.items()}
+    for address, op, args, text in block:
         if op == "s_nop":
             clock += int(args[0], 0) + 1
             continue
         if op.startswith("v_mfma"):
             if args[0].startswith("a["):
-                count += 1
-                for r in (r for a in args[1:4] for r in _registers(a)):
-                    if clock - written.get(r, -99) < 3:
-                        found.append(text)
+                if any(clock - written.get(r, -99) < 3 for a in args[1:4] for r in _registers(a)):
+                    found[address] = text
                 for r in _registers(args[0]):
                     formed[r] = clock
         elif op.startswith("v_"):
-            for r in (r for a in args for r in _registers(a)):
-                if r[0] == "a" and clock - formed.get(r, -99) < 12:
-                    found.append(text)
+            if any(r[0] == "a" and clock - formed.get(r, -99) < 12 for a in args for r in _registers(a)):
+                found[address] = text
             for a in args[:2 if op.startswith(("v_permlane32_swap", "v_add_co", "v_div_scale")) else 1]:
                 for r in _registers(a):
                     written[r] = clock
@@ -59,11 +66,45 @@ def _hazards(listing):
                 written.pop(r, None)
         elif op.startswith("buffer_load"):
             if any(r[0] == "s" and clock - written.get(r, -99) < 6 for a in args for r in _registers(a.split(" ")[0])):
-                found.append(text)
+                found[address] = text
         elif "store" in op or op.startswith("ds_write"):
             if any(r[0] == "a" and clock - formed.get(r, -99) < 12 for a in args for r in _registers(a.split(" ")[0])):
-                found.append(text)
+                found[address] = text
         clock += 1
+    return tuple({r: clock - at for r, at in state.items() if clock - at < 12} for state in (written, formed))
+
+
+def _hazards(listing):
+    """(MFMAs on accumulation registers, findings).  Along every path, loops and branches followed: an operand of such an MFMA that a
+    vector instruction wrote needs two wait states between them, a vector instruction or store that reads its result eleven (eight passes;
+    an instruction counts as one wait state, s_nop n as n + 1).  A buffer load needs five behind a vector instruction that wrote its
+    scalar operand."""
+    count, found = 0, []
+    for code in _instructions(listing):
+        count += sum(op.startswith("v_mfma") and args[0].startswith("a[") for _, op, args, _ in code)
+        at = {address: i for i, (address, *_) in enumerate(code)}
+        goes = {}                                       # branches: index -> index of the target (None: outside)
+        for i, (address, op, args, _) in enumerate(code):
+            if op.startswith(("s_branch", "s_cbranch")):
+                jump = int(args[0].split()[0], 0)
+                goes[i] = at.get(address + 4 + 4 * (jump - 65536 if jump > 32767 else jump))
+        ends = [i for i, (_, op, *_) in enumerate(code) if op.startswith(("s_endpgm", "s_setpc"))]
+        heads = sorted({0, *(i + 1 for i in (*goes, *ends)), *(t for t in goes.values() if t is not None)} - {len(code)})
+        behind = dict(zip(heads, heads[1:] + [len(code)]))
+        entry, todo, bad = {h: ({}, {}) for h in heads}, list(heads) if code else [], {}
+        while todo:                                     # to a fixed point: a register's wait states only fall
+            h = todo.pop(0)
+            out, last = _scan(code[h:behind[h]], *entry[h], bad), behind[h] - 1
+            into = [goes[last]] if last in goes else []
+            if last not in ends and not code[last][1].startswith("s_branch") and behind[h] < len(code):
+                into.append(behind[h])
+            for t in (t for t in into if t is not None):
+                lower = [(mine, r, n) for mine, new in zip(entry[t], out) for r, n in new.items() if n < mine.get(r, 99)]
+                for mine, r, n in lower:
+                    mine[r] = n
+                if lower and t not in todo:
+                    todo.append(t)
+        found += bad.values()
     return count, found
 
 
@@ -74,6 +115,11 @@ def test_wait_states_checker_sees_planted_hazards():
     assert _hazards(mfma + "\n scratch_store_dwordx4 off, a[0:3], off")[1]
     first, load = "v_readfirstlane_b32 s5, v1\n s_nop ", "\n buffer_load_dwordx4 v2, s[4:7], 0 offen lds"
     assert _hazards(first + "3" + load)[1] and not _hazards(first + "4" + load)[1]
+    # at the head of a loop, behind the last MFMA of its body (a branch counts four bytes from its own end); behind a branch around the wait
+    loop = "v_accvgpr_read_b32 v1, a15\n s_nop 12\n " + mfma + "\n s_nop {}\n s_cbranch_scc1 65531\n s_endpgm"
+    assert _hazards(loop.format(8))[1] and not _hazards(loop.format(9))[1]
+    around = mfma + "\n s_cbranch_scc1 {}\n s_nop 11\n s_nop 0\n v_accvgpr_read_b32 v1, a15"
+    assert _hazards(around.format(2))[1] and _hazards(around.format(1))[1] and not _hazards(around.format(0))[1]
 
 
 def test_inline_mfmas_keep_their_wait_states(tmp_path):
