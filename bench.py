@@ -324,7 +324,7 @@ def main():
     kern = {   # algorithmic flop per launch of the three attention kernels (selected pairs only)
         "attn_fwd": ("dsa_tile_fwd_kernel", 4 * unit),          # QK^T + PV
         "bwd_dq": ("dsa_tile_dq_kernel", 6 * unit),   # QK^T + dO V^T + dS K
-        # QK^T + dO V^T + P^T dO + dS^T Q (head_dim 256: the producer/consumer form, each half of head_dim forms S and dP)
+        # QK^T + dO V^T + P^T dO + dS^T Q
         "bwd_dkv": ("dsa_tile_dkv_kernel", 8 * unit),
     }
     dom = max(kern, key=lambda name: stage_ms[name])
