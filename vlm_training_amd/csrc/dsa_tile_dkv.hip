@@ -18,7 +18,7 @@
 // instructions (210 with a selection), 60 LDS reads and as many scalar ones take 3000 - and the chip's power (MFMA busy 0.69 of a CU's
 // time, 1.85 GHz under this load).  Same box, us, against the kernels before (eight waves; at head_dim 128 one wave per chain, P handed
 // over in LDS; at 256 each half of head_dim formed S and dP; q and dO through registers): 32 768 tokens dense 2630 -> 2200, with a
-// selection 2680 -> 2285; head_dim 256, 16 384 tokens in short segments 548 -> 327; towers at head_dim 64 / 72, whole backward
+// selection 2680 -> 2240; head_dim 256, 16 384 tokens in short segments 548 -> 327 (in finer pieces 309); towers at head_dim 64 / 72, whole backward
 // 553 -> 440 / 1131 -> 976; one segment of 4096 / 12 288 tokens 451 -> 300 / 2430 -> 2000.  32 keys per wave at head_dim 128: 2440
 // dense, each operand read feeding one MFMA, but a walk's step 1600 instead of 3000 clocks: 1000 tokens, forward and backward, 118 -> 99
 // (64 keys: 124).
