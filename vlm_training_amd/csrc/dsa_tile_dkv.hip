@@ -541,10 +541,14 @@ static hipError_t launch_dkv_gs(unsigned grid, hipStream_t stream, const DkvArgs
 }
 template <int D, bool HAS_IDX>
 static hipError_t launch_dkv_kg(unsigned grid, hipStream_t stream, const DkvArgs &a) {
-#if !DKV_UNALIGNED
+#if DKV_UNALIGNED
+    // (head_dim 128: with the copies, two groups spill - 4 heads per kv head, 4096 and 2000 tokens without a mask 2190 us, one group 1761, 1000
+    // and 300 causal 161 / 98, 4096 720 / 740)
+    return launch_dkv_gs<D, D == 128 ? 1 : 2, HAS_IDX>(grid, stream, a);
+#else
     if (dkv_key_groups(a.d_real, a.T, a.N, a.Hq, a.Hkv, a.causal) == 1) return launch_dkv_gs<D, 1, HAS_IDX>(grid, stream, a);
-#endif
     return launch_dkv_gs<D, 2, HAS_IDX>(grid, stream, a);
+#endif
 }
 // grid: workgroups (one per key tile or piece, and kv head).  The file is compiled twice, the second time (DKV_UNALIGNED) for q or dO on no
 // 16-byte boundary; k and v lie on one (the entry points see to it).
