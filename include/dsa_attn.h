@@ -194,8 +194,9 @@ int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const float *lse, c
 /*
  * Tuning knob (process-wide, no reference counterpart): query rows whose position in their segment is
  * below top_k * crossover run on the dense MFMA tile kernels with the selection as a bitmap mask, the
- * rest on the gather kernels.  Default 24 (one 131 072-token sequence with top-k 2048: forward 101 -> 96 ms and
- * dQ 107 -> 104 ms against 16; 32 is level with it); 0 = gather only; INT_MAX/top_k or more = tiles only.
+ * rest on the gather kernels.  0 = gather only; INT_MAX/top_k or more = tiles only.  At the default, 24, head_dim 128 with two
+ * to four heads per kv head splits otherwise: segments of 18 * top_k tokens and more run their rows from position 16 * top_k on in
+ * the compacted walk of dsa_tile_sel.hip (up to 75 * top_k, 150 with two heads, the rest gathered), shorter ones on the tile kernels.
  * idx == NULL (dense causal attention) always uses the tile kernels.
  */
 int dsa_set_tile_crossover(int crossover);

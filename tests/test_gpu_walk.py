@@ -1,0 +1,78 @@
+"""The compacted walk (late rows, two to four heads per kv head): the lines to the tile and gather kernels, the ends of blocks, lists and segments."""
+import math
+
+import pytest
+import torch
+
+from tests.util import assert_close_bf16
+from vlm_training_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+DEV, D = "cuda", 128
+
+
+def _reference(q, k, v, dout, sel, scale):
+    """Out, log-sum-exp and gradients in 64 bits; ``sel`` (T,T): which keys a query attends.  Rows without a key: zero, -inf."""
+    q, k, v = (x.double().requires_grad_(True) for x in (q, k, v))
+    G = q.shape[1] // k.shape[1]
+    s = torch.einsum("thd,shd->hts", q, k.repeat_interleave(G, 1)) * scale
+    s = s.masked_fill(~sel, -math.inf)
+    top = s.detach().amax(-1, keepdim=True).clamp(min=-1e300)
+    e = (s - top).exp()
+    z = e.sum(-1, keepdim=True)
+    out = torch.einsum("hts,shd->thd", e / z.clamp(min=1e-300), v.repeat_interleave(G, 1))
+    out.backward(dout.double())
+    return out.detach(), (top + z.log()).squeeze(-1).detach(), q.grad, k.grad, v.grad
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,K,kind,scale", [
+    (4, 1, (641, 256, 257, 97), 8, "random", None),      # tiles to 256, walk to 768: rows on either side of a block of 96 queries
+    (8, 2, (1000,), 8, "random", None),                  # and the gather beyond 768
+    (4, 2, (1400, 300), 8, "random", None),              # two heads per kv head: the gather from 1280 on
+    (3, 1, (700,), 16, "random", -0.1),                  # a group of three, a negative scale
+    (8, 2, (897, 705), 40, "runs", None),                # every key of a block wanted by some query: four steps
+    (4, 1, (769,), 8, "classes", None),                  # keys 16 apart: one class of the block's rows
+    (6, 2, (640,), 12, "empty", None)])                  # queries that select nothing
+def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
+    print("compacted walk", Hq, Hkv, lens, K, kind, flush=True)
+    assert _lib.load().dsa_get_tile_crossover() == 24
+    g = torch.Generator().manual_seed(Hq * K + len(lens))
+    T, cu = sum(lens), [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    q, k, v, dout = (torch.randn(T, h, D, generator=g).mul_(0.5).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    idx, n = torch.full((T, K), -1, dtype=torch.int32), torch.zeros(T, dtype=torch.int32)
+    sel = torch.zeros(T, T, dtype=torch.bool)
+    for a, b in zip(cu[:-1], cu[1:]):
+        for t in range(a, b):
+            pos = t - a
+            if kind == "random" or pos < K:
+                keys = torch.randperm(pos + 1, generator=g)[:K]
+            elif kind == "runs":
+                keys = torch.arange(K) + int(torch.randint(0, pos + 2 - K, (1,), generator=g))
+            elif kind == "classes":
+                keys = (torch.arange(K) * 16 + pos % 16).clamp(max=pos).unique()
+            else:
+                keys = torch.randperm(pos + 1, generator=g)[:K if pos % 3 else 0]
+            keys = keys.sort().values + a
+            n[t] = len(keys)
+            idx[t, :len(keys)] = keys.int()
+            sel[t, keys] = True
+    scale = D ** -0.5 if scale is None else scale
+    want = _reference(q, k, v, dout, sel, scale)
+    d = [x.to(DEV) for x in (q, k, v, idx, n, torch.tensor(cu, dtype=torch.int32), dout)]
+    out, lse = ops.attn_fwd(*d[:6], max(lens), scale, True)[:2]
+    # the backward takes log-sum-exps that are finite, as those of rows with a key are
+    dq, dk, dv = ops.attn_bwd(d[6], *d[:3], out, lse.clamp(min=-1e30), *d[3:6], max(lens), scale, causal=True)
+    torch.cuda.synchronize()
+    some = n > 0
+    late = torch.cat([torch.arange(m) >= 16 * K + 255 for m in lens])    # (the tile kernels have no result for a row without a key)
+    assert bool((out.cpu()[late & ~some] == 0).all()) and bool((dq.cpu()[late & ~some] == 0).all())
+    rows = some | late
+    for name, got, ref in (("out", out, want[0]), ("dq", dq, want[2])):
+        assert_close_bf16(got.cpu()[rows], ref[rows], name)
+    got, ref = lse.cpu().T[rows], want[1].T[rows].float()
+    assert torch.equal(got.isinf(), ref.isinf()) and float((got - ref)[~ref.isinf()].abs().max()) < 2e-3   # (bf16 products are exact in fp32)
+    if bool(some.all()):
+        assert_close_bf16(dk, want[3], "dk")
+        assert_close_bf16(dv, want[4], "dv")

@@ -21,6 +21,11 @@ hipError_t dsa_launch_indexer(const void *q_idx, const void *k_idx, const void *
 hipError_t dsa_launch_attn_fwd(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K, float scale, int pos_min,
                                void *out, float *lse, hipStream_t stream);
+hipError_t dsa_launch_sel_fwd(const void *q, const void *k, const void *v, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
+                              int Hq, int Hkv, float scale, int pos_min, int pos_max, int split_len, void *out, float *lse, hipStream_t stream);
+hipError_t dsa_launch_sel_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
+                             const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float scale, int pos_min,
+                             int pos_max, int split_len, void *dq, hipStream_t stream);
 hipError_t dsa_launch_delta(const void *dout, const void *out, int T, int Hq, int D, float *delta, hipStream_t stream);
 hipError_t dsa_launch_bitmap(const int32_t *idx, const int32_t *n, const int32_t *cu, int N, int T, int K, int ldw,
                              uint32_t *bitmap, hipStream_t stream);
@@ -37,11 +42,11 @@ hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, 
                                 const int32_t *n, const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K,
                                 float scale, float *partial, float *mass, hipStream_t stream);
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
                                int causal, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                              int Hq, int Hkv, int D, float scale, int pos_split, int causal, void *dq, const void *out_for_delta,
+                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int causal, void *dq, const void *out_for_delta,
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
@@ -268,7 +273,8 @@ static int check_attn(int T, int N, const int32_t *cu, int Hq, int Hkv, int D, i
 // Query rows whose position in their segment is below top_k * crossover are handled by the tile
 // kernels (their selection covers more than 1/crossover of the causal window), the rest by the
 // gather kernels.  Process-wide tuning knob; 0 = gather only, a huge value = tile only.
-static std::atomic<int> g_tile_crossover{24};          // read on every launch, possibly from several host threads
+#define DSA_TILE_CROSSOVER 24
+static std::atomic<int> g_tile_crossover{DSA_TILE_CROSSOVER};          // read on every launch, possibly from several host threads
 extern "C" int dsa_set_tile_crossover(int crossover) {
     if (crossover < 0) return fail(DSA_ERR_ARG, "crossover=%d must be >= 0", crossover);
     g_tile_crossover.store(crossover, std::memory_order_relaxed);
@@ -276,12 +282,30 @@ extern "C" int dsa_set_tile_crossover(int crossover) {
 }
 extern "C" int dsa_get_tile_crossover(void) { return g_tile_crossover.load(std::memory_order_relaxed); }
 
-// first query position handled by the gather kernels (multiple of 128, the coarsest tile block)
-static int pos_split_for(const int32_t *idx, int K) {
-    if (!idx) return INT32_MAX;                       // dense causal: tiles everywhere
-    const int64_t p = (int64_t)K * g_tile_crossover.load(std::memory_order_relaxed);
-    if (p >= INT32_MAX - 256) return INT32_MAX;
-    return (int)((p + 255) / 256 * 256);          // a multiple of every tile kernel's query block
+// Positions that the tile kernels (below `tiles`), the compacted walk (dsa_tile_sel.hip: below `walk`) and the gather kernels (the rest) take in
+// segments of at least `len` tokens; multiples of 256, the coarsest block of a tile kernel.  Shorter segments are the tile kernels' whole (a
+// segment's own length decides, so that any upper bound of the longest one gives the same bits).
+// The compacted walk stands between the other two at head_dim 128 with two to four heads per kv head, unless the crossover was set.  Its rows cost
+// what the 32-key steps of their blocks cost, a gathered row what its K keys do, so that the gather is the better one again once rows are long
+// (K = 128, 32 768 tokens, two kv heads of 4: forward 0.46 ms gathered, 0.88 walked), the sooner the fewer queries a wave holds.  One
+// document, 32 heads over 8 kv heads, K = 2048, gather from 24 K on (tiles up to there) -> walk from 16 K on, forward / backward, ms:
+// 131 072 tokens 94.5 / 299 -> 57.3 / 277, 65 536 30.3 / 86.5 -> 21.1 / 78.0, 49 152 16.7 / 49.9 -> 15.0 / 46.8, 40 000 11.2 / 34.2 -> 11.0 / 33.5,
+// 36 000 9.1 / 27.7 -> 9.8 / 27.3, 33 000 7.7 / 22.5 -> 8.9 / 23.7 (few long walks behind the tiles' launch): from segments of 18 K on.  With 8
+// and 16 heads per kv head (32 768 tokens, two kv heads, K = 512) the gather is the faster one from 16 K on: forward 1.45 and 1.71 ms
+// against 1.84 and 3.29; at head_dim 64 with 4 heads too, 0.59 against 0.81.
+struct RowSplit {
+    int tiles, walk, len;
+    bool past_tiles(int max_seqlen) const { return max_seqlen > tiles && max_seqlen >= len; }
+};
+static RowSplit row_split_for(const int32_t *idx, int Hq, int Hkv, int D, int K) {
+    if (!idx) return {INT32_MAX, INT32_MAX, 0};       // dense causal: tiles everywhere
+    auto line = [&](int64_t times) {
+        const int64_t p = K * times;
+        return p >= INT32_MAX - 256 ? INT32_MAX : (int)((p + 255) / 256 * 256);
+    };
+    const int crossover = g_tile_crossover.load(std::memory_order_relaxed), G = Hq / Hkv;
+    if (crossover == DSA_TILE_CROSSOVER && D == 128 && G >= 2 && G <= 4) return {line(16), line(G == 2 ? 150 : 75), line(18)};
+    return {line(crossover), line(crossover), 0};
 }
 
 extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_idx) {
@@ -299,11 +323,11 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, const int32
     if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
-    const int split = pos_split_for(idx, K);
+    const RowSplit rows = row_split_for(idx, Hq, Hkv, D, K);
     const int ldw = bitmap_ldw(max_seqlen);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = hipSuccess;
-    if (split > 0) {
+    if (rows.tiles > 0) {
         uint32_t *bitmap = nullptr;
         if (idx) {
             const size_t need = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
@@ -316,11 +340,15 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, const int32
             }
         }
         const int64_t strides[6] = {(int64_t)Hq * D, D, (int64_t)Hkv * D, D, (int64_t)Hkv * D, D};
-        e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, split, causal, out, lse, st);
+        e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len, causal, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "tile forward launch");
     }
-    if (max_seqlen > split) {
-        e = dsa_launch_attn_fwd(q, k, v, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, split, out, lse, st);
+    if (rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
+        e = dsa_launch_sel_fwd(q, k, v, (const uint32_t *)ws, ldw, cu, N, T, Hq, Hkv, softmax_scale, rows.tiles, rows.walk, rows.len, out, lse, st);
+        if (e != hipSuccess) return hip_fail(e, "compacted forward launch");
+    }
+    if (max_seqlen > rows.walk) {
+        e = dsa_launch_attn_fwd(q, k, v, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "gather forward launch");
     }
     return DSA_OK;
@@ -551,7 +579,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
                         uint32_t *bitmap, float *partial, size_t partial_bytes, int32_t *order, int parts, hipStream_t st) {
     const int ldw = bitmap_ldw(max_seqlen);
     if (idx && (size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
-    const int split = pos_split_for(idx, K);
+    const RowSplit rows = row_split_for(idx, Hq, Hkv, D, K);
     hipError_t e = hipSuccess;
     // the two passes side by side on two streams: launches of few workgroups only (larger ones fill the GPU alone)
     std::unique_lock<std::mutex> ov_lock;
@@ -569,7 +597,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     // delta = rowsum(dO * O): a pass of its own, unless the tile dQ kernel of the same call owns every query row
     // (no row beyond the tile/gather split) - then that kernel forms it from the dO rows it loads anyway - and the
     // key side, which reads every delta, runs after it
-    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && split > 0 && max_seqlen <= split && !ov;
+    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.past_tiles(max_seqlen) && !ov;
     int listed = 0;                                      // the launch order of the key tiles is there
     if ((parts & DSA_BWD_DELTA) && ov) {
         e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, idx != nullptr, causal, order, partial, partial_bytes, delta, st);
@@ -599,13 +627,17 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
         if (e != hipSuccess) rc = hip_fail(e, "tile dkv launch");
     }
     if (rc == DSA_OK && (parts & DSA_BWD_DQ)) {
-        if (split > 0) {
-            e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, split, causal, dq,
+        if (rows.tiles > 0) {
+            e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len, causal, dq,
                                    fuse_delta ? out : nullptr, delta, sq);
             if (e != hipSuccess) rc = hip_fail(e, "tile dq launch");
         }
-        if (rc == DSA_OK && max_seqlen > split) {
-            e = dsa_launch_gather_dq(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, split, dq, sq);
+        if (rc == DSA_OK && rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
+            e = dsa_launch_sel_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, softmax_scale, rows.tiles, rows.walk, rows.len, dq, sq);
+            if (e != hipSuccess) rc = hip_fail(e, "compacted dq launch");
+        }
+        if (rc == DSA_OK && max_seqlen > rows.walk) {
+            e = dsa_launch_gather_dq(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, dq, sq);
             if (e != hipSuccess) rc = hip_fail(e, "gather dq launch");
         }
     }
@@ -671,7 +703,7 @@ extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const 
     if (int rc = check_bwd(dout, q, k, v, out, lse, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
     if (T == 0) return DSA_OK;
     if (idx) {
-        if (pos_split_for(idx, K) <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
+        if (row_split_for(idx, Hq, Hkv, D, K).tiles <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
         const size_t have = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
         if (!fwd_ws || fwd_ws_bytes < have) return fail(DSA_ERR_WORKSPACE, "forward workspace (selection bitmap): have %zu bytes, need %zu", fwd_ws_bytes, have);
     }
@@ -731,7 +763,7 @@ extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_hea
             return fail(DSA_ERR_ARG, "strides must be multiples of 8, token strides below 2^24");
     if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) return fail(DSA_ERR_ARG, "tensors must lie on 16-byte boundaries");
     if (T == 0) return DSA_OK;
-    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, causal, out, lse,
+    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, causal, out, lse,
                                              (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "tile forward launch");
 }

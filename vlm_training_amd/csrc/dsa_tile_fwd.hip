@@ -36,7 +36,7 @@ template <int D, bool HAS_IDX, int NW, bool NEG>
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
-    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int causal,
+    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int causal,
     bf16_t *__restrict__ out, float *__restrict__ lse) {
     typedef DirectTile<D> TL;
     constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;   // MFMAs of S, of P V (head_dim 80: five and six)
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
-    if (qc0 >= pos_split || qc0 >= L) return;           // rows past the split belong to the gather kernel
+    if ((qc0 >= pos_split && L >= split_len) || qc0 >= L) return;   // rows past the split are not the tile kernels'
     const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
 
     const int r = wv * 32 + j;
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 
 template <int D, bool HAS_IDX>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int causal,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
     const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false>;
@@ -364,19 +364,19 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
-                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, causal, (bf16_t *)out, lse);
+                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, causal, (bf16_t *)out, lse);
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
 // without a bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
 extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                          int pos_split, int causal, void *out, float *lse, hipStream_t stream) {
+                                          int pos_split, int split_len, int causal, void *out, float *lse, hipStream_t stream) {
     int gs = 0;
     while ((1 << gs) < Hq / Hkv) ++gs;
     scale = logit_scale(scale);
     hipError_t e = hipErrorInvalidValue;
-#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, causal, out, lse)
+#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, causal, out, lse)
     if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
         else if (d_real <= 128) FWD_CASE(128, true);
