@@ -1,4 +1,4 @@
-"""The compacted walk (late rows, two to four heads per kv head): the lines to the tile and gather kernels, the ends of blocks, lists and segments."""
+"""The compacted walks (thin selections): the lines to the tile and gather kernels, the ends of blocks, lists and segments."""
 import math
 
 import pytest
@@ -76,3 +76,48 @@ def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
     if bool(some.all()):
         assert_close_bf16(dk, want[3], "dk")
         assert_close_bf16(dv, want[4], "dv")
+
+
+@pytest.mark.parametrize("G,lens,kind", [
+    (4, (1700, 900, 500), "random"),     # 26 K = 1664: the walk takes the first segment, the tile kernel the others
+    (3, (1790, 1400), "random"),         # a group of three; 1790 keys: the last workgroup's 62, the last wave's 14
+    (4, (1664, 1663), "runs"),           # every query of a block wants a key of the tile, or none does
+    (8, (1921, 1200), "same"),           # sixteen keys that all queries want: large probabilities, lists that are full
+    (16, (2000, 1100), "classes")])      # queries of one residue: one class of the block's rows
+def test_keys_of_the_compacted_walk(G, lens, kind):
+    print("compacted walk, key side", G, lens, kind, flush=True)
+    Hkv, K, T, scale = 64, 64, sum(lens), D ** -0.5
+    assert _lib.load().dsa_get_tile_crossover() == 24 and (T // 128 + len(lens)) * Hkv > 1536
+    g = torch.Generator(device=DEV).manual_seed(G)
+    q, k, v, dout = (torch.randn(T, h, D, generator=g, device=DEV).mul_(0.5).bfloat16() for h in (G * Hkv, Hkv, Hkv, G * Hkv))
+    idx, n = torch.full((T, K), -1, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
+    sel, a, cu = torch.zeros(T, T, dtype=torch.bool, device=DEV), 0, [0]
+    for m in lens:
+        r = torch.rand(m, m, generator=g, device=DEV)                  # the K largest of a row are its keys
+        pos = torch.arange(m, device=DEV)
+        if kind == "runs":
+            r += (pos[None, :] // K == (pos[:, None] * 7 // 320) % 30).float()
+        elif kind == "same":
+            r += (pos[None, :] % 97 < 1).float()
+        elif kind == "classes":
+            r += (pos[None, :] % 16 == pos[:, None] % 4).float()
+        r.masked_fill_(pos[None, :] > pos[:, None], -1.0)
+        top = r.topk(min(K, m)).indices
+        s = torch.zeros(m, m, dtype=torch.bool, device=DEV).scatter_(1, top, True) & (pos[None, :] <= pos[:, None])
+        sel[a:a + m, a:a + m] = s
+        n[a:a + m] = s.sum(1).int()
+        order = torch.where(s, pos[None, :], m).sort(1).values[:, :K]
+        idx[a:a + m, :order.shape[1]] = torch.where(order < m, order + a, -1).int()
+        a += m
+        cu.append(a)
+    cu = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    out, lse = ops.attn_fwd(q, k, v, idx, n, cu, max(lens), scale, True)[:2]
+    dq, dk, dv = ops.attn_bwd(dout, q, k, v, out, lse, idx, n, cu, max(lens), scale, causal=True)
+    again = ops.attn_bwd(dout, q, k, v, out, lse, idx, n, cu, max(lens), scale, causal=True)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip((dq, dk, dv), again))
+    for h in range(0, Hkv, 9):
+        rows = slice(h * G, (h + 1) * G)
+        want = _reference(q[:, rows], k[:, h:h + 1], v[:, h:h + 1], dout[:, rows], sel, scale)
+        for name, got, ref in (("out", out[:, rows], want[0]), ("dq", dq[:, rows], want[2]), ("dk", dk[:, h:h + 1], want[3]), ("dv", dv[:, h:h + 1], want[4])):
+            assert_close_bf16(got, ref, f"{name} of kv head {h}")

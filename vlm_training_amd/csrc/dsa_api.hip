@@ -26,6 +26,9 @@ hipError_t dsa_launch_sel_fwd(const void *q, const void *k, const void *v, const
 hipError_t dsa_launch_sel_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
                              const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float scale, int pos_min,
                              int pos_max, int split_len, void *dq, hipStream_t stream);
+hipError_t dsa_launch_selkv(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
+                            const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, float scale, int split_len,
+                            void *dk, void *dv, hipStream_t stream);
 hipError_t dsa_launch_delta(const void *dout, const void *out, int T, int Hq, int D, float *delta, hipStream_t stream);
 hipError_t dsa_launch_bitmap(const int32_t *idx, const int32_t *n, const int32_t *cu, int N, int T, int K, int ldw,
                              uint32_t *bitmap, hipStream_t stream);
@@ -50,7 +53,7 @@ hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, co
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                               int Hq, int Hkv, int D, float scale, int causal, int32_t *order, int listed, float *partial,
+                               int Hq, int Hkv, int D, float scale, int causal, int skip_len, int32_t *order, int listed, float *partial,
                                size_t partial_bytes, void *dk, void *dv, hipStream_t stream);
 hipError_t dsa_launch_tile_order_delta(const void *dout, const void *out, const int32_t *cu, int N, int T, int Hq, int Hkv, int D,
                                        int has_idx, int causal, int32_t *order, const float *partial, size_t partial_bytes,
@@ -306,6 +309,19 @@ static RowSplit row_split_for(const int32_t *idx, int Hq, int Hkv, int D, int K)
     const int crossover = g_tile_crossover.load(std::memory_order_relaxed), G = Hq / Hkv;
     if (crossover == DSA_TILE_CROSSOVER && D == 128 && G >= 2 && G <= 4) return {line(16), line(G == 2 ? 150 : 75), line(18)};
     return {line(crossover), line(crossover), 0};
+}
+
+// The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,
+// three and more heads per kv head, launches that the tile kernel does not cut into pieces (its workgroups, 192 keys each, are cut nowhere: four
+// rounds of them end level).  Tile kernel -> walk, whole backward, ms, 32 heads over 8 kv heads, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5,
+// 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226; K = 512, 57 344 tokens 50.8 -> 33.7; K = 1024, 65 536 tokens, 4 heads over each of
+// 4 kv heads 35.2 -> 28.7, 8 over each of 8 134 -> 102, 16 over each of 8 255 -> 182.
+static int key_walk_len(const int32_t *idx, const void *q, const void *dout, int T, int N, int Hq, int Hkv, int D, int K) {
+    const int G = Hq / Hkv;
+    if (!idx || D != 128 || G < 3 || ((int64_t)T / 128 + N) * Hkv <= dkv_pieces_max_wg(D) || (((uintptr_t)q | (uintptr_t)dout) & 15) ||
+        g_tile_crossover.load(std::memory_order_relaxed) != DSA_TILE_CROSSOVER)
+        return INT32_MAX;
+    return (int)std::min<int64_t>((int64_t)K * 26, INT32_MAX);
 }
 
 extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_idx) {
@@ -620,12 +636,16 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
         sq = ov->aux;
     }
     int rc = DSA_OK;
+    const int walk_len = key_walk_len(idx, q, dout, T, N, Hq, Hkv, D, K);
+    auto key_side = [&]() {
+        hipError_t e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, walk_len, order, listed,
+                                           partial, partial_bytes, dk, dv, st);
+        if (e == hipSuccess && max_seqlen >= walk_len)
+            e = dsa_launch_selkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, softmax_scale, walk_len, dk, dv, st);
+        return e == hipSuccess ? DSA_OK : hip_fail(e, "dkv launch");
+    };
     // (side by side, the key side is issued first: it is the longer pass and starts with its longest walks)
-    if (ov) {
-        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, listed, partial,
-                                partial_bytes, dk, dv, st);
-        if (e != hipSuccess) rc = hip_fail(e, "tile dkv launch");
-    }
+    if (ov) rc = key_side();
     if (rc == DSA_OK && (parts & DSA_BWD_DQ)) {
         if (rows.tiles > 0) {
             e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len, causal, dq,
@@ -641,11 +661,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
             if (e != hipSuccess) rc = hip_fail(e, "gather dq launch");
         }
     }
-    if (rc == DSA_OK && !ov && (parts & DSA_BWD_DKV)) {
-        e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, order, listed, partial,
-                                partial_bytes, dk, dv, st);
-        if (e != hipSuccess) rc = hip_fail(e, "tile dkv launch");
-    }
+    if (rc == DSA_OK && !ov && (parts & DSA_BWD_DKV)) rc = key_side();
     if (ov) {                                            // joined also after a failed launch: the caller's stream stays whole
         e = hipEventRecord(ov->join, ov->aux);
         if (e == hipSuccess) e = hipStreamWaitEvent(st, ov->join, 0);

@@ -685,12 +685,12 @@ extern "C" hipError_t dsa_launch_tile_order_delta(const void *dout, const void *
 }
 extern "C" hipError_t dsa_launch_dkv_tiles(unsigned grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                                            const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                                           int T, int Hq, int Hkv, int d_real, float scale, int causal, const int32_t *order, float *partial,
+                                           int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len, const int32_t *order, float *partial,
                                            void *dk, void *dv);
 // listed: dsa_launch_tile_order_delta has left the list in `order`
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
-                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal,
+                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len,
                                           int32_t *order, int listed, float *partial, size_t partial_bytes, void *dk, void *dv,
                                           hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
@@ -699,7 +699,7 @@ extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const
     if (!p.listed) order = nullptr;
     else if (!listed) hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, p.o, order);
     if (!p.pieces) partial = nullptr;
-    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv);
+    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, skip_len, order, partial, dk, dv);
     if (e != hipSuccess) return e;
     if (p.pieces)
         hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(p.tiles_ub, Hkv, p.pitch / 8), dim3(256), 0, stream, order,

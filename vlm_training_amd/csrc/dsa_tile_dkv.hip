@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv,
-    float scale, float logit_scale, int causal, int d_real, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
+    float scale, float logit_scale, int causal, int d_real, int skip_len, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
     bf16_t *__restrict__ dv) {
     typedef DirectTile<D> TL;
     constexpr int RING = dkv_ring<D, KG>(), NW = 4 / KG, KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     int s0, L, blk, piece, mslot, pb;
     if (!locate_key_tile(order, cu, N, blockIdx.x / Hkv, s0, L, blk, piece, mslot, pb)) return;
     if (HAS_IDX) L = min(L, ldw * 32);                   // a bitmap row has ldw words whatever the caller's max_seqlen
-    if (blk * 128 >= L) return;                          // (whole workgroup, before its first barrier)
+    if (blk * 128 >= L || (HAS_IDX && L >= skip_len)) return;     // (whole workgroup, before its first barrier; long segments may be the compacted walk's)
     const int c0 = blk * 128, kc = c0 + wv * 32 * KG;    // the wave's first key
     const float scale_log2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(logit_scale * LOG2E_F))), inv_scale = 1.f / logit_scale;
     // the walk: queries q0 .. Lq-1 in nblocks steps (step s handles block nblocks-1-s) - all queries that can see this key tile, or
@@ -512,7 +512,7 @@ struct DkvArgs {
     const int32_t *cu;
     int N, T, Hq, Hkv, d_real;
     float scale, logit_scale;
-    int causal;
+    int causal, skip_len;
     const int32_t *order;
     float *partial;
     void *dk, *dv;
@@ -525,7 +525,7 @@ static hipError_t launch_dkv(unsigned grid, hipStream_t stream, const DkvArgs &a
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256 / KG), lds, stream, (const bf16_t *)a.dout, (const bf16_t *)a.q, (const bf16_t *)a.k,
-                       (const bf16_t *)a.v, a.lse, a.delta, a.bitmap, a.ldw, a.cu, a.N, a.T, a.Hq, a.Hkv, a.scale, a.logit_scale, a.causal, a.d_real, a.order,
+                       (const bf16_t *)a.v, a.lse, a.delta, a.bitmap, a.ldw, a.cu, a.N, a.T, a.Hq, a.Hkv, a.scale, a.logit_scale, a.causal, a.d_real, a.skip_len, a.order,
                        a.partial, (bf16_t *)a.dk, (bf16_t *)a.dv);
     return hipGetLastError();
 }
@@ -553,7 +553,7 @@ static hipError_t launch_dkv_kg(unsigned grid, hipStream_t stream, const DkvArgs
 // grid: workgroups (one per key tile or piece, and kv head).  The file is compiled twice, the second time (DKV_UNALIGNED) for q or dO on no
 // 16-byte boundary; k and v lie on one (the entry points see to it).
 #define DKV_LAUNCH_ARGS unsigned grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v, const float *lse, \
-    const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal,   \
+    const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len,   \
     const int32_t *order, float *partial, void *dk, void *dv
 extern "C" hipError_t dsa_launch_dkv_tiles_unaligned(DKV_LAUNCH_ARGS);
 #if DKV_UNALIGNED
@@ -561,9 +561,9 @@ extern "C" hipError_t dsa_launch_dkv_tiles_unaligned(DKV_LAUNCH_ARGS) {
 #else
 extern "C" hipError_t dsa_launch_dkv_tiles(DKV_LAUNCH_ARGS) {
     if (((uintptr_t)q | (uintptr_t)dout) & 15)
-        return dsa_launch_dkv_tiles_unaligned(grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, order, partial, dk, dv);
+        return dsa_launch_dkv_tiles_unaligned(grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, skip_len, order, partial, dk, dv);
 #endif
-    const DkvArgs a{dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, logit_scale(scale), causal, order, partial, dk, dv};
+    const DkvArgs a{dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, logit_scale(scale), causal, skip_len, order, partial, dk, dv};
     if (bitmap) switch (d_real) {
         case 64: return launch_dkv_kg<64, true>(grid, stream, a);
         case 128: return launch_dkv_kg<128, true>(grid, stream, a);

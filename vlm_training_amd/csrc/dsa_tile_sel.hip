@@ -15,29 +15,15 @@
 // 16 K of 131 072 tokens, K = 2048, 32 heads over 8 kv heads, the whole forward / backward, ms: gathered 94.5 / 299; here with eight waves and a step's
 // chain of reads and MFMAs open to its latency 76 / 297, twelve waves, lists built a block ahead 65 / 293, operands read ahead and nothing spilled
 // 56 / 280, exponentials behind the MFMAs of dP 57 / 275.  With twelve waves a spilled register read in the loop waits for the blocks on their way into LDS (+ 25 %).
-#include "dsa_tile.h"
+#include "dsa_sel.h"
 
 #define SEL_KEYS 128                                     // keys of a block
-#define SEL_LOADERS 8                                    // waves that request K and V
 #define SEL_AHEAD 2                                      // operands read ahead
 // waves of a workgroup: three to a SIMD (more hide more of a step's chain of reads and MFMAs), two for dQ
 constexpr int sel_waves(bool bwd) { return bwd ? 8 : 12; }
-// Rows of a block lie one behind the other; chunk c of row r (16 bytes) sits at position c ^ x(r).  x depends on the row's class r & 15:
-// sixteen rows of different classes at one chunk (row-wise operand) and four rows of neighbouring classes at four neighbouring chunks
-// (transposed operand) each cover the 64 banks once.
-struct SelBlock {
-    static constexpr int D = 128, ROW_B = 2 * D, CPR = D / 8, BYTES = SEL_KEYS * ROW_B;
-    static constexpr int LOAD_ROWS = 1024 / ROW_B, LOADS = BYTES / 1024, LPW = LOADS / SEL_LOADERS;   // wave loads of a block
-    static_assert(SEL_LOADERS * LOAD_ROWS % 16 == 0, "a wave's loads are of rows of the same classes");
-    __device__ __forceinline__ static int xor_of(int cl) { return (cl & 3) << 2 | cl >> 2; }
-    // a row's list entry: where it lies, its XOR in the place of the chunk
-    __device__ __forceinline__ static int entry(int r) { return r * ROW_B | xor_of(r & 15) << 4; }
-};
 // LDS: two blocks of K and V | of each wave: selection words of three blocks, two lists
 constexpr int SEL_WORD_B = 256, SEL_LIST_B = SEL_KEYS * 4, SEL_WAVE_B = 3 * SEL_WORD_B + 2 * SEL_LIST_B;
-constexpr size_t sel_lds_bytes(bool bwd) { return 4 * (size_t)SelBlock::BYTES + sel_waves(bwd) * SEL_WAVE_B; }
-
-template <class T> __device__ __forceinline__ T lds_read(uint32_t at) { return *(__attribute__((address_space(3))) const T *)at; }
+constexpr size_t sel_lds_bytes(bool bwd) { return 4 * (size_t)SelBlock<SEL_KEYS>::BYTES + sel_waves(bwd) * SEL_WAVE_B; }
 
 // BWD: dQ (acc, out = dq) instead of the forward (acc, out, lse)
 template <int GSHIFT, bool BWD>
@@ -46,7 +32,7 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
     const float *__restrict__ lse_in, const float *__restrict__ delta, const uint32_t *__restrict__ bitmap, int ldw,
     const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, float scale, float logit_scale_, int pos_min, int pos_max, int split_len, bf16_t *__restrict__ out,
     float *__restrict__ lse) {
-    typedef SelBlock BL;
+    typedef SelBlock<SEL_KEYS> BL;
     constexpr int D = BL::D, KS = D / 16, DT = D / 32, QW = 32 >> GSHIFT, NW = sel_waves(BWD), QBW = NW * QW;
     extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_lds[];
 
@@ -69,8 +55,7 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
     const uint32_t lds0 = lds_address(dyn_lds);
     const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k + ((int64_t)s0 * Hkv + kvh) * D);
     const unsigned char *vptr = reinterpret_cast<const unsigned char *>(v + ((int64_t)s0 * Hkv + kvh) * D);
-    const int lrow = wv * BL::LOAD_ROWS + lane / BL::CPR;                 // (a wave's later loads lie whole rows of the buffer further on)
-    const int voff[1] = {lrow * tok_b + ((lane % BL::CPR) ^ BL::xor_of(lrow & 15)) * 16};
+    const int voff[1] = {BL::load_row(wv, lane) * tok_b + BL::load_chunk(wv, lane) * 16};       // (a wave's later loads lie whole rows of the buffer further on)
     const int q0 = qc0 + wv * QW, wq0 = min(q0, L - 1);                   // the wave's first query
     const unsigned char *wptr = reinterpret_cast<const unsigned char *>(bitmap + (int64_t)(s0 + wq0) * ldw);
     const int wave_at = 4 * BL::BYTES + wv * SEL_WAVE_B;
@@ -155,7 +140,7 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
         list[lane] = e0;
         list[lane + 64] = e0;
         if (m0) list[r0] = e0 | m0;
-        if (m1) list[r0 + (m0 ? 1 : 0)] = (e0 + ((uint32_t)(16 * BL::ROW_B) << 16)) | m1;
+        if (m1) list[r0 + (m0 ? 1 : 0)] = (e0 + ((uint32_t)BL::entry(16) << 16)) | m1;
         return (int)__popcll(b0) + (int)__popcll(b1);
     };
     wait_vmcnt<0>();
@@ -175,18 +160,19 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
         int n_next = 0;
         auto step = [&](auto first_, int st) __attribute__((always_inline)) {
             constexpr bool FIRST = decltype(first_)::value;
-            const int er = (lds_read<uint16_t>(er_at + list_at + 4 * st) | at) ^ (h << 4);
+            const int er = (lds_read<uint16_t>(er_at + list_at + 4 * st) | at) ^ (h << 4), er1 = er ^ 32;
             int et[4];
             const uint32_t ets = et_at + list_at + 4 * st, sets = set_at + list_at + 4 * st;
 #pragma unroll
             for (int u = 0; u < 4; ++u) et[u] = (lds_read<uint16_t>(ets + 64 * (u & 1) + 4 * (u >> 1)) | at) ^ tr_in;
             u32x4 set[4];                                // of slots 8 u + 4 h + i: element (u / 2 + 2 i) % 4 of set[2 (u % 2) + i / 2]
             auto row_op = [&](int ks, int operand) __attribute__((always_inline)) {
-                return *((__attribute__((address_space(3))) const bf16x8 *)((er ^ (ks << 5)) + operand * BL::BYTES));
+                return lds_read<bf16x8>((ks & 1 ? er1 : er) + (ks >> 1) * BL::COLUMN_B + operand * BL::BYTES);
             };
             auto tr_op = [&](int i) __attribute__((always_inline)) {                    // keys of half i / DT, d-tile i % DT
                 const int pair = i / DT, dt = i % DT;
-                return tr_pair((lds_u8 *)((et[2 * pair] ^ (dt << 6)) + (BWD ? 0 : BL::BYTES)), (lds_u8 *)((et[2 * pair + 1] ^ (dt << 6)) + (BWD ? 0 : BL::BYTES)));
+                constexpr int OPERAND = BWD ? 0 : BL::BYTES;
+                return tr_pair((lds_u8 *)(et[2 * pair] + dt * BL::COLUMN_B + OPERAND), (lds_u8 *)(et[2 * pair + 1] + dt * BL::COLUMN_B + OPERAND));
             };
             auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
             constexpr int NR = BWD ? 2 * KS : KS, NT = 2 * DT;
