@@ -164,6 +164,25 @@ int dsa_attn_fwd_saved_bitmap(const void *q, const void *k, const void *v, const
                               int dtype, int max_seqlen, int causal, void *out, float *lse, const void *bitmap,
                               size_t bitmap_bytes, void *stream);
 
+/*
+ * The same without idx and n, for callers that never look at them: dsa_index_topk_words leaves the bitmap alone, and
+ * dsa_attn_fwd_words / dsa_attn_bwd_words are dsa_attn_fwd_saved_bitmap / dsa_attn_bwd_saved_bitmap on such a bitmap
+ * (K: the top_k it was made with).  dsa_attn_reads_list says (1) whether those two would hand rows of segments up to
+ * max_seqlen to kernels that gather by the list; the calls here keep every row on the kernels that read the bitmap, right
+ * for any row and the same bits where the answer is 0, slower than the gather where it is 1.
+ */
+int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen);
+int dsa_index_topk_words(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu_seqlens, int T, int N,
+                         int Hi, int Di, int K, float scale, int dtype, int max_seqlen, void *bitmap, size_t bitmap_bytes,
+                         void *ws, size_t ws_bytes, void *stream);
+int dsa_attn_fwd_words(const void *q, const void *k, const void *v, const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv,
+                       int D, int K, float softmax_scale, int dtype, int max_seqlen, void *out, float *lse,
+                       const void *bitmap, size_t bitmap_bytes, void *stream);
+int dsa_attn_bwd_words(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
+                       const int32_t *cu_seqlens, int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale,
+                       int dtype, int max_seqlen, void *dq, void *dk, void *dv, const void *bitmap, size_t bitmap_bytes,
+                       void *scratch, size_t scratch_bytes, void *stream);
+
 /* Bytes of workspace dsa_attn_fwd needs (the inverted selection bitmap; 0 without idx). */
 size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_idx);
 

@@ -52,6 +52,14 @@ _SIGNATURES = {
     "dsa_get_tile_crossover": (c_int, []),
     "dsa_index_topk_bitmap": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                       c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
+    "dsa_attn_reads_list": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "dsa_index_topk_words": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                                     c_int, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
+    "dsa_attn_fwd_words": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                                   c_int, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "dsa_attn_bwd_words": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                   c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p,
+                                   c_size_t, c_void_p]),
     "dsa_attn_fwd_saved_bitmap": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                           c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
                                           c_size_t, c_void_p]),

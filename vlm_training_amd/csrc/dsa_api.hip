@@ -165,11 +165,11 @@ static inline int bitmap_ldw(int max_seqlen) { return (max_seqlen + 31) / 32; } 
 // the selected keys are kept; bitmap != NULL: the top-k kernel also leaves the inverted selection there
 static int index_topk_impl(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu, int T, int N,
                            int Hi, int Di, int K, float scale, int dtype, int max_seqlen, int32_t *idx, int32_t *n,
-                           float *sel_scores, uint32_t *bitmap, void *ws, size_t ws_bytes, void *stream) {
+                           float *sel_scores, uint32_t *bitmap, void *ws, size_t ws_bytes, void *stream, bool words_only = false) {
     if (int rc = check_packed(T, N, cu)) return rc;
     if (K < 1) return fail(DSA_ERR_ARG, "top_k=%d must be >= 1", K);
     if (max_seqlen < 1 || max_seqlen > T) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
-    if (!idx || !n) return fail(DSA_ERR_ARG, "null output pointer");
+    if ((!idx || !n) && !words_only) return fail(DSA_ERR_ARG, "null output pointer");
     if (T == 0) return DSA_OK;
     const int64_t ld = score_ld(max_seqlen);
     int64_t rows = ws ? (int64_t)(ws_bytes / ((size_t)ld * 4)) : 0;
@@ -259,16 +259,16 @@ extern "C" int dsa_indexer_kl(const float *sel_scores, const float *mass, const 
     return e == hipSuccess ? DSA_OK : hip_fail(e, "indexer KL launch");
 }
 
-static int check_attn(int T, int N, const int32_t *cu, int Hq, int Hkv, int D, int K, int dtype, const int32_t *idx,
+static int check_attn(int T, int N, const int32_t *cu, int Hq, int Hkv, int D, int K, int dtype, bool selected, const int32_t *idx,
                       const int32_t *n) {
     if (int rc = check_packed(T, N, cu)) return rc;
     if (dtype != DSA_DTYPE_BF16) return fail(DSA_ERR_UNSUPPORTED, "q/k/v must be bf16 (dtype code %d)", dtype);
     if (Hq < 1 || Hkv < 1 || Hq % Hkv) return fail(DSA_ERR_ARG, "Hq=%d must be a positive multiple of Hkv=%d", Hq, Hkv);
     if (Hq / Hkv > 16) return fail(DSA_ERR_UNSUPPORTED, "Hq/Hkv=%d: at most 16 query heads per kv head", Hq / Hkv);
-    if (!(D == 64 || D == 128 || D == 256 || (D == 96 && !idx)))
+    if (!(D == 64 || D == 128 || D == 256 || (D == 96 && !selected)))
         return fail(DSA_ERR_UNSUPPORTED, "head_dim=%d: need 64, 128 or 256 (96 as well without a key selection)", D);
     if ((idx == nullptr) != (n == nullptr)) return fail(DSA_ERR_ARG, "idx and n must both be given or both be null");
-    if (idx && K < 1) return fail(DSA_ERR_ARG, "top_k=%d must be >= 1", K);
+    if (selected && K < 1) return fail(DSA_ERR_ARG, "top_k=%d must be >= 1", K);
     if ((int64_t)T * Hkv >= ((int64_t)1 << 31)) return fail(DSA_ERR_UNSUPPORTED, "T*Hkv too large for one launch");
     return DSA_OK;
 }
@@ -300,15 +300,22 @@ struct RowSplit {
     int tiles, walk, len;
     bool past_tiles(int max_seqlen) const { return max_seqlen > tiles && max_seqlen >= len; }
 };
-static RowSplit row_split_for(const int32_t *idx, int Hq, int Hkv, int D, int K) {
-    if (!idx) return {INT32_MAX, INT32_MAX, 0};       // dense causal: tiles everywhere
+static RowSplit row_split_for(bool selected, const int32_t *idx, int Hq, int Hkv, int D, int K) {
+    if (!selected) return {INT32_MAX, INT32_MAX, 0};       // dense causal: tiles everywhere
     auto line = [&](int64_t times) {
         const int64_t p = K * times;
         return p >= INT32_MAX - 256 ? INT32_MAX : (int)((p + 255) / 256 * 256);
     };
     const int crossover = g_tile_crossover.load(std::memory_order_relaxed), G = Hq / Hkv;
-    if (crossover == DSA_TILE_CROSSOVER && D == 128 && G >= 2 && G <= 4) return {line(16), line(G == 2 ? 150 : 75), line(18)};
+    const bool walks = crossover == DSA_TILE_CROSSOVER && D == 128 && G >= 2 && G <= 4;
+    if (!idx) return {walks ? line(16) : INT32_MAX, INT32_MAX, walks ? line(18) : 0};    // (no list to gather by)
+    if (walks) return {line(16), line(G == 2 ? 150 : 75), line(18)};
     return {line(crossover), line(crossover), 0};
+}
+extern "C" int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen) {
+    if (Hkv < 1 || Hq < Hkv || K < 1) return 1;
+    static const int32_t some = 0;
+    return max_seqlen > row_split_for(true, &some, Hq, Hkv, D, K).walk;
 }
 
 // The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,
@@ -316,9 +323,9 @@ static RowSplit row_split_for(const int32_t *idx, int Hq, int Hkv, int D, int K)
 // rounds of them end level).  Tile kernel -> walk, whole backward, ms, 32 heads over 8 kv heads, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5,
 // 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226; K = 512, 57 344 tokens 50.8 -> 33.7; K = 1024, 65 536 tokens, 4 heads over each of
 // 4 kv heads 35.2 -> 28.7, 8 over each of 8 134 -> 102, 16 over each of 8 255 -> 182.
-static int key_walk_len(const int32_t *idx, const void *q, const void *dout, int T, int N, int Hq, int Hkv, int D, int K) {
+static int key_walk_len(bool selected, const void *q, const void *dout, int T, int N, int Hq, int Hkv, int D, int K) {
     const int G = Hq / Hkv;
-    if (!idx || D != 128 || G < 3 || ((int64_t)T / 128 + N) * Hkv <= dkv_pieces_max_wg(D) || (((uintptr_t)q | (uintptr_t)dout) & 15) ||
+    if (!selected || D != 128 || G < 3 || ((int64_t)T / 128 + N) * Hkv <= dkv_pieces_max_wg(D) || (((uintptr_t)q | (uintptr_t)dout) & 15) ||
         g_tile_crossover.load(std::memory_order_relaxed) != DSA_TILE_CROSSOVER)
         return INT32_MAX;
     return (int)std::min<int64_t>((int64_t)K * 26, INT32_MAX);
@@ -330,22 +337,22 @@ extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_id
 }
 
 // build_bitmap == 0: ws already holds the bitmap of idx/n (it is only read)
-static int attn_fwd_run(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n, const int32_t *cu,
+static int attn_fwd_run(const void *q, const void *k, const void *v, bool selected, const int32_t *idx, const int32_t *n, const int32_t *cu,
                         int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, int causal,
                         void *out, float *lse, void *ws, size_t ws_bytes, int build_bitmap, void *stream) {
-    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
-    if (!causal && idx) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
+    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, selected, idx, n)) return rc;
+    if (!causal && selected) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
     if (!q || !k || !v || !out || !lse) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
-    const RowSplit rows = row_split_for(idx, Hq, Hkv, D, K);
+    const RowSplit rows = row_split_for(selected, idx, Hq, Hkv, D, K);
     const int ldw = bitmap_ldw(max_seqlen);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = hipSuccess;
     if (rows.tiles > 0) {
         uint32_t *bitmap = nullptr;
-        if (idx) {
+        if (selected) {
             const size_t need = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
             if (!ws || ws_bytes < need) return fail(DSA_ERR_WORKSPACE, "forward workspace: have %zu bytes, need %zu", ws_bytes, need);
             if ((size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
@@ -374,7 +381,7 @@ extern "C" int dsa_attn_fwd(const void *q, const void *k, const void *v, const i
                             const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale,
                             int dtype, int max_seqlen, int causal, void *out, float *lse, void *ws, size_t ws_bytes,
                             void *stream) {
-    return attn_fwd_run(q, k, v, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, causal, out, lse, ws, ws_bytes,
+    return attn_fwd_run(q, k, v, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, causal, out, lse, ws, ws_bytes,
                         1, stream);
 }
 
@@ -383,7 +390,14 @@ extern "C" int dsa_attn_fwd_saved_bitmap(const void *q, const void *k, const voi
                                          int dtype, int max_seqlen, int causal, void *out, float *lse, const void *bitmap,
                                          size_t bitmap_bytes, void *stream) {
     if (!idx) return fail(DSA_ERR_ARG, "a saved bitmap belongs to a selection: idx is null");
-    return attn_fwd_run(q, k, v, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, causal, out, lse,
+    return attn_fwd_run(q, k, v, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, causal, out, lse,
+                        const_cast<void *>(bitmap), bitmap_bytes, 0, stream);
+}
+
+extern "C" int dsa_attn_fwd_words(const void *q, const void *k, const void *v, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
+                                  float softmax_scale, int dtype, int max_seqlen, void *out, float *lse, const void *bitmap, size_t bitmap_bytes,
+                                  void *stream) {
+    return attn_fwd_run(q, k, v, true, nullptr, nullptr, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, 1, out, lse,
                         const_cast<void *>(bitmap), bitmap_bytes, 0, stream);
 }
 
@@ -399,6 +413,17 @@ extern "C" int dsa_index_topk_bitmap(const void *q_idx, const void *k_idx, const
                            (uint32_t *)bitmap, ws, ws_bytes, stream);
 }
 
+extern "C" int dsa_index_topk_words(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu, int T, int N, int Hi, int Di, int K,
+                                    float scale, int dtype, int max_seqlen, void *bitmap, size_t bitmap_bytes, void *ws, size_t ws_bytes,
+                                    void *stream) {
+    if (T > 0 && max_seqlen >= 1) {
+        const size_t need = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
+        if (!bitmap || bitmap_bytes < need) return fail(DSA_ERR_WORKSPACE, "selection bitmap: have %zu bytes, need %zu", bitmap_bytes, need);
+    }
+    return index_topk_impl(q_idx, k_idx, w_idx, cu, T, N, Hi, Di, K, scale, dtype, max_seqlen, nullptr, nullptr, nullptr, (uint32_t *)bitmap, ws,
+                           ws_bytes, stream, true);
+}
+
 // ---- attention mass of the selected keys (training target of the indexer) ---------------------------
 // bitmap + one (T,K) fp32 table per group of kv heads (none when one group takes all kv heads)
 extern "C" size_t dsa_attn_mass_workspace_bytes(int T, int N, int Hq, int Hkv, int D, int K, int max_seqlen) {
@@ -412,7 +437,7 @@ extern "C" size_t dsa_attn_mass_workspace_bytes(int T, int N, int Hq, int Hkv, i
 static int attn_mass_run(const void *q, const void *k, const float *lse, const int32_t *idx, const int32_t *n, const int32_t *cu,
                          int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, float *mass,
                          const void *saved_bitmap, size_t saved_bytes, void *ws, size_t ws_bytes, void *stream) {
-    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
+    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx != nullptr, idx, n)) return rc;
     if (!q || !k || !lse || !idx || !n || !mass) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (int rc = check_aligned(k, k, "k")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
@@ -590,12 +615,12 @@ extern "C" size_t dsa_attn_bwd_bitmap_offset(int T, int Hq) {
 
 // the backward proper: every buffer named, so that the two entry points below differ only in where the buffers live
 static int attn_bwd_run(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
-                        const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
+                        bool selected, const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
                         float softmax_scale, int max_seqlen, int causal, void *dq, void *dk, void *dv, float *delta,
                         uint32_t *bitmap, float *partial, size_t partial_bytes, int32_t *order, int parts, hipStream_t st) {
     const int ldw = bitmap_ldw(max_seqlen);
-    if (idx && (size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
-    const RowSplit rows = row_split_for(idx, Hq, Hkv, D, K);
+    if (selected && (size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
+    const RowSplit rows = row_split_for(selected, idx, Hq, Hkv, D, K);
     hipError_t e = hipSuccess;
     // the two passes side by side on two streams: launches of few workgroups only (larger ones fill the GPU alone)
     std::unique_lock<std::mutex> ov_lock;
@@ -616,7 +641,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.past_tiles(max_seqlen) && !ov;
     int listed = 0;                                      // the launch order of the key tiles is there
     if ((parts & DSA_BWD_DELTA) && ov) {
-        e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, idx != nullptr, causal, order, partial, partial_bytes, delta, st);
+        e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, selected, causal, order, partial, partial_bytes, delta, st);
         if (e == hipSuccess) listed = 1;
         else if (e != hipErrorNotReady) return hip_fail(e, "order and delta launch");   // (not ready: this launch needs no list)
     }
@@ -636,7 +661,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
         sq = ov->aux;
     }
     int rc = DSA_OK;
-    const int walk_len = key_walk_len(idx, q, dout, T, N, Hq, Hkv, D, K);
+    const int walk_len = key_walk_len(selected, q, dout, T, N, Hq, Hkv, D, K);
     auto key_side = [&]() {
         hipError_t e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, walk_len, order, listed,
                                            partial, partial_bytes, dk, dv, st);
@@ -671,10 +696,10 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
 }
 
 static int check_bwd(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
-                     const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
+                     bool selected, const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
                      int dtype, int max_seqlen, int causal, const void *dq, const void *dk, const void *dv) {
-    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx, n)) return rc;
-    if (!causal && idx) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
+    if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, selected, idx, n)) return rc;
+    if (!causal && selected) return fail(DSA_ERR_ARG, "a key selection (idx) implies causal attention");
     if (!dout || !q || !k || !v || !out || !lse || !dq || !dk || !dv) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
@@ -686,7 +711,7 @@ extern "C" int dsa_attn_bwd_parts(const void *dout, const void *q, const void *k
                                   int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen,
                                   int causal, void *dq, void *dk, void *dv, void *ws, size_t ws_bytes, int parts,
                                   void *stream) {
-    if (int rc = check_bwd(dout, q, k, v, out, lse, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
+    if (int rc = check_bwd(dout, q, k, v, out, lse, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
     if (T == 0) return DSA_OK;
     const size_t need = dsa_attn_bwd_workspace_bytes(T, Hq, max_seqlen, idx != nullptr);
     if (!ws || ws_bytes < need) return fail(DSA_ERR_WORKSPACE, "backward workspace: have %zu bytes, need %zu", ws_bytes, need);
@@ -695,7 +720,7 @@ extern "C" int dsa_attn_bwd_parts(const void *dout, const void *q, const void *k
     int32_t *order = (int32_t *)((char *)ws + need - align_up(dsa_tile_order_bytes(T), 256));
     const size_t partial_bytes = dsa_tile_dkv_partial_bytes(T);
     float *partial = partial_bytes ? (float *)((char *)order - align_up(partial_bytes, 256)) : nullptr;
-    return attn_bwd_run(dout, q, k, v, out, lse, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
+    return attn_bwd_run(dout, q, k, v, out, lse, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
                         delta, bitmap, partial, partial_bytes, order, parts, (hipStream_t)stream);
 }
 
@@ -711,15 +736,14 @@ extern "C" size_t dsa_attn_bwd_scratch_bytes(int T, int N, int Hq, int Hkv, int 
            align_up(dsa_tile_order_bytes(T), 256);
 }
 
-extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const void *k, const void *v, const void *out,
-                                         const float *lse, const int32_t *idx, const int32_t *n, const int32_t *cu, int T,
-                                         int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype,
-                                         int max_seqlen, int causal, void *dq, void *dk, void *dv, const void *fwd_ws,
-                                         size_t fwd_ws_bytes, void *scratch, size_t scratch_bytes, void *stream) {
-    if (int rc = check_bwd(dout, q, k, v, out, lse, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
+static int attn_bwd_saved(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse, bool selected,
+                          const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale,
+                          int dtype, int max_seqlen, int causal, void *dq, void *dk, void *dv, const void *fwd_ws, size_t fwd_ws_bytes, void *scratch,
+                          size_t scratch_bytes, void *stream) {
+    if (int rc = check_bwd(dout, q, k, v, out, lse, selected, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
     if (T == 0) return DSA_OK;
-    if (idx) {
-        if (row_split_for(idx, Hq, Hkv, D, K).tiles <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
+    if (selected) {
+        if (row_split_for(selected, idx, Hq, Hkv, D, K).tiles <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
         const size_t have = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
         if (!fwd_ws || fwd_ws_bytes < have) return fail(DSA_ERR_WORKSPACE, "forward workspace (selection bitmap): have %zu bytes, need %zu", fwd_ws_bytes, have);
     }
@@ -730,9 +754,25 @@ extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const 
     float *partial = partial_bytes ? (float *)((char *)scratch + align_up((size_t)T * Hq * 4, 256)) : nullptr;
     int32_t *order = (int32_t *)((char *)scratch + need - align_up(dsa_tile_order_bytes(T), 256));
     // the kernels only read the bitmap; the forward's workspace is not written here
-    uint32_t *bitmap = idx ? const_cast<uint32_t *>((const uint32_t *)fwd_ws) : nullptr;
-    return attn_bwd_run(dout, q, k, v, out, lse, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
+    uint32_t *bitmap = selected ? const_cast<uint32_t *>((const uint32_t *)fwd_ws) : nullptr;
+    return attn_bwd_run(dout, q, k, v, out, lse, selected, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
                         delta, bitmap, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream);
+}
+
+extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const void *k, const void *v, const void *out,
+                                         const float *lse, const int32_t *idx, const int32_t *n, const int32_t *cu, int T,
+                                         int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype,
+                                         int max_seqlen, int causal, void *dq, void *dk, void *dv, const void *fwd_ws,
+                                         size_t fwd_ws_bytes, void *scratch, size_t scratch_bytes, void *stream) {
+    return attn_bwd_saved(dout, q, k, v, out, lse, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, causal, dq, dk, dv,
+                          fwd_ws, fwd_ws_bytes, scratch, scratch_bytes, stream);
+}
+
+extern "C" int dsa_attn_bwd_words(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse, const int32_t *cu,
+                                  int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, void *dq, void *dk,
+                                  void *dv, const void *bitmap, size_t bitmap_bytes, void *scratch, size_t scratch_bytes, void *stream) {
+    return attn_bwd_saved(dout, q, k, v, out, lse, true, nullptr, nullptr, cu, T, N, Hq, Hkv, D, K, softmax_scale, dtype, max_seqlen, 1, dq, dk, dv,
+                          bitmap, bitmap_bytes, scratch, scratch_bytes, stream);
 }
 
 extern "C" int dsa_dense_bwd_rows(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
@@ -740,14 +780,14 @@ extern "C" int dsa_dense_bwd_rows(const void *dout, const void *q, const void *k
                                   int max_seqlen, int causal, void *dq, void *dk, void *dv, void *scratch, size_t scratch_bytes,
                                   void *stream) {
     if (D < 8 || D > 128 || D % 8) return fail(DSA_ERR_UNSUPPORTED, "head_dim=%d: need a multiple of 8 up to 128", D);
-    if (int rc = check_bwd(dout, q, k, v, out, lse, nullptr, nullptr, cu, T, N, Hq, Hkv, 64, 0, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
+    if (int rc = check_bwd(dout, q, k, v, out, lse, false, nullptr, nullptr, cu, T, N, Hq, Hkv, 64, 0, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
     if (T == 0) return DSA_OK;
     const size_t need = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
     if (!scratch || scratch_bytes < need) return fail(DSA_ERR_WORKSPACE, "backward scratch: have %zu bytes, need %zu", scratch_bytes, need);
     const size_t partial_bytes = bwd_partial_bytes_for(T, N, Hkv, D);
     float *partial = partial_bytes ? (float *)((char *)scratch + align_up((size_t)T * Hq * 4, 256)) : nullptr;
     int32_t *order = (int32_t *)((char *)scratch + need - align_up(dsa_tile_order_bytes(T), 256));
-    return attn_bwd_run(dout, q, k, v, out, lse, nullptr, nullptr, cu, T, N, Hq, Hkv, D, 0, softmax_scale, max_seqlen, causal, dq, dk, dv,
+    return attn_bwd_run(dout, q, k, v, out, lse, false, nullptr, nullptr, cu, T, N, Hq, Hkv, D, 0, softmax_scale, max_seqlen, causal, dq, dk, dv,
                         (float *)scratch, nullptr, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream);
 }
 
@@ -770,7 +810,7 @@ extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_hea
                                      int64_t v_tok, int64_t v_head, const int32_t *cu, int T, int N, int Hq, int Hkv, int D,
                                      float softmax_scale, int dtype, int max_seqlen, int causal, void *out, float *lse, void *stream) {
     if (D < 8 || D > 256 || D % 8) return fail(DSA_ERR_UNSUPPORTED, "head_dim=%d: need a multiple of 8 up to 256", D);
-    if (int rc = check_attn(T, N, cu, Hq, Hkv, 64, 0, dtype, nullptr, nullptr)) return rc;     // (head_dim checked above)
+    if (int rc = check_attn(T, N, cu, Hq, Hkv, 64, 0, dtype, false, nullptr, nullptr)) return rc;     // (head_dim checked above)
     if (!q || !k || !v || !out || !lse) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     const int64_t strides[6] = {q_tok, q_head, k_tok, k_head, v_tok, v_head};

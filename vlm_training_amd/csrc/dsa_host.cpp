@@ -87,23 +87,28 @@ double index_scale_of(std::optional<double> s, int64_t Hi, int64_t Di) {
 }
 
 struct Selection { Tensor idx, n, scores; };
-// selection of every row; `bitmap` (may be undefined) receives the inverted selection
+// selection of every row; `bitmap` (may be undefined) receives the inverted selection, alone without want_list
 Selection select_keys(const Tensor &qi, const Tensor &ki, const Tensor &wi, const Tensor &cu, int max_seqlen, int64_t K, double scale,
-                      bool want_scores, const Tensor &bitmap) {
+                      bool want_scores, const Tensor &bitmap, bool want_list = true) {
     TORCH_CHECK_VALUE(qi.dim() == 3 && ki.dim() == 2 && wi.dim() == 2, "indexer tensors must be q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi)");
     const int64_t T = qi.size(0), Hi = qi.size(1), Di = qi.size(2);
     TORCH_CHECK_VALUE(ki.size(0) == T && ki.size(1) == Di && wi.size(0) == T && wi.size(1) == Hi, "indexer tensor shapes disagree");
     TORCH_CHECK_VALUE(K >= 1, "top_k must be >= 1");
     Selection s;
-    s.idx = empty({T, K}, at::kInt, qi);
-    s.n = empty({T}, at::kInt, qi);
+    if (want_list) {
+        s.idx = empty({T, K}, at::kInt, qi);
+        s.n = empty({T}, at::kInt, qi);
+    }
     if (want_scores) s.scores = empty({T, K}, at::kFloat, qi);
     const size_t ws_bytes = (max_seqlen > K || want_scores) ? dsa_index_topk_workspace_bytes((int)T, max_seqlen, (int)K) : 0;
     const Tensor ws = empty_bytes(ws_bytes, qi);
     const IndexInputs in = index_inputs(qi, ki, wi);
-    int32_t *idx = s.idx.data_ptr<int32_t>(), *n = s.n.data_ptr<int32_t>();
+    int32_t *idx = const_cast<int32_t *>(iptr(s.idx)), *n = const_cast<int32_t *>(iptr(s.n));
     const int N = (int)cu.numel() - 1;
-    if (bitmap.defined())
+    if (!want_list)
+        check(dsa_index_topk_words(ptr(in.q), ptr(in.k), ptr(in.w), iptr(cu), (int)T, N, (int)Hi, (int)Di, (int)K, (float)scale, DSA_DTYPE_BF16,
+                                   max_seqlen, ptr(bitmap), (size_t)bitmap.numel(), ptr(ws), ws_bytes, stream_of(qi)), "dsa_index_topk_words");
+    else if (bitmap.defined())
         check(dsa_index_topk_bitmap(ptr(in.q), ptr(in.k), ptr(in.w), iptr(cu), (int)T, N, (int)Hi, (int)Di, (int)K, (float)scale, DSA_DTYPE_BF16,
                                     max_seqlen, idx, n, fptr(s.scores), ptr(bitmap), (size_t)bitmap.numel(), ptr(ws), ws_bytes, stream_of(qi)),
               "dsa_index_topk_bitmap");
@@ -129,16 +134,21 @@ struct AttnArgs {
     double scale;
     bool causal, want_mass, split;
     at::ScalarType dtype;
+    int64_t words_k;                                     // keys per row of a selection that is there as its bitmap alone, else 0
 };
+bool carried_split(at::ScalarType dtype, int64_t D) { return dtype == at::kFloat && 4 * D <= 256; }
 
 void attn_forward_kernels(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &idx, const Tensor &n, const Tensor &cu, const AttnArgs &a,
                           const Tensor &ws, bool bitmap_ready, const Tensor &out, const Tensor &lse) {
     const int T = (int)q.size(0), Hq = (int)q.size(1), D = (int)q.size(2), Hkv = (int)k.size(1), N = (int)cu.numel() - 1;
     const int K = idx.defined() ? (int)idx.size(1) : 0;
     const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-    if (!idx.defined() && D % 64)                        // rows between the kernels' head_dims, read where they lie
+    if (!idx.defined() && !a.words_k && D % 64)          // rows between the kernels' head_dims, read where they lie
         check(dsa_dense_fwd_strided(ptr(q), q.stride(0), D, ptr(k), k.stride(0), D, ptr(v), v.stride(0), D, iptr(cu), T, N, Hq, Hkv, D, (float)a.scale,
                                     DSA_DTYPE_BF16, (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
+    else if (a.words_k)
+        check(dsa_attn_fwd_words(ptr(q), ptr(k), ptr(v), iptr(cu), T, N, Hq, Hkv, D, (int)a.words_k, (float)a.scale, DSA_DTYPE_BF16, (int)a.max_seqlen,
+                                 ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd_words");
     else if (bitmap_ready)
         check(dsa_attn_fwd_saved_bitmap(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, DSA_DTYPE_BF16,
                                         (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd_saved_bitmap");
@@ -189,7 +199,7 @@ AttnForward attn_forward(const Tensor &q, const Tensor &k, const Tensor &v, cons
     f.lse = empty({Hq, T}, at::kFloat, q);
     // the selection bitmap - left by the top-k kernel (`bitmap`), else built by the forward - is kept for the backward
     // (with the tile crossover at 0 no kernel reads one)
-    const bool tiles = idx.defined() && dsa_get_tile_crossover() > 0;
+    const bool tiles = a.words_k || (idx.defined() && dsa_get_tile_crossover() > 0);
     if (tiles) f.ws = bitmap.defined() ? bitmap : empty_bytes(dsa_attn_fwd_workspace_bytes((int)T, (int)a.max_seqlen, 1), q);
     attn_forward_kernels(f.qb, f.kb, f.vb, idx, n, cu, a, f.ws, tiles && bitmap.defined(), f.out, f.lse);
     if (a.split) {
@@ -206,11 +216,12 @@ AttnForward attn_forward(const Tensor &q, const Tensor &k, const Tensor &v, cons
 class AttnNode : public torch::autograd::Function<AttnNode> {
 public:
     static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, const OptTensor &idx_,
-                                 const OptTensor &n_, const OptTensor &bitmap_, int64_t max_seqlen, double scale, bool causal, bool want_mass) {
+                                 const OptTensor &n_, const OptTensor &bitmap_, int64_t max_seqlen, double scale, bool causal, bool want_mass,
+                                 int64_t words_k) {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::OptionalDeviceGuard guard(q.device());
         const Tensor idx = idx_.value_or(Tensor()), n = n_.value_or(Tensor());
-        const AttnArgs a{max_seqlen, scale, causal, want_mass, q.scalar_type() == at::kFloat && 4 * q.size(2) <= 256, q.scalar_type()};
+        const AttnArgs a{max_seqlen, scale, causal, want_mass, carried_split(q.scalar_type(), q.size(2)), q.scalar_type(), words_k};
         const AttnForward f = attn_forward(q, k, v, cu, idx, n, bitmap_.value_or(Tensor()), a);
         ctx->save_for_backward({f.qb, f.kb, f.vb, f.out, f.lse, cu, idx, n, f.ws});
         ctx->saved_data["m"] = max_seqlen;
@@ -218,6 +229,7 @@ public:
         ctx->saved_data["c"] = causal;
         ctx->saved_data["t"] = (int64_t)a.dtype;
         ctx->saved_data["p"] = a.split;
+        ctx->saved_data["w"] = words_k;
         if (!want_mass) return {f.res};
         ctx->mark_non_differentiable({f.mass});
         ctx->set_materialize_grads(false);               // (no (T,K) table of zeros as the mass's gradient)
@@ -234,6 +246,7 @@ public:
         const int causal = ctx->saved_data["c"].toBool();
         const auto dtype = (at::ScalarType)ctx->saved_data["t"].toInt();
         const bool split = ctx->saved_data["p"].toBool();
+        const int words_k = (int)ctx->saved_data["w"].toInt();
         const int T = (int)q.size(0), Hq = (int)q.size(1), D = (int)q.size(2), Hkv = (int)k.size(1), N = (int)cu.numel() - 1;
         const int K = idx.defined() ? (int)idx.size(1) : 0;
         const Tensor g = grads[0].defined() ? grads[0] : at::zeros({T, Hq, split ? D / 4 : D}, out.options());
@@ -246,11 +259,17 @@ public:
             db = as_bf16(g);
         }
         Tensor dq = empty({T, Hq, D}, at::kBFloat16, q), dk = empty({T, Hkv, D}, at::kBFloat16, q), dv = empty({T, Hkv, D}, at::kBFloat16, q);
-        if (!idx.defined() && D % 64) {
+        if (!idx.defined() && !words_k && D % 64) {
             const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
             const Tensor scratch = empty_bytes(sc_bytes, q);
             check(dsa_dense_bwd_rows(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(cu), T, N, Hq, Hkv, D, (float)scale, DSA_DTYPE_BF16,
                                      max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(scratch), sc_bytes, stream_of(q)), "dsa_dense_bwd_rows");
+        } else if (words_k) {
+            const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
+            const Tensor scratch = empty_bytes(sc_bytes, q);
+            check(dsa_attn_bwd_words(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(cu), T, N, Hq, Hkv, D, words_k, (float)scale,
+                                     DSA_DTYPE_BF16, max_seqlen, ptr(dq), ptr(dk), ptr(dv), ptr(ws), (size_t)ws.numel(), ptr(scratch), sc_bytes,
+                                     stream_of(q)), "dsa_attn_bwd_words");
         } else if (ws.defined() || !idx.defined()) {                               // the forward's bitmap is read where it lies
             const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
             const Tensor scratch = empty_bytes(sc_bytes, q);
@@ -271,7 +290,7 @@ public:
         } else if (dtype != at::kBFloat16) {
             dq = dq.to(dtype); dk = dk.to(dtype); dv = dv.to(dtype);
         }
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -302,7 +321,8 @@ Picked checked_selection(const OptTensor &idx, const OptTensor &n, int64_t T, co
 }
 
 variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu_, int64_t max_seqlen, const OptTensor &idx_,
-                        const OptTensor &n_, double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
+                        const OptTensor &n_, double scale, bool causal, bool want_mass, const OptTensor &bitmap,
+                        int64_t words_k = 0) {
     no_forward_mode({&q, &k, &v}, "attention");
     need_gpu(q); need_gpu(k); need_gpu(v); need_gpu(cu_);
     const Qkv sh = checked_qkv(q, k, v);
@@ -311,16 +331,16 @@ variable_list attn_node(const Tensor &q, const Tensor &k, const Tensor &v, const
     const Tensor cu = checked_cu(cu_);
     const Picked sel = checked_selection(idx_, n_, sh.T, q);
     const OptTensor idx = sel.idx.defined() ? OptTensor(sel.idx) : std::nullopt, n = sel.n.defined() ? OptTensor(sel.n) : std::nullopt;
-    TORCH_CHECK_VALUE(idx || (!want_mass && !bitmap), "the attention mass and the bitmap belong to a selection");
+    TORCH_CHECK_VALUE(idx || words_k || (!want_mass && !bitmap), "the attention mass and the bitmap belong to a selection");
     TORCH_CHECK_VALUE(!bitmap || (bitmap->scalar_type() == at::kByte && bitmap->is_contiguous() && bitmap->device() == q.device()),
                       "the bitmap must be contiguous bytes on ", q.device());
     if (!needs_grad(q, k, v)) {
         at::AutoDispatchBelowADInplaceOrView below;
-        const AttnArgs a{max_seqlen, scale, causal, want_mass, q.scalar_type() == at::kFloat && 4 * q.size(2) <= 256, q.scalar_type()};
+        const AttnArgs a{max_seqlen, scale, causal, want_mass, carried_split(q.scalar_type(), q.size(2)), q.scalar_type(), words_k};
         AttnForward f = attn_forward(q, k, v, cu, idx.value_or(Tensor()), n.value_or(Tensor()), bitmap.value_or(Tensor()), a);
         return want_mass ? variable_list{f.res, f.mass} : variable_list{f.res};
     }
-    return AttnNode::apply(q, k, v, cu, idx, n, bitmap, max_seqlen, scale, causal, want_mass);
+    return AttnNode::apply(q, k, v, cu, idx, n, bitmap, max_seqlen, scale, causal, want_mass, words_k);
 }
 
 // q, k and v can go to the dense forward as they lie in memory: no transposing copy, no padding of the head_dim
@@ -373,8 +393,12 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
     const double scale = softmax_scale ? *softmax_scale : std::pow((double)sh.D, -0.5);
     const bool sparse = iq || ik || iw;
     TORCH_CHECK_VALUE(causal || !sparse, "DSA key selection is defined for causal attention only");
+    int64_t d_kernel = 0;
+    for (const int64_t d : {64, 96, 128, 256})           // head_dim 96 only without a key selection
+        if (d >= sh.D && !(sparse && d == 96)) { d_kernel = d; break; }
     Selection sel;
     Tensor bitmap;
+    int64_t words_k = 0;
     if (sparse) {
         TORCH_CHECK_VALUE(iq && ik && iw && top_k, "DSA needs indexer_q, indexer_k, indexer_w and top_k together");
         TORCH_CHECK_VALUE(iq->dim() >= 1 && iq->size(0) == sh.T, "indexer tensors must cover the same T packed tokens as q");
@@ -383,13 +407,16 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
         // the top-k kernel leaves the inverted selection here: forward and backward read it, nothing builds it again
         if (dsa_get_tile_crossover() > 0) bitmap = empty_bytes(dsa_attn_fwd_workspace_bytes((int)sh.T, (int)max_seqlen, 1), q_);
         TORCH_CHECK_VALUE(iq->dim() == 3, "indexer tensors must be q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi)");
-        sel = select_keys(*iq, *ik, *iw, cu, (int)max_seqlen, *top_k, index_scale_of(index_scale, iq->size(1), iq->size(2)), return_scores, bitmap);
+        // ... and writes no list where the caller asks for none and no row is one for the kernels that gather by it
+        if (bitmap.defined() && !return_indices && !return_mass && !return_scores &&
+            !dsa_attn_reads_list((int)sh.Hq, (int)sh.Hkv, (int)(carried_split(q_.scalar_type(), d_kernel) ? 4 * d_kernel : d_kernel), (int)*top_k,
+                                 (int)max_seqlen))
+            words_k = *top_k;
+        sel = select_keys(*iq, *ik, *iw, cu, (int)max_seqlen, *top_k, index_scale_of(index_scale, iq->size(1), iq->size(2)), return_scores, bitmap,
+                          !words_k);
     } else {
         TORCH_CHECK_VALUE(!return_indices && !return_scores, "return_indices / return_scores need the indexer inputs");
     }
-    int64_t d_kernel = 0;
-    for (const int64_t d : {64, 96, 128, 256})           // head_dim 96 only without a key selection
-        if (d >= sh.D && !(sparse && d == 96)) { d_kernel = d; break; }
     TORCH_CHECK_VALUE(d_kernel, "head_dim ", sh.D, " is beyond the kernels' largest (256)");
     TORCH_CHECK_VALUE(sparse || !return_mass, "return_mass needs the indexer inputs");
     Tensor q = q_, k = k_, v = v_;
@@ -404,7 +431,7 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
     }
     variable_list r = attn_node(q.contiguous(), k.contiguous(), v.contiguous(), cu, max_seqlen, sel.idx.defined() ? OptTensor(sel.idx) : std::nullopt,
                                 sel.n.defined() ? OptTensor(sel.n) : std::nullopt, scale, causal, return_mass,
-                                bitmap.defined() ? OptTensor(bitmap) : std::nullopt);
+                                bitmap.defined() ? OptTensor(bitmap) : std::nullopt, words_k);
     variable_list res{d_kernel != sh.D ? r[0].narrow(-1, 0, sh.D) : r[0]};
     if (return_indices) { res.push_back(sel.idx); res.push_back(sel.n); }
     if (return_mass) res.push_back(r[1]);
@@ -751,7 +778,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const auto nogil = py::call_guard<py::gil_scoped_release>();
     m.def("varlen_attn", &varlen_attn, nogil);
     m.def("hf_dense_forward", &hf_dense_forward, nogil);
-    m.def("attn_node", &attn_node, nogil);
+    m.def("attn_node", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu, int64_t max_seqlen, const OptTensor &idx, const OptTensor &n,
+                          double scale, bool causal, bool want_mass, const OptTensor &bitmap) {
+        return attn_node(q, k, v, cu, max_seqlen, idx, n, scale, causal, want_mass, bitmap);
+    }, nogil);
     m.def("indexer_kl_loss", &indexer_kl_loss, nogil);
     m.def("qk_norm_rope", &qk_norm_rope, nogil);
     m.def("sigmoid_gate", &sigmoid_gate, nogil);
