@@ -166,8 +166,9 @@ int dsa_attn_fwd_saved_bitmap(const void *q, const void *k, const void *v, const
 
 /*
  * The same without idx and n, for callers that never look at them: dsa_index_topk_words leaves the bitmap alone, and
- * dsa_attn_fwd_words / dsa_attn_bwd_words are dsa_attn_fwd_saved_bitmap / dsa_attn_bwd_saved_bitmap on such a bitmap
- * (K: the top_k it was made with).  dsa_attn_reads_list says (1) whether those two would hand rows of segments up to
+ * dsa_attn_fwd_words / dsa_attn_bwd_words are dsa_attn_fwd_saved_bitmap / dsa_attn_bwd_saved_bitmap on such a bitmap or one
+ * that dsa_index_topk_bitmap left (K: the top_k it was made with; rows at positions below it are taken to attend all of
+ * their window).  dsa_attn_reads_list says (1) whether those two would hand rows of segments up to
  * max_seqlen to kernels that gather by the list; the calls here keep every row on the kernels that read the bitmap, right
  * for any row and the same bits where the answer is 0, slower than the gather where it is 1.
  */

@@ -44,29 +44,36 @@ def test_words_alone_are_those_beside_the_list(segs, K, ties):
 @pytest.mark.parametrize("Hq,Hkv,D,segs,K,dtype", [
     (8, 2, 128, (1280, 290, 7), 16, torch.bfloat16),     # past 16 K the compacted walk, up to the last row before the gather begins
     (8, 2, 128, (1281, 290), 16, torch.bfloat16),        # and the first of the gather: the list is written after all
-    (4, 4, 64, (600, 41), 32, torch.bfloat16), (6, 2, 80, (500,), 40, torch.bfloat16), (4, 2, 256, (700,), 48, torch.bfloat16),
-    (8, 4, 48, (513, 200), 64, torch.float32), (4, 2, 128, (300,), 32, torch.float32)])
+    (8, 2, 128, (500, 190, 250), 200, torch.bfloat16),   # blocks of queries that keep their whole window, also one that ends with its segment
+    (4, 4, 64, (600, 41), 256, torch.bfloat16), (6, 2, 80, (500,), 127, torch.bfloat16), (4, 2, 256, (700, 64), 130, torch.bfloat16),
+    (4, 1, 256, (333,), 32, torch.bfloat16), (8, 4, 48, (513, 200), 64, torch.float32), (4, 2, 128, (300,), 129, torch.float32)])
 def test_attention_without_the_list(Hq, Hkv, D, segs, K, dtype):
-    """The operator asked for no list against the same call that returns it: outputs and gradients bit for bit, also where
-    the two crossover settings on either side move every row to the kernels of the list or of the bitmap."""
+    """The operator, with and without the list returned, against attention that was handed the list and builds its own bitmap: outputs
+    and gradients bit for bit, also at crossovers that move every row to the kernels of the list or of the bitmap in the operator."""
     print("attention from words", Hq, Hkv, D, segs, K, dtype, flush=True)
     g = torch.Generator().manual_seed(D + K)
     T, cu = sum(segs), torch.tensor([0] + list(segs)).cumsum(0).int().to(DEV)
     mk = lambda *s: torch.randn(*s, generator=g).mul_(0.5).to(dtype).to(DEV)
     q, k, v, do, qi, ki, wi = mk(T, Hq, D), mk(T, Hkv, D), mk(T, Hkv, D), mk(T, Hq, D), mk(T, 4, 64), mk(T, 64), mk(T, 4)
-    lib = _lib.load()
-    old = lib.dsa_get_tile_crossover()
+    lib, host = _lib.load(), _lib.host()
+    old, pad = lib.dsa_get_tile_crossover(), {48: 16, 80: 48}.get(D, 0)
     try:
         for crossover in (old, 0, 3):
             _lib.check(lib.dsa_set_tile_crossover(crossover), "dsa_set_tile_crossover")
-            res = []
-            for listed in (True, False):
+            res, picked = [], None
+            for listed in (True, False, None):
                 a, b, c = (x.clone().requires_grad_(True) for x in (q, k, v))
-                out = ops.dsa_varlen_attn(a, b, c, cu, max(segs), indexer_q=qi, indexer_k=ki, indexer_w=wi, top_k=K, return_indices=listed)
-                out = out[0] if listed else out
+                if listed is None:
+                    wide = [torch.nn.functional.pad(x, (0, pad)) for x in (a, b, c)]
+                    out = host.attn_node(*wide, cu, max(segs), *picked, D ** -0.5, True, False, None)[0][..., :D]
+                else:
+                    out = ops.dsa_varlen_attn(a, b, c, cu, max(segs), indexer_q=qi, indexer_k=ki, indexer_w=wi, top_k=K, return_indices=listed)
+                if listed:
+                    out, *picked = out
                 out.backward(do)
                 res.append((out.detach(), a.grad, b.grad, c.grad))
-            for x, y in zip(*res):
-                assert torch.equal(x, y)
+            for got in res[:2]:
+                for x, y in zip(got, res[2]):
+                    assert torch.equal(x, y)
     finally:
         lib.dsa_set_tile_crossover(old)

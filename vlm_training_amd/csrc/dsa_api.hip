@@ -46,10 +46,10 @@ hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, 
                                 float scale, float *partial, float *mass, hipStream_t stream);
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
-                               int causal, void *out, float *lse, hipStream_t stream);
+                               int window, int causal, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int causal, void *dq, const void *out_for_delta,
+                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta,
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
@@ -336,6 +336,7 @@ extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_id
     return align_up((size_t)T * bitmap_ldw(max_seqlen) * 4, 256);
 }
 
+// idx null with `selected`: ws holds a bitmap that a selection of K keys per row left, so that rows at positions below K attend all of their window
 // build_bitmap == 0: ws already holds the bitmap of idx/n (it is only read)
 static int attn_fwd_run(const void *q, const void *k, const void *v, bool selected, const int32_t *idx, const int32_t *n, const int32_t *cu,
                         int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, int causal,
@@ -363,7 +364,8 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, bool select
             }
         }
         const int64_t strides[6] = {(int64_t)Hq * D, D, (int64_t)Hkv * D, D, (int64_t)Hkv * D, D};
-        e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len, causal, out, lse, st);
+        e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
+                                idx ? 0 : K, causal, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "tile forward launch");
     }
     if (rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
@@ -673,8 +675,8 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     if (ov) rc = key_side();
     if (rc == DSA_OK && (parts & DSA_BWD_DQ)) {
         if (rows.tiles > 0) {
-            e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len, causal, dq,
-                                   fuse_delta ? out : nullptr, delta, sq);
+            e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
+                                   idx ? 0 : K, causal, dq, fuse_delta ? out : nullptr, delta, sq);
             if (e != hipSuccess) rc = hip_fail(e, "tile dq launch");
         }
         if (rc == DSA_OK && rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
@@ -819,7 +821,7 @@ extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_hea
             return fail(DSA_ERR_ARG, "strides must be multiples of 8, token strides below 2^24");
     if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) return fail(DSA_ERR_ARG, "tensors must lie on 16-byte boundaries");
     if (T == 0) return DSA_OK;
-    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, causal, out, lse,
+    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, 0, causal, out, lse,
                                              (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "tile forward launch");
 }

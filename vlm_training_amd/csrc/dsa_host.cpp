@@ -134,7 +134,7 @@ struct AttnArgs {
     double scale;
     bool causal, want_mass, split;
     at::ScalarType dtype;
-    int64_t words_k;                                     // keys per row of a selection that is there as its bitmap alone, else 0
+    int64_t words_k;                                     // keys per row of a selection whose bitmap is all that attention reads, else 0
 };
 bool carried_split(at::ScalarType dtype, int64_t D) { return dtype == at::kFloat && 4 * D <= 256; }
 
@@ -223,7 +223,7 @@ public:
         const Tensor idx = idx_.value_or(Tensor()), n = n_.value_or(Tensor());
         const AttnArgs a{max_seqlen, scale, causal, want_mass, carried_split(q.scalar_type(), q.size(2)), q.scalar_type(), words_k};
         const AttnForward f = attn_forward(q, k, v, cu, idx, n, bitmap_.value_or(Tensor()), a);
-        ctx->save_for_backward({f.qb, f.kb, f.vb, f.out, f.lse, cu, idx, n, f.ws});
+        ctx->save_for_backward({f.qb, f.kb, f.vb, f.out, f.lse, cu, words_k ? Tensor() : idx, words_k ? Tensor() : n, f.ws});
         ctx->saved_data["m"] = max_seqlen;
         ctx->saved_data["s"] = scale;
         ctx->saved_data["c"] = causal;
@@ -407,13 +407,13 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
         // the top-k kernel leaves the inverted selection here: forward and backward read it, nothing builds it again
         if (dsa_get_tile_crossover() > 0) bitmap = empty_bytes(dsa_attn_fwd_workspace_bytes((int)sh.T, (int)max_seqlen, 1), q_);
         TORCH_CHECK_VALUE(iq->dim() == 3, "indexer tensors must be q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi)");
-        // ... and writes no list where the caller asks for none and no row is one for the kernels that gather by it
-        if (bitmap.defined() && !return_indices && !return_mass && !return_scores &&
+        // ... alone, unless some row is one for the kernels that gather by the list; nothing writes a list then that the caller did not ask for
+        if (bitmap.defined() &&
             !dsa_attn_reads_list((int)sh.Hq, (int)sh.Hkv, (int)(carried_split(q_.scalar_type(), d_kernel) ? 4 * d_kernel : d_kernel), (int)*top_k,
                                  (int)max_seqlen))
             words_k = *top_k;
         sel = select_keys(*iq, *ik, *iw, cu, (int)max_seqlen, *top_k, index_scale_of(index_scale, iq->size(1), iq->size(2)), return_scores, bitmap,
-                          !words_k);
+                          !words_k || return_indices || return_mass || return_scores);
     } else {
         TORCH_CHECK_VALUE(!return_indices && !return_scores, "return_indices / return_scores need the indexer inputs");
     }

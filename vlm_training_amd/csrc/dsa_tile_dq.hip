@@ -8,7 +8,7 @@
 // with dP(t+1), the logits and exponentials P(t+1) behind them, then S(t+2), the products and packing of dS(t+1) behind it; operand reads
 // run four ahead through all of it, in pairs where two groups share them.  K and V tiles go from memory straight into LDS, rings of five
 // and three: step t requests K(t+4), V(t+3) and the selection words of tile t+3, at its end waits for what step t-1 requested and meets
-// the one barrier.  Tiles that every row attends whole run without mask arithmetic.
+// the one barrier.  Tiles that every row attends whole run without mask arithmetic (with a selection: in blocks inside the first K positions).
 //
 // What bounds it: the issue of one instruction stream per SIMD - at head_dim 128 48 MFMAs (1536 clocks) beside about 125 vector
 // instructions (195 with a mask), 33 LDS reads and 70 scalar ones - and the chip's power.  Same box, us, against the kernels before
@@ -27,7 +27,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift,
-    float scale, int pos_split, int split_len, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
+    float scale, int pos_split, int split_len, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
     typedef DirectTile<D> TL;
     constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;
@@ -326,8 +326,8 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const std::false_type no;
     step(yes, no, yes, -1);
     int t = 0;
-    if (!HAS_IDX) {                                      // tiles that every row of the block attends whole: no mask arithmetic
-        const int whole = (causal ? qc0 + 1 : L) / 32;
+    {                                                    // tiles that every row of the block attends whole: no mask arithmetic
+        const int whole = (HAS_IDX && min(qc0 + QBW, L) > window ? 0 : causal ? qc0 + 1 : L) / 32;
         for (; t + 1 < whole; ++t) step(no, yes, yes, t);     // (rows that do not exist may turn to NaN: a row is one lane's)
     }
     for (; t + 1 < ntiles; ++t) step(yes, yes, yes, t);
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
 template <int D, bool HAS_IDX, int RG>
 static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int gs,
-                              int d_real, float scale, int pos_split, int split_len, int causal, void *dq, const void *out_for_delta, float *delta_out) {
+                              int d_real, float scale, int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta, float *delta_out) {
     constexpr int NW = 4;
     constexpr size_t lds = dq_lds_bytes<D, NW>(HAS_IDX);
     const auto kernel = &dsa_tile_dq_kernel<D, HAS_IDX, NW, RG>;
@@ -376,7 +376,7 @@ static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW * RG) >> gs) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)dout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta,
-                       bitmap, ldw, cu, N, T, Hq, Hkv, gs, scale, pos_split, split_len, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
+                       bitmap, ldw, cu, N, T, Hq, Hkv, gs, scale, pos_split, split_len, window, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
     return hipGetLastError();
 }
 // 32 rows per wave instead of 64: each walk is then twice as fast, two workgroups share a CU, and blocks are half as long, which wastes fewer
@@ -395,16 +395,17 @@ static bool dq_one_row_group(int causal, int T, int N, int Hkv, int gs) {
     if (wg > 1024) return false;
     return T / N < 1500 || (rows / 128 * Hkv + 255) / 256 < 2 * (((2 * (rows / 256) + N) * Hkv + 511) / 512);
 }
-// d_real: elements of a row, without a selection any multiple of 8 (dense_kernel_dim).  out_for_delta != null: the kernel forms
+// d_real: elements of a row, without a selection any multiple of 8 (dense_kernel_dim).  window: rows of a bitmap at positions below it attend
+// all of their causal window (0: nothing is known).  out_for_delta != null: the kernel forms
 // delta = rowsum(dO * O) of its rows itself and writes it to delta_out
 extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,
                                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                         int pos_split, int split_len, int causal, void *dq, const void *out_for_delta, float *delta_out,
+                                         int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta, float *delta_out,
                                          hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
     const bool one_group = dq_one_row_group(causal, T, N, Hkv, gs);
-#define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, causal, dq, out_for_delta, delta_out
+#define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, dq, out_for_delta, delta_out
 #define DQ_CASE(D_, HI) return one_group ? launch_dq_i<D_, HI, 1>(DQ_ARGS) : launch_dq_i<D_, HI, 2>(DQ_ARGS)
     if (bitmap) switch (d_real) {
         case 64: DQ_CASE(64, true);

@@ -16,8 +16,10 @@
 // read as zero.  The selection words take the same way, each wave its own rows' into its own slots.
 //
 // What bounds it: the power of the chip (MFMA busy 0.61 of a CU's time without a selection, at 1.79 GHz) and, with a selection, the
-// vector instructions (about 92 and 16 exponentials beside 16 MFMAs at head_dim 128, 32 of them the mask); without one the softmax of
-// tiles every row attends whole drops the mask.  Both make every instruction beside the MFMAs count: a tile's buffer size comes from two
+// vector instructions (about 92 and 16 exponentials beside 16 MFMAs at head_dim 128, 32 of them the mask); the softmax of tiles every row
+// attends whole drops the mask: all but the last without a selection, those of blocks inside the first K positions with one (`window`; the
+// same in dQ.  Step of 8192 tokens, K = 1024: 300.2 -> 295.4 us, forward of 16 384 in mixed segments, K = 2048: 673 -> 661; not at head_dim 256,
+// where the second loop's spilled registers took 3 % of a step instead).  Both make every instruction beside the MFMAs count: a tile's buffer size comes from two
 // constants, its pieces follow one another under one buffer, operand addresses move on in place.  Same box, us, against a size formed per
 // piece, addresses formed per tile and eight waves per workgroup in large launches: 32 768 tokens dense 1289 -> 1229, with a selection
 // 1408 -> 1371; 8192 tokens with a selection 62.5 -> 59; 512 tokens 15.9 -> 15.1; head_dim 256, 16 384 tokens 210 -> 195; vision towers at
@@ -36,7 +38,7 @@ template <int D, bool HAS_IDX, int NW, bool NEG>
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
-    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int causal,
+    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int window, int causal,
     bf16_t *__restrict__ out, float *__restrict__ lse) {
     typedef DirectTile<D> TL;
     constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;   // MFMAs of S, of P V (head_dim 80: five and six)
@@ -300,10 +302,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         meet();
     };
     int tt = 0;
-    if (!HAS_IDX) {
+    if constexpr (!HAS_IDX || D <= 128) {
         // tiles every row of the block attends whole: the softmax without mask arithmetic (a loop of its own, not a branch
-        // in the loop: two bodies that meet again would keep two sets of accumulators)
-        const int whole = (causal ? qc0 : L) / 32;
+        // in the loop: two bodies that meet again would keep two sets of accumulators); at head_dim 256 a selection leaves it no registers
+        const int whole = (HAS_IDX && min(qc0 + QBW, L) > window ? 0 : causal ? qc0 : L) / 32;
         for (; tt + 3 < ntiles && tt + 2 < whole; tt += 2) {
             full_step(no, tt, pE, sO, pO, sE);
             full_step(no, tt + 1, pO, sE, pE, sO);
@@ -355,7 +357,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 
 template <int D, bool HAS_IDX>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int causal,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int window, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
     const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false>;
@@ -364,19 +366,19 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
-                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, causal, (bf16_t *)out, lse);
+                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, window, causal, (bf16_t *)out, lse);
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
-// without a bitmap only); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
+// without a bitmap only); window: rows of a bitmap at positions below it attend all of their causal window (0: nothing is known); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
 extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                          int pos_split, int split_len, int causal, void *out, float *lse, hipStream_t stream) {
+                                          int pos_split, int split_len, int window, int causal, void *out, float *lse, hipStream_t stream) {
     int gs = 0;
     while ((1 << gs) < Hq / Hkv) ++gs;
     scale = logit_scale(scale);
     hipError_t e = hipErrorInvalidValue;
-#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, causal, out, lse)
+#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, out, lse)
     if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
         else if (d_real <= 128) FWD_CASE(128, true);
