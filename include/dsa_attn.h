@@ -43,6 +43,8 @@ typedef enum {
 
 #define DSA_DTYPE_BF16 0
 #define DSA_DTYPE_FP32 1 /* accepted by the Python host only (it rounds to bf16 first) */
+#define DSA_DTYPE_SPLIT_BF16 2 /* attention forward and backward, D = 256: bf16 rows as dsa_split_bf16_stack lays fp32 rows of 64 out.  Only the
+                                * parts that dsa_split_bf16_combine reads of dq, dk and dv are written */
 
 /* Library identification, e.g. "dsa-attn-gfx950 0.1".  (no reference counterpart) */
 const char *dsa_version(void);

@@ -15,6 +15,7 @@ HOST_PATH = os.path.join(_HERE, "_dsa_host.so")
 
 DSA_DTYPE_BF16 = 0
 DSA_DTYPE_FP32 = 1
+DSA_DTYPE_SPLIT_BF16 = 2
 DSA_NORM_OFFSET, DSA_NORM_WEIGHT_BF16 = 1, 2                                               # norm_flags of the prologue
 DSA_BWD_DELTA, DSA_BWD_BITMAP, DSA_BWD_DQ, DSA_BWD_DKV, DSA_BWD_ALL = 1, 2, 4, 8, 15      # parts of dsa_attn_bwd_parts
 

@@ -46,14 +46,14 @@ hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, 
                                 float scale, float *partial, float *mass, hipStream_t stream);
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
-                               int window, int causal, void *out, float *lse, hipStream_t stream);
+                               int window, int carried, int causal, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta,
+                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int window, int carried, int causal, void *dq, const void *out_for_delta,
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                               int Hq, int Hkv, int D, float scale, int causal, int skip_len, int32_t *order, int listed, float *partial,
+                               int Hq, int Hkv, int D, float scale, int carried, int causal, int skip_len, int32_t *order, int listed, float *partial,
                                size_t partial_bytes, void *dk, void *dv, hipStream_t stream);
 hipError_t dsa_launch_tile_order_delta(const void *dout, const void *out, const int32_t *cu, int N, int T, int Hq, int Hkv, int D,
                                        int has_idx, int causal, int32_t *order, const float *partial, size_t partial_bytes,
@@ -262,7 +262,8 @@ extern "C" int dsa_indexer_kl(const float *sel_scores, const float *mass, const 
 static int check_attn(int T, int N, const int32_t *cu, int Hq, int Hkv, int D, int K, int dtype, bool selected, const int32_t *idx,
                       const int32_t *n) {
     if (int rc = check_packed(T, N, cu)) return rc;
-    if (dtype != DSA_DTYPE_BF16) return fail(DSA_ERR_UNSUPPORTED, "q/k/v must be bf16 (dtype code %d)", dtype);
+    if (dtype != DSA_DTYPE_BF16 && !(dtype == DSA_DTYPE_SPLIT_BF16 && D == 256))
+        return fail(DSA_ERR_UNSUPPORTED, "q/k/v must be bf16 (dtype code %d)", dtype);
     if (Hq < 1 || Hkv < 1 || Hq % Hkv) return fail(DSA_ERR_ARG, "Hq=%d must be a positive multiple of Hkv=%d", Hq, Hkv);
     if (Hq / Hkv > 16) return fail(DSA_ERR_UNSUPPORTED, "Hq/Hkv=%d: at most 16 query heads per kv head", Hq / Hkv);
     if (!(D == 64 || D == 128 || D == 256 || (D == 96 && !selected)))
@@ -365,7 +366,7 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, bool select
         }
         const int64_t strides[6] = {(int64_t)Hq * D, D, (int64_t)Hkv * D, D, (int64_t)Hkv * D, D};
         e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
-                                idx ? 0 : K, causal, out, lse, st);
+                                idx ? 0 : K, dtype == DSA_DTYPE_SPLIT_BF16, causal, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "tile forward launch");
     }
     if (rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
@@ -439,6 +440,7 @@ extern "C" size_t dsa_attn_mass_workspace_bytes(int T, int N, int Hq, int Hkv, i
 static int attn_mass_run(const void *q, const void *k, const float *lse, const int32_t *idx, const int32_t *n, const int32_t *cu,
                          int T, int N, int Hq, int Hkv, int D, int K, float softmax_scale, int dtype, int max_seqlen, float *mass,
                          const void *saved_bitmap, size_t saved_bytes, void *ws, size_t ws_bytes, void *stream) {
+    if (dtype == DSA_DTYPE_SPLIT_BF16) return fail(DSA_ERR_UNSUPPORTED, "q/k/v must be bf16 (dtype code %d)", dtype);
     if (int rc = check_attn(T, N, cu, Hq, Hkv, D, K, dtype, idx != nullptr, idx, n)) return rc;
     if (!q || !k || !lse || !idx || !n || !mass) return fail(DSA_ERR_ARG, "null tensor pointer");
     if (int rc = check_aligned(k, k, "k")) return rc;
@@ -619,7 +621,8 @@ extern "C" size_t dsa_attn_bwd_bitmap_offset(int T, int Hq) {
 static int attn_bwd_run(const void *dout, const void *q, const void *k, const void *v, const void *out, const float *lse,
                         bool selected, const int32_t *idx, const int32_t *n, const int32_t *cu, int T, int N, int Hq, int Hkv, int D, int K,
                         float softmax_scale, int max_seqlen, int causal, void *dq, void *dk, void *dv, float *delta,
-                        uint32_t *bitmap, float *partial, size_t partial_bytes, int32_t *order, int parts, hipStream_t st) {
+                        uint32_t *bitmap, float *partial, size_t partial_bytes, int32_t *order, int parts, hipStream_t st,
+                        bool carried = false) {
     const int ldw = bitmap_ldw(max_seqlen);
     if (selected && (size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
     const RowSplit rows = row_split_for(selected, idx, Hq, Hkv, D, K);
@@ -665,7 +668,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     int rc = DSA_OK;
     const int walk_len = key_walk_len(selected, q, dout, T, N, Hq, Hkv, D, K);
     auto key_side = [&]() {
-        hipError_t e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, causal, walk_len, order, listed,
+        hipError_t e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, carried, causal, walk_len, order, listed,
                                            partial, partial_bytes, dk, dv, st);
         if (e == hipSuccess && max_seqlen >= walk_len)
             e = dsa_launch_selkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, softmax_scale, walk_len, dk, dv, st);
@@ -676,7 +679,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     if (rc == DSA_OK && (parts & DSA_BWD_DQ)) {
         if (rows.tiles > 0) {
             e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
-                                   idx ? 0 : K, causal, dq, fuse_delta ? out : nullptr, delta, sq);
+                                   idx ? 0 : K, carried, causal, dq, fuse_delta ? out : nullptr, delta, sq);
             if (e != hipSuccess) rc = hip_fail(e, "tile dq launch");
         }
         if (rc == DSA_OK && rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
@@ -723,7 +726,7 @@ extern "C" int dsa_attn_bwd_parts(const void *dout, const void *q, const void *k
     const size_t partial_bytes = dsa_tile_dkv_partial_bytes(T);
     float *partial = partial_bytes ? (float *)((char *)order - align_up(partial_bytes, 256)) : nullptr;
     return attn_bwd_run(dout, q, k, v, out, lse, idx != nullptr, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
-                        delta, bitmap, partial, partial_bytes, order, parts, (hipStream_t)stream);
+                        delta, bitmap, partial, partial_bytes, order, parts, (hipStream_t)stream, dtype == DSA_DTYPE_SPLIT_BF16);
 }
 
 // Scratch of the backward that nothing outlives: delta, the launch order of the key tiles and - only for launches small
@@ -758,7 +761,8 @@ static int attn_bwd_saved(const void *dout, const void *q, const void *k, const 
     // the kernels only read the bitmap; the forward's workspace is not written here
     uint32_t *bitmap = selected ? const_cast<uint32_t *>((const uint32_t *)fwd_ws) : nullptr;
     return attn_bwd_run(dout, q, k, v, out, lse, selected, idx, n, cu, T, N, Hq, Hkv, D, K, softmax_scale, max_seqlen, causal, dq, dk, dv,
-                        delta, bitmap, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream);
+                        delta, bitmap, partial, partial_bytes, order, DSA_BWD_ALL & ~DSA_BWD_BITMAP, (hipStream_t)stream,
+                        dtype == DSA_DTYPE_SPLIT_BF16);
 }
 
 extern "C" int dsa_attn_bwd_saved_bitmap(const void *dout, const void *q, const void *k, const void *v, const void *out,
@@ -821,7 +825,7 @@ extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_hea
             return fail(DSA_ERR_ARG, "strides must be multiples of 8, token strides below 2^24");
     if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) return fail(DSA_ERR_ARG, "tensors must lie on 16-byte boundaries");
     if (T == 0) return DSA_OK;
-    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, 0, causal, out, lse,
+    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, 0, 0, causal, out, lse,
                                              (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "tile forward launch");
 }

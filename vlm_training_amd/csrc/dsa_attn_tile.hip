@@ -521,7 +521,7 @@ extern "C" size_t dsa_tile_order_bytes(int T) { return ((size_t)order_entries_ca
 // rows of D elements (`pitch` in the partial sums).  Grid: (cut tiles at most, kv heads, pitch / 8 slices of 256 units).
 __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_t *__restrict__ order, int cap,
                                                                     const float *__restrict__ partial, const int32_t *__restrict__ cu,
-                                                                    int N, int Hkv, int D, int pitch, int qb, int seq_clamp, float scale,
+                                                                    int N, int Hkv, int D, int pitch, int qb, int seq_clamp, float scale, int carried,
                                                                     bf16_t *__restrict__ dk, bf16_t *__restrict__ dv) {
     if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(order[2])) return;
     const int entry = __builtin_amdgcn_readfirstlane(order[4 + 4 * cap + blockIdx.x]);
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256) void dsa_dkv_pieces_reduce_kernel(const int32_
     // a thread's unit: eight columns of a row, in the two halves of a wave's store
     const int DT = pitch / 32, unit = blockIdx.z * 256 + threadIdx.x, j = unit & 31, part = unit >> 5;     // part: [dK | dV][key group][d-tile][8 columns]
     const int m = part / (16 * DT), grp = part / (4 * DT) % 4, col = part % (4 * DT) * 8, key = grp * 32 + j;
-    if (m > 1 || key >= min(128, L - c0) || col >= D) return;
+    if (m > 1 || key >= min(128, L - c0) || col >= D || (carried && !carried_chunk(col / 8, m))) return;
     const int64_t slot_f = 2 * 128 * (int64_t)pitch;         // floats per (slot, kv head)
     const float *src = partial + ((int64_t)mslot * Hkv + kvh) * slot_f + part * 256 + j * 4;
     f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
@@ -685,12 +685,12 @@ extern "C" hipError_t dsa_launch_tile_order_delta(const void *dout, const void *
 }
 extern "C" hipError_t dsa_launch_dkv_tiles(unsigned grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
                                            const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
-                                           int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len, const int32_t *order, float *partial,
-                                           void *dk, void *dv);
+                                           int T, int Hq, int Hkv, int d_real, float scale, int carried, int causal, int skip_len, const int32_t *order,
+                                           float *partial, void *dk, void *dv);
 // listed: dsa_launch_tile_order_delta has left the list in `order`
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
-                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len,
+                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int carried, int causal, int skip_len,
                                           int32_t *order, int listed, float *partial, size_t partial_bytes, void *dk, void *dv,
                                           hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
@@ -699,11 +699,12 @@ extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const
     if (!p.listed) order = nullptr;
     else if (!listed) hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, p.o, order);
     if (!p.pieces) partial = nullptr;
-    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, skip_len, order, partial, dk, dv);
+    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, carried,
+                                              causal, skip_len, order, partial, dk, dv);
     if (e != hipSuccess) return e;
     if (p.pieces)
         hipLaunchKernelGGL(dsa_dkv_pieces_reduce_kernel, dim3(p.tiles_ub, Hkv, p.pitch / 8), dim3(256), 0, stream, order,
-                           p.o.cap, partial, cu, N, Hkv, d_real, p.pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale,
+                           p.o.cap, partial, cu, N, Hkv, d_real, p.pitch, 32 >> gs, bitmap ? ldw * 32 : 0x7fffffff, scale, carried,
                            (bf16_t *)dk, (bf16_t *)dv);
     return hipGetLastError();
 }

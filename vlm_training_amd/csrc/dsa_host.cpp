@@ -137,6 +137,7 @@ struct AttnArgs {
     int64_t words_k;                                     // keys per row of a selection whose bitmap is all that attention reads, else 0
 };
 bool carried_split(at::ScalarType dtype, int64_t D) { return dtype == at::kFloat && 4 * D <= 256; }
+int rows_code(bool split, int D) { return split && D == 256 ? DSA_DTYPE_SPLIT_BF16 : DSA_DTYPE_BF16; }
 
 void attn_forward_kernels(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &idx, const Tensor &n, const Tensor &cu, const AttnArgs &a,
                           const Tensor &ws, bool bitmap_ready, const Tensor &out, const Tensor &lse) {
@@ -147,13 +148,13 @@ void attn_forward_kernels(const Tensor &q, const Tensor &k, const Tensor &v, con
         check(dsa_dense_fwd_strided(ptr(q), q.stride(0), D, ptr(k), k.stride(0), D, ptr(v), v.stride(0), D, iptr(cu), T, N, Hq, Hkv, D, (float)a.scale,
                                     DSA_DTYPE_BF16, (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), stream_of(q)), "dsa_dense_fwd_strided");
     else if (a.words_k)
-        check(dsa_attn_fwd_words(ptr(q), ptr(k), ptr(v), iptr(cu), T, N, Hq, Hkv, D, (int)a.words_k, (float)a.scale, DSA_DTYPE_BF16, (int)a.max_seqlen,
+        check(dsa_attn_fwd_words(ptr(q), ptr(k), ptr(v), iptr(cu), T, N, Hq, Hkv, D, (int)a.words_k, (float)a.scale, rows_code(a.split, D), (int)a.max_seqlen,
                                  ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd_words");
     else if (bitmap_ready)
-        check(dsa_attn_fwd_saved_bitmap(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, DSA_DTYPE_BF16,
+        check(dsa_attn_fwd_saved_bitmap(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, rows_code(a.split, D),
                                         (int)a.max_seqlen, a.causal, ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd_saved_bitmap");
     else
-        check(dsa_attn_fwd(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, DSA_DTYPE_BF16, (int)a.max_seqlen,
+        check(dsa_attn_fwd(ptr(q), ptr(k), ptr(v), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)a.scale, rows_code(a.split, D), (int)a.max_seqlen,
                            a.causal, ptr(out), fptr(lse), ptr(ws), ws_bytes, stream_of(q)), "dsa_attn_fwd");
 }
 
@@ -268,19 +269,19 @@ public:
             const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
             const Tensor scratch = empty_bytes(sc_bytes, q);
             check(dsa_attn_bwd_words(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(cu), T, N, Hq, Hkv, D, words_k, (float)scale,
-                                     DSA_DTYPE_BF16, max_seqlen, ptr(dq), ptr(dk), ptr(dv), ptr(ws), (size_t)ws.numel(), ptr(scratch), sc_bytes,
+                                     rows_code(split, D), max_seqlen, ptr(dq), ptr(dk), ptr(dv), ptr(ws), (size_t)ws.numel(), ptr(scratch), sc_bytes,
                                      stream_of(q)), "dsa_attn_bwd_words");
         } else if (ws.defined() || !idx.defined()) {                               // the forward's bitmap is read where it lies
             const size_t sc_bytes = dsa_attn_bwd_scratch_bytes(T, N, Hq, Hkv, D);
             const Tensor scratch = empty_bytes(sc_bytes, q);
             check(dsa_attn_bwd_saved_bitmap(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K,
-                                            (float)scale, DSA_DTYPE_BF16, max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(ws),
+                                            (float)scale, rows_code(split, D), max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(ws),
                                             ws.defined() ? (size_t)ws.numel() : 0, ptr(scratch), sc_bytes, stream_of(q)), "dsa_attn_bwd_saved_bitmap");
         } else {
             const size_t ws_bytes = dsa_attn_bwd_workspace_bytes(T, Hq, max_seqlen, 1);
             const Tensor w = empty_bytes(ws_bytes, q);
             check(dsa_attn_bwd(ptr(db), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), iptr(idx), iptr(n), iptr(cu), T, N, Hq, Hkv, D, K, (float)scale,
-                               DSA_DTYPE_BF16, max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(w), ws_bytes, stream_of(q)), "dsa_attn_bwd");
+                               rows_code(split, D), max_seqlen, causal, ptr(dq), ptr(dk), ptr(dv), ptr(w), ws_bytes, stream_of(q)), "dsa_attn_bwd");
         }
         if (split) {
             const Tensor oq = empty({T, Hq, D / 4}, at::kFloat, q), ok = empty({T, Hkv, D / 4}, at::kFloat, q), ov = empty({T, Hkv, D / 4}, at::kFloat, q);

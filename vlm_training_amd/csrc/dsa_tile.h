@@ -209,6 +209,13 @@ __device__ __forceinline__ void buffer_load_lds16_n(buffer_rsrc rsrc, const int 
                      "\n\ts_add_u32 m0, m0, %7\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\ts_add_u32 m0, m0, %8\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds"
                      : : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds), "n"(N0), "n"(N1), "n"(N2) : "memory", "m0", "scc");
 }
+// fp32 tensors of head_dim 64 come as rows of 256, four parts of 64 (dsa_split_bf16_stack): the last part is zeros, and of a result two
+// parts are read.  `CARRIED` kernels of head_dim 256 run 12 of the 16 k-steps and the four 32-wide d-tiles that are read: parts 0 and 1
+// (out, dK) or 0 and 2 (dQ, dV), the same bits.  2048 tokens in four segments, 8 heads over 2, us, all of a row -> those: forward 34 -> 28.7,
+// dQ 41 -> 31, dK/dV 42 -> 29.5 (of it 5 to 10 a fixed start and end).
+#define DSA_CARRIED_KS 12
+__host__ __device__ constexpr int carried_tile(int dt) { return dt < 2 ? dt : dt + 2; }      // d-tile of parts 0 | 2
+__device__ __forceinline__ bool carried_chunk(int c, bool second) { return second ? !(c & 8) && c < 24 : c < 16; }   // 16-byte chunk c of parts 0 | 2 (second), 0 | 1
 // Order of a phase's NR row-wise and NT transposed operands: `PRE` transposed ones, then both kinds evenly mixed.
 template <int NR, int NT, int PRE>
 struct PhaseOrder {

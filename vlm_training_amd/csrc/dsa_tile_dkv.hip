@@ -33,7 +33,7 @@ template <int D, int KG> constexpr int dkv_aux_bytes() { return dkv_ring<D, KG>(
 template <int D, int KG> constexpr size_t dkv_lds_bytes() {
     return dkv_ring<D, KG>() * 2 * (size_t)DirectTile<D>::BYTES + 4 / KG * (size_t)dkv_aux_bytes<D, KG>();
 }
-template <int D, int KG, bool HAS_IDX, int GSHIFT, bool UNALIGNED>
+template <int D, int KG, bool HAS_IDX, int GSHIFT, bool UNALIGNED, bool CARRIED>
 __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
@@ -41,7 +41,9 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     float scale, float logit_scale, int causal, int d_real, int skip_len, const int32_t *__restrict__ order, float *__restrict__ partial, bf16_t *__restrict__ dk,
     bf16_t *__restrict__ dv) {
     typedef DirectTile<D> TL;
-    constexpr int RING = dkv_ring<D, KG>(), NW = 4 / KG, KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;
+    constexpr int RING = dkv_ring<D, KG>(), NW = 4 / KG;
+    constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT;
+    auto tile_of = [](int dt, bool of_v) __attribute__((always_inline)) { return CARRIED && of_v ? carried_tile(dt) : dt; };
     constexpr int LPW = TL::LOADS / NW, LPS = 2 * LPW + (HAS_IDX ? 2 : 1);
     constexpr int Gp = 1 << GSHIFT, QB = 32 >> GSHIFT;
     constexpr int RPW = Gp < 4 ? Gp : 4;                 // neighbouring rows of a lane that are one query's
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = Hq / Hkv;
-    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
+    const int dr = HAS_IDX || CARRIED ? D : d_real, chunks = CARRIED ? 2 * KS : dr / 8;   // elements and 16-byte chunks of a row in memory
     const int kvh = blockIdx.x % Hkv;
     int s0, L, blk, piece, mslot, pb;
     if (!locate_key_tile(order, cu, N, blockIdx.x / Hkv, s0, L, blk, piece, mslot, pb)) return;
@@ -231,7 +233,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
         return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(aR[TL::row_q(ks)] + TL::row_imm(ks) + off);
     };
     auto tr_op = [&](int i, int off) __attribute__((always_inline)) {
-        const int pair = i / DT, dt = i % DT;
+        const int pair = i / DT, dt = tile_of(i % DT, off != 0);   // (off: the operand is of dO)
         return tr_pair(aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair) + off, aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair + 1) + off);
     };
     const int jb = 31 - j, key_bias = (causal ? 0 : 0x40000000) - kc - 31;      // key_bias + jb = bias - the lane's first key
@@ -453,15 +455,16 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     step(yes, yes, no, s);
     wait_vmcnt<0>();                                     // no load is left on its way into LDS
     if (npieces > 1) {                                   // a piece of the walk: fp32 partial sums, added by the reduction
-        float *const p = piece_partial(partial, mslot, piece, Hkv, kvh, DT);
+        constexpr int TD = (D + 31) / 32;
+        float *const p = piece_partial(partial, mslot, piece, Hkv, kvh, TD);
 #pragma unroll
         for (int g = 0; g < KG; ++g)
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 settle(dkacc[g][dt]);
                 settle(dvacc[g][dt]);
-                store_c_tile_f32(p + ((wv * KG + g) * DT + dt) * 1024, dkacc[g][dt], lane);
-                store_c_tile_f32(p + ((4 + wv * KG + g) * DT + dt) * 1024, dvacc[g][dt], lane);
+                store_c_tile_f32(p + ((wv * KG + g) * TD + dt) * 1024, dkacc[g][dt], lane);
+                store_c_tile_f32(p + ((4 + wv * KG + g) * TD + tile_of(dt, true)) * 1024, dvacc[g][dt], lane);
             }
         return;
     }
@@ -487,7 +490,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
                     const uint32_t b0 = pack2bf(acc[8 * i + 4] * mul, acc[8 * i + 5] * mul), b1 = pack2bf(acc[8 * i + 6] * mul, acc[8 * i + 7] * mul);
                     const auto r0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
                     const auto r1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-                    *reinterpret_cast<u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(j, 4 * dt + 2 * i + h)) = u32x4{r0[0], r1[0], r0[1], r1[1]};
+                    *reinterpret_cast<u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(j, 4 * tile_of(dt, m) + 2 * i + h)) = u32x4{r0[0], r1[0], r0[1], r1[1]};
                 }
             }
 #pragma unroll
@@ -497,7 +500,7 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
 #pragma unroll
             for (int i = 0; i < TL::LOADS; ++i) {
                 const int row = i * TL::LOAD_ROWS + lane / TL::CPR, c = lane % TL::CPR, key = kc + 32 * g + row;
-                if (key < L && c < chunks)
+                if (key < L && (CARRIED ? carried_chunk(c, m) : c < chunks))
                     *reinterpret_cast<u32x4 *>((m ? dv : dk) + ((int64_t)(s0 + key) * Hkv + kvh) * dr + c * 8) =
                         *reinterpret_cast<const u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(row, c));
             }
@@ -517,10 +520,10 @@ struct DkvArgs {
     float *partial;
     void *dk, *dv;
 };
-template <int D, int KG, bool HAS_IDX, int GS>
+template <int D, int KG, bool HAS_IDX, bool CARRIED, int GS>
 static hipError_t launch_dkv(unsigned grid, hipStream_t stream, const DkvArgs &a) {
     constexpr size_t lds = dkv_lds_bytes<D, KG>();
-    const auto kernel = &dsa_tile_dkv_kernel<D, KG, HAS_IDX, GS, DKV_UNALIGNED>;
+    const auto kernel = &dsa_tile_dkv_kernel<D, KG, HAS_IDX, GS, DKV_UNALIGNED, CARRIED>;
     // (LDS above 64 KiB is asked for on every launch: neither a second device nor a second thread can meet a kernel never configured)
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -529,14 +532,14 @@ static hipError_t launch_dkv(unsigned grid, hipStream_t stream, const DkvArgs &a
                        a.partial, (bf16_t *)a.dk, (bf16_t *)a.dv);
     return hipGetLastError();
 }
-template <int D, int KG, bool HAS_IDX>
+template <int D, int KG, bool HAS_IDX, bool CARRIED = false>
 static hipError_t launch_dkv_gs(unsigned grid, hipStream_t stream, const DkvArgs &a) {
     switch (group_shift(a.Hq, a.Hkv)) {
-        case 0: return launch_dkv<D, KG, HAS_IDX, 0>(grid, stream, a);
-        case 1: return launch_dkv<D, KG, HAS_IDX, 1>(grid, stream, a);
-        case 2: return launch_dkv<D, KG, HAS_IDX, 2>(grid, stream, a);
-        case 3: return launch_dkv<D, KG, HAS_IDX, 3>(grid, stream, a);
-        default: return launch_dkv<D, KG, HAS_IDX, 4>(grid, stream, a);
+        case 0: return launch_dkv<D, KG, HAS_IDX, CARRIED, 0>(grid, stream, a);
+        case 1: return launch_dkv<D, KG, HAS_IDX, CARRIED, 1>(grid, stream, a);
+        case 2: return launch_dkv<D, KG, HAS_IDX, CARRIED, 2>(grid, stream, a);
+        case 3: return launch_dkv<D, KG, HAS_IDX, CARRIED, 3>(grid, stream, a);
+        default: return launch_dkv<D, KG, HAS_IDX, CARRIED, 4>(grid, stream, a);
     }
 }
 template <int D, bool HAS_IDX>
@@ -551,9 +554,9 @@ static hipError_t launch_dkv_kg(unsigned grid, hipStream_t stream, const DkvArgs
 #endif
 }
 // grid: workgroups (one per key tile or piece, and kv head).  The file is compiled twice, the second time (DKV_UNALIGNED) for q or dO on no
-// 16-byte boundary; k and v lie on one (the entry points see to it).
+// 16-byte boundary (no CARRIED form there: all of the rows); k and v lie on one (the entry points see to it).
 #define DKV_LAUNCH_ARGS unsigned grid, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v, const float *lse, \
-    const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int causal, int skip_len,   \
+    const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int carried, int causal, int skip_len,   \
     const int32_t *order, float *partial, void *dk, void *dv
 extern "C" hipError_t dsa_launch_dkv_tiles_unaligned(DKV_LAUNCH_ARGS);
 #if DKV_UNALIGNED
@@ -561,7 +564,11 @@ extern "C" hipError_t dsa_launch_dkv_tiles_unaligned(DKV_LAUNCH_ARGS) {
 #else
 extern "C" hipError_t dsa_launch_dkv_tiles(DKV_LAUNCH_ARGS) {
     if (((uintptr_t)q | (uintptr_t)dout) & 15)
-        return dsa_launch_dkv_tiles_unaligned(grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, causal, skip_len, order, partial, dk, dv);
+        return dsa_launch_dkv_tiles_unaligned(grid, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, carried, causal, skip_len, order, partial, dk, dv);
+    if (carried) {
+        const DkvArgs c{dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, logit_scale(scale), causal, skip_len, order, partial, dk, dv};
+        return bitmap ? launch_dkv_gs<256, 1, true, true>(grid, stream, c) : launch_dkv_gs<256, 1, false, true>(grid, stream, c);
+    }
 #endif
     const DkvArgs a{dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, logit_scale(scale), causal, skip_len, order, partial, dk, dv};
     if (bitmap) switch (d_real) {

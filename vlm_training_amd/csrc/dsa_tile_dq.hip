@@ -22,7 +22,7 @@
 #define DQ_RV 3                                          // V tiles: V(t+1) to V(t+3)
 template <int D, int NW> constexpr size_t dq_lds_bytes(bool has_idx) { return (DQ_RK + DQ_RV) * (size_t)DirectTile<D>::BYTES + (has_idx ? NW * 4 * 256 : 0); }
 
-template <int D, bool HAS_IDX, int NW, int RG>
+template <int D, bool HAS_IDX, int NW, int RG, bool CARRIED>
 __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
@@ -30,7 +30,8 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     float scale, int pos_split, int split_len, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
     typedef DirectTile<D> TL;
-    constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;
+    constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT;
+    auto tile_of = [](int dt) __attribute__((always_inline)) { return CARRIED ? carried_tile(dt) : dt; };
     constexpr int LPW = TL::LOADS / NW;                  // wave loads per wave, step and operand
     constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);     // everything a wave requests in a step
     constexpr int AHEAD = 4;                             // operands read ahead
@@ -41,7 +42,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = Hq / Hkv, kvh = blockIdx.x % Hkv, QBW = (NW * RG * 32) >> gshift;
-    const int dr = HAS_IDX ? D : d_real, chunks = dr / 8;   // elements and 16-byte chunks of a row in memory
+    const int dr = HAS_IDX || CARRIED ? D : d_real, chunks = CARRIED ? 2 * KS : dr / 8;   // elements and 16-byte chunks of a row in memory
     int s0, L, blk;
     if (!LOCATE_QUERY_BLOCK(causal, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
         return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(aR[TL::row_q(ks)] + TL::row_imm(ks));
     };
     auto tr_op = [&](int i) __attribute__((always_inline)) {              // MFMA i of dQ: keys of half i / DT, d-tile i % DT
-        const int pair = i / DT, dt = i % DT;
+        const int pair = i / DT, dt = tile_of(i % DT);
         return tr_pair(aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair), aT[TL::tr_q(dt)] + TL::tr_imm(dt, 2 * pair + 1));
     };
     auto advance = [&](lds_u8 *(&a)[4], int by) __attribute__((always_inline)) {
@@ -352,26 +353,26 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
                 const uint32_t b0 = pack2bf(a[8 * i + 4] * scale, a[8 * i + 5] * scale), b1 = pack2bf(a[8 * i + 6] * scale, a[8 * i + 7] * scale);
                 const auto x0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
                 const auto x1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-                *reinterpret_cast<u32x4 *>(rows_out + chunk_at(32 * g + j, 4 * dt + 2 * i + h)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
+                *reinterpret_cast<u32x4 *>(rows_out + chunk_at(32 * g + j, 4 * tile_of(dt) + 2 * i + h)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
             }
         }
 #pragma unroll
     for (int i = 0; i < RG * TL::LOADS; ++i) {
         const int row = i * TL::LOAD_ROWS + lane / TL::CPR, c = lane % TL::CPR, r = r0 + row;
         const int qcol = qc0 + (r >> gshift), head = r & ((1 << gshift) - 1);
-        if (qcol < L && head < G && c < chunks)
+        if (qcol < L && head < G && (CARRIED ? carried_chunk(c, true) : c < chunks))
             *reinterpret_cast<u32x4 *>(dq + ((int64_t)(s0 + qcol) * Hq + kvh * G + head) * dr + c * 8) =
                 *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(row, c));
     }
 }
 
-template <int D, bool HAS_IDX, int RG>
+template <int D, bool HAS_IDX, int RG, bool CARRIED = false>
 static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int gs,
                               int d_real, float scale, int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta, float *delta_out) {
     constexpr int NW = 4;
     constexpr size_t lds = dq_lds_bytes<D, NW>(HAS_IDX);
-    const auto kernel = &dsa_tile_dq_kernel<D, HAS_IDX, NW, RG>;
+    const auto kernel = &dsa_tile_dq_kernel<D, HAS_IDX, NW, RG, CARRIED>;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW * RG) >> gs) + N + 1) * Hkv));
@@ -396,17 +397,18 @@ static bool dq_one_row_group(int causal, int T, int N, int Hkv, int gs) {
     return T / N < 1500 || (rows / 128 * Hkv + 255) / 256 < 2 * (((2 * (rows / 256) + N) * Hkv + 511) / 512);
 }
 // d_real: elements of a row, without a selection any multiple of 8 (dense_kernel_dim).  window: rows of a bitmap at positions below it attend
-// all of their causal window (0: nothing is known).  out_for_delta != null: the kernel forms
+// all of their causal window (0: nothing is known).  carried: see DSA_CARRIED_KS.  out_for_delta != null: the kernel forms
 // delta = rowsum(dO * O) of its rows itself and writes it to delta_out
 extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,
                                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                         int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta, float *delta_out,
+                                         int pos_split, int split_len, int window, int carried, int causal, void *dq, const void *out_for_delta, float *delta_out,
                                          hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
     const bool one_group = dq_one_row_group(causal, T, N, Hkv, gs);
 #define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, dq, out_for_delta, delta_out
 #define DQ_CASE(D_, HI) return one_group ? launch_dq_i<D_, HI, 1>(DQ_ARGS) : launch_dq_i<D_, HI, 2>(DQ_ARGS)
+    if (carried) return bitmap ? launch_dq_i<256, true, 1, true>(DQ_ARGS) : launch_dq_i<256, false, 1, true>(DQ_ARGS);
     if (bitmap) switch (d_real) {
         case 64: DQ_CASE(64, true);
         case 128: DQ_CASE(128, true);

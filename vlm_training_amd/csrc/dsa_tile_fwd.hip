@@ -34,15 +34,16 @@ constexpr size_t fwd_lds_bytes(bool has_idx) { return 8 * (size_t)DirectTile<D>:
 // NEG: the softmax scale is negative.  A masked key's logit is -inf in front of the scale, and the largest one is searched for there, so
 // the kernel's scale is positive and the sign goes into q (an instance of its own: at head_dim 256 as little as a test of the sign in front
 // of the loop made it spill).
-template <int D, bool HAS_IDX, int NW, bool NEG>
+template <int D, bool HAS_IDX, int NW, bool NEG, bool CARRIED>
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
     const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int window, int causal,
     bf16_t *__restrict__ out, float *__restrict__ lse) {
     typedef DirectTile<D> TL;
-    constexpr int KS = D / 16, DT = (D + 31) / 32, NP = 2 * DT;   // MFMAs of S, of P V (head_dim 80: five and six)
-    static_assert(KS <= NP);
+    // MFMAs of S, of P V (head_dim 80: five and six) and pairs of a step (one of each while there are)
+    constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT, NS = KS > NP ? KS : NP;
+    static_assert(KS <= NP || D > 128);
     constexpr int LPW = (TL::LOADS + NW - 1) / NW;          // wave loads per wave, step and operand
     constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);        // everything a wave requests in a step
     static_assert(TL::LOADS % NW == 0, "every wave loads the same number of pieces");
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int klim = causal ? qcol : L - 1;             // last key column this row may attend (dense mode)
 
     // ---- requests ----
-    const int chunks = d_real / 8;
+    const int chunks = CARRIED ? 2 * KS : d_real / 8;
     const int64_t k_step = 32 * k_tok * 2, v_step = 32 * v_tok * 2;      // bytes per tile
     const unsigned char *kptr = reinterpret_cast<const unsigned char *>(k + (int64_t)s0 * k_tok + (int64_t)kvh * k_head);
     const unsigned char *vptr = reinterpret_cast<const unsigned char *>(v + (int64_t)s0 * v_tok + (int64_t)kvh * v_head);
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         // The softmax of an element is a chain of dependent instructions (mask, scale, exponential, sum, pack) and a wave
         // issues in order: behind each MFMA stand the first part of one element's chain, the exponential of the element before
         // and the sum of the one before that, so that no instruction waits for the one in front of it.
-        constexpr int H = 2 * NP - 2;                   // half-steps an element can start in
+        constexpr int H = 2 * NS - 2;                   // half-steps an element can start in
         float y[16], e[16];
         auto behind = [&](int hs) __attribute__((always_inline)) {
 #pragma unroll
@@ -269,15 +270,15 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
+        for (int i = 0; i < (NEXT ? NS : NP); ++i) {
+            if (i < NP) oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
             // this step's requests, spread over its first half: one after the other they would queue for the way into LDS
 #pragma unroll
             for (int r_ = 0; r_ < (HAS_IDX ? 3 : 2); ++r_)
                 if (REQ && r_ * (NP / 2) / 3 == i) request(t_, r_);
             // refill: the operand a few pairs on, of this step's tiles or, past their end, of the next step's
             if (i == NP - VA && SM) advance(va_, t_ + 1);
-            if (i + VA < NP || SM) vr[i % VA] = read_v((i + VA) % NP);
+            if (i < NP && (i + VA < NP || SM)) vr[i % VA] = read_v((i + VA) % NP);
             if (SM) behind(2 * i);
             else __builtin_amdgcn_sched_barrier(0);
             if (NEXT && i < KS) {
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         meet();
     };
     int tt = 0;
-    if constexpr (!HAS_IDX || D <= 128) {
+    if constexpr (!HAS_IDX || D <= 128 || CARRIED) {
         // tiles every row of the block attends whole: the softmax without mask arithmetic (a loop of its own, not a branch
         // in the loop: two bodies that meet again would keep two sets of accumulators); at head_dim 256 a selection leaves it no registers
         const int whole = (HAS_IDX && min(qc0 + QBW, L) > window ? 0 : causal ? qc0 : L) / 32;
@@ -351,16 +352,22 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         bf16_t *op = out + ((int64_t)t * Hq + hq) * d_real;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, oacc[dt], inv, h, chunks - 4 * dt);
+        if (CARRIED) {                                   // V's third part is its first one, the last one zeros
+            store_c_tile(op + 128, oacc[0], inv, h, 4);
+            store_c_tile(op + 160, oacc[1], inv, h, 4);
+            store_c_tile(op + 192, zero16(), inv, h, 4);
+            store_c_tile(op + 224, zero16(), inv, h, 4);
+        }
         if (h == 0) lse[(int64_t)hq * T + t] = (mrun + log2f(l)) * LN2_F;
     }
 }
 
-template <int D, bool HAS_IDX>
+template <int D, bool HAS_IDX, bool CARRIED = false>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int window, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
-    const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false>;
+    const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true, CARRIED> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false, CARRIED>;
     constexpr size_t lds = fwd_lds_bytes<D, NW>(HAS_IDX);
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -370,16 +377,19 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
-// without a bitmap only); window: rows of a bitmap at positions below it attend all of their causal window (0: nothing is known); st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
+// without a bitmap only); window: rows of a bitmap at positions below it attend all of their causal window (0: nothing is known); carried: see DSA_CARRIED_KS; st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
 extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                          int pos_split, int split_len, int window, int causal, void *out, float *lse, hipStream_t stream) {
+                                          int pos_split, int split_len, int window, int carried, int causal, void *out, float *lse, hipStream_t stream) {
     int gs = 0;
     while ((1 << gs) < Hq / Hkv) ++gs;
     scale = logit_scale(scale);
     hipError_t e = hipErrorInvalidValue;
-#define FWD_CASE(D_, HI) e = launch_fwd_i<D_, HI>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, out, lse)
-    if (bitmap) {
+#define FWD_CASE(D_, ...) e = launch_fwd_i<D_, __VA_ARGS__>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, out, lse)
+    if (carried) {
+        if (bitmap) FWD_CASE(256, true, true);
+        else FWD_CASE(256, false, true);
+    } else if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
         else if (d_real <= 128) FWD_CASE(128, true);
         else if (d_real <= 256) FWD_CASE(256, true);
