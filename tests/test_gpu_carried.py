@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from vlm_training_amd import _lib
+from vlm_training_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -48,3 +48,29 @@ def test_carried_rows_give_the_bits_of_whole_rows(Hq, Hkv, segs, K, causal, scal
         assert torch.equal(whole, part)
     assert lib.dsa_attn_fwd(p(q), p(k), p(v), p(idx), p(n), p(cu), T, N, Hq, Hkv, 128, K, scale, _lib.DSA_DTYPE_SPLIT_BF16, ms, causal, p(out), p(lse),
                             p(ws), ws.numel(), stream) == -2
+
+
+@pytest.mark.parametrize("Hq,Hkv,segs,K,causal,dtype", [
+    (16, 2, (700, 65, 129), 100, True, torch.bfloat16),  # a selection with whole windows; gathered rows (past 24 K) in none
+    (4, 4, (1, 500), 64, True, torch.bfloat16), (6, 2, (257,), 300, True, torch.bfloat16), (16, 1, (1500, 40), 64, True, torch.bfloat16),
+    (8, 4, (400, 31), None, True, torch.bfloat16), (2, 1, (128, 333), None, False, torch.bfloat16),
+    (4, 1, (300, 64), 50, True, torch.float32), (2, 2, (350,), None, True, torch.float32)])
+def test_both_passes_in_one_launch_give_the_bits_of_two(Hq, Hkv, segs, K, causal, dtype):
+    print("one launch", Hq, Hkv, segs, K, causal, dtype, flush=True)
+    lib, D = _lib.load(), 256 if dtype == torch.bfloat16 else 64
+    g = torch.Generator().manual_seed(Hq + sum(segs))
+    T, cu = sum(segs), torch.tensor([0] + list(segs)).cumsum(0).int().to(DEV)
+    mk = lambda *s: torch.randn(*s, generator=g).mul_(0.5).to(dtype).to(DEV)
+    q, k, v, do = mk(T, Hq, D), mk(T, Hkv, D), mk(T, Hkv, D), mk(T, Hq, D)
+    sel = dict(indexer_q=mk(T, 4, 64), indexer_k=mk(T, 64), indexer_w=mk(T, 4), top_k=K) if K else dict(causal=causal)
+    res, old = [], lib.dsa_get_bwd_overlap()
+    try:
+        for mode in (0, 2):
+            _lib.check(lib.dsa_set_bwd_overlap(mode), "dsa_set_bwd_overlap")
+            a, b, c = (x.clone().requires_grad_(True) for x in (q, k, v))
+            ops.dsa_varlen_attn(a, b, c, cu, max(segs), **sel).backward(do)
+            res.append((a.grad, b.grad, c.grad))
+    finally:
+        lib.dsa_set_bwd_overlap(old)
+    for one, two in zip(*res):
+        assert torch.equal(one, two)

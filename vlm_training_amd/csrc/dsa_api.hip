@@ -44,6 +44,7 @@ size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw);
 hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, const uint32_t *bitmap, int ldw,
                                 const int32_t *n, const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K,
                                 float scale, float *partial, float *mass, hipStream_t stream);
+struct DqBeside { int window; void *dq; };                // (dQ in the key side's launch)
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
                                int window, int carried, int causal, void *out, float *lse, hipStream_t stream);
@@ -54,7 +55,7 @@ hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, co
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
                                int Hq, int Hkv, int D, float scale, int carried, int causal, int skip_len, int32_t *order, int listed, float *partial,
-                               size_t partial_bytes, void *dk, void *dv, hipStream_t stream);
+                               size_t partial_bytes, void *dk, void *dv, const DqBeside *beside, hipStream_t stream);
 hipError_t dsa_launch_tile_order_delta(const void *dout, const void *out, const int32_t *cu, int N, int T, int Hq, int Hkv, int D,
                                        int has_idx, int causal, int32_t *order, const float *partial, size_t partial_bytes,
                                        float *delta, hipStream_t stream);
@@ -489,7 +490,7 @@ extern "C" int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const fl
 // mode 1 runs the passes side by side for key-side launches of at most this many workgroups (larger ones fill the GPU
 // alone) whose work bound T * max_seqlen * Hq * D reaches the second figure: below it the host issues a step more slowly than
 // the GPU runs it, and the fork, the join and the pass over dO and O (with the key side's list in the same launch) cost more
-// than the overlap gains.  Step times, one after the other -> side by side: fp32 2048 tokens 217 -> 170 us; head_dim 128 packed
+// than the overlap gains (head_dim 256 has both passes in one launch instead).  Step times, one after the other -> side by side: head_dim 128 packed
 // rows of 4096-8192 tokens, 5-19 % less; 10 000-16 384 tokens, 0-3 % less; 1000 tokens at 2e9, 130 -> 105; 700 tokens at 7e8,
 // level.  Without a causal mask the walks of a segment are all equally long, and small launches win nothing.
 #define DSA_BWD_OVERLAP_MAX_WG (6 * 256)
@@ -631,7 +632,12 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     std::unique_lock<std::mutex> ov_lock;
     OverlapCtx *ov = nullptr;
     const int ov_mode = g_bwd_overlap.load(std::memory_order_relaxed);
-    if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0) {
+    // head_dim 256: both passes in one launch (dsa_tile_bwd.hip), whatever its size.  Backward, us, one after the other with delta from dQ -> one launch:
+    // 16 heads over 2: 700 and 300 tokens 114 -> 81, eight segments of 512 132 -> 122, 16 of 1000 604 -> 570, 4 of 4096 1854 -> 1735, 4 of 8192 6397 -> 6440;
+    // fp32 rows of 64, 8 heads over 2: 75 -> 60, 82 -> 69, 287 -> 271, 727 -> 677, 2405 -> 2410; without a causal mask, eight of 700 330 -> 258.
+    const bool one_launch = ov_mode > 0 && (parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && D == 256 && max_seqlen <= rows.tiles &&
+                            !(((uintptr_t)q | (uintptr_t)dout) & 15);
+    if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0 && !one_launch) {
         const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);     // (head_dim 256: one workgroup per CU, half as many fill it)
         const double work = (double)T * max_seqlen * Hq * D;
         if (ov_mode == 2 || (dkv_wg <= DSA_BWD_OVERLAP_MAX_WG && work >= (causal ? DSA_BWD_OVERLAP_MIN_WORK : DSA_BWD_OVERLAP_MIN_WORK_FULL))) {
@@ -643,9 +649,9 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     // delta = rowsum(dO * O): a pass of its own, unless the tile dQ kernel of the same call owns every query row
     // (no row beyond the tile/gather split) - then that kernel forms it from the dO rows it loads anyway - and the
     // key side, which reads every delta, runs after it
-    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.past_tiles(max_seqlen) && !ov;
+    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.past_tiles(max_seqlen) && !ov && !one_launch;
     int listed = 0;                                      // the launch order of the key tiles is there
-    if ((parts & DSA_BWD_DELTA) && ov) {
+    if ((parts & DSA_BWD_DELTA) && (ov || one_launch)) {
         e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, selected, causal, order, partial, partial_bytes, delta, st);
         if (e == hipSuccess) listed = 1;
         else if (e != hipErrorNotReady) return hip_fail(e, "order and delta launch");   // (not ready: this launch needs no list)
@@ -667,16 +673,17 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     }
     int rc = DSA_OK;
     const int walk_len = key_walk_len(selected, q, dout, T, N, Hq, Hkv, D, K);
+    const DqBeside beside{idx ? 0 : K, dq};
     auto key_side = [&]() {
         hipError_t e = dsa_launch_tile_dkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, carried, causal, walk_len, order, listed,
-                                           partial, partial_bytes, dk, dv, st);
+                                           partial, partial_bytes, dk, dv, one_launch ? &beside : nullptr, st);
         if (e == hipSuccess && max_seqlen >= walk_len)
             e = dsa_launch_selkv(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, softmax_scale, walk_len, dk, dv, st);
         return e == hipSuccess ? DSA_OK : hip_fail(e, "dkv launch");
     };
     // (side by side, the key side is issued first: it is the longer pass and starts with its longest walks)
     if (ov) rc = key_side();
-    if (rc == DSA_OK && (parts & DSA_BWD_DQ)) {
+    if (rc == DSA_OK && (parts & DSA_BWD_DQ) && !one_launch) {
         if (rows.tiles > 0) {
             e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
                                    idx ? 0 : K, carried, causal, dq, fuse_delta ? out : nullptr, delta, sq);

@@ -687,19 +687,25 @@ extern "C" hipError_t dsa_launch_dkv_tiles(unsigned grid, hipStream_t stream, co
                                            const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
                                            int T, int Hq, int Hkv, int d_real, float scale, int carried, int causal, int skip_len, const int32_t *order,
                                            float *partial, void *dk, void *dv);
-// listed: dsa_launch_tile_order_delta has left the list in `order`
+extern "C" hipError_t dsa_launch_dkv_dq_tiles(unsigned key_blocks, hipStream_t stream, const void *dout, const void *q, const void *k, const void *v,
+                                              const float *lse, const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N,
+                                              int T, int Hq, int Hkv, float scale, int carried, int causal, const int32_t *order, float *partial,
+                                              void *dk, void *dv, int window, void *dq);
+// listed: dsa_launch_tile_order_delta has left the list in `order`.  beside: null, or dQ in the same launch (head_dim 256)
 extern "C" hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v,
                                           const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
                                           const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale, int carried, int causal, int skip_len,
                                           int32_t *order, int listed, float *partial, size_t partial_bytes, void *dk, void *dv,
-                                          hipStream_t stream) {
+                                          const DqBeside *beside, hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
     const DkvPlan p = dkv_plan(T, N, Hq, Hkv, d_real, bitmap != nullptr, causal, order, partial, partial_bytes);
     dim3 grid((unsigned)((p.pieces ? p.o.item_cap : p.tiles_ub + 1) * Hkv));
     if (!p.listed) order = nullptr;
     else if (!listed) hipLaunchKernelGGL(dsa_tile_order_kernel, dim3(1), dim3(1024), 0, stream, cu, N, p.o, order);
     if (!p.pieces) partial = nullptr;
-    const hipError_t e = dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, carried,
+    const hipError_t e = beside ? dsa_launch_dkv_dq_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, carried, causal,
+                                                          order, partial, dk, dv, beside->window, beside->dq) :
+                         dsa_launch_dkv_tiles(grid.x, stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, carried,
                                               causal, skip_len, order, partial, dk, dv);
     if (e != hipSuccess) return e;
     if (p.pieces)
