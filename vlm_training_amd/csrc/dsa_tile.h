@@ -54,36 +54,6 @@ __device__ __forceinline__ void store_c_tile(bf16_t *row_dt, const f32x16 &acc, 
     }
 }
 
-// slot -> (segment, block) for blocks of `blk` columns handed out segment by segment; within a segment
-// the blocks are numbered from the end when `reverse` (heaviest causal blocks first).  Returns false
-// for spare slots.  The segment bounds are fetched 64 segments at a time, one per lane (one memory
-// round trip instead of one per segment), and walked with lane reads.
-__device__ __forceinline__ bool locate_block(const int32_t *cu, int N, int slot, int blk, bool reverse, int &s0, int &L,
-                                             int &b) {
-    const int lane = threadIdx.x & 63;
-    for (int base = 0; base < N; base += 64) {
-        const int seg = min(base + lane, N - 1);
-        const int lo = cu[seg], len = cu[seg + 1] - lo;
-        const int cnt = min(64, N - base);
-        for (int w = 0; w < cnt; ++w) {
-            L = __builtin_amdgcn_readlane(len, w);
-            const int nb = (L + blk - 1) / blk;
-            if (slot < nb) {
-                s0 = __builtin_amdgcn_readlane(lo, w);
-                b = reverse ? nb - 1 - slot : slot;
-                return true;
-            }
-            slot -= nb;
-        }
-    }
-    return false;
-}
-
-// The same hand-out, heaviest block first over the whole batch: slot 0 takes the last block of the longest segment,
-// then every block with the next lower index in segment order, and so on - a block's walk grows with its index, so
-// long walks start first wherever their segment lies in the batch (with the segment-by-segment order the long
-// walks of a late segment start late and the launch ends on them).  For up to 64 segments (their lengths live in
-// one wave's lanes); larger batches fall back to the segment-by-segment order.
 // Sum / maximum (of values >= 0) over the wave, wave-uniform: DPP steps inside the rows of sixteen lanes, then across them -
 // no LDS round trips (the search below takes about ten of these sums in front of a workgroup's first load; by lane
 // shuffles they cost it 2 us).
@@ -99,6 +69,47 @@ __device__ __forceinline__ int wave_fold_i(int x, F f) {
 }
 __device__ __forceinline__ int wave_sum_i(int x) { return wave_fold_i(x, [](int a, int b) { return a + b; }); }
 __device__ __forceinline__ int wave_max_i(int x) { return wave_fold_i(x, [](int a, int b) { return max(a, b); }); }
+// Sums over the lanes up to and with one's own, the same way
+__device__ __forceinline__ int wave_prefix_i(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+
+// slot -> (segment, block) for blocks of `blk` columns handed out segment by segment; within a segment
+// the blocks are numbered from the end when `reverse` (heaviest causal blocks first).  Returns false
+// for spare slots.  The segments are searched 64 at a time, one per lane: where one's blocks begin is a sum over the lanes in front (a walk from
+// segment to segment took a workgroup 3100 clocks with 16 of them, 8200 with 64).
+__device__ __forceinline__ bool locate_block(const int32_t *cu, int N, int slot, int blk, bool reverse, int &s0, int &L,
+                                             int &b) {
+    const int lane = threadIdx.x & 63;
+    for (int base = 0; base < N; base += 64) {
+        const int seg = min(base + lane, N - 1);
+        const int lo = cu[seg], len = cu[seg + 1] - lo;
+        const int nb = base + lane < N ? (len + blk - 1) / blk : 0, upto = wave_prefix_i(nb);
+        const uint64_t past = __builtin_amdgcn_ballot_w64(upto > slot);
+        if (past) {
+            const int w = (int)__builtin_ctzll(past);
+            s0 = __builtin_amdgcn_readlane(lo, w);
+            L = __builtin_amdgcn_readlane(len, w);
+            const int n = __builtin_amdgcn_readlane(nb, w), at = slot - (__builtin_amdgcn_readlane(upto, w) - n);
+            b = reverse ? n - 1 - at : at;
+            return true;
+        }
+        slot -= __builtin_amdgcn_readlane(upto, 63);
+    }
+    return false;
+}
+
+// The same hand-out, heaviest block first over the whole batch: slot 0 takes the last block of the longest segment,
+// then every block with the next lower index in segment order, and so on - a block's walk grows with its index, so
+// long walks start first wherever their segment lies in the batch (with the segment-by-segment order the long
+// walks of a late segment start late and the launch ends on them).  For up to 64 segments (their lengths live in
+// one wave's lanes); larger batches fall back to the segment-by-segment order.
 __device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, int N, int slot, int blk, int &s0, int &L,
                                                             int &b) {
     if (N > 64) return locate_block(cu, N, slot, blk, true, s0, L, b);
@@ -134,8 +145,8 @@ __device__ __forceinline__ bool locate_block_heaviest_first(const int32_t *cu, i
 // Without a causal mask the walks of a segment are equally long and there is nothing to balance inside it: segment by segment
 // (12 288 patches of 13 images, forward and backward: 485 us, in the batch-wide order 549).
 #define DSA_BATCH_ORDER_MAX_BLOCKS (6 * 256)
-#define LOCATE_QUERY_BLOCK(causal, cu, N, slot, blk, s0, L, b)                                                   \
-    ((causal) && gridDim.x <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
+#define LOCATE_QUERY_BLOCK(causal, blocks, cu, N, slot, blk, s0, L, b)                                           \
+    ((causal) && (blocks) <= DSA_BATCH_ORDER_MAX_BLOCKS ? locate_block_heaviest_first(cu, N, slot, blk, s0, L, b)          \
                                              : locate_block(cu, N, slot, blk, true, s0, L, b))
 
 // ---- LDS tiles filled straight from memory ------------------------------------------------------------------------------
@@ -182,6 +193,23 @@ struct DirectTile {
     static constexpr int tr_imm(int dt, int v) { return (D == 64 ? 0 : (dt >> 2) * 256) + v * (8 / GROUP) * GROUP_B; }
 };
 
+// Where the rows of a wave lie that a piece of a tile holds, a row being a (query, head of the kv group): rows first + p * LOAD_ROWS + l of the
+// wave's first query on, l = lane / CPR.  A piece never splits a query's heads unevenly, so that a row's place is a sum of what the piece
+// and what the lane says.
+template <class TL>
+struct WaveRows {
+    int gshift, lane_query, lane_head;
+    __device__ __forceinline__ WaveRows(int gshift_, int lane) : gshift(gshift_), lane_query((lane / TL::CPR) >> gshift_), lane_head((lane / TL::CPR) & ((1 << gshift_) - 1)) {}
+    // of row first + p * LOAD_ROWS + l: the query behind the wave's first one, the head
+    __device__ __forceinline__ int query(int p, int first = 0) const { return ((first + p * TL::LOAD_ROWS) >> gshift) + lane_query; }
+    __device__ __forceinline__ int head(int p, int first = 0) const { return ((first + p * TL::LOAD_ROWS) & ((1 << gshift) - 1)) + lane_head; }
+    // its byte offset from the first query's first head: tok_b, head_b bytes from one query, one head to the next
+    __device__ __forceinline__ int place(int tok_b, int head_b) const { return lane_query * tok_b + lane_head * head_b; }
+    __device__ __forceinline__ int piece(int p, int tok_b, int head_b, int first = 0) const {
+        return ((first + p * TL::LOAD_ROWS) >> gshift) * tok_b + ((first + p * TL::LOAD_ROWS) & ((1 << gshift) - 1)) * head_b;
+    }
+};
+
 // ---- one wave per SIMD: sums in accumulation registers, phases of mixed operands ----
 // c += a b with c in accumulation registers, named here: left to itself the compiler keeps 128 to 256 registers of sums where the
 // vector instructions need them, and spills.  It does not see an MFMA in this statement, so its hazards are held by hand: an operand
@@ -192,6 +220,12 @@ __device__ __forceinline__ void mfma32_agpr(f32x16 &c, bf16x8 a, bf16x8 b, bool 
     if (last) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+a"(c) : "v"(a), "v"(b));
     else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     __builtin_amdgcn_sched_barrier(0);                   // (nor does it see where the vector instructions behind it belong)
+}
+// the same behind operands that the compiler may have just moved or formed: it waits for them itself
+__device__ __forceinline__ void mfma32_agpr_late(f32x16 &c, bf16x8 a, bf16x8 b, bool last) {
+    if (last) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+a"(c) : "v"(a), "v"(b));
+    else asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    __builtin_amdgcn_sched_barrier(0);
 }
 // the tuple's value lies in accumulation registers here; in front of its uses: the tuples leave them one by one
 __device__ __forceinline__ void settle(f32x16 &c) { asm volatile("" : "+a"(c)); }

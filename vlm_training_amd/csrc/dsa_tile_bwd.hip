@@ -16,7 +16,7 @@ __global__ __launch_bounds__(256, 1) void dsa_tile_dkv_kernel_and_dq(
         dkv_block<256, 1, HAS_IDX, GSHIFT, false, CARRIED>(blockIdx.x, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, logit_scale,
                                                            causal, 256, INT32_MAX, order, partial, dk, dv);
     else
-        dq_block<256, HAS_IDX, 4, 1, CARRIED>(blockIdx.x - key_blocks, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, GSHIFT, scale,
+        dq_block<256, HAS_IDX, 4, 1, CARRIED>(blockIdx.x - key_blocks, gridDim.x - key_blocks, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, GSHIFT, scale,
                                               INT32_MAX, 0, window, causal, 256, dq, nullptr, nullptr);
 }
 

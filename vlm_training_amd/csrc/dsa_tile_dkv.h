@@ -479,6 +479,9 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     // a workgroup).  16-byte chunk c of row r sits at c ^ x(r): sixteen rows at one chunk and the chunks of a row each cover the banks once.
     barrier_only();                                      // the ring is read out
     unsigned char *const rows_out = dyn_lds + wv * (2 * KG * 32 * TL::ROW_B);
+    int lane_ = lane;                                    // (places are formed here: the loop needs its registers)
+    asm volatile("" : "+v"(lane_));
+    const int h_ = lane_ >> 5, j_ = lane_ & 31;
     auto chunk_at = [&](int row, int c) __attribute__((always_inline)) {
         return row * TL::ROW_B + ((c ^ (D == 64 ? (row >> 1) & 7 : row & 15)) << 4);
     };
@@ -497,18 +500,24 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
                     const uint32_t b0 = pack2bf(acc[8 * i + 4] * mul, acc[8 * i + 5] * mul), b1 = pack2bf(acc[8 * i + 6] * mul, acc[8 * i + 7] * mul);
                     const auto r0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
                     const auto r1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-                    *reinterpret_cast<u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(j, 4 * tile_of(dt, m) + 2 * i + h)) = u32x4{r0[0], r1[0], r0[1], r1[1]};
+                    *reinterpret_cast<u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(j_, 4 * tile_of(dt, m) + 2 * i + h_)) = u32x4{r0[0], r1[0], r0[1], r1[1]};
                 }
             }
 #pragma unroll
     for (int g = 0; g < KG; ++g)
 #pragma unroll
         for (int m = 0; m < 2; ++m)
+            for (int part = 0; part < (TL::LOADS > 8 ? 2 : 1); ++part) {  // (up to eight rows read in front of their stores)
+                constexpr int NL = TL::LOADS > 8 ? 8 : TL::LOADS;
+                const int row0 = part * NL * TL::LOAD_ROWS + lane_ / TL::CPR, c = lane_ % TL::CPR, key0 = kc + 32 * g + row0;
+                u32x4 x[NL];
 #pragma unroll
-            for (int i = 0; i < TL::LOADS; ++i) {
-                const int row = i * TL::LOAD_ROWS + lane / TL::CPR, c = lane % TL::CPR, key = kc + 32 * g + row;
-                if (key < L && (CARRIED ? carried_chunk(c, m) : c < chunks))
-                    *reinterpret_cast<u32x4 *>((m ? dv : dk) + ((int64_t)(s0 + key) * Hkv + kvh) * dr + c * 8) =
-                        *reinterpret_cast<const u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(row, c));
+                for (int i = 0; i < NL; ++i)
+                    x[i] = *reinterpret_cast<const u32x4 *>(rows_out + (2 * g + m) * 32 * TL::ROW_B + chunk_at(row0 + i * TL::LOAD_ROWS, c));
+                unsigned char *const to = reinterpret_cast<unsigned char *>((m ? dv : dk) + ((int64_t)(s0 + key0) * Hkv + kvh) * dr + c * 8);
+#pragma unroll
+                for (int i = 0; i < NL; ++i)
+                    if (key0 + i * TL::LOAD_ROWS < L && (CARRIED ? carried_chunk(c, m) : c < chunks))
+                        *reinterpret_cast<u32x4 *>(to + i * TL::LOAD_ROWS * Hkv * dr * 2) = x[i];
             }
 }

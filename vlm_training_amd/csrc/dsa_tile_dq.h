@@ -23,9 +23,9 @@
 #define DQ_RV 3                                          // V tiles: V(t+1) to V(t+3)
 template <int D, int NW> constexpr size_t dq_lds_bytes(bool has_idx) { return (DQ_RK + DQ_RV) * (size_t)DirectTile<D>::BYTES + (has_idx ? NW * 4 * 256 : 0); }
 
-// One workgroup of a launch, number `block`
+// Workgroup `block` of `blocks`
 template <int D, bool HAS_IDX, int NW, int RG, bool CARRIED>
-__device__ __forceinline__ void dq_block(int block,
+__device__ __forceinline__ void dq_block(int block, int blocks,
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift,
@@ -46,7 +46,7 @@ __device__ __forceinline__ void dq_block(int block,
     const int G = Hq / Hkv, kvh = block % Hkv, QBW = (NW * RG * 32) >> gshift;
     const int dr = HAS_IDX || CARRIED ? D : d_real, chunks = CARRIED ? 2 * KS : dr / 8;   // elements and 16-byte chunks of a row in memory
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(causal, cu, N, block / Hkv, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(causal, blocks, cu, N, block / Hkv, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                   // a bitmap row has ldw words whatever the caller's max_seqlen
@@ -358,12 +358,18 @@ __device__ __forceinline__ void dq_block(int block,
                 *reinterpret_cast<u32x4 *>(rows_out + chunk_at(32 * g + j, 4 * tile_of(dt) + 2 * i + h)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
             }
         }
+    // (a group's rows read in front of its first store: a read and its store in turn would wait for the LDS each time)
+    const WaveRows<TL> wr(gshift, lane);
+    const int q0 = qc0 + (r0 >> gshift), to_tok = Hq * dr * 2, c = lane % TL::CPR, place = wr.place(to_tok, dr * 2) + c * 16;
+    unsigned char *const to = reinterpret_cast<unsigned char *>(dq + ((int64_t)(s0 + q0) * Hq + kvh * G) * dr);
 #pragma unroll
-    for (int i = 0; i < RG * TL::LOADS; ++i) {
-        const int row = i * TL::LOAD_ROWS + lane / TL::CPR, c = lane % TL::CPR, r = r0 + row;
-        const int qcol = qc0 + (r >> gshift), head = r & ((1 << gshift) - 1);
-        if (qcol < L && head < G && (CARRIED ? carried_chunk(c, true) : c < chunks))
-            *reinterpret_cast<u32x4 *>(dq + ((int64_t)(s0 + qcol) * Hq + kvh * G + head) * dr + c * 8) =
-                *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(row, c));
+    for (int g = 0; g < RG; ++g) {
+        u32x4 x[TL::LOADS];
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i) x[i] = *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(32 * g + i * TL::LOAD_ROWS + lane / TL::CPR, c));
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i)
+            if (q0 + wr.query(i, 32 * g) < L && wr.head(i, 32 * g) < G && (CARRIED ? carried_chunk(c, true) : c < chunks))
+                *reinterpret_cast<u32x4 *>(to + (place + wr.piece(i, to_tok, dr * 2, 32 * g))) = x[i];
     }
 }

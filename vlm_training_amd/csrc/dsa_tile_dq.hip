@@ -8,7 +8,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift,
     float scale, int pos_split, int split_len, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
-    dq_block<D, HAS_IDX, NW, RG, CARRIED>(blockIdx.x, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, scale, pos_split, split_len, window, causal, d_real, dq, out_for_delta, delta_out);
+    dq_block<D, HAS_IDX, NW, RG, CARRIED>(blockIdx.x, gridDim.x, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, scale, pos_split, split_len, window, causal, d_real, dq, out_for_delta, delta_out);
 }
 
 template <int D, bool HAS_IDX, int RG, bool CARRIED = false>

@@ -18,14 +18,20 @@
 // What bounds it: the power of the chip (MFMA busy 0.61 of a CU's time without a selection, at 1.79 GHz) and, with a selection, the
 // vector instructions (about 92 and 16 exponentials beside 16 MFMAs at head_dim 128, 32 of them the mask); the softmax of tiles every row
 // attends whole drops the mask: all but the last without a selection, those of blocks inside the first K positions with one (`window`; the
-// same in dQ.  Step of 8192 tokens, K = 1024: 300.2 -> 295.4 us, forward of 16 384 in mixed segments, K = 2048: 673 -> 661; not at head_dim 256,
-// where the second loop's spilled registers took 3 % of a step instead).  Both make every instruction beside the MFMAs count: a tile's buffer size comes from two
+// same in dQ.  Step of 8192 tokens, K = 1024: 300.2 -> 295.4 us, forward of 16 384 in mixed segments, K = 2048: 673 -> 661).  Both make every instruction beside the MFMAs count: a tile's buffer size comes from two
 // constants, its pieces follow one another under one buffer, operand addresses move on in place.  Same box, us, against a size formed per
 // piece, addresses formed per tile and eight waves per workgroup in large launches: 32 768 tokens dense 1289 -> 1229, with a selection
 // 1408 -> 1371; 8192 tokens with a selection 62.5 -> 59; 512 tokens 15.9 -> 15.1; head_dim 256, 16 384 tokens 210 -> 195; vision towers at
 // head_dim 72 354 -> 335, at 64 282 -> 269.  Four waves per workgroup, two workgroups per CU: eight waves that share each staged tile took
 // 1255 dense.  64 rows per wave, one wave per SIMD: level at 32 768 tokens (MFMA busy 0.52 at 1.95 GHz), slower in short launches.
-// At head_dim 256 the loop must not read spilled registers: such a read waits for every tile on its way into LDS (+ 20 %).
+// What a block costs beside its tiles, clocks at head_dim 256 / 128: 26 000 / 15 000 when its segment was searched for one by one, q read where it lies
+// (each load touches 32 rows), the first tiles waited for all together and the output stored 32 bytes of a row at a time.  Search by a prefix
+// sum, q through LDS in whole rows, S(0) and S(1) as soon as K(0) and K(1) are there, output in whole rows.  Forward of 16 384 tokens, us,
+// head_dim 128, 16 heads over 8, segments of 64 / 256 / 1024 / 2048: 215 / 68.6 / 95.7 / 164.8 -> 45 / 51.5 / 91 / 162; head_dim 256, 16 heads over 2, of 64 / 256 /
+// 512 / 1024 / 2048: 227 / 151 / 165 / 214 / 316 -> 106 / 129 / 142 / 190 / 308, there most of the rest is q and the output at 3 to 5 TB/s, which one workgroup per CU
+// does not hide.
+// At head_dim 256 the sums lie in accumulation registers by name: left to the compiler the loops of three of the four instances read spilled
+// registers, and such a read waits for every tile on its way into LDS (+ 20 %).
 #include "dsa_tile.h"
 
 template <int D, int NW>
@@ -44,6 +50,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     // MFMAs of S, of P V (head_dim 80: five and six) and pairs of a step (one of each while there are)
     constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT, NS = KS > NP ? KS : NP;
     static_assert(KS <= NP || D > 128);
+    constexpr bool AGPR = D > 128;                          // the sums in accumulation registers, by name (mfma32_agpr_late)
     constexpr int LPW = (TL::LOADS + NW - 1) / NW;          // wave loads per wave, step and operand
     constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);        // everything a wave requests in a step
     static_assert(TL::LOADS % NW == 0, "every wave loads the same number of pieces");
@@ -53,7 +60,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = Hq / Hkv, kvh = blockIdx.x % Hkv, QBW = (NW * 32) >> gshift;
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(causal, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(causal, gridDim.x, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
@@ -111,24 +118,55 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             next(wptr, tile + 1 < ntiles ? 4 : 0);       // (past the block's tiles: the last word again, never used)
         }
     };
+    // The wave's rows of q, whole rows at a time into the V slot of its number and from there into registers (read where they lie, each load
+    // would touch 32 rows); rows that are not on 16-byte boundaries or too far apart for an offset: where they lie
     bf16x8 qB[KS];
-    const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
-        if (NEG) qB[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, qB[ks]) ^ 0x80008000u);
-    }
-    load_k(0); load_w(0); load_k(1); load_w(1); load_v(0); load_k(2); load_w(2); load_v(1); load_k(3); load_w(3); load_v(2);
-
     TL tl;
     tl.init(lane);
+    const bool staged = !((reinterpret_cast<uintptr_t>(q) | (uintptr_t)(q_tok * 2) | (uintptr_t)(q_head * 2)) & 15) &&
+                        31 * q_tok + (int64_t)(G - 1) * q_head < (1 << 30) - D;
+    if (staged) {
+        const buffer_rsrc rows = make_buffer_rsrc(q + (int64_t)(s0 + wq0) * q_tok + (int64_t)kvh * G * q_head, 0x7fffffff);
+        const WaveRows<TL> wr(gshift, lane);
+        const int there = L - (qc0 + ((wv * 32) >> gshift)), tok_b = (int)q_tok * 2, head_b = (int)q_head * 2, place = wr.place(tok_b, head_b);
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i) {
+            const int c = (lane % TL::CPR) ^ TL::xor_of(i * TL::LOAD_ROWS + lane / TL::CPR);
+            const int off[1] = {wr.query(i) < there && wr.head(i) < G && c < chunks ? place + wr.piece(i, tok_b, head_b) + c * 16 : (int)0x80000000};
+            buffer_load_lds16_n<1, 0, 0, 0>(rows, off, lds0 + (4 + wv) * TL::BYTES + TL::load_lds(i));
+        }
+    }
+    load_k(0); load_w(0); load_k(1); load_w(1); load_k(2); load_w(2); load_k(3); load_w(3);
+    constexpr int AFTER_K1 = 2 * LPW + (HAS_IDX ? 2 : 0);
+    if (staged) {
+        wait_vmcnt<AFTER_K1>();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            qB[ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>((lds_u8 *)dyn_lds + (4 + wv) * TL::BYTES + tl.rowq[TL::row_q(ks)] + TL::row_imm(ks));
+    } else {
+        const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
+    }
+    if (NEG) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qB[ks] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, qB[ks]) ^ 0x80008000u);
+    }
     f32x16 oacc[DT], sE, sO;                            // S of even and of odd tiles
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) oacc[dt] = zero16();
+    for (int dt = 0; dt < DT; ++dt) {
+        oacc[dt] = zero16();
+        if (AGPR) settle(oacc[dt]);
+    }
     uint32_t pE[8], pO[8];                              // P of even and of odd tiles, packed (keys 0-15 | 16-31)
     float mrun = -INFINITY, lsum = 0.f;
-    wait_vmcnt<0>();
-    barrier_only();
+    auto meet_read = [&]() __attribute__((always_inline)) {               // (what this wave reads of LDS is read)
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        barrier_only();
+    };
+    wait_vmcnt<AFTER_K1>();                             // K(0) and K(1) are there
+    meet_read();
+    load_v(0); load_v(1); load_v(2);
 
     lds_u8 *ka_[4], *va_[4];                            // operand addresses: of the K tile of S(t+2) and of V(t)
 #pragma unroll
@@ -175,8 +213,13 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             if (mloc > mrun) {
                 const float alpha = fast_exp2(mrun - mloc);   // mrun = -inf: 0, and the sums are 0
                 lsum *= alpha;
+                if (AGPR) asm volatile("s_nop 11" : : : "memory");
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+                for (int dt = 0; dt < DT; ++dt) {
+                    if (AGPR) ::settle(oacc[dt]);
+                    oacc[dt] *= alpha;
+                    if (AGPR) ::settle(oacc[dt]);
+                }
                 mrun = mloc;
             }
             const float mneg = (mrun == -INFINITY) ? 0.f : -mrun;
@@ -211,7 +254,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         for (int i = 0; i < 8; ++i) pE[i] = 0u;
         settle(sE, live(word_of(0)), pE, psum);
     }
-    __syncthreads();                                    // every wave is done with K(0) and K(1): their slots may be filled again
+    wait_vmcnt<2 * LPW>();                              // all but V(1) and V(2)
+    meet_read();                                        // every wave is done with K(0) and K(1): their slots may be filled again
     load_k(4);
     constexpr int KA = KS % 5 == 0 ? 5 : KS % 4 ? 3 : 4, VA = NP % 4 ? 3 : 4;   // (divide KS and NP: an operand keeps its register from step to step)
     static_assert(KS % KA == 0 && NP % VA == 0);
@@ -271,7 +315,10 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         };
 #pragma unroll
         for (int i = 0; i < (NEXT ? NS : NP); ++i) {
-            if (i < NP) oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
+            if (i < NP) {
+                if (AGPR) mfma32_agpr_late(oacc[i % DT], vr[i % VA], i < DT ? pB0 : pB1, !SM);
+                else oacc[i % DT] = mfma32(vr[i % VA], i < DT ? pB0 : pB1, oacc[i % DT]);
+            }
             // this step's requests, spread over its first half: one after the other they would queue for the way into LDS
 #pragma unroll
             for (int r_ = 0; r_ < (HAS_IDX ? 3 : 2); ++r_)
@@ -303,9 +350,9 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         meet();
     };
     int tt = 0;
-    if constexpr (!HAS_IDX || D <= 128 || CARRIED) {
+    {
         // tiles every row of the block attends whole: the softmax without mask arithmetic (a loop of its own, not a branch
-        // in the loop: two bodies that meet again would keep two sets of accumulators); at head_dim 256 a selection leaves it no registers
+        // in the loop: two bodies that meet again would keep two sets of accumulators)
         const int whole = (HAS_IDX && min(qc0 + QBW, L) > window ? 0 : causal ? qc0 : L) / 32;
         for (; tt + 3 < ntiles && tt + 2 < whole; tt += 2) {
             full_step(no, tt, pE, sO, pO, sE);
@@ -346,20 +393,47 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     }
     wait_vmcnt<0>();                                    // no load is left on its way into LDS when the workgroup ends
 
-    float l = half_sum_f(lsum);
-    if (row_ok) {
-        const float inv = 1.f / l;
-        bf16_t *op = out + ((int64_t)t * Hq + hq) * d_real;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) store_c_tile(op + dt * 32, oacc[dt], inv, h, chunks - 4 * dt);
-        if (CARRIED) {                                   // V's third part is its first one, the last one zeros
-            store_c_tile(op + 128, oacc[0], inv, h, 4);
-            store_c_tile(op + 160, oacc[1], inv, h, 4);
-            store_c_tile(op + 192, zero16(), inv, h, 4);
-            store_c_tile(op + 224, zero16(), inv, h, 4);
-        }
-        if (h == 0) lse[(int64_t)hq * T + t] = (mrun + log2f(l)) * LN2_F;
+    const float l = half_sum_f(lsum), inv = 1.f / l;
+    // (where the rows lie is formed again: the loop needs its registers)
+    int tid_ = tid;
+    asm volatile("" : "+v"(tid_));
+    const int lane_ = tid_ & 63, h_ = lane_ >> 5, j_ = lane_ & 31;
+    {
+        const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
+        if (qc < L && hd < G && h_ == 0) lse[(int64_t)(kvh * G + hd) * T + s0 + qc] = (mrun + log2f(l)) * LN2_F;
     }
+    // whole rows per store, through LDS (as in dQ)
+    barrier_only();                                     // the rings are read out
+    unsigned char *const rows_out = dyn_lds + wv * (32 * TL::ROW_B);
+    auto chunk_at = [&](int row, int c) __attribute__((always_inline)) {
+        return row * TL::ROW_B + ((c ^ (D == 64 ? (row >> 1) & 7 : row & 15)) << 4);
+    };
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {                   // (chunks 4 dt + 2 i + h, as in store_c_tile)
+            f32x16 &a = oacc[dt];
+            if (AGPR && i == 0) ::settle(a);
+            const uint32_t a0 = pack2bf(a[8 * i] * inv, a[8 * i + 1] * inv), a1 = pack2bf(a[8 * i + 2] * inv, a[8 * i + 3] * inv);
+            const uint32_t b0 = pack2bf(a[8 * i + 4] * inv, a[8 * i + 5] * inv), b1 = pack2bf(a[8 * i + 6] * inv, a[8 * i + 7] * inv);
+            const auto x0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
+            const auto x1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+            *reinterpret_cast<u32x4 *>(rows_out + chunk_at(j_, 4 * dt + 2 * i + h_)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
+        }
+    // (all of them read in front of the first store: a read and its store in turn would wait for the LDS each time)
+    u32x4 x[TL::LOADS];
+    const int c = lane_ % TL::CPR;
+#pragma unroll
+    for (int i = 0; i < TL::LOADS; ++i) {
+        x[i] = *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(i * TL::LOAD_ROWS + lane_ / TL::CPR, CARRIED ? c & 15 : c));
+        if (CARRIED && c >= 24) x[i] = u32x4{0u, 0u, 0u, 0u};             // (V's third part is its first one, the last one zeros)
+    }
+    const WaveRows<TL> wr(gshift, lane_);
+    const int q0 = qc0 + ((wv * 32) >> gshift), tok_b = Hq * d_real * 2, place = wr.place(tok_b, d_real * 2) + c * 16;
+    unsigned char *const to = reinterpret_cast<unsigned char *>(out + ((int64_t)(s0 + q0) * Hq + kvh * G) * d_real);
+#pragma unroll
+    for (int i = 0; i < TL::LOADS; ++i)
+        if (q0 + wr.query(i) < L && wr.head(i) < G && (CARRIED || c < chunks)) *reinterpret_cast<u32x4 *>(to + (place + wr.piece(i, tok_b, d_real * 2))) = x[i];
 }
 
 template <int D, bool HAS_IDX, bool CARRIED = false>
@@ -377,29 +451,38 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
-// without a bitmap only); window: rows of a bitmap at positions below it attend all of their causal window (0: nothing is known); carried: see DSA_CARRIED_KS; st: token and head stride of q, k and v in elements (rows of 16-byte alignment)
-extern "C" hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                          int pos_split, int split_len, int window, int carried, int causal, void *out, float *lse, hipStream_t stream) {
-    int gs = 0;
-    while ((1 << gs) < Hq / Hkv) ++gs;
-    scale = logit_scale(scale);
-    hipError_t e = hipErrorInvalidValue;
-#define FWD_CASE(D_, ...) e = launch_fwd_i<D_, __VA_ARGS__>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, out, lse)
+// without a bitmap only); window: rows of a bitmap at positions below it attend all of their causal window (0: nothing is known); carried: see
+// DSA_CARRIED_KS; st: token and head stride of q, k and v in elements (rows of 16-byte alignment).  The file is compiled twice, the second time
+// (FWD_256) for head_dim 256, with results of MFMA builtins in vector registers: the sums have the accumulation registers.
+#define FWD_LAUNCH_ARGS const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, \
+    int Hq, int Hkv, int d_real, float scale, int pos_split, int split_len, int window, int carried, int causal, void *out, float *lse, hipStream_t stream
+#define FWD_CASE(D_, ...) e = launch_fwd_i<D_, __VA_ARGS__>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, group_shift(Hq, Hkv), d_real, logit_scale(scale), \
+                                                            pos_split, split_len, window, causal, out, lse)
+extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS);
+#if FWD_256
+extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS) {
+    hipError_t e;
     if (carried) {
         if (bitmap) FWD_CASE(256, true, true);
         else FWD_CASE(256, false, true);
-    } else if (bitmap) {
+    } else if (bitmap) FWD_CASE(256, true);
+    else FWD_CASE(256, false);
+    return e != hipSuccess ? e : hipGetLastError();
+}
+#else
+extern "C" hipError_t dsa_launch_tile_fwd(FWD_LAUNCH_ARGS) {
+    if (d_real > 256) return hipErrorInvalidValue;
+    if (d_real > 128) return dsa_launch_tile_fwd_256(q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, split_len, window, carried, causal, out, lse, stream);
+    hipError_t e;
+    if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
-        else if (d_real <= 128) FWD_CASE(128, true);
-        else if (d_real <= 256) FWD_CASE(256, true);
+        else FWD_CASE(128, true);
     } else {
         if (d_real <= 64) FWD_CASE(64, false);
         else if (d_real <= 80) FWD_CASE(80, false);
         else if (d_real <= 96) FWD_CASE(96, false);
-        else if (d_real <= 128) FWD_CASE(128, false);
-        else if (d_real <= 256) FWD_CASE(256, false);
+        else FWD_CASE(128, false);
     }
-#undef FWD_CASE
     return e != hipSuccess ? e : hipGetLastError();
 }
+#endif

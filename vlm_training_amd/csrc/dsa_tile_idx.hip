@@ -170,7 +170,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void dsa_tile_idxq_kernel
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j = lane & 31;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(true, cu, N, blockIdx.x, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(true, gridDim.x, cu, N, blockIdx.x, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = min(__builtin_amdgcn_readfirstlane(L), ldw * 32);
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = Hq / Hkv, kvh = blockIdx.x % Hkv;
     int s0, L, blk;
-    if (!LOCATE_QUERY_BLOCK(true, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
+    if (!LOCATE_QUERY_BLOCK(true, gridDim.x, cu, N, blockIdx.x / Hkv, QBW, s0, L, blk)) return;
     s0 = __builtin_amdgcn_readfirstlane(s0);
     L = __builtin_amdgcn_readfirstlane(L);
     L = min(L, ldw * 32);                               // a bitmap row has ldw words whatever the caller's max_seqlen
