@@ -84,13 +84,36 @@ __device__ __forceinline__ void dq_block(int block, int blocks,
             asm volatile("" : "+s"(wptr));
         }
     };
+    auto request_first = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
-        load_tile(kptr, u, u * TL::BYTES);
-        if (u < 2) {
-            load_tile(vptr, u, K_END + u * TL::BYTES);
-            load_w(u);
+        for (int u = 0; u < 3; ++u) {
+            load_tile(kptr, u, u * TL::BYTES);
+            if (u < 2) {
+                load_tile(vptr, u, K_END + u * TL::BYTES);
+                load_w(u);
+            }
         }
+    };
+    // One row group: the wave's rows of q and dO come in whole rows through the rings' eight slots, in front of the tiles (read where they lie, each
+    // load would touch 32 rows: 8000 clocks of a block at head_dim 256); not where they are off 16-byte addresses
+    TL tl;
+    tl.init(lane);
+    static_assert(DQ_RK + DQ_RV == 2 * NW, "");
+    const bool staged = RG == 1 && !(((uintptr_t)q | (uintptr_t)dout) & 15) && (int64_t)Hq * dr < (1 << 24);
+    if (staged) {
+        const WaveRows<TL> wr(gshift, lane);
+        const int row_b = dr * 2, q_b = Hq * row_b, there = L - (qc0 + (r0 >> gshift)), place = wr.place(q_b, row_b);
+        const int64_t base = ((int64_t)(s0 + wq0) * Hq + kvh * G) * dr;
+        const buffer_rsrc q_rows = make_buffer_rsrc(q + base, 0x7fffffff), do_rows = make_buffer_rsrc(dout + base, 0x7fffffff);
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i) {
+            const int c = (lane % TL::CPR) ^ TL::xor_of(i * TL::LOAD_ROWS + lane / TL::CPR);
+            const int off[1] = {wr.query(i) < there && wr.head(i) < G && c < chunks ? place + wr.piece(i, q_b, row_b) + c * 16 : (int)0x80000000};
+            buffer_load_lds16_n<1, 0, 0, 0>(q_rows, off, lds0 + wv * TL::BYTES + TL::load_lds(i));
+            buffer_load_lds16_n<1, 0, 0, 0>(do_rows, off, lds0 + (NW + wv) * TL::BYTES + TL::load_lds(i));
+        }
+    } else {
+        request_first();
     }
     // rows of the wave: (query, head of the group), RG groups of 32; a lane holds row j of each group, half h of every 16 elements
     bf16x8 qB[RG][KS], doB[RG][KS];
@@ -106,12 +129,25 @@ __device__ __forceinline__ void dq_block(int block, int blocks,
         const int t = s0 + min(qcol, L - 1), hq = kvh * G + min(head, G - 1);
         klim[g] = row_ok ? (causal ? qcol : L - 1) : -1;
         row_mask[g] = row_ok ? 0xffffffffu : 0u;
+        if (staged) {
+            wait_vmcnt<0>();                             // (the wave's own pieces)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
-            const bool there = row_ok && (HAS_IDX || 2 * ks + h < chunks);
-            qB[g][ks] = there ? load_bf16x8(q + off) : zero_bf16x8();
-            doB[g][ks] = there ? load_bf16x8(dout + off) : zero_bf16x8();
+            for (int ks = 0; ks < KS; ++ks) {
+                lds_u8 *const at = (lds_u8 *)dyn_lds + wv * TL::BYTES + tl.rowq[TL::row_q(ks)] + TL::row_imm(ks);
+                qB[g][ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(at);
+                doB[g][ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(at + NW * TL::BYTES);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+            barrier_only();                              // every wave has its rows: the slots may be filled
+            request_first();
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const int64_t off = ((int64_t)t * Hq + hq) * dr + 16 * ks + 8 * h;
+                const bool there = row_ok && (HAS_IDX || 2 * ks + h < chunks);
+                qB[g][ks] = there ? load_bf16x8(q + off) : zero_bf16x8();
+                doB[g][ks] = there ? load_bf16x8(dout + off) : zero_bf16x8();
+            }
         }
         neg_lse2[g] = -lse[(int64_t)hq * T + t] * LOG2E_F;
         // delta = rowsum(dO * O) of the lane's row: read, or - when every query row of the launch belongs to this kernel -
@@ -153,8 +189,6 @@ __device__ __forceinline__ void dq_block(int block, int blocks,
     }
     lds_u8 *aR[4], *aT[4];                               // operand addresses: row-wise of K(0), transposed of K(t)
     {
-        TL tl;
-        tl.init(lane);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             aR[i] = (lds_u8 *)dyn_lds + tl.rowq[i];
