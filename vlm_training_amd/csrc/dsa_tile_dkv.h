@@ -149,6 +149,46 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
             asm volatile("" : "+v"(wp));
         }
     };
+    bf16x8 kB[KG][KS], vB[KG][KS];
+    TL tl;
+    tl.init(lane);
+    // The wave's rows of k and v (past the segment its last one) come in whole rows through eight slots of the ring, in front of the blocks (as q
+    // and dO in dQ)
+    if constexpr (!UNALIGNED) {
+        const int first = min(kc, L - 1), kv_b = Hkv * dr * 2;
+        const int64_t base = ((int64_t)(s0 + first) * Hkv + kvh) * dr;
+        const buffer_rsrc k_rows = make_buffer_rsrc(k + base, 0x7fffffff), v_rows = make_buffer_rsrc(v + base, 0x7fffffff);
+#pragma unroll
+        for (int g = 0; g < KG; ++g)
+#pragma unroll
+            for (int i = 0; i < TL::LOADS; ++i) {
+                const int row = i * TL::LOAD_ROWS + lane / TL::CPR, c = (lane % TL::CPR) ^ TL::xor_of(row);
+                const int off[1] = {c < chunks ? (min(kc + 32 * g + row, L - 1) - first) * kv_b + c * 16 : (int)0x80000000};
+                buffer_load_lds16_n<1, 0, 0, 0>(k_rows, off, lds0 + (wv * KG + g) * TL::BYTES + TL::load_lds(i));
+                buffer_load_lds16_n<1, 0, 0, 0>(v_rows, off, lds0 + (4 + wv * KG + g) * TL::BYTES + TL::load_lds(i));
+            }
+        wait_vmcnt<0>();                                 // (the wave's own pieces)
+#pragma unroll
+        for (int g = 0; g < KG; ++g)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                lds_u8 *const at = (lds_u8 *)dyn_lds + (wv * KG + g) * TL::BYTES + tl.rowq[TL::row_q(ks)] + TL::row_imm(ks);
+                kB[g][ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(at);
+                vB[g][ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>(at + 4 * TL::BYTES);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        barrier_only();                                  // every wave has its rows: the slots may be filled
+    } else {
+#pragma unroll
+        for (int g = 0; g < KG; ++g)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const int64_t at = ((int64_t)(s0 + min(kc + 32 * g + j, L - 1)) * Hkv + kvh) * dr + 16 * ks + 8 * h;
+                const bool there = HAS_IDX || 2 * ks + h < chunks;
+                kB[g][ks] = there ? load_bf16x8(k + at) : zero_bf16x8();
+                vB[g][ks] = there ? load_bf16x8(v + at) : zero_bf16x8();
+            }
+    }
     load_rows(0);
     load_words(0);
     if (last > 0) {                                      // leaving block 0: undo its clamps
@@ -163,21 +203,12 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
         load_words(b + 1);
     }
     unsigned char *const klast = aux + RING * 512 + 1536 + lane * 16, *const vlast = klast + 2048;
-    bf16x8 kB[KG][KS], vB[KG][KS];
 #pragma unroll
-    for (int g = 0; g < KG; ++g) {
-        const int64_t krow = (int64_t)(s0 + min(kc + 32 * g + j, L - 1)) * Hkv + kvh;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bool there = HAS_IDX || 2 * ks + h < chunks;
-            kB[g][ks] = there ? load_bf16x8(k + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
-            vB[g][ks] = there ? load_bf16x8(v + krow * dr + 16 * ks + 8 * h) : zero_bf16x8();
-        }
+    for (int g = 0; g < KG; ++g)
         if (TIGHT) {
             *reinterpret_cast<bf16x8 *>(klast + g * 1024) = kB[g][KS - 1];
             *reinterpret_cast<bf16x8 *>(vlast + g * 1024) = vB[g][KS - 1];
         }
-    }
     f32x16 dkacc[KG][DT], dvacc[KG][DT];
 #pragma unroll
     for (int g = 0; g < KG; ++g)
@@ -224,8 +255,6 @@ __global__ __launch_bounds__(256 / KG, 1) void dsa_tile_dkv_kernel(
     bf16x8 op[AHEAD];
     lds_u8 *aR[4], *aT[4];                               // operand addresses: row-wise of block s+1, transposed of block s
     {
-        TL tl;
-        tl.init(lane);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             aR[i] = (lds_u8 *)dyn_lds + tl.rowq[i];
