@@ -40,7 +40,10 @@ constexpr size_t fwd_lds_bytes(bool has_idx) { return 8 * (size_t)DirectTile<D>:
 // NEG: the softmax scale is negative.  A masked key's logit is -inf in front of the scale, and the largest one is searched for there, so
 // the kernel's scale is positive and the sign goes into q (an instance of its own: at head_dim 256 as little as a test of the sign in front
 // of the loop made it spill).
-template <int D, bool HAS_IDX, int NW, bool NEG, bool CARRIED>
+// AGPR: the sums in accumulation registers, by name (mfma32_agpr_late).  ROUNDS: more than one round of workgroups; a launch of one reads q
+// where it lies, beside the tiles, and stores the output so: each way through LDS is one more latency of the block, and nothing else uses the
+// path to memory (197 tokens 8.8 against 9.2 us; from two rounds on 1.5 to 5 % less with them).
+template <int D, bool HAS_IDX, int NW, bool NEG, bool CARRIED, bool AGPR, bool ROUNDS>
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
@@ -50,7 +53,6 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     // MFMAs of S, of P V (head_dim 80: five and six) and pairs of a step (one of each while there are)
     constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT, NS = KS > NP ? KS : NP;
     static_assert(KS <= NP || D > 128);
-    constexpr bool AGPR = D > 128;                          // the sums in accumulation registers, by name (mfma32_agpr_late)
     constexpr int LPW = (TL::LOADS + NW - 1) / NW;          // wave loads per wave, step and operand
     constexpr int LPS = 2 * LPW + (HAS_IDX ? 1 : 0);        // everything a wave requests in a step
     static_assert(TL::LOADS % NW == 0, "every wave loads the same number of pieces");
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     bf16x8 qB[KS];
     TL tl;
     tl.init(lane);
-    const bool staged = !((reinterpret_cast<uintptr_t>(q) | (uintptr_t)(q_tok * 2) | (uintptr_t)(q_head * 2)) & 15) &&
+    const bool staged = ROUNDS && !((reinterpret_cast<uintptr_t>(q) | (uintptr_t)(q_tok * 2) | (uintptr_t)(q_head * 2)) & 15) &&
                         31 * q_tok + (int64_t)(G - 1) * q_head < (1 << 30) - D;
     if (staged) {
         const buffer_rsrc rows = make_buffer_rsrc(q + (int64_t)(s0 + wq0) * q_tok + (int64_t)kvh * G * q_head, 0x7fffffff);
@@ -136,17 +138,23 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
             buffer_load_lds16_n<1, 0, 0, 0>(rows, off, lds0 + (4 + wv) * TL::BYTES + TL::load_lds(i));
         }
     }
-    load_k(0); load_w(0); load_k(1); load_w(1); load_k(2); load_w(2); load_k(3); load_w(3);
+    if (!staged) {
+        const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
+    }
+    load_k(0); load_w(0); load_k(1); load_w(1);
+    if (!staged) load_v(0);
+    load_k(2); load_w(2);
+    if (!staged) load_v(1);
+    load_k(3); load_w(3);
+    if (!staged) load_v(2);
     constexpr int AFTER_K1 = 2 * LPW + (HAS_IDX ? 2 : 0);
     if (staged) {
         wait_vmcnt<AFTER_K1>();
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             qB[ks] = *reinterpret_cast<__attribute__((address_space(3))) const bf16x8 *>((lds_u8 *)dyn_lds + (4 + wv) * TL::BYTES + tl.rowq[TL::row_q(ks)] + TL::row_imm(ks));
-    } else {
-        const bf16_t *const qrow = q + (int64_t)t * q_tok + (int64_t)hq * q_head;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qB[ks] = row_ok && 2 * ks + h < chunks ? load_bf16x8(qrow + 16 * ks + 8 * h) : zero_bf16x8();
     }
     if (NEG) {
 #pragma unroll
@@ -164,9 +172,12 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
         barrier_only();
     };
-    wait_vmcnt<AFTER_K1>();                             // K(0) and K(1) are there
+    if (staged) wait_vmcnt<AFTER_K1>();                 // K(0) and K(1) are there
+    else wait_vmcnt<0>();
     meet_read();
-    load_v(0); load_v(1); load_v(2);
+    if (staged) {
+        load_v(0); load_v(1); load_v(2);
+    }
 
     lds_u8 *ka_[4], *va_[4];                            // operand addresses: of the K tile of S(t+2) and of V(t)
 #pragma unroll
@@ -396,56 +407,77 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     const float l = half_sum_f(lsum), inv = 1.f / l;
     // (where the rows lie is formed again: the loop needs its registers)
     int tid_ = tid;
-    asm volatile("" : "+v"(tid_));
+    if (ROUNDS || D > 128) asm volatile("" : "+v"(tid_));
     const int lane_ = tid_ & 63, h_ = lane_ >> 5, j_ = lane_ & 31;
     {
         const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
         if (qc < L && hd < G && h_ == 0) lse[(int64_t)(kvh * G + hd) * T + s0 + qc] = (mrun + log2f(l)) * LN2_F;
     }
-    // whole rows per store, through LDS (as in dQ)
-    barrier_only();                                     // the rings are read out
-    unsigned char *const rows_out = dyn_lds + wv * (32 * TL::ROW_B);
-    auto chunk_at = [&](int row, int c) __attribute__((always_inline)) {
-        return row * TL::ROW_B + ((c ^ (D == 64 ? (row >> 1) & 7 : row & 15)) << 4);
-    };
+    if constexpr (!ROUNDS) {
+        const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
+        if (qc < L && hd < G) {
+            bf16_t *const row = out + ((int64_t)(s0 + qc) * Hq + kvh * G + hd) * d_real;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {                   // (chunks 4 dt + 2 i + h, as in store_c_tile)
-            f32x16 &a = oacc[dt];
-            if (AGPR && i == 0) ::settle(a);
-            const uint32_t a0 = pack2bf(a[8 * i] * inv, a[8 * i + 1] * inv), a1 = pack2bf(a[8 * i + 2] * inv, a[8 * i + 3] * inv);
-            const uint32_t b0 = pack2bf(a[8 * i + 4] * inv, a[8 * i + 5] * inv), b1 = pack2bf(a[8 * i + 6] * inv, a[8 * i + 7] * inv);
-            const auto x0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
-            const auto x1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-            *reinterpret_cast<u32x4 *>(rows_out + chunk_at(j_, 4 * dt + 2 * i + h_)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
+            for (int dt = 0; dt < DT; ++dt) {
+                if (AGPR) ::settle(oacc[dt]);
+                store_c_tile(row + dt * 32, oacc[dt], inv, h_, chunks - 4 * dt);
+            }
+            if (CARRIED) {                              // V's third part is its first one, the last one zeros
+                store_c_tile(row + 128, oacc[0], inv, h_, 4);
+                store_c_tile(row + 160, oacc[1], inv, h_, 4);
+                store_c_tile(row + 192, zero16(), inv, h_, 4);
+                store_c_tile(row + 224, zero16(), inv, h_, 4);
+            }
         }
-    // (all of them read in front of the first store: a read and its store in turn would wait for the LDS each time)
-    u32x4 x[TL::LOADS];
-    const int c = lane_ % TL::CPR;
+    } else {
+        // whole rows per store, through LDS (as in dQ)
+        barrier_only();                                     // the rings are read out
+        unsigned char *const rows_out = dyn_lds + wv * (32 * TL::ROW_B);
+        auto chunk_at = [&](int row, int c) __attribute__((always_inline)) {
+            return row * TL::ROW_B + ((c ^ (D == 64 ? (row >> 1) & 7 : row & 15)) << 4);
+        };
 #pragma unroll
-    for (int i = 0; i < TL::LOADS; ++i) {
-        x[i] = *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(i * TL::LOAD_ROWS + lane_ / TL::CPR, CARRIED ? c & 15 : c));
-        if (CARRIED && c >= 24) x[i] = u32x4{0u, 0u, 0u, 0u};             // (V's third part is its first one, the last one zeros)
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {                   // (chunks 4 dt + 2 i + h, as in store_c_tile)
+                f32x16 &a = oacc[dt];
+                if (AGPR && i == 0) ::settle(a);
+                const uint32_t a0 = pack2bf(a[8 * i] * inv, a[8 * i + 1] * inv), a1 = pack2bf(a[8 * i + 2] * inv, a[8 * i + 3] * inv);
+                const uint32_t b0 = pack2bf(a[8 * i + 4] * inv, a[8 * i + 5] * inv), b1 = pack2bf(a[8 * i + 6] * inv, a[8 * i + 7] * inv);
+                const auto x0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
+                const auto x1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+                *reinterpret_cast<u32x4 *>(rows_out + chunk_at(j_, 4 * dt + 2 * i + h_)) = u32x4{x0[0], x1[0], x0[1], x1[1]};
+            }
+        // (all of them read in front of the first store: a read and its store in turn would wait for the LDS each time)
+        u32x4 x[TL::LOADS];
+        const int c = lane_ % TL::CPR;
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i) {
+            x[i] = *reinterpret_cast<const u32x4 *>(rows_out + chunk_at(i * TL::LOAD_ROWS + lane_ / TL::CPR, CARRIED ? c & 15 : c));
+            if (CARRIED && c >= 24) x[i] = u32x4{0u, 0u, 0u, 0u};             // (V's third part is its first one, the last one zeros)
+        }
+        const WaveRows<TL> wr(gshift, lane_);
+        const int q0 = qc0 + ((wv * 32) >> gshift), tok_b = Hq * d_real * 2, place = wr.place(tok_b, d_real * 2) + c * 16;
+        unsigned char *const to = reinterpret_cast<unsigned char *>(out + ((int64_t)(s0 + q0) * Hq + kvh * G) * d_real);
+#pragma unroll
+        for (int i = 0; i < TL::LOADS; ++i)
+            if (q0 + wr.query(i) < L && wr.head(i) < G && (CARRIED || c < chunks)) *reinterpret_cast<u32x4 *>(to + (place + wr.piece(i, tok_b, d_real * 2))) = x[i];
     }
-    const WaveRows<TL> wr(gshift, lane_);
-    const int q0 = qc0 + ((wv * 32) >> gshift), tok_b = Hq * d_real * 2, place = wr.place(tok_b, d_real * 2) + c * 16;
-    unsigned char *const to = reinterpret_cast<unsigned char *>(out + ((int64_t)(s0 + q0) * Hq + kvh * G) * d_real);
-#pragma unroll
-    for (int i = 0; i < TL::LOADS; ++i)
-        if (q0 + wr.query(i) < L && wr.head(i) < G && (CARRIED || c < chunks)) *reinterpret_cast<u32x4 *>(to + (place + wr.piece(i, tok_b, d_real * 2))) = x[i];
 }
 
-template <int D, bool HAS_IDX, bool CARRIED = false>
+template <int D, bool HAS_IDX, bool CARRIED = false, bool AGPR = (D > 128)>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int window, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
-    const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true, CARRIED> : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false, CARRIED>;
+    const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
+    const bool rounds = grid.x > (D > 128 ? 256 : 512);     // (one or two workgroups per CU)
+    const auto kernel = scale < 0.f ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, true, CARRIED, AGPR, true>
+                        : rounds    ? &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false, CARRIED, AGPR, true>
+                                    : &dsa_tile_fwd_kernel<D, HAS_IDX, NW, false, CARRIED, AGPR, false>;
     constexpr size_t lds = fwd_lds_bytes<D, NW>(HAS_IDX);
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
                        st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, window, causal, (bf16_t *)out, lse);
     return hipSuccess;
@@ -466,13 +498,13 @@ extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS) {
         if (bitmap) FWD_CASE(256, true, true);
         else FWD_CASE(256, false, true);
     } else if (bitmap) FWD_CASE(256, true);
-    else FWD_CASE(256, false);
+    else FWD_CASE(256, false);                           // (of a negative scale)
     return e != hipSuccess ? e : hipGetLastError();
 }
 #else
 extern "C" hipError_t dsa_launch_tile_fwd(FWD_LAUNCH_ARGS) {
     if (d_real > 256) return hipErrorInvalidValue;
-    if (d_real > 128) return dsa_launch_tile_fwd_256(q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, split_len, window, carried, causal, out, lse, stream);
+    if (d_real > 128 && (bitmap || carried || scale < 0.f)) return dsa_launch_tile_fwd_256(q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, split_len, window, carried, causal, out, lse, stream);
     hipError_t e;
     if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
@@ -481,7 +513,8 @@ extern "C" hipError_t dsa_launch_tile_fwd(FWD_LAUNCH_ARGS) {
         if (d_real <= 64) FWD_CASE(64, false);
         else if (d_real <= 80) FWD_CASE(80, false);
         else if (d_real <= 96) FWD_CASE(96, false);
-        else FWD_CASE(128, false);
+        else if (d_real <= 128) FWD_CASE(128, false);
+        else FWD_CASE(256, false, false, false);         // (without a mask in its loop it spills nothing there, and takes 2 to 4 % less)
     }
     return e != hipSuccess ? e : hipGetLastError();
 }

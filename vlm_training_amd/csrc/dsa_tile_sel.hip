@@ -11,7 +11,7 @@
 // past L2 at 131 072 tokens).
 //
 // What bounds it: the LDS (operand rows of a list lie where they lie: 1.9 instead of 1.0 clocks a read; busy 0.58 of the time), the vector
-// instructions (about 125 a step, 45 more a block for the list) and the spread of the waves' steps between two barriers.  Rows beyond
+// instructions (about 100 a step, 45 more a block for the list) and the spread of the waves' steps between two barriers.  Rows beyond
 // 16 K of 131 072 tokens, K = 2048, 32 heads over 8 kv heads, the whole forward / backward, ms: gathered 94.5 / 299; here with eight waves and a step's
 // chain of reads and MFMAs open to its latency 76 / 297, twelve waves, lists built a block ahead 65 / 293, operands read ahead and nothing spilled
 // 56 / 280, exponentials behind the MFMAs of dP 57 / 275.  With twelve waves a spilled register read in the loop waits for the blocks on their way into LDS (+ 25 %).

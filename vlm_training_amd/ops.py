@@ -254,7 +254,8 @@ def indexer_kl_loss(indexer_q, indexer_k, indexer_w, mass, cu_seqlens, max_seqle
 
 
 def set_tile_crossover(crossover: int) -> int:
-    """Rows with pos < top_k * crossover use the MFMA tile kernels, later rows the gather kernels.
+    """Rows with pos < top_k * crossover use the MFMA tile kernels, later rows the gather kernels; at the default (24) long
+    segments at head_dim 128 with two to four heads per kv head have compacted walks between the two, and on the key side.
     Returns the previous value (tests use it to drive each path on its own)."""
     lib = _lib.load()
     old = lib.dsa_get_tile_crossover()
@@ -264,8 +265,8 @@ def set_tile_crossover(crossover: int) -> int:
 
 def set_bwd_overlap(mode: int) -> int:
     """0: the backward's passes run one after the other on the caller's stream; 1 (default): launches of few
-    workgroups run dQ beside dK/dV on a second stream of the library's own; 2: every launch does.  Same bits in every
-    mode.  Returns the previous mode."""
+    workgroups run dQ beside dK/dV on a second stream of the library's own, and at head_dim 256 one launch holds both; 2: every
+    launch runs them side by side.  Same bits in every mode.  Returns the previous mode."""
     lib = _lib.load()
     old = lib.dsa_get_bwd_overlap()
     _lib.check(lib.dsa_set_bwd_overlap(int(mode)), "dsa_set_bwd_overlap")

@@ -53,10 +53,10 @@ class Workload:
         return P, S
 
     def executed_pairs(self, crossover: int = 24) -> Tuple[int, int]:
-        """(query side, key side): the (query, key) pairs the tile kernels put through the matrix cores.  They walk
-        whole tiles with the selection as a mask, so every causal pair of a visited tile is computed: on the query side
-        (forward, dQ) the causal pairs of the rows below the tile/gather split (positions < top_k * crossover, rounded up
-        to 256), on the key side (dK/dV) every causal pair."""
+        """(query side, key side): the (query, key) pairs a walk of whole tiles with the selection as a mask puts through
+        the matrix cores: on the query side (forward, dQ) the causal pairs of the rows at positions < top_k * crossover
+        (rounded up to 256), on the key side (dK/dV) every causal pair.  Long segments with thin selections run fewer: their
+        late rows, and the key side from 26 * top_k tokens on, are compacted walks or gathers."""
         split = (self.top_k * crossover + 255) // 256 * 256
         q_side = sum(min(L, split) * (min(L, split) + 1) // 2 for L in self.seg_lens)
         return q_side, self.pair_counts()[0]
