@@ -405,31 +405,31 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     wait_vmcnt<0>();                                    // no load is left on its way into LDS when the workgroup ends
 
     const float l = half_sum_f(lsum), inv = 1.f / l;
-    // (where the rows lie is formed again: the loop needs its registers)
-    int tid_ = tid;
-    if (ROUNDS || D > 128) asm volatile("" : "+v"(tid_));
-    const int lane_ = tid_ & 63, h_ = lane_ >> 5, j_ = lane_ & 31;
-    {
-        const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
-        if (qc < L && hd < G && h_ == 0) lse[(int64_t)(kvh * G + hd) * T + s0 + qc] = (mrun + log2f(l)) * LN2_F;
-    }
     if constexpr (!ROUNDS) {
-        const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
-        if (qc < L && hd < G) {
-            bf16_t *const row = out + ((int64_t)(s0 + qc) * Hq + kvh * G + hd) * d_real;
+        if (row_ok) {
+            if (h == 0) lse[(int64_t)hq * T + t] = (mrun + log2f(l)) * LN2_F;
+            bf16_t *const row = out + ((int64_t)t * Hq + hq) * d_real;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 if (AGPR) ::settle(oacc[dt]);
-                store_c_tile(row + dt * 32, oacc[dt], inv, h_, chunks - 4 * dt);
+                store_c_tile(row + dt * 32, oacc[dt], inv, h, chunks - 4 * dt);
             }
             if (CARRIED) {                              // V's third part is its first one, the last one zeros
-                store_c_tile(row + 128, oacc[0], inv, h_, 4);
-                store_c_tile(row + 160, oacc[1], inv, h_, 4);
-                store_c_tile(row + 192, zero16(), inv, h_, 4);
-                store_c_tile(row + 224, zero16(), inv, h_, 4);
+                store_c_tile(row + 128, oacc[0], inv, h, 4);
+                store_c_tile(row + 160, oacc[1], inv, h, 4);
+                store_c_tile(row + 192, zero16(), inv, h, 4);
+                store_c_tile(row + 224, zero16(), inv, h, 4);
             }
         }
     } else {
+        // (where the rows lie is formed again: the loop needs its registers)
+        int tid_ = tid;
+        asm volatile("" : "+v"(tid_));
+        const int lane_ = tid_ & 63, h_ = lane_ >> 5, j_ = lane_ & 31;
+        {
+            const int qc = qc0 + ((wv * 32 + j_) >> gshift), hd = j_ & ((1 << gshift) - 1);
+            if (qc < L && hd < G && h_ == 0) lse[(int64_t)(kvh * G + hd) * T + s0 + qc] = (mrun + log2f(l)) * LN2_F;
+        }
         // whole rows per store, through LDS (as in dQ)
         barrier_only();                                     // the rings are read out
         unsigned char *const rows_out = dyn_lds + wv * (32 * TL::ROW_B);
