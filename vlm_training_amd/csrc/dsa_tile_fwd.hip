@@ -265,7 +265,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
         for (int i = 0; i < 8; ++i) pE[i] = 0u;
         settle(sE, live(word_of(0)), pE, psum);
     }
-    wait_vmcnt<2 * LPW>();                              // all but V(1) and V(2)
+    wait_vmcnt<LPW>();                                  // all but V(2): step 0 reads its first operands of V(1) itself
     meet_read();                                        // every wave is done with K(0) and K(1): their slots may be filled again
     load_k(4);
     constexpr int KA = KS % 5 == 0 ? 5 : KS % 4 ? 3 : 4, VA = NP % 4 ? 3 : 4;   // (divide KS and NP: an operand keeps its register from step to step)
