@@ -21,5 +21,9 @@ struct SelBlock {
     static constexpr int COLUMN_B = 256;
     __device__ __forceinline__ static int entry(int r) { return (r >> 2) * 1024 + (r & 3) * 64 + mix(r >> 2 & 3) * 16; }
 };
-template <class T> __device__ __forceinline__ T lds_read(uint32_t at) { return *(__attribute__((address_space(3))) const T *)at; }
+// (may_alias: a list's entries are written as words and read by halves)
+template <class T> __device__ __forceinline__ T lds_read(uint32_t at) {
+    typedef T __attribute__((may_alias)) any;
+    return *(__attribute__((address_space(3))) const any *)at;
+}
 
