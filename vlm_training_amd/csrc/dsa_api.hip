@@ -44,7 +44,6 @@ size_t dsa_indexer_bwd_partial_bytes(int T, int Di, int ldw);
 hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, const uint32_t *bitmap, int ldw,
                                 const int32_t *n, const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K,
                                 float scale, float *partial, float *mass, hipStream_t stream);
-struct DqBeside { int window; void *dq; };                // (dQ in the key side's launch)
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
                                int window, int carried, int causal, void *out, float *lse, hipStream_t stream);

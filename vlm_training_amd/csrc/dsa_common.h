@@ -34,6 +34,8 @@ static inline int dkv_key_groups(int D, int T, int N, int Hq, int Hkv, int causa
     const int64_t wg = ((int64_t)T / 128 + N) * Hkv;
     return wg < 96 || (wg <= dkv_pieces_max_wg(D) && wg * T / N * rows <= 40000 * 32) ? 1 : 2;
 }
+// dQ in the key side's launch, where one holds both passes (dsa_tile_bwd.hip)
+struct DqBeside { int window; void *dq; };
 #define LOG2E_F 1.4426950408889634f
 #define LN2_F 0.6931471805599453f
 

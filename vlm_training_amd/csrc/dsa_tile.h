@@ -260,8 +260,6 @@ struct PhaseOrder {
 };
 
 // ---- walks of key tiles (dK, dV) ----
-// the query side, where one launch holds both passes (dsa_tile_bwd.hip)
-struct DqBeside { int window; void *dq; };
 #define DSA_ORDER_MAX_SEGS 4096
 // the tile (and the piece of its walk) of workgroup slot `slot`: from the order table when there is one, else
 // segment by segment
