@@ -217,8 +217,10 @@ int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const float *lse, c
  * Tuning knob (process-wide, no reference counterpart): query rows whose position in their segment is
  * below top_k * crossover run on the dense MFMA tile kernels with the selection as a bitmap mask, the
  * rest on the gather kernels.  0 = gather only; INT_MAX/top_k or more = tiles only.  At the default, 24, head_dim 128 with two
- * to four heads per kv head splits otherwise: segments of 18 * top_k tokens and more run their rows from position 16 * top_k on in
- * the compacted walk of dsa_tile_sel.hip (up to 75 * top_k, 150 with two heads, the rest gathered), shorter ones on the tile kernels.
+ * to four heads per kv head splits otherwise: segments of 18 * top_k tokens and more (26 with two heads) that have rows enough for a launch of
+ * its own, by themselves or with the others of a batch of long ones, run their rows from position 16 * top_k on in the compacted walk of
+ * dsa_tile_sel.hip (up to 75 * top_k, 150 with two heads, the rest gathered); elsewhere the tile kernels go on to 75 * top_k with two heads.
+ * A row's low bits depend on the kernel that takes it.
  * idx == NULL (dense causal attention) always uses the tile kernels.
  */
 int dsa_set_tile_crossover(int crossover);

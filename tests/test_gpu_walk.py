@@ -26,21 +26,25 @@ def _reference(q, k, v, dout, sel, scale):
 
 
 @pytest.mark.parametrize("Hq,Hkv,lens,K,kind,scale", [
-    (4, 1, (641, 256, 257, 97), 8, "random", None),      # tiles to 256, walk to 768: rows on either side of a block of 96 queries
-    (8, 2, (1000,), 8, "random", None),                  # and the gather beyond 768
-    (4, 2, (1400, 300), 8, "random", None),              # two heads per kv head: the gather from 1280 on
-    (3, 1, (700,), 16, "random", -0.1),                  # a group of three, a negative scale
-    (8, 2, (897, 705), 40, "runs", None),                # every key of a block wanted by some query: four steps
-    (4, 1, (769,), 8, "classes", None),                  # keys 16 apart: one class of the block's rows
-    (6, 2, (640,), 12, "empty", None)])                  # queries that select nothing
+    # (heads enough for the walk to take segments from 350 tokens on, or from 150 where the segments of a batch are as long on average)
+    (288, 72, (641, 256, 257, 97), 8, "random", None),   # tiles to 256, walk to 768: rows on either side of a block of 96 queries
+    (296, 74, (1000, 334, 333) + (21,) * 20, 8, "random", None),      # and the gather beyond 768; segments on either side of the walk's line
+    (440, 220, (1400, 300), 8, "random", None),          # two heads per kv head: the gather from 1280 on
+    (288, 96, (700,), 16, "random", -0.1),               # a group of three, a negative scale
+    (296, 74, (1025, 705), 40, "runs", None),             # every key of a block wanted by some query: four steps
+    (288, 72, (769,), 8, "classes", None),               # keys 16 apart: one class of the block's rows
+    (288, 96, (640,), 12, "empty", None)])               # queries that select nothing
 def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
     print("compacted walk", Hq, Hkv, lens, K, kind, flush=True)
-    assert _lib.load().dsa_get_tile_crossover() == 24
+    lib, G = _lib.load(), Hq // Hkv
+    first = 16 * K + (100000 // Hq if G == 2 else 15250 // Hkv)         # the shortest segment that walks
+    assert lib.dsa_get_tile_crossover() == 24 and max(lens) >= max(first, (26 if G == 2 else 18) * K)
     g = torch.Generator().manual_seed(Hq * K + len(lens))
     T, cu = sum(lens), [0]
     for n in lens:
         cu.append(cu[-1] + n)
-    q, k, v, dout = (torch.randn(T, h, D, generator=g).mul_(0.5).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    gd = torch.Generator(device=DEV).manual_seed(Hq * K + len(lens))
+    q, k, v, dout = (torch.randn(T, h, D, generator=gd, device=DEV).mul_(0.5).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
     idx, n = torch.full((T, K), -1, dtype=torch.int32), torch.zeros(T, dtype=torch.int32)
     sel = torch.zeros(T, T, dtype=torch.bool)
     for a, b in zip(cu[:-1], cu[1:]):
@@ -59,23 +63,27 @@ def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
             idx[t, :len(keys)] = keys.int()
             sel[t, keys] = True
     scale = D ** -0.5 if scale is None else scale
-    want = _reference(q, k, v, dout, sel, scale)
-    d = [x.to(DEV) for x in (q, k, v, idx, n, torch.tensor(cu, dtype=torch.int32), dout)]
+    sel = sel.to(DEV)
+    d = [q, k, v] + [x.to(DEV) for x in (idx, n, torch.tensor(cu, dtype=torch.int32))] + [dout]
     out, lse = ops.attn_fwd(*d[:6], max(lens), scale, True)[:2]
     # the backward takes log-sum-exps that are finite, as those of rows with a key are
     dq, dk, dv = ops.attn_bwd(d[6], *d[:3], out, lse.clamp(min=-1e30), *d[3:6], max(lens), scale, causal=True)
     torch.cuda.synchronize()
-    some = n > 0
-    late = torch.cat([torch.arange(m) >= 16 * K + 255 for m in lens])    # (the tile kernels have no result for a row without a key)
-    assert bool((out.cpu()[late & ~some] == 0).all()) and bool((dq.cpu()[late & ~some] == 0).all())
+    some = (n > 0).to(DEV)
+    late = torch.cat([torch.arange(m) >= 16 * K + 255 for m in lens]).to(DEV)      # (the tile kernels have no result for a row without a key)
+    if kind == "empty":
+        assert bool((out[late & ~some] == 0).all()) and bool((dq[late & ~some] == 0).all())
     rows = some | late
-    for name, got, ref in (("out", out, want[0]), ("dq", dq, want[2])):
-        assert_close_bf16(got.cpu()[rows], ref[rows], name)
-    got, ref = lse.cpu().T[rows], want[1].T[rows].float()
-    assert torch.equal(got.isinf(), ref.isinf()) and float((got - ref)[~ref.isinf()].abs().max()) < 2e-3   # (bf16 products are exact in fp32)
-    if bool(some.all()):
-        assert_close_bf16(dk, want[3], "dk")
-        assert_close_bf16(dv, want[4], "dv")
+    for h in range(0, Hkv, 23):
+        hs = slice(h * G, (h + 1) * G)
+        want = _reference(q[:, hs], k[:, h:h + 1], v[:, h:h + 1], dout[:, hs], sel, scale)
+        for name, got, ref in (("out", out[:, hs], want[0]), ("dq", dq[:, hs], want[2])):
+            assert_close_bf16(got[rows], ref[rows], f"{name} of kv head {h}")
+        got, ref = lse[hs].T[rows], want[1].T[rows].float()
+        assert torch.equal(got.isinf(), ref.isinf()) and float((got - ref)[~ref.isinf()].abs().max()) < 2e-3   # (bf16 products are exact in fp32)
+        if bool(some.all()):
+            assert_close_bf16(dk[:, h:h + 1], want[3], f"dk of kv head {h}")
+            assert_close_bf16(dv[:, h:h + 1], want[4], f"dv of kv head {h}")
 
 
 @pytest.mark.parametrize("G,lens,kind", [

@@ -19,8 +19,8 @@ hipError_t dsa_launch_indexer(const void *q_idx, const void *k_idx, const void *
                               int Hi, int Di, float scale, int row_begin, int row_end, int skip_dense_k,
                               float *scores, int64_t ld, hipStream_t stream);
 hipError_t dsa_launch_attn_fwd(const void *q, const void *k, const void *v, const int32_t *idx, const int32_t *n,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K, float scale, int pos_min,
-                               void *out, float *lse, hipStream_t stream);
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K, float scale, int pos_min, int split_len,
+                               int pos_short, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_sel_fwd(const void *q, const void *k, const void *v, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
                               int Hq, int Hkv, float scale, int pos_min, int pos_max, int split_len, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_sel_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse, const float *delta,
@@ -34,8 +34,8 @@ hipError_t dsa_launch_bitmap(const int32_t *idx, const int32_t *n, const int32_t
                              uint32_t *bitmap, hipStream_t stream);
 hipError_t dsa_launch_gather_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                 const float *delta, const int32_t *idx, const int32_t *n, const int32_t *cu, int N,
-                                int T, int Hq, int Hkv, int D, int K, float scale, int pos_min, void *dq,
-                                hipStream_t stream);
+                                int T, int Hq, int Hkv, int D, int K, float scale, int pos_min,
+                                int split_len, int pos_short, void *dq, hipStream_t stream);
 hipError_t dsa_launch_indexer_bwd(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *idx, const int32_t *n, const float *dscore, const float *grad,
                                   const uint32_t *bitmap, int32_t *prefix, float *w_f32, int ldw, const int32_t *cu, int N, int T, int Hi,
                                   int Di, int K, float cscale, void *dq_idx, void *dk_idx, void *dw, int dw_bf16, float *partial,
@@ -46,10 +46,11 @@ hipError_t dsa_launch_tile_mass(const void *q, const void *k, const float *lse, 
                                 float scale, float *partial, float *mass, hipStream_t stream);
 hipError_t dsa_launch_tile_fwd(const void *q, const void *k, const void *v, const int64_t *strides, const uint32_t *bitmap, int ldw,
                                const int32_t *cu, int N, int T, int Hq, int Hkv, int D, float scale, int pos_split, int split_len,
-                               int window, int carried, int causal, void *out, float *lse, hipStream_t stream);
+                               int pos_short, int window, int carried, int causal, void *out, float *lse, hipStream_t stream);
 hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
-                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int window, int carried, int causal, void *dq, const void *out_for_delta,
+                              int Hq, int Hkv, int D, float scale, int pos_split, int split_len, int pos_short, int window, int carried, int causal,
+                              void *dq, const void *out_for_delta,
                               float *delta_out, hipStream_t stream);
 hipError_t dsa_launch_tile_dkv(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                                const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T,
@@ -286,37 +287,61 @@ extern "C" int dsa_set_tile_crossover(int crossover) {
 }
 extern "C" int dsa_get_tile_crossover(void) { return g_tile_crossover.load(std::memory_order_relaxed); }
 
-// Positions that the tile kernels (below `tiles`), the compacted walk (dsa_tile_sel.hip: below `walk`) and the gather kernels (the rest) take in
-// segments of at least `len` tokens; multiples of 256, the coarsest block of a tile kernel.  Shorter segments are the tile kernels' whole (a
-// segment's own length decides, so that any upper bound of the longest one gives the same bits).
+// Who takes a query row, by its position and its segment's length (a segment's own, so that any upper bound of the longest one gives the same
+// bits): in segments of at least `len` tokens the tile kernels below `tiles`, the compacted walk (dsa_tile_sel.hip) below `walk`, the gather
+// kernels from there on; in shorter ones the tile kernels below `below`, the gather kernels from there on.  Multiples of 256, the coarsest block of
+// a tile kernel.
 // The compacted walk stands between the other two at head_dim 128 with two to four heads per kv head, unless the crossover was set.  Its rows cost
 // what the 32-key steps of their blocks cost, a gathered row what its K keys do, so that the gather is the better one again once rows are long
 // (K = 128, 32 768 tokens, two kv heads of 4: forward 0.46 ms gathered, 0.88 walked), the sooner the fewer queries a wave holds.  One
 // document, 32 heads over 8 kv heads, K = 2048, gather from 24 K on (tiles up to there) -> walk from 16 K on, forward / backward, ms:
 // 131 072 tokens 94.5 / 299 -> 57.3 / 277, 65 536 30.3 / 86.5 -> 21.1 / 78.0, 49 152 16.7 / 49.9 -> 15.0 / 46.8, 40 000 11.2 / 34.2 -> 11.0 / 33.5,
-// 36 000 9.1 / 27.7 -> 9.8 / 27.3, 33 000 7.7 / 22.5 -> 8.9 / 23.7 (few long walks behind the tiles' launch): from segments of 18 K on.  With 8
-// and 16 heads per kv head (32 768 tokens, two kv heads, K = 512) the gather is the faster one from 16 K on: forward 1.45 and 1.71 ms
-// against 1.84 and 3.29; at head_dim 64 with 4 heads too, 0.59 against 0.81.
+// 36 000 9.1 / 27.7 -> 9.8 / 27.3, 33 000 7.7 / 22.5 -> 8.9 / 23.7.  With 8 and 16 heads per kv head (32 768 tokens, two kv heads, K = 512) the
+// gather is the faster one from 16 K on: forward 1.45 and 1.71 ms against 1.84 and 3.29; at head_dim 64 with 4 heads too, 0.59 against 0.81.
+// The walk is a launch of its own behind the tiles', as long as its longest row's walk however few the rows are, and the backward forms delta in
+// a pass of its own again: it takes rows to win that back.  Forward + backward, us, tiles to 24 K and gather -> walk, by the rows past 16 K
+// times the heads.  One segment, 32 heads over 8, K = 512: 34 000 2616 -> 2761, 67 000 3222 -> 3261, 132 000 4535 -> 4370; K = 256: 34 000 974 -> 993, 67 000
+// 1250 -> 1274, 99 000 1653 -> 1571; K = 128: 34 000 402 -> 469, 50 000 535 -> 531, 83 000 752 -> 705.  8 over 2, K = 512: 33 000 1264 -> 1481, 49 000 1704 -> 1755,
+// 82 000 2546 -> 2398; K = 128: 56 000 (all that the walk may take) 616 -> 656.  Several segments of 18 to 36 K, 8 over 2, K = 64: 36 000 526 -> 549, 56 000 539 -> 559, 88 000
+// 608 -> 599; 32 over 8: 142 000 1792 -> 1809, 548 000 2847 -> 2455.
+// Two heads per kv head, 16 over 8: one segment, K = 512: 66 000 2369 -> 2590, 99 000 3134 -> 3313, 164 000 5103 -> 4645; K = 256: 83 000 1403 -> 1449, 132 000
+// 2340 -> 2192; and a wave holds twice the queries, so that rows have to be thinner (full launches of 24 K: 1133 -> 1203, 28 K: 1351 -> 1283).  The gather,
+// which reads a key's rows for two heads, is slower than the tiles wherever the walk does not stand (36 K: 1558 and 1750, 70 K: 2696 and 2824).
+#define DSA_WALK_ROWS 61000                              // rows times heads (of groups padded to a power of two), at least
+#define DSA_WALK_ROWS_2 100000                           // with two heads per kv head
 struct RowSplit {
-    int tiles, walk, len;
-    bool past_tiles(int max_seqlen) const { return max_seqlen > tiles && max_seqlen >= len; }
+    int tiles, walk, len, below;
+    bool walks(int max_seqlen) const { return walk > tiles && max_seqlen > tiles && max_seqlen >= len; }
+    // (the only segment of a batch has all of its tokens)
+    bool gathers(int max_seqlen, int T, int N) const { return max_seqlen > walk || (max_seqlen > below && len > below + 1 && (N != 1 || T < len)); }
 };
-static RowSplit row_split_for(bool selected, const int32_t *idx, int Hq, int Hkv, int D, int K) {
-    if (!selected) return {INT32_MAX, INT32_MAX, 0};       // dense causal: tiles everywhere
+// (N = 0: of a segment whose batch is not known, which takes no fewer rows than any batch)
+static RowSplit row_split_for(bool selected, const int32_t *idx, int T, int N, int Hq, int Hkv, int D, int K) {
+    if (!selected) return {INT32_MAX, INT32_MAX, 0, INT32_MAX};           // dense causal: tiles everywhere
     auto line = [&](int64_t times) {
         const int64_t p = K * times;
         return p >= INT32_MAX - 256 ? INT32_MAX : (int)((p + 255) / 256 * 256);
     };
     const int crossover = g_tile_crossover.load(std::memory_order_relaxed), G = Hq / Hkv;
-    const bool walks = crossover == DSA_TILE_CROSSOVER && D == 128 && G >= 2 && G <= 4;
-    if (!idx) return {walks ? line(16) : INT32_MAX, INT32_MAX, walks ? line(18) : 0};    // (no list to gather by)
-    if (walks) return {line(16), line(G == 2 ? 150 : 75), line(18)};
-    return {line(crossover), line(crossover), 0};
+    const bool two = G == 2;
+    if (crossover != DSA_TILE_CROSSOVER || D != 128 || G < 2 || G > 4) {
+        const int split = idx ? line(crossover) : INT32_MAX;
+        return {split, split, 0, split};
+    }
+    // the rows a segment has by itself, or, where the segments of the batch are long on average, as many segments like it as there are tokens for
+    auto tokens_for = [&](int64_t times, double rows) { return (int)std::min(K * (double)times + rows, (double)INT32_MAX); };
+    const int heads = Hkv << (two ? 1 : 2), least = line(two ? 26 : 18);
+    const double rows = two ? DSA_WALK_ROWS_2 : DSA_WALK_ROWS, all = (double)T * heads;
+    const int alone = std::max(least, tokens_for(16, rows / heads)), many = all > rows ? std::max(least, tokens_for(16, 16. * K * rows / (all - rows))) : INT32_MAX;
+    RowSplit s{line(16), line(two ? 150 : 75), N > 0 && T / N >= many ? std::min(many, alone) : alone, line(two ? 75 : crossover)};
+    if (s.len > s.walk) s.tiles = s.walk = s.below, s.len = 0;            // (rows too thin for the walk before there are enough of them)
+    if (!idx) s = {s.len ? s.tiles : INT32_MAX, INT32_MAX, s.len, INT32_MAX};             // no list to gather by
+    return s;
 }
 extern "C" int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen) {
     if (Hkv < 1 || Hq < Hkv || K < 1) return 1;
     static const int32_t some = 0;
-    return max_seqlen > row_split_for(true, &some, Hq, Hkv, D, K).walk;
+    return row_split_for(true, &some, 0, 0, Hq, Hkv, D, K).gathers(max_seqlen, 0, 0);
 }
 
 // The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,
@@ -348,7 +373,7 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, bool select
     if (int rc = check_aligned(k, v, "k and v")) return rc;
     if (max_seqlen < 1 || max_seqlen > (T > 0 ? T : 1)) return fail(DSA_ERR_ARG, "max_seqlen=%d outside [1,T=%d]", max_seqlen, T);
     if (T == 0) return DSA_OK;
-    const RowSplit rows = row_split_for(selected, idx, Hq, Hkv, D, K);
+    const RowSplit rows = row_split_for(selected, idx, T, N, Hq, Hkv, D, K);
     const int ldw = bitmap_ldw(max_seqlen);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = hipSuccess;
@@ -366,15 +391,15 @@ static int attn_fwd_run(const void *q, const void *k, const void *v, bool select
         }
         const int64_t strides[6] = {(int64_t)Hq * D, D, (int64_t)Hkv * D, D, (int64_t)Hkv * D, D};
         e = dsa_launch_tile_fwd(q, k, v, strides, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
-                                idx ? 0 : K, dtype == DSA_DTYPE_SPLIT_BF16, causal, out, lse, st);
+                                rows.below, idx ? 0 : K, dtype == DSA_DTYPE_SPLIT_BF16, causal, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "tile forward launch");
     }
-    if (rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
+    if (rows.walks(max_seqlen)) {
         e = dsa_launch_sel_fwd(q, k, v, (const uint32_t *)ws, ldw, cu, N, T, Hq, Hkv, softmax_scale, rows.tiles, rows.walk, rows.len, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "compacted forward launch");
     }
-    if (max_seqlen > rows.walk) {
-        e = dsa_launch_attn_fwd(q, k, v, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, out, lse, st);
+    if (rows.gathers(max_seqlen, T, N)) {
+        e = dsa_launch_attn_fwd(q, k, v, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, rows.len, rows.below, out, lse, st);
         if (e != hipSuccess) return hip_fail(e, "gather forward launch");
     }
     return DSA_OK;
@@ -625,7 +650,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
                         bool carried = false) {
     const int ldw = bitmap_ldw(max_seqlen);
     if (selected && (size_t)ldw * 4 > 64 * 1024) return fail(DSA_ERR_UNSUPPORTED, "max_seqlen=%d: selection bitmap row exceeds 64 KiB of LDS", max_seqlen);
-    const RowSplit rows = row_split_for(selected, idx, Hq, Hkv, D, K);
+    const RowSplit rows = row_split_for(selected, idx, T, N, Hq, Hkv, D, K);
     hipError_t e = hipSuccess;
     // the two passes side by side on two streams: launches of few workgroups only (larger ones fill the GPU alone)
     std::unique_lock<std::mutex> ov_lock;
@@ -634,7 +659,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     // head_dim 256: both passes in one launch (dsa_tile_bwd.hip), whatever its size.  Backward, us, one after the other with delta from dQ -> one launch:
     // 16 heads over 2: 700 and 300 tokens 114 -> 81, eight segments of 512 132 -> 122, 16 of 1000 604 -> 570, 4 of 4096 1854 -> 1735, 4 of 8192 6397 -> 6440;
     // fp32 rows of 64, 8 heads over 2: 75 -> 60, 82 -> 69, 287 -> 271, 727 -> 677, 2405 -> 2410; without a causal mask, eight of 700 330 -> 258.
-    const bool one_launch = ov_mode > 0 && (parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && D == 256 && max_seqlen <= rows.tiles &&
+    const bool one_launch = ov_mode > 0 && (parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && D == 256 && max_seqlen <= rows.below &&
                             !(((uintptr_t)q | (uintptr_t)dout) & 15);
     if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0 && !one_launch) {
         const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);     // (head_dim 256: one workgroup per CU, half as many fill it)
@@ -648,7 +673,7 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     // delta = rowsum(dO * O): a pass of its own, unless the tile dQ kernel of the same call owns every query row
     // (no row beyond the tile/gather split) - then that kernel forms it from the dO rows it loads anyway - and the
     // key side, which reads every delta, runs after it
-    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.past_tiles(max_seqlen) && !ov && !one_launch;
+    const bool fuse_delta = (parts & DSA_BWD_DELTA) && (parts & DSA_BWD_DQ) && rows.tiles > 0 && !rows.walks(max_seqlen) && !rows.gathers(max_seqlen, T, N) && !ov && !one_launch;
     int listed = 0;                                      // the launch order of the key tiles is there
     if ((parts & DSA_BWD_DELTA) && (ov || one_launch)) {
         e = dsa_launch_tile_order_delta(dout, out, cu, N, T, Hq, Hkv, D, selected, causal, order, partial, partial_bytes, delta, st);
@@ -685,15 +710,15 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     if (rc == DSA_OK && (parts & DSA_BWD_DQ) && !one_launch) {
         if (rows.tiles > 0) {
             e = dsa_launch_tile_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, D, softmax_scale, rows.tiles, rows.len,
-                                   idx ? 0 : K, carried, causal, dq, fuse_delta ? out : nullptr, delta, sq);
+                                   rows.below, idx ? 0 : K, carried, causal, dq, fuse_delta ? out : nullptr, delta, sq);
             if (e != hipSuccess) rc = hip_fail(e, "tile dq launch");
         }
-        if (rc == DSA_OK && rows.past_tiles(max_seqlen) && rows.walk > rows.tiles) {
+        if (rc == DSA_OK && rows.walks(max_seqlen)) {
             e = dsa_launch_sel_dq(dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, softmax_scale, rows.tiles, rows.walk, rows.len, dq, sq);
             if (e != hipSuccess) rc = hip_fail(e, "compacted dq launch");
         }
-        if (rc == DSA_OK && max_seqlen > rows.walk) {
-            e = dsa_launch_gather_dq(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, dq, sq);
+        if (rc == DSA_OK && rows.gathers(max_seqlen, T, N)) {
+            e = dsa_launch_gather_dq(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, D, K, softmax_scale, rows.walk, rows.len, rows.below, dq, sq);
             if (e != hipSuccess) rc = hip_fail(e, "gather dq launch");
         }
     }
@@ -754,7 +779,7 @@ static int attn_bwd_saved(const void *dout, const void *q, const void *k, const 
     if (int rc = check_bwd(dout, q, k, v, out, lse, selected, idx, n, cu, T, N, Hq, Hkv, D, K, dtype, max_seqlen, causal, dq, dk, dv)) return rc;
     if (T == 0) return DSA_OK;
     if (selected) {
-        if (row_split_for(selected, idx, Hq, Hkv, D, K).tiles <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
+        if (row_split_for(selected, idx, T, N, Hq, Hkv, D, K).tiles <= 0) return fail(DSA_ERR_ARG, "with the tile crossover at 0 the forward builds no bitmap: use dsa_attn_bwd");
         const size_t have = dsa_attn_fwd_workspace_bytes(T, max_seqlen, 1);
         if (!fwd_ws || fwd_ws_bytes < have) return fail(DSA_ERR_WORKSPACE, "forward workspace (selection bitmap): have %zu bytes, need %zu", fwd_ws_bytes, have);
     }
@@ -831,7 +856,7 @@ extern "C" int dsa_dense_fwd_strided(const void *q, int64_t q_tok, int64_t q_hea
             return fail(DSA_ERR_ARG, "strides must be multiples of 8, token strides below 2^24");
     if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) return fail(DSA_ERR_ARG, "tensors must lie on 16-byte boundaries");
     if (T == 0) return DSA_OK;
-    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, 0, 0, causal, out, lse,
+    const hipError_t e = dsa_launch_tile_fwd(q, k, v, strides, nullptr, 0, cu, N, T, Hq, Hkv, D, softmax_scale, INT32_MAX, 0, INT32_MAX, 0, 0, causal, out, lse,
                                              (hipStream_t)stream);
     return e == hipSuccess ? DSA_OK : hip_fail(e, "tile forward launch");
 }

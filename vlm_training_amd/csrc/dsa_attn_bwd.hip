@@ -28,15 +28,15 @@ __global__ __launch_bounds__(64) void dsa_bwd_dq_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *__restrict__ delta,
     const int32_t *__restrict__ idx, const int32_t *__restrict__ nsel, const int32_t *__restrict__ cu, int N, int T,
-    int Hq, int Hkv, int K, float scale, int pos_min, bf16_t *__restrict__ dq) {
+    int Hq, int Hkv, int K, float scale, int pos_min, int split_len, int pos_short, bf16_t *__restrict__ dq) {
     constexpr int KS = D / 32, DT = D / 16, ROW_B = D * 2 + 8;
     __shared__ __attribute__((aligned(16))) unsigned char klds[32 * ROW_B];
 
     const int lane = threadIdx.x, g = lane >> 4, m = lane & 15;
     const int kvh = blockIdx.x / T, t = blockIdx.x % T;
     const int G = Hq / Hkv;
-    const int s0 = cu[find_segment_wave(cu, N, t)];
-    if (t - s0 < pos_min) return;                     // rows before the split belong to the tile kernel
+    const int seg = find_segment_wave(cu, N, t), s0 = cu[seg];
+    if (t - s0 < (cu[seg + 1] - s0 >= split_len ? pos_min : pos_short)) return;     // rows before the split belong to the tile kernels
     // the count is held to [0, K] and every row id to the batch: a bad list cannot reach outside the tensors
     const int nt = HAS_IDX ? min(nsel[t], K) : (t - s0 + 1);
     const int32_t *irow = HAS_IDX ? idx + (int64_t)t * K : nullptr;
@@ -214,28 +214,28 @@ extern "C" hipError_t dsa_launch_bitmap(const int32_t *idx, const int32_t *n, co
 template <int D>
 static hipError_t launch_dq(const void *dout, const void *q, const void *k, const void *v, const float *lse,
                             const float *delta, const int32_t *idx, const int32_t *n, const int32_t *cu, int N, int T,
-                            int Hq, int Hkv, int K, float scale, int pos_min, void *dq, hipStream_t stream) {
+                            int Hq, int Hkv, int K, float scale, int pos_min, int split_len, int pos_short, void *dq, hipStream_t stream) {
     const dim3 gq((unsigned)((int64_t)T * Hkv));
     if (idx)
         hipLaunchKernelGGL((dsa_bwd_dq_kernel<D, true>), gq, dim3(64), 0, stream, (const bf16_t *)dout,
                            (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, idx, n, cu, N, T, Hq,
-                           Hkv, K, scale, pos_min, (bf16_t *)dq);
+                           Hkv, K, scale, pos_min, split_len, pos_short, (bf16_t *)dq);
     else
         hipLaunchKernelGGL((dsa_bwd_dq_kernel<D, false>), gq, dim3(64), 0, stream, (const bf16_t *)dout,
                            (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta, idx, n, cu, N, T, Hq,
-                           Hkv, K, scale, pos_min, (bf16_t *)dq);
+                           Hkv, K, scale, pos_min, split_len, pos_short, (bf16_t *)dq);
     return hipGetLastError();
 }
 
 extern "C" hipError_t dsa_launch_gather_dq(const void *dout, const void *q, const void *k, const void *v,
                                            const float *lse, const float *delta, const int32_t *idx, const int32_t *n,
                                            const int32_t *cu, int N, int T, int Hq, int Hkv, int D, int K, float scale,
-                                           int pos_min, void *dq, hipStream_t stream) {
+                                           int pos_min, int split_len, int pos_short, void *dq, hipStream_t stream) {
     if (T == 0) return hipSuccess;
     switch (D) {
-        case 64: return launch_dq<64>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, dq, stream);
-        case 128: return launch_dq<128>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, dq, stream);
-        case 256: return launch_dq<256>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, dq, stream);
+        case 64: return launch_dq<64>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, split_len, pos_short, dq, stream);
+        case 128: return launch_dq<128>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, split_len, pos_short, dq, stream);
+        case 256: return launch_dq<256>(dout, q, k, v, lse, delta, idx, n, cu, N, T, Hq, Hkv, K, scale, pos_min, split_len, pos_short, dq, stream);
         default: return hipErrorInvalidValue;
     }
 }

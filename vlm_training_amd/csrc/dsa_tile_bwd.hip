@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256, 1) void dsa_tile_dkv_kernel_and_dq(
                                                            causal, 256, INT32_MAX, order, partial, dk, dv);
     else
         dq_block<256, HAS_IDX, 4, 1, CARRIED>(blockIdx.x - key_blocks, gridDim.x - key_blocks, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, GSHIFT, scale,
-                                              INT32_MAX, 0, window, causal, 256, dq, nullptr, nullptr);
+                                              INT32_MAX, 0, INT32_MAX, window, causal, 256, dq, nullptr, nullptr);
 }
 
 template <bool HAS_IDX, int GS, bool CARRIED>

@@ -29,7 +29,7 @@ __device__ __forceinline__ void dq_block(int block, int blocks,
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift,
-    float scale, int pos_split, int split_len, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
+    float scale, int pos_split, int split_len, int pos_short, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
     typedef DirectTile<D> TL;
     constexpr int KS = CARRIED ? DSA_CARRIED_KS : D / 16, DT = CARRIED ? 4 : (D + 31) / 32, NP = 2 * DT;
@@ -51,7 +51,7 @@ __device__ __forceinline__ void dq_block(int block, int blocks,
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                   // a bitmap row has ldw words whatever the caller's max_seqlen
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
-    if ((qc0 >= pos_split && L >= split_len) || qc0 >= L) return;   // rows past the split are not the tile kernels'
+    if (qc0 >= (L >= split_len ? pos_split : pos_short) || qc0 >= L) return;       // rows past the split are not the tile kernels'
     const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
 
     // ---- requests ----

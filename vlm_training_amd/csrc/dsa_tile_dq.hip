@@ -6,15 +6,15 @@ __global__ __launch_bounds__(NW * 64, 1) void dsa_tile_dq_kernel(
     const bf16_t *__restrict__ dout, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, const float *__restrict__ lse, const float *delta,
     const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift,
-    float scale, int pos_split, int split_len, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
+    float scale, int pos_split, int split_len, int pos_short, int window, int causal, int d_real, bf16_t *__restrict__ dq, const bf16_t *__restrict__ out_for_delta,
     float *delta_out) {
-    dq_block<D, HAS_IDX, NW, RG, CARRIED>(blockIdx.x, gridDim.x, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, scale, pos_split, split_len, window, causal, d_real, dq, out_for_delta, delta_out);
+    dq_block<D, HAS_IDX, NW, RG, CARRIED>(blockIdx.x, gridDim.x, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gshift, scale, pos_split, split_len, pos_short, window, causal, d_real, dq, out_for_delta, delta_out);
 }
 
 template <int D, bool HAS_IDX, int RG, bool CARRIED = false>
 static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *q, const void *k, const void *v, const float *lse,
                               const float *delta, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, int Hq, int Hkv, int gs,
-                              int d_real, float scale, int pos_split, int split_len, int window, int causal, void *dq, const void *out_for_delta, float *delta_out) {
+                              int d_real, float scale, int pos_split, int split_len, int pos_short, int window, int causal, void *dq, const void *out_for_delta, float *delta_out) {
     constexpr int NW = 4;
     constexpr size_t lds = dq_lds_bytes<D, NW>(HAS_IDX);
     const auto kernel = &dsa_tile_dq_kernel<D, HAS_IDX, NW, RG, CARRIED>;
@@ -22,7 +22,7 @@ static hipError_t launch_dq_i(hipStream_t stream, const void *dout, const void *
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW * RG) >> gs) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)dout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, lse, delta,
-                       bitmap, ldw, cu, N, T, Hq, Hkv, gs, scale, pos_split, split_len, window, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
+                       bitmap, ldw, cu, N, T, Hq, Hkv, gs, scale, pos_split, split_len, pos_short, window, causal, d_real, (bf16_t *)dq, (const bf16_t *)out_for_delta, delta_out);
     return hipGetLastError();
 }
 // 32 rows per wave instead of 64: each walk is then twice as fast, two workgroups share a CU, and blocks are half as long, which wastes fewer
@@ -47,11 +47,11 @@ static bool dq_one_row_group(int causal, int T, int N, int Hkv, int gs) {
 extern "C" hipError_t dsa_launch_tile_dq(const void *dout, const void *q, const void *k, const void *v,
                                          const float *lse, const float *delta, const uint32_t *bitmap, int ldw,
                                          const int32_t *cu, int N, int T, int Hq, int Hkv, int d_real, float scale,
-                                         int pos_split, int split_len, int window, int carried, int causal, void *dq, const void *out_for_delta, float *delta_out,
+                                         int pos_split, int split_len, int pos_short, int window, int carried, int causal, void *dq, const void *out_for_delta, float *delta_out,
                                          hipStream_t stream) {
     const int gs = group_shift(Hq, Hkv);
     const bool one_group = dq_one_row_group(causal, T, N, Hkv, gs);
-#define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, window, causal, dq, out_for_delta, delta_out
+#define DQ_ARGS stream, dout, q, k, v, lse, delta, bitmap, ldw, cu, N, T, Hq, Hkv, gs, d_real, scale, pos_split, split_len, pos_short, window, causal, dq, out_for_delta, delta_out
 #define DQ_CASE(D_, HI) return one_group ? launch_dq_i<D_, HI, 1>(DQ_ARGS) : launch_dq_i<D_, HI, 2>(DQ_ARGS)
     if (carried) return bitmap ? launch_dq_i<256, true, 1, true>(DQ_ARGS) : launch_dq_i<256, false, 1, true>(DQ_ARGS);
     if (bitmap) switch (d_real) {

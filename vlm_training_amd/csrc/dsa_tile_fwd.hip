@@ -47,7 +47,7 @@ template <int D, bool HAS_IDX, int NW, bool NEG, bool CARRIED, bool AGPR, bool R
 __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_tile_fwd_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, int64_t q_tok, int64_t q_head,
     int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head, const uint32_t *__restrict__ bitmap, int ldw,
-    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int window, int causal,
+    const int32_t *__restrict__ cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale_log2, int pos_split, int split_len, int pos_short, int window, int causal,
     bf16_t *__restrict__ out, float *__restrict__ lse) {
     typedef DirectTile<D> TL;
     // MFMAs of S, of P V (head_dim 80: five and six) and pairs of a step (one of each while there are)
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
-    if ((qc0 >= pos_split && L >= split_len) || qc0 >= L) return;   // rows past the split are not the tile kernels'
+    if (qc0 >= (L >= split_len ? pos_split : pos_short) || qc0 >= L) return;       // rows past the split are not the tile kernels'
     const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
 
     const int r = wv * 32 + j;
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
 
 template <int D, bool HAS_IDX, bool CARRIED = false, bool AGPR = (D > 128)>
 static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw,
-                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int window, int causal,
+                               const int32_t *cu, int N, int T, int Hq, int Hkv, int gshift, int d_real, float scale, int pos_split, int split_len, int pos_short, int window, int causal,
                                void *out, float *lse) {
     constexpr int NW = 4;
     const dim3 grid((unsigned)(((int64_t)T / ((32 * NW) >> gshift) + N + 1) * Hkv));
@@ -479,7 +479,7 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, st[0], st[1], st[2], st[3],
-                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, window, causal, (bf16_t *)out, lse);
+                       st[4], st[5], bitmap, ldw, cu, N, T, Hq, Hkv, gshift, d_real, fabsf(scale) * LOG2E_F, pos_split, split_len, pos_short, window, causal, (bf16_t *)out, lse);
     return hipSuccess;
 }
 // d_real: the head_dim of the tensors, a multiple of 8 (the kernel of the next head_dim of 64, 80, 96, 128, 256 runs it; 80 and 96
@@ -487,9 +487,9 @@ static hipError_t launch_fwd_i(hipStream_t stream, const void *q, const void *k,
 // DSA_CARRIED_KS; st: token and head stride of q, k and v in elements (rows of 16-byte alignment).  The file is compiled twice, the second time
 // (FWD_256) for head_dim 256, with results of MFMA builtins in vector registers: the sums have the accumulation registers.
 #define FWD_LAUNCH_ARGS const void *q, const void *k, const void *v, const int64_t *st, const uint32_t *bitmap, int ldw, const int32_t *cu, int N, int T, \
-    int Hq, int Hkv, int d_real, float scale, int pos_split, int split_len, int window, int carried, int causal, void *out, float *lse, hipStream_t stream
+    int Hq, int Hkv, int d_real, float scale, int pos_split, int split_len, int pos_short, int window, int carried, int causal, void *out, float *lse, hipStream_t stream
 #define FWD_CASE(D_, ...) e = launch_fwd_i<D_, __VA_ARGS__>(stream, q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, group_shift(Hq, Hkv), d_real, logit_scale(scale), \
-                                                            pos_split, split_len, window, causal, out, lse)
+                                                            pos_split, split_len, pos_short, window, causal, out, lse)
 extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS);
 #if FWD_256
 extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS) {
@@ -504,7 +504,7 @@ extern "C" hipError_t dsa_launch_tile_fwd_256(FWD_LAUNCH_ARGS) {
 #else
 extern "C" hipError_t dsa_launch_tile_fwd(FWD_LAUNCH_ARGS) {
     if (d_real > 256) return hipErrorInvalidValue;
-    if (d_real > 128 && (bitmap || carried || scale < 0.f)) return dsa_launch_tile_fwd_256(q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, split_len, window, carried, causal, out, lse, stream);
+    if (d_real > 128 && (bitmap || carried || scale < 0.f)) return dsa_launch_tile_fwd_256(q, k, v, st, bitmap, ldw, cu, N, T, Hq, Hkv, d_real, scale, pos_split, split_len, pos_short, window, carried, causal, out, lse, stream);
     hipError_t e;
     if (bitmap) {
         if (d_real <= 64) FWD_CASE(64, true);
