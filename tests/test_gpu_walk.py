@@ -87,14 +87,14 @@ def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
 
 
 @pytest.mark.parametrize("G,lens,kind", [
-    (4, (1700, 900, 500), "random"),     # 26 K = 1664: the walk takes the first segment, the tile kernel the others
-    (3, (1790, 1400), "random"),         # a group of three; 1790 keys: the last workgroup's 62, the last wave's 14
-    (4, (1664, 1663), "runs"),           # every query of a block wants a key of the tile, or none does
+    (4, (1700, 900, 500), "random"),     # 40 K = 1600: the walk takes the first segment, the tile kernel the others
+    (3, (1934, 1919), "random"),         # a group of three, 48 K = 1920; 1934 keys: the last workgroup's 14, one wave's
+    (4, (1600, 1599), "runs"),           # every query of a block wants a key of the tile, or none does
     (8, (1921, 1200), "same"),           # sixteen keys that all queries want: large probabilities, lists that are full
     (16, (2000, 1100), "classes")])      # queries of one residue: one class of the block's rows
 def test_keys_of_the_compacted_walk(G, lens, kind):
     print("compacted walk, key side", G, lens, kind, flush=True)
-    Hkv, K, T, scale = 64, 64, sum(lens), D ** -0.5
+    Hkv, K, T, scale = 64, 40, sum(lens), D ** -0.5
     assert _lib.load().dsa_get_tile_crossover() == 24 and (T // 128 + len(lens)) * Hkv > 1536
     g = torch.Generator(device=DEV).manual_seed(G)
     q, k, v, dout = (torch.randn(T, h, D, generator=g, device=DEV).mul_(0.5).bfloat16() for h in (G * Hkv, Hkv, Hkv, G * Hkv))

@@ -346,15 +346,21 @@ extern "C" int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen
 
 // The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,
 // three and more heads per kv head, launches that the tile kernel does not cut into pieces (its workgroups, 192 keys each, are cut nowhere: four
-// rounds of them end level).  Tile kernel -> walk, whole backward, ms, 32 heads over 8 kv heads, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5,
-// 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226; K = 512, 57 344 tokens 50.8 -> 33.7; K = 1024, 65 536 tokens, 4 heads over each of
-// 4 kv heads 35.2 -> 28.7, 8 over each of 8 134 -> 102, 16 over each of 8 255 -> 182.
+// rounds of them end level).  A walk pays for building the list of every block of queries, and adds the rounding remainder of P to dV where a step
+// has a probability of 2^-7, the tile kernel where a block has one of 2^-6: with up to 64 keys a row both do nearly always, with some hundred the
+// walk alone.  dK and dV alone, tile kernel / walk, by tokens a segment in 40 000 to 64 000:
+// K = 16, 32, 64, 32 heads over 8: of 28 K 0.94 to 1.1, of 40 K (K = 32, 64) 0.84 to 0.98, of 56 K 0.69 to 0.84, 3 over each of 4: 0.99 to 1.13 up to 36 K, 0.91 to 0.98 from 40 K;
+// K = 128, 32 over 8 / 3 over each of 4 / 8 over each of 8: 4608 tokens 1.05 to 1.10 / 1.35 / 0.99 to 1.05, 7168 0.88 to 0.91 / 1.02 to 1.07 / 0.84 to 0.86, 10 240 0.75 / 0.90 / 0.70;
+// K = 256: 7680 1.02 to 1.04 / 1.16 to 1.20 / 0.99 to 1.01, 11 264 0.84 / 0.94 / 0.81; K = 512: 13 568 0.97 / 1.04 to 1.14 / 0.94, 18 432 0.90 / 0.90 / 0.88; K = 1024:
+// 27 136 0.98 to 1.01 / 0.95 / 0.96, 36 864 0.88 / - / 0.87.  Whole backward, ms, 32 over 8, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5,
+// 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226.
 static int key_walk_len(bool selected, const void *q, const void *dout, int T, int N, int Hq, int Hkv, int D, int K) {
     const int G = Hq / Hkv;
     if (!selected || D != 128 || G < 3 || ((int64_t)T / 128 + N) * Hkv <= dkv_pieces_max_wg(D) || (((uintptr_t)q | (uintptr_t)dout) & 15) ||
         g_tile_crossover.load(std::memory_order_relaxed) != DSA_TILE_CROSSOVER)
         return INT32_MAX;
-    return (int)std::min<int64_t>((int64_t)K * 26, INT32_MAX);
+    const bool three = G == 3;                           // (a quarter of the walk's rows is padding)
+    return (int)std::min<int64_t>(K <= 64 ? K * (three ? 48 : 40) : (int64_t)K * 24 + (three ? 6144 : 4608), INT32_MAX);
 }
 
 extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_idx) {
