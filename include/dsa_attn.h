@@ -234,8 +234,9 @@ int dsa_get_tile_crossover(void);
  * what the overlap gains) the query side runs on a second stream of the library's own (default priority, one per device, created
  * on the first such call outside a capture) between a fork and a join event on the caller's stream, so that to the
  * caller the whole call is still ordered on the stream it passed; under stream capture the second stream joins the
- * capture through those events.  0: never (one stream).  2: for every launch size.  Results are the same bits in all
- * modes.  dsa_indexer_bwd runs its query side and its key side the same way (mode 1: up to 16 384 tokens).
+ * capture through those events.  At head_dim 256 (q and dout on 16-byte boundaries, every row the tile kernels') one launch holds both passes
+ * instead, in mode 1 up to 300 000 rows T * Hq or where segments have at most 256 tokens on average; beyond that they run one after the other.
+ * 0: never (one stream, two launches).  2: for every launch size.  Results are the same bits in all modes.  dsa_indexer_bwd runs its query side and its key side the same way (mode 1: up to 16 384 tokens).
  */
 int dsa_set_bwd_overlap(int mode);
 int dsa_get_bwd_overlap(void);

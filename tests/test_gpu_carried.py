@@ -54,7 +54,10 @@ def test_carried_rows_give_the_bits_of_whole_rows(Hq, Hkv, segs, K, causal, scal
     (16, 2, (700, 65, 129), 100, True, torch.bfloat16),  # a selection with whole windows; gathered rows (past 24 K) in none
     (4, 4, (1, 500), 64, True, torch.bfloat16), (6, 2, (257,), 300, True, torch.bfloat16), (16, 1, (1500, 40), 64, True, torch.bfloat16),
     (8, 4, (400, 31), None, True, torch.bfloat16), (2, 1, (128, 333), None, False, torch.bfloat16),
-    (4, 1, (300, 64), 50, True, torch.float32), (2, 2, (350,), None, True, torch.float32)])
+    (4, 1, (300, 64), 50, True, torch.float32), (2, 2, (350,), None, True, torch.float32),
+    # by default one launch up to 300 000 rows, or of short segments; past that one pass after the other
+    (100, 25, (1700, 1300), None, True, torch.bfloat16), (100, 25, (1701, 1300), 900, True, torch.bfloat16), (120, 30, (256,) * 10, None, True, torch.bfloat16),
+    (304, 76, (1000,), None, False, torch.float32)])
 def test_both_passes_in_one_launch_give_the_bits_of_two(Hq, Hkv, segs, K, causal, dtype):
     print("one launch", Hq, Hkv, segs, K, causal, dtype, flush=True)
     lib, D = _lib.load(), 256 if dtype == torch.bfloat16 else 64
@@ -65,12 +68,12 @@ def test_both_passes_in_one_launch_give_the_bits_of_two(Hq, Hkv, segs, K, causal
     sel = dict(indexer_q=mk(T, 4, 64), indexer_k=mk(T, 64), indexer_w=mk(T, 4), top_k=K) if K else dict(causal=causal)
     res, old = [], lib.dsa_get_bwd_overlap()
     try:
-        for mode in (0, 2):
+        for mode in (0, 1, 2):
             _lib.check(lib.dsa_set_bwd_overlap(mode), "dsa_set_bwd_overlap")
             a, b, c = (x.clone().requires_grad_(True) for x in (q, k, v))
             ops.dsa_varlen_attn(a, b, c, cu, max(segs), **sel).backward(do)
             res.append((a.grad, b.grad, c.grad))
     finally:
         lib.dsa_set_bwd_overlap(old)
-    for one, two in zip(*res):
-        assert torch.equal(one, two)
+    for apart, default, one in zip(*res):
+        assert torch.equal(apart, default) and torch.equal(apart, one)

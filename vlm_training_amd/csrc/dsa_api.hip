@@ -524,6 +524,7 @@ extern "C" int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const fl
 // rows of 4096-8192 tokens, 5-19 % less; 10 000-16 384 tokens, 0-3 % less; 1000 tokens at 2e9, 130 -> 105; 700 tokens at 7e8,
 // level.  Without a causal mask the walks of a segment are all equally long, and small launches win nothing.
 #define DSA_BWD_OVERLAP_MAX_WG (6 * 256)
+#define DSA_ONE_LAUNCH_ROWS 300000                       // (query, head) rows of a launch of both passes, at most (attn_bwd_run)
 #define DSA_BWD_OVERLAP_MIN_WORK 2.0e9
 #define DSA_BWD_OVERLAP_MIN_WORK_FULL 6.0e10
 struct OverlapCtx {
@@ -662,12 +663,16 @@ static int attn_bwd_run(const void *dout, const void *q, const void *k, const vo
     std::unique_lock<std::mutex> ov_lock;
     OverlapCtx *ov = nullptr;
     const int ov_mode = g_bwd_overlap.load(std::memory_order_relaxed);
-    // head_dim 256: both passes in one launch (dsa_tile_bwd.hip), whatever its size.  Backward, us, one after the other with delta from dQ -> one launch:
-    // 16 heads over 2: 700 and 300 tokens 114 -> 81, eight segments of 512 132 -> 122, 16 of 1000 604 -> 570, 4 of 4096 1854 -> 1735, 4 of 8192 6397 -> 6440;
-    // fp32 rows of 64, 8 heads over 2: 75 -> 60, 82 -> 69, 287 -> 271, 727 -> 677, 2405 -> 2410; without a causal mask, eight of 700 330 -> 258.
-    const bool one_launch = ov_mode > 0 && (parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && D == 256 && max_seqlen <= rows.below &&
-                            !(((uintptr_t)q | (uintptr_t)dout) & 15);
-    if ((parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0 && !one_launch) {
+    // head_dim 256: both passes in one launch (dsa_tile_bwd.hip), or, where that does not pay, one after the other.  It saves a launch and the idle CUs of
+    // the key side's end; the pass over dO and O that dQ has inside it when it runs first comes back, and that grows with the rows.  Backward, us, one
+    // after the other -> one launch, 16 heads over 2: 300 tokens 73 -> 54, 2500 253 -> 190, eight segments of 512 137 -> 118, 16 of 1000 562 -> 537, 4 of 4000 2009 ->
+    // 1593, 4 of 8000 (512 000 rows) 5852 -> 5852, 48 of 1000 (768 000) 1590 -> 1616; 16 over 4: 16 000 tokens 5718 -> 5682, 4 of 8000 with a selection 5712 -> 5872;
+    // 8 over 8: 4 of 4000 814 -> 804, 48 of 1000 (384 000) 1013 -> 1042; 32 over 8: 4 of 4000 (512 000) 3108 -> 3182, 4 of 8000 11 560 -> 11 813; fp32 rows of 64, 16 over 8: 4 of
+    // 4000 1197 -> 1194, 4 of 8000 4399 -> 4553, 48 of 1000 1502 -> 1558.  200 segments of 100 (640 000) 743 -> 674: of short ones whatever the rows.
+    const bool both = (parts & DSA_BWD_DQ) && (parts & DSA_BWD_DKV) && ov_mode > 0;
+    const bool may_share = both && D == 256 && max_seqlen <= rows.below && !(((uintptr_t)q | (uintptr_t)dout) & 15);
+    const bool one_launch = may_share && (ov_mode == 2 || (int64_t)T * Hq <= DSA_ONE_LAUNCH_ROWS || T / 256 <= N);
+    if (both && !may_share) {
         const int64_t dkv_wg = ((int64_t)T / 128 + N) * Hkv * (D > 128 ? 2 : 1);     // (head_dim 256: one workgroup per CU, half as many fill it)
         const double work = (double)T * max_seqlen * Hq * D;
         if (ov_mode == 2 || (dkv_wg <= DSA_BWD_OVERLAP_MAX_WG && work >= (causal ? DSA_BWD_OVERLAP_MIN_WORK : DSA_BWD_OVERLAP_MIN_WORK_FULL))) {

@@ -265,8 +265,8 @@ def set_tile_crossover(crossover: int) -> int:
 
 def set_bwd_overlap(mode: int) -> int:
     """0: the backward's passes run one after the other on the caller's stream; 1 (default): launches of few
-    workgroups run dQ beside dK/dV on a second stream of the library's own, and at head_dim 256 one launch holds both; 2: every
-    launch runs them side by side.  Same bits in every mode.  Returns the previous mode."""
+    workgroups run dQ beside dK/dV on a second stream of the library's own, and at head_dim 256 one launch holds both (up to
+    300 000 rows, or of short segments); 2: every launch runs them side by side.  Same bits in every mode.  Returns the previous mode."""
     lib = _lib.load()
     old = lib.dsa_get_bwd_overlap()
     _lib.check(lib.dsa_set_bwd_overlap(int(mode)), "dsa_set_bwd_overlap")
