@@ -129,3 +129,43 @@ def test_keys_of_the_compacted_walk(G, lens, kind):
         want = _reference(q[:, rows], k[:, h:h + 1], v[:, h:h + 1], dout[:, rows], sel, scale)
         for name, got, ref in (("out", out[:, rows], want[0]), ("dq", dq[:, rows], want[2]), ("dk", dk[:, h:h + 1], want[3]), ("dv", dv[:, h:h + 1], want[4])):
             assert_close_bf16(got, ref, f"{name} of kv head {h}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,K,empty", [(288, 72, (1200, 60, 700), 16, False), (440, 220, (1500,), 16, True), (288, 96, (900,), 12, True)])
+def test_what_a_key_holds_reaches_the_rows_that_selected_it(Hq, Hkv, lens, K, empty):
+    """Inf and NaN in keys, queries and gradients: rows of the walk hold what the gather kernels give, which read a row's own keys alone."""
+    print("walk, not finite", Hq, Hkv, lens, K, flush=True)
+    T, cu, g = sum(lens), torch.tensor([0, *lens]).cumsum(0).int(), torch.Generator(device=DEV).manual_seed(Hkv)
+    q, k, v, dout = (torch.randn(T, h, D, generator=g, device=DEV).mul_(0.5).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    idx, n, pos = torch.full((T, K), -1, dtype=torch.int32), torch.zeros(T, dtype=torch.int32), torch.cat([torch.arange(m) for m in lens])
+    cg = torch.Generator().manual_seed(Hkv)
+    for a, m in zip(cu.tolist(), lens):
+        for p in range(m):
+            keys = torch.randperm(p + 1, generator=cg)[:0 if empty and p > K and p % 5 == 0 else K].sort().values + a
+            n[a + p], idx[a + p, :len(keys)] = len(keys), keys.int()
+    v[100, :, 5], v[333, :, :], k[210, :, 9] = math.inf, math.nan, math.nan
+    k[417, ::2, 3], v[520, 1::2, 77] = -math.inf, -math.inf
+    q[600, ::3, 0], dout[640, ::5, 11] = math.inf, math.nan
+    d = [x.to(DEV) for x in (idx, n, cu)]
+    scale, res, old = D ** -0.5, [], _lib.load().dsa_get_tile_crossover()
+    assert old == 24
+    try:
+        for crossover in (old, 0):
+            ops.set_tile_crossover(crossover)
+            out, lse = ops.attn_fwd(q, k, v, *d, max(lens), scale, True)[:2]
+            if crossover:
+                first = (out, lse)
+            dq = ops.attn_bwd(dout, q, k, v, first[0], first[1].clamp(min=-1e30), *d, max(lens), scale, causal=True)[0]
+            res.append((out, lse.T, dq))
+    finally:
+        ops.set_tile_crossover(old)
+    late = (pos >= (16 * K + 255) // 256 * 256).to(DEV) & torch.cat([torch.full((m,), m >= 600) for m in lens]).to(DEV)
+    touched = torch.isin(idx, torch.tensor([100, 333, 210, 417, 520])).any(1).to(DEV)
+    touched[600] = touched[640] = True
+    assert int((late & ~touched).sum()) > 100 and int((late & touched).sum()) > 20
+    for name, a, b in zip(("out", "lse", "dq"), *res):
+        a, b = a[late].float(), b[late].float()
+        assert bool((a.isfinite() == b.isfinite()).all()), name             # (a gathered row's last key also stands behind its end, with 0: Inf turns to NaN)
+        assert bool(a[~touched[late]].isfinite().all()) or name == "lse" and empty
+        there = b.isfinite()
+        assert_close_bf16(a[there], b[there], name)
