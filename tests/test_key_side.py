@@ -130,12 +130,13 @@ def test_inline_mfmas_keep_their_wait_states(tmp_path):
     count, kernels, found = 0, set(), []
     for name in sorted(os.listdir(tmp_path)):
         path = tmp_path / name
-        held = {k for k in (b"dsa_tile_dkv_kernel", b"dsa_tile_dq_kernel", b"dsa_tile_fwd_kernel", b"dsa_tile_idxg_kernel") if name.endswith("gfx950") and k in path.read_bytes()}
+        held = {k for k in (b"dsa_tile_dkv_kernel", b"dsa_tile_dkv_kernel_and_dq", b"dsa_tile_dq_kernel", b"dsa_tile_fwd_kernel", b"dsa_tile_idxg_kernel", b"dsa_tile_sel_kernel",
+                            b"dsa_tile_selkv_kernel") if name.endswith("gfx950") and k in path.read_bytes()}
         if held:
             kernels |= held
             c, f = _hazards(subprocess.run([OBJDUMP, "-d", str(path)], check=True, capture_output=True, text=True).stdout)
             count, found = count + c, found + f
-    assert len(kernels) == 4 and count > 1000 and not found, (kernels, count, found[:5])
+    assert len(kernels) == 7 and count > 1000 and not found, (kernels, count, found[:5])
 
 
 def _case(D, Hq, Hkv, lens, seed):
