@@ -111,7 +111,7 @@ def test_bound_above_the_lds_cache_keeps_short_rows_on_the_cached_select():
 @pytest.mark.timeout(900)
 def test_long_single_sequence_by_invariants_and_sampled_rows():
     """C4 as benchmarked (one causal sequence of 131 072 tokens, top-k 2048): the chunked score/select loop over 64
-    chunks, the gather kernels at long range, bitmap rows of 4096 words.  Checked by statements that hold at any size
+    chunks, the compacted walks at long range, bitmap rows of 4096 words.  Checked by statements that hold at any size
     (as for the headline configuration), and on sampled query rows against the oracle: selection bit-exact on the
     GPU's own scores of that row, out and dq of sampled query rows and dk, dv of sampled key rows within tolerance."""
     _log("C4 full size")
@@ -143,10 +143,12 @@ def test_long_single_sequence_by_invariants_and_sampled_rows():
     assert torch.allclose(a, b, rtol=2e-2, atol=2e-2 * float(a.abs().max())), (a, b)
     want = t["dout"].float().sum(0).view(w.Hkv, G, w.D).sum(1)
     assert torch.allclose(dv.float().sum(0), want, rtol=2e-2, atol=2e-2 * float(want.abs().max()))
-    # sampled rows: around top_k, around the select kernel's LDS cache, around the tile/gather crossover, the end
-    X = lib.dsa_get_tile_crossover() * K                 # first row of the gather kernels (a multiple of 256 here)
-    assert K < X < T and X % 256 == 0
-    rows = [0, 1, K - 1, K, K + 1, 8191, 8192, 8193, X - 1, X, X + 1, 65535, 100003, T - 2, T - 1]
+    # sampled rows: around top_k, around the select kernel's LDS cache, on both sides of the first row of the compacted walk and of the end
+    # of its first block (96 queries from 32 736 on, in dQ 64 from 32 768 on), where the gather would begin, the end
+    X, Y = 16 * K, lib.dsa_get_tile_crossover() * K
+    assert lib.dsa_get_tile_crossover() == 24 and K < X < Y < T and X % 256 == 0
+    assert not lib.dsa_attn_reads_list(w.Hq, w.Hkv, w.D, K, T)          # (no row is the gather's)
+    rows = [0, 1, K - 1, K, K + 1, 8191, 8192, 8193, X - 1, X, X + 1, X + 63, X + 64, Y - 1, Y, 65535, 100003, T - 2, T - 1]
     scale = (w.Di ** -0.5) * (w.Hi ** -0.5)
     st = torch.cuda.current_stream().cuda_stream
     row_sc = torch.empty((1, T), dtype=torch.float32, device=DEV)
@@ -170,9 +172,9 @@ def test_long_single_sequence_by_invariants_and_sampled_rows():
     e1 = assert_close_bf16(out[rows], ref.detach(), "out (sampled rows)")
     e2 = assert_close_bf16(dq[rows], qc.grad[rows], "dq (sampled rows)")
     _log(f"  C4 sampled rows: out ({e1[0]:.2e},{e1[1]:.6f}) dq ({e2[0]:.2e},{e2[1]:.6f})")
-    # dk and dv of sampled key rows (first key tile, around top_k, around the select cache and the tile/gather crossover,
-    # the last tile): every query that selected the key is looked up in idx and attended over its own keys by the oracle
-    keys = [17, K, 8192, X, 100003, T - 70, T - 1]
+    # dk and dv of sampled key rows (the walk's first workgroup of 192 keys and the edge to its second, around top_k and the select cache, the
+    # first row of the query side's walk, the last tile): every query that selected the key is looked up in idx and attended over its own keys by the oracle
+    keys = [17, 191, 192, K, 8192, X, 100003, T - 70, T - 1]
     want_dk, want_dv = R.sparse_attention_key_rows(t["q"].cpu(), t["k"].cpu(), t["v"].cpu(), t["dout"].cpu(), idx_c, n_c, keys)
     e3 = assert_close_bf16(dk[keys], want_dk, "dk (sampled key rows)")
     e4 = assert_close_bf16(dv[keys], want_dv, "dv (sampled key rows)")
