@@ -321,22 +321,21 @@ def main():
     wk = w.work()
     S = wk["S"]
     unit = w.Hq * w.D * S                 # one flop-unit: a multiply-add pass over every selected (query, key, head, d)
-    kern = {   # algorithmic flop per launch of the three attention kernels (selected pairs only)
-        "attn_fwd": ("dsa_tile_fwd_kernel", 4 * unit),          # QK^T + PV
-        "bwd_dq": ("dsa_tile_dq_kernel", 6 * unit),   # QK^T + dO V^T + dS K
-        # QK^T + dO V^T + P^T dO + dS^T Q
-        "bwd_dkv": ("dsa_tile_dkv_kernel", 8 * unit),
+    # What the matrix cores actually execute: the tile kernels compute every causal pair of a visited tile and mask the unselected
+    # ones, so their MFMA rate is the selected-pair rate times (executed pairs / selected pairs).  A side of which other kernels take
+    # the thin rows or keys (the compacted walks, the gather) goes by their name and has no such figure.
+    xq, xk = w.executed_pairs(ops._lib.load().dsa_get_tile_crossover())
+    walks = w.D == 128 and ops._lib.load().dsa_get_tile_crossover() == 24
+    kern = {   # algorithmic flop per launch of the three attention kernels (selected pairs only), executed pairs
+        "attn_fwd": ("dsa_tile_fwd_kernel" if xq else "dsa_tile_sel_kernel" if walks else "dsa_attn_fwd_kernel", 4 * unit, xq),    # QK^T + PV
+        "bwd_dq": ("dsa_tile_dq_kernel" if xq else "dsa_tile_sel_kernel (dQ)" if walks else "dsa_bwd_dq_kernel", 6 * unit, xq),     # QK^T + dO V^T + dS K
+        "bwd_dkv": ("dsa_tile_dkv_kernel" if xk else "dsa_tile_selkv_kernel", 8 * unit, xk),   # QK^T + dO V^T + P^T dO + dS^T Q
     }
     dom = max(kern, key=lambda name: stage_ms[name])
-    dom_kernel, dom_flop = kern[dom]
+    dom_kernel, dom_flop, dom_pairs = kern[dom]
     achieved = dom_flop / (stage_ms[dom] * 1e-3) / 1e12
-    # what the matrix cores actually execute: the tile kernels compute every causal pair of a visited tile and mask
-    # the unselected ones, so their MFMA rate is the selected-pair rate times (executed pairs / selected pairs)
-    xq, xk = w.executed_pairs(ops._lib.load().dsa_get_tile_crossover())
-    executed_pairs = {"attn_fwd": xq, "bwd_dq": xq, "bwd_dkv": xk}
-    executed = dom_flop / S * executed_pairs[dom] / (stage_ms[dom] * 1e-3) / 1e12
-    executed_by_kernel = {kern[name][0]: kern[name][1] / S * executed_pairs[name] / (stage_ms[name] * 1e-3) / 1e12 / PEAK_MFMA_BF16_TFLOPS
-                          for name in kern}
+    executed_frac = lambda name: kern[name][2] and kern[name][1] / S * kern[name][2] / (stage_ms[name] * 1e-3) / 1e12 / PEAK_MFMA_BF16_TFLOPS
+    executed_by_kernel = {kern[name][0]: executed_frac(name) for name in kern}
     t_roof_ms = {
         "index_topk": max(wk["F1"] / (PEAK_MFMA_BF16_TFLOPS * 1e12), wk["B2"] / (PEAK_HBM_GBS * 1e9)) * 1e3,
         "attn_fwd": max(wk["F3"] / (PEAK_MFMA_BF16_TFLOPS * 1e12), wk["B3"] / (PEAK_HBM_GBS * 1e9)) * 1e3,
@@ -372,8 +371,8 @@ def main():
                                f"indexer {w.Hi}x{w.Di}, top_k={w.top_k}, fwd+bwd"},
         "roofline": {"bound": "mfma", "kernel": dom_kernel, "achieved": achieved, "peak": PEAK_MFMA_BF16_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_MFMA_BF16_TFLOPS,
-                     "executed": executed, "executed_frac": executed / PEAK_MFMA_BF16_TFLOPS,
-                     "executed_pairs_over_selected": executed_pairs[dom] / S, "executed_frac_by_kernel": executed_by_kernel,
+                     "executed": dom_pairs and executed_frac(dom) * PEAK_MFMA_BF16_TFLOPS, "executed_frac": executed_frac(dom),
+                     "executed_pairs_over_selected": dom_pairs and dom_pairs / S, "executed_frac_by_kernel": executed_by_kernel,
                      "traffic": traffic,
                      "traffic_source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of an earlier run of this command, scaled by a 1 GiB copy (profiles/)",
                      "algorithmic_flop": dom_flop, "avg_ms": stage_ms[dom]},

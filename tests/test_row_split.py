@@ -22,3 +22,13 @@ def test_rows_that_the_list_is_read_for(Hq, Hkv, K, longest, listed):
     assert lib.dsa_attn_reads_list(Hq, Hkv, 128, K, longest) == listed
     # elsewhere one line, wherever the heads stand
     assert lib.dsa_attn_reads_list(Hq, Hkv, 64, K, longest) == (longest > (24 * K + 255) // 256 * 256)
+
+
+def test_pairs_of_a_workload_are_counted_where_the_tile_kernels_take_all():
+    from vlm_training_amd import workloads as W
+    for w in (W.C1, W.C2, W.C3, W.C5):
+        assert w.executed_pairs() == (w.pair_counts()[0],) * 2
+    assert W.C4.executed_pairs() == (None, None)         # late rows and the key side are the compacted walks'
+    few = W.head_shard(W.C4, 8)                          # (one kv head: key tiles cut into pieces, never walked)
+    assert few.executed_pairs() == (None, few.pair_counts()[0])
+    assert W.C3.executed_pairs(crossover=0) == (None, W.C3.pair_counts()[0])

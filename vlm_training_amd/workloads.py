@@ -8,7 +8,7 @@ one more segment (data/energon_dataloader.py:431-464, models/qwen3_vl/model.py:7
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Dict, List, Tuple
+from typing import Dict, List, Optional, Tuple
 
 import torch
 
@@ -52,14 +52,17 @@ class Workload:
             S += d * (d + 1) // 2 + max(0, L - self.top_k) * self.top_k
         return P, S
 
-    def executed_pairs(self, crossover: int = 24) -> Tuple[int, int]:
-        """(query side, key side): the (query, key) pairs a walk of whole tiles with the selection as a mask puts through
-        the matrix cores: on the query side (forward, dQ) the causal pairs of the rows at positions < top_k * crossover
-        (rounded up to 256), on the key side (dK/dV) every causal pair.  Long segments with thin selections run fewer: their
-        late rows, and the key side from 26 * top_k tokens on, are compacted walks or gathers."""
-        split = (self.top_k * crossover + 255) // 256 * 256
-        q_side = sum(min(L, split) * (min(L, split) + 1) // 2 for L in self.seg_lens)
-        return q_side, self.pair_counts()[0]
+    def executed_pairs(self, crossover: int = 24) -> Tuple[Optional[int], Optional[int]]:
+        """(query side, key side): the (query, key) pairs that the tile kernels put through the matrix cores when they take every row (forward, dQ) and
+        every key (dK/dV) - every causal pair.  None for a side of which segments are long enough for other kernels, whose pairs go by the
+        selection: rows gathered past top_k * crossover, or, at the default crossover and head_dim 128, the compacted walks of rows past 16 * top_k
+        (two to four heads per kv head) and of keys (three and more, from 24 * top_k + 4608 tokens on, 40 * top_k up to 64 keys a row, in launches too
+        large to be cut into pieces)."""
+        G, K, causal = self.Hq // self.Hkv, self.top_k, self.pair_counts()[0]
+        walks = crossover == 24 and self.D == 128
+        rows = K * (16 if walks and 2 <= G <= 4 else crossover)
+        keys = (24 * K + 4608 if K > 64 else 40 * K) if walks and G >= 3 and (self.T // 128 + len(self.seg_lens)) * self.Hkv > 1536 else self.max_seqlen + 1
+        return causal if self.max_seqlen <= rows else None, causal if self.max_seqlen < keys else None
 
     def work(self) -> Dict[str, float]:
         """Algorithmic flop / byte counts per fwd+bwd pass (bf16 element = 2 bytes)."""
