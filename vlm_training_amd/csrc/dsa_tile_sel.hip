@@ -10,8 +10,9 @@
 // walk takes four, and a block read from L2 serves all queries of the workgroup (the gather kernels read every row's keys on its own: 0.6 TB
 // past L2 at 131 072 tokens).
 //
-// What bounds it: the LDS (operand rows of a list lie where they lie: 1.9 instead of 1.0 clocks a read; busy 0.58 of the time), the vector
-// instructions (about 100 a step, 45 more a block for the list) and the spread of the waves' steps between two barriers.  Rows beyond
+// What bounds it: the LDS (operand rows of a list lie where they lie: 1.8 clocks a read instead of 1.0, dQ 2.1; busy 0.53 and 0.57 of the time at
+// 131 072 tokens), the vector instructions (about 100 a step, 45 more a block for the list; 0.47 and 0.36 of a SIMD's time, MFMAs 0.33 and 0.37) and the
+// spread of the waves' steps between two barriers.  Rows beyond
 // 16 K of 131 072 tokens, K = 2048, 32 heads over 8 kv heads, the whole forward / backward, ms: gathered 94.5 / 299; here with eight waves and a step's
 // chain of reads and MFMAs open to its latency 76 / 297, twelve waves, lists built a block ahead 65 / 293, operands read ahead and nothing spilled
 // 56 / 280, exponentials behind the MFMAs of dP 57 / 275.  With twelve waves a spilled register read in the loop waits for the blocks on their way into LDS (+ 25 %).
@@ -24,6 +25,93 @@ constexpr int sel_waves(bool bwd) { return bwd ? 8 : 12; }
 // LDS: two blocks of K and V | of each wave: selection words of three blocks, two lists
 constexpr int SEL_WORD_B = 256, SEL_LIST_B = SEL_KEYS * 4, SEL_WAVE_B = 3 * SEL_WORD_B + 2 * SEL_LIST_B;
 constexpr size_t sel_lds_bytes(bool bwd) { return 4 * (size_t)SelBlock<SEL_KEYS>::BYTES + sel_waves(bwd) * SEL_WAVE_B; }
+
+// One row, the same for all lanes, over its own keys alone: sixteen lanes to a key, four keys at a time, fp32 throughout.
+template <bool BWD>
+__device__ __forceinline__ void sel_redo_row(const bf16_t *q, const bf16_t *k, const bf16_t *v, const bf16_t *dout, const float *lse_in, const float *delta,
+                                             const uint32_t *bitmap, int ldw, int T, int Hq, int Hkv, float scale, float scale_log2, int s0, int L, int kvh, int t, int hq,
+                                             bf16_t *out, float *lse) {
+    constexpr int D = 128;
+    const int lane = threadIdx.x & 63, g = lane >> 4, sub = lane & 15;
+    auto eight = [](const bf16_t *p, float (&x)[8]) __attribute__((always_inline)) {
+        const u32x4 w = __builtin_bit_cast(u32x4, load_bf16x8(p));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
+    };
+    auto over_key = [](float x) __attribute__((always_inline)) {          // sum over the sixteen lanes of a key
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        return x;
+    };
+    const int64_t at = ((int64_t)t * Hq + hq) * D + sub * 8;
+    float qf[8], df[8], acc[8], m = -INFINITY, l = 0.f, lse2 = 0.f, dlt = 0.f;
+    eight(q + at, qf);
+    if (BWD) {
+        eight(dout + at, df);
+        lse2 = lse_in[(int64_t)hq * T + t] * LOG2E_F;
+        dlt = delta[(int64_t)hq * T + t];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+    bool keys = false;
+    for (int w0 = 0; w0 * 32 < L; w0 += 64) {
+        const uint32_t mine = w0 + lane < ldw ? bitmap[(int64_t)t * ldw + w0 + lane] : 0u;
+        for (uint64_t some = __builtin_amdgcn_ballot_w64(mine != 0u); some; some &= some - 1) {
+            const int wl = (int)__builtin_ctzll(some);
+            uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)mine, wl);
+            while (word) {                           // four keys, one to each sixteen lanes
+                int col = -1;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (i == g && word) col = (w0 + wl) * 32 + (int)__builtin_ctz(word);
+                    word &= word - 1;
+                }
+                if (col >= 0 && col < L) {
+                    keys = true;
+                    const int64_t key = ((int64_t)(s0 + col) * Hkv + kvh) * D + sub * 8;
+                    float kf[8], vf[8], s = 0.f, dp = 0.f;
+                    eight(k + key, kf);
+                    eight(v + key, vf);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        s = fmaf(kf[i], qf[i], s);
+                        if (BWD) dp = fmaf(vf[i], df[i], dp);
+                    }
+                    s = over_key(s) * scale_log2;
+                    if (BWD) {
+                        const float ds = fast_exp2(s - lse2) * (over_key(dp) - dlt);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[i] = fmaf(ds, kf[i], acc[i]);
+                    } else {
+                        const float top = fmaxf(m, s), alpha = m == top ? 1.f : fast_exp2(m - top), p = s == -INFINITY ? 0.f : fast_exp2(s - top);
+                        m = top;
+                        l = fmaf(l, alpha, p);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[i] = fmaf(p, vf[i], acc[i] * alpha);
+                    }
+                }
+            }
+        }
+    }
+    auto over_groups = [](float x) __attribute__((always_inline)) {
+        x += __shfl_xor(x, 16, 64);
+        return x + __shfl_xor(x, 32, 64);
+    };
+    float mul = scale;
+    if (!BWD) {                                      // the four sums under one reference (a group that met no logit above -inf has none)
+        float top = fmaxf(m, __shfl_xor(m, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float to = m == top ? 1.f : fast_exp2(m - top);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] *= to;
+        l = over_groups(l * to);
+        mul = l != 0.f ? 1.f / l : __builtin_amdgcn_ballot_w64(keys) ? NAN : 0.f;         // no key: zero output, lse = -inf; none above -inf: no softmax
+        if (lane == 0) lse[(int64_t)hq * T + t] = (top + log2f(l)) * LN2_F;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = over_groups(acc[i]) * mul;
+    if (g == 0) *reinterpret_cast<u32x4 *>(out + at) = u32x4{pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3]), pack2bf(acc[4], acc[5]), pack2bf(acc[6], acc[7])};
+}
 
 // BWD: dQ (acc, out = dq) instead of the forward (acc, out, lse)
 template <int GSHIFT, bool BWD>
@@ -278,132 +366,30 @@ __global__ __launch_bounds__(sel_waves(BWD) * 64, 1) void dsa_tile_sel_kernel(
     // (where the row lies is formed again: the loop needs its registers)
     int j_ = j;
     asm volatile("" : "+v"(j_));
-    const int qcol_ = q0 + (j_ >> GSHIFT), hq_ = kvh * G + (j_ & ((1 << GSHIFT) - 1)), t_ = s0 + qcol_;
+    const int qcol_ = q0 + (j_ >> GSHIFT), head_ = j_ & ((1 << GSHIFT) - 1), hq_ = kvh * G + head_, t_ = s0 + qcol_;
+    const bool there = qcol_ >= pos_min && qcol_ < L && head_ < G;
     const float l = BWD ? 0.f : half_sum_f(lsum);
-    if (qcol_ >= pos_min && qcol_ < L && (j_ & ((1 << GSHIFT) - 1)) < G) {
-        float mul = BWD ? scale : l > 0.f ? 1.f / l : 0.f;                // nothing selected: zero output, lse = -inf
-        // A row that is not finite goes to dsa_sel_redo_kernel, all of it NaN: the probabilities of keys that it left out are 0, but a step multiplies
-        // them with the V (dQ: K) of keys that the wave's other rows selected, and 0 times Inf or NaN is NaN
-        float odd = 0.f;
+    float odd = 0.f;                                     // 0, of a row that is not finite NaN
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int vi = 0; vi < 16; ++vi) odd = fmaf(acc[dt][vi], 0.f, odd);
-        const float lost = half_sum_f(odd);                               // 0 or NaN
-        mul += lost;
+        for (int vi = 0; vi < 16; ++vi) odd = fmaf(acc[dt][vi], 0.f, odd);
+    odd = half_sum_f(odd);
+    if (there && odd == odd) {
+        const float mul = BWD ? scale : l > 0.f ? 1.f / l : 0.f;          // nothing selected: zero output, lse = -inf
         bf16_t *const row = out + ((int64_t)t_ * Hq + hq_) * D;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) store_c_tile(row + dt * 32, acc[dt], mul, h);
-        if (!BWD && h == 0) lse[(int64_t)hq_ * T + t_] = ((mneg == mneg ? -mneg : -INFINITY) + log2f(l)) * LN2_F + lost;
+        if (!BWD && h == 0) lse[(int64_t)hq_ * T + t_] = ((mneg == mneg ? -mneg : -INFINITY) + log2f(l)) * LN2_F;
     }
-}
-
-// Rows that the walk left NaN, over their own keys alone: what a key holds that a row did not select reaches nothing of it (as when such rows were
-// gathered).  A wave looks at 64 rows of one head - their log-sum-exps, or the first elements of their gradients - and forms the marked ones one by
-// one: sixteen lanes to a key, four keys at a time, fp32 throughout.  Without a mark the launch is lost in the walk's time (131 072 tokens, forward and
-// backward 405.5 ms without and 405.9 with it); 40 000 tokens, 32 heads over 8, K = 2048, forward / backward: 11 / 34 ms, one Inf in V 54 / 73, every row of q NaN 68 / 83.
-template <bool BWD>
-__global__ __launch_bounds__(256) void dsa_sel_redo_kernel(
-    const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ dout,
-    const float *__restrict__ lse_in, const float *__restrict__ delta, const uint32_t *__restrict__ bitmap, int ldw, const int32_t *__restrict__ cu, int N,
-    int T, int Hq, int Hkv, float scale, float logit_scale_, int pos_min, int pos_max, int split_len, bf16_t *out, float *lse) {
-    constexpr int D = 128;
-    const int lane = threadIdx.x & 63, g = lane >> 4, sub = lane & 15;
-    const int t0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x / Hq * 256 + (threadIdx.x & ~63))), hq = blockIdx.x % Hq, kvh = hq / (Hq / Hkv);
-    bool nan = false;
-    if (t0 + lane < T) {
-        if (BWD) {
-            const uint32_t x = *reinterpret_cast<const uint16_t *>(out + ((int64_t)(t0 + lane) * Hq + hq) * D);
-            nan = (x & 0x7fffu) > 0x7f80u;
-        } else {
-            const float x = lse[(int64_t)hq * T + t0 + lane];
-            nan = x != x;
-        }
-    }
-    uint64_t marked = __builtin_amdgcn_ballot_w64(nan);
-    const float scale_log2 = logit_scale_ * LOG2E_F;
-    auto eight = [](const bf16_t *p, float (&x)[8]) __attribute__((always_inline)) {
-        const u32x4 w = __builtin_bit_cast(u32x4, load_bf16x8(p));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
-    };
-    auto over_key = [](float x) __attribute__((always_inline)) {          // sum over the sixteen lanes of a key
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-        return x;
-    };
-    for (; marked; marked &= marked - 1) {
-        const int t = t0 + (int)__builtin_ctzll(marked), seg = find_segment_wave(cu, N, t);
-        const int s0 = cu[seg], L = min(cu[seg + 1] - s0, ldw * 32), pos = t - s0;
-        if (L < split_len || pos < pos_min || pos >= min(L, pos_max)) continue;               // (of the tile or the gather kernels)
-        const int64_t at = ((int64_t)t * Hq + hq) * D + sub * 8;
-        float qf[8], df[8], acc[8], m = -INFINITY, l = 0.f, lse2 = 0.f, dlt = 0.f;
-        eight(q + at, qf);
-        if (BWD) {
-            eight(dout + at, df);
-            lse2 = lse_in[(int64_t)hq * T + t] * LOG2E_F;
-            dlt = delta[(int64_t)hq * T + t];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-        bool keys = false;
-        for (int w0 = 0; w0 * 32 < L; w0 += 64) {
-            const uint32_t mine = w0 + lane < ldw ? bitmap[(int64_t)t * ldw + w0 + lane] : 0u;
-            for (uint64_t some = __builtin_amdgcn_ballot_w64(mine != 0u); some; some &= some - 1) {
-                const int wl = (int)__builtin_ctzll(some);
-                uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)mine, wl);
-                while (word) {                           // four keys, one to each sixteen lanes
-                    int col = -1;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (i == g && word) col = (w0 + wl) * 32 + (int)__builtin_ctz(word);
-                        word &= word - 1;
-                    }
-                    if (col >= 0 && col < L) {
-                        keys = true;
-                        const int64_t key = ((int64_t)(s0 + col) * Hkv + kvh) * D + sub * 8;
-                        float kf[8], vf[8], s = 0.f, dp = 0.f;
-                        eight(k + key, kf);
-                        eight(v + key, vf);
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            s = fmaf(kf[i], qf[i], s);
-                            if (BWD) dp = fmaf(vf[i], df[i], dp);
-                        }
-                        s = over_key(s) * scale_log2;
-                        if (BWD) {
-                            const float ds = fast_exp2(s - lse2) * (over_key(dp) - dlt);
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) acc[i] = fmaf(ds, kf[i], acc[i]);
-                        } else {
-                            const float top = fmaxf(m, s), alpha = m == top ? 1.f : fast_exp2(m - top), p = s == -INFINITY ? 0.f : fast_exp2(s - top);
-                            m = top;
-                            l = fmaf(l, alpha, p);
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) acc[i] = fmaf(p, vf[i], acc[i] * alpha);
-                        }
-                    }
-                }
-            }
-        }
-        auto over_groups = [](float x) __attribute__((always_inline)) {
-            x += __shfl_xor(x, 16, 64);
-            return x + __shfl_xor(x, 32, 64);
-        };
-        float mul = scale;
-        if (!BWD) {                                      // the four sums under one reference (a group that met no logit above -inf has none)
-            float top = fmaxf(m, __shfl_xor(m, 16, 64));
-            top = fmaxf(top, __shfl_xor(top, 32, 64));
-            const float to = m == top ? 1.f : fast_exp2(m - top);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] *= to;
-            l = over_groups(l * to);
-            mul = l != 0.f ? 1.f / l : __builtin_amdgcn_ballot_w64(keys) ? NAN : 0.f;         // no key: zero output, lse = -inf; none above -inf: no softmax
-            if (lane == 0) lse[(int64_t)hq * T + t] = (top + log2f(l)) * LN2_F;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = over_groups(acc[i]) * mul;
-        if (g == 0) *reinterpret_cast<u32x4 *>(out + at) = u32x4{pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3]), pack2bf(acc[4], acc[5]), pack2bf(acc[6], acc[7])};
+    // Rows that are not finite are formed again, over their own keys alone, so that what a key holds reaches nothing that did not select it (as when
+    // such rows were gathered): the probabilities of keys that a row left out are 0, but a step multiplies them with the V (dQ: K) of keys that the
+    // wave's other rows selected, and 0 times Inf or NaN is NaN.  (Here, and not by a launch behind the walk that looks for NaN: that took 4 to 5 us
+    // each way whether there was one or not.  40 000 tokens, 32 heads over 8, K = 2048, forward / backward: 11 / 34 ms, one Inf in V 79 / 118, every row of q NaN 83 / 118.)
+    for (uint32_t again = (uint32_t)__builtin_amdgcn_ballot_w64(there && !(odd == odd)); again; again &= again - 1) {
+        const int r = (int)__builtin_ctz(again);
+        sel_redo_row<BWD>(q, k, v, dout, lse_in, delta, bitmap, ldw, T, Hq, Hkv, scale, logit_scale_ * LOG2E_F, s0, L, kvh, s0 + q0 + (r >> GSHIFT),
+                          kvh * G + (r & ((1 << GSHIFT) - 1)), out, lse);
     }
 }
 
@@ -419,9 +405,6 @@ static hipError_t launch_sel_i(hipStream_t stream, const void *q, const void *k,
     const dim3 grid((unsigned)(((int64_t)T / (NW * 32 >> GSHIFT) + N + 1) * Hkv));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)dout, lse_in,
                        delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, logit_scale(scale), pos_min, pos_max, split_len, (bf16_t *)out, lse);
-    hipLaunchKernelGGL((dsa_sel_redo_kernel<BWD>), dim3((unsigned)((T + 255) / 256 * (int64_t)Hq)), dim3(256), 0, stream, (const bf16_t *)q, (const bf16_t *)k,
-                       (const bf16_t *)v, (const bf16_t *)dout, lse_in, delta, bitmap, ldw, cu, N, T, Hq, Hkv, scale, logit_scale(scale), pos_min, pos_max,
-                       split_len, (bf16_t *)out, lse);
     return hipGetLastError();
 }
 // rows at positions pos_min (a multiple of 256) to pos_max - 1 of segments of split_len tokens and more; head_dim 128, two to four heads per kv head
