@@ -172,9 +172,11 @@ int dsa_attn_fwd_saved_bitmap(const void *q, const void *k, const void *v, const
  * that dsa_index_topk_bitmap left (K: the top_k it was made with; rows at positions below it are taken to attend all of
  * their window).  dsa_attn_reads_list says (1) whether those two would hand rows of segments up to
  * max_seqlen to kernels that gather by the list; the calls here keep every row on the kernels that read the bitmap, right
- * for any row and the same bits where the answer is 0, slower than the gather where it is 1.
+ * for any row and the same bits where the answer is 0, slower than the gather where it is 1.  dsa_attn_batch_reads_list: the same of a
+ * batch of T tokens in N segments, 0 also where dsa_attn_reads_list would need to know them.
  */
 int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen);
+int dsa_attn_batch_reads_list(int Hq, int Hkv, int D, int K, int T, int N, int max_seqlen);
 int dsa_index_topk_words(const void *q_idx, const void *k_idx, const void *w_idx, const int32_t *cu_seqlens, int T, int N,
                          int Hi, int Di, int K, float scale, int dtype, int max_seqlen, void *bitmap, size_t bitmap_bytes,
                          void *ws, size_t ws_bytes, void *stream);
@@ -219,7 +221,8 @@ int dsa_attn_mass_saved_bitmap(const void *q, const void *k, const float *lse, c
  * rest on the gather kernels.  0 = gather only; INT_MAX/top_k or more = tiles only.  At the default, 24, head_dim 128 with two
  * to four heads per kv head splits otherwise: segments of 18 * top_k tokens and more (26 with two heads) that have rows enough for a launch of
  * its own, by themselves or with the others of a batch of long ones, run their rows from position 16 * top_k on in the compacted walk of
- * dsa_tile_sel.hip (up to 75 * top_k, 150 with two heads, the rest gathered); elsewhere the tile kernels go on to 75 * top_k with two heads.
+ * dsa_tile_sel.hip (up to 75 * top_k, 150 with two heads, the rest gathered); elsewhere the tile kernels take segments up to 32 * top_k whole (with two
+ * heads rows up to 75 * top_k and segments up to 100 whole), and all segments too short for the walk where it begins at 48 * top_k or before in a batch.
  * A row's low bits depend on the kernel that takes it.
  * idx == NULL (dense causal attention) always uses the tile kernels.
  */

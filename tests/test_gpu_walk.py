@@ -26,10 +26,11 @@ def _reference(q, k, v, dout, sel, scale):
 
 
 @pytest.mark.parametrize("Hq,Hkv,lens,K,kind,scale", [
-    # (heads enough for the walk to take segments from 350 tokens on, or from 150 where the segments of a batch are as long on average)
+    # (heads enough for the walk to take segments from 290 tokens on, or from 150 where the segments of a batch are as long on average)
     (288, 72, (641, 256, 257, 97), 8, "random", None),   # tiles to 256, walk to 768: rows on either side of a block of 96 queries
-    (296, 74, (1000, 334, 333) + (21,) * 20, 8, "random", None),      # and the gather beyond 768; segments on either side of the walk's line
+    (296, 74, (1000, 290, 289) + (21,) * 20, 8, "random", None),      # and the gather beyond 768; segments on either side of the walk's line
     (440, 220, (1400, 300), 8, "random", None),          # two heads per kv head: the gather from 1280 on
+    (80, 40, (900, 770, 768), 8, "random", None),        # fewer of them: segments longer than the tiles reach
     (288, 96, (700,), 16, "random", -0.1),               # a group of three, a negative scale
     (296, 74, (1025, 705), 40, "runs", None),             # every key of a block wanted by some query: four steps
     (288, 72, (769,), 8, "classes", None),               # keys 16 apart: one class of the block's rows
@@ -37,7 +38,8 @@ def _reference(q, k, v, dout, sel, scale):
 def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
     print("compacted walk", Hq, Hkv, lens, K, kind, flush=True)
     lib, G = _lib.load(), Hq // Hkv
-    first = 16 * K + (100000 // Hq if G == 2 else 15250 // Hkv)         # the shortest segment that walks
+    past_tiles = (75 * K + 255) // 256 * 256 + 1
+    first = min(16 * K + 100000 // Hq, max(past_tiles, 16 * K + 40000 // Hq)) if G == 2 else 16 * K + 12000 // Hkv      # the shortest segment that walks
     assert lib.dsa_get_tile_crossover() == 24 and max(lens) >= max(first, (26 if G == 2 else 18) * K)
     g = torch.Generator().manual_seed(Hq * K + len(lens))
     T, cu = sum(lens), [0]

@@ -45,6 +45,8 @@ def test_words_alone_are_those_beside_the_list(segs, K, ties):
     (576, 144, 128, (1280, 290, 7), 16, torch.bfloat16),  # past 16 K the compacted walk, up to the last row before the gather begins
     (576, 144, 128, (1281, 290), 16, torch.bfloat16),    # and the first of the gather: the list is written after all
     (8, 2, 128, (600, 384, 290), 16, torch.bfloat16),    # too few heads for the walk: rows past 24 K gathered
+    (64, 16, 128, (500, 430, 405, 400, 295), 16, torch.bfloat16),    # segments from 406 tokens on walked, shorter ones on the tiles past 24 K too: no list for this batch
+    (8, 2, 128, (513, 512, 290), 16, torch.bfloat16),    # all of a segment of 32 K on the tiles, a longer one's rows past 24 K gathered
     (8, 2, 128, (500, 190, 250), 200, torch.bfloat16),   # blocks of queries that keep their whole window, also one that ends with its segment
     (4, 4, 64, (600, 41), 256, torch.bfloat16), (6, 2, 80, (500,), 127, torch.bfloat16), (4, 2, 256, (700, 64), 130, torch.bfloat16),
     (4, 1, 256, (333,), 32, torch.bfloat16), (8, 4, 48, (513, 200), 64, torch.float32), (4, 2, 128, (300,), 129, torch.float32)])

@@ -54,6 +54,7 @@ _SIGNATURES = {
     "dsa_index_topk_bitmap": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                       c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
     "dsa_attn_reads_list": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "dsa_attn_batch_reads_list": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "dsa_index_topk_words": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                      c_int, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
     "dsa_attn_fwd_words": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int,

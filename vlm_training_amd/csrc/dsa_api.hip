@@ -299,23 +299,29 @@ extern "C" int dsa_get_tile_crossover(void) { return g_tile_crossover.load(std::
 // 36 000 9.1 / 27.7 -> 9.8 / 27.3, 33 000 7.7 / 22.5 -> 8.9 / 23.7.  With 8 and 16 heads per kv head (32 768 tokens, two kv heads, K = 512) the
 // gather is the faster one from 16 K on: forward 1.45 and 1.71 ms against 1.84 and 3.29; at head_dim 64 with 4 heads too, 0.59 against 0.81.
 // The walk is a launch of its own behind the tiles', as long as its longest row's walk however few the rows are, and the backward forms delta in
-// a pass of its own again: it takes rows to win that back.  Forward + backward, us, tiles to 24 K and gather -> walk, by the rows past 16 K
-// times the heads.  One segment, 32 heads over 8, K = 512: 34 000 2616 -> 2761, 67 000 3222 -> 3261, 132 000 4535 -> 4370; K = 256: 34 000 974 -> 993, 67 000
-// 1250 -> 1274, 99 000 1653 -> 1571; K = 128: 34 000 402 -> 469, 50 000 535 -> 531, 83 000 752 -> 705.  8 over 2, K = 512: 33 000 1264 -> 1481, 49 000 1704 -> 1755,
-// 82 000 2546 -> 2398; K = 128: 56 000 (all that the walk may take) 616 -> 656.  Several segments of 18 to 36 K, 8 over 2, K = 64: 36 000 526 -> 549, 56 000 539 -> 559, 88 000
-// 608 -> 599; 32 over 8: 142 000 1792 -> 1809, 548 000 2847 -> 2455.
-// Two heads per kv head, 16 over 8: one segment, K = 512: 66 000 2369 -> 2590, 99 000 3134 -> 3313, 164 000 5103 -> 4645; K = 256: 83 000 1403 -> 1449, 132 000
-// 2340 -> 2192; and a wave holds twice the queries, so that rows have to be thinner (full launches of 24 K: 1133 -> 1203, 28 K: 1351 -> 1283).  The gather,
-// which reads a key's rows for two heads, is slower than the tiles wherever the walk does not stand (36 K: 1558 and 1750, 70 K: 2696 and 2824).
-#define DSA_WALK_ROWS 61000                              // rows times heads (of groups padded to a power of two), at least
-#define DSA_WALK_ROWS_2 100000                           // with two heads per kv head
+// a pass of its own again: it takes rows to win that back.  Operator steps, walk over tiles and gather, 4 to 32 heads of four per kv head, K = 64 to 1024, one segment
+// and three, by the rows past 16 K times the heads: 20 000 to 40 000 1.00 to 1.28, 40 000 to 50 000 1.00 to 1.10 (segments of 34 and 40 K 0.96), 50 000 to 60 000 0.93 to
+// 1.05, 60 000 to 70 000 0.94 to 1.02, 80 000 to 100 000 0.93 to 1.02, 110 000 to 130 000 0.89 to 0.96.
+// Two heads per kv head: a wave holds twice the queries, so that rows have to be thinner, and more of them: 40 000 to 50 000 1.07 to 1.14 (segments of 80 K and more
+// 0.94 to 0.98), 60 000 to 80 000 0.99 to 1.07, 90 000 to 100 000 1.00 to 1.05, 100 000 to 120 000 0.94 to 1.02, 140 000 0.91 to 1.01.  The gather, which reads a key's rows for two
+// heads, is slower than the tiles wherever the walk does not stand (36 K: 1558 and 1750 us, 70 K: 2696 and 2824).
+// A batch without rows for the gather is spared two launches and the selection's list: segments that pass 24 K by less than a third stay on the tiles
+// (tile_rows_end), and in batches whose longer ones are walked, from 48 K on at the latest, all shorter ones.  Steps, us, gather from 24 K -> tiles:
+// 12 heads over 4, K = 64, 1607 tokens 173 -> 147, 32 over 8 with segments of 31 K and 6 K 316 -> 278, K = 128, 28 K 0.96 on average; from K = 512 on level.
+// Beyond, 34 K: 4 over 1, K = 64, 162 -> 180, K = 128 340 -> 374.
+#define DSA_WALK_ROWS 48000                              // rows times heads (of groups padded to a power of two), at least
+#define DSA_WALK_ROWS_2 100000                           // with two heads per kv head,
+#define DSA_WALK_ROWS_2_LONG 40000                       // of segments that pass the tiles
 struct RowSplit {
     int tiles, walk, len, below;
     bool walks(int max_seqlen) const { return walk > tiles && max_seqlen > tiles && max_seqlen >= len; }
     // (the only segment of a batch has all of its tokens)
-    bool gathers(int max_seqlen, int T, int N) const { return max_seqlen > walk || (max_seqlen > below && len > below + 1 && (N != 1 || T < len)); }
+    bool gathers(int max_seqlen, int T, int N) const {
+        return (max_seqlen > walk && max_seqlen >= len) || (max_seqlen < len ? tile_rows_end(max_seqlen, tiles, len, below) < max_seqlen
+                                                                             : tile_rows_end(len - 1, tiles, len, below) < len - 1 && (N != 1 || T < len));
+    }
 };
-// (N = 0: of a segment whose batch is not known, which takes no fewer rows than any batch)
+// (N = 0: of a segment whose batch is not known, which takes no fewer rows to walk than any batch)
 static RowSplit row_split_for(bool selected, const int32_t *idx, int T, int N, int Hq, int Hkv, int D, int K) {
     if (!selected) return {INT32_MAX, INT32_MAX, 0, INT32_MAX};           // dense causal: tiles everywhere
     auto line = [&](int64_t times) {
@@ -328,20 +334,30 @@ static RowSplit row_split_for(bool selected, const int32_t *idx, int T, int N, i
         const int split = idx ? line(crossover) : INT32_MAX;
         return {split, split, 0, split};
     }
-    // the rows a segment has by itself, or, where the segments of the batch are long on average, as many segments like it as there are tokens for
-    auto tokens_for = [&](int64_t times, double rows) { return (int)std::min(K * (double)times + rows, (double)INT32_MAX); };
+    // tokens of a segment that has `rows` by itself, or, where the segments of the batch are long on average, with as many like it as there are tokens for
     const int heads = Hkv << (two ? 1 : 2), least = line(two ? 26 : 18);
-    const double rows = two ? DSA_WALK_ROWS_2 : DSA_WALK_ROWS, all = (double)T * heads;
-    const int alone = std::max(least, tokens_for(16, rows / heads)), many = all > rows ? std::max(least, tokens_for(16, 16. * K * rows / (all - rows))) : INT32_MAX;
-    RowSplit s{line(16), line(two ? 150 : 75), N > 0 && T / N >= many ? std::min(many, alone) : alone, line(two ? 75 : crossover)};
-    if (s.len > s.walk) s.tiles = s.walk = s.below, s.len = 0;            // (rows too thin for the walk before there are enough of them)
-    if (!idx) s = {s.len ? s.tiles : INT32_MAX, INT32_MAX, s.len, INT32_MAX};             // no list to gather by
+    const double all = (double)T * heads;
+    auto len_for = [&](double rows) {
+        auto past = [&](double more) { return std::max(least, (int)std::min(16. * K + more, (double)INT32_MAX)); };
+        const int alone = past(rows / heads), many = all > rows ? past(16. * K * rows / (all - rows)) : INT32_MAX;
+        return N > 0 && T / N >= many ? std::min(many, alone) : alone;
+    };
+    RowSplit s{line(16), line(two ? 150 : 75), len_for(two ? DSA_WALK_ROWS_2 : DSA_WALK_ROWS), line(two ? 75 : crossover)};
+    if (two && s.len > s.below) s.len = std::min(s.len, std::max(s.below + 1, len_for(DSA_WALK_ROWS_2_LONG)));
+    if (s.len > s.walk) s = {s.below, s.below, INT32_MAX, s.below};       // (rows too thin for the walk before there are enough of them)
+    else if (N > 1 && s.len <= line(48)) s.below = std::max(s.below, s.len - 1);
+    if (!idx) s = {s.tiles, INT32_MAX, s.len, INT32_MAX};                 // no list to gather by
     return s;
 }
 extern "C" int dsa_attn_reads_list(int Hq, int Hkv, int D, int K, int max_seqlen) {
     if (Hkv < 1 || Hq < Hkv || K < 1) return 1;
     static const int32_t some = 0;
     return row_split_for(true, &some, 0, 0, Hq, Hkv, D, K).gathers(max_seqlen, 0, 0);
+}
+extern "C" int dsa_attn_batch_reads_list(int Hq, int Hkv, int D, int K, int T, int N, int max_seqlen) {
+    if (Hkv < 1 || Hq < Hkv || K < 1) return 1;
+    static const int32_t some = 0;
+    return row_split_for(true, &some, T, N, Hq, Hkv, D, K).gathers(max_seqlen, T, N);
 }
 
 // The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,

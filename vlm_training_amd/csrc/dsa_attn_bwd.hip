@@ -36,7 +36,7 @@ __global__ __launch_bounds__(64) void dsa_bwd_dq_kernel(
     const int kvh = blockIdx.x / T, t = blockIdx.x % T;
     const int G = Hq / Hkv;
     const int seg = find_segment_wave(cu, N, t), s0 = cu[seg];
-    if (t - s0 < (cu[seg + 1] - s0 >= split_len ? pos_min : pos_short)) return;     // rows before the split belong to the tile kernels
+    if (t - s0 < tile_rows_end(cu[seg + 1] - s0, pos_min, split_len, pos_short)) return;     // rows before the split belong to the tile kernels
     // the count is held to [0, K] and every row id to the batch: a bad list cannot reach outside the tensors
     const int nt = HAS_IDX ? min(nsel[t], K) : (t - s0 + 1);
     const int32_t *irow = HAS_IDX ? idx + (int64_t)t * K : nullptr;

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(64) void dsa_attn_fwd_kernel(
     const int kvh = blockIdx.x / T, t = blockIdx.x % T;
     const int G = Hq / Hkv;
     const int seg = find_segment_wave(cu, N, t), s0 = cu[seg];
-    if (t - s0 < (cu[seg + 1] - s0 >= split_len ? pos_min : pos_short)) return;     // rows before the split belong to the tile kernels
+    if (t - s0 < tile_rows_end(cu[seg + 1] - s0, pos_min, split_len, pos_short)) return;     // rows before the split belong to the tile kernels
     // a caller's own list is trusted for its order only: the count is held to [0, K] and every row id to the batch, so
     // that a bad list gives a wrong result, never an access outside the tensors
     const int nt = HAS_IDX ? min(nsel[t], K) : (t - s0 + 1);

@@ -34,6 +34,11 @@ static inline int dkv_key_groups(int D, int T, int N, int Hq, int Hkv, int causa
     const int64_t wg = ((int64_t)T / 128 + N) * Hkv;
     return wg < 96 || (wg <= dkv_pieces_max_wg(D) && wg * T / N * rows <= 40000 * 32) ? 1 : 2;
 }
+// The split of a selection's rows (row_split_for): the first row of a segment of L tokens that is not the tile kernels'.  pos_split in segments of split_len
+// tokens and more, in shorter ones pos_short, but all of a segment that is up to a third longer than that.
+__host__ __device__ static inline int tile_rows_end(int L, int pos_split, int split_len, int pos_short) {
+    return L >= split_len ? pos_split : L - pos_short > pos_short / 3 ? pos_short : L;
+}
 // dQ in the key side's launch, where one holds both passes (dsa_tile_bwd.hip)
 struct DqBeside { int window; void *dq; };
 #define LOG2E_F 1.4426950408889634f

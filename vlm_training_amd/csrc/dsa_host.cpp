@@ -410,8 +410,8 @@ variable_list varlen_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, 
         TORCH_CHECK_VALUE(iq->dim() == 3, "indexer tensors must be q_idx (T,Hi,Di), k_idx (T,Di), w_idx (T,Hi)");
         // ... alone, unless some row is one for the kernels that gather by the list; nothing writes a list then that the caller did not ask for
         if (bitmap.defined() &&
-            !dsa_attn_reads_list((int)sh.Hq, (int)sh.Hkv, (int)(carried_split(q_.scalar_type(), d_kernel) ? 4 * d_kernel : d_kernel), (int)*top_k,
-                                 (int)max_seqlen))
+            !dsa_attn_batch_reads_list((int)sh.Hq, (int)sh.Hkv, (int)(carried_split(q_.scalar_type(), d_kernel) ? 4 * d_kernel : d_kernel), (int)*top_k,
+                                       (int)sh.T, (int)cu.numel() - 1, (int)max_seqlen))
             words_k = *top_k;
         sel = select_keys(*iq, *ik, *iw, cu, (int)max_seqlen, *top_k, index_scale_of(index_scale, iq->size(1), iq->size(2)), return_scores, bitmap,
                           !words_k || return_indices || return_mass || return_scores);

@@ -67,7 +67,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 128 && NW == 4) ? 2 : 1) void dsa_ti
     L = __builtin_amdgcn_readfirstlane(L);
     if (HAS_IDX) L = min(L, ldw * 32);                  // a bitmap row has ldw words whatever the caller's max_seqlen
     const int qc0 = __builtin_amdgcn_readfirstlane(blk) * QBW;
-    if (qc0 >= (L >= split_len ? pos_split : pos_short) || qc0 >= L) return;       // rows past the split are not the tile kernels'
+    if (qc0 >= min(L, tile_rows_end(L, pos_split, split_len, pos_short))) return;       // rows past the split are not the tile kernels'
     const int ntiles = (causal ? min(qc0 + QBW - 1, L - 1) : L - 1) / 32 + 1;
 
     const int r = wv * 32 + j;
