@@ -90,7 +90,7 @@ def test_rows_of_the_compacted_walk(Hq, Hkv, lens, K, kind, scale):
 
 @pytest.mark.parametrize("G,lens,kind", [
     (4, (1700, 900, 500), "random"),     # 40 K = 1600: the walk takes the first segment, the tile kernel the others
-    (3, (1934, 1919), "random"),         # a group of three, 48 K = 1920; 1934 keys: the last workgroup's 14, one wave's
+    (3, (1614, 1599), "random"),         # a group of three; 1614 keys: the last workgroup's 78, the last wave's 14
     (4, (1600, 1599), "runs"),           # every query of a block wants a key of the tile, or none does
     (8, (1921, 1200), "same"),           # sixteen keys that all queries want: large probabilities, lists that are full
     (16, (2000, 1100), "classes")])      # queries of one residue: one class of the block's rows

@@ -363,20 +363,20 @@ extern "C" int dsa_attn_batch_reads_list(int Hq, int Hkv, int D, int K, int T, i
 // The key side of segments of at least this many tokens is the compacted walk's (dsa_tile_selkv.hip) rather than the tile kernel's: head_dim 128,
 // three and more heads per kv head, launches that the tile kernel does not cut into pieces (its workgroups, 192 keys each, are cut nowhere: four
 // rounds of them end level).  A walk pays for building the list of every block of queries, and adds the rounding remainder of P to dV where a step
-// has a probability of 2^-7, the tile kernel where a block has one of 2^-6: with up to 64 keys a row both do nearly always, with some hundred the
-// walk alone.  dK and dV alone, tile kernel / walk, by tokens a segment in 40 000 to 64 000:
-// K = 16, 32, 64, 32 heads over 8: of 28 K 0.94 to 1.1, of 40 K (K = 32, 64) 0.84 to 0.98, of 56 K 0.69 to 0.84, 3 over each of 4: 0.99 to 1.13 up to 36 K, 0.91 to 0.98 from 40 K;
-// K = 128, 32 over 8 / 3 over each of 4 / 8 over each of 8: 4608 tokens 1.05 to 1.10 / 1.35 / 0.99 to 1.05, 7168 0.88 to 0.91 / 1.02 to 1.07 / 0.84 to 0.86, 10 240 0.75 / 0.90 / 0.70;
-// K = 256: 7680 1.02 to 1.04 / 1.16 to 1.20 / 0.99 to 1.01, 11 264 0.84 / 0.94 / 0.81; K = 512: 13 568 0.97 / 1.04 to 1.14 / 0.94, 18 432 0.90 / 0.90 / 0.88; K = 1024:
-// 27 136 0.98 to 1.01 / 0.95 / 0.96, 36 864 0.88 / - / 0.87.  Whole backward, ms, 32 over 8, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5,
-// 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226.
+// has a probability of 2^-7, the tile kernel where a block has one of 2^-6: up to some hundred keys a row both do nearly always, with flat rows of
+// 128 to some 200 the walk alone.  dK and dV alone, walk over tile kernel, random scores, 30 000 / 56 000 tokens in all, 32 heads over 8 (24 over 8 the same):
+// K = 32: segments of 33 K 1.00 / 0.91, 40 K 0.96 / 0.87; K = 64: 33 K 1.06 / 0.99, 36 K 0.91 / 0.85, 60 K 0.74 / 0.70; K = 96: 28 K 1.00 / 0.93, 40 K 0.86 / 0.82;
+// K = 128: 36 K 1.13 / 1.03, 45 K 1.11 / 1.00, 52 K 0.98 / 0.93; K = 192: 40 K 1.07, 52 K 0.99 / 0.94; K = 256: 30 K 1.06, 33 K 1.01 / 1.00, 40 K 0.91; K = 512: 24 K 1.02 / 1.06,
+// 30 K 1.00, 40 K 0.87; K = 1024: 24 K 0.98 / 1.05, 28 K 1.02, 36 K 0.92.  64 over 16: K = 128, 36 K 1.01, 45 K 0.91; K = 256, 36 K 0.95.  With fewer kv heads
+// it pays later: 16 over 4, 56 000 tokens: K = 64, 45 K 1.08, 60 K 0.78; K = 128, 60 K 1.02; K = 256, 36 K 1.09; K = 512, 36 K 0.93.  Whole backward, ms,
+// 32 over 8, K = 2048: 40 000 tokens 34.0 -> 35.5, 49 152 47.5 -> 48.5, 57 344 63.3 -> 61.7, 65 536 79.5 -> 75.8, 81 920 117.9 -> 106.6, 131 072 281 -> 226.
 static int key_walk_len(bool selected, const void *q, const void *dout, int T, int N, int Hq, int Hkv, int D, int K) {
     const int G = Hq / Hkv;
     if (!selected || D != 128 || G < 3 || ((int64_t)T / 128 + N) * Hkv <= dkv_pieces_max_wg(D) || (((uintptr_t)q | (uintptr_t)dout) & 15) ||
         g_tile_crossover.load(std::memory_order_relaxed) != DSA_TILE_CROSSOVER)
         return INT32_MAX;
-    const bool three = G == 3;                           // (a quarter of the walk's rows is padding)
-    return (int)std::min<int64_t>(K <= 64 ? K * (three ? 48 : 40) : (int64_t)K * 24 + (three ? 6144 : 4608), INT32_MAX);
+    const int64_t len = K <= 112 ? K * 40ll : K < 256 ? K * 50ll : K * 24ll + 3072;
+    return (int)std::min<int64_t>(Hkv < 8 ? len * 6 / 5 : len, INT32_MAX);
 }
 
 extern "C" size_t dsa_attn_fwd_workspace_bytes(int T, int max_seqlen, int has_idx) {

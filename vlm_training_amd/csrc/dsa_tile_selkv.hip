@@ -9,8 +9,9 @@
 // on 16x16x32 MFMA tiles.  At one selected key in forty two thirds of the queries are left out.  Every key row is reduced by one wave in a
 // fixed query order: no atomics, bit-reproducible.
 //
-// What bounds it: nothing alone - at 65 536 tokens and one selected key in thirty the LDS is busy for 0.54 of the time, vector instructions (98 a step
-// beside 32 MFMAs) take 0.48, the matrix cores 0.42 - but their sum and the spread of the waves' steps between two barriers.  Backward of 131 072
+// What bounds it: nothing alone - at 131 072 tokens and one selected key in forty the LDS is busy for 0.52 of the time (0.13 of it bank conflicts), vector
+// instructions (98 a step beside 32 MFMAs) take 0.43, the matrix cores 0.37 - but their sum, 0.87 of a SIMD's issue slots, and the spread of the waves'
+// steps between two barriers.  Backward of 131 072
 // tokens, K = 2048, ms: tile kernel 281; here with 32 keys a wave, eight waves and V in LDS (twice the queries per wave, two waves to a SIMD) 258,
 // 16 keys and twelve waves 238, rows of a step picked by class (1.7 -> 1.1 clocks a read) 226.  An odd tile as a step of its own (half the reads):
 // two step bodies share the sums badly, 20 spilled registers.

@@ -56,12 +56,12 @@ class Workload:
         """(query side, key side): the (query, key) pairs that the tile kernels put through the matrix cores when they take every row (forward, dQ) and
         every key (dK/dV) - every causal pair.  None for a side of which segments are long enough for other kernels, whose pairs go by the
         selection: rows gathered past top_k * crossover, or, at the default crossover and head_dim 128, the compacted walks of rows past 16 * top_k
-        (two to four heads per kv head) and of keys (three and more, from 24 * top_k + 4608 tokens on, 40 * top_k up to 64 keys a row, in launches too
-        large to be cut into pieces)."""
+        (two to four heads per kv head) and of keys (three and more, in segments of 24 * top_k + 3072 or 40 * top_k tokens at the least and in launches
+        too large to be cut into pieces)."""
         G, K, causal = self.Hq // self.Hkv, self.top_k, self.pair_counts()[0]
         walks = crossover == 24 and self.D == 128
         rows = K * (16 if walks and 2 <= G <= 4 else crossover)
-        keys = (24 * K + 4608 if K > 64 else 40 * K) if walks and G >= 3 and (self.T // 128 + len(self.seg_lens)) * self.Hkv > 1536 else self.max_seqlen + 1
+        keys = min(24 * K + 3072, 40 * K) if walks and G >= 3 and (self.T // 128 + len(self.seg_lens)) * self.Hkv > 1536 else self.max_seqlen + 1
         return causal if self.max_seqlen <= rows else None, causal if self.max_seqlen < keys else None
 
     def work(self) -> Dict[str, float]:
