@@ -10,7 +10,7 @@
 // walk takes four, and a block read from L2 serves all queries of the workgroup (the gather kernels read every row's keys on its own: 0.6 TB
 // past L2 at 131 072 tokens).
 //
-// What bounds it: the LDS (operand rows of a list lie where they lie: 1.8 clocks a read instead of 1.0, dQ 2.1; busy 0.53 and 0.57 of the time at
+// What bounds it: the LDS (operand rows of a list lie where they lie: 1.8 clocks a read instead of 1.0, dQ 2.1; busy 0.53 and 0.56 of the time at
 // 131 072 tokens), the vector instructions (about 100 a step, 45 more a block for the list; 0.47 and 0.36 of a SIMD's time, MFMAs 0.33 and 0.37) and the
 // spread of the waves' steps between two barriers.  Rows beyond
 // 16 K of 131 072 tokens, K = 2048, 32 heads over 8 kv heads, the whole forward / backward, ms: gathered 94.5 / 299; here with eight waves and a step's
